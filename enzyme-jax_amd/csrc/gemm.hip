@@ -11,8 +11,7 @@
 //   NT  Y  = X . W^T    (A k-contiguous, B k-contiguous)   forward
 //   NN  dX = dY . W     (A k-contiguous, B k-major)        input adjoint
 //   TN  dW = dY^T . X   (A k-major,      B k-major)        weight adjoint
-// Generic path (fp32, or bf16 with shapes/alignments the fast path does not
-// take): v_mfma_f32_32x32x2_f32 with predicated scalar loads.
+// fp32: gemm_f32.hip.  Generic path (shapes/alignments that neither takes): v_mfma_f32_32x32x2_f32 with predicated scalar loads.
 #include <stdlib.h>
 #include <type_traits>
 #include <utility>
@@ -1245,37 +1244,24 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const T* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// fp32 products on aligned operands.  The 15M-parameter model's projections are 256 x 288 x 288: few tiles, and a
-// block's time is its serial chain of K-steps, so the work is cut fine: a block owns a 32x32 tile of C and its four wavefronts each take a quarter
-// of K, reading their operand fragments straight from global memory in the v_mfma_f32_32x32x2_f32 layout (lane l
-// supplies A[l % 32][l / 32] and B[l / 32][l % 32]).  The contraction index of an instruction is the lane half
-// g = l / 32; instruction t of an 8-wide chunk contracts k = k0 + 4 g + t, so a k-contiguous operand is read in
-// 16-byte pieces and a k-major one in 128-byte rows.  The four partial tiles are added in wavefront order through
-// LDS (fixed order: run-to-run identical bits).
+// fp32 products whose stored rows are not multiples of four elements (a vocabulary of odd size; gemm_f32.hip has the
+// others).  A block owns a 32x32 tile of C and its four wavefronts each take a quarter of K, reading their operand
+// fragments straight from global memory in the v_mfma_f32_32x32x2_f32 layout (lane l supplies A[l % 32][l / 32] and
+// B[l / 32][l % 32]).  The contraction index of an instruction is the lane half g = l / 32; instruction t of an 8-wide
+// chunk contracts k = k0 + 4 g + t, so a k-contiguous operand is read in 16-byte pieces and a k-major one in 128-byte
+// rows.  The four partial tiles are added in wavefront order through LDS (fixed order: run-to-run identical bits).
 // ---------------------------------------------------------------------------
-// GROUPED: blockIdx.z picks one of grp.count independent products of one shape (GemmGroup with sum == 0, its pointers
-// read as float).
-// NW wavefronts share K; U 8-wide chunks are in flight per step.  ONCE: a wavefront's share of K is at most U chunks
-// (K <= 96 NW), so everything is requested up front and the block waits for memory once: a short contraction is a
-// chain of load latencies otherwise (256 x 288 x 288: 10 us in three steps).
-template <bool A_KMAJOR, bool B_KMAJOR, bool GROUPED = false, int NW = 4, int U = 4, bool ONCE = false>
-__global__ __launch_bounds__(NW * 64) void gemm_f32_small_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                                 const float* R, float* C, int M, int N, int K, int64_t lda,
-                                                                 int64_t ldb, int64_t ldr, int64_t ldc,
-                                                                 std::conditional_t<GROUPED, GemmGroup, NoGroup> grp,
-                                                                 float* __restrict__ part = nullptr, int kps = 0) {
+template <bool A_KMAJOR, bool B_KMAJOR>
+__global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float* __restrict__ A, const float* __restrict__ B, const float* R,
+                                                             float* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldr,
+                                                             int64_t ldc, float* __restrict__ part, int kps) {
+  constexpr int NW = 4, U = 4;          // wavefronts that share K; 8-wide chunks in flight per step
   __shared__ float red[NW - 1][16][64];
-  if constexpr (GROUPED) {
-    A = reinterpret_cast<const float*>(grp.A[blockIdx.z]);
-    B = reinterpret_cast<const float*>(grp.B[blockIdx.z]);
-    R = reinterpret_cast<const float*>(grp.R[blockIdx.z]);
-    C = reinterpret_cast<float*>(grp.C[blockIdx.z]);
-  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = lane & 31, g = lane >> 5;
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
   const int mi = m0 + i < M ? m0 + i : M - 1, ni = n0 + i < N ? n0 + i : N - 1;      // clamped: those results are not stored
-  // split-K (part != nullptr, not GROUPED): plane blockIdx.z takes kps (a multiple of 8 NW) of K and leaves its
+  // split-K (part != nullptr): plane blockIdx.z takes kps (a multiple of 8 NW) of K and leaves its
   // 32 x 32 partial in part[z][M][N] for gemm_splitk_reduce_kernel
   const int kb = part != nullptr ? (int)blockIdx.z * kps : 0;
   const int kend = part != nullptr && kb + kps < K ? kb + kps : K;
@@ -1311,28 +1297,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_small_kernel(const float* __
     }
   };
   if (ks < ke) load(ks, a, b);
-  if constexpr (ONCE) {
-    if (ks < ke) {
+  float an[U][4], bn[U][4];
+  for (int k0 = ks; k0 < ke; k0 += 8 * U) {
+    const bool more = k0 + 8 * U < ke;
+    if (more) load(k0 + 8 * U, an, bn);            // in flight while this step is multiplied
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][t], b[u][t], acc, 0, 0, 0);
+    if (more) {
 #pragma unroll
       for (int u = 0; u < U; u++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][t], b[u][t], acc, 0, 0, 0);
-    }
-  } else {
-    float an[U][4], bn[U][4];
-    for (int k0 = ks; k0 < ke; k0 += 8 * U) {
-      const bool more = k0 + 8 * U < ke;
-      if (more) load(k0 + 8 * U, an, bn);            // in flight while this step is multiplied
-#pragma unroll
-      for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][t], b[u][t], acc, 0, 0, 0);
-      if (more) {
-#pragma unroll
-        for (int u = 0; u < U; u++)
-#pragma unroll
-          for (int t = 0; t < 4; t++) { a[u][t] = an[u][t]; b[u][t] = bn[u][t]; }
-      }
+        for (int t = 0; t < 4; t++) { a[u][t] = an[u][t]; b[u][t] = bn[u][t]; }
     }
   }
   if (wave > 0) {
@@ -1360,140 +1337,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_small_kernel(const float* __
       }
     }
   }
-}
-
-// ---------------------------------------------------------------------------
-// fp32 products that fill the chip with 128 x 128 tiles (the logits and their adjoints: 256 x 32000 x 288 and its
-// two transposes): the same matrix instruction fed from LDS.  The K-split kernel above has every 32 x 32 tile read
-// its own 64 operand rows from the L2 (8 flop per byte), which bounds it at 35-55 TFLOP/s.  Here a block of four
-// wavefronts (2 x 2, 64 x 64 each = four 32 x 32 accumulators) stages 128 x 32 pieces of both operands per step:
-// a k-contiguous operand as [row][32 + 4] (a lane reads its 4 consecutive k as one 16-byte piece), a k-major one as
-// [k][128] (four 4-byte reads, lanes along the rows).  Global loads of step s+1 are in flight while step s is
-// multiplied (held in registers, written to LDS between two barriers).  part / kps as in the kernel above (planes of K).
-// Needs 16-byte aligned bases and leading dimensions that are multiples of 4.
-// ---------------------------------------------------------------------------
-template <bool A_KMAJOR, bool B_KMAJOR>
-__global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                             const float* R, float* C, int M, int N, int K, int64_t lda,
-                                                             int64_t ldb, int64_t ldr, int64_t ldc, float* __restrict__ part,
-                                                             int kps) {
-  constexpr int BT = 128, BK = 32, KC_LD = BK + 4;
-  constexpr int A_FLOATS = A_KMAJOR ? BK * BT : BT * KC_LD, B_FLOATS = B_KMAJOR ? BK * BT : BT * KC_LD;
-  __shared__ __attribute__((aligned(16))) float sA[A_FLOATS];
-  __shared__ __attribute__((aligned(16))) float sB[B_FLOATS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int i = lane & 31, g = lane >> 5;
-  const int m0 = blockIdx.y * BT, n0 = blockIdx.x * BT;
-  const int kb = part != nullptr ? (int)blockIdx.z * kps : 0;
-  const int kend = part != nullptr && kb + kps < K ? kb + kps : K;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-
-  // global -> registers: four 16-byte pieces of each operand per thread and step; zero outside the operand
-  auto gload = [&](const float* X, int64_t ld, bool kmajor, int row0, int rows, int k0, float4 (&v)[4]) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int idx = tid + 256 * q;
-      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (!kmajor) {
-        const int row = row0 + (idx >> 3), k = k0 + (idx & 7) * 4;
-        if (row < rows) {
-          const float* p = X + (int64_t)row * ld + k;
-          if (k + 4 <= kend) x = *reinterpret_cast<const float4*>(p);
-          else {
-            if (k < kend) x.x = p[0];
-            if (k + 1 < kend) x.y = p[1];
-            if (k + 2 < kend) x.z = p[2];
-          }
-        }
-      } else {
-        const int k = k0 + (idx >> 5), row = row0 + (idx & 31) * 4;
-        if (k < kend) {
-          const float* p = X + (int64_t)k * ld + row;
-          if (row + 4 <= rows) x = *reinterpret_cast<const float4*>(p);
-          else {
-            if (row < rows) x.x = p[0];
-            if (row + 1 < rows) x.y = p[1];
-            if (row + 2 < rows) x.z = p[2];
-          }
-        }
-      }
-      v[q] = x;
-    }
-  };
-  auto sstore = [&](float* sX, bool kmajor, const float4 (&v)[4]) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int idx = tid + 256 * q;
-      if (!kmajor) *reinterpret_cast<float4*>(sX + (idx >> 3) * KC_LD + (idx & 7) * 4) = v[q];
-      else *reinterpret_cast<float4*>(sX + (idx >> 5) * BT + (idx & 31) * 4) = v[q];
-    }
-  };
-  // the four k of chunk j (8 wide) that this lane contracts, for tile row r of an operand
-  auto frag = [&](const float* sX, bool kmajor, int r, int j, float (&f)[4]) {
-    if (!kmajor) {
-      const float4 x = *reinterpret_cast<const float4*>(sX + r * KC_LD + 8 * j + 4 * g);
-      f[0] = x.x; f[1] = x.y; f[2] = x.z; f[3] = x.w;
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; t++) f[t] = sX[(8 * j + 4 * g + t) * BT + r];
-    }
-  };
-
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[a][b][r] = 0.f;
-
-  float4 va[4], vb[4];
-  gload(A, lda, A_KMAJOR, m0, M, kb, va);
-  gload(B, ldb, B_KMAJOR, n0, N, kb, vb);
-  for (int k0 = kb; k0 < kend; k0 += BK) {
-    sstore(sA, A_KMAJOR, va);
-    sstore(sB, B_KMAJOR, vb);
-    __syncthreads();
-    if (k0 + BK < kend) {                                // in flight while this step is multiplied
-      gload(A, lda, A_KMAJOR, m0, M, k0 + BK, va);
-      gload(B, ldb, B_KMAJOR, n0, N, k0 + BK, vb);
-    }
-#pragma unroll
-    for (int j = 0; j < BK / 8; j++) {
-      float fa[2][4], fb[2][4];
-#pragma unroll
-      for (int a = 0; a < 2; a++) frag(sA, A_KMAJOR, wm + a * 32 + i, j, fa[a]);
-#pragma unroll
-      for (int b = 0; b < 2; b++) frag(sB, B_KMAJOR, wn + b * 32 + i, j, fb[b]);
-#pragma unroll
-      for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-          for (int b = 0; b < 2; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][t], fb[b][t], acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();                                     // every wavefront is done with this step's tiles
-  }
-  // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32 x 32 tile
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++) {
-      const int col = n0 + wn + b * 32 + i;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int row = m0 + wm + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
-        if (row < M && col < N) {
-          float v = acc[a][b][r];
-          if (part != nullptr) {
-            part[((int64_t)blockIdx.z * M + row) * N + col] = v;
-          } else {
-            if (R != nullptr) v += R[(int64_t)row * ldr + col];
-            C[(int64_t)row * ldc + col] = v;
-          }
-        }
-      }
-    }
 }
 
 // VEC: a thread owns four consecutive columns of a row (N, ldr and ldc multiples of 4, rows of R and C aligned for one
@@ -1895,6 +1738,20 @@ static int launch_generic(hipStream_t st, const void* A, const void* B, const vo
   return EMI_OK;
 }
 
+// gemm_f32.hip adds its planes with the same kernel
+int launch_f32_splitk_reduce(hipStream_t st, const float* part, const float* R, float* C, int M, int N, int splits, int64_t ldr,
+                             int64_t ldc) {
+  launch_splitk_reduce<float>(st, part, R, C, M, N, splits, ldr, ldc);
+  EMI_CHECK_LAUNCH("emi_gemm(fp32 split-K reduce)");
+  return EMI_OK;
+}
+
+// gemm_f32.hip
+int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
+                    void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
+                    int64_t ldc, int trans_a, int trans_b, int sum);
+size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum);
+
 // gemm_skinny.hip
 int launch_skinny(hipStream_t st, const void* A, const void* B, const void* R, void* C, void* workspace, size_t workspace_bytes,
                   int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr, int64_t ldc, int trans_a, int trans_b,
@@ -1915,7 +1772,9 @@ extern "C" size_t emi_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
   int splits = generic_splits(M, N, K);
   if (dtype == EMI_BF16 && bf16_splits(M, N, K) > splits) splits = bf16_splits(M, N, K);
   if (dtype == EMI_BF16 && pingpong_splits(M, N, K, !trans_a && trans_b) > splits) splits = pingpong_splits(M, N, K, true);
-  return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+  const size_t need = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+  const size_t f32 = dtype == EMI_F32 ? gemm_f32_workspace_bytes(M, N, K, 1, 0) : 0;
+  return f32 > need ? f32 : need;
 }
 
 extern "C" int emi_gemm(emi_stream_t stream, const void* A, const void* B, const void* R, void* C, int64_t M, int64_t N,
@@ -1965,92 +1824,39 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
     }
     return launch_generic<bf16>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
   }
-  // fp32 on 16-byte aligned k-contiguous rows: 32x32 tiles, K split over the block's wavefronts, operands straight from global memory (at every size measured
-  // this beats the LDS-staged kernel, whose loads are element-wise: 1024^3 45 vs 3 TFLOP/s, 2048^3 55 vs 13)
+  {
+    const int rc = launch_f32_gemm(st, 1, &A, &B, &R, &C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0);
+    if (rc >= 0) return rc;
+  }
+  // rows that do not divide into 16-byte pieces, k-contiguous ones at least aligned: 32x32 tiles, K split over the block's
+  // wavefronts, operands straight from global memory (this beats the LDS-staged kernel, whose loads are element-wise:
+  // 1024^3 45 vs 3 TFLOP/s, 2048^3 55 vs 13)
   if (K > 0 && (M + 31) / 32 <= 65535 &&
       (trans_a || ((reinterpret_cast<uintptr_t>(A) & 15) == 0 && lda % 4 == 0)) &&
       (!trans_b || ((reinterpret_cast<uintptr_t>(B) & 15) == 0 && ldb % 4 == 0))) {
     dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32));
     const int splits = generic_splits(M, N, K);
-    // 128 x 128 tiles staged through LDS once they fill the chip (alone or as planes of K)
-    const bool tiled_ok = (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0 &&
-                          lda % 4 == 0 && ldb % 4 == 0;
-    const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+    float* part = nullptr;
+    int kps = 0;
     if (splits > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
         workspace_bytes >= (size_t)splits * M * N * sizeof(float)) {
-      // few tiles and a long contraction (dX = dY . Wcls of a small batch): planes of K on the same kernel, partials
-      // added in fixed order by the reduce kernel (256 x 288 x 32000: 130 us on the LDS-staged kernel)
-      int kps = (int)((((K + splits - 1) / splits) + 31) / 32 * 32);
+      // few tiles and a long contraction: planes of K, added in fixed order by the reduce kernel
+      kps = (int)((((K + splits - 1) / splits) + 31) / 32 * 32);
       grid.z = (unsigned)((K + kps - 1) / kps);
-      float* part = static_cast<float*>(workspace);
-      if (tiled_ok && tiles128 * grid.z >= 192) {
-        // one block per CU and no second round: at most 256 / tiles planes (never more than the workspace holds)
-        const int64_t want = 256 / tiles128 < splits ? 256 / tiles128 : splits;
-        kps = (int)((((K + want - 1) / want) + 31) / 32 * 32);
-        grid.z = (unsigned)((K + kps - 1) / kps);
-        const dim3 gridt((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128), grid.z);
-#define EMI_F32_TILED_SPLIT(AKM, BKM)                                                                                      \
-  hipLaunchKernelGGL((gemm_f32_tiled_kernel<AKM, BKM>), gridt, dim3(256), 0, st, static_cast<const float*>(A),             \
-                     static_cast<const float*>(B), static_cast<const float*>(nullptr), static_cast<float*>(C), (int)M,     \
-                     (int)N, (int)K, lda, ldb, ldr, ldc, part, kps)
-        if (!trans_a && trans_b) EMI_F32_TILED_SPLIT(false, false);
-        else if (!trans_a && !trans_b) EMI_F32_TILED_SPLIT(false, true);
-        else if (trans_a && !trans_b) EMI_F32_TILED_SPLIT(true, true);
-        else EMI_F32_TILED_SPLIT(true, false);
-#undef EMI_F32_TILED_SPLIT
-        EMI_CHECK_LAUNCH("emi_gemm(fp32 tiled split-K)");
-        launch_splitk_reduce<float>(st, part, R, C, (int)M, (int)N, (int)grid.z, ldr, ldc);
-        EMI_CHECK_LAUNCH("emi_gemm(fp32 split-K reduce)");
-        return EMI_OK;
-      }
-#define EMI_F32_SPLIT(AKM, BKM)                                                                                            \
-  hipLaunchKernelGGL((gemm_f32_small_kernel<AKM, BKM, false, 4, 4, false>), grid, dim3(256), 0, st,                        \
-                     static_cast<const float*>(A), static_cast<const float*>(B), static_cast<const float*>(nullptr),       \
-                     static_cast<float*>(C), (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, NoGroup{}, part, kps)
-      if (!trans_a && trans_b) EMI_F32_SPLIT(false, false);
-      else if (!trans_a && !trans_b) EMI_F32_SPLIT(false, true);
-      else if (trans_a && !trans_b) EMI_F32_SPLIT(true, true);
-      else EMI_F32_SPLIT(true, false);
-#undef EMI_F32_SPLIT
-      EMI_CHECK_LAUNCH("emi_gemm(fp32 split-K)");
-      launch_splitk_reduce<float>(st, part, R, C, (int)M, (int)N, (int)grid.z, ldr, ldc);
-      EMI_CHECK_LAUNCH("emi_gemm(fp32 split-K reduce)");
-      return EMI_OK;
+      part = static_cast<float*>(workspace);
     }
-#define EMI_F32_SMALL_V(AKM, BKM, NWV, UV, ONCEV)                                                                          \
-  hipLaunchKernelGGL((gemm_f32_small_kernel<AKM, BKM, false, NWV, UV, ONCEV>), grid, dim3(NWV * 64), 0, st,                \
-                     static_cast<const float*>(A), static_cast<const float*>(B), static_cast<const float*>(R),             \
-                     static_cast<float*>(C), (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, NoGroup{})
-    if (tiled_ok && tiles128 >= 192) {
-      const dim3 gridt((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));
-#define EMI_F32_TILED(AKM, BKM)                                                                                            \
-  hipLaunchKernelGGL((gemm_f32_tiled_kernel<AKM, BKM>), gridt, dim3(256), 0, st, static_cast<const float*>(A),             \
+#define EMI_F32_SMALL(AKM, BKM)                                                                                            \
+  hipLaunchKernelGGL((gemm_f32_small_kernel<AKM, BKM>), grid, dim3(256), 0, st, static_cast<const float*>(A),              \
                      static_cast<const float*>(B), static_cast<const float*>(R), static_cast<float*>(C), (int)M, (int)N,   \
-                     (int)K, lda, ldb, ldr, ldc, static_cast<float*>(nullptr), 0)
-      if (!trans_a && trans_b) EMI_F32_TILED(false, false);
-      else if (!trans_a && !trans_b) EMI_F32_TILED(false, true);
-      else if (trans_a && !trans_b) EMI_F32_TILED(true, true);
-      else EMI_F32_TILED(true, false);
-#undef EMI_F32_TILED
-      EMI_CHECK_LAUNCH("emi_gemm(fp32 tiled)");
-      return EMI_OK;
-    }
-    // few blocks: latency decides, everything is requested at once; many blocks: the stepped form, whose smaller
-    // register footprint keeps more wavefronts resident
-    const bool few = (int64_t)grid.x * grid.y <= 1024;
-#define EMI_F32_SMALL(AKM, BKM)                                            \
-  do {                                                                     \
-    if (few && K <= 384) EMI_F32_SMALL_V(AKM, BKM, 4, 12, true);           \
-    else if (few && K <= 768) EMI_F32_SMALL_V(AKM, BKM, 8, 12, true);      \
-    else EMI_F32_SMALL_V(AKM, BKM, 4, 4, false);                           \
-  } while (0)
+                     (int)K, lda, ldb, ldr, ldc, part, kps)
     if (!trans_a && trans_b) EMI_F32_SMALL(false, false);
     else if (!trans_a && !trans_b) EMI_F32_SMALL(false, true);
     else if (trans_a && !trans_b) EMI_F32_SMALL(true, true);
     else EMI_F32_SMALL(true, false);
 #undef EMI_F32_SMALL
-#undef EMI_F32_SMALL_V
     EMI_CHECK_LAUNCH("emi_gemm(fp32 small)");
+    if (part != nullptr)
+      return launch_f32_splitk_reduce(st, part, static_cast<const float*>(R), static_cast<float*>(C), (int)M, (int)N, (int)grid.z, ldr, ldc);
     return EMI_OK;
   }
   return launch_generic<float>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
@@ -2128,6 +1934,10 @@ extern "C" size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t
     const size_t grouped = splits > 1 ? (size_t)count * splits * M * N * sizeof(float) : 0;
     if (grouped > need) need = grouped;
   }
+  if (count >= 2 && count <= kMaxGroup && dtype == EMI_F32 && M > 0 && N > 0 && K > 0) {
+    const size_t grouped = gemm_f32_workspace_bytes(M, N, K, count, sum ? 1 : 0);
+    if (grouped > need) need = grouped;
+  }
   return need;
 }
 
@@ -2185,47 +1995,17 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
       return launch_bf16_grouped<true, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
     }
   }
-  if (dtype == EMI_F32 && count >= 2 && !sum && K > 0 && M > 8 && (M + 31) / 32 <= 65535 && lda >= (trans_a ? M : K) &&
-      ldb >= (trans_b ? K : N) && ldc >= N && (trans_a || lda % 4 == 0) && (!trans_b || ldb % 4 == 0) &&
-      !(generic_splits(M, N, K) > 1 && (int64_t)count * ((M + 63) / 64) * ((N + 63) / 64) < 128)) {
-    bool ok = true, any_r = false, all_r = true;
-    for (int i = 0; i < count && ok; i++)
-      ok = (trans_a || (reinterpret_cast<uintptr_t>(A[i]) & 15) == 0) && (!trans_b || (reinterpret_cast<uintptr_t>(B[i]) & 15) == 0);
-    for (int i = 0; i < count; i++) {
+  if (dtype == EMI_F32 && count >= 2 && K > 0 && M > 8 && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && ldc >= N) {
+    bool any_r = false, all_r = true;
+    for (int i = 0; i < nout; i++) {
       const bool has = R != nullptr && R[i] != nullptr;
       any_r = any_r || has;
       all_r = all_r && has;
     }
-    if (ok && (!any_r || (all_r && ldr >= N))) {
-      // the fp32 kernel, one grid plane per product
-      GemmGroup g{};
-      g.count = count;
-      for (int i = 0; i < count; i++) {
-        g.A[i] = static_cast<const uint16_t*>(A[i]);
-        g.B[i] = static_cast<const uint16_t*>(B[i]);
-        g.R[i] = any_r ? static_cast<const uint16_t*>(R[i]) : nullptr;
-        g.C[i] = static_cast<uint16_t*>(C[i]);
-      }
-      const dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)count);
-#define EMI_F32_GROUPED_V(AKM, BKM, NWV, UV, ONCEV)                                                                        \
-  hipLaunchKernelGGL((gemm_f32_small_kernel<AKM, BKM, true, NWV, UV, ONCEV>), grid, dim3(NWV * 64), 0, st,                 \
-                     static_cast<const float*>(A[0]), static_cast<const float*>(B[0]), static_cast<const float*>(nullptr), \
-                     static_cast<float*>(C[0]), (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, g)
-      const bool few = (int64_t)grid.x * grid.y * grid.z <= 1024;
-#define EMI_F32_GROUPED(AKM, BKM)                                          \
-  do {                                                                     \
-    if (few && K <= 384) EMI_F32_GROUPED_V(AKM, BKM, 4, 12, true);         \
-    else if (few && K <= 768) EMI_F32_GROUPED_V(AKM, BKM, 8, 12, true);    \
-    else EMI_F32_GROUPED_V(AKM, BKM, 4, 4, false);                         \
-  } while (0)
-      if (!trans_a && trans_b) EMI_F32_GROUPED(false, false);
-      else if (!trans_a && !trans_b) EMI_F32_GROUPED(false, true);
-      else if (trans_a && !trans_b) EMI_F32_GROUPED(true, true);
-      else EMI_F32_GROUPED(true, false);
-#undef EMI_F32_GROUPED
-#undef EMI_F32_GROUPED_V
-      EMI_CHECK_LAUNCH("emi_gemm_grouped(fp32)");
-      return EMI_OK;
+    if (!any_r || (all_r && ldr >= N)) {
+      const int rc = launch_f32_gemm(st, count, A, B, any_r ? R : nullptr, C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc,
+                                     trans_a, trans_b, sum ? 1 : 0);
+      if (rc >= 0) return rc;
     }
   }
   // one product after the other; summed: each launch adds onto the result of the one before

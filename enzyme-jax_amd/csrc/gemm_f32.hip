@@ -1,0 +1,391 @@
+// fp32 products on v_mfma_f32_32x32x2_f32, operands streamed global -> LDS.
+//
+//   C[M,N] = op(A) . op(B) [+ R]      fp32 throughout
+//
+// An fp32 matrix instruction keeps its SIMD's matrix core busy for 64 cycles and needs 512 bytes of operands, a quarter
+// of what the LDS delivers in that time to four SIMDs: nothing but the matrix cores has to be the limit, provided that
+// loads are in flight all the time and that every CU has the same share of the work.  So: a ring of NST LDS stages of BK
+// k each, filled by direct-to-LDS loads (16 bytes a lane, no staging registers) NST - 1 stages ahead, one barrier per
+// stage, and three shapes of block between which the launcher chooses by how the tiles divide over the CUs (f32_plan()).
+// Measured, us, against 32 x 32 tiles read straight from global memory and 128 x 128 tiles staged through registers
+// (NT / NN / TN form): 256 x 288 x 288: 8.2 -> 4.8 / 7.5 -> 5.3 / 7.5 -> 4.8; 256 x 288 x 768 12.6 -> 7.5; 2000 x 768 x 768
+// 53 -> 30; 2000 x 768 x 2048 90 -> 59; 2048 x 768 x 2000 (TN) 122 -> 56 (113 TFLOP/s); 300 x 4096 x 11008 441 -> 237;
+// 4096^3 1258 -> 988 (139 TFLOP/s of 157).  What is left on the small ones is the latency of the first loads and the launch.
+#include <type_traits>
+
+#include "emi_device.h"
+
+namespace emi {
+
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
+#define EMI_LDS __attribute__((address_space(3)))
+constexpr uint32_t kOob = 0x80000000u;   // beyond any buffer's num_records: loads return 0
+
+// Several products of one shape in one launch.  sum == 0: C[i] = op(A[i]) . op(B[i]) [+ R[i]];  sum == 1: every product
+// is accumulated into the tile of C[0] (+ R[0]), pair after pair.
+constexpr int kMaxF32Group = 48;
+struct F32Group {
+  const float* A[kMaxF32Group];
+  const float* B[kMaxF32Group];
+  const float* R[kMaxF32Group];
+  float* C[kMaxF32Group];
+  int count, sum;
+};
+struct F32Single {};
+
+// gemm.hip: adds `splits` planes [M, N] (+ R) into C in plane order
+int launch_f32_splitk_reduce(hipStream_t st, const float* part, const float* R, float* C, int M, int N, int splits, int64_t ldr, int64_t ldc);
+
+template <int N> __device__ __forceinline__ void f32_wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+}
+
+// One operand of a block: ROWS rows (of A: rows of C; of B: columns of C) by BK of the contraction per stage.
+// k-contiguous (KM == false, stored [row][k]): LDS rows of BK floats, 16-byte piece c of row r at piece c ^ swz(r), which
+// spreads the 16 rows that one pass of a ds_read_b128 serves over all banks.
+// k-major (KM == true, stored [k][row]): LDS rows of ROWS floats.  A fragment read takes 32 consecutive columns of k-row
+// 8j + t and of k-row 8j + 4 + t; pieces of a row with bit 2 of k set are stored 32 columns across (ROWS >= 64), or
+// such a row takes its neighbour's place (ROWS == 32, two rows per bank line), so that the two do not share banks.
+template <int ROWS, int BK, int NW, bool KM> struct F32Operand {
+  static constexpr int BYTES = ROWS * BK * 4;
+  static constexpr int LOADS = BYTES / 1024 / NW;                 // 1 KiB wave-loads per wavefront and stage
+  static_assert(LOADS >= 1, "a stage is smaller than one pass of the block");
+  static constexpr int CPR = (KM ? ROWS : BK) / 4;                // 16-byte pieces per LDS row
+  static __device__ __forceinline__ int swz(int r) { return CPR == 8 ? ((r >> 1) & 7) : (r & 15); }
+
+  // what this lane's it-th load of a stage fetches: byte offset from the stage's corner of the operand (kOob: outside)
+  // and, k-contiguous, the k of its piece (k-major pieces past the contraction lie past num_records)
+  uint32_t voff[LOADS];
+  int lk[LOADS];
+  __device__ __forceinline__ void init(int wave, int lane, int rows_left, int ld) {
+#pragma unroll
+    for (int it = 0; it < LOADS; it++) {
+      const int slot = (it * NW + wave) * 64 + lane, r = slot / CPR, pc = slot % CPR;
+      if constexpr (KM) {
+        const int k = ROWS == 32 ? r ^ ((r >> 2) & 1) : r;
+        const int col = (ROWS == 32 ? pc : pc ^ (8 * ((k >> 2) & 1))) * 4;
+        lk[it] = 0;
+        voff[it] = col < rows_left ? (uint32_t)(k * ld + col) * 4u : kOob;
+      } else {
+        lk[it] = (pc ^ swz(r)) * 4;
+        voff[it] = r < rows_left ? (uint32_t)(r * ld + lk[it]) * 4u : kOob;
+      }
+    }
+  }
+  // corner: the operand at the block's first row and the stage's first k, of which `left` are left to contract
+  __device__ __forceinline__ void issue(const float* corner, EMI_LDS uint8_t* lds, int wave, int rows, int ld, int left) const {
+    const uint32_t bytes = left <= 0 ? 0u : (uint32_t)(KM ? ((left < BK ? left : BK) - 1) * ld + rows : (rows - 1) * ld + left) * 4u;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(corner), 0, bytes, 0x00020000);
+#pragma unroll
+    for (int it = 0; it < LOADS; it++) {
+      const uint32_t v = KM || lk[it] < left ? voff[it] : kOob;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds + (it * NW + wave) * 1024, 16, v, 0, 0, 0);
+    }
+  }
+  // the four k (8j + 4g .. + 3) of tile row `row` that this lane contracts
+  static __device__ __forceinline__ void frag(const EMI_LDS uint8_t* lds, int row, int g, int j, float (&f)[4]) {
+    if constexpr (KM) {
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const int k = 8 * j + 4 * g + t;
+        const int at = ROWS == 32 ? (k ^ g) * ROWS + row : k * ROWS + (row ^ (32 * g));
+        f[t] = *reinterpret_cast<const EMI_LDS float*>(lds + at * 4);
+      }
+    } else {
+      typedef __attribute__((__vector_size__(4 * sizeof(float)))) float v4;
+      const v4 x = *reinterpret_cast<const EMI_LDS v4*>(lds + row * (BK * 4) + (((2 * j + g) ^ swz(row)) << 4));
+      f[0] = x[0]; f[1] = x[1]; f[2] = x[2]; f[3] = x[3];
+    }
+  }
+};
+
+// WM x WN wavefronts tile the block's BM x BN; WK wavefronts share the k of every stage (chunk j of 8 to wavefront
+// j % WK) and are added in wavefront order at the end.  The contraction index of an instruction is the lane half g:
+// instruction t of chunk j contracts k = 8j + 4g + t, so that a k-contiguous operand is read in 16-byte pieces.
+// part != nullptr: split-K, split z owns the stages [z * steps_per_split, ...) of the contraction (of the whole sum, where
+// products are summed) and leaves its tile in part[z][M][N] for the reduction over splits.
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool AKM, bool BKM, bool GROUPED>
+__global__ __launch_bounds__(WM* WN* WK * 64) void gemm_f32_pipe_kernel(const float* A, const float* B, const float* R, float* C, int M,
+                                                                        int N, int K, int lda, int ldb, int64_t ldr, int64_t ldc,
+                                                                        float* part, int steps_per_split,
+                                                                        std::conditional_t<GROUPED, F32Group, F32Single> grp) {
+  constexpr int NW = WM * WN * WK;
+  constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
+  constexpr int CH = BK / 8 / WK;                                 // 8-wide chunks per wavefront and stage
+  static_assert(WK == 1 || (TM == 1 && TN == 1 && WM == 1 && WN == 1), "wavefronts share k on a single 32 x 32 tile");
+  static_assert(NST >= 2 && CH >= 1, "stages");
+  using OA = F32Operand<BM, BK, NW, AKM>;
+  using OB = F32Operand<BN, BK, NW, BKM>;
+  constexpr int STAGE = OA::BYTES + OB::BYTES;
+  constexpr int LPT = OA::LOADS + OB::LOADS;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+  EMI_LDS uint8_t* smem = (EMI_LDS uint8_t*)smem_raw;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 31, g = lane >> 5;
+  const int wk = WK == 1 ? 0 : wave, wm = WK == 1 ? wave / WN : 0, wn = WK == 1 ? wave % WN : 0;
+
+  // workgroup ids go round the XCDs: give each XCD (own L2) a run of neighbouring tiles; splits and products outermost
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+  const int nb = gridDim.x, per = nb >> 3, rem = nb & 7, xcd = blockIdx.x & 7;
+  const int pid = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  const int outer = pid / tiles, tile = pid - outer * tiles;
+  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+  const int ksteps = (K + BK - 1) / BK;
+  int step0 = 0, nsteps = ksteps;
+  if constexpr (GROUPED) {
+    if (grp.sum) {
+      nsteps *= grp.count;
+    } else {
+      A = grp.A[outer];
+      B = grp.B[outer];
+      R = grp.R[outer];
+      C = grp.C[outer];
+    }
+  }
+  if (part != nullptr) {
+    step0 = outer * steps_per_split;
+    nsteps = nsteps - step0 < steps_per_split ? nsteps - step0 : steps_per_split;
+    part += (int64_t)outer * M * N;
+  }
+  const int rows_a = M - m0 < BM ? M - m0 : BM, rows_b = N - n0 < BN ? N - n0 : BN;
+  OA oa;
+  OB ob;
+  oa.init(wave, lane, rows_a, lda);
+  ob.init(wave, lane, rows_b, ldb);
+  const int64_t a_row = AKM ? m0 : (int64_t)m0 * lda, b_row = BKM ? n0 : (int64_t)n0 * ldb;
+  const int64_t a_k = AKM ? lda : 1, b_k = BKM ? ldb : 1;          // elements per k
+
+  // stages in issue order; past the last one the loads still go out (as zeros) so that the number in flight is constant
+  int at_pair = 0, at_k = step0 * BK, at_slot = 0, to_issue = nsteps;
+  if constexpr (GROUPED) {
+    if (grp.sum) {
+      at_pair = step0 / ksteps;
+      at_k = (step0 - at_pair * ksteps) * BK;
+      A = grp.A[at_pair];
+      B = grp.B[at_pair];
+    }
+  }
+  auto issue = [&]() __attribute__((always_inline)) {
+    const int left = to_issue-- > 0 ? K - at_k : 0;
+    EMI_LDS uint8_t* s = smem + at_slot * STAGE;
+    oa.issue(A + a_row + at_k * a_k, s, wave, rows_a, lda, left);
+    ob.issue(B + b_row + at_k * b_k, s + OA::BYTES, wave, rows_b, ldb, left);
+    at_slot = at_slot + 1 < NST ? at_slot + 1 : 0;
+    at_k += BK;
+    if constexpr (GROUPED) {
+      if (at_k >= K && to_issue > 0) {
+        at_k = 0;
+        at_pair++;
+        A = grp.A[at_pair];
+        B = grp.B[at_pair];
+      }
+    }
+  };
+
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int a = 0; a < TM; a++)
+#pragma unroll
+    for (int b = 0; b < TN; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[a][b][r] = 0.f;
+
+#pragma unroll
+  for (int s = 0; s < NST - 1; s++) issue();
+  int slot = 0;
+  for (int t = 0; t < nsteps; t++) {
+    f32_wait_vmcnt<(NST - 2) * LPT>();                     // this stage has landed
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();                          // everyone's part of it, and the stage before is free again
+    __builtin_amdgcn_sched_barrier(0);
+    issue();
+    const EMI_LDS uint8_t* sa = smem + slot * STAGE;
+    const EMI_LDS uint8_t* sb = sa + OA::BYTES;
+    slot = slot + 1 < NST ? slot + 1 : 0;
+    float fa[2][TM][4], fb[2][TN][4];
+    auto read = [&](int c, float (&pa)[TM][4], float (&pb)[TN][4]) __attribute__((always_inline)) {
+      const int j = c * WK + wk;
+#pragma unroll
+      for (int a = 0; a < TM; a++) OA::frag(sa, wm * (BM / WM) + a * 32 + i, g, j, pa[a]);
+#pragma unroll
+      for (int b = 0; b < TN; b++) OB::frag(sb, wn * (BN / WN) + b * 32 + i, g, j, pb[b]);
+    };
+    read(0, fa[0], fb[0]);
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+      if (c + 1 < CH) read(c + 1, fa[(c + 1) & 1], fb[(c + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);                   // the next chunk's reads stay ahead of this one's products
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+          for (int b = 0; b < TN; b++)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[c & 1][a][q], fb[c & 1][b][q], acc[a][b], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32 x 32 tile
+  auto put = [&](int row, int col, float v) __attribute__((always_inline)) {
+    if (row < M && col < N) {
+      if (part != nullptr) {
+        part[(int64_t)row * N + col] = v;
+      } else {
+        if (R != nullptr) v += R[(int64_t)row * ldr + col];
+        C[(int64_t)row * ldc + col] = v;
+      }
+    }
+  };
+  f32_wait_vmcnt<0>();                                     // the zero-filled loads past the end
+  if constexpr (WK > 1) {
+    __syncthreads();
+    EMI_LDS float* red = (EMI_LDS float*)smem;             // [WK][32][32 + 1]
+#pragma unroll
+    for (int r = 0; r < 16; r++) red[(wk * 32 + (r >> 2) * 8 + g * 4 + (r & 3)) * 33 + i] = acc[0][0][r];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 1024 / (NW * 64); e++) {
+      const int at = e * NW * 64 + threadIdx.x, row = at >> 5, col = at & 31;
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < WK; w++) v += red[(w * 32 + row) * 33 + col];
+      put(m0 + row, n0 + col, v);
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          put(m0 + wm * (BM / WM) + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3), n0 + wn * (BN / WN) + b * 32 + i, acc[a][b][r]);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+
+struct F32Call {
+  const float *A, *B, *R;
+  float* C;
+  int M, N, K, lda, ldb;
+  int64_t ldr, ldc;
+  float* part;
+  int splits;
+  const F32Group* grp;       // nullptr: the single product of A and B
+};
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool AKM, bool BKM, bool GROUPED>
+static int launch_f32_one(hipStream_t st, const F32Call& c) {
+  auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, GROUPED>;
+  constexpr int smem = NST * (BM + BN) * BK * 4;
+  static_assert(WK == 1 || smem >= WK * 32 * 33 * 4, "the wavefronts' tiles meet in the ring");
+  static bool configured = false;   // idempotent; a race only repeats the call
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+    configured = true;
+  }
+  const int steps = ((c.K + BK - 1) / BK) * (GROUPED && c.grp->sum ? c.grp->count : 1);
+  const int sps = (steps + c.splits - 1) / c.splits, nz = (steps + sps - 1) / sps;
+  const int outer = GROUPED && !c.grp->sum ? c.grp->count : nz;
+  const int tiles = ((c.M + BM - 1) / BM) * ((c.N + BN - 1) / BN);
+  float* part = outer == nz && nz > 1 ? c.part : nullptr;
+  if constexpr (GROUPED)
+    hipLaunchKernelGGL(kern, dim3(tiles * outer), dim3(WM * WN * WK * 64), smem, st, c.A, c.B, c.R, c.C, c.M, c.N, c.K, c.lda, c.ldb,
+                       c.ldr, c.ldc, part, sps, *c.grp);
+  else
+    hipLaunchKernelGGL(kern, dim3(tiles * outer), dim3(WM * WN * WK * 64), smem, st, c.A, c.B, c.R, c.C, c.M, c.N, c.K, c.lda, c.ldb,
+                       c.ldr, c.ldc, part, sps, F32Single{});
+  EMI_CHECK_LAUNCH("emi_gemm(fp32)");
+  if (part != nullptr) return launch_f32_splitk_reduce(st, part, c.R, c.C, c.M, c.N, nz, c.ldr, c.ldc);
+  return EMI_OK;
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST>
+static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int trans_b) {
+#define EMI_F32_PIPE(AKM, BKM)                                                                          \
+  return c.grp != nullptr ? launch_f32_one<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, true>(st, c)          \
+                          : launch_f32_one<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, false>(st, c)
+  if (!trans_a && trans_b) EMI_F32_PIPE(false, false);
+  if (!trans_a && !trans_b) EMI_F32_PIPE(false, true);
+  if (trans_a && !trans_b) EMI_F32_PIPE(true, true);
+  EMI_F32_PIPE(true, false);
+#undef EMI_F32_PIPE
+}
+
+// Which block and how many splits.  The estimate is of the CU with the most blocks, in microseconds, with the rates that
+// each block shape was measured at: a stage of 32 k of a 128 x 128 tile takes 2.0 alone on a CU and 1.92 next to others
+// (139 TFLOP/s on 4096^3; the matrix cores' own limit is 157), a 64 x 64 tile 0.72 alone, 1.13 for two blocks and 0.54 a
+// block from four on, a stage of 64 k of a 32 x 32 tile whose wavefronts share k 0.42 alone, 0.36 a block from three on.
+// The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s).
+struct F32Plan {
+  int config, splits;
+};
+static F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum) {
+  struct Shape { int tile, bk; double fixed, rate[4]; };              // rate[b - 1]: per stage, b blocks on the CU; the last one per block
+  static const Shape shapes[3] = {{128, 32, 4.0, {2.0, 3.84, 5.76, 1.92}}, {64, 32, 3.0, {0.72, 1.13, 1.60, 0.54}}, {32, 64, 2.5, {0.42, 0.72, 1.08, 0.36}}};
+  F32Plan best{2, 1};
+  double least = 1e30;
+  for (int c = 0; c < 3; c++) {
+    const Shape& s = shapes[c];
+    const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
+    const int64_t blocks = (M + s.tile - 1) / s.tile * ((N + s.tile - 1) / s.tile) * (sum ? 1 : count);
+    if (blocks > 0x3fffffff) continue;
+    for (int64_t z = 1; z <= 64 && (z == 1 || (steps >= 4 * z && (sum || count == 1))); z++) {
+      const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
+      const double t = s.fixed + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
+      if (t < least) {
+        least = t;
+        best = F32Plan{c, (int)z};
+      }
+    }
+  }
+  return best;
+}
+
+size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum) {
+  const int z = f32_plan(M, N, K, count, sum).splits;
+  return z > 1 ? (size_t)z * M * N * sizeof(float) : 0;
+}
+
+// C[i] = op(A[i]) . op(B[i]) [+ R[i]] for i < count, or with `sum` the one sum of the products (+ R[0]).  Returns -1 for
+// operands that the kernels' 16-byte pieces do not fit (the caller has other kernels for those).
+int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
+                    void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
+                    int64_t ldc, int trans_a, int trans_b, int sum) {
+  // pieces are four elements along the stored rows; a stage's panel of an operand is addressed with 31 bits
+  if (K <= 0 || count > kMaxF32Group || lda % 4 || ldb % 4 || (trans_a ? M : K) % 4 || (trans_b ? K : N) % 4 ||
+      128 * lda + K >= 0x1fffffff || 128 * ldb + K >= 0x1fffffff)
+    return -1;
+  F32Group g{};
+  for (int i = 0; i < count; i++) {
+    if ((reinterpret_cast<uintptr_t>(A[i]) | reinterpret_cast<uintptr_t>(B[i])) & 15) return -1;
+    g.A[i] = static_cast<const float*>(A[i]);
+    g.B[i] = static_cast<const float*>(B[i]);
+  }
+  for (int i = 0; i < (sum ? 1 : count); i++) {
+    g.R[i] = R != nullptr ? static_cast<const float*>(R[i]) : nullptr;
+    g.C[i] = static_cast<float*>(C[i]);
+  }
+  g.count = count;
+  g.sum = sum;
+  F32Plan p = f32_plan(M, N, K, count, sum);
+  if (p.splits > 1 && (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
+                       workspace_bytes < (size_t)p.splits * M * N * sizeof(float)))
+    p.splits = 1;
+  const F32Call c{g.A[0], g.B[0], g.R[0], g.C[0], (int)M, (int)N, (int)K, (int)lda, (int)ldb, ldr, ldc, static_cast<float*>(workspace),
+                  p.splits, count > 1 ? &g : nullptr};
+  switch (p.config) {
+    case 0: return launch_f32_shape<128, 128, 4, 2, 1, 32, 2>(st, c, trans_a, trans_b);
+    case 1: return launch_f32_shape<64, 64, 2, 2, 1, 32, 2>(st, c, trans_a, trans_b);
+    default: return launch_f32_shape<32, 32, 1, 1, 8, 64, 5>(st, c, trans_a, trans_b);
+  }
+}
+
+}  // namespace emi

@@ -1,0 +1,47 @@
+"""The fp32 GEMM kernels at the sizes where their tiles, stages and splits end: every block shape, each layout, one
+product, a group of independent ones and a group summed into one, against float64 products.  An fp32 sum of n products in
+any order is within n * 2^-24 * sum |a b| of the exact one, to first order (its roundings, one per term and one per
+product, are each at most half a unit in the last place of a partial sum); twice that is allowed."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, ref, bound, what):
+    err = np.abs(host(got) - ref)
+    assert np.all(err <= bound), "%s: worst error / bound %.2f" % (what, float(np.max(err / bound)))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,count", [
+    (4, 4, 4, 2),            # less than one piece of every stage
+    (32, 32, 64, 3),         # exactly one 32-tile and one stage
+    (36, 28, 68, 3),         # a ragged row of tiles, one piece past a stage
+    (100, 512, 516, 3),      # 32-tiles, ragged rows
+    (12, 20, 20004, 2),      # a single tile: splits of a long contraction, ragged last stage
+    (704, 2812, 1028, 2),    # 64-tiles, ragged columns
+    (1996, 772, 2052, 2),    # 64-tiles, splits; summed: splits that straddle the products
+    (2052, 2044, 68, 2),     # 128-tiles, ragged both ways
+])
+def test_f32_tiles_stages_and_splits(ta, tb, M, N, K, count):
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + 3 * N + 7 * K + 2 * ta + tb)
+    As, Ars = zip(*[dev(rng.standard_normal((K, M) if ta else (M, K)), "f32") for _ in range(count)])
+    Bs, Brs = zip(*[dev(rng.standard_normal((N, K) if tb else (K, N)), "f32") for _ in range(count)])
+    Rs, Rrs = zip(*[dev(rng.standard_normal((M, N)), "f32") for _ in range(count)])
+    mm = lambda f: [f(a.T if ta else a) @ f(b.T if tb else b) for a, b in zip(Ars, Brs)]
+    prods, mags = mm(lambda t: t), mm(np.abs)
+    eps = 2.0 ** -23
+    bounds = [(K + 2) * eps * (m + np.abs(r)) for m, r in zip(mags, Rrs)]
+    _check(ops.gemm(As[0], Bs[0], bool(ta), bool(tb)), prods[0], bounds[0], "one product")
+    _check(ops.gemm(As[0], Bs[0], bool(ta), bool(tb), Rs[0]), prods[0] + Rrs[0], bounds[0], "one product + residual")
+    for o, p, r, b in zip(ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), list(Rs)), prods, Rrs, bounds):
+        _check(o, p + r, b, "group + residual")
+    total = ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), [Rs[0]], sum_into_one=True)
+    _check(total, sum(prods) + Rrs[0], (count * K + 2) * eps * (sum(mags) + np.abs(Rrs[0])), "summed + residual")
+    again = ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), [Rs[0]], sum_into_one=True)
+    assert torch.equal(total, again)          # fixed order of summation
