@@ -127,12 +127,15 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_f32_pipe_kernel(const fl
   const int i = lane & 31, g = lane >> 5;
   const int wk = WK == 1 ? 0 : wave, wm = WK == 1 ? wave / WN : 0, wn = WK == 1 ? wave % WN : 0;
 
-  // workgroup ids go round the XCDs: give each XCD (own L2) a run of neighbouring tiles; splits and products outermost
+  // workgroup ids go round the XCDs: give each XCD (own L2) a run of neighbouring tiles, eight tile rows deep, so that it
+  // reads a few panels of both operands many times; splits and products outermost
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN, tiles = tiles_m * tiles_n;
   const int nb = gridDim.x, per = nb >> 3, rem = nb & 7, xcd = blockIdx.x & 7;
   const int pid = xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
   const int outer = pid / tiles, tile = pid - outer * tiles;
-  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+  const int first_m = tile / (8 * tiles_n) * 8, deep = tiles_m - first_m < 8 ? tiles_m - first_m : 8;
+  const int in_group = tile - first_m * tiles_n;
+  const int m0 = (first_m + in_group % deep) * BM, n0 = in_group / deep * BN;
   const int ksteps = (K + BK - 1) / BK;
   int step0 = 0, nsteps = ksteps;
   if constexpr (GROUPED) {
@@ -323,7 +326,8 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 // each block shape was measured at: a stage of 32 k of a 128 x 128 tile takes 2.0 alone on a CU and 1.92 next to others
 // (139 TFLOP/s on 4096^3; the matrix cores' own limit is 157), a 64 x 64 tile 0.72 alone, 1.13 for two blocks and 0.54 a
 // block from four on, a stage of 64 k of a 32 x 32 tile whose wavefronts share k 0.42 alone, 0.36 a block from three on.
-// The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s).
+// The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s); results over 4 M elements, whose planes
+// leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split.
 struct F32Plan {
   int config, splits;
 };
@@ -331,13 +335,14 @@ static F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum) {
   struct Shape { int tile, bk; double fixed, rate[4]; };              // rate[b - 1]: per stage, b blocks on the CU; the last one per block
   static const Shape shapes[3] = {{128, 32, 4.0, {2.0, 3.84, 5.76, 1.92}}, {64, 32, 3.0, {0.72, 1.13, 1.60, 0.54}}, {32, 64, 2.5, {0.42, 0.72, 1.08, 0.36}}};
   F32Plan best{2, 1};
+  const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && M > 8 && K > 8;
   double least = 1e30;
   for (int c = 0; c < 3; c++) {
     const Shape& s = shapes[c];
     const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
     const int64_t blocks = (M + s.tile - 1) / s.tile * ((N + s.tile - 1) / s.tile) * (sum ? 1 : count);
     if (blocks > 0x3fffffff) continue;
-    for (int64_t z = 1; z <= 64 && (z == 1 || (steps >= 4 * z && (sum || count == 1))); z++) {
+    for (int64_t z = 1; z <= 64 && (z == 1 || (may_split && steps >= 4 * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
       const double t = s.fixed + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
