@@ -17,6 +17,7 @@
 #include <utility>
 
 #include "emi_device.h"
+#include "gemm_plan.h"
 
 namespace emi {
 
@@ -1485,8 +1486,26 @@ static int grouped_splits(int64_t M, int64_t N, int64_t K, int count) {
   return (int)(s < 2 ? 1 : (s > 64 ? 64 : s));
 }
 
-// The 128x128 kernel on a group of products (GemmGroup): one launch, count times the tiles (or, summed, count times
-// the contraction).
+template <bool AK, bool BKM>
+static int launch_bf16_pingpong_grouped(hipStream_t st, const GemmGroup& g, int M, int N, int K, int lda, int ldb, int ldr, int ldc,
+                                        uint32_t a_bytes, uint32_t b_bytes, int vec_ok) {
+  constexpr int smem = 2 * 65536;
+  static bool configured = false;   // idempotent; a race only repeats the call
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_pingpong_kernel<AK, BKM, true>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm_grouped: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+    configured = true;
+  }
+  const int tiles = ((M + 255) / 256) * ((N + 255) / 256);
+  hipLaunchKernelGGL((gemm_bf16_pingpong_kernel<AK, BKM, true>), dim3(tiles * g.count), dim3(512), smem, st, g.A[0], g.B[0], g.R[0],
+                     g.C[0], M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok, g);
+  EMI_CHECK_LAUNCH("emi_gemm_grouped(256-tiles)");
+  return EMI_OK;
+}
+
+// Products with a k-major A: the 128x128 kernel on a group of them (GemmGroup): one launch, count times the tiles (or,
+// summed, count times the contraction).
 template <bool AK, bool BKM>
 static int launch_bf16_grouped(hipStream_t st, const GemmGroup& g, int M, int N, int K, int lda, int ldb, int ldr, int ldc,
                                uint32_t a_bytes, uint32_t b_bytes, void* workspace, size_t workspace_bytes) {
@@ -1505,23 +1524,11 @@ static int launch_bf16_grouped(hipStream_t st, const GemmGroup& g, int M, int N,
   }
   const int big_tiles = ((M + 255) / 256) * ((N + 255) / 256);
   const int64_t group_tiles = (int64_t)big_tiles * g.count, rounds = (group_tiles + 255) / 256;
-  if (!g.sum && group_tiles >= 192 && (4 * group_tiles >= 3 * rounds * 256 || K >= 4096)) {
-    // enough 256x256 tiles over the whole group to fill the chip: the ping-pong kernel, product-major.  With a short
-    // contraction a last round that leaves most CUs idle costs more than the larger tile gains (3 x [8192, 768] x 768:
-    // 288 tiles, 48 us against 43 us on 128x128 tiles); with a long one it does not (12 x [768, 2048] x 8192: 351 vs 462 us).
-    constexpr int smem_pp = 2 * 65536;
-    static bool configured_pp = false;
-    if (!configured_pp) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_pingpong_kernel<AK, BKM, true>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, smem_pp);
-      if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm_grouped: cannot reserve %d bytes of LDS: %s", smem_pp, hipGetErrorString(e));
-      configured_pp = true;
-    }
-    hipLaunchKernelGGL((gemm_bf16_pingpong_kernel<AK, BKM, true>), dim3(big_tiles * g.count), dim3(512), smem_pp, st, g.A[0], g.B[0],
-                       g.R[0], g.C[0], M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok, g);
-    EMI_CHECK_LAUNCH("emi_gemm_grouped(256-tiles)");
-    return EMI_OK;
-  }
+  // enough 256x256 tiles over the whole group to fill the chip: the ping-pong kernel, product-major.  With a short
+  // contraction a last round that leaves most CUs idle costs more than the larger tile gains; with a long one it does not
+  // (12 x [768, 2048] x 8192: 351 vs 462 us).
+  if (!g.sum && group_tiles >= 192 && (4 * group_tiles >= 3 * rounds * 256 || K >= 4096))
+    return launch_bf16_pingpong_grouped<AK, BKM>(st, g, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok);
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   const int splits = g.sum ? 1 : grouped_splits(M, N, K, g.count);
   if (splits > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
@@ -1635,14 +1642,14 @@ static int launch_bf16_rope(hipStream_t st, const void* A, const void* B, void* 
   return EMI_OK;
 }
 
-// Split-K on the 256x256 ping-pong kernel: k-contiguous products with too few 256-tiles for that kernel, too many
-// 128-tiles for bf16_splits and a long contraction (dX of the classifier of a small model, [8192, 32000] x [32000, 768]:
-// 96 tiles of 256, 384 of 128).  The 128-tile kernel runs those at 0.75 PFLOP/s (two blocks on half the CUs, one on the
-// others); four splits are 384 ping-pong blocks at 1.1 PFLOP/s plus the reduction of 4 x M x N fp32 partials.
+// Split-K on the 256x256 ping-pong kernel for results of more than 4 M elements (bf16_plan splits the smaller ones):
+// k-contiguous products with too few 256-tiles to fill the chip and a long contraction (dX of the classifier of a small
+// model, [8192, 32000] x [32000, 768], is 96 tiles: 128-tiles run it at 0.75 PFLOP/s, four splits are 384 ping-pong blocks
+// at 1.1 PFLOP/s plus the reduction of 4 x M x N fp32 partials).
 static int pingpong_splits(int64_t M, int64_t N, int64_t K, bool k_contiguous) {
-  if (!k_contiguous || K < 8192) return 1;
-  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256), t128 = ((M + 127) / 128) * ((N + 127) / 128);
-  if (big >= 192 || t128 <= 128 || big > 128) return 1;
+  if (!k_contiguous || K < 8192 || M * N <= (4 << 20)) return 1;
+  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
+  if (big > 128) return 1;
   int64_t s = (320 + big - 1) / big;
   if (s > 8) s = 8;
   while (s > 1 && K / s < 2048) s--;
@@ -1683,26 +1690,43 @@ static int bf16_splits(int64_t M, int64_t N, int64_t K) {
   return (int)(s < 2 ? 1 : (s > 64 ? 64 : s));
 }
 
-template <bool AK, bool BKM>
-static int launch_bf16_layout(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K,
-                              int lda, int ldb, int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, void* workspace,
-                              size_t workspace_bytes) {
+static bool workspace_holds(const void* workspace, size_t workspace_bytes, int splits, int64_t M, int64_t N) {
+  return workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+         workspace_bytes >= (size_t)splits * M * N * sizeof(float);
+}
+
+// A k-major (the weight gradients): 256x256 tiles (the ping-pong kernel) when they fill the chip, else 128x128.
+template <bool BKM>
+static int launch_bf16_kmajor(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K, int lda, int ldb,
+                              int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, void* workspace, size_t workspace_bytes) {
   const int splits = bf16_splits(M, N, K);
-  if (splits > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
-      workspace_bytes >= (size_t)splits * M * N * sizeof(float))
-    return launch_bf16<128, 128, 64, 2, 2, 2, AK, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes,
-                                                      static_cast<float*>(workspace), splits);
-  if constexpr (!AK && !BKM) {
-    const int pps = pingpong_splits(M, N, K, true);
-    if (pps > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
-        workspace_bytes >= (size_t)pps * M * N * sizeof(float))
-      return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes,
-                                         static_cast<float*>(workspace), pps);
-  }
-  // 256x256 tiles (the ping-pong kernel) when they fill the chip, else 128x128.
+  if (splits > 1 && workspace_holds(workspace, workspace_bytes, splits, M, N))
+    return launch_bf16<128, 128, 64, 2, 2, 2, true, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes,
+                                                         static_cast<float*>(workspace), splits);
   const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-  if (big_tiles >= 192) return launch_bf16_pingpong<AK, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
-  return launch_bf16<128, 128, 64, 2, 2, 2, AK, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
+  if (big_tiles >= 192) return launch_bf16_pingpong<true, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
+  return launch_bf16<128, 128, 64, 2, 2, 2, true, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
+}
+
+// A k-contiguous: the ping-pong kernel or one of the shapes of gemm_bf16_pipe.hip, with or without splits of K.
+static int launch_bf16_kcontig(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K, int lda, int ldb,
+                               int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, int trans_b, void* workspace,
+                               size_t workspace_bytes) {
+  const int pps = pingpong_splits(M, N, K, trans_b);
+  if (pps > 1 && workspace_holds(workspace, workspace_bytes, pps, M, N))
+    return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, static_cast<float*>(workspace), pps);
+  Bf16Plan plan = bf16_plan(M, N, K, 1, 0, trans_b);
+  if (plan.splits > 1 && !workspace_holds(workspace, workspace_bytes, plan.splits, M, N)) plan.splits = 1;
+  float* part = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
+  if (plan.shape == 0) {
+    if (part != nullptr)
+      return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, part, plan.splits);
+    return trans_b ? launch_bf16_pingpong<false, false>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes)
+                   : launch_bf16_pingpong<false, true>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
+  }
+  const int vec_ok = (reinterpret_cast<uintptr_t>(C) & 15) == 0 && ldc % 8 == 0 &&
+                     (R == nullptr || ((reinterpret_cast<uintptr_t>(R) & 15) == 0 && ldr % 8 == 0));
+  return launch_bf16_pipe(st, plan, 1, &A, &B, &R, &C, part, M, N, K, lda, ldb, ldr, ldc, vec_ok, trans_b, 0);
 }
 
 template <typename T>
@@ -1738,7 +1762,13 @@ static int launch_generic(hipStream_t st, const void* A, const void* B, const vo
   return EMI_OK;
 }
 
-// gemm_f32.hip adds its planes with the same kernel
+// gemm_f32.hip and gemm_bf16_pipe.hip add their planes with the same kernel
+int launch_bf16_splitk_reduce(hipStream_t st, const float* part, const uint16_t* R, uint16_t* C, int M, int N, int splits, int64_t ldr,
+                              int64_t ldc) {
+  launch_splitk_reduce<bf16>(st, part, R, C, M, N, splits, ldr, ldc);
+  EMI_CHECK_LAUNCH("emi_gemm(split-K reduce)");
+  return EMI_OK;
+}
 int launch_f32_splitk_reduce(hipStream_t st, const float* part, const float* R, float* C, int M, int N, int splits, int64_t ldr,
                              int64_t ldc) {
   launch_splitk_reduce<float>(st, part, R, C, M, N, splits, ldr, ldc);
@@ -1770,8 +1800,11 @@ extern "C" size_t emi_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
   // few tiles and a long contraction: split-K partials (the larger of what the fp32 / odd-shape path and the
   // 128x128 bf16 kernel would use, since alignment decides between them at launch time)
   int splits = generic_splits(M, N, K);
-  if (dtype == EMI_BF16 && bf16_splits(M, N, K) > splits) splits = bf16_splits(M, N, K);
-  if (dtype == EMI_BF16 && pingpong_splits(M, N, K, !trans_a && trans_b) > splits) splits = pingpong_splits(M, N, K, true);
+  if (dtype == EMI_BF16) {
+    int s = trans_a ? bf16_splits(M, N, K) : pingpong_splits(M, N, K, trans_b);
+    if (!trans_a && s == 1) s = bf16_plan(M, N, K, 1, 0, trans_b).splits;
+    if (s > splits) splits = s;
+  }
   const size_t need = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
   const size_t f32 = dtype == EMI_F32 ? gemm_f32_workspace_bytes(M, N, K, 1, 0) : 0;
   return f32 > need ? f32 : need;
@@ -1814,13 +1847,11 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
     if (fast) {
       const int m = (int)M, n = (int)N, k = (int)K;
       const uint32_t ab = (uint32_t)a_bytes, bb = (uint32_t)b_bytes;
-      if (!trans_a && trans_b)
-        return launch_bf16_layout<false, false>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
-      if (!trans_a && !trans_b)
-        return launch_bf16_layout<false, true>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
-      if (trans_a && !trans_b)
-        return launch_bf16_layout<true, true>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
-      return launch_bf16_layout<true, false>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
+      if (!trans_a)
+        return launch_bf16_kcontig(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, trans_b, workspace, workspace_bytes);
+      if (!trans_b)
+        return launch_bf16_kmajor<true>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
+      return launch_bf16_kmajor<false>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
     }
     return launch_generic<bf16>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
   }
@@ -1929,9 +1960,9 @@ extern "C" int emi_gemm_rope(emi_stream_t stream, const void* X, const void* W, 
 extern "C" size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, int sum,
                                                     int dtype) {
   size_t need = emi_gemm_workspace_bytes(M, N, K, trans_a, trans_b, dtype);          // the one-by-one fallback
-  if (count >= 2 && count <= kMaxGroup && !sum && dtype == EMI_BF16 && M > 0 && N > 0 && K > 0) {
-    const int splits = grouped_splits(M, N, K, count);
-    const size_t grouped = splits > 1 ? (size_t)count * splits * M * N * sizeof(float) : 0;
+  if (count >= 2 && count <= kMaxGroup && dtype == EMI_BF16 && M > 0 && N > 0 && K > 0) {
+    const int splits = trans_a ? (sum ? 1 : count * grouped_splits(M, N, K, count)) : bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b).splits;
+    const size_t grouped = splits > (trans_a && !sum ? count : 1) ? (size_t)splits * M * N * sizeof(float) : 0;
     if (grouped > need) need = grouped;
   }
   if (count >= 2 && count <= kMaxGroup && dtype == EMI_F32 && M > 0 && N > 0 && K > 0) {
@@ -1986,10 +2017,17 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
       }
       const int m = (int)M, n = (int)N, k = (int)K;
       const uint32_t ab = (uint32_t)a_bytes, bb = (uint32_t)b_bytes;
-      if (!trans_a && trans_b)
-        return launch_bf16_grouped<false, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
-      if (!trans_a && !trans_b)
-        return launch_bf16_grouped<false, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
+      if (!trans_a) {
+        int vec_ok = ldc % 8 == 0 && ldr % 8 == 0;
+        for (int i = 0; i < nout; i++) vec_ok = vec_ok && al16(C[i]) && al16(g.R[i]);
+        Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b);
+        if (plan.splits > 1 && !workspace_holds(workspace, workspace_bytes, plan.splits, M, N)) plan.splits = 1;
+        if (plan.shape == 0)
+          return trans_b ? launch_bf16_pingpong_grouped<false, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok)
+                         : launch_bf16_pingpong_grouped<false, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok);
+        return launch_bf16_pipe(st, plan, count, A, B, any_r ? R : nullptr, C, plan.splits > 1 ? static_cast<float*>(workspace) : nullptr, m,
+                                n, k, (int)lda, (int)ldb, ldr, ldc, vec_ok, trans_b, sum ? 1 : 0);
+      }
       if (trans_a && !trans_b)
         return launch_bf16_grouped<true, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
       return launch_bf16_grouped<true, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);

@@ -139,7 +139,7 @@ int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, const void* R
  *   sum == 0:  C[i] = op(A[i]) . op(B[i]) [+ R[i]]            (entries may repeat: one X against three weights)
  *   sum == 1:  C[0] = sum_i op(A[i]) . op(B[i]) [+ R[0]]      (products added in index order)
  * Shapes, leading dimensions and flags as for emi_gemm, the same for every product.  Small aligned bf16 products run
- * as one launch of the 128x128 kernel; anything else runs as `count` emi_gemm_ws calls with the same results up to the
+ * as one launch; anything else runs as `count` emi_gemm_ws calls with the same results up to the
  * rounding of the intermediate sums (sum == 1 then rounds C[0] to its type between products).  The workspace (size
  * from emi_gemm_grouped_workspace_bytes, may be null) holds split-K partials. */
 #define EMI_GEMM_GROUP_MAX 48

@@ -1,0 +1,48 @@
+"""The bf16 GEMM's block shapes for few tokens and narrow results, at the sizes where their tiles, stages and splits end:
+one product, a group of independent ones and a group summed into one, B k-contiguous and k-major, against float64 products
+of the stored values.  The result is an fp32 sum rounded once to bf16: half a unit in the last place of the result (2^-9
+relative) plus the roundings of the sum, at most n * 2^-24 * sum |a b| to first order; twice that sum is allowed."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, ref, mag, n, what):
+    bound = 2.0 ** -8 * np.abs(ref) + (n + 2) * 2.0 ** -23 * mag
+    err = np.abs(host(got) - ref)
+    assert np.all(err <= bound), "%s: worst error / bound %.2f" % (what, float(np.max(err / bound)))
+
+
+@pytest.mark.parametrize("tb", [1, 0])
+@pytest.mark.parametrize("M,N,K,count", [
+    (9, 8, 8, 2),             # less than one piece of every stage
+    (33, 24, 264, 3),         # 32-tiles whose wavefronts share k (k-contiguous B), one piece past a stage
+    (64, 768, 768, 3),        # exact 32-tiles
+    (40, 104, 8200, 2),       # few tiles, long contraction: splits, a ragged last stage
+    (300, 1400, 520, 2),      # 64-tiles, ragged rows and columns
+    (777, 2040, 776, 2),      # 128 x 64 tiles, ragged
+    (1000, 4088, 520, 2),     # 128-tiles, three stages
+    (3000, 1032, 328, 2),     # 128-tiles, two to a CU; summed: one pass over both
+    (600, 2056, 4104, 2),     # splits; summed: splits that straddle the products
+    (300, 1000, 16392, 2),    # 256-tiles with splits (k-contiguous B)
+])
+def test_bf16_tiles_stages_and_splits(tb, M, N, K, count):
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + 3 * N + 7 * K + tb)
+    As, Ars = zip(*[dev(rng.standard_normal((M, K)), "bf16") for _ in range(count)])
+    Bs, Brs = zip(*[dev(rng.standard_normal((N, K) if tb else (K, N)), "bf16") for _ in range(count)])
+    Rs, Rrs = zip(*[dev(rng.standard_normal((M, N)), "bf16") for _ in range(count)])
+    mm = lambda f: [f(a) @ f(b.T if tb else b) for a, b in zip(Ars, Brs)]
+    prods, mags = mm(lambda t: t), mm(np.abs)
+    _check(ops.gemm(As[0], Bs[0], False, bool(tb)), prods[0], mags[0], K, "one product")
+    _check(ops.gemm(As[0], Bs[0], False, bool(tb), Rs[0]), prods[0] + Rrs[0], mags[0] + np.abs(Rrs[0]), K, "one product + residual")
+    for o, p, r, m in zip(ops.gemm_grouped(list(As), list(Bs), False, bool(tb), list(Rs)), prods, Rrs, mags):
+        _check(o, p + r, m + np.abs(r), K, "group + residual")
+    total = ops.gemm_grouped(list(As), list(Bs), False, bool(tb), [Rs[0]], sum_into_one=True)
+    _check(total, sum(prods) + Rrs[0], sum(mags) + np.abs(Rrs[0]), count * K, "summed + residual")
+    again = ops.gemm_grouped(list(As), list(Bs), False, bool(tb), [Rs[0]], sum_into_one=True)
+    assert torch.equal(total, again)          # fixed order of summation
