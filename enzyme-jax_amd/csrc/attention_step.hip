@@ -61,7 +61,17 @@ template <typename T, bool VEC> struct Elems {   // VEC: 16-byte chunks; else si
 struct StepShape {
   int heads, seq_kv, head_dim;
   int64_t q_sb, q_sh, kv_sb, kv_sh, kv_ss;
+  int kpb = kKeysPerBlock;                       // keys per block
+  // the whole-step path (llama_step.hip): the last key, the token's own, lies outside the cache, in rows of its own
+  const void *k_tail = nullptr, *v_tail = nullptr;
+  void *dk_tail = nullptr, *dv_tail = nullptr;
 };
+
+// Row s of a head's cache (base: the head's first row), or the token's own row (tail: its row of all heads; off: the
+// head's columns in it).
+template <typename T> __device__ __forceinline__ T* kv_row(T* base, T* tail, int64_t off, int s, const StepShape& sh) {
+  return tail != nullptr && s == sh.seq_kv - 1 ? tail + off : base + (int64_t)s * sh.kv_ss;
+}
 
 __device__ __forceinline__ float sum16(float v) {          // over the 16 lanes that share a key
   v += __shfl_xor(v, 1, kWave);
@@ -121,21 +131,22 @@ __device__ __forceinline__ void reduce_keys(float (&acc)[MAXC][NE], int nch, flo
 // lane keeps 16 / NCH (at least 2) keys in flight.
 template <typename T, bool VEC, int NCH>
 __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict__ q, const T* __restrict__ k,
-                                                            const T* __restrict__ v, float* __restrict__ part, StepShape sh,
-                                                            float scale) {
+                                                            const T* __restrict__ v, float* __restrict__ part, T* __restrict__ o,
+                                                            float* __restrict__ lse, StepShape sh, float scale) {
   constexpr int NE = Elems<T, VEC>::N, MAXC = NCH, kUnroll = NCH >= 8 ? 2 : 16 / NCH;
   __shared__ float scores[kKeysPerBlock];
   __shared__ float scratch[4];
   __shared__ float red[kRedFloats];
   const int bh = blockIdx.y, b = bh / sh.heads, h = bh % sh.heads;
-  const int s0 = blockIdx.x * kKeysPerBlock;
-  const int s1 = s0 + kKeysPerBlock < sh.seq_kv ? s0 + kKeysPerBlock : sh.seq_kv;
+  const int s0 = blockIdx.x * sh.kpb;
+  const int s1 = s0 + sh.kpb < sh.seq_kv ? s0 + sh.kpb : sh.seq_kv;
   const int l16 = threadIdx.x & 15, slot = threadIdx.x >> 4;       // 16 key slots per block
   const int nchunks = sh.head_dim / NE;                            // chunks per row
   const int nch = (nchunks - l16 + 15) / 16;                       // chunks of this lane: l16, l16 + 16, ...
   const T* qrow = q + b * sh.q_sb + h * sh.q_sh;
   const T* kbase = k + b * sh.kv_sb + h * sh.kv_sh;
   const T* vbase = v + b * sh.kv_sb + h * sh.kv_sh;
+  const T *ktail = static_cast<const T*>(sh.k_tail), *vtail = static_cast<const T*>(sh.v_tail);
 
   float qf[MAXC][NE];
 #pragma unroll
@@ -150,7 +161,7 @@ __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict_
       const int s = sb + 16 * u;
       dot[u] = 0.f;
       if (s < s1) {
-        const T* krow = kbase + (int64_t)s * sh.kv_ss;
+        const T* krow = kv_row(kbase, ktail, h * sh.kv_sh, s, sh);
 #pragma unroll
         for (int c = 0; c < MAXC; c++)
           if (c < nch) {
@@ -191,7 +202,7 @@ __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict_
     for (int u = 0; u < kUnroll; u++) {
       const int s = sb + 16 * u;
       if (s < s1) {
-        const T* vrow = vbase + (int64_t)s * sh.kv_ss;
+        const T* vrow = kv_row(vbase, vtail, h * sh.kv_sh, s, sh);
 #pragma unroll
         for (int c = 0; c < MAXC; c++)
           if (c < nch) Elems<T, VEC>::load(vrow + (l16 + 16 * c) * NE, vf[u][c]);
@@ -212,6 +223,21 @@ __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict_
     }
   }
   reduce_keys<MAXC, NE>(acc, nch, red);
+  if (gridDim.x == 1) {                                    // all keys in one block: nothing to combine
+    if (threadIdx.x < 16) {
+      const float inv = 1.0f / sum;
+      T* orow = o + b * sh.q_sb + h * sh.q_sh;
+#pragma unroll
+      for (int c = 0; c < MAXC; c++)
+        if (c < nch) {
+#pragma unroll
+          for (int e = 0; e < NE; e++) acc[c][e] *= inv;
+          Elems<T, VEC>::store(orow + (l16 + 16 * c) * NE, acc[c]);
+        }
+      if (threadIdx.x == 0) lse[bh] = mx + __logf(sum);
+    }
+    return;
+  }
   if (threadIdx.x < 16) {
     // partial of this block: [head_dim] unnormalised output, then max and sum
     float* out = part + ((int64_t)bh * gridDim.x + blockIdx.x) * (sh.head_dim + 2);
@@ -234,9 +260,9 @@ __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict_
 // memory system sees the whole request at once.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_step_fwd1_kernel(const T* __restrict__ q, const T* __restrict__ k,
-                                                             const T* __restrict__ v, float* __restrict__ part, StepShape sh,
-                                                             float scale) {
-  constexpr int NE = Chunk<T>::N, KPS = kKeysPerBlock / 16 / 2;      // keys per slot and half
+                                                             const T* __restrict__ v, float* __restrict__ part, T* __restrict__ o,
+                                                             float* __restrict__ lse, StepShape sh, float scale) {
+  constexpr int NE = Chunk<T>::N, KPS = kKeysPerBlock / 16 / 2;      // keys per slot and pass
   typedef typename Vec16<T>::type raw_t;
   __shared__ float scratch[4];
   __shared__ float red[kRedFloats];
@@ -246,6 +272,9 @@ __global__ __launch_bounds__(256) void attn_step_fwd1_kernel(const T* __restrict
   const T* qrow = q + b * sh.q_sb + h * sh.q_sh + l16 * NE;
   const T* kbase = k + b * sh.kv_sb + h * sh.kv_sh + l16 * NE;
   const T* vbase = v + b * sh.kv_sb + h * sh.kv_sh + l16 * NE;
+  const T *ktail = static_cast<const T*>(sh.k_tail), *vtail = static_cast<const T*>(sh.v_tail);
+  const int64_t tail_off = h * sh.kv_sh + l16 * NE;
+  const int s_end = (int)(blockIdx.x + 1) * sh.kpb < sh.seq_kv ? (int)(blockIdx.x + 1) * sh.kpb : sh.seq_kv;
   float qf[NE];
 #pragma unroll
   for (int e = 0; e < NE; e++) qf[e] = 0.f;
@@ -255,20 +284,18 @@ __global__ __launch_bounds__(256) void attn_step_fwd1_kernel(const T* __restrict
   float acc[1][NE];
 #pragma unroll
   for (int e = 0; e < NE; e++) acc[0][e] = 0.f;
-  // two halves of 16 keys per slot: registers hold 16 K and 16 V chunks at a time
+  // passes of 16 keys per slot: registers hold 16 K and 16 V chunks at a time
 #pragma unroll 1
-  for (int half = 0; half < 2; half++) {
-    const int s0 = blockIdx.x * kKeysPerBlock + half * (kKeysPerBlock / 2);
-    if (s0 >= sh.seq_kv) break;
+  for (int s0 = blockIdx.x * sh.kpb; s0 < s_end; s0 += KPS * 16) {
     raw_t kr[KPS], vr[KPS];
 #pragma unroll
     for (int u = 0; u < KPS; u++) {
       const int s = s0 + slot + 16 * u;
       kr[u] = Vec16<T>::zero();
       vr[u] = Vec16<T>::zero();
-      if (mine && s < sh.seq_kv) {
-        kr[u] = stream_load(reinterpret_cast<const raw_t*>(kbase + (int64_t)s * sh.kv_ss));     // the cache rows are read once
-        vr[u] = stream_load(reinterpret_cast<const raw_t*>(vbase + (int64_t)s * sh.kv_ss));
+      if (mine && s < s_end) {
+        kr[u] = stream_load(reinterpret_cast<const raw_t*>(kv_row(kbase, ktail, tail_off, s, sh)));     // the cache rows are read once
+        vr[u] = stream_load(reinterpret_cast<const raw_t*>(kv_row(vbase, vtail, tail_off, s, sh)));
       }
     }
     float sc[KPS];
@@ -280,7 +307,7 @@ __global__ __launch_bounds__(256) void attn_step_fwd1_kernel(const T* __restrict
       float dot = 0.f;
 #pragma unroll
       for (int e = 0; e < NE; e++) dot = fmaf(qf[e], kf[e], dot);
-      sc[u] = s0 + slot + 16 * u < sh.seq_kv ? sum16(dot) * scale : -INFINITY;
+      sc[u] = s0 + slot + 16 * u < s_end ? sum16(dot) * scale : -INFINITY;
       hm = fmaxf(hm, sc[u]);
     }
     // running maximum per slot (online softmax): rescale what has been accumulated so far
@@ -307,6 +334,16 @@ __global__ __launch_bounds__(256) void attn_step_fwd1_kernel(const T* __restrict
   for (int e = 0; e < NE; e++) acc[0][e] *= w;
   float bsum = block_sum(l16 == 0 ? sum * w : 0.f, scratch);
   reduce_keys<1, NE>(acc, mine ? 1 : 0, red);
+  if (gridDim.x == 1) {                                    // all keys in one block: nothing to combine
+    if (threadIdx.x < 16) {
+      const float inv = 1.0f / bsum;
+#pragma unroll
+      for (int e = 0; e < NE; e++) acc[0][e] *= inv;
+      if (mine) Chunk<T>::store(o + b * sh.q_sb + h * sh.q_sh + l16 * NE, acc[0]);
+      if (threadIdx.x == 0) lse[bh] = bm + __logf(bsum);
+    }
+    return;
+  }
   if (threadIdx.x < 16) {
     float* out = part + ((int64_t)bh * gridDim.x + blockIdx.x) * (sh.head_dim + 2);
     if (mine) {
@@ -383,12 +420,13 @@ __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict_
   constexpr int NE = E::N, MAXC = NCH, U = NCH >= 4 ? 1 : 4 / NCH;      // keys per slot and batch
   __shared__ float red[kRedFloats];
   const int bh = blockIdx.y, b = bh / sh.heads, h = bh % sh.heads;
-  const int s0 = blockIdx.x * kKeysPerBlock;
-  const int s1 = s0 + kKeysPerBlock < sh.seq_kv ? s0 + kKeysPerBlock : sh.seq_kv;
+  const int s0 = blockIdx.x * sh.kpb;
+  const int s1 = s0 + sh.kpb < sh.seq_kv ? s0 + sh.kpb : sh.seq_kv;
   const int l16 = threadIdx.x & 15, slot = threadIdx.x >> 4;
   const int nchunks = sh.head_dim / NE;
   const int nch = (nchunks - l16 + 15) / 16;
   const int64_t qoff = b * sh.q_sb + h * sh.q_sh, kvoff = b * sh.kv_sb + h * sh.kv_sh;
+  const T *ktail = static_cast<const T*>(sh.k_tail), *vtail = static_cast<const T*>(sh.v_tail);
   const float L = lse[bh];
 
   float qf[MAXC][NE], dof[MAXC][NE];
@@ -422,11 +460,11 @@ __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict_
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int s = sb + 16 * u < s1 ? sb + 16 * u : s1 - 1;
-      const int64_t row = kvoff + (int64_t)s * sh.kv_ss;
+      const T *krow = kv_row(k + kvoff, ktail, h * sh.kv_sh, s, sh), *vrow = kv_row(v + kvoff, vtail, h * sh.kv_sh, s, sh);
 #pragma unroll
       for (int c = 0; c < MAXC; c++) {
-        kr[u][c] = E::load_raw(k + row + coff[c]);
-        vr[u][c] = E::load_raw(v + row + coff[c]);
+        kr[u][c] = E::load_raw(krow + coff[c]);
+        vr[u][c] = E::load_raw(vrow + coff[c]);
       }
     }
   };
@@ -452,8 +490,8 @@ __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict_
       if (s < s1) {
         const float p = __expf(dot * scale - L);
         const float ds = p * (dp - delta) * scale;
-        T* dkrow = dk + kvoff + (int64_t)s * sh.kv_ss;
-        T* dvrow = dv + kvoff + (int64_t)s * sh.kv_ss;
+        T* dkrow = kv_row(dk + kvoff, static_cast<T*>(sh.dk_tail), h * sh.kv_sh, s, sh);
+        T* dvrow = kv_row(dv + kvoff, static_cast<T*>(sh.dv_tail), h * sh.kv_sh, s, sh);
 #pragma unroll
         for (int c = 0; c < MAXC; c++)
           if (c < nch) {
@@ -527,8 +565,8 @@ __global__ __launch_bounds__(256) void attn_step_jvp_kernel(const T* __restrict_
   __shared__ float red[kRedFloats];
   __shared__ float scratch[4];
   const int bh = blockIdx.y, b = bh / sh.heads, h = bh % sh.heads;
-  const int s0 = blockIdx.x * kKeysPerBlock;
-  const int s1 = s0 + kKeysPerBlock < sh.seq_kv ? s0 + kKeysPerBlock : sh.seq_kv;
+  const int s0 = blockIdx.x * sh.kpb;
+  const int s1 = s0 + sh.kpb < sh.seq_kv ? s0 + sh.kpb : sh.seq_kv;
   const int l16 = threadIdx.x & 15, slot = threadIdx.x >> 4;
   const int nchunks = sh.head_dim / NE;
   const int nch = (nchunks - l16 + 15) / 16;
@@ -663,7 +701,103 @@ int check_step(const char* name, int64_t batch, int64_t heads, int64_t seq_kv, i
   return EMI_OK;
 }
 
+// Launches the forward kernel (sh.kpb keys per block) and, when the keys of a head span several blocks, the combine.
+int launch_step_fwd(hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, float* part, const StepShape& sh,
+                    int bh, bool vec, float scale, int dtype) {
+  const int ne = dtype == EMI_BF16 ? 8 : 4;
+  const int nsplit = (sh.seq_kv + sh.kpb - 1) / sh.kpb;
+  const dim3 grid((unsigned)nsplit, (unsigned)bh);
+#define EMI_STEP_FWD(T, VEC, NCH)                                                                                       \
+  do {                                                                                                                   \
+    hipLaunchKernelGGL((attn_step_fwd_kernel<T, VEC, NCH>), grid, dim3(256), 0, st, (const T*)q, (const T*)k,            \
+                       (const T*)v, part, (T*)o, lse, sh, scale);                                                        \
+    EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
+    if (nsplit > 1)                                                                                                      \
+      hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)o, lse, sh, nsplit); \
+  } while (0)
+#define EMI_STEP_FWD1(T)                                                                                                \
+  do {                                                                                                                   \
+    hipLaunchKernelGGL(attn_step_fwd1_kernel<T>, grid, dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, part,    \
+                       (T*)o, lse, sh, scale);                                                                           \
+    EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
+    if (nsplit > 1)                                                                                                      \
+      hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)o, lse, sh, nsplit); \
+  } while (0)
+#define EMI_STEP_FWD_T(T)                                              \
+  do {                                                                 \
+    if (!vec) EMI_STEP_FWD(T, false, 16);                              \
+    else if (nch <= 1) EMI_STEP_FWD1(T);                               \
+    else if (nch <= 2) EMI_STEP_FWD(T, true, 2);                       \
+    else EMI_STEP_FWD(T, true, 4);                                     \
+  } while (0)
+  const int nch = (int)((sh.head_dim / ne + 15) / 16);      // 16-byte chunks per lane
+  if (dtype == EMI_BF16) EMI_STEP_FWD_T(bf16);
+  else EMI_STEP_FWD_T(float);
+#undef EMI_STEP_FWD_T
+#undef EMI_STEP_FWD1
+#undef EMI_STEP_FWD
+  EMI_CHECK_LAUNCH("emi_attn_step_fwd(combine)");
+  return EMI_OK;
+}
+
+// Launches the adjoint kernel and, unless dq is null (the caller sums the blocks' shares in `part` itself), the sum of dQ.
+int launch_step_bwd(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const float* lse, const void* d_o,
+                    void* dq, void* dk, void* dv, float* part, const StepShape& sh, int bh, bool vec, float scale, int dtype) {
+  const int ne = dtype == EMI_BF16 ? 8 : 4;
+  const int nsplit = (sh.seq_kv + sh.kpb - 1) / sh.kpb;
+  const dim3 grid((unsigned)nsplit, (unsigned)bh);
+#define EMI_STEP_BWD(T, VEC, NCH)                                                                                       \
+  do {                                                                                                                   \
+    hipLaunchKernelGGL((attn_step_bwd_kernel<T, VEC, NCH>), grid, dim3(256), 0, st, (const T*)q, (const T*)k,            \
+                       (const T*)v, (const T*)o, lse, (const T*)d_o, part, (T*)dk, (T*)dv, sh, scale);                   \
+    EMI_CHECK_LAUNCH("emi_attn_step_bwd");                                                                               \
+    if (dq != nullptr)                                                                                                   \
+      hipLaunchKernelGGL(attn_step_dq_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)dq, sh, nsplit);         \
+  } while (0)
+#define EMI_STEP_BWD_T(T)                                              \
+  do {                                                                 \
+    if (!vec) EMI_STEP_BWD(T, false, 16);                              \
+    else if (nch <= 1) EMI_STEP_BWD(T, true, 1);                       \
+    else if (nch <= 2) EMI_STEP_BWD(T, true, 2);                       \
+    else EMI_STEP_BWD(T, true, 4);                                     \
+  } while (0)
+  const int nch = (int)((sh.head_dim / ne + 15) / 16);      // 16-byte chunks per lane
+  if (dtype == EMI_BF16) EMI_STEP_BWD_T(bf16);
+  else EMI_STEP_BWD_T(float);
+#undef EMI_STEP_BWD_T
+#undef EMI_STEP_BWD
+  EMI_CHECK_LAUNCH("emi_attn_step_bwd(dq)");
+  return EMI_OK;
+}
+
 }  // namespace
+
+// The whole-step path (llama_step.hip): one query per head of all `heads` (rows of heads * head_dim elements) against the
+// cache [pos, heads * head_dim] and the token's own k and v rows.  Every row is 16-byte aligned.
+int launch_llama_step_attn_fwd(hipStream_t st, const void* q, const void* k_cache, const void* v_cache, const void* k_tail,
+                               const void* v_tail, void* o, float* lse, float* part, int heads, int pos, int head_dim, int keys_per_block,
+                               float scale, int dtype) {
+  const int64_t D = (int64_t)heads * head_dim;
+  StepShape sh{heads, pos + 1, head_dim, D, head_dim, (int64_t)pos * D, head_dim, D};
+  sh.kpb = keys_per_block;
+  sh.k_tail = k_tail;
+  sh.v_tail = v_tail;
+  return launch_step_fwd(st, q, k_cache, v_cache, o, lse, part, sh, heads, true, scale, dtype);
+}
+// dq stays as the blocks' shares in part [heads][blocks][head_dim + 2].
+int launch_llama_step_attn_bwd(hipStream_t st, const void* q, const void* k_cache, const void* v_cache, const void* k_tail,
+                               const void* v_tail, const void* o, const float* lse, const void* d_o, void* dk_cache, void* dv_cache,
+                               void* dk_tail, void* dv_tail, float* part, int heads, int pos, int head_dim, int keys_per_block, float scale,
+                               int dtype) {
+  const int64_t D = (int64_t)heads * head_dim;
+  StepShape sh{heads, pos + 1, head_dim, D, head_dim, (int64_t)pos * D, head_dim, D};
+  sh.kpb = keys_per_block;
+  sh.k_tail = k_tail;
+  sh.v_tail = v_tail;
+  sh.dk_tail = dk_tail;
+  sh.dv_tail = dv_tail;
+  return launch_step_bwd(st, q, k_cache, v_cache, o, lse, d_o, nullptr, dk_cache, dv_cache, part, sh, heads, true, scale, dtype);
+}
 }  // namespace emi
 
 using namespace emi;
@@ -691,40 +825,8 @@ extern "C" int emi_attn_step_fwd(emi_stream_t stream, const void* q, const void*
   const int ne = dtype == EMI_BF16 ? 8 : 4;
   const bool vec = head_dim % ne == 0 && q_stride_b % ne == 0 && q_stride_h % ne == 0 && kv_stride_b % ne == 0 &&
                    kv_stride_h % ne == 0 && kv_stride_s % ne == 0 && al16(q) && al16(k) && al16(v);
-  const int nsplit = (int)((seq_kv + kKeysPerBlock - 1) / kKeysPerBlock);
-  const dim3 grid((unsigned)nsplit, (unsigned)(batch * heads));
   float* part = static_cast<float*>(workspace);
-#define EMI_STEP_FWD(T, VEC, NCH)                                                                                       \
-  do {                                                                                                                   \
-    hipLaunchKernelGGL((attn_step_fwd_kernel<T, VEC, NCH>), grid, dim3(256), 0, st, (const T*)q, (const T*)k,            \
-                       (const T*)v, part, sh, scale);                                                                    \
-    EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
-    hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)(batch * heads)), dim3(64), 0, st, part, (T*)o, lse,  \
-                       sh, nsplit);                                                                                      \
-  } while (0)
-#define EMI_STEP_FWD1(T)                                                                                                \
-  do {                                                                                                                   \
-    hipLaunchKernelGGL(attn_step_fwd1_kernel<T>, grid, dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, part,    \
-                       sh, scale);                                                                                       \
-    EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
-    hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)(batch * heads)), dim3(64), 0, st, part, (T*)o, lse,  \
-                       sh, nsplit);                                                                                      \
-  } while (0)
-#define EMI_STEP_FWD_T(T)                                              \
-  do {                                                                 \
-    if (!vec) EMI_STEP_FWD(T, false, 16);                              \
-    else if (nch <= 1) EMI_STEP_FWD1(T);                               \
-    else if (nch <= 2) EMI_STEP_FWD(T, true, 2);                       \
-    else EMI_STEP_FWD(T, true, 4);                                     \
-  } while (0)
-  const int nch = (int)((head_dim / ne + 15) / 16);      // 16-byte chunks per lane
-  if (dtype == EMI_BF16) EMI_STEP_FWD_T(bf16);
-  else EMI_STEP_FWD_T(float);
-#undef EMI_STEP_FWD_T
-#undef EMI_STEP_FWD1
-#undef EMI_STEP_FWD
-  EMI_CHECK_LAUNCH("emi_attn_step_fwd(combine)");
-  return EMI_OK;
+  return launch_step_fwd(st, q, k, v, o, lse, part, sh, (int)(batch * heads), vec, scale, dtype);
 }
 
 extern "C" int emi_attn_step_bwd(emi_stream_t stream, const void* q, const void* k, const void* v, const void* o,
@@ -746,31 +848,8 @@ extern "C" int emi_attn_step_bwd(emi_stream_t stream, const void* q, const void*
   const bool vec = head_dim % ne == 0 && q_stride_b % ne == 0 && q_stride_h % ne == 0 && kv_stride_b % ne == 0 &&
                    kv_stride_h % ne == 0 && kv_stride_s % ne == 0 && al16(q) && al16(k) && al16(v) && al16(o) && al16(d_o) &&
                    al16(dk) && al16(dv);
-  const int nsplit = (int)((seq_kv + kKeysPerBlock - 1) / kKeysPerBlock);
-  const dim3 grid((unsigned)nsplit, (unsigned)(batch * heads));
   float* part = static_cast<float*>(workspace);
-#define EMI_STEP_BWD(T, VEC, NCH)                                                                                       \
-  do {                                                                                                                   \
-    hipLaunchKernelGGL((attn_step_bwd_kernel<T, VEC, NCH>), grid, dim3(256), 0, st, (const T*)q, (const T*)k,            \
-                       (const T*)v, (const T*)o, lse, (const T*)d_o, part, (T*)dk, (T*)dv, sh, scale);                   \
-    EMI_CHECK_LAUNCH("emi_attn_step_bwd");                                                                               \
-    hipLaunchKernelGGL(attn_step_dq_kernel<T>, dim3((unsigned)(batch * heads)), dim3(64), 0, st, part, (T*)dq, sh,       \
-                       nsplit);                                                                                          \
-  } while (0)
-#define EMI_STEP_BWD_T(T)                                              \
-  do {                                                                 \
-    if (!vec) EMI_STEP_BWD(T, false, 16);                              \
-    else if (nch <= 1) EMI_STEP_BWD(T, true, 1);                       \
-    else if (nch <= 2) EMI_STEP_BWD(T, true, 2);                       \
-    else EMI_STEP_BWD(T, true, 4);                                     \
-  } while (0)
-  const int nch = (int)((head_dim / ne + 15) / 16);      // 16-byte chunks per lane
-  if (dtype == EMI_BF16) EMI_STEP_BWD_T(bf16);
-  else EMI_STEP_BWD_T(float);
-#undef EMI_STEP_BWD_T
-#undef EMI_STEP_BWD
-  EMI_CHECK_LAUNCH("emi_attn_step_bwd(dq)");
-  return EMI_OK;
+  return launch_step_bwd(st, q, k, v, o, lse, d_o, dq, dk, dv, part, sh, (int)(batch * heads), vec, scale, dtype);
 }
 
 extern "C" int emi_attn_step_jvp(emi_stream_t stream, const void* q, const void* k, const void* v, const void* o,

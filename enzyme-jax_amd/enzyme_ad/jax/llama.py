@@ -57,13 +57,18 @@ def forward_step(x, config, weights, key_cache, value_cache, eps=1e-5, theta=100
     (test/llama.py:35-238): x is the residual stream of one token [dim];
     key_cache / value_cache are [n_layers, pos, kv_dim] and the token sits at
     position pos = key_cache.shape[1].  Returns the final RMSNorm of the residual
-    stream.  Every projection is a mat-vec (weight-bandwidth-bound kernels)."""
+    stream.  Every projection is a mat-vec (weight-bandwidth-bound kernels).  One operator runs the whole step where it
+    applies (`ops.llama_step`); forward mode and odd shapes take the operators below one by one."""
     n_layers, n_heads = config["n_layers"], config["n_heads"]
     if config.get("n_kv_heads", n_heads) != n_heads:
         # the reference reshapes k with `dim`, not `kv_dim` (:162,171): it only runs with equal head counts
         raise ValueError("forward_step: n_kv_heads must equal n_heads")
     dim = x.shape[-1]
     pos = key_cache.shape[1]
+    stacks = [weights[k] for k in ops.STEP_WEIGHTS]
+    if ops.llama_step_applies(x, stacks, key_cache, value_cache, n_heads):
+        table = ops.rope_table(1, dim // n_heads, theta, pos, x.device)
+        return ops.llama_step(x, stacks, key_cache, value_cache, n_heads, table, eps)
     for i in range(n_layers):
         lw = {k: ops.select(weights[k], i) for k in LAYER_KEYS}
         xb = ops.rmsnorm(x, lw["rms_att_weight"], eps)                                    # :145

@@ -1098,6 +1098,57 @@ def attention_step(q, k_cache, v_cache, n_heads, scale=None, return_lse=False):
     return (o, lse) if return_lse else o
 
 
+STEP_WEIGHTS = ("rms_att_weight", "wq", "wk", "wv", "wo", "rms_ffn_weight", "w1", "w2", "w3", "rms_final_weight")
+
+
+def llama_step_applies(x, weights, key_cache, value_cache, n_heads):
+    """Whether `llama_step` serves these operands (else the step runs operator by operator): reverse or no
+    differentiation, one dtype, contiguous stacks whose rows are whole 16-byte pieces, at least one earlier position."""
+    if Forward._active is not None or x.dim() != 1 or key_cache.dim() != 3 or key_cache.shape != value_cache.shape:
+        return False
+    L_, pos, D = key_cache.shape
+    w1 = weights[6]
+    H = w1.shape[-2] if w1.dim() == 3 else 0
+    shapes = [(L_, D), (L_, D, D), (L_, D, D), (L_, D, D), (L_, D, D), (L_, D), (L_, H, D), (L_, D, H), (L_, H, D), (D,)]
+    for t, s in zip((x, key_cache, value_cache, *weights), [(D,), (L_, pos, D), (L_, pos, D)] + shapes):
+        if t.shape != s or t.dtype != x.dtype or not t.is_contiguous() or t.data_ptr() & 15 or not t.is_cuda:
+            return False
+    return x.dtype in _DTYPES and N.lib().emi_llama_step_saved_bytes(L_, D, H, n_heads, pos, _code(x)) != 0
+
+
+def llama_step(x, weights, key_cache, value_cache, n_heads, table, eps=1e-5, scale=None):
+    """The reference's single-token step (test/llama.py:35-238) as one operator: `weights` in the order of STEP_WEIGHTS,
+    stacked per layer, `table` the fp32 (cos, sin) pairs of the token's position ([pairs, 2], repeated over the row).  The
+    same values and gradients as the operators of llama.forward_step up to the rounding of what lies between two
+    products, which here stays in fp32 (emi_llama_step_fwd / _bwd)."""
+    weights = list(weights)
+    _dev(x, *weights, key_cache, value_cache, table)
+    L_, pos, D = key_cache.shape
+    H = weights[6].shape[1]
+    lib, code = N.lib(), _code(x)
+    if scale is None:
+        scale = 1.0 / math.sqrt(D // n_heads)
+    pairs = table.numel() // 2
+    dims = (L_, D, H, n_heads, pos, eps, float(scale), code)
+    nbytes = lib.emi_llama_step_saved_bytes(L_, D, H, n_heads, pos, code)
+    saved = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    y = torch.empty_like(x)
+    wptr = _ptr_table(weights)
+    N.check(lib.emi_llama_step_fwd(_stream(), wptr, _p(x), _p(key_cache), _p(value_cache), _p(table), pairs, _p(y), _p(saved), nbytes, *dims))
+    operands = (x, *weights, key_cache, value_cache)
+
+    def rule(c, acc):
+        grads = [torch.empty_like(t) for t in operands]
+        nb = lib.emi_llama_step_bwd_workspace_bytes(L_, D, H, n_heads, pos, code)
+        ws = torch.empty(nb, dtype=torch.uint8, device=x.device)
+        N.check(lib.emi_llama_step_bwd(_stream(), _ptr_table(weights), _p(x), _p(key_cache), _p(value_cache), _p(table), pairs, _p(saved),
+                                       _p(c.contiguous()), _ptr_table(grads), _p(ws), nb, *dims))
+        return [_accumulate(a, g) for a, g in zip(acc, grads)]
+
+    Tape.record(operands, y, rule)
+    return y
+
+
 def embedding(tokens, table):
     """table[tokens] (the lookup commented out at test/llama.py:109-113)."""
     _dev(tokens, table)

@@ -989,6 +989,124 @@ def _fuse_blocks(run_ops, func):
     return [place.get(id(op), op) for op in run_ops if id(op) not in drop]
 
 
+def _step_view(run_ops, consts):
+    """The list as `_fuse_step` reads it: reshapes gone (a value and its reshapes are one name), this library's custom
+    calls of a one-token program under the names of the clusters they were printed from."""
+    alias, out = {}, []
+    root = lambda v: alias.get(v, v)
+    for op in run_ops:
+        if op.name == "reshape":
+            alias[op.results[0]] = root(op.operands[0])
+            continue
+        name, attrs, operands = op.name, op.attrs, [root(o) for o in op.operands]
+        if name == "custom_call":
+            cfg, target = attrs["config"], attrs["target"]
+            if target == "emi_rmsnorm_fwd":
+                name, attrs = "emi.rmsnorm", {"eps": cfg.get("eps", 1e-5)}
+            elif target == "emi_swiglu_fwd":
+                name, attrs = "emi.swiglu", {}
+            elif target == "emi_gemm" and cfg.get("trans_b", False) and not cfg.get("trans_a", False) and op.types[0].shape[0] == 1:
+                name, attrs = "emi.linear", {}
+            elif target == "emi_rope" and not cfg.get("inverse", False) and operands[1] in consts:
+                name, attrs, operands = "emi.rope", {"table": np.asarray(consts[operands[1]], dtype=np.float32).reshape(-1, 2)}, operands[:1]
+            elif target == "emi_attn_step_fwd" and op.types[0].shape[0] == 1:
+                name, attrs = "emi.attention_step", {"scale": cfg["scale"], "heads": op.types[0].shape[1]}
+        out.append((Op(name, list(op.results), operands, attrs, op.types), op))
+    return out, root
+
+
+def _fuse_step(run_ops, func):
+    """The operator list with the whole single-token step (test/llama.py:35-238) as one `emi.llama_step`, or None when
+    the list is not that program: L layers of norm, q / k / v, rotation, cache rows with the token's own appended,
+    attention, wo with residual, norm, w1 / w3, SwiGLU, w2 with residual - layer l on slice l of stacks of L slices, each
+    interior value used only there - and a final norm.  The form `optimize_module` prints (custom calls) is one of its
+    spellings."""
+    consts = {op.results[0]: op.attrs["value"] for op in run_ops if op.name == "constant"}
+    view, root = _step_view(run_ops, consts)
+    rets = set(root(o) for op, _ in view if op.name == "return" for o in op.operands)
+    shape = {a: t.shape for a, t in func.args}
+    use, producer, original = {}, {}, {}
+    for op, was in view:
+        original[id(op)] = was
+        for r in op.results:
+            producer[r] = op
+        for o in op.operands:
+            use.setdefault(o, []).append(op)
+
+    def made(value, name, n_operands, n_users=1):
+        op = producer.get(value)
+        ok = (op is not None and op.name == name and len(op.operands) == n_operands and op.results[0] == value
+              and len(use.get(value, ())) == n_users and value not in rets)
+        if not ok:
+            raise LookupError
+        return op
+
+    def slice_of(value, l):
+        op = made(value, "emi.select", 1)
+        if op.attrs["index"] != l or op.operands[0] not in shape:
+            raise LookupError
+        return op.operands[0]
+
+    def cache(value, l):
+        cat = made(value, "concatenate", 2)
+        if cat.attrs["dim"] != 0:
+            raise LookupError
+        return slice_of(cat.operands[0], l), cat.operands[1]
+
+    def layer(att, l):
+        rq = made(att.operands[0], "emi.rope", 1)
+        kc, k = cache(att.operands[1], l)
+        vc, v = cache(att.operands[2], l)
+        rk = made(k, "emi.rope", 1)
+        lq, lk, lv = made(rq.operands[0], "emi.linear", 2), made(rk.operands[0], "emi.linear", 2), made(v, "emi.linear", 2)
+        norm = made(lq.operands[0], "emi.rmsnorm", 2, 3)
+        x = norm.operands[0]
+        (lo,) = use[att.results[0]]
+        if lo.name != "emi.linear" or len(lo.operands) != 3 or lo.operands[0] != att.results[0] or lo.operands[2] != x:
+            raise LookupError
+        x1 = lo.results[0]
+        norm2 = next((u for u in use.get(x1, ()) if u.name == "emi.rmsnorm" and u.operands[0] == x1), None)
+        l2 = next((u for u in use.get(x1, ()) if u.name == "emi.linear" and len(u.operands) == 3 and u.operands[2] == x1), None)
+        if norm2 is None or l2 is None or len(use[x1]) != 2 or x1 in rets or made(norm2.results[0], "emi.rmsnorm", 2, 2) is not norm2:
+            raise LookupError
+        sg = made(l2.operands[0], "emi.swiglu", 2)
+        l1, l3 = made(sg.operands[0], "emi.linear", 2), made(sg.operands[1], "emi.linear", 2)
+        if (any(o.operands[0] != norm.results[0] for o in (lk, lv)) or any(o.operands[0] != norm2.results[0] for o in (l1, l3))
+                or norm.attrs["eps"] != norm2.attrs["eps"] or not np.array_equal(rq.attrs["table"], rk.attrs["table"])
+                or any(r in use or r in rets for r in att.results[1:])):
+            raise LookupError
+        stacks = [slice_of(w, l) for w in (norm.operands[1], lq.operands[1], lk.operands[1], lv.operands[1], lo.operands[1],
+                                           norm2.operands[1], l1.operands[1], l2.operands[1], l3.operands[1])] + [kc, vc]
+        return x, l2.results[0], stacks, (norm.attrs["eps"], att.attrs["scale"], att.attrs["heads"]), rq.attrs["table"]
+
+    try:
+        atts = [op for op, _ in view if op.name == "emi.attention_step"]
+        if not atts or any(len(use.get(a.results[0], ())) != 1 or a.results[0] in rets for a in atts):
+            return None
+        layers = [layer(a, l) for l, a in enumerate(atts)]
+        for a, b in zip(layers, layers[1:]):
+            # layer l's result: the norm and the residual of layer l + 1
+            if b[0] != a[1] or b[2:4] != a[2:4] or not np.array_equal(a[4], b[4]) or len(use[a[1]]) != 2 or a[1] in rets:
+                return None
+        _, out, stacks, (eps, scale, heads), table = layers[-1]
+        if any(shape[w][0] != len(layers) for w in stacks) or len(set(stacks)) != len(stacks):
+            return None
+        (final,) = use.get(out, ())
+        if final.name != "emi.rmsnorm" or out in rets or final.operands[0] != out or final.operands[1] not in shape or final.attrs["eps"] != eps:
+            return None
+    except (LookupError, ValueError):
+        return None
+    step = Op("emi.llama_step", final.results, [layers[0][0]] + stacks[:9] + [final.operands[1]] + stacks[9:],
+              {"eps": eps, "scale": scale, "heads": heads, "table": np.ascontiguousarray(table, dtype=np.float32),
+               "printed": original[id(final)].name == "custom_call"}, final.types)
+    new, live = [], set()
+    for op in reversed([step if op is original[id(final)] else op for op in run_ops]):
+        if op.name == "return" or any(r in live for r in op.results):      # what only the step's inside used is gone
+            live.update(op.operands)
+            new.append(op)
+    return new[::-1]
+
+
 def _match_rmsnorm(op, d, tb):
     # root: a product of three factors, (w * x) * bcast(ss) or w * (x * bcast(ss)) in any
     # operand order, ss = 1 / sqrt(dot(x, x) / n + eps) or rsqrt(...)
@@ -1628,6 +1746,7 @@ class Executable:
         self._consts = {}
         for f in self.funcs.values():
             f.run_ops = _fuse_blocks(_fold_selects(f), f) if fuse else f.ops
+            f.step_ops = _fuse_step(f.run_ops, f) if fuse else None
 
     def signature(self, fn="main"):
         f = self._func(fn)
@@ -1646,6 +1765,13 @@ class Executable:
             host = torch.from_numpy(np.ascontiguousarray(op.attrs["value"]).reshape(-1)).reshape(ty.shape)
             hit = self._consts[key] = host.to(TORCH_DTYPES[ty.dtype]).to(device)       # trace-time constant upload
         return hit
+
+    def _table(self, op, device):
+        key = (id(op), "table", str(device))
+        table = self._consts.get(key)
+        if table is None:
+            table = self._consts[key] = torch.from_numpy(op.attrs["table"]).to(device)
+        return table
 
     def run(self, args, fn="main"):
         f = self._func(fn)
@@ -1666,7 +1792,16 @@ class Executable:
             env[name] = a
         if device is None:
             device = torch.device("cuda", torch.cuda.current_device())
-        for op in getattr(f, "run_ops", f.ops):
+        run_ops = getattr(f, "run_ops", f.ops)
+        if getattr(f, "step_ops", None) is not None:
+            step = next(op for op in f.step_ops if op.name == "emi.llama_step")
+            xs = [env.get(o) for o in step.operands]
+            # a program of custom calls that is only run keeps them one by one, as a client with the handlers runs it (the
+            # same bits); differentiated here, it is the operator of the text it was printed from
+            as_printed = step.attrs["printed"] and ops.Tape._active is None
+            if xs[0] is not None and not as_printed and ops.llama_step_applies(xs[0], xs[1:11], xs[11], xs[12], step.attrs["heads"]):
+                run_ops = f.step_ops
+        for op in run_ops:
             if op.name == "return":
                 return [env[o] for o in op.operands]
             outs = self._apply(f, op, [env[o] for o in op.operands], device)
@@ -1731,6 +1866,10 @@ class Executable:
             return [H.pad(xs[0], op.attrs["low"], op.attrs["high"], op.attrs["interior"], op.types[0].shape)]
         if n == "call":
             return self.run(xs, op.attrs["callee"])
+        if n == "emi.llama_step":
+            a = op.attrs
+            y = ops.llama_step(xs[0], xs[1:11], xs[11], xs[12], a["heads"], self._table(op, device), a["eps"], a["scale"])
+            return [y if op.types[0].shape == tuple(y.shape) else ops.reshape(y, op.types[0].shape)]
         if n == "custom_call":
             return self._custom_call(op, xs)
         if n == "emi.linear":
@@ -1779,11 +1918,7 @@ class Executable:
         if n == "emi.swiglu":
             return [ops.swiglu(_packed(xs[0]), _packed(xs[1]))]
         if n == "emi.rope":
-            key = (id(op), "table", str(device))
-            table = self._consts.get(key)
-            if table is None:
-                table = self._consts[key] = torch.from_numpy(op.attrs["table"]).to(device)
-            return [ops.rotate_pairs(_packed(xs[0]), table)]
+            return [ops.rotate_pairs(_packed(xs[0]), self._table(op, device))]
         if n == "emi.softmax_dot":
             q, k, v = xs
             return [ops.attention_step(_packed(q), _packed(k), _packed(v), 1, op.attrs["scale"])]

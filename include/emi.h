@@ -259,6 +259,26 @@ int emi_attn_jvp(emi_stream_t stream, const void* q, const void* k, const void* 
                  int64_t heads, int64_t seq, int64_t head_dim, int64_t stride_b, int64_t stride_h,
                  int64_t stride_s, float scale, int causal, int dtype);
 
+/* The whole single-token step of test/llama.py:35-238 and its reverse, one call each.
+ * weights: the ten arrays rms_att_weight[L, D], wq, wk, wv, wo[L, D, D], rms_ffn_weight[L, D],
+ * w1[L, H, D], w2[L, D, H], w3[L, H, D], rms_final_weight[D]; x, y[D]; key_cache, value_cache
+ * [L, pos, D] (pos >= 1; the token sits at position pos); rope_table: fp32 (cos, sin) of the
+ * token's position, table_pairs entries, pair i of a row turned by entry i mod table_pairs.
+ * `saved` (emi_llama_step_saved_bytes) is written by the forward call and read by the reverse
+ * one.  grads: the thirteen results dx, the ten weights' in the order above, the two caches'.
+ * emi_llama_step_saved_bytes is 0 for shapes the calls do not take (dim, hidden and head_dim
+ * must be multiples of 16 bytes, dim <= 8192, head_dim <= 256). */
+size_t emi_llama_step_saved_bytes(int64_t layers, int64_t dim, int64_t hidden, int64_t heads, int64_t pos, int dtype);
+size_t emi_llama_step_bwd_workspace_bytes(int64_t layers, int64_t dim, int64_t hidden, int64_t heads, int64_t pos, int dtype);
+int emi_llama_step_fwd(emi_stream_t stream, const void* const* weights, const void* x, const void* key_cache,
+                       const void* value_cache, const float* rope_table, int64_t table_pairs, void* y, void* saved,
+                       size_t saved_bytes, int64_t layers, int64_t dim, int64_t hidden, int64_t heads, int64_t pos,
+                       float eps, float scale, int dtype);
+int emi_llama_step_bwd(emi_stream_t stream, const void* const* weights, const void* x, const void* key_cache,
+                       const void* value_cache, const float* rope_table, int64_t table_pairs, const void* saved,
+                       const void* dy, void* const* grads, void* workspace, size_t workspace_bytes, int64_t layers,
+                       int64_t dim, int64_t hidden, int64_t heads, int64_t pos, float eps, float scale, int dtype);
+
 /* Forward mode of the single-token attention (emi_attn_step_fwd's layout, o and lse from
  * it): to = sum_s p_s (tS_s v_s + tv_s) - (sum_s p_s tS_s) o with tS_s = scale (tq.k_s + q.tk_s).
  * Null tq / tk / tv = zero tangent.  workspace: emi_attn_step_workspace_bytes(). */

@@ -1,0 +1,73 @@
+"""The single-token step as one operator (ops.llama_step): the value and all thirteen cotangents against the oracle's
+forward_step / forward_step_vjp at the sizes where its kernels change - rows shorter and longer than a batch of loads, one
+and several key blocks per head, one and two 16-byte pieces of a head per lane, one and several bands and column groups of
+the adjoint products - and the operators it stands for, which forward mode and odd shapes still take."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import llama_ref as L
+from gpu_util import dev, check, rel_err, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(dt, dim, hidden, layers, heads, pos, seed):
+    cfg = dict(dim=dim, hidden_dim=hidden, n_layers=layers, n_heads=heads, n_kv_heads=heads, vocab_size=8, seq_len=pos + 1)
+    rng = np.random.Generator(np.random.PCG64(seed))
+    w = L.make_weights(cfg, seed, std=1.0 / np.sqrt(dim), embedding=False, norm_gain="uniform")
+    w.pop("wcls", None)
+    wd, wr = {}, {}
+    for k, a in w.items():
+        wd[k], wr[k] = dev(a, dt)
+    arrays = [rng.standard_normal(s) for s in ((dim,), (layers, pos, dim), (layers, pos, dim), (dim,))]
+    return cfg, wd, wr, [dev(a, dt) for a in arrays]
+
+
+@pytest.mark.parametrize("dt,dim,hidden,layers,heads,pos", [
+    ("f32", 288, 768, 2, 6, 1),           # the reference's own sizes
+    ("f32", 288, 768, 2, 6, 255),         # exactly one pass of keys
+    ("f32", 288, 768, 1, 6, 256),         # one key more: the token's own row opens a second block
+    ("f32", 512, 516, 1, 4, 700),         # two pieces of a head per lane, several key blocks
+    ("f32", 516, 36, 2, 3, 40),           # rows just over two batches; short ffn
+    ("bf16", 64, 40, 3, 2, 3),
+    ("bf16", 1024, 2816, 2, 8, 300),      # head_dim 128
+    ("bf16", 1056, 264, 1, 11, 129),      # rows just over two batches
+    ("f32", 200, 40, 1, 4, 5),            # head_dim 50: operator by operator
+    ("bf16", 2112, 5632, 1, 12, 520),     # head_dim 176: two pieces per lane; two column groups in the adjoint
+    ("bf16", 4096, 1024, 1, 32, 1030),
+])
+def test_llama_step_matches_oracle(dt, dim, hidden, layers, heads, pos):
+    from enzyme_ad.jax import llama, ops, vjp
+    cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), (dy, dyr)) = _inputs(dt, dim, hidden, layers, heads, pos, dim + pos)
+    applies = ops.llama_step_applies(x, [wd[k] for k in ops.STEP_WEIGHTS], kc, vc, heads)
+    assert applies == (dim != 200)
+    y, pull = vjp(lambda x, w, k, v: llama.forward_step(x, cfg, w, k, v), x, wd, kc, vc)
+    gx, gw, gk, gv = pull(dy)
+    ry, rdx, rgw, rdk, rdv = L.forward_step_vjp(xr, cfg, wr, kcr, vcr, dyr)
+    check(y, ry, dt, "y")
+    check(gx, rdx, dt, "dx")
+    check(gk, rdk, dt, "dkey_cache")
+    check(gv, rdv, dt, "dvalue_cache")
+    for k in wd:
+        # dwk is the outer product of one key's cotangent, per head p scale (dO . v - dO . o) q: the two products cancel.
+        # Their operands are rounded to 2^-9, so with z = dO . (v - o) in units of |dO| |v - o| / sqrt(head_dim) a head's
+        # row is off by about 2^-8 / |z|; twelve or more heads have one at |z| ~ 0.1, i.e. 4e-2
+        # (measured here: 2.3e-2, and 4.6e-2 operator by operator).
+        check(gw[k], rgw[k], dt, "d" + k, factor=2.0 if k == "wk" and dt == "bf16" else 1.0)
+
+
+def test_llama_step_accumulates_and_repeats():
+    """The step's cotangents add to what other uses of its operands contribute, and are the same bits run to run."""
+    from enzyme_ad.jax import llama, ops, vjp
+    cfg, wd, wr, ((x, _), (kc, _), (vc, _), (dy, _)) = _inputs("f32", 96, 64, 2, 2, 5, 3)
+
+    def f(x, w, k, v):
+        return ops.add(llama.forward_step(x, cfg, w, k, v), x)
+
+    y, pull = vjp(f, x, wd, kc, vc)
+    a, b = pull(dy), pull(dy)
+    _, plain = vjp(lambda x, w, k, v: llama.forward_step(x, cfg, w, k, v), x, wd, kc, vc)
+    c = plain(dy)
+    assert torch.equal(a[0], b[0]) and all(torch.equal(a[1][k], b[1][k]) for k in wd)
+    assert rel_err(host(a[0]), host(c[0]) + host(dy)) < 1e-6
