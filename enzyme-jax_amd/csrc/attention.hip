@@ -498,7 +498,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_kernel(const uint16_t* _
           }
           mt = fmaxf(mt, s[T][r]);
         }
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      mt = max_xor32(mt);
       const float m_new = fmaxf(m, mt * scale_log2e);      // running max in the scaled log2 domain
       const float alpha = fast_exp2(m - m_new);
       float rs = 0.f;
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_kernel(const uint16_t* _
   // 16-byte, row-contiguous stores.  Chunk c of row r sits at chunk c ^ (r % CH), the two
   // 8-byte halves swapped when (r / CH) is odd: conflict free for both access shapes.
   // (the loop ended with all loads landed and a barrier: the LDS is idle)
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor32(l);
   {
     constexpr int CH = D / 8, RB = D * 2;
     EMI_LDS uint8_t* wl = smem + wave * (32 * RB);
@@ -753,7 +753,7 @@ __global__ __launch_bounds__(512) void attn_fwd_pp_kernel(const uint16_t* __rest
     for (int T = 0; T < 2; T++)
 #pragma unroll
       for (int r = 0; r < 16; r++) mt = fmaxf(mt, s[T][r]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * scale_log2e;
+    mt = max_xor32(mt) * scale_log2e;
     if (__builtin_amdgcn_ballot_w64(mt > m + 8.0f) != 0) {      // wave-uniform, rare after the first tiles
       const float m_new = fmaxf(m, mt);
       const float alpha = fast_exp2(m - m_new);
@@ -819,7 +819,7 @@ __global__ __launch_bounds__(512) void attn_fwd_pp_kernel(const uint16_t* __rest
   // 16-byte, row-contiguous stores.  Chunk c of row r sits at chunk c ^ (r % CH), the two
   // 8-byte halves swapped when (r / CH) is odd: conflict free for both access shapes.
   phase_end();                                        // every wavefront's loads have landed
-  l += __shfl_xor(l, 32, 64);
+  l = sum_xor32(l);
   {
     constexpr int CH = D / 8, RB = D * 2;
     EMI_LDS uint8_t* wl = smem + wave * (32 * RB);
@@ -915,7 +915,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t
     for (int m = D / 32; m >= 1; m >>= 1)
 #pragma unroll
       for (int t = 0; t < m; t++) cs[t] += cs[t + m];
-    dl = cs[0] + __shfl_xor(cs[0], 32, 64);
+    dl = sum_xor32(cs[0]);
     if (qrow < seq && lane < 32) {
       delta_out[(int64_t)bh * seq + qrow] = dl * delta_sign;
       lse2_out[(int64_t)bh * seq + qrow] = L2;
@@ -1393,7 +1393,7 @@ __global__ __launch_bounds__(256) void attn_jvp_bf16_kernel(const uint16_t* __re
   }
 
   // a lane pair (l, l ^ 32) holds the two halves of a query's keys
-  mu += __shfl_xor(mu, 32, 64);
+  mu = sum_xor32(mu);
   {
     constexpr int CH = D / 8, RB = D * 2;
     EMI_LDS uint8_t* wl = smem + wave * (32 * RB);

@@ -114,12 +114,10 @@ __device__ __forceinline__ void store_cols(float* __restrict__ row, int lane, co
 }
 
 __device__ __forceinline__ float groups_max(float x) {      // over the four lanes that share l % 16
-  x = fmaxf(x, __shfl_xor(x, 16, 64));
-  return fmaxf(x, __shfl_xor(x, 32, 64));
+  return max_xor32(max_xor16(x));
 }
 __device__ __forceinline__ float groups_sum(float x) {
-  x += __shfl_xor(x, 16, 64);
-  return x + __shfl_xor(x, 32, 64);
+  return sum_xor32(sum_xor16(x));
 }
 
 // Forward: o = softmax(scale q k^T) v, lse = log-sum-exp of the scaled scores.

@@ -73,13 +73,7 @@ template <typename T> __device__ __forceinline__ T* kv_row(T* base, T* tail, int
   return tail != nullptr && s == sh.seq_kv - 1 ? tail + off : base + (int64_t)s * sh.kv_ss;
 }
 
-__device__ __forceinline__ float sum16(float v) {          // over the 16 lanes that share a key
-  v += __shfl_xor(v, 1, kWave);
-  v += __shfl_xor(v, 2, kWave);
-  v += __shfl_xor(v, 4, kWave);
-  v += __shfl_xor(v, 8, kWave);
-  return v;
-}
+__device__ __forceinline__ float sum16(float v) { return row16_sum(v); }          // over the 16 lanes that share a key
 
 // Block-wide reductions through a 4-float LDS scratch.
 __device__ __forceinline__ float block_max(float v, float* scratch) {
@@ -109,8 +103,7 @@ __device__ __forceinline__ void reduce_keys(float (&acc)[MAXC][NE], int nch, flo
 #pragma unroll
     for (int e = 0; e < NE; e++) {
       float v = acc[c][e];
-      v += __shfl_xor(v, 16, kWave);
-      v += __shfl_xor(v, 32, kWave);
+      v = sum_xor32(sum_xor16(v));
       if ((threadIdx.x & 63) < 16 && c < nch) red[(wave * MAXC + c) * 16 * NE + l16 * NE + e] = v;
     }
   __syncthreads();

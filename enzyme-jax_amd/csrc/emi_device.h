@@ -195,15 +195,50 @@ template <> struct ChunkCached<bf16> {
   }
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+// Lane exchanges without the LDS (a __shfl goes through it: ~60 cycles each).  ror16<N>: the value N lanes back within each
+// row of 16 lanes; on values that repeat every 2N lanes that is the value of lane ^ N.  pair32 / pair16: the values of
+// lanes l and l ^ 32 (l ^ 16) as a pair, in the same order for both.
+template <int N> __device__ __forceinline__ float ror16(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, true));
 }
+typedef uint32_t emi_u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ emi_u32x2_t pair32(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return emi_u32x2_t{r[0], r[1]};
+}
+__device__ __forceinline__ emi_u32x2_t pair16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return emi_u32x2_t{r[0], r[1]};
+}
+__device__ __forceinline__ float row16_sum(float v) {          // over the 16 lanes of a row
+  v += ror16<8>(v);
+  v += ror16<4>(v);
+  v += ror16<2>(v);
+  return v + ror16<1>(v);
+}
+__device__ __forceinline__ float sum_xor32(float v) {          // over lanes l and l ^ 32
+  const emi_u32x2_t p = pair32(v);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float sum_xor16(float v) {
+  const emi_u32x2_t p = pair16(v);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float max_xor32(float v) {
+  const emi_u32x2_t p = pair32(v);
+  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float max_xor16(float v) {
+  const emi_u32x2_t p = pair16(v);
+  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float wave_sum(float v) { return row16_sum(sum_xor16(sum_xor32(v))); }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+  v = max_xor16(max_xor32(v));
+  v = fmaxf(v, ror16<8>(v));
+  v = fmaxf(v, ror16<4>(v));
+  v = fmaxf(v, ror16<2>(v));
+  return fmaxf(v, ror16<1>(v));
 }
 
 }  // namespace emi

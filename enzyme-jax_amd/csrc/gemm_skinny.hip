@@ -180,9 +180,7 @@ __global__ __launch_bounds__(1024) void gemv_nn_kernel(const T* __restrict__ A, 
 #pragma unroll
     for (int e = 0; e < V; e++) {
       float v = acc[m][e];
-      v += __shfl_xor(v, 8, kWave);
-      v += __shfl_xor(v, 16, kWave);
-      v += __shfl_xor(v, 32, kWave);
+      v = sum_xor32(sum_xor16(v + ror16<8>(v)));
       if ((threadIdx.x & 63) < 8) part[threadIdx.x >> 6][m][cl * V + e] = v;
     }
   __syncthreads();

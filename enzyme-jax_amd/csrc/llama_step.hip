@@ -490,7 +490,7 @@ struct StepDims {
   int kpb() const {
     const int64_t keys = pos + 1;
     if (keys <= 256) return 256;
-    const int64_t want = (keys * heads / 256 + 63) / 64 * 64;
+    const int64_t want = (keys * heads / 512 + 63) / 64 * 64;
     return (int)(want < 128 ? 128 : want > 512 ? 512 : want);
   }
   int nsplit() const { return (int)((pos + 1 + kpb() - 1) / kpb()); }
