@@ -1839,9 +1839,10 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
     const int64_t a_bytes = ((a_rows - 1) * lda + (trans_a ? M : K)) * 2;
     const int64_t b_bytes = ((b_rows - 1) * ldb + (trans_b ? K : N)) * 2;
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    // The fast path moves 16-byte chunks: rows must start 16-byte aligned and
-    // row lengths in the contiguous dimension must be multiples of 8 elements.
-    const bool fast = K > 0 && al16(A) && al16(B) && (lda % 8 == 0) && (ldb % 8 == 0) && (K % 8 == 0) &&
+    // The fast path moves 16-byte chunks: rows must start 16-byte aligned and row lengths in the contiguous dimension of
+    // each operand must be multiples of 8 elements.  K is none where both are k-major (dW = dY^T . X over any number of
+    // tokens: 300 tokens of a 4096-wide layer on the generic kernel took 4.4 of the 6.1 ms of its forward and adjoint).
+    const bool fast = K > 0 && al16(A) && al16(B) && (lda % 8 == 0) && (ldb % 8 == 0) && (K % 8 == 0 || (trans_a && !trans_b)) &&
                       (!trans_a || M % 8 == 0) && (trans_b || N % 8 == 0) && a_bytes < 0x7fffff00LL &&
                       b_bytes < 0x7fffff00LL && ldr <= 0x7fffffff && ldc <= 0x7fffffff;
     if (fast) {
@@ -1991,8 +1992,8 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
     const int64_t a_bytes = ((a_rows - 1) * lda + (trans_a ? M : K)) * 2;
     const int64_t b_bytes = ((b_rows - 1) * ldb + (trans_b ? K : N)) * 2;
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    fast = lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && ldc >= N && (lda % 8 == 0) && (ldb % 8 == 0) && (K % 8 == 0) &&
-           (!trans_a || M % 8 == 0) && (trans_b || N % 8 == 0) && a_bytes < 0x7fffff00LL && b_bytes < 0x7fffff00LL &&
+    fast = lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && ldc >= N && (lda % 8 == 0) && (ldb % 8 == 0) &&
+           (K % 8 == 0 || (trans_a && !trans_b)) && (!trans_a || M % 8 == 0) && (trans_b || N % 8 == 0) && a_bytes < 0x7fffff00LL && b_bytes < 0x7fffff00LL &&
            ldr <= 0x7fffffff && ldc <= 0x7fffffff && ((M + 255) / 256) * ((N + 255) / 256) < 192;
     for (int i = 0; i < count && fast; i++) fast = al16(A[i]) && al16(B[i]);
     // a residual on some results only would need a null check per product: all or none

@@ -46,3 +46,24 @@ def test_bf16_tiles_stages_and_splits(tb, M, N, K, count):
     _check(total, sum(prods) + Rrs[0], sum(mags) + np.abs(Rrs[0]), count * K, "summed + residual")
     again = ops.gemm_grouped(list(As), list(Bs), False, bool(tb), [Rs[0]], sum_into_one=True)
     assert torch.equal(total, again)          # fixed order of summation
+
+
+@pytest.mark.parametrize("M,N,K,count", [
+    (136, 72, 3, 2),          # fewer tokens than a k-row group
+    (256, 264, 77, 3),        # 128-tiles, a ragged last stage
+    (264, 136, 4099, 2),      # splits of a long odd contraction
+    (4096, 3080, 301, 1),     # 256-tiles
+    (256, 256, 301, 48),      # a group that fills the chip with 256-tiles
+])
+def test_bf16_weight_gradients_of_any_number_of_tokens(M, N, K, count):
+    """dW = dY^T . X: both operands are k-major, K (the tokens) is a multiple of nothing."""
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + N + K)
+    As, Ars = zip(*[dev(rng.standard_normal((K, M)), "bf16") for _ in range(count)])
+    Bs, Brs = zip(*[dev(rng.standard_normal((K, N)), "bf16") for _ in range(count)])
+    r, rr = dev(rng.standard_normal((M, N)), "bf16")
+    prods, mags = [a.T @ b for a, b in zip(Ars, Brs)], [np.abs(a).T @ np.abs(b) for a, b in zip(Ars, Brs)]
+    _check(ops.gemm(As[0], Bs[0], True, False, r), prods[0] + rr, mags[0] + np.abs(rr), K, "one product + residual")
+    if count > 1:
+        for o, p, m in zip(ops.gemm_grouped(list(As), list(Bs), True, False), prods, mags):
+            _check(o, p, m, K, "group")
