@@ -586,9 +586,15 @@ def gemm(a, b, trans_a=False, trans_b=False, residual=None, out=None):
     return c
 
 
+_IN_PLACE_TOKENS = 3072
+
+
 def _weight_in_place(rows2d, w):
-    """dX = dY . W reads W as stored (k-major) rather than through a transposed copy."""
-    return rows2d.shape[0] <= 8 or rows2d.dtype == torch.float32
+    """dX = dY . W reads W as stored (k-major) rather than through a transposed copy: always in fp32, whose kernels read
+    either layout at one speed, and in bf16 while the transposes cost more than the k-major form does.  Forward and
+    adjoint of a layer, transposed / in place: dim 4096 on 1 x 300 tokens 1080 / 868 us, on 2 x 1500 3750 / 3615; the
+    dim-768 model on 1 x 1000 4520 / 4310, on 4 x 1024 6107 / 6133, on 8 x 1024 9750 / 9776."""
+    return rows2d.dtype == torch.float32 or rows2d.shape[0] <= _IN_PLACE_TOKENS
 
 
 def _ptr_table(ts):
@@ -701,12 +707,9 @@ def matmul_nt(x, w, residual=None):
     def rule(c, acc):
         c2 = c.reshape(-1, Nout)
         ax = None if acc[0] is None else acc[0].reshape(-1, K)
-        # dX = dY . W: W is transposed first (2|W| bytes of HBM traffic, shared by nothing
-        # else) so that the contraction index is innermost in both operands: the
-        # k-contiguous kernel beats the k-major one by more than the transpose costs.
-        # With a handful of tokens (the single-token step) W is read in place, once; so it is in fp32, whose
-        # kernels read either layout at the same speed.  (Reading small bf16 weights in place was tried for the
-        # 768-wide model: the whole step came out 1.4 % slower than with the transposes.)
+        # dX = dY . W.  Over many tokens W is transposed first (2|W| bytes of HBM traffic, shared by nothing else) so that
+        # the contraction index is innermost in both operands: the k-contiguous kernel beats the k-major one by more than
+        # the transpose costs.
         if _weight_in_place(c2, w):
             dx = gemm(c2, w, False, False, ax).reshape(x.shape)
         else:
@@ -797,17 +800,22 @@ def ffn(xb, w1, w3, w2, residual=None):
             dw2 = target
         else:
             dw2 = gemm(c2, g, True, False, acc[3])
-        # (dh1, dh3) = SwiGLU adjoint of dY . W2, in the epilogue of that product
+        # (dh1, dh3) = SwiGLU adjoint of dY . W2, in the epilogue of that product where it has one
         dh1, dh3 = torch.empty_like(h1), torch.empty_like(h3)
-        nbytes = lib.emi_gemm_swiglu_bwd_workspace_bytes(T, Hn, K, _code(c2))
-        one_launch = T % 256 == 0 and Hn % 256 == 0 and (T // 256) * (Hn // 256) >= 192      # else dY . W2 goes through a workspace
-        ws = None if one_launch else torch.empty(nbytes, dtype=torch.uint8, device=c2.device)
-        N.check(lib.emi_gemm_swiglu_bwd(_stream(), _p(c2), _p(_transpose_shared(w2)), _p(h1), _p(h3), _p(dh1), _p(dh3), _p(ws),
-                                        nbytes if ws is not None else 0, T, Hn, K, _code(c2)))
+        one_launch = T % 256 == 0 and Hn % 256 == 0 and (T // 256) * (Hn // 256) >= 192
+        in_place = _weight_in_place(c2, w2) and not one_launch
+        if in_place:
+            dg = gemm(c2, w2, False, False)
+            N.check(lib.emi_swiglu_bwd(_stream(), _p(h1), _p(h3), _p(dg), _p(dh1), _p(dh3), h1.numel(), _code(c2)))
+        else:
+            nbytes = lib.emi_gemm_swiglu_bwd_workspace_bytes(T, Hn, K, _code(c2))
+            ws = None if one_launch else torch.empty(nbytes, dtype=torch.uint8, device=c2.device)
+            N.check(lib.emi_gemm_swiglu_bwd(_stream(), _p(c2), _p(_transpose_shared(w2)), _p(h1), _p(h3), _p(dh1), _p(dh3), _p(ws),
+                                            nbytes if ws is not None else 0, T, Hn, K, _code(c2)))
         # the group's rule: dX summed over the two branches, dW1 / dW3 grouped or deferred
         ax = None if acc[0] is None else acc[0].reshape(-1, K)
-        dx = gemm_grouped([dh1, dh3], [_transpose_shared(w1), _transpose_shared(w3)], False, True, None if ax is None else [ax],
-                          sum_into_one=True).reshape(xb.shape)
+        wb = [w1, w3] if in_place else [_transpose_shared(w1), _transpose_shared(w3)]
+        dx = gemm_grouped([dh1, dh3], wb, False, not in_place, None if ax is None else [ax], sum_into_one=True).reshape(xb.shape)
         t1, t3 = _grad_target(w1, acc[1]), _grad_target(w3, acc[2])
         if t1 is not None and t3 is not None:
             _defer_dw(dh1, x2, t1)
