@@ -18,7 +18,7 @@ OBJDIR = os.path.join(LIBDIR, "obj")
 
 HIP_SOURCES = ["elementwise.hip", "gemm.hip", "gemm_f32.hip", "gemm_bf16_pipe.hip", "gemm_skinny.hip", "attention.hip", "attention_f32.hip", "attention_step.hip", "llama_step.hip", "forward_mode.hip",
                "tensor_ops.hip", "cross_entropy.hip"]
-CXX_SOURCES = ["status.cc", "ffi_handlers.cc"]
+CXX_SOURCES = ["status.cc", "ffi_handlers.cc", "llama_layers.cc"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-I", os.path.join(os.path.dirname(HERE), "include")]

@@ -1,0 +1,348 @@
+// Decoder layers over whole sequences (test/llama.py:144-233, batched and causal) as one call each way: forward through L
+// layers whose weights are stacked, and the reverse pass with every gradient.
+//
+// No kernel of its own: it issues the launchers of emi.h in the order in which ops.attention_block, ops.ffn and their rules
+// do.  A layer is nine to twelve launches forward and about twenty in reverse, and a small model's are 3 to 10 us each, less
+// than a Python operator costs: the dim-288 model on 256 tokens spent 2.6 ms on the host for 1.25 ms of kernels.
+// In reverse the weight gradients dW = dY^T X feed nothing else, so they wait until `group` layers are done and run grouped
+// by shape (q, k, v, o; w1, w3; w2), which fills the chip where one layer's would not; a group of one runs them in place.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "../../include/emi.h"
+
+extern "C" int emi_fail(int code, const char* fmt, ...);
+
+namespace {
+
+enum { kAtt, kQ, kK, kV, kO, kFfn, kW1, kW2, kW3, kWeights };      // the order of the stacked weights
+
+struct Dims {
+  int64_t L, B, S, D, H, heads;
+  float eps, scale;
+  int dtype;
+  int64_t T() const { return B * S; }
+  int64_t hd() const { return D / heads; }
+  size_t elt() const { return dtype == EMI_BF16 ? 2 : 4; }
+  bool ok() const {
+    return L > 0 && B > 0 && S > 0 && D > 0 && H > 0 && heads > 0 && D % heads == 0 && hd() % 2 == 0 && D % 8 == 0 && H % 8 == 0 &&
+           (dtype == EMI_F32 || dtype == EMI_BF16) && T() > 8;
+  }
+  bool tiles(int64_t n) const { return T() % 256 == 0 && n % 256 == 0 && (T() / 256) * (n / 256) >= 192; }
+  // the kernels with RoPE in their epilogues (ops.attention_block)
+  bool rope_attention() const { return dtype == EMI_BF16 && (hd() == 64 || hd() == 128) && S >= 128; }
+  bool rope_projection() const { return rope_attention() && tiles(D); }
+  bool swiglu_epilogue() const { return dtype == EMI_BF16 && T() >= 256; }
+};
+
+struct Carve {                                            // consecutive 256-byte aligned pieces of a buffer
+  uint8_t* base;
+  size_t at;
+  void* take(size_t bytes) {
+    void* p = base + at;
+    at += (bytes + 255) / 256 * 256;
+    return p;
+  }
+};
+inline void* part(void* p, size_t bytes) { return static_cast<uint8_t*>(p) + bytes; }
+inline const void* part(const void* p, size_t bytes) { return static_cast<const uint8_t*>(p) + bytes; }
+
+struct Saved {                                            // of one layer
+  void *xb1, *q, *k, *v, *att, *x1, *xb2, *h1, *h3, *g, *out;
+  float* lse;
+};
+Saved carve_saved(void* base, const Dims& d, size_t* bytes = nullptr) {
+  Carve c{static_cast<uint8_t*>(base), 0};
+  const size_t td = (size_t)d.T() * d.D * d.elt(), th = (size_t)d.T() * d.H * d.elt();
+  Saved s;
+  s.xb1 = c.take(td);
+  s.q = c.take(3 * td);                                   // side by side: q and k are rotated by one launch
+  s.k = part(s.q, td);
+  s.v = part(s.q, 2 * td);
+  s.att = c.take(td);
+  s.x1 = c.take(td);
+  s.xb2 = c.take(td);
+  s.h1 = c.take(th);
+  s.h3 = c.take(th);
+  s.g = c.take(th);
+  s.out = c.take(td);
+  s.lse = static_cast<float*>(c.take((size_t)d.B * d.heads * d.S * sizeof(float)));
+  if (bytes != nullptr) *bytes = c.at;
+  return s;
+}
+
+struct Cots {                                             // cotangents of one layer
+  void *dq, *dk, *dv, *dx1, *dh1, *dh3, *dx;
+};
+Cots carve_cots(void* base, const Dims& d, size_t* bytes = nullptr) {
+  Carve c{static_cast<uint8_t*>(base), 0};
+  const size_t td = (size_t)d.T() * d.D * d.elt(), th = (size_t)d.T() * d.H * d.elt();
+  Cots s;
+  s.dq = c.take(3 * td);
+  s.dk = part(s.dq, td);
+  s.dv = part(s.dq, 2 * td);
+  s.dx1 = c.take(td);
+  s.dh1 = c.take(th);
+  s.dh3 = c.take(th);
+  s.dx = c.take(td);
+  if (bytes != nullptr) *bytes = c.at;
+  return s;
+}
+
+size_t most(std::initializer_list<size_t> v) {
+  size_t m = 0;
+  for (size_t x : v)
+    if (x > m) m = x;
+  return m;
+}
+
+size_t forward_scratch(const Dims& d) {
+  const int64_t T = d.T();
+  return most({emi_gemm_grouped_workspace_bytes(3, T, d.D, d.D, 0, 1, 0, d.dtype), emi_gemm_grouped_workspace_bytes(2, T, d.H, d.D, 0, 1, 0, d.dtype),
+               emi_gemm_workspace_bytes(T, d.D, d.D, 0, 1, d.dtype), emi_gemm_workspace_bytes(T, d.H, d.D, 0, 1, d.dtype),
+               emi_gemm_workspace_bytes(T, d.D, d.H, 0, 1, d.dtype)});
+}
+
+struct ReverseScratch {
+  void *dxb, *dg, *ws;
+  size_t ws_bytes;
+};
+ReverseScratch carve_reverse(void* base, const Dims& d, int group, int transposed, size_t* bytes) {
+  Carve c{static_cast<uint8_t*>(base), 0};
+  const int64_t T = d.T();
+  ReverseScratch s;
+  s.dxb = c.take((size_t)T * d.D * d.elt());
+  s.dg = c.take((size_t)T * d.H * d.elt());
+  const int tb = transposed;
+  int m4 = 4 * group, m2 = 2 * group, m1 = group;
+  if (m4 > 48) m4 = 48;
+  if (m2 > 48) m2 = 48;
+  if (m1 > 48) m1 = 48;
+  size_t need = most({emi_gemm_workspace_bytes(T, d.H, d.D, 0, tb, d.dtype), emi_gemm_workspace_bytes(T, d.D, d.D, 0, tb, d.dtype),
+                      emi_gemm_grouped_workspace_bytes(2, T, d.D, d.H, 0, tb, 1, d.dtype),
+                      emi_gemm_grouped_workspace_bytes(3, T, d.D, d.D, 0, tb, 1, d.dtype), emi_rmsnorm_bwd_workspace_bytes(T, d.D),
+                      emi_attn_bwd_workspace_bytes(d.B, d.heads, d.S, d.hd())});
+  for (int i = 1; i <= m4; i++) need = most({need, emi_gemm_grouped_workspace_bytes(i, d.D, d.D, T, 1, 0, 0, d.dtype)});
+  for (int i = 1; i <= m2; i++) need = most({need, emi_gemm_grouped_workspace_bytes(i, d.H, d.D, T, 1, 0, 0, d.dtype)});
+  for (int i = 1; i <= m1; i++) need = most({need, emi_gemm_grouped_workspace_bytes(i, d.D, d.H, T, 1, 0, 0, d.dtype)});
+  s.ws_bytes = need;
+  s.ws = c.take(need);
+  if (bytes != nullptr) *bytes = c.at;
+  return s;
+}
+
+#define EMI_TRY(call)            \
+  do {                           \
+    if (int rc__ = (call)) return rc__; \
+  } while (0)
+
+int forward_layer(emi_stream_t st, const void* const* w, const void* x, const float* table, const Saved& s, void* out, void* ws, size_t wsb,
+                  const Dims& d) {
+  const int64_t T = d.T(), D = d.D, H = d.H;
+  EMI_TRY(emi_rmsnorm_fwd(st, x, w[kAtt], s.xb1, T, D, d.eps, d.dtype));
+  if (d.rope_projection()) {
+    EMI_TRY(emi_gemm_rope(st, s.xb1, w[kQ], s.q, table, T, D, D, d.S, d.hd(), d.dtype));
+    EMI_TRY(emi_gemm_rope(st, s.xb1, w[kK], s.k, table, T, D, D, d.S, d.hd(), d.dtype));
+    EMI_TRY(emi_gemm_ws(st, s.xb1, w[kV], nullptr, s.v, ws, wsb, T, D, D, D, D, D, D, 0, 1, d.dtype));
+  } else {
+    const void *a[3] = {s.xb1, s.xb1, s.xb1}, *b[3] = {w[kQ], w[kK], w[kV]};
+    void* c[3] = {s.q, s.k, s.v};
+    EMI_TRY(emi_gemm_grouped(st, 3, a, b, nullptr, c, ws, wsb, T, D, D, D, D, D, D, 0, 1, 0, d.dtype));
+    EMI_TRY(emi_rope(st, s.q, table, s.q, 2 * d.B, d.S, d.heads, d.hd(), 0, d.dtype));
+  }
+  EMI_TRY(emi_attn_fwd(st, s.q, s.k, s.v, s.att, s.lse, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
+  EMI_TRY(emi_gemm_ws(st, s.att, w[kO], x, s.x1, ws, wsb, T, D, D, D, D, D, D, 0, 1, d.dtype));
+  EMI_TRY(emi_rmsnorm_fwd(st, s.x1, w[kFfn], s.xb2, T, D, d.eps, d.dtype));
+  if (d.swiglu_epilogue()) {
+    EMI_TRY(emi_gemm_ws(st, s.xb2, w[kW1], nullptr, s.h1, ws, wsb, T, H, D, D, D, H, H, 0, 1, d.dtype));
+    EMI_TRY(emi_gemm_swiglu_fwd(st, s.xb2, w[kW3], s.h1, s.h3, s.g, T, H, D, d.dtype));
+  } else {
+    const void *a[2] = {s.xb2, s.xb2}, *b[2] = {w[kW1], w[kW3]};
+    void* c[2] = {s.h1, s.h3};
+    EMI_TRY(emi_gemm_grouped(st, 2, a, b, nullptr, c, ws, wsb, T, H, D, D, D, H, H, 0, 1, 0, d.dtype));
+    EMI_TRY(emi_swiglu_fwd(st, s.h1, s.h3, s.g, T * H, d.dtype));
+  }
+  return emi_gemm_ws(st, s.g, w[kW2], s.x1, out, ws, wsb, T, D, H, H, H, D, D, 0, 1, d.dtype);
+}
+
+// dW = dY^T X of one shape, waiting to run as one launch.
+struct Pending {
+  const void *a[48], *b[48];
+  void* c[48];
+  int n = 0;
+};
+int flush(emi_stream_t st, Pending& p, int64_t M, int64_t N, int64_t T, const ReverseScratch& r, int dtype) {
+  if (p.n == 0) return EMI_OK;
+  const int n = p.n;
+  p.n = 0;
+  if (n == 1) return emi_gemm_ws(st, p.a[0], p.b[0], nullptr, p.c[0], r.ws, r.ws_bytes, M, N, T, M, N, N, N, 1, 0, dtype);
+  return emi_gemm_grouped(st, n, p.a, p.b, nullptr, p.c, r.ws, r.ws_bytes, M, N, T, M, N, N, N, 1, 0, 0, dtype);
+}
+int wait(emi_stream_t st, Pending& p, const void* dy, const void* x, void* dw, int64_t M, int64_t N, int64_t T, const ReverseScratch& r,
+         int dtype) {
+  if (p.n == 48) EMI_TRY(flush(st, p, M, N, T, r, dtype));
+  p.a[p.n] = dy;
+  p.b[p.n] = x;
+  p.c[p.n++] = dw;
+  return EMI_OK;
+}
+
+int check_layers(const char* name, const Dims& d, const void* const* w, std::initializer_list<const void*> ptrs) {
+  if (!d.ok())
+    return emi_fail(EMI_INVALID_ARGUMENT, "%s: unsupported shape (layers=%lld batch=%lld seq=%lld dim=%lld hidden=%lld heads=%lld dtype=%d)", name,
+                    (long long)d.L, (long long)d.B, (long long)d.S, (long long)d.D, (long long)d.H, (long long)d.heads, d.dtype);
+  if (w == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "%s: null weight table", name);
+  for (int i = 0; i < kWeights; i++)
+    if (w[i] == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "%s: weight %d is null", name, i);
+  for (const void* p : ptrs)
+    if (p == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "%s: null buffer", name);
+  return EMI_OK;
+}
+
+size_t weight_elements(int i, const Dims& d) {            // of one layer
+  switch (i) {
+    case kAtt: case kFfn: return (size_t)d.D;
+    case kW1: case kW2: case kW3: return (size_t)d.D * d.H;
+    default: return (size_t)d.D * d.D;
+  }
+}
+
+}  // namespace
+
+extern "C" size_t emi_llama_layers_saved_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype) {
+  const Dims d{1, batch, seq, dim, hidden, heads, 0.f, 0.f, dtype};
+  if (!d.ok()) return 0;
+  size_t n = 0;
+  carve_saved(nullptr, d, &n);
+  return n;
+}
+
+extern "C" size_t emi_llama_layers_fwd_workspace_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype) {
+  const Dims d{1, batch, seq, dim, hidden, heads, 0.f, 0.f, dtype};
+  return d.ok() ? forward_scratch(d) : 0;
+}
+
+extern "C" size_t emi_llama_layers_cotangent_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype) {
+  const Dims d{1, batch, seq, dim, hidden, heads, 0.f, 0.f, dtype};
+  if (!d.ok()) return 0;
+  size_t n = 0;
+  carve_cots(nullptr, d, &n);
+  return n;
+}
+
+extern "C" size_t emi_llama_layers_bwd_workspace_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int group,
+                                                       int transposed, int dtype) {
+  const Dims d{1, batch, seq, dim, hidden, heads, 0.f, 0.f, dtype};
+  if (!d.ok() || group < 1) return 0;
+  size_t n = 0;
+  carve_reverse(nullptr, d, group, transposed, &n);
+  return n;
+}
+
+extern "C" int emi_llama_layers_fwd(emi_stream_t stream, const void* const* weights, const void* x, const float* rope_table, void* y,
+                                    void* const* saved, int keep, void* workspace, size_t workspace_bytes, int64_t layers, int64_t batch,
+                                    int64_t seq, int64_t dim, int64_t hidden, int64_t heads, float eps, float scale, int dtype) {
+  const Dims d{layers, batch, seq, dim, hidden, heads, eps, scale, dtype};
+  if (int rc = check_layers("emi_llama_layers_fwd", d, weights, {x, rope_table, y, saved})) return rc;
+  const size_t need = forward_scratch(d);
+  if (need && (workspace == nullptr || workspace_bytes < need))
+    return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_fwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+  for (int64_t l = 0; l < layers; l++) {
+    const void* w[kWeights];
+    for (int i = 0; i < kWeights; i++) w[i] = part(weights[i], weight_elements(i, d) * (size_t)l * d.elt());
+    void* buffer = saved[keep ? l : 0];
+    if (buffer == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_fwd: null buffer for layer %lld", (long long)l);
+    const Saved s = carve_saved(buffer, d);
+    void* out = l + 1 < layers ? s.out : y;
+    EMI_TRY(forward_layer(stream, w, x, rope_table, s, out, workspace, workspace_bytes, d));
+    x = out;
+  }
+  return EMI_OK;
+}
+
+extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weights, void* const* transposed, const void* x,
+                                    const float* rope_table, void* const* saved, const void* dy, const void* dx_add, void* dx,
+                                    void* const* grads, void* const* cotangents, int group, void* workspace, size_t workspace_bytes,
+                                    int64_t layers, int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, float eps,
+                                    float scale, int dtype) {
+  const Dims d{layers, batch, seq, dim, hidden, heads, eps, scale, dtype};
+  if (int rc = check_layers("emi_llama_layers_bwd", d, weights, {x, rope_table, saved, dy, dx, grads, cotangents, workspace})) return rc;
+  if (group < 1) return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_bwd: group %d", group);
+  for (int i = 0; i < kWeights; i++)
+    if (grads[i] == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_bwd: gradient %d is null", i);
+  size_t need = 0;
+  const ReverseScratch r = carve_reverse(workspace, d, group, transposed != nullptr, &need);
+  if (workspace_bytes < need)
+    return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_bwd: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+  const int64_t T = d.T(), D = d.D, H = d.H;
+  const int tb = transposed != nullptr;                   // dX = dY . W as NT on W^T, or NN on W as stored
+  if (tb)
+    for (int i : {kQ, kK, kV, kO, kW1, kW2, kW3}) {       // every layer's transpose by one launch per stack
+      if (transposed[i] == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_bwd: no room for transpose %d", i);
+      const int64_t rows = i == kW1 || i == kW3 ? H : D, cols = i == kW2 ? H : D;
+      const int64_t out[3] = {layers, cols, rows}, ss[3] = {rows * cols, 1, cols}, ds[3] = {rows * cols, rows, 1};
+      EMI_TRY(layers == 1 ? emi_transpose(stream, weights[i], transposed[i], rows, cols, dtype)
+                          : emi_strided_copy(stream, weights[i], transposed[i], 3, out, ss, 0, ds, 0, (int)d.elt()));
+    }
+  Pending sq, up, down;                                   // [D, D], [H, D], [D, H]
+  const int64_t hd = d.hd();
+  for (int64_t l = layers - 1; l >= 0; l--) {
+    const void *w[kWeights], *b[kWeights];
+    void* g[kWeights];
+    for (int i = 0; i < kWeights; i++) {
+      const size_t off = weight_elements(i, d) * (size_t)l * d.elt();
+      w[i] = part(weights[i], off);
+      b[i] = tb && transposed[i] != nullptr ? part(static_cast<const void*>(transposed[i]), off) : w[i];
+      g[i] = part(grads[i], off);
+    }
+    const Saved s = carve_saved(saved[l], d);
+    const int64_t done = layers - 1 - l;
+    const Cots c = carve_cots(cotangents[done % group], d);
+    const void* x_l = l == 0 ? x : carve_saved(saved[l - 1], d).out;
+    EMI_TRY(wait(stream, down, dy, s.g, g[kW2], D, H, T, r, dtype));
+    if (group == 1) EMI_TRY(flush(stream, down, D, H, T, r, dtype));        // dy's place is taken by this layer's dx below
+    if (tb && d.swiglu_epilogue()) {
+      EMI_TRY(emi_gemm_swiglu_bwd(stream, dy, b[kW2], s.h1, s.h3, c.dh1, c.dh3, r.dg, (size_t)T * H * d.elt(), T, H, D, dtype));
+    } else {
+      EMI_TRY(emi_gemm_ws(stream, dy, b[kW2], nullptr, r.dg, r.ws, r.ws_bytes, T, H, D, D, tb ? D : H, H, H, 0, tb, dtype));
+      EMI_TRY(emi_swiglu_bwd(stream, s.h1, s.h3, r.dg, c.dh1, c.dh3, T * H, dtype));
+    }
+    {
+      const void *a2[2] = {c.dh1, c.dh3}, *b2[2] = {b[kW1], b[kW3]};
+      void* out[1] = {r.dxb};
+      EMI_TRY(emi_gemm_grouped(stream, 2, a2, b2, nullptr, out, r.ws, r.ws_bytes, T, D, H, H, tb ? H : D, D, D, 0, tb, 1, dtype));
+    }
+    EMI_TRY(emi_rmsnorm_bwd(stream, s.x1, w[kFfn], r.dxb, dy, c.dx1, g[kFfn], r.ws, r.ws_bytes, T, D, d.eps, dtype));
+    EMI_TRY(emi_gemm_ws(stream, c.dx1, b[kO], nullptr, r.dxb, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, dtype));
+    if (d.rope_attention()) {
+      EMI_TRY(emi_attn_bwd_rope(stream, s.q, s.k, s.v, s.att, s.lse, r.dxb, c.dq, c.dk, c.dv, rope_table, r.ws, r.ws_bytes, d.B, d.heads, d.S, hd,
+                                d.S * D, hd, D, d.scale, 1, dtype));
+    } else {
+      EMI_TRY(emi_attn_bwd(stream, s.q, s.k, s.v, s.att, s.lse, r.dxb, c.dq, c.dk, c.dv, r.ws, r.ws_bytes, d.B, d.heads, d.S, hd, d.S * D, hd, D,
+                           d.scale, 1, dtype));
+      EMI_TRY(emi_rope(stream, c.dq, rope_table, c.dq, 2 * d.B, d.S, d.heads, hd, 1, dtype));
+    }
+    {
+      const void *a3[3] = {c.dq, c.dk, c.dv}, *b3[3] = {b[kQ], b[kK], b[kV]};
+      void* out[1] = {r.dxb};
+      EMI_TRY(emi_gemm_grouped(stream, 3, a3, b3, nullptr, out, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, 1, dtype));
+    }
+    // the first layer's cotangent leaves; a caller's accumulated one is added by its own launch
+    void* dx_l = l == 0 ? dx : c.dx;
+    EMI_TRY(emi_rmsnorm_bwd(stream, x_l, w[kAtt], r.dxb, c.dx1, dx_l, g[kAtt], r.ws, r.ws_bytes, T, D, d.eps, dtype));
+    if (l == 0 && dx_add != nullptr) EMI_TRY(emi_add(stream, dx, dx_add, dx, T * D, dtype));
+    EMI_TRY(wait(stream, sq, c.dq, s.xb1, g[kQ], D, D, T, r, dtype));
+    EMI_TRY(wait(stream, sq, c.dk, s.xb1, g[kK], D, D, T, r, dtype));
+    EMI_TRY(wait(stream, sq, c.dv, s.xb1, g[kV], D, D, T, r, dtype));
+    EMI_TRY(wait(stream, sq, c.dx1, s.att, g[kO], D, D, T, r, dtype));
+    EMI_TRY(wait(stream, up, c.dh1, s.xb2, g[kW1], H, D, T, r, dtype));
+    EMI_TRY(wait(stream, up, c.dh3, s.xb2, g[kW3], H, D, T, r, dtype));
+    if ((done + 1) % group == 0 || l == 0) {
+      EMI_TRY(flush(stream, sq, D, D, T, r, dtype));
+      EMI_TRY(flush(stream, up, H, D, T, r, dtype));
+      EMI_TRY(flush(stream, down, D, H, T, r, dtype));
+    }
+    dy = dx_l;
+  }
+  return EMI_OK;
+}

@@ -1157,6 +1157,73 @@ def llama_step(x, weights, key_cache, value_cache, n_heads, table, eps=1e-5, sca
     return y
 
 
+def llama_layers_apply(x, weights, n_heads):
+    """Whether `llama_layers` serves these operands (else a layer runs operator by operator): reverse or no
+    differentiation, one dtype, contiguous aligned stacks, rows of whole 16-byte pieces, more than a few tokens."""
+    if Forward._active is not None or x.dim() != 3 or x.dtype not in _DTYPES:
+        return False
+    w1 = weights[6]
+    stack = w1.shape[:-2]
+    if w1.dim() not in (2, 3):
+        return False
+    B, S, D = x.shape
+    H = w1.shape[-2]
+    sq, up, down, row = stack + (D, D), stack + (H, D), stack + (D, H), stack + (D,)
+    for t, s in zip((x, *weights), (x.shape, row, sq, sq, sq, sq, row, up, down, up)):
+        if t.shape != s or t.dtype != x.dtype or not t.is_contiguous() or t.data_ptr() & 15 or not t.is_cuda:
+            return False
+    return N.lib().emi_llama_layers_saved_bytes(B, S, D, H, n_heads, _code(x)) != 0
+
+
+def llama_layers(x, weights, n_heads, table, eps=1e-5, scale=None):
+    """The decoder layers of test/llama.py:144-233 over x [B, S, dim] as one operator: `weights` in the order of
+    llama.LAYER_KEYS, each stacked over the layers (or, for one layer, not stacked), `table` the fp32 (cos, sin)
+    [S, head_dim/2, 2].  The launches, values and gradients of rmsnorm, attention_block, matmul_nt and ffn per layer
+    (emi_llama_layers_fwd / _bwd issue them natively); weight gradients of one shape run grouped over as many layers as
+    _PENDING_DW_BYTES of cotangents allow."""
+    weights = list(weights)
+    _dev(x, *weights, table)
+    B, S, D = x.shape
+    L_, H = (weights[6].shape[0] if weights[6].dim() == 3 else 1), weights[6].shape[-2]
+    lib, code = N.lib(), _code(x)
+    if scale is None:
+        scale = 1.0 / math.sqrt(D // n_heads)
+    shape = (B, S, D, H, n_heads)
+    dims = (L_,) + shape + (eps, float(scale), code)
+    nsaved = lib.emi_llama_layers_saved_bytes(*shape, code)
+    keep = Tape._active is not None
+    saved = [torch.empty(nsaved, dtype=torch.uint8, device=x.device) for _ in range(L_ if keep else 1)]
+    nws = lib.emi_llama_layers_fwd_workspace_bytes(*shape, code)
+    ws = torch.empty(nws, dtype=torch.uint8, device=x.device) if nws else None
+    y = torch.empty_like(x)
+    N.check(lib.emi_llama_layers_fwd(_stream(), _ptr_table(weights), _p(x), _p(table), _p(y), _ptr_table(saved), int(keep), _p(ws), nws, *dims))
+
+    def rule(c, acc):
+        c = c.contiguous()
+        T = B * S
+        grads, out = [], []
+        for w, a in zip(weights, acc[1:]):
+            t = _grad_target(w, a)
+            grads.append(torch.empty_like(w) if t is None else t)
+        # transposed weights where dX = dY . W is k-contiguous (see _weight_in_place), and for the SwiGLU adjoint's epilogue
+        epilogue = T % 256 == 0 and H % 256 == 0 and (T // 256) * (H // 256) >= 192
+        turn = x.dtype == torch.bfloat16 and (epilogue or not _weight_in_place(x.reshape(T, D), weights[1]))
+        wt = [torch.empty_like(w) if turn and w.dim() == weights[6].dim() else None for w in weights]
+        nct = lib.emi_llama_layers_cotangent_bytes(*shape, code)
+        # a stack whose products fill the chip one by one gains nothing from waiting
+        group = 1 if ((D + 255) // 256) ** 2 >= 192 else max(1, min(L_, _PENDING_DW_BYTES // nct))
+        cts = [torch.empty(nct, dtype=torch.uint8, device=x.device) for _ in range(group)]
+        nb = lib.emi_llama_layers_bwd_workspace_bytes(*shape, group, int(turn), code)
+        work = torch.empty(nb, dtype=torch.uint8, device=x.device)
+        dx = torch.empty_like(x)
+        N.check(lib.emi_llama_layers_bwd(_stream(), _ptr_table(weights), _ptr_table(wt) if turn else None, _p(x), _p(table), _ptr_table(saved),
+                                         _p(c), _p(acc[0]), _p(dx), _ptr_table(grads), _ptr_table(cts), group, _p(work), nb, *dims))
+        return [dx] + [_accumulate(a, g) for a, g in zip(acc[1:], grads)]
+
+    Tape.record((x, *weights), y, rule)
+    return y
+
+
 def embedding(tokens, table):
     """table[tokens] (the lookup commented out at test/llama.py:109-113)."""
     _dev(tokens, table)

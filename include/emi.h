@@ -279,6 +279,31 @@ int emi_llama_step_bwd(emi_stream_t stream, const void* const* weights, const vo
                        const void* dy, void* const* grads, void* workspace, size_t workspace_bytes, int64_t layers,
                        int64_t dim, int64_t hidden, int64_t heads, int64_t pos, float eps, float scale, int dtype);
 
+/* `layers` decoder layers of test/llama.py:144-233 over whole sequences, forward and reverse, one
+ * call each.  weights: nine arrays, per-layer ones stacked: rms_att_weight[L, D], wq, wk, wv,
+ * wo[L, D, D], rms_ffn_weight[L, D], w1[L, H, D], w2[L, D, H], w3[L, H, D]; x, y[B, S, D];
+ * rope_table: fp32 (cos, sin) [S, head_dim / 2].  saved: a buffer of emi_llama_layers_saved_bytes
+ * per layer, or with keep == 0 one for all of them (no reverse pass follows).
+ * Reverse: grads are the nine weights' (all written), dx the input's cotangent, plus dx_add unless
+ * null.  The weight gradients wait until `group` layers are done and run grouped by shape;
+ * cotangents: `group` buffers of emi_llama_layers_cotangent_bytes.  transposed: null (the adjoint
+ * products read the weights in place), or room for the transposes of the seven matrices' stacks
+ * (entries 0 and 5 unused).  emi_llama_layers_saved_bytes is 0 for shapes the calls do not take
+ * (dim and hidden multiples of 8, an even head_dim, more than 8 tokens). */
+size_t emi_llama_layers_saved_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype);
+size_t emi_llama_layers_fwd_workspace_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype);
+size_t emi_llama_layers_cotangent_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype);
+size_t emi_llama_layers_bwd_workspace_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int group,
+                                            int transposed, int dtype);
+int emi_llama_layers_fwd(emi_stream_t stream, const void* const* weights, const void* x, const float* rope_table, void* y,
+                         void* const* saved, int keep, void* workspace, size_t workspace_bytes, int64_t layers, int64_t batch,
+                         int64_t seq, int64_t dim, int64_t hidden, int64_t heads, float eps, float scale, int dtype);
+int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weights, void* const* transposed, const void* x,
+                         const float* rope_table, void* const* saved, const void* dy, const void* dx_add, void* dx,
+                         void* const* grads, void* const* cotangents, int group, void* workspace, size_t workspace_bytes,
+                         int64_t layers, int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, float eps,
+                         float scale, int dtype);
+
 /* Forward mode of the single-token attention (emi_attn_step_fwd's layout, o and lse from
  * it): to = sum_s p_s (tS_s v_s + tv_s) - (sum_s p_s tS_s) o with tS_s = scale (tq.k_s + q.tk_s).
  * Null tq / tk / tv = zero tangent.  workspace: emi_attn_step_workspace_bytes(). */
