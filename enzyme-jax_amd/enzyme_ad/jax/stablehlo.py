@@ -1107,6 +1107,85 @@ def _fuse_step(run_ops, func):
     return new[::-1]
 
 
+def _fuse_layers(run_ops, func):
+    """Runs of whole decoder layers (rmsnorm_rows -> attention_block -> linear + residual -> rmsnorm_rows -> ffn + residual,
+    test/llama.py:144-233) as one `emi.llama_layers` each: all L layers on the slices of stacks of L, in order, or single
+    layers on whole weights; every interior value used only there.  attrs["parts"] keeps the operators, for operands that
+    ops.llama_layers does not take."""
+    rets = set(o for op in func.ops if op.name == "return" for o in op.operands)
+    use, producer = {}, {r: op for op in run_ops for r in op.results}
+    for op in run_ops:
+        for o in op.operands:
+            use.setdefault(o, []).append(op)
+
+    def made(value, name, n_operands, users):
+        op = producer.get(value)
+        if (op is None or op.name != name or len(op.operands) != n_operands or value in rets
+                or [id(u) for u in use.get(value, ())] != [id(u) for u in users]):
+            raise LookupError
+        return op
+
+    def layer(ffn):
+        x1 = ffn.operands[4]
+        norm2 = made(ffn.operands[0], "emi.rmsnorm_rows", 2, [ffn])
+        lo = made(x1, "emi.linear", 3, [norm2, ffn])
+        att = made(lo.operands[0], "emi.attention_block", 4, [lo])
+        norm1 = made(att.operands[0], "emi.rmsnorm_rows", 2, [att])
+        x = norm1.operands[0]
+        if norm2.operands[0] != x1 or lo.operands[2] != x or norm1.attrs["eps"] != norm2.attrs["eps"] or not att.attrs["causal"]:
+            raise LookupError
+        weights = [norm1.operands[1], *att.operands[1:], lo.operands[1], norm2.operands[1], ffn.operands[1], ffn.operands[3], ffn.operands[2]]
+        return x, weights, [norm1, att, lo, norm2, ffn], (norm1.attrs["eps"], att.attrs["scale"], att.attrs["heads"]), att.attrs["table"]
+
+    found = []
+    for op in run_ops:
+        if op.name == "emi.ffn" and len(op.operands) == 5:
+            try:
+                found.append(layer(op))
+            except LookupError:
+                pass
+    by_input = {f[0]: f for f in found}
+
+    def stacks(f, l):
+        sel = [producer.get(w) for w in f[1]]
+        if any(s is None or s.name != "emi.select" or s.attrs["index"] != l or len(use[s.results[0]]) != 1 for s in sel):
+            return None, None
+        return [s.operands[0] for s in sel], sel
+
+    shape = {a: t.shape for a, t in func.args}
+    gone, place = set(), {}
+    for f in found:
+        first, sel = stacks(f, 0)
+        if first is None:
+            if any(producer.get(w) is not None and producer[w].name == "emi.select" for w in f[1]):
+                continue
+            chain, weights, inside = [f], f[1], []
+        else:
+            chain, weights, inside = [f], first, list(sel)
+            while len(chain) < shape[first[0]][0]:
+                last = chain[-1]
+                out = last[2][-1].results[0]
+                nxt = by_input.get(out)
+                names, sel = stacks(nxt, len(chain)) if nxt is not None else (None, None)
+                # the result of a layer: the norm and the residual of the next
+                if names != first or nxt[3] != f[3] or not np.array_equal(nxt[4], f[4]) or out in rets or len(use[out]) != 2:
+                    chain = None
+                    break
+                chain.append(nxt)
+                inside += sel
+            if chain is None or any(shape.get(w, (0,))[0] != len(chain) for w in first):
+                continue
+        parts = [op for op in run_ops if id(op) in {id(o) for c in chain for o in c[2]} | {id(o) for o in inside}]
+        last = parts[-1]
+        eps, scale, heads = f[3]
+        place[id(last)] = Op("emi.llama_layers", last.results, [f[0]] + weights,
+                             {"eps": eps, "scale": scale, "heads": heads, "table": f[4], "parts": parts}, last.types)
+        gone.update(id(o) for o in parts if o is not last)
+    if not place:
+        return run_ops
+    return [place.get(id(op), op) for op in run_ops if id(op) not in gone]
+
+
 def _match_rmsnorm(op, d, tb):
     # root: a product of three factors, (w * x) * bcast(ss) or w * (x * bcast(ss)) in any
     # operand order, ss = 1 / sqrt(dot(x, x) / n + eps) or rsqrt(...)
@@ -1747,6 +1826,7 @@ class Executable:
         for f in self.funcs.values():
             f.run_ops = _fuse_blocks(_fold_selects(f), f) if fuse else f.ops
             f.step_ops = _fuse_step(f.run_ops, f) if fuse else None
+            f.layer_ops = _fuse_layers(f.run_ops, f) if fuse else f.ops
 
     def signature(self, fn="main"):
         f = self._func(fn)
@@ -1770,7 +1850,7 @@ class Executable:
         key = (id(op), "table", str(device))
         table = self._consts.get(key)
         if table is None:
-            table = self._consts[key] = torch.from_numpy(op.attrs["table"]).to(device)
+            table = self._consts[key] = torch.from_numpy(op.attrs["table"]).to(device).contiguous()
         return table
 
     def run(self, args, fn="main"):
@@ -1792,7 +1872,7 @@ class Executable:
             env[name] = a
         if device is None:
             device = torch.device("cuda", torch.cuda.current_device())
-        run_ops = getattr(f, "run_ops", f.ops)
+        run_ops = getattr(f, "layer_ops", f.ops)
         if getattr(f, "step_ops", None) is not None:
             step = next(op for op in f.step_ops if op.name == "emi.llama_step")
             xs = [env.get(o) for o in step.operands]
@@ -1801,17 +1881,27 @@ class Executable:
             as_printed = step.attrs["printed"] and ops.Tape._active is None
             if xs[0] is not None and not as_printed and ops.llama_step_applies(xs[0], xs[1:11], xs[11], xs[12], step.attrs["heads"]):
                 run_ops = f.step_ops
+        result = self._walk(f, run_ops, env, device)
+        if result is None:
+            raise ParseError("function %s has no return" % fn)
+        return result
+
+    def _walk(self, f, run_ops, env, device):
         for op in run_ops:
+            xs = [env[o] for o in op.operands]
             if op.name == "return":
-                return [env[o] for o in op.operands]
-            outs = self._apply(f, op, [env[o] for o in op.operands], device)
+                return xs
+            if op.name == "emi.llama_layers" and not ops.llama_layers_apply(xs[0], xs[1:], op.attrs["heads"]):
+                self._walk(f, op.attrs["parts"], env, device)
+                continue
+            outs = self._apply(f, op, xs, device)
             if len(outs) != len(op.results):
                 raise RuntimeError("%s produced %d values for %d results" % (op.name, len(outs), len(op.results)))
             for r, v, ty in zip(op.results, outs, op.types):
                 if v is not None and tuple(v.shape) != ty.shape:
                     raise RuntimeError("%s: result %s has shape %s, the text says %r" % (op.name, r, tuple(v.shape), ty))
                 env[r] = v
-        raise ParseError("function %s has no return" % fn)
+        return None
 
     def _apply(self, f, op, xs, device):
         n = op.name
@@ -1866,6 +1956,8 @@ class Executable:
             return [H.pad(xs[0], op.attrs["low"], op.attrs["high"], op.attrs["interior"], op.types[0].shape)]
         if n == "call":
             return self.run(xs, op.attrs["callee"])
+        if n == "emi.llama_layers":
+            return [ops.llama_layers(xs[0], xs[1:], op.attrs["heads"], self._table(op, device), op.attrs["eps"], op.attrs["scale"])]
         if n == "emi.llama_step":
             a = op.attrs
             y = ops.llama_step(xs[0], xs[1:11], xs[11], xs[12], a["heads"], self._table(op, device), a["eps"], a["scale"])
@@ -1884,13 +1976,9 @@ class Executable:
             x, w1, w3, w2 = (_packed(t) for t in xs[:4])
             return [ops.ffn(x, w1, w3, w2, residual=_packed(xs[4]) if len(xs) > 4 else None)]
         if n == "emi.attention_block":
-            key = (id(op), "table", str(device))
-            table = self._consts.get(key)
-            if table is None:
-                table = self._consts[key] = torch.from_numpy(op.attrs["table"]).to(device).contiguous()
             x, wq, wk, wv = (_packed(t) for t in xs)
             return [ops.attention_block(x, wq, wk, wv, op.attrs["heads"], scale=op.attrs["scale"], causal=op.attrs["causal"],
-                                        table=table)]
+                                        table=self._table(op, device))]
         if n == "emi.rmsnorm_rows":
             x, w = _packed(xs[0]), _packed(xs[1])
             return [ops.rmsnorm(x, w, op.attrs["eps"])]

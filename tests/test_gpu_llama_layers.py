@@ -1,0 +1,101 @@
+"""Decoder layers as one operator (ops.llama_layers): the value and every cotangent against the oracle's layers where its
+launches change - one layer and several, weight gradients grouped over the layers or not, weights read in place and turned,
+ragged token counts - from Python and from a program's text; and the operators it stands for, under forward mode."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import llama_ref as L
+from gpu_util import dev, check, rel_err, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(dt, dim, hidden, layers, heads, batch, seq):
+    cfg = dict(dim=dim, hidden_dim=hidden, n_layers=layers, n_heads=heads, n_kv_heads=heads, vocab_size=8, seq_len=seq)
+    rng = np.random.Generator(np.random.PCG64(dim + seq))
+    w = L.make_weights(cfg, dim + seq, std=1.0 / np.sqrt(dim), embedding=False, norm_gain="uniform")
+    wd, wr = {}, {}
+    for k, a in w.items():
+        if k not in ("wcls", "rms_final_weight"):
+            wd[k], wr[k] = dev(a, dt)
+    x, xr = dev(rng.standard_normal((batch, seq, dim)), dt)
+    dy, dyr = dev(rng.standard_normal((batch, seq, dim)), dt)
+    return cfg, wd, wr, x, xr, dy, dyr
+
+
+def _reference(xr, wr, dyr, layers, heads):
+    caches, h = [], xr
+    for i in range(layers):
+        h, cache = L.layer_fwd(h, L._layer_weights(wr, i), heads)
+        caches.append(cache)
+    d, grads = dyr, {k: np.zeros(v.shape) for k, v in wr.items()}
+    for i in reversed(range(layers)):
+        d, g = L.layer_bwd(d, L._layer_weights(wr, i), caches[i], heads)
+        for k in grads:
+            grads[k][i] = g[k]
+    return h, d, grads
+
+
+@pytest.mark.parametrize("dt,dim,hidden,layers,heads,batch,seq,pending", [
+    ("f32", 288, 768, 3, 6, 1, 9, None),
+    ("f32", 128, 264, 2, 2, 3, 77, 1),        # one layer's cotangents at a time
+    ("bf16", 128, 256, 3, 2, 2, 131, None),   # all layers in one group
+    ("bf16", 256, 264, 1, 2, 1, 640, None),
+    ("bf16", 128, 136, 2, 1, 4, 801, None),   # more tokens than are worth reading a weight in place for
+])
+def test_llama_layers_match_oracle(dt, dim, hidden, layers, heads, batch, seq, pending, monkeypatch):
+    from enzyme_ad.jax import llama, ops, vjp
+    if pending is not None:
+        monkeypatch.setattr(ops, "_PENDING_DW_BYTES", pending)
+    cfg, wd, wr, x, xr, dy, dyr = _inputs(dt, dim, hidden, layers, heads, batch, seq)
+    table = ops.rope_table(seq, dim // heads, device=x.device)
+    names = llama.LAYER_KEYS
+    assert ops.llama_layers_apply(x, [wd[k] for k in names], heads)
+
+    def f(x, w):
+        return ops.add(ops.llama_layers(x, [w[k] for k in names], heads, table), x)      # a second cotangent of x
+
+    y, pull = vjp(f, x, wd)
+    gx, gw = pull(dy)
+    ry, rdx, rgw = _reference(xr, wr, dyr, layers, heads)
+    check(y, ry + xr, dt, "y")
+    check(gx, rdx + dyr, dt, "dx")
+    for k in names:
+        check(gw[k], rgw[k], dt, "d" + k)
+    assert torch.equal(f(x, wd), y)           # without a tape one buffer serves all layers: the same bits
+
+
+def test_llama_layers_of_a_text():
+    """A program's text runs its layers as this operator and gives the bits of the model built in Python; under forward
+    mode it runs the operators the layers were made of."""
+    from enzyme_ad.jax import hlo_call, jvp, llama, stablehlo, vjp
+    from enzyme_ad.jax.llama_text import MODEL_ORDER, llama_model_text
+    cfg, wd, wr, x, xr, dy, _ = _inputs("f32", 96, 160, 2, 2, 1, 33)
+    cfg = dict(cfg, vocab_size=64)
+    rng = np.random.Generator(np.random.PCG64(5))
+    text, _ = llama_model_text(cfg, 1, 33, "f32", None)
+    w = dict(wd, rms_final_weight=dev(rng.uniform(0.5, 1.5, 96), "f32")[0], wcls=dev(rng.standard_normal((64, 96)) * 0.1, "f32")[0],
+             token_embedding_table=dev(rng.standard_normal((64, 96)), "f32")[0])
+    tokens = torch.from_numpy(rng.integers(0, 64, (1, 33)).astype(np.int32)).cuda()
+    exe = stablehlo.compile_text(text)
+    assert [o.name for o in exe.funcs["main"].layer_ops].count("emi.llama_layers") == 1
+    args = [w[k] for k in MODEL_ORDER]
+
+    def fn(*a):
+        return hlo_call(tokens, *a, source=text)[0]
+
+    got, pull = vjp(fn, *args)
+    c = dev(rng.standard_normal(tuple(got.shape)), "f32")[0]
+    ref, ref_pull = vjp(lambda w: llama.forward(tokens, cfg, w, logits=True), w)
+    assert rel_err(host(got), host(ref).reshape(got.shape)) < 1e-5      # the angles come from the text's constants
+    grads, (ref_grads,) = pull(c), ref_pull(c.reshape(ref.shape))
+    for k, g in zip(MODEL_ORDER, grads):
+        assert rel_err(host(g), host(ref_grads[k])) < 1e-4, k
+    tangents = [dev(rng.standard_normal(tuple(a.shape)) * 0.1, "f32")[0] for a in args]
+    value, tangent = jvp(fn, tuple(args), tuple(tangents))
+    assert rel_err(host(value), host(got)) < 1e-5
+    # <c, J t> = <J^T c, t>
+    a = float((c.double() * tangent.double()).sum())
+    b = sum(float((g.double() * t.double()).sum()) for g, t in zip(grads, tangents))
+    assert abs(a - b) <= 1e-4 * max(abs(a), float(c.double().norm() * tangent.double().norm()) * 1e-2)
