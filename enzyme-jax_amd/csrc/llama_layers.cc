@@ -300,7 +300,9 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     const Cots c = carve_cots(cotangents[done % group], d);
     const void* x_l = l == 0 ? x : carve_saved(saved[l - 1], d).out;
     EMI_TRY(wait(stream, down, dy, s.g, g[kW2], D, H, T, r, dtype));
-    if (group == 1) EMI_TRY(flush(stream, down, D, H, T, r, dtype));        // dy's place is taken by this layer's dx below
+    // the group's last layer writes its dx where the dy of the group's first one lies (the last slot's dx, of the group before)
+    const bool ends_group = (done + 1) % group == 0 || l == 0;
+    if (ends_group) EMI_TRY(flush(stream, down, D, H, T, r, dtype));
     if (tb && d.swiglu_epilogue()) {
       EMI_TRY(emi_gemm_swiglu_bwd(stream, dy, b[kW2], s.h1, s.h3, c.dh1, c.dh3, r.dg, (size_t)T * H * d.elt(), T, H, D, dtype));
     } else {
@@ -337,10 +339,9 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     EMI_TRY(wait(stream, sq, c.dx1, s.att, g[kO], D, D, T, r, dtype));
     EMI_TRY(wait(stream, up, c.dh1, s.xb2, g[kW1], H, D, T, r, dtype));
     EMI_TRY(wait(stream, up, c.dh3, s.xb2, g[kW3], H, D, T, r, dtype));
-    if ((done + 1) % group == 0 || l == 0) {
+    if (ends_group) {
       EMI_TRY(flush(stream, sq, D, D, T, r, dtype));
       EMI_TRY(flush(stream, up, H, D, T, r, dtype));
-      EMI_TRY(flush(stream, down, D, H, T, r, dtype));
     }
     dy = dx_l;
   }

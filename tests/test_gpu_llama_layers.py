@@ -38,6 +38,7 @@ def _reference(xr, wr, dyr, layers, heads):
 
 
 @pytest.mark.parametrize("dt,dim,hidden,layers,heads,batch,seq,pending", [
+    ("f32", 64, 72, 5, 2, 1, 33, 2),          # groups of two: the second one's first dy lies in the last slot of the first
     ("f32", 288, 768, 3, 6, 1, 9, None),
     ("f32", 128, 264, 2, 2, 3, 77, 1),        # one layer's cotangents at a time
     ("bf16", 128, 256, 3, 2, 2, 131, None),   # all layers in one group
@@ -46,9 +47,10 @@ def _reference(xr, wr, dyr, layers, heads):
 ])
 def test_llama_layers_match_oracle(dt, dim, hidden, layers, heads, batch, seq, pending, monkeypatch):
     from enzyme_ad.jax import llama, ops, vjp
-    if pending is not None:
-        monkeypatch.setattr(ops, "_PENDING_DW_BYTES", pending)
     cfg, wd, wr, x, xr, dy, dyr = _inputs(dt, dim, hidden, layers, heads, batch, seq)
+    if pending is not None:
+        layer_bytes = ops.N.lib().emi_llama_layers_cotangent_bytes(batch, seq, dim, hidden, heads, ops._code(x))
+        monkeypatch.setattr(ops, "_PENDING_DW_BYTES", pending * layer_bytes)
     table = ops.rope_table(seq, dim // heads, device=x.device)
     names = llama.LAYER_KEYS
     assert ops.llama_layers_apply(x, [wd[k] for k in names], heads)
