@@ -1488,9 +1488,9 @@ int launch_attn_jvp_mfma(hipStream_t st, const void* q, const void* k, const voi
 int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int64_t batch,
                              int64_t heads, int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale,
                              int causal);
-int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* d_o, const float* lse,
-                             const float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads, int64_t seq,
-                             int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal);
+int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                             const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
+                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal);
 
 }  // namespace emi
 
@@ -1624,15 +1624,7 @@ static int attn_bwd_impl(emi_stream_t stream, const void* q, const void* k, cons
   const dim3 grid4((unsigned)((seq + 3) / 4), bh);
   const bool fast = mfma_ok(a, dtype, {q, k, v, o, d_o, dq, dk, dv});
   const float delta_sign = -1.0f;          // the MFMA kernels accumulate dP onto -delta
-  if (fast) {
-    // the dQ kernel computes delta and lse * log2(e) for its own queries and leaves them for the dK/dV kernel
-  } else if (dtype == EMI_BF16)
-    hipLaunchKernelGGL(attn_delta_kernel<bf16>, grid4, dim3(256), 0, st, (const bf16*)o, (const bf16*)d_o, delta, shp,
-                       (int)head_dim);
-  else
-    hipLaunchKernelGGL(attn_delta_kernel<float>, grid4, dim3(256), 0, st, (const float*)o, (const float*)d_o, delta, shp,
-                       (int)head_dim);
-  EMI_CHECK_LAUNCH("emi_attn_bwd(delta)");
+  // on the matrix-core paths the dQ kernel computes delta (and lse * log2(e)) for its own queries and leaves them for dK/dV
   if (fast) {
     const uint32_t head_bytes = (uint32_t)(((seq - 1) * stride_s + head_dim) * 2);
     const dim3 grid((unsigned)((seq + 127) / 128), bh);
@@ -1657,10 +1649,17 @@ static int attn_bwd_impl(emi_stream_t stream, const void* q, const void* k, cons
     return EMI_OK;
   }
   if (dtype == EMI_F32) {
-    const int rc = launch_attn_bwd_f32_mfma(st, q, k, v, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, stride_b,
+    const int rc = launch_attn_bwd_f32_mfma(st, q, k, v, o, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, stride_b,
                                             stride_h, stride_s, scale, causal);
     if (rc >= 0) return rc;
   }
+  if (dtype == EMI_BF16)
+    hipLaunchKernelGGL(attn_delta_kernel<bf16>, grid4, dim3(256), 0, st, (const bf16*)o, (const bf16*)d_o, delta, shp,
+                       (int)head_dim);
+  else
+    hipLaunchKernelGGL(attn_delta_kernel<float>, grid4, dim3(256), 0, st, (const float*)o, (const float*)d_o, delta, shp,
+                       (int)head_dim);
+  EMI_CHECK_LAUNCH("emi_attn_bwd(delta)");
   const int vec4 = rows_vec4(dtype, head_dim, shp.sb, shp.sh, shp.ss, {q, k, v, d_o});
   if (dtype == EMI_BF16) {
     hipLaunchKernelGGL(attn_bwd_dq_generic_kernel<bf16>, grid4, dim3(256), 0, st, (const bf16*)q, (const bf16*)k,

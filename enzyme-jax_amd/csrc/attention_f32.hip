@@ -3,11 +3,17 @@
 // for head_dim a multiple of 16 up to 128 and rows that start on 16-byte boundaries.  Replaces the per-head
 // loop of test/llama.py:178-206 with the softmax of :13-18 for the fp32 configurations (stories15M: 6 heads x 48).
 //
-// One wavefront owns 16 queries (forward, dQ) or 16 keys (dK/dV) and walks the other sequence axis 64 rows
-// at a time; operands come straight from global memory (L1/L2 serve the reuse between wavefronts), so there is
-// no LDS and no barrier.  As on the bf16 path everything is computed transposed: the score tile is
-// S^T[other row, own row], so lane l owns row l % 16 for its whole life, its softmax statistics are per-lane
-// scalars, and the probabilities leave the accumulator already in the B-operand layout of the second product.
+// A block of four wavefronts owns 16 queries (forward, dQ) or 16 keys (dK/dV). The 16-row tiles of the other sequence axis
+// are dealt to the wavefronts in turn, each accumulates over its own tiles, and the four partial results are added
+// through the LDS at the end (the forward pass scales them to a common maximum first); that is the only barrier. Operands
+// come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
+// 16 rows are one chain of them, so with one wavefront per 16 rows (the earlier form) the longest row set the time and too
+// few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 24,
+// 24 heads x 1000 x 64 89 / 280 -> 56 / 161 (55 / 48 TFLOP/s), 64 heads x 2048 x 128 1329 / 4010 -> 795 / 2907 (86 / 59);
+// the loads of K, V and Q through the L1 come next.
+// As on the bf16 path everything is computed transposed: the score tile is S^T[other row, own row], so lane l owns row
+// l % 16 for its whole life, its softmax statistics are per-lane scalars, and the probabilities leave the accumulator
+// already in the B-operand layout of the second product.
 //
 // Operand layouts of v_mfma_f32_16x16x4_f32 (D = A . B, A 16x4, B 4x16): lane l supplies A[l % 16][l / 16] and
 // B[l / 16][l % 16]; register r of lane l receives D[4 (l / 16) + r][l % 16].  The contraction index of one
@@ -33,6 +39,7 @@ struct AttnShapeF32 {
 };
 
 constexpr float kMasked = -1.0e30f;
+constexpr int kWaves = 4;      // per block; merge_store deals the accumulator's four registers to them
 
 __device__ __forceinline__ f32q_t mfma_f32(float a, float b, f32q_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -65,31 +72,15 @@ __device__ __forceinline__ f32q_t rows_dot(const float (&x)[NT][4], const float 
 }
 
 // acc += X[row0 .. row0 + 15]^T . W, where w[t] of lane l is W[row0 + 4 (l / 16) + t][l % 16] (the layout rows_dot
-// leaves): acc[n][r] of lane l is output element (own row l % 16, column NT (4 (l / 16) + r) + n).
-template <int NT>
-__device__ __forceinline__ void add_cols(const float* __restrict__ head, int64_t ss, int row0, int last, int lane,
-                                         const f32q_t w, f32q_t (&acc)[NT]) {
-#pragma unroll
-  for (int t = 0; t < 4; t++) {
-    int r = row0 + 4 * (lane >> 4) + t;
-    r = r < last ? r : last;                 // rows past the end carry weight 0
-    const float* p = head + (int64_t)r * ss + NT * (lane & 15);
-    float x[NT];
-#pragma unroll
-    for (int n = 0; n < NT; n++) x[n] = p[n];
-#pragma unroll
-    for (int n = 0; n < NT; n++) acc[n] = mfma_f32(x[n], w[t], acc[n]);
-  }
-}
-
-// The two halves of add_cols, for callers that issue the loads well before the weights exist.
+// leaves): acc[n][r] of lane l is output element (own row l % 16, column NT (4 (l / 16) + r) + n).  In two halves, so that
+// the loads can be issued well before the weights exist.
 template <int NT>
 __device__ __forceinline__ void load_cols(const float* __restrict__ head, int64_t ss, int row0, int last, int lane,
                                           float (&x)[4][NT]) {
 #pragma unroll
   for (int t = 0; t < 4; t++) {
     int r = row0 + 4 * (lane >> 4) + t;
-    r = r < last ? r : last;
+    r = r < last ? r : last;                 // rows past the end carry weight 0
     const float* p = head + (int64_t)r * ss + NT * (lane & 15);
 #pragma unroll
     for (int n = 0; n < NT; n++) x[t][n] = p[n];
@@ -103,14 +94,38 @@ __device__ __forceinline__ void mma_cols(const float (&x)[4][NT], const f32q_t w
     for (int n = 0; n < NT; n++) acc[n] = mfma_f32(x[t][n], w[t], acc[n]);
 }
 
+// Adds the four wavefronts' accumulators and stores the sum: wavefront w takes register w of every lane, that is NT
+// consecutive elements of each of the 16 rows.  `mul[i]` scales wavefront i's share.  The LDS is free afterwards.
 template <int NT>
-__device__ __forceinline__ void store_cols(float* __restrict__ row, int lane, const f32q_t (&acc)[NT], float mul) {
+__device__ __forceinline__ void merge_store(float* __restrict__ row, bool write, int lane, int wave, const f32q_t (&acc)[NT],
+                                            const float (&mul)[kWaves], float (&buf)[kWaves][kWaves * NT][64]) {
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    float* p = row + NT * (4 * (lane >> 4) + r);
+  for (int r = 0; r < 4; r++)
 #pragma unroll
-    for (int n = 0; n < NT; n++) p[n] = acc[n][r] * mul;
+    for (int n = 0; n < NT; n++) buf[wave][r * NT + n][lane] = acc[n][r];
+  __syncthreads();
+  float x[NT];
+#pragma unroll
+  for (int n = 0; n < NT; n++) {
+    x[n] = 0.f;
+#pragma unroll
+    for (int i = 0; i < kWaves; i++) x[n] += buf[i][wave * NT + n][lane] * mul[i];
   }
+  if (write) {
+    float* p = row + NT * (4 * (lane >> 4) + wave);
+#pragma unroll
+    for (int n = 0; n < NT; n++) p[n] = x[n];
+  }
+}
+
+// Which 16 rows and which head a block has.  Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its
+// own; here every XCD gets a run of whole heads, so that a head's other operands are fetched into one L2 instead of eight.
+struct BlockRows { int tile, bh; };
+__device__ __forceinline__ BlockRows block_rows(int tiles) {
+  const int total = (int)(gridDim.x * gridDim.y), id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  const int per = total >> 3, extra = total & 7, xcd = id & 7;
+  const int w = xcd * per + (xcd < extra ? xcd : extra) + (id >> 3);
+  return {w % tiles, w / tiles};
 }
 
 __device__ __forceinline__ float groups_max(float x) {      // over the four lanes that share l % 16
@@ -122,12 +137,17 @@ __device__ __forceinline__ float groups_sum(float x) {
 
 // Forward: o = softmax(scale q k^T) v, lse = log-sum-exp of the scaled scores.
 template <int NT>
-__global__ __launch_bounds__(64) void attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                          const float* __restrict__ v, float* __restrict__ o,
-                                                          float* __restrict__ lse, AttnShapeF32 sh, float scale, int causal) {
-  const int lane = threadIdx.x, G = lane >> 4;
-  const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * 16;          // longest causal rows first
-  const int bh = blockIdx.y;
+__global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                   const float* __restrict__ v, float* __restrict__ o,
+                                                                   float* __restrict__ lse, AttnShapeF32 sh, float scale,
+                                                                   int causal) {
+  __shared__ float buf[kWaves][kWaves * NT][64];
+  __shared__ float stat[2][kWaves][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
+  const int tiles = (sh.seq + 15) >> 4;
+  const BlockRows own = block_rows(tiles);
+  const int q0 = (tiles - 1 - own.tile) * 16;                     // longest causal rows first
+  const int bh = own.bh;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
   const int last = sh.seq - 1;
   const int myq = q0 + (lane & 15);
@@ -138,81 +158,85 @@ __global__ __launch_bounds__(64) void attn_fwd_f32_kernel(const float* __restric
   f32q_t acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) acc[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
-  constexpr bool AHEAD = NT <= 4;      // head_dim <= 64: all K and V operands of a 64-key step fit in registers, so
-                                       // their loads are issued together and the step waits for memory once
-  for (int k0 = 0; k0 < nkeys; k0 += 64) {
-    f32q_t s[4];
+  // U key tiles per step, all their operands requested before the first product (one wait for memory per step)
+  constexpr int U = NT <= 4 ? 2 : 1;
+  for (int k0 = 16 * wave; k0 < nkeys; k0 += 16 * kWaves * U) {
+    f32q_t s[U];
+    float kf[U][NT][4], vx[U][4][NT];
     float mx = kMasked;
-    float kfa[AHEAD ? 4 : 1][NT][4], vxa[AHEAD ? 4 : 1][4][NT];
-    if constexpr (AHEAD) {
 #pragma unroll
-      for (int kt = 0; kt < 4; kt++)
-        if (k0 + 16 * kt < nkeys) load_rows<NT>(k + base, sh.ss, k0 + 16 * kt, last, lane, kfa[kt]);
+    for (int u = 0; u < U; u++)
+      if (k0 + 16 * kWaves * u < nkeys) load_rows<NT>(k + base, sh.ss, k0 + 16 * kWaves * u, last, lane, kf[u]);
 #pragma unroll
-      for (int kt = 0; kt < 4; kt++)
-        if (k0 + 16 * kt < nkeys) load_cols<NT>(v + base, sh.ss, k0 + 16 * kt, last, lane, vxa[kt]);
-    }
+    for (int u = 0; u < U; u++)
+      if (k0 + 16 * kWaves * u < nkeys) load_cols<NT>(v + base, sh.ss, k0 + 16 * kWaves * u, last, lane, vx[u]);
 #pragma unroll
-    for (int kt = 0; kt < 4; kt++) {
-      const int kb = k0 + 16 * kt;
-      if (kb < nkeys) {
-        if constexpr (AHEAD) {
-          s[kt] = rows_dot<NT>(kfa[kt], qf);
-        } else {
-          float kf[NT][4];
-          load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
-          s[kt] = rows_dot<NT>(kf, qf);
-        }
-      } else {
-        s[kt] = f32q_t{0.f, 0.f, 0.f, 0.f};
-      }
+    for (int u = 0; u < U; u++) {
+      const int kb = k0 + 16 * kWaves * u;
+      if (kb < nkeys) s[u] = rows_dot<NT>(kf[u], qf);
+      else s[u] = f32q_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int key = kb + 4 * G + r;
         const bool valid = key < nkeys && (!causal || key <= myq);
-        s[kt][r] = valid ? s[kt][r] * scale : kMasked;
-        mx = fmaxf(mx, s[kt][r]);
+        s[u][r] = valid ? s[u][r] * scale : kMasked;
+        mx = fmaxf(mx, s[u][r]);
       }
     }
-    // key 0 is visible to every query, so the running maximum is finite from the first tile on
+    // every tile that starts below nkeys has a key that the query sees, so the running maximum is finite from the first on
     const float m_new = fmaxf(m, groups_max(mx));
     const float alpha = expf(m - m_new);
     float psum = 0.f;
 #pragma unroll
-    for (int kt = 0; kt < 4; kt++)
+    for (int u = 0; u < U; u++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        s[kt][r] = expf(s[kt][r] - m_new);
-        psum += s[kt][r];
+        s[u][r] = expf(s[u][r] - m_new);
+        psum += s[u][r];
       }
     lsum = lsum * alpha + psum;               // this lane's share of the row sum; the groups are added at the end
 #pragma unroll
     for (int n = 0; n < NT; n++) acc[n] *= alpha;
 #pragma unroll
-    for (int kt = 0; kt < 4; kt++)
-      if (k0 + 16 * kt < nkeys) {
-        if constexpr (AHEAD) mma_cols<NT>(vxa[kt], s[kt], acc);
-        else add_cols<NT>(v + base, sh.ss, k0 + 16 * kt, last, lane, s[kt], acc);
-      }
+    for (int u = 0; u < U; u++)
+      if (k0 + 16 * kWaves * u < nkeys) mma_cols<NT>(vx[u], s[u], acc);
     m = m_new;
   }
   lsum = groups_sum(lsum);
-  if (myq < sh.seq) {
-    store_cols<NT>(o + base + (int64_t)myq * sh.ss, lane, acc, 1.f / lsum);
-    if (G == 0) lse[(int64_t)bh * sh.seq + myq] = m + logf(lsum);
+  if (G == 0) {
+    stat[0][wave][lane] = m;
+    stat[1][wave][lane] = lsum;
   }
+  __syncthreads();
+  float mul[kWaves], top = kMasked, sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < kWaves; i++) top = fmaxf(top, stat[0][i][lane & 15]);     // wavefront 0 has key 0: finite
+#pragma unroll
+  for (int i = 0; i < kWaves; i++) {
+    mul[i] = expf(stat[0][i][lane & 15] - top);                                 // 0 for a wavefront without a tile
+    sum += stat[1][i][lane & 15] * mul[i];
+  }
+#pragma unroll
+  for (int i = 0; i < kWaves; i++) mul[i] *= 1.f / sum;
+  merge_store<NT>(o + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, mul, buf);
+  if (wave == 0 && G == 0 && myq < sh.seq) lse[(int64_t)bh * sh.seq + myq] = top + logf(sum);
 }
 
-// dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T.
+// dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T, delta = rowsum(dO * O), which it also
+// leaves for the dK/dV kernel.
 template <int NT>
-__global__ __launch_bounds__(64) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                             const float* __restrict__ v, const float* __restrict__ d_o,
-                                                             const float* __restrict__ lse, const float* __restrict__ delta,
-                                                             float* __restrict__ dq, AttnShapeF32 sh, float scale,
-                                                             int causal) {
-  const int lane = threadIdx.x, G = lane >> 4;
-  const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * 16;
-  const int bh = blockIdx.y;
+__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                      const float* __restrict__ v, const float* __restrict__ o,
+                                                                      const float* __restrict__ d_o,
+                                                                      const float* __restrict__ lse, float* __restrict__ delta,
+                                                                      float* __restrict__ dq, AttnShapeF32 sh, float scale,
+                                                                      int causal) {
+  __shared__ float buf[kWaves][kWaves * NT][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
+  const int tiles = (sh.seq + 15) >> 4;
+  const BlockRows own = block_rows(tiles);
+  const int q0 = (tiles - 1 - own.tile) * 16;
+  const int bh = own.bh;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
   const int last = sh.seq - 1;
   const int myq = q0 + (lane & 15);
@@ -220,51 +244,56 @@ __global__ __launch_bounds__(64) void attn_bwd_dq_f32_kernel(const float* __rest
   float qf[NT][4], dof[NT][4];
   load_rows<NT>(q + base, sh.ss, q0, last, lane, qf);
   load_rows<NT>(d_o + base, sh.ss, q0, last, lane, dof);
-  const float L = lse[(int64_t)bh * sh.seq + qc], dl = delta[(int64_t)bh * sh.seq + qc];
+  const float L = lse[(int64_t)bh * sh.seq + qc];
+  float dl = 0.f;
+  {
+    float of[NT][4];
+    load_rows<NT>(o + base, sh.ss, q0, last, lane, of);
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) dl += of[c][t] * dof[c][t];
+    dl = groups_sum(dl);
+    if (wave == 0 && G == 0 && myq < sh.seq) delta[(int64_t)bh * sh.seq + myq] = dl;
+  }
   const int nkeys = causal ? (q0 + 16 < sh.seq ? q0 + 16 : sh.seq) : sh.seq;
   f32q_t acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) acc[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
-  // U key tiles per step, all their operands requested before the first product (one wait for memory per step)
-  constexpr int U = NT <= 3 ? 4 : (NT <= 4 ? 2 : 1);      // (166 registers at NT = 4: three wavefronts per SIMD)
-  for (int kb0 = 0; kb0 < nkeys; kb0 += 16 * U) {
-    float kf[U][NT][4], vf[U][NT][4], kx[U][4][NT];
+  for (int kb = 16 * wave; kb < nkeys; kb += 16 * kWaves) {
+    float kf[NT][4], vf[NT][4], kx[4][NT];
+    load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
+    load_rows<NT>(v + base, sh.ss, kb, last, lane, vf);
+    load_cols<NT>(k + base, sh.ss, kb, last, lane, kx);        // for dQ += dS . K
+    f32q_t s = rows_dot<NT>(kf, qf);
+    const f32q_t dp = rows_dot<NT>(vf, dof);
 #pragma unroll
-    for (int u = 0; u < U; u++)
-      if (kb0 + 16 * u < nkeys) {
-        load_rows<NT>(k + base, sh.ss, kb0 + 16 * u, last, lane, kf[u]);
-        load_rows<NT>(v + base, sh.ss, kb0 + 16 * u, last, lane, vf[u]);
-        load_cols<NT>(k + base, sh.ss, kb0 + 16 * u, last, lane, kx[u]);        // for dQ += dS . K
-      }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int kb = kb0 + 16 * u;
-      if (kb >= nkeys) break;
-      f32q_t s = rows_dot<NT>(kf[u], qf);
-      const f32q_t dp = rows_dot<NT>(vf[u], dof);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int key = kb + 4 * G + r;
-        const bool valid = key < nkeys && (!causal || key <= myq);
-        const float p = valid ? expf(s[r] * scale - L) : 0.f;
-        s[r] = p * (dp[r] - dl) * scale;
-      }
-      mma_cols<NT>(kx[u], s, acc);
+    for (int r = 0; r < 4; r++) {
+      const int key = kb + 4 * G + r;
+      const bool valid = key < nkeys && (!causal || key <= myq);
+      const float p = valid ? expf(s[r] * scale - L) : 0.f;
+      s[r] = p * (dp[r] - dl) * scale;
     }
+    mma_cols<NT>(kx, s, acc);
   }
-  if (myq < sh.seq) store_cols<NT>(dq + base + (int64_t)myq * sh.ss, lane, acc, 1.f);
+  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
+  merge_store<NT>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf);
 }
 
-// dV = P^T dO, dK = scale dS^T Q: one wavefront per 16 keys, walking the queries that see them.
+// dV = P^T dO, dK = scale dS^T Q: a block per 16 keys, walking the queries that see them.
 template <int NT>
-__global__ __launch_bounds__(64) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                              const float* __restrict__ v, const float* __restrict__ d_o,
-                                                              const float* __restrict__ lse, const float* __restrict__ delta,
-                                                              float* __restrict__ dk, float* __restrict__ dv,
-                                                              AttnShapeF32 sh, float scale, int causal) {
-  const int lane = threadIdx.x, G = lane >> 4;
-  const int key0 = (int)blockIdx.x * 16;                           // the earliest keys see the most queries
-  const int bh = blockIdx.y;
+__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                       const float* __restrict__ v,
+                                                                       const float* __restrict__ d_o,
+                                                                       const float* __restrict__ lse,
+                                                                       const float* __restrict__ delta, float* __restrict__ dk,
+                                                                       float* __restrict__ dv, AttnShapeF32 sh, float scale,
+                                                                       int causal) {
+  __shared__ float buf[kWaves][kWaves * NT][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
+  const BlockRows own = block_rows((sh.seq + 15) >> 4);
+  const int key0 = own.tile * 16;                                  // the earliest keys see the most queries
+  const int bh = own.bh;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
   const int last = sh.seq - 1;
   const int mykey = key0 + (lane & 15);
@@ -276,48 +305,36 @@ __global__ __launch_bounds__(64) void attn_bwd_dkv_f32_kernel(const float* __res
   f32q_t acck[NT], accv[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) acck[n] = accv[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
-  // U query tiles per step, operands (and the rows' lse / delta) requested together; two tiles only while the
-  // registers allow three wavefronts per SIMD to stay resident
-  constexpr int U = NT <= 3 ? 2 : 1;
-  for (int qb0 = causal ? key0 : 0; qb0 < sh.seq; qb0 += 16 * U) {
-    float qf[U][NT][4], dof[U][NT][4], qx[U][4][NT], dox[U][4][NT], lq[U][4], dq_[U][4];
+  for (int qb = (causal ? key0 : 0) + 16 * wave; qb < sh.seq; qb += 16 * kWaves) {
+    float qf[NT][4], dof[NT][4], qx[4][NT], dox[4][NT], lq[4], dq_[4];
+    load_rows<NT>(q + base, sh.ss, qb, last, lane, qf);
+    load_rows<NT>(d_o + base, sh.ss, qb, last, lane, dof);
+    load_cols<NT>(d_o + base, sh.ss, qb, last, lane, dox);    // for dV += P^T . dO
+    load_cols<NT>(q + base, sh.ss, qb, last, lane, qx);       // for dK += dS^T . Q
 #pragma unroll
-    for (int u = 0; u < U; u++)
-      if (qb0 + 16 * u < sh.seq) {
-        load_rows<NT>(q + base, sh.ss, qb0 + 16 * u, last, lane, qf[u]);
-        load_rows<NT>(d_o + base, sh.ss, qb0 + 16 * u, last, lane, dof[u]);
-        load_cols<NT>(d_o + base, sh.ss, qb0 + 16 * u, last, lane, dox[u]);    // for dV += P^T . dO
-        load_cols<NT>(q + base, sh.ss, qb0 + 16 * u, last, lane, qx[u]);       // for dK += dS^T . Q
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int qi = qb0 + 16 * u + 4 * G + r;
-          const int qc = qi < last ? qi : last;
-          lq[u][r] = lrow[qc];
-          dq_[u][r] = drow[qc];
-        }
-      }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int qb = qb0 + 16 * u;
-      if (qb >= sh.seq) break;
-      f32q_t s = rows_dot<NT>(qf[u], kf);               // register r: query qb + 4 G + r, key mykey
-      f32q_t dp = rows_dot<NT>(dof[u], vf);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int qi = qb + 4 * G + r;
-        const bool valid = qi < sh.seq && (!causal || mykey <= qi);
-        const float p = valid ? expf(s[r] * scale - lq[u][r]) : 0.f;
-        s[r] = p;
-        dp[r] = p * (dp[r] - dq_[u][r]) * scale;
-      }
-      mma_cols<NT>(dox[u], s, accv);
-      mma_cols<NT>(qx[u], dp, acck);
+    for (int r = 0; r < 4; r++) {
+      const int qi = qb + 4 * G + r;
+      const int qc = qi < last ? qi : last;
+      lq[r] = lrow[qc];
+      dq_[r] = drow[qc];
     }
+    f32q_t s = rows_dot<NT>(qf, kf);                   // register r: query qb + 4 G + r, key mykey
+    f32q_t dp = rows_dot<NT>(dof, vf);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int qi = qb + 4 * G + r;
+      const bool valid = qi < sh.seq && (!causal || mykey <= qi);
+      const float p = valid ? expf(s[r] * scale - lq[r]) : 0.f;
+      s[r] = p;
+      dp[r] = p * (dp[r] - dq_[r]) * scale;
+    }
+    mma_cols<NT>(dox, s, accv);
+    mma_cols<NT>(qx, dp, acck);
   }
-  if (mykey < sh.seq) {
-    store_cols<NT>(dk + base + (int64_t)mykey * sh.ss, lane, acck, 1.f);
-    store_cols<NT>(dv + base + (int64_t)mykey * sh.ss, lane, accv, 1.f);
-  }
+  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
+  merge_store<NT>(dk + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, acck, one, buf);
+  __syncthreads();
+  merge_store<NT>(dv + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, accv, one, buf);
 }
 
 static bool f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
@@ -349,28 +366,29 @@ int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL(attn_fwd_f32_kernel<NT>, grid, dim3(64), 0, st, (const float*)q, (const float*)k,
+                        hipLaunchKernelGGL(attn_fwd_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q, (const float*)k,
                                            (const float*)v, (float*)o, lse, shp, scale, causal));
   EMI_CHECK_LAUNCH("emi_attn_fwd(fp32 mfma)");
   return EMI_OK;
 }
 
-// dQ, dK, dV on the fp32 matrix-core path given delta = rowsum(dO * O); -1 when the operands do not qualify.
-int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* d_o, const float* lse,
-                             const float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads, int64_t seq,
-                             int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal) {
-  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, d_o, dq, dk, dv})) return -1;
+// dQ, dK, dV on the fp32 matrix-core path (delta: scratch for rowsum(dO * O)); -1 when the operands do not qualify.
+int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                             const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
+                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal) {
+  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL(attn_bwd_dkv_f32_kernel<NT>, grid, dim3(64), 0, st, (const float*)q, (const float*)k,
-                                           (const float*)v, (const float*)d_o, lse, delta, (float*)dk, (float*)dv, shp, scale,
-                                           causal));
-  EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dkv)");
-  EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL(attn_bwd_dq_f32_kernel<NT>, grid, dim3(64), 0, st, (const float*)q, (const float*)k,
-                                           (const float*)v, (const float*)d_o, lse, delta, (float*)dq, shp, scale, causal));
+                        hipLaunchKernelGGL(attn_bwd_dq_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q,
+                                           (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, delta,
+                                           (float*)dq, shp, scale, causal));
   EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dq)");
+  EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
+                        hipLaunchKernelGGL(attn_bwd_dkv_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q,
+                                           (const float*)k, (const float*)v, (const float*)d_o, lse, delta, (float*)dk,
+                                           (float*)dv, shp, scale, causal));
+  EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dkv)");
   return EMI_OK;
 }
 
