@@ -19,7 +19,6 @@
 #include <initializer_list>
 #include <type_traits>
 #include <utility>
-#include <stdlib.h>
 
 #include "emi_device.h"
 
@@ -425,26 +424,29 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 __device__ __forceinline__ int acc_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
 // ---------------------------------------------------------------------------
-// Forward: block = 4 waves x 32 queries, KV tiles of 64 keys.
+// Forward: block = 4 wavefronts.  QW = 4: 32 queries each, key tiles of 64 for all of them.  QW = 1: the same 32 queries
+// for all, a step is 128 keys of which each wavefront takes 32, and the four partial results are brought to a common
+// maximum and added through the LDS at the end.
 // ---------------------------------------------------------------------------
-template <int D>
+template <int D, int QW>
 __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_kernel(const uint16_t* __restrict__ q,
                                                             const uint16_t* __restrict__ k,
                                                             const uint16_t* __restrict__ v, uint16_t* __restrict__ o,
                                                             float* __restrict__ lse, AttnShape sh, uint32_t head_bytes,
                                                             float scale_log2e, int causal) {
-  constexpr int BQ = 128, BKV = 64, NW = 4;
+  constexpr int NW = 4, BQ = 32 * QW, SHARE = QW == 4 ? 64 : 32, BKV = SHARE * NW / QW;
   constexpr int TILE = BKV * D * 2, STAGE = 2 * TILE;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
   EMI_LDS uint8_t* smem = (EMI_LDS uint8_t*)smem_raw;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row_in_tile = QW == 4 ? 0 : wave * SHARE;
   int blk, bh;
   attn_block_coords(&blk, &bh);
   const int qblk = gridDim.x - 1 - blk;              // longest rows first
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
   const int seq = sh.seq;
-  const int q0 = qblk * BQ + wave * 32;
+  const int q0 = qblk * BQ + (QW == 4 ? wave * 32 : 0);
   const int qrow = q0 + (lane & 31);
 
   bf16x8_t qf[D / 16];
@@ -475,35 +477,39 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_kernel(const uint16_t* _
     }
     const EMI_LDS uint8_t* sK = smem + (j & 1) * STAGE;
     const EMI_LDS uint8_t* sV = sK + TILE;
-    const int key0 = j * BKV;
-    if (!(causal && key0 > q0 + 31)) {     // wave-uniform: this tile is not entirely in the future
-      f32x16_t s[2];
+    const int key0 = j * BKV + row_in_tile;
+    if (!(causal && key0 > q0 + 31) && key0 < seq) {     // wave-uniform: some query sees a key of this share
+      constexpr int NT = SHARE / 32;
+      f32x16_t s[NT];
 #pragma unroll
-      for (int T = 0; T < 2; T++) {
+      for (int T = 0; T < NT; T++) {
 #pragma unroll
         for (int r = 0; r < 16; r++) s[T][r] = 0.f;
 #pragma unroll
         for (int t = 0; t < D / 16; t++)
-          s[T] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(sK, T * 32, t, lane), qf[t], s[T], 0, 0, 0);
+          s[T] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(sK, row_in_tile + T * 32, t, lane), qf[t], s[T], 0, 0, 0);
       }
-      const bool need_mask = (causal && key0 + BKV - 1 > q0) || key0 + BKV > seq;
+      const bool need_mask = (causal && key0 + SHARE - 1 > q0) || key0 + SHARE > seq;
       float mt = kNegBig;
+      if (need_mask) {                                   // one branch, not one per score
 #pragma unroll
-      for (int T = 0; T < 2; T++)
+        for (int T = 0; T < NT; T++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          if (need_mask) {
+          for (int r = 0; r < 16; r++) {
             const int key = key0 + T * 32 + acc_row(r, lane);
             if ((causal && key > qrow) || key >= seq) s[T][r] = kNegBig;
           }
-          mt = fmaxf(mt, s[T][r]);
-        }
+      }
+#pragma unroll
+      for (int T = 0; T < NT; T++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) mt = fmaxf(mt, s[T][r]);
       mt = max_xor32(mt);
       const float m_new = fmaxf(m, mt * scale_log2e);      // running max in the scaled log2 domain
       const float alpha = fast_exp2(m - m_new);
       float rs = 0.f;
 #pragma unroll
-      for (int T = 0; T < 2; T++)
+      for (int T = 0; T < NT; T++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const float p = fast_exp2(fmaf(s[T][r], scale_log2e, -m_new));
@@ -517,13 +523,13 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_kernel(const uint16_t* _
 #pragma unroll
         for (int r = 0; r < 16; r++) acc_o[dt][r] *= alpha;
 #pragma unroll
-      for (int T = 0; T < 2; T++)
+      for (int T = 0; T < NT; T++)
 #pragma unroll
         for (int sI = 0; sI < 2; sI++) {
           const bf16x8_t pf = acc_to_frag(s[T], sI);
 #pragma unroll
           for (int dt = 0; dt < D / 32; dt++)
-            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(col_frag<D>(sV, T * 32 + sI * 16, dt * 32, lane), pf,
+            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(col_frag<D>(sV, row_in_tile + T * 32 + sI * 16, dt * 32, lane), pf,
                                                                 acc_o[dt], 0, 0, 0);
         }
     }
@@ -538,6 +544,44 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_kernel(const uint16_t* _
   // 8-byte halves swapped when (r / CH) is odd: conflict free for both access shapes.
   // (the loop ended with all loads landed and a barrier: the LDS is idle)
   l = sum_xor32(l);
+  if constexpr (QW == 1) {
+    EMI_LDS float* part = (EMI_LDS float*)smem;                          // [wavefront][accumulator register][lane]
+    EMI_LDS float* stat = part + NW * (D / 2) * 64;                      // [maximum, sum][wavefront][query]
+    static_assert((NW * (D / 2) * 64 + 2 * NW * 32) * 4 <= 2 * STAGE, "LDS");
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) part[(wave * (D / 2) + dt * 16 + r) * 64 + lane] = acc_o[dt][r];
+    if (lane < 32) stat[wave * 32 + lane] = m, stat[(NW + wave) * 32 + lane] = l;
+    __syncthreads();
+    float top = kNegBig, mul[NW], sum = 0.f;                             // wavefront 0 has key 0, which every query sees
+#pragma unroll
+    for (int w = 0; w < NW; w++) top = fmaxf(top, stat[w * 32 + (lane & 31)]);
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      mul[w] = fast_exp2(stat[w * 32 + (lane & 31)] - top);              // 0 for a wavefront that saw no key
+      sum += stat[(NW + w) * 32 + (lane & 31)] * mul[w];
+    }
+    const float inv = 1.0f / sum;
+    if (qrow < seq) {
+      if (wave == 0 && lane < 32) lse[(int64_t)bh * seq + qrow] = (top + __builtin_amdgcn_logf(sum)) * kLn2;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; dt++) {                              // wavefront w stores register quad w
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          x[e] = 0.f;
+#pragma unroll
+          for (int w = 0; w < NW; w++) x[e] += part[(w * (D / 2) + dt * 16 + 4 * wave + e) * 64 + lane] * mul[w];
+        }
+        uint2 u;
+        u.x = pack_bf16x2(x[0] * inv, x[1] * inv);
+        u.y = pack_bf16x2(x[2] * inv, x[3] * inv);
+        *reinterpret_cast<uint2*>(o + base + (int64_t)qrow * sh.ss + dt * 32 + 8 * wave + 4 * (lane >> 5)) = u;
+      }
+    }
+    return;
+  }
   {
     constexpr int CH = D / 8, RB = D * 2;
     EMI_LDS uint8_t* wl = smem + wave * (32 * RB);
@@ -863,7 +907,7 @@ __device__ __forceinline__ void unrope_quad(const float* t, float& x0, float& x1
 // of eight elements of a row), written as delta * delta_sign to delta_out and lse * log2(e) to lse2_out for the dK/dV kernel, which then has
 // to run after this one.  Without `o`, delta comes in through `delta`.
 // ---------------------------------------------------------------------------
-template <int D>
+template <int D, int QW>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t* __restrict__ q,
                                                                const uint16_t* __restrict__ k,
                                                                const uint16_t* __restrict__ v,
@@ -875,7 +919,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t
                                                                float delta_sign, const float* __restrict__ unrope,
                                                                const uint16_t* __restrict__ o, float* __restrict__ delta_out,
                                                                float* __restrict__ lse2_out) {
-  constexpr int BQ = 128, BKV = 64, NW = 4;
+  constexpr int NW = 4, BQ = 32 * QW, SHARE = QW == 4 ? 64 : 32, BKV = SHARE * NW / QW;
   constexpr int TILE = BKV * D * 2, STAGE = 2 * TILE;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
   EMI_LDS uint8_t* smem = (EMI_LDS uint8_t*)smem_raw;
@@ -886,7 +930,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t
   const int qblk = gridDim.x - 1 - blk;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
   const int seq = sh.seq;
-  const int q0 = qblk * BQ + wave * 32;
+  const int q0 = qblk * BQ + (QW == 4 ? wave * 32 : 0);
+  const int row_in_tile = QW == 4 ? 0 : wave * SHARE;
   const int qrow = q0 + (lane & 31);
   const float scale_log2e = scale * kLog2e;
 
@@ -916,7 +961,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t
 #pragma unroll
       for (int t = 0; t < m; t++) cs[t] += cs[t + m];
     dl = sum_xor32(cs[0]);
-    if (qrow < seq && lane < 32) {
+    if (qrow < seq && lane < 32 && (QW == 4 || wave == 0)) {
       delta_out[(int64_t)bh * seq + qrow] = dl * delta_sign;
       lse2_out[(int64_t)bh * seq + qrow] = L2;
     }
@@ -948,34 +993,36 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t
     }
     const EMI_LDS uint8_t* sK = smem + (j & 1) * STAGE;
     const EMI_LDS uint8_t* sV = sK + TILE;
-    const int key0 = j * BKV;
-    if (!(causal && key0 > q0 + 31)) {
-      const bool need_mask = (causal && key0 + BKV - 1 > q0) || key0 + BKV > seq;
+    const int key0 = j * BKV + row_in_tile;
+    if (!(causal && key0 > q0 + 31) && key0 < seq) {
+      const bool need_mask = (causal && key0 + SHARE - 1 > q0) || key0 + SHARE > seq;
 #pragma unroll 1
-      for (int T = 0; T < 2; T++) {
+      for (int T = 0; T < SHARE / 32; T++) {
         f32x16_t s, dp;
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = 0.f, dp[r] = 0.f;
 #pragma unroll
         for (int t = 0; t < D / 16; t++) {
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(sK, T * 32, t, lane), qf[t], s, 0, 0, 0);
-          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(sV, T * 32, t, lane), dof[t], dp, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(sK, row_in_tile + T * 32, t, lane), qf[t], s, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(sV, row_in_tile + T * 32, t, lane), dof[t], dp, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          float p = fast_exp2(s[r] * scale_log2e - L2);
-          if (need_mask) {
+        for (int r = 0; r < 16; r++) s[r] = fast_exp2(s[r] * scale_log2e - L2);
+        if (need_mask) {                                 // one branch; tested per score it kept the exponentials apart
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
             const int key = key0 + T * 32 + acc_row(r, lane);
-            if ((causal && key > qrow) || key >= seq) p = 0.f;
+            if ((causal && key > qrow) || key >= seq) s[r] = 0.f;
           }
-          s[r] = p * (dp[r] - dl);
         }
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] *= dp[r] - dl;
 #pragma unroll
         for (int sI = 0; sI < 2; sI++) {
           const bf16x8_t dsf = acc_to_frag(s, sI);
 #pragma unroll
           for (int dt = 0; dt < D / 32; dt++)
-            acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(col_frag<D>(sK, T * 32 + sI * 16, dt * 32, lane), dsf,
+            acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(col_frag<D>(sK, row_in_tile + T * 32 + sI * 16, dt * 32, lane), dsf,
                                                               acc[dt], 0, 0, 0);
         }
       }
@@ -983,14 +1030,32 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_bf16_kernel(const uint16_t
     __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
   }
+  if constexpr (QW == 1) {                     // add the four partial sums; wavefront w keeps register quad w of each
+    EMI_LDS float* part = (EMI_LDS float*)smem;
+    static_assert(NW * (D / 2) * 64 * 4 <= 2 * STAGE, "LDS");
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) part[(wave * (D / 2) + dt * 16 + r) * 64 + lane] = acc[dt][r];
+    __syncthreads();
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float x = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) x += part[(w * (D / 2) + dt * 16 + 4 * wave + e) * 64 + lane];
+        acc[dt][e] = x;
+      }
+  }
   if (qrow < seq) {
     uint16_t* out = dq + base + (int64_t)qrow * sh.ss;
     const float* trow = unrope ? unrope + (int64_t)qrow * D : nullptr;     // D/2 (cos, sin) pairs per position
 #pragma unroll
     for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
-      for (int jj = 0; jj < 4; jj++) {
-        const int dcol = dt * 32 + 8 * jj + 4 * (lane >> 5);
+      for (int jj = 0; jj < QW; jj++) {
+        const int dcol = dt * 32 + 8 * (QW == 4 ? jj : wave) + 4 * (lane >> 5);
         float x0 = acc[dt][4 * jj] * scale, x1 = acc[dt][4 * jj + 1] * scale, x2 = acc[dt][4 * jj + 2] * scale,
               x3 = acc[dt][4 * jj + 3] * scale;
         if (trow != nullptr) unrope_quad(trow + dcol, x0, x1, x2, x3);
@@ -1507,6 +1572,19 @@ static inline int rows_vec4(int dtype, int64_t head_dim, int64_t sb, int64_t sh,
   return 1;
 }
 
+// Whether the forward and dQ kernels give a block 32 queries and deal the keys to its wavefronts (QW = 1), rather than 32
+// queries to each of them.  Four times the blocks, each a quarter as long; but four times the reads of K and V, so it
+// pays while the blocks run at one time: two per CU at head_dim 64, one at 128 (two stages of 128 keys in the LDS).  With 512
+// keys and more a second round still does.  Forward, us, 32-query blocks | others: heads x seq x head_dim
+//   12 x 777 x 64 9.4 | 18.3   12 x 2048 x 64 26 | 33   32 x 1024 x 64 15.7 | 19.2   96 x 128 x 64 5.7 | 6.6   96 x 256 x 64 9.7 | 8.7
+//   8 x 1024 x 128 15.7 | 27   32 x 512 x 128 15.1 | 16.7   12 x 1024 x 128 24.6 | 27   12 x 2048 x 128 63 | 47   96 x 128 x 128 11 | 8.6
+// and the adjoint with it: 12 x 777 x 64 31 | 38, 32 x 512 x 128 40 | 43, 32 x 777 x 128 69 | 58.  Up to 64 keys there is nothing
+// to deal (equal forward, adjoint 11.0 | 10.4).
+static bool split_keys(int64_t seq, int64_t bh, int64_t head_dim) {
+  const int64_t blocks = (seq + 31) / 32 * bh, at_once = head_dim == 64 ? 512 : 256;
+  return seq > 64 && blocks <= (seq >= 512 ? 2 * at_once : at_once);
+}
+
 extern "C" size_t emi_attn_fwd_workspace_bytes(int64_t batch, int64_t heads, int64_t seq, int64_t head_dim) {
   (void)batch; (void)heads; (void)seq; (void)head_dim;
   return 0;          // the forward kernels need no scratch (V is transposed by the LDS reads)
@@ -1527,8 +1605,10 @@ extern "C" int emi_attn_fwd_ws(emi_stream_t stream, const void* q, const void* k
   if (mfma_ok(a, dtype, {q, k, v, o})) {
     const uint32_t head_bytes = (uint32_t)(((seq - 1) * stride_s + head_dim) * 2);
     const float sl2 = scale * kLog2e;
-    // 256-query blocks; at 512 keys and fewer the 128-query kernel below is faster (25 vs 31 us at 16 x 12 x 512 x 64)
-    if (seq > 512) {
+    const bool few = split_keys(seq, bh, head_dim);
+    // 256-query blocks for long sequences; at 512 keys and fewer 128-query blocks are faster (25 vs 31 us at 16 x 12 x 512 x 64),
+    // and up to 1024 also where the last block of 256 would be less than half full (96 x 777 x 128 34 vs 38 us)
+    if (!few && seq > 512 && (seq > 1024 || (seq - 1) % 256 >= 128)) {
       const dim3 gridp((unsigned)((seq + 255) / 256), bh);
 #define EMI_ATTN_FWD_PP(DD)                                                                                          \
   do {                                                                                                               \
@@ -1543,18 +1623,22 @@ extern "C" int emi_attn_fwd_ws(emi_stream_t stream, const void* q, const void* k
       EMI_CHECK_LAUNCH("emi_attn_fwd");
       return EMI_OK;
     }
-    const dim3 grid((unsigned)((seq + 127) / 128), bh);
+#define EMI_ATTN_FWD(DD, QW)                                                                                         \
+  do {                                                                                                               \
+    constexpr int smem = 2 * 2 * (QW == 4 ? 64 : 128) * DD * 2;                                                      \
+    if (int rc = reserve_lds(attn_fwd_bf16_kernel<DD, QW>, smem, "emi_attn_fwd")) return rc;                         \
+    hipLaunchKernelGGL((attn_fwd_bf16_kernel<DD, QW>), dim3((unsigned)((seq + 32 * QW - 1) / (32 * QW)), bh), dim3(256), smem, \
+                       st, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse, shp, head_bytes, sl2,  \
+                       causal);                                                                                      \
+  } while (0)
     if (head_dim == 128) {
-      constexpr int smem = 2 * 2 * 64 * 128 * 2;
-      if (int rc = reserve_lds(attn_fwd_bf16_kernel<128>, smem, "emi_attn_fwd")) return rc;
-      hipLaunchKernelGGL(attn_fwd_bf16_kernel<128>, grid, dim3(256), smem, st, (const uint16_t*)q, (const uint16_t*)k,
-                         (const uint16_t*)v, (uint16_t*)o, lse, shp, head_bytes, sl2, causal);
+      if (few) EMI_ATTN_FWD(128, 1);
+      else EMI_ATTN_FWD(128, 4);
     } else {
-      constexpr int smem = 2 * 2 * 64 * 64 * 2;
-      if (int rc = reserve_lds(attn_fwd_bf16_kernel<64>, smem, "emi_attn_fwd")) return rc;
-      hipLaunchKernelGGL(attn_fwd_bf16_kernel<64>, grid, dim3(256), smem, st, (const uint16_t*)q, (const uint16_t*)k,
-                         (const uint16_t*)v, (uint16_t*)o, lse, shp, head_bytes, sl2, causal);
+      if (few) EMI_ATTN_FWD(64, 1);
+      else EMI_ATTN_FWD(64, 4);
     }
+#undef EMI_ATTN_FWD
     EMI_CHECK_LAUNCH("emi_attn_fwd");
     return EMI_OK;
   }
@@ -1628,23 +1712,36 @@ static int attn_bwd_impl(emi_stream_t stream, const void* q, const void* k, cons
   if (fast) {
     const uint32_t head_bytes = (uint32_t)(((seq - 1) * stride_s + head_dim) * 2);
     const dim3 grid((unsigned)((seq + 127) / 128), bh);
-#define EMI_ATTN_BWD_LAUNCH(DD)                                                                                          \
+    const bool few = split_keys(seq, bh, head_dim);
+#define EMI_ATTN_DQ(DD, QW)                                                                                              \
   do {                                                                                                                   \
-    constexpr int smem_q = 2 * 2 * 64 * DD * 2;                                                                          \
-    constexpr int smem_sp = 6 * 64 * DD * 2 + 3 * 512;                                                                   \
-    if (int rc = reserve_lds(attn_bwd_dq_bf16_kernel<DD>, smem_q, "emi_attn_bwd")) return rc;                            \
-    hipLaunchKernelGGL(attn_bwd_dq_bf16_kernel<DD>, grid, dim3(256), smem_q, st, (const uint16_t*)q, (const uint16_t*)k, \
-                       (const uint16_t*)v, (const uint16_t*)d_o, lse, (const float*)nullptr, (uint16_t*)dq, shp,         \
-                       head_bytes, scale, causal, delta_sign, unrope, (const uint16_t*)o, delta, lse2);                  \
+    constexpr int smem = 2 * 2 * (QW == 4 ? 64 : 128) * DD * 2;                                                          \
+    if (int rc = reserve_lds(attn_bwd_dq_bf16_kernel<DD, QW>, smem, "emi_attn_bwd")) return rc;                          \
+    hipLaunchKernelGGL((attn_bwd_dq_bf16_kernel<DD, QW>), dim3((unsigned)((seq + 32 * QW - 1) / (32 * QW)), bh), dim3(256), smem, \
+                       st, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, lse,        \
+                       (const float*)nullptr, (uint16_t*)dq, shp, head_bytes, scale, causal, delta_sign, unrope,         \
+                       (const uint16_t*)o, delta, lse2);                                                                 \
     EMI_CHECK_LAUNCH("emi_attn_bwd(dq)");                                                                                \
+  } while (0)
+#define EMI_ATTN_DKV(DD)                                                                                                 \
+  do {                                                                                                                   \
+    constexpr int smem_sp = 6 * 64 * DD * 2 + 3 * 512;                                                                   \
     if (int rc = reserve_lds(attn_bwd_dkv_sp_kernel<DD>, smem_sp, "emi_attn_bwd")) return rc;                            \
     hipLaunchKernelGGL(attn_bwd_dkv_sp_kernel<DD>, grid, dim3(256), smem_sp, st, (const uint16_t*)q,                     \
                        (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)d_o, lse2, delta, (uint16_t*)dk,         \
                        (uint16_t*)dv, shp, head_bytes, scale, causal, unrope);                                           \
   } while (0)
-    if (head_dim == 128) EMI_ATTN_BWD_LAUNCH(128);
-    else EMI_ATTN_BWD_LAUNCH(64);
-#undef EMI_ATTN_BWD_LAUNCH
+    if (head_dim == 128) {
+      if (few) EMI_ATTN_DQ(128, 1);
+      else EMI_ATTN_DQ(128, 4);
+      EMI_ATTN_DKV(128);
+    } else {
+      if (few) EMI_ATTN_DQ(64, 1);
+      else EMI_ATTN_DQ(64, 4);
+      EMI_ATTN_DKV(64);
+    }
+#undef EMI_ATTN_DQ
+#undef EMI_ATTN_DKV
     EMI_CHECK_LAUNCH("emi_attn_bwd(dkv)");
     return EMI_OK;
   }
