@@ -1607,9 +1607,11 @@ extern "C" int emi_attn_fwd_ws(emi_stream_t stream, const void* q, const void* k
     const float sl2 = scale * kLog2e;
     const bool few = split_keys(seq, bh, head_dim);
     // 256-query blocks for long sequences; at 512 keys and fewer 128-query blocks are faster (25 vs 31 us at 16 x 12 x 512 x 64),
-    // and up to 1024 also where the last block of 256 would be less than half full (96 x 777 x 128 34 vs 38 us)
-    if (!few && seq > 512 && (seq > 1024 || (seq - 1) % 256 >= 128)) {
-      const dim3 gridp((unsigned)((seq + 255) / 256), bh);
+    // and up to 1024 also where the last block of 256 would be less than half full, unless all blocks of 256 run at one time
+    // and their longest one ends sooner (us, 128 | 256 queries: 96 x 780 x 128 34 | 38, 128 x 600 x 64 20 | 29, and with at most
+    // 256 blocks 60 x 780 x 128 29 | 25.5, 60 x 780 x 64 20.7 | 19.5, 40 x 854 x 128 29 | 25)
+    const dim3 gridp((unsigned)((seq + 255) / 256), bh);
+    if (!few && seq > 512 && (seq > 1024 || (seq - 1) % 256 >= 128 || (int64_t)gridp.x * bh <= 256)) {
 #define EMI_ATTN_FWD_PP(DD)                                                                                          \
   do {                                                                                                               \
     constexpr int smem = 3 * 2 * 64 * DD * 2;                                                                        \

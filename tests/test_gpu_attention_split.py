@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
     (4, 24, 170, 64),       # more 32-query blocks than run at one time: 128-query blocks
     (4, 12, 190, 128),
     (4, 24, 520, 64),       # 128-query blocks above 512 keys: the last block of 256 would be nearly empty
+    (3, 20, 530, 128),      # blocks of 256 all the same: they run at one time
 ])
 def test_bf16_attention_key_shares(B, h, S, d, layout, causal):
     from enzyme_ad.jax import ops
