@@ -66,7 +66,7 @@ template <typename T> struct NormGemv {
   float eps;
 };
 
-template <typename T, int MODE, int UN>
+template <typename T, int MODE, int UN, bool WHOLE>       // WHOLE: rows are whole batches
 __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
   using Raw = typename ChunkCached<T>::Raw;
   constexpr int V = ChunkCached<T>::N, BATCH = 64 * V * UN;
@@ -85,7 +85,8 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
       r1 = a.w[1] + (int64_t)p * a.K;
     }
   };
-  // unconditional: a piece past the row re-reads its start and meets a zero of the vector
+  // unconditional: a piece past the row re-reads its start and is dropped when it is summed (a zero of the vector alone
+  // would make a NaN of an infinite weight there)
   auto issue = [&](const T* r0, const T* r1, int b, Raw(&x0)[UN], Raw(&x1)[UN]) {
 #pragma unroll
     for (int u = 0; u < UN; u++) {
@@ -132,9 +133,11 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
 #pragma unroll
     for (int u = 0; u < UN; u++) {
       float w0[V], w1[V];
-      ChunkCached<T>::unpack(x0[u], w0);
-      ChunkCached<T>::unpack(x1[u], w1);
       const int c = b * 64 * UN + u * 64 + lane;
+      const Raw none{};
+      const bool in_row = WHOLE || c * V < a.K;
+      ChunkCached<T>::unpack(in_row ? x0[u] : none, w0);
+      ChunkCached<T>::unpack(in_row ? x1[u] : none, w1);
 #pragma unroll
       for (int h = 0; h < V / 4; h++) {
         const f4 xv = *reinterpret_cast<const f4*>(xs + (h * pieces + c) * 4);
@@ -202,11 +205,12 @@ template <typename T, int MODE> int launch_norm_gemv(hipStream_t st, const NormG
   const int P = MODE == 0 ? 3 * a.N / 2 : a.N;
   // two blocks a CU: each normalises the vector once for all its pairs
   const unsigned grid = (unsigned)((P + 3) / 4 < 512 ? (P + 3) / 4 : 512);
-#define EMI_NORM_GEMV(UN)                                                                            \
-  do {                                                                                               \
-    constexpr int batch = 64 * V * UN;                                                               \
-    const size_t lds = (size_t)((a.K + batch - 1) / batch) * batch * sizeof(float);                  \
-    hipLaunchKernelGGL((step_norm_gemv_kernel<T, MODE, UN>), dim3(grid), dim3(256), lds, st, a);     \
+#define EMI_NORM_GEMV(UN)                                                                                                      \
+  do {                                                                                                                         \
+    constexpr int batch = 64 * V * UN;                                                                                         \
+    const size_t lds = (size_t)((a.K + batch - 1) / batch) * batch * sizeof(float);                                            \
+    if (a.K % batch == 0) hipLaunchKernelGGL((step_norm_gemv_kernel<T, MODE, UN, true>), dim3(grid), dim3(256), lds, st, a);                   \
+    else hipLaunchKernelGGL((step_norm_gemv_kernel<T, MODE, UN, false>), dim3(grid), dim3(256), lds, st, a);                                   \
   } while (0)
   if (a.K <= 64 * V * 2) EMI_NORM_GEMV(2);
   else EMI_NORM_GEMV(8);

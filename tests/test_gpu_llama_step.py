@@ -71,3 +71,28 @@ def test_llama_step_accumulates_and_repeats():
     c = plain(dy)
     assert torch.equal(a[0], b[0]) and all(torch.equal(a[1][k], b[1][k]) for k in wd)
     assert rel_err(host(a[0]), host(c[0]) + host(dy)) < 1e-6
+
+
+def _own_key_out_of_reach(wd, wr, xr, pos, heads):
+    """One infinite weight at the start of a row of wk that gives the token's own key a score of -infinity in one head."""
+    dim = xr.shape[0]
+    d = dim // heads
+    cos, sin = (t[0] for t in L.rope_angles(1, d, pos0=pos))
+    xb = L.rmsnorm(xr, wr["rms_att_weight"][0])
+    q = (wr["wq"][0] @ xb).reshape(heads, d // 2, 2)
+    rq = np.stack([cos * q[..., 0] - sin * q[..., 1], sin * q[..., 0] + cos * q[..., 1]], -1)
+    # a key row whose element 2 i is infinite is turned into (cos, sin) times that: one sign in both products with rq
+    side = np.sign(rq * np.stack([cos, sin], -1))
+    h, i = np.argwhere((side[..., 0] == side[..., 1]) & (np.abs(rq).min(-1) > 0.1))[0]
+    wr["wk"][0, h * d + 2 * i, 0] = -side[h, i, 0] * np.sign(xb[0]) * np.inf
+    wd["wk"][0, h * d + 2 * i, 0] = float(wr["wk"][0, h * d + 2 * i, 0])
+
+
+@pytest.mark.parametrize("dt,dim,heads", [("f32", 288, 6), ("f32", 516, 3), ("bf16", 768, 12)])
+def test_llama_step_drops_what_lies_past_a_row(dt, dim, heads):
+    """Rows that are no whole number of batches of loads: an infinite weight at a row's start counts once, where it stands.
+    The key it makes infinite has a weight of exactly 0, so everything stays finite."""
+    from enzyme_ad.jax import llama
+    cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), _) = _inputs(dt, dim, 64, 1, heads, 5, 7)
+    _own_key_out_of_reach(wd, wr, xr, 5, heads)
+    check(llama.forward_step(x, cfg, wd, kc, vc), L.forward_step(xr, cfg, wr, kcr, vcr), dt, "y")
