@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict_
   mx = block_max(mx, scratch);
   float sum = 0.f;
   for (int s = threadIdx.x; s < s1 - s0; s += 256) {
-    const float p = __expf(scores[s] - mx);
+    const float p = scores[s] == -INFINITY ? 0.f : __expf(scores[s] - mx);      // a block may hold nothing else
     scores[s] = p;
     sum += p;
   }

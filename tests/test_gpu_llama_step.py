@@ -96,3 +96,11 @@ def test_llama_step_drops_what_lies_past_a_row(dt, dim, heads):
     cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), _) = _inputs(dt, dim, 64, 1, heads, 5, 7)
     _own_key_out_of_reach(wd, wr, xr, 5, heads)
     check(llama.forward_step(x, cfg, wd, kc, vc), L.forward_step(xr, cfg, wr, kcr, vcr), dt, "y")
+
+
+def test_llama_step_whose_last_block_holds_no_finite_score():
+    """Two pieces of a head per lane, and the token's own key alone in the last block of keys with a score of -infinity."""
+    from enzyme_ad.jax import llama
+    cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), _) = _inputs("f32", 384, 64, 1, 3, 256, 7)
+    _own_key_out_of_reach(wd, wr, xr, 256, 3)
+    check(llama.forward_step(x, cfg, wd, kc, vc), L.forward_step(xr, cfg, wr, kcr, vcr), "f32", "y")
