@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void attn_step_fwd_kernel(const T* __restrict_
     }
   }
   reduce_keys<MAXC, NE>(acc, nch, red);
-  if (gridDim.x == 1) {                                    // all keys in one block: nothing to combine
+  if (o != nullptr) {                                      // all keys in one block: nothing to combine
     if (threadIdx.x < 16) {
       const float inv = 1.0f / sum;
       T* orow = o + b * sh.q_sb + h * sh.q_sh;
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(256) void attn_step_fwd1_kernel(const T* __restrict
   for (int e = 0; e < NE; e++) acc[0][e] *= w;
   float bsum = block_sum(l16 == 0 ? sum * w : 0.f, scratch);
   reduce_keys<1, NE>(acc, mine ? 1 : 0, red);
-  if (gridDim.x == 1) {                                    // all keys in one block: nothing to combine
+  if (o != nullptr) {                                      // all keys in one block: nothing to combine
     if (threadIdx.x < 16) {
       const float inv = 1.0f / bsum;
 #pragma unroll
@@ -694,26 +694,29 @@ int check_step(const char* name, int64_t batch, int64_t heads, int64_t seq_kv, i
   return EMI_OK;
 }
 
-// Launches the forward kernel (sh.kpb keys per block) and, when the keys of a head span several blocks, the combine.
+// Launches the forward kernel (sh.kpb keys per block) and the combine.  A head whose keys are in one block has nothing to
+// combine: its block stores the result itself (o is then given to the kernel), in pieces of 16 bytes where it reads so;
+// an o that those do not fit goes through the combine, which stores single elements.
 int launch_step_fwd(hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, float* part, const StepShape& sh,
                     int bh, bool vec, float scale, int dtype) {
   const int ne = dtype == EMI_BF16 ? 8 : 4;
   const int nsplit = (sh.seq_kv + sh.kpb - 1) / sh.kpb;
+  const bool direct = nsplit == 1 && (!vec || al16(o));
   const dim3 grid((unsigned)nsplit, (unsigned)bh);
 #define EMI_STEP_FWD(T, VEC, NCH)                                                                                       \
   do {                                                                                                                   \
     hipLaunchKernelGGL((attn_step_fwd_kernel<T, VEC, NCH>), grid, dim3(256), 0, st, (const T*)q, (const T*)k,            \
-                       (const T*)v, part, (T*)o, lse, sh, scale);                                                        \
+                       (const T*)v, part, direct ? (T*)o : nullptr, lse, sh, scale);                                     \
     EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
-    if (nsplit > 1)                                                                                                      \
+    if (!direct)                                                                                                         \
       hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)o, lse, sh, nsplit); \
   } while (0)
 #define EMI_STEP_FWD1(T)                                                                                                \
   do {                                                                                                                   \
     hipLaunchKernelGGL(attn_step_fwd1_kernel<T>, grid, dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, part,    \
-                       (T*)o, lse, sh, scale);                                                                           \
+                       direct ? (T*)o : nullptr, lse, sh, scale);                                                        \
     EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
-    if (nsplit > 1)                                                                                                      \
+    if (!direct)                                                                                                         \
       hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)o, lse, sh, nsplit); \
   } while (0)
 #define EMI_STEP_FWD_T(T)                                              \

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import llama_ref as L
-from gpu_util import dev, host, check
+from gpu_util import dev, host, check, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -165,3 +165,22 @@ def test_step_form_forward_mode_adjoint_identity():
     rhs = float(np.sum(host(gx) * host(tx)) + np.sum(host(gkc) * host(tkc)) + np.sum(host(gvc) * host(tvc)) +
                 sum(np.sum(host(gw[k]) * host(tw[k])) for k in w))
     assert abs(lhs - rhs) <= 1e-4 * max(abs(lhs), abs(rhs)), (lhs, rhs)
+
+
+@pytest.mark.parametrize("dt,heads,d,keys", [("f32", 6, 48, 9), ("f32", 3, 128, 9), ("bf16", 4, 128, 9), ("bf16", 3, 176, 512), ("f32", 6, 48, 513)])
+def test_step_attention_takes_a_result_that_is_not_aligned(dt, heads, d, keys):
+    """o starts one element behind a 16-byte boundary, all operands on one: the values of an aligned o, nothing around them."""
+    from enzyme_ad.jax import _native as N, ops
+    rng = np.random.default_rng(d + keys)
+    q, k, v = (dev(rng.standard_normal(s), dt)[0] for s in ((heads * d,), (keys, heads * d), (keys, heads * d)))
+    want, want_lse = ops.attention_step(q, k, v, heads, return_lse=True)
+    room = torch.full((heads * d + 16,), 7.0, dtype=q.dtype, device="cuda")
+    o, lse = room[1:heads * d + 1], torch.empty((1, heads), dtype=torch.float32, device="cuda")
+    nbytes = N.lib().emi_attn_step_workspace_bytes(1, heads, keys, d)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    D = heads * d
+    N.check(N.lib().emi_attn_step_fwd(ops._stream(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), ws.data_ptr(), nbytes,
+                                      1, heads, keys, d, D, d, keys * D, d, D, 1.0 / float(np.sqrt(d)), ops._code(q)))
+    check(o, host(want), dt, "o")
+    assert torch.equal(room[:1], room.new_tensor([7.0])) and bool((room[D + 1:] == 7.0).all())
+    assert rel_err(host(lse), host(want_lse)) < 1e-5
