@@ -73,8 +73,9 @@ def forward_step(x, config, weights, key_cache, value_cache, eps=1e-5, theta=100
         raise ValueError("forward_step: n_kv_heads must equal n_heads")
     dim = x.shape[-1]
     pos = key_cache.shape[1]
-    stacks = [weights[k] for k in ops.STEP_WEIGHTS]
-    if ops.llama_step_applies(x, stacks, key_cache, value_cache, n_heads):
+    stacks = [weights[k] for k in ops.STEP_WEIGHTS] if n_layers else None
+    # (the operator runs every layer of the stacks: a config of fewer or more takes the ones below)
+    if stacks and key_cache.shape[0] == n_layers and ops.llama_step_applies(x, stacks, key_cache, value_cache, n_heads):
         table = ops.rope_table(1, dim // n_heads, theta, pos, x.device)
         return ops.llama_step(x, stacks, key_cache, value_cache, n_heads, table, eps)
     for i in range(n_layers):

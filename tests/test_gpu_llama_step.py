@@ -104,3 +104,22 @@ def test_llama_step_whose_last_block_holds_no_finite_score():
     cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), _) = _inputs("f32", 384, 64, 1, 3, 256, 7)
     _own_key_out_of_reach(wd, wr, xr, 256, 3)
     check(llama.forward_step(x, cfg, wd, kc, vc), L.forward_step(xr, cfg, wr, kcr, vcr), "f32", "y")
+
+
+@pytest.mark.parametrize("n_layers", [0, 1, 2, 5])
+def test_llama_step_runs_as_many_layers_as_the_config_says(n_layers):
+    """Fewer layers than the stacks hold leave the rest alone; more go round them (`ops.select`), with and without a tape."""
+    from enzyme_ad.jax import llama, vjp
+    cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), (dy, dyr)) = _inputs("f32", 96, 64, 3, 2, 5, 3)
+    cfg = dict(cfg, n_layers=n_layers)
+    turn = [i % 3 for i in range(n_layers)]
+    wt = {k: a if k == "rms_final_weight" else a[turn] for k, a in wr.items()}
+    y, pull = vjp(lambda x, w, k, v: llama.forward_step(x, cfg, w, k, v), x, wd, kc, vc)
+    check(llama.forward_step(x, cfg, wd, kc, vc), L.forward_step(xr, cfg, wt, kcr[turn], vcr[turn]), "f32", "y")
+    if n_layers in (1, 2):
+        gw = pull(dy)[1]
+        ref = L.forward_step_vjp(xr, cfg, wt, kcr[turn], vcr[turn], dyr)[2]
+        assert torch.equal(y, llama.forward_step(x, cfg, wd, kc, vc))
+        for k in ("wq", "w2"):
+            check(gw[k][:n_layers], ref[k], "f32", "d" + k)
+            assert not gw[k][n_layers:].any()
