@@ -16,8 +16,9 @@ LAYER_KEYS = ("rms_att_weight", "wq", "wk", "wv", "wo", "rms_ffn_weight", "w1", 
 def layer(x, lw, n_heads, eps=1e-5, theta=10000.0):
     """One decoder layer (test/llama.py:144-233).  x: [B, S, dim]."""
     weights = [lw[k] for k in LAYER_KEYS]
-    # (slices of stacks keep the operators below, which gather the weight gradients of all layers into grouped launches)
-    if not any(hasattr(w, "_emi_stack") for w in weights) and ops.llama_layers_apply(x, weights, n_heads):
+    # (slices of stacks keep the operators below, which gather the weight gradients of all layers into grouped launches;
+    # whole stacks are no layer, and refused there)
+    if weights[6].dim() == 2 and not any(hasattr(w, "_emi_stack") for w in weights) and ops.llama_layers_apply(x, weights, n_heads):
         return ops.llama_layers(x, weights, n_heads, ops.rope_table(x.shape[1], x.shape[2] // n_heads, theta, 0, x.device), eps)
     xb = ops.rmsnorm(x, lw["rms_att_weight"], eps)                 # :145
     att = ops.attention_block(xb, lw["wq"], lw["wk"], lw["wv"], n_heads, theta)     # :149-209 (RoPE in the epilogues)
@@ -34,8 +35,8 @@ def forward(x, config, weights, logits=False, eps=1e-5, theta=10000.0):
     n_layers, n_heads = config["n_layers"], config["n_heads"]
     if not x.is_floating_point():
         x = ops.embedding(x, weights["token_embedding_table"])
-    stacks = [weights[k] for k in LAYER_KEYS]
-    if stacks[6].shape[0] == n_layers and ops.llama_layers_apply(x, stacks, n_heads):
+    stacks = [weights[k] for k in LAYER_KEYS] if n_layers else None
+    if stacks and stacks[6].dim() == 3 and stacks[6].shape[0] == n_layers and ops.llama_layers_apply(x, stacks, n_heads):
         x = ops.llama_layers(x, stacks, n_heads, ops.rope_table(x.shape[1], x.shape[2] // n_heads, theta, 0, x.device), eps)
     else:
         for i in range(n_layers):

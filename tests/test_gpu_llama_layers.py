@@ -101,3 +101,15 @@ def test_llama_layers_of_a_text():
     a = float((c.double() * tangent.double()).sum())
     b = sum(float((g.double() * t.double()).sum()) for g, t in zip(grads, tangents))
     assert abs(a - b) <= 1e-4 * max(abs(a), float(c.double().norm() * tangent.double().norm()) * 1e-2)
+
+
+def test_a_stack_is_no_layer_and_a_layer_no_stack():
+    """`llama.layer` takes one layer's weights and `llama.forward` stacks of them; neither takes the other's."""
+    from enzyme_ad.jax import llama
+    cfg, wd, _, x, _, _, _ = _inputs("f32", 64, 72, 2, 2, 1, 33)
+    with pytest.raises(ValueError):
+        llama.layer(x, wd, 2)
+    final = dict(rms_final_weight=torch.ones(64, device="cuda"))
+    with pytest.raises(ValueError):
+        llama.forward(x, dict(cfg, n_layers=72), dict({k: w[0] for k, w in wd.items()}, **final))
+    assert torch.equal(llama.forward(x, dict(cfg, n_layers=0), final), llama.ops.rmsnorm(x, final["rms_final_weight"]))
