@@ -19,7 +19,7 @@ def layer(x, lw, n_heads, eps=1e-5, theta=10000.0):
     # (slices of stacks keep the operators below, which gather the weight gradients of all layers into grouped launches;
     # whole stacks are no layer, and refused there)
     if weights[6].dim() == 2 and not any(hasattr(w, "_emi_stack") for w in weights) and ops.llama_layers_apply(x, weights, n_heads):
-        return ops.llama_layers(x, weights, n_heads, ops.rope_table(x.shape[1], x.shape[2] // n_heads, theta, 0, x.device), eps)
+        return ops._llama_layers(x, weights, n_heads, ops.rope_table(x.shape[1], x.shape[2] // n_heads, theta, 0, x.device), eps)
     xb = ops.rmsnorm(x, lw["rms_att_weight"], eps)                 # :145
     att = ops.attention_block(xb, lw["wq"], lw["wk"], lw["wv"], n_heads, theta)     # :149-209 (RoPE in the epilogues)
     x = ops.matmul_nt(att, lw["wo"], residual=x)                   # :211-215
@@ -37,7 +37,7 @@ def forward(x, config, weights, logits=False, eps=1e-5, theta=10000.0):
         x = ops.embedding(x, weights["token_embedding_table"])
     stacks = [weights[k] for k in LAYER_KEYS] if n_layers else None
     if stacks and stacks[6].dim() == 3 and stacks[6].shape[0] == n_layers and ops.llama_layers_apply(x, stacks, n_heads):
-        x = ops.llama_layers(x, stacks, n_heads, ops.rope_table(x.shape[1], x.shape[2] // n_heads, theta, 0, x.device), eps)
+        x = ops._llama_layers(x, stacks, n_heads, ops.rope_table(x.shape[1], x.shape[2] // n_heads, theta, 0, x.device), eps)
     else:
         for i in range(n_layers):
             lw = {k: ops.select(weights[k], i) for k in LAYER_KEYS}
@@ -78,7 +78,7 @@ def forward_step(x, config, weights, key_cache, value_cache, eps=1e-5, theta=100
     # (the operator runs every layer of the stacks: a config of fewer or more takes the ones below)
     if stacks and key_cache.shape[0] == n_layers and ops.llama_step_applies(x, stacks, key_cache, value_cache, n_heads):
         table = ops.rope_table(1, dim // n_heads, theta, pos, x.device)
-        return ops.llama_step(x, stacks, key_cache, value_cache, n_heads, table, eps)
+        return ops._llama_step(x, stacks, key_cache, value_cache, n_heads, table, eps)
     for i in range(n_layers):
         lw = {k: ops.select(weights[k], i) for k in LAYER_KEYS}
         xb = ops.rmsnorm(x, lw["rms_att_weight"], eps)                                    # :145

@@ -1131,7 +1131,19 @@ def llama_step(x, weights, key_cache, value_cache, n_heads, table, eps=1e-5, sca
     products, which here stays in fp32 (emi_llama_step_fwd / _bwd)."""
     weights = list(weights)
     _dev(x, *weights, key_cache, value_cache, table)
+    _same_dtype(x, *weights, key_cache, value_cache)
+    if len(weights) != len(STEP_WEIGHTS) or not llama_step_applies(x, weights, key_cache, value_cache, n_heads):
+        raise ValueError("llama_step: x %s, caches %s / %s, %d heads and these weights, or forward mode, are not served (see llama_step_applies)" %
+                         (tuple(x.shape), tuple(key_cache.shape), tuple(value_cache.shape), n_heads))
+    return _llama_step(x, weights, key_cache, value_cache, n_heads, table, eps, scale)
+
+
+def _llama_step(x, weights, key_cache, value_cache, n_heads, table, eps=1e-5, scale=None):
+    """llama_step on operands that llama_step_applies has accepted."""
     L_, pos, D = key_cache.shape
+    if table.dtype != torch.float32 or table.shape[-1:] != (2,) or not table.is_contiguous() or not table.is_cuda or table.numel() == 0 or \
+            (D // 2) % (table.numel() // 2):
+        raise ValueError("llama_step: table %s/%s for rows of %d pairs" % (tuple(table.shape), table.dtype, D // 2))
     H = weights[6].shape[1]
     lib, code = N.lib(), _code(x)
     if scale is None:
@@ -1183,7 +1195,18 @@ def llama_layers(x, weights, n_heads, table, eps=1e-5, scale=None):
     _PENDING_DW_BYTES of cotangents allow."""
     weights = list(weights)
     _dev(x, *weights, table)
+    _same_dtype(x, *weights)
+    if len(weights) != 9 or not llama_layers_apply(x, weights, n_heads):
+        raise ValueError("llama_layers: x %s with %d heads and these weights, or forward mode, are not served (see llama_layers_apply)" %
+                         (tuple(x.shape), n_heads))
+    return _llama_layers(x, weights, n_heads, table, eps, scale)
+
+
+def _llama_layers(x, weights, n_heads, table, eps=1e-5, scale=None):
+    """llama_layers on operands that llama_layers_apply has accepted."""
     B, S, D = x.shape
+    if table.dtype != torch.float32 or tuple(table.shape) != (S, D // n_heads // 2, 2) or not table.is_contiguous() or not table.is_cuda:
+        raise ValueError("llama_layers: table %s/%s for x %s with %d heads" % (tuple(table.shape), table.dtype, tuple(x.shape), n_heads))
     L_, H = (weights[6].shape[0] if weights[6].dim() == 3 else 1), weights[6].shape[-2]
     lib, code = N.lib(), _code(x)
     if scale is None:

@@ -1957,10 +1957,10 @@ class Executable:
         if n == "call":
             return self.run(xs, op.attrs["callee"])
         if n == "emi.llama_layers":
-            return [ops.llama_layers(xs[0], xs[1:], op.attrs["heads"], self._table(op, device), op.attrs["eps"], op.attrs["scale"])]
+            return [ops._llama_layers(xs[0], xs[1:], op.attrs["heads"], self._table(op, device), op.attrs["eps"], op.attrs["scale"])]
         if n == "emi.llama_step":
             a = op.attrs
-            y = ops.llama_step(xs[0], xs[1:11], xs[11], xs[12], a["heads"], self._table(op, device), a["eps"], a["scale"])
+            y = ops._llama_step(xs[0], xs[1:11], xs[11], xs[12], a["heads"], self._table(op, device), a["eps"], a["scale"])
             return [y if op.types[0].shape == tuple(y.shape) else ops.reshape(y, op.types[0].shape)]
         if n == "custom_call":
             return self._custom_call(op, xs)

@@ -113,3 +113,23 @@ def test_a_stack_is_no_layer_and_a_layer_no_stack():
     with pytest.raises(ValueError):
         llama.forward(x, dict(cfg, n_layers=72), dict({k: w[0] for k, w in wd.items()}, **final))
     assert torch.equal(llama.forward(x, dict(cfg, n_layers=0), final), llama.ops.rmsnorm(x, final["rms_final_weight"]))
+
+
+def test_llama_layers_refuse_what_they_do_not_serve():
+    """Operands that the call would read out of range or mistake for something else raise on the host."""
+    from enzyme_ad.jax import llama, ops
+    _, wd, _, x, _, _, _ = _inputs("f32", 64, 72, 2, 2, 1, 33)
+    w, table = [wd[k] for k in llama.LAYER_KEYS], ops.rope_table(33, 32, device=x.device)
+    ops.llama_layers(x, w, 2, table)
+    for bad in (ops.rope_table(32, 32, device=x.device), ops.rope_table(33, 16, device=x.device), table.double(), table.bfloat16(), table.reshape(33, 32)):
+        with pytest.raises(ValueError):
+            ops.llama_layers(x, w, 2, bad)
+    for i, t in ((6, w[6][:, :-8].contiguous()), (7, w[6]), (1, w[1][:1].contiguous()), (0, w[0][:, :60].contiguous())):
+        with pytest.raises(ValueError):
+            ops.llama_layers(x, w[:i] + [t] + w[i + 1:], 2, table)
+    with pytest.raises(ValueError):
+        ops.llama_layers(x, w[:8], 2, table)
+    with pytest.raises(TypeError):
+        ops.llama_layers(x.bfloat16(), w, 2, table)
+    with ops.Forward(), pytest.raises(ValueError):
+        ops.llama_layers(x, w, 2, table)

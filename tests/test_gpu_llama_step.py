@@ -123,3 +123,25 @@ def test_llama_step_runs_as_many_layers_as_the_config_says(n_layers):
         for k in ("wq", "w2"):
             check(gw[k][:n_layers], ref[k], "f32", "d" + k)
             assert not gw[k][n_layers:].any()
+
+
+def test_llama_step_refuses_what_it_does_not_serve():
+    """Operands that the call would read out of range or mistake for something else raise on the host."""
+    from enzyme_ad.jax import ops
+    _, wd, _, ((x, _), (kc, _), (vc, _), _) = _inputs("f32", 96, 64, 2, 2, 5, 3)
+    w, table = [wd[k] for k in ops.STEP_WEIGHTS], ops.rope_table(1, 48, pos0=5, device=x.device)
+    ops.llama_step(x, w, kc, vc, 2, table)
+    for bad in (table.double(), table.bfloat16(), table[:, :7].contiguous(), table[:, :0], table.reshape(-1, 1)):
+        with pytest.raises(ValueError):
+            ops.llama_step(x, w, kc, vc, 2, bad)
+    for i, t in ((6, w[6][:, :-4].contiguous()), (7, w[6]), (1, w[1][:1].contiguous()), (9, w[9][:95].contiguous())):
+        with pytest.raises(ValueError):
+            ops.llama_step(x, w[:i] + [t] + w[i + 1:], kc, vc, 2, table)
+    with pytest.raises(ValueError):
+        ops.llama_step(x, w[:9], kc, vc, 2, table)
+    with pytest.raises(ValueError):
+        ops.llama_step(x, w, kc, vc[:, :-1].contiguous(), 2, table)
+    with pytest.raises(TypeError):
+        ops.llama_step(x.bfloat16(), w, kc, vc, 2, table)
+    with ops.Forward(), pytest.raises(ValueError):
+        ops.llama_step(x, w, kc, vc, 2, table)
