@@ -1715,8 +1715,7 @@ static int launch_bf16_kcontig(hipStream_t st, const void* A, const void* B, con
   const int pps = pingpong_splits(M, N, K, trans_b);
   if (pps > 1 && workspace_holds(workspace, workspace_bytes, pps, M, N))
     return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, static_cast<float*>(workspace), pps);
-  Bf16Plan plan = bf16_plan(M, N, K, 1, 0, trans_b);
-  if (plan.splits > 1 && !workspace_holds(workspace, workspace_bytes, plan.splits, M, N)) plan.splits = 1;
+  const Bf16Plan plan = bf16_plan(M, N, K, 1, 0, trans_b, splits_held(workspace, workspace_bytes, M, N));
   float* part = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
   if (plan.shape == 0) {
     if (part != nullptr)
@@ -1802,7 +1801,7 @@ extern "C" size_t emi_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
   int splits = generic_splits(M, N, K);
   if (dtype == EMI_BF16) {
     int s = trans_a ? bf16_splits(M, N, K) : pingpong_splits(M, N, K, trans_b);
-    if (!trans_a && s == 1) s = bf16_plan(M, N, K, 1, 0, trans_b).splits;
+    if (!trans_a && s == 1) s = bf16_plan(M, N, K, 1, 0, trans_b, kAnySplits).splits;
     if (s > splits) splits = s;
   }
   const size_t need = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
@@ -1962,7 +1961,7 @@ extern "C" size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t
                                                     int dtype) {
   size_t need = emi_gemm_workspace_bytes(M, N, K, trans_a, trans_b, dtype);          // the one-by-one fallback
   if (count >= 2 && count <= kMaxGroup && dtype == EMI_BF16 && M > 0 && N > 0 && K > 0) {
-    const int splits = trans_a ? (sum ? 1 : count * grouped_splits(M, N, K, count)) : bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b).splits;
+    const int splits = trans_a ? (sum ? 1 : count * grouped_splits(M, N, K, count)) : bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b, kAnySplits).splits;
     const size_t grouped = splits > (trans_a && !sum ? count : 1) ? (size_t)splits * M * N * sizeof(float) : 0;
     if (grouped > need) need = grouped;
   }
@@ -2021,8 +2020,7 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
       if (!trans_a) {
         int vec_ok = ldc % 8 == 0 && ldr % 8 == 0;
         for (int i = 0; i < nout; i++) vec_ok = vec_ok && al16(C[i]) && al16(g.R[i]);
-        Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b);
-        if (plan.splits > 1 && !workspace_holds(workspace, workspace_bytes, plan.splits, M, N)) plan.splits = 1;
+        const Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b, splits_held(workspace, workspace_bytes, M, N));
         if (plan.shape == 0)
           return trans_b ? launch_bf16_pingpong_grouped<false, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok)
                          : launch_bf16_pingpong_grouped<false, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok);

@@ -393,7 +393,7 @@ static int launch_pipe_shape(hipStream_t st, const PipeCall& c, int trans_b) {
 // 5 a 32 x 32 tile whose eight wavefronts share stages of 256 k (0.55).  The reduction over splits is a launch of its own;
 // results over 4 M elements, whose planes leave the caches, are not split (but see pingpong_splits of gemm.hip), nor are
 // the products of a few tokens, which have kernels of their own (gemm_skinny.hip).
-Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b) {
+Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b, int64_t most) {
   struct Shape { int bm, bn, bk; double fixed, rate[3], more; };        // rate[b - 1]: per stage, b blocks on the CU; more: per block from four on
   static const Shape shapes[6] = {{256, 256, 64, 4.0, {1.0, 2.0, 3.0}, 1.0},  {128, 128, 64, 4.0, {0.61, 0.90, 1.45}, 0.50},
                                   {128, 128, 64, 3.5, {0.57, 1.14, 1.71}, 0.57}, {128, 64, 64, 3.0, {0.36, 0.62, 1.0}, 0.33},
@@ -408,7 +408,7 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
     const int64_t blocks = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * (sum ? 1 : count);
     if (blocks > 0x3fffffff) continue;
     const bool split = may_split && (c != 0 || trans_b);
-    for (int64_t z = 1; z <= 16 && (z == 1 || (split && steps >= 4 * z)); z++) {
+    for (int64_t z = 1; z <= 16 && z <= most && (z == 1 || (split && steps >= 4 * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
       double stage = b < 4 ? s.rate[b - 1] : s.more * b;
       if (c == 0) stage *= 1.0 + 0.45 * (blocks * z < 256 ? blocks * z / 256.0 : 1.0);

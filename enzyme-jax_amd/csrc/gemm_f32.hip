@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "emi_device.h"
+#include "gemm_plan.h"
 
 namespace emi {
 
@@ -328,10 +329,7 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 // block from four on, a stage of 64 k of a 32 x 32 tile whose wavefronts share k 0.42 alone, 0.36 a block from three on.
 // The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s); results over 4 M elements, whose planes
 // leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split.
-struct F32Plan {
-  int config, splits;
-};
-static F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum) {
+F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int64_t most) {
   struct Shape { int tile, bk; double fixed, rate[4]; };              // rate[b - 1]: per stage, b blocks on the CU; the last one per block
   static const Shape shapes[3] = {{128, 32, 4.0, {2.0, 3.84, 5.76, 1.92}}, {64, 32, 3.0, {0.72, 1.13, 1.60, 0.54}}, {32, 64, 2.5, {0.42, 0.72, 1.08, 0.36}}};
   F32Plan best{2, 1};
@@ -342,7 +340,7 @@ static F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum) {
     const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
     const int64_t blocks = (M + s.tile - 1) / s.tile * ((N + s.tile - 1) / s.tile) * (sum ? 1 : count);
     if (blocks > 0x3fffffff) continue;
-    for (int64_t z = 1; z <= 64 && (z == 1 || (may_split && steps >= 4 * z)); z++) {
+    for (int64_t z = 1; z <= 64 && z <= most && (z == 1 || (may_split && steps >= 4 * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
       const double t = s.fixed + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
@@ -355,7 +353,7 @@ static F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum) {
 }
 
 size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum) {
-  const int z = f32_plan(M, N, K, count, sum).splits;
+  const int z = f32_plan(M, N, K, count, sum, kAnySplits).splits;
   return z > 1 ? (size_t)z * M * N * sizeof(float) : 0;
 }
 
@@ -380,10 +378,7 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   }
   g.count = count;
   g.sum = sum;
-  F32Plan p = f32_plan(M, N, K, count, sum);
-  if (p.splits > 1 && (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
-                       workspace_bytes < (size_t)p.splits * M * N * sizeof(float)))
-    p.splits = 1;
+  const F32Plan p = f32_plan(M, N, K, count, sum, splits_held(workspace, workspace_bytes, M, N));
   const F32Call c{g.A[0], g.B[0], g.R[0], g.C[0], (int)M, (int)N, (int)K, (int)lda, (int)ldb, ldr, ldc, static_cast<float*>(workspace),
                   p.splits, count > 1 ? &g : nullptr};
   switch (p.config) {

@@ -1,4 +1,4 @@
-// What gemm.hip and gemm_bf16_pipe.hip agree on about a bf16 product whose A is k-contiguous.
+// Which blocks and how many splits of K a product runs on: bf16 products whose A is k-contiguous, and fp32 products.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -9,7 +9,24 @@ struct Bf16Plan {
   int shape;        // 0: the 256 x 256 ping-pong kernel of gemm.hip; otherwise a block shape of gemm_bf16_pipe.hip
   int splits;       // splits of K
 };
-Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b);
+struct F32Plan {
+  int config;       // 0: blocks of 128 x 128, 1: 64 x 64, 2: 32 x 32 (gemm_f32.hip)
+  int splits;
+};
+
+// The best of the plans with at most `most` splits.  A shape that was chosen for its splits is a poor one without them, so
+// a call plans with the splits that its workspace holds, and one without a workspace for a single pass over K (us, planned
+// so | the blocks of the split plan in a single pass, B k-contiguous; bf16: 256 x 11008 x 4096 36 | 65, 300 x 4096 x 11008
+// 60 | 104, 512 x 768 x 32000 89 | 238; fp32: 256 x 4096 x 11008 247 | 677, 512 x 768 x 32000 330 | 1955).
+constexpr int64_t kAnySplits = 1 << 20;
+Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b, int64_t most);      // gemm_bf16_pipe.hip
+F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int64_t most);                     // gemm_f32.hip
+
+inline int64_t splits_held(const void* workspace, size_t bytes, int64_t M, int64_t N) {
+  if (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0) return 1;
+  const int64_t n = (int64_t)(bytes / ((size_t)M * N * sizeof(float)));
+  return n < 1 ? 1 : n < kAnySplits ? n : kAnySplits;
+}
 
 int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void* const* A, const void* const* B, const void* const* R,
                      void* const* C, float* part, int M, int N, int K, int lda, int ldb, int64_t ldr, int64_t ldc, int vec_ok, int trans_b,

@@ -158,6 +158,33 @@ def test_gemm_padded_leading_dimensions(ops, dt, ta, tb, M, N, K, pad):
     assert bool((C[:, N:] == 7.0).all()), "wrote outside the window"
 
 
+@pytest.mark.parametrize("planes", [0, 2])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("tb,M,N,K,count", [(1, 300, 1000, 4104, 1), (0, 300, 1000, 4104, 1), (1, 520, 1400, 4104, 2), (1, 48, 104, 8200, 1)])
+def test_gemm_with_room_for_few_planes(dt, tb, M, N, K, count, planes):
+    """Products that are split over K where the workspace allows it (count: summed into one), with none and with room for
+    two planes: the same product, and nothing written past the room."""
+    import ctypes
+    import torch
+    from enzyme_ad.jax import _native as nat
+    _say("gemm, few planes", dt, tb, M, N, K, count, planes)
+    rng = np.random.default_rng(M + K + tb)
+    As, Ars = zip(*[dev(rng.standard_normal((M, K)), dt) for _ in range(count)])
+    Bs, Brs = zip(*[dev(rng.standard_normal((N, K) if tb else (K, N)), dt) for _ in range(count)])
+    ref = sum(a @ (b.T if tb else b) for a, b in zip(Ars, Brs))
+    lib = nat.lib()
+    code = nat.EMI_F32 if dt == "f32" else nat.EMI_BF16
+    room = planes * M * N * 4
+    assert lib.emi_gemm_grouped_workspace_bytes(count, M, N, K, 0, tb, int(count > 1), code) > room
+    ws = torch.full((room + 4096,), 7, dtype=torch.uint8, device="cuda")
+    C = torch.empty((M, N), dtype=As[0].dtype, device="cuda")
+    table = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    nat.check(lib.emi_gemm_grouped(torch.cuda.current_stream().cuda_stream, count, table(As), table(Bs), None, table([C]),
+                                   ws.data_ptr() if planes else None, room, M, N, K, K, K if tb else N, N, N, 0, tb, int(count > 1), code))
+    check(C, ref, dt, "gemm")
+    assert bool((ws[room:] == 7).all())
+
+
 GROUPED_SHAPES = [
     (256, 384, 320),     # one launch of the 128-tile kernel, K not a multiple of 64
     (200, 136, 72),      # ragged tiles

@@ -76,6 +76,32 @@ def test_plain_launchers_reject_bad_arguments_before_touching_the_gpu():
     assert lib.emi_gemm_workspace_bytes(8192, 768, 32000, 0, 1, 11) == 0
 
 
+class _Plan(C.Structure):
+    _fields_ = [("shape", C.c_int), ("splits", C.c_int)]
+
+
+@pytest.mark.parametrize("dtype,M,N,K,count,total", [
+    ("bf16", 256, 11008, 4096, 1, 0), ("bf16", 300, 11008, 4096, 1, 0), ("bf16", 300, 1000, 16392, 1, 0), ("bf16", 512, 768, 32000, 1, 0),
+    ("bf16", 300, 4096, 11008, 2, 1), ("f32", 256, 4096, 11008, 1, 0), ("f32", 512, 768, 32000, 1, 0), ("f32", 300, 4096, 4096, 3, 1)])
+def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K, count, total):
+    """Without room for the planes the blocks are not those that the splits were to multiply: there are more of them, enough
+    for half of the 256 CUs or the smallest ones there are.  With room for some planes there are at most as many splits."""
+    lib = _lib()
+    plan, blocks, trans_b = ((lib._ZN3emi9bf16_planEllliiil, [(256, 256), (128, 128), (128, 128), (128, 64), (64, 64), (32, 32)], (1,))
+                             if dtype == "bf16" else (lib._ZN3emi8f32_planEllliil, [(128, 128), (64, 64), (32, 32)], ()))
+    plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * (2 + len(trans_b)) + [C.c_int64]
+    tiles = lambda p: -(-M // blocks[p.shape][0]) * -(-N // blocks[p.shape][1])
+    free, one = (plan(M, N, K, count, total, *trans_b, most) for most in (1 << 20, 1))
+    assert free.splits > 1 and one.splits == 1
+    assert tiles(one) > tiles(free) and (tiles(one) >= 128 or one.shape == len(blocks) - 1)
+    for most in range(2, free.splits + 2):
+        assert 1 <= plan(M, N, K, count, total, *trans_b, most).splits <= most
+    code = 16 if dtype == "bf16" else 11
+    need = (lib.emi_gemm_grouped_workspace_bytes(count, M, N, K, 0, 1, total, code) if count > 1 else
+            lib.emi_gemm_workspace_bytes(M, N, K, 0, 1, code))
+    assert need >= free.splits * M * N * 4
+
+
 def _handler(name):
     lib = _lib()
     fn = getattr(lib, name)
