@@ -1252,17 +1252,26 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const T* __restrict__
 // chunk contracts k = k0 + 4 g + t, so a k-contiguous operand is read in 16-byte pieces and a k-major one in 128-byte
 // rows.  The four partial tiles are added in wavefront order through LDS (fixed order: run-to-run identical bits).
 // ---------------------------------------------------------------------------
-template <bool A_KMAJOR, bool B_KMAJOR>
-__global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float* __restrict__ A, const float* __restrict__ B, const float* R,
-                                                             float* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldr,
-                                                             int64_t ldc, float* __restrict__ part, int kps) {
-  constexpr int NW = 4, U = 4;          // wavefronts that share K; 8-wide chunks in flight per step
+// GROUPED: blockIdx.z picks one of grp.count independent products of one shape (GemmGroup with sum == 0, its pointers read
+// as float).  NW wavefronts share K, U 8-wide chunks are in flight per step.  ONCE: a wavefront's share of K is at most U
+// chunks (K <= 8 U NW), so everything is requested up front and the block waits for memory once.
+template <bool A_KMAJOR, bool B_KMAJOR, bool GROUPED, int NW, int U, bool ONCE>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_small_kernel(const float* __restrict__ A, const float* __restrict__ B, const float* R,
+                                                                 float* C, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldr,
+                                                                 int64_t ldc, float* __restrict__ part, int kps,
+                                                                 std::conditional_t<GROUPED, GemmGroup, NoGroup> grp) {
   __shared__ float red[NW - 1][16][64];
+  if constexpr (GROUPED) {
+    A = reinterpret_cast<const float*>(grp.A[blockIdx.z]);
+    B = reinterpret_cast<const float*>(grp.B[blockIdx.z]);
+    R = reinterpret_cast<const float*>(grp.R[blockIdx.z]);
+    C = reinterpret_cast<float*>(grp.C[blockIdx.z]);
+  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = lane & 31, g = lane >> 5;
   const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
   const int mi = m0 + i < M ? m0 + i : M - 1, ni = n0 + i < N ? n0 + i : N - 1;      // clamped: those results are not stored
-  // split-K (part != nullptr): plane blockIdx.z takes kps (a multiple of 8 NW) of K and leaves its
+  // split-K (part != nullptr, not GROUPED): plane blockIdx.z takes kps (a multiple of 8 NW) of K and leaves its
   // 32 x 32 partial in part[z][M][N] for gemm_splitk_reduce_kernel
   const int kb = part != nullptr ? (int)blockIdx.z * kps : 0;
   const int kend = part != nullptr && kb + kps < K ? kb + kps : K;
@@ -1298,19 +1307,28 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float* __rest
     }
   };
   if (ks < ke) load(ks, a, b);
-  float an[U][4], bn[U][4];
-  for (int k0 = ks; k0 < ke; k0 += 8 * U) {
-    const bool more = k0 + 8 * U < ke;
-    if (more) load(k0 + 8 * U, an, bn);            // in flight while this step is multiplied
-#pragma unroll
-    for (int u = 0; u < U; u++)
-#pragma unroll
-      for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][t], b[u][t], acc, 0, 0, 0);
-    if (more) {
+  if constexpr (ONCE) {
+    if (ks < ke) {
 #pragma unroll
       for (int u = 0; u < U; u++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) { a[u][t] = an[u][t]; b[u][t] = bn[u][t]; }
+        for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][t], b[u][t], acc, 0, 0, 0);
+    }
+  } else {
+    float an[U][4], bn[U][4];
+    for (int k0 = ks; k0 < ke; k0 += 8 * U) {
+      const bool more = k0 + 8 * U < ke;
+      if (more) load(k0 + 8 * U, an, bn);            // in flight while this step is multiplied
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][t], b[u][t], acc, 0, 0, 0);
+      if (more) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int t = 0; t < 4; t++) { a[u][t] = an[u][t]; b[u][t] = bn[u][t]; }
+      }
     }
   }
   if (wave > 0) {
@@ -1761,6 +1779,41 @@ static int launch_generic(hipStream_t st, const void* A, const void* B, const vo
   return EMI_OK;
 }
 
+// gemm_f32_small_kernel on one product (grp == nullptr; with `part` in grid_z planes of kps) or on a group of them.
+static int launch_f32_small(hipStream_t st, const GemmGroup* grp, const void* A, const void* B, const void* R, void* C, int M, int N, int K,
+                            int64_t lda, int64_t ldb, int64_t ldr, int64_t ldc, int trans_a, int trans_b, float* part, int kps, int grid_z) {
+  const dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)grid_z);
+#define EMI_F32_SMALL(AKM, BKM, GROUPED, NWV, UV, ONCEV, GRP)                                                                \
+  hipLaunchKernelGGL((gemm_f32_small_kernel<AKM, BKM, GROUPED, NWV, UV, ONCEV>), grid, dim3(NWV * 64), 0, st,                \
+                     static_cast<const float*>(A), static_cast<const float*>(B), static_cast<const float*>(R),              \
+                     static_cast<float*>(C), M, N, K, lda, ldb, ldr, ldc, part, kps, GRP)
+#define EMI_F32_SMALL_G(AKM, BKM, NWV, UV, ONCEV)                                      \
+  do {                                                                                 \
+    if (grp != nullptr) EMI_F32_SMALL(AKM, BKM, true, NWV, UV, ONCEV, *grp);           \
+    else EMI_F32_SMALL(AKM, BKM, false, NWV, UV, ONCEV, NoGroup{});                    \
+  } while (0)
+#define EMI_F32_SMALL_T(NWV, UV, ONCEV)                                                \
+  do {                                                                                 \
+    if (!trans_a && trans_b) EMI_F32_SMALL_G(false, false, NWV, UV, ONCEV);            \
+    else if (!trans_a && !trans_b) EMI_F32_SMALL_G(false, true, NWV, UV, ONCEV);       \
+    else if (trans_a && !trans_b) EMI_F32_SMALL_G(true, true, NWV, UV, ONCEV);         \
+    else EMI_F32_SMALL_G(true, false, NWV, UV, ONCEV);                                 \
+  } while (0)
+  // Few blocks and a contraction of more than a step or two: everything is requested at once, by eight wavefronts where it
+  // is longer; up to 256 the step form is the faster one, and with many blocks, whose other wavefronts hide the loads (us,
+  // at once | in steps, A and B k-major: 256 x 1001 x 768 9.7 | 12.7, 999 x 501 x 300 9.7 | 10.7, 257 x 289 x 256 7.2 | 6.3,
+  // 100 x 101 x 64 6.7 | 4.5).  A group takes one launch: 12 x 257 x 289 x 256 18.5 us against 76 one by one.
+  const bool few = part == nullptr && K > 256 && (int64_t)grid.x * grid.y * grid.z <= 1024;
+  if (few && K <= 384) EMI_F32_SMALL_T(4, 12, true);
+  else if (few && K <= 768) EMI_F32_SMALL_T(8, 12, true);
+  else EMI_F32_SMALL_T(4, 4, false);
+#undef EMI_F32_SMALL_T
+#undef EMI_F32_SMALL_G
+#undef EMI_F32_SMALL
+  EMI_CHECK_LAUNCH("emi_gemm(fp32, odd rows)");
+  return EMI_OK;
+}
+
 // gemm_f32.hip and gemm_bf16_pipe.hip add their planes with the same kernel
 int launch_bf16_splitk_reduce(hipStream_t st, const float* part, const uint16_t* R, uint16_t* C, int M, int N, int splits, int64_t ldr,
                               int64_t ldc) {
@@ -1865,30 +1918,16 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
   if (K > 0 && (M + 31) / 32 <= 65535 &&
       (trans_a || ((reinterpret_cast<uintptr_t>(A) & 15) == 0 && lda % 4 == 0)) &&
       (!trans_b || ((reinterpret_cast<uintptr_t>(B) & 15) == 0 && ldb % 4 == 0))) {
-    dim3 grid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32));
     const int splits = generic_splits(M, N, K);
-    float* part = nullptr;
-    int kps = 0;
-    if (splits > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
-        workspace_bytes >= (size_t)splits * M * N * sizeof(float)) {
+    if (splits > 1 && workspace_holds(workspace, workspace_bytes, splits, M, N)) {
       // few tiles and a long contraction: planes of K, added in fixed order by the reduce kernel
-      kps = (int)((((K + splits - 1) / splits) + 31) / 32 * 32);
-      grid.z = (unsigned)((K + kps - 1) / kps);
-      part = static_cast<float*>(workspace);
+      const int kps = (int)((((K + splits - 1) / splits) + 31) / 32 * 32), planes = (int)((K + kps - 1) / kps);
+      float* part = static_cast<float*>(workspace);
+      if (const int rc = launch_f32_small(st, nullptr, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, part, kps, planes))
+        return rc;
+      return launch_f32_splitk_reduce(st, part, static_cast<const float*>(R), static_cast<float*>(C), (int)M, (int)N, planes, ldr, ldc);
     }
-#define EMI_F32_SMALL(AKM, BKM)                                                                                            \
-  hipLaunchKernelGGL((gemm_f32_small_kernel<AKM, BKM>), grid, dim3(256), 0, st, static_cast<const float*>(A),              \
-                     static_cast<const float*>(B), static_cast<const float*>(R), static_cast<float*>(C), (int)M, (int)N,   \
-                     (int)K, lda, ldb, ldr, ldc, part, kps)
-    if (!trans_a && trans_b) EMI_F32_SMALL(false, false);
-    else if (!trans_a && !trans_b) EMI_F32_SMALL(false, true);
-    else if (trans_a && !trans_b) EMI_F32_SMALL(true, true);
-    else EMI_F32_SMALL(true, false);
-#undef EMI_F32_SMALL
-    EMI_CHECK_LAUNCH("emi_gemm(fp32 small)");
-    if (part != nullptr)
-      return launch_f32_splitk_reduce(st, part, static_cast<const float*>(R), static_cast<float*>(C), (int)M, (int)N, (int)grid.z, ldr, ldc);
-    return EMI_OK;
+    return launch_f32_small(st, nullptr, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, nullptr, 0, 1);
   }
   return launch_generic<float>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
 }
@@ -2043,6 +2082,23 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
       const int rc = launch_f32_gemm(st, count, A, B, any_r ? R : nullptr, C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc,
                                      trans_a, trans_b, sum ? 1 : 0);
       if (rc >= 0) return rc;
+      // independent products with odd rows: one grid plane each, unless one by one they would be split over K and together
+      // they still leave the chip idle
+      bool ok = !sum && (M + 31) / 32 <= 65535 && (trans_a || lda % 4 == 0) && (!trans_b || ldb % 4 == 0) &&
+                !(generic_splits(M, N, K) > 1 && (int64_t)count * ((M + 63) / 64) * ((N + 63) / 64) < 128);
+      for (int i = 0; i < count && ok; i++)
+        ok = (trans_a || (reinterpret_cast<uintptr_t>(A[i]) & 15) == 0) && (!trans_b || (reinterpret_cast<uintptr_t>(B[i]) & 15) == 0);
+      if (ok) {
+        GemmGroup g{};
+        g.count = count;
+        for (int i = 0; i < count; i++) {
+          g.A[i] = static_cast<const uint16_t*>(A[i]);
+          g.B[i] = static_cast<const uint16_t*>(B[i]);
+          g.R[i] = any_r ? static_cast<const uint16_t*>(R[i]) : nullptr;
+          g.C[i] = static_cast<uint16_t*>(C[i]);
+        }
+        return launch_f32_small(st, &g, A[0], B[0], nullptr, C[0], (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, nullptr, 0, count);
+      }
     }
   }
   // one product after the other; summed: each launch adds onto the result of the one before

@@ -45,3 +45,27 @@ def test_f32_tiles_stages_and_splits(ta, tb, M, N, K, count):
     _check(total, sum(prods) + Rrs[0], (count * K + 2) * eps * (sum(mags) + np.abs(Rrs[0])), "summed + residual")
     again = ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), [Rs[0]], sum_into_one=True)
     assert torch.equal(total, again)          # fixed order of summation
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,count", [
+    (9, 3, 4, 2), (31, 33, 256, 3), (65, 101, 260, 2), (33, 63, 384, 48), (129, 31, 388, 3), (63, 97, 768, 2), (97, 33, 772, 3),
+    (33, 31, 4100, 2),       # splits one by one
+    (321, 801, 520, 5),      # more than 1024 blocks
+])
+def test_f32_rows_that_are_no_whole_pieces(ta, tb, M, N, K, count):
+    """k-major operands with odd rows, k-contiguous ones of whole 16-byte pieces: the contraction at the edges of the
+    forms that take all of it at once, one product and a group with and without residuals."""
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + 3 * N + 7 * K + 2 * ta + tb)
+    As, Ars = zip(*[dev(rng.standard_normal((K, M) if ta else (M, K)), "f32") for _ in range(count)])
+    Bs, Brs = zip(*[dev(rng.standard_normal((N, K) if tb else (K, N)), "f32") for _ in range(count)])
+    Rs, Rrs = zip(*[dev(rng.standard_normal((M, N)), "f32") for _ in range(count)])
+    mm = lambda f: [f(a.T if ta else a) @ f(b.T if tb else b) for a, b in zip(Ars, Brs)]
+    prods, mags = mm(lambda t: t), mm(np.abs)
+    bounds = [(K + 2) * 2.0 ** -23 * (m + np.abs(r)) for m, r in zip(mags, Rrs)]
+    _check(ops.gemm(As[0], Bs[0], bool(ta), bool(tb), Rs[0]), prods[0] + Rrs[0], bounds[0], "one product + residual")
+    for o, p, b in zip(ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb)), prods, bounds):
+        _check(o, p, b, "group")
+    for o, p, r, b in zip(ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), list(Rs)), prods, Rrs, bounds):
+        _check(o, p + r, b, "group + residual")
