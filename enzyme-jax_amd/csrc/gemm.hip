@@ -1358,6 +1358,139 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_small_kernel(const float* __
   }
 }
 
+// ---------------------------------------------------------------------------
+// fp32 windows of larger buffers: rows that start on 16-byte boundaries but are no whole number of pieces (gemm_f32.hip
+// would read what lies past them), with 128 x 128 tiles enough to fill the chip.  A block of four wavefronts (2 x 2, 64 x 64
+// each = four 32 x 32 accumulators) stages 128 x 32 pieces of both operands per step, the last piece of a row element by
+// element: a k-contiguous operand as [row][32 + 4] (a lane reads its 4 consecutive k as one 16-byte piece), a k-major one
+// as [k][128] (four 4-byte reads, lanes along the rows).  Global loads of step s+1 are in flight while step s is
+// multiplied (held in registers, written to LDS between two barriers).  part / kps as in the kernel above (planes of K).
+// us, this | the kernel above, NT / NN / TN: 4094^3 1295 / 1320 / 1447 | 2878 / 2757 / 2293, 254 x 32002 x 286 54 / 55 / 59 | 124 / 118 / 108.
+// ---------------------------------------------------------------------------
+template <bool A_KMAJOR, bool B_KMAJOR>
+__global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                             const float* R, float* C, int M, int N, int K, int64_t lda,
+                                                             int64_t ldb, int64_t ldr, int64_t ldc, float* __restrict__ part,
+                                                             int kps) {
+  constexpr int BT = 128, BK = 32, KC_LD = BK + 4;
+  constexpr int A_FLOATS = A_KMAJOR ? BK * BT : BT * KC_LD, B_FLOATS = B_KMAJOR ? BK * BT : BT * KC_LD;
+  __shared__ __attribute__((aligned(16))) float sA[A_FLOATS];
+  __shared__ __attribute__((aligned(16))) float sB[B_FLOATS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int i = lane & 31, g = lane >> 5;
+  const int m0 = blockIdx.y * BT, n0 = blockIdx.x * BT;
+  const int kb = part != nullptr ? (int)blockIdx.z * kps : 0;
+  const int kend = part != nullptr && kb + kps < K ? kb + kps : K;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+
+  // global -> registers: four 16-byte pieces of each operand per thread and step; zero outside the operand
+  auto gload = [&](const float* X, int64_t ld, bool kmajor, int row0, int rows, int k0, float4 (&v)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int idx = tid + 256 * q;
+      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (!kmajor) {
+        const int row = row0 + (idx >> 3), k = k0 + (idx & 7) * 4;
+        if (row < rows) {
+          const float* p = X + (int64_t)row * ld + k;
+          if (k + 4 <= kend) x = *reinterpret_cast<const float4*>(p);
+          else {
+            if (k < kend) x.x = p[0];
+            if (k + 1 < kend) x.y = p[1];
+            if (k + 2 < kend) x.z = p[2];
+          }
+        }
+      } else {
+        const int k = k0 + (idx >> 5), row = row0 + (idx & 31) * 4;
+        if (k < kend) {
+          const float* p = X + (int64_t)k * ld + row;
+          if (row + 4 <= rows) x = *reinterpret_cast<const float4*>(p);
+          else {
+            if (row < rows) x.x = p[0];
+            if (row + 1 < rows) x.y = p[1];
+            if (row + 2 < rows) x.z = p[2];
+          }
+        }
+      }
+      v[q] = x;
+    }
+  };
+  auto sstore = [&](float* sX, bool kmajor, const float4 (&v)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int idx = tid + 256 * q;
+      if (!kmajor) *reinterpret_cast<float4*>(sX + (idx >> 3) * KC_LD + (idx & 7) * 4) = v[q];
+      else *reinterpret_cast<float4*>(sX + (idx >> 5) * BT + (idx & 31) * 4) = v[q];
+    }
+  };
+  // the four k of chunk j (8 wide) that this lane contracts, for tile row r of an operand
+  auto frag = [&](const float* sX, bool kmajor, int r, int j, float (&f)[4]) {
+    if (!kmajor) {
+      const float4 x = *reinterpret_cast<const float4*>(sX + r * KC_LD + 8 * j + 4 * g);
+      f[0] = x.x; f[1] = x.y; f[2] = x.z; f[3] = x.w;
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; t++) f[t] = sX[(8 * j + 4 * g + t) * BT + r];
+    }
+  };
+
+  f32x16_t acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[a][b][r] = 0.f;
+
+  float4 va[4], vb[4];
+  gload(A, lda, A_KMAJOR, m0, M, kb, va);
+  gload(B, ldb, B_KMAJOR, n0, N, kb, vb);
+  for (int k0 = kb; k0 < kend; k0 += BK) {
+    sstore(sA, A_KMAJOR, va);
+    sstore(sB, B_KMAJOR, vb);
+    __syncthreads();
+    if (k0 + BK < kend) {                                // in flight while this step is multiplied
+      gload(A, lda, A_KMAJOR, m0, M, k0 + BK, va);
+      gload(B, ldb, B_KMAJOR, n0, N, k0 + BK, vb);
+    }
+#pragma unroll
+    for (int j = 0; j < BK / 8; j++) {
+      float fa[2][4], fb[2][4];
+#pragma unroll
+      for (int a = 0; a < 2; a++) frag(sA, A_KMAJOR, wm + a * 32 + i, j, fa[a]);
+#pragma unroll
+      for (int b = 0; b < 2; b++) frag(sB, B_KMAJOR, wn + b * 32 + i, j, fb[b]);
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+          for (int b = 0; b < 2; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][t], fb[b][t], acc[a][b], 0, 0, 0);
+    }
+    __syncthreads();                                     // every wavefront is done with this step's tiles
+  }
+  // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32 x 32 tile
+#pragma unroll
+  for (int a = 0; a < 2; a++)
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      const int col = n0 + wn + b * 32 + i;
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int row = m0 + wm + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
+        if (row < M && col < N) {
+          float v = acc[a][b][r];
+          if (part != nullptr) {
+            part[((int64_t)blockIdx.z * M + row) * N + col] = v;
+          } else {
+            if (R != nullptr) v += R[(int64_t)row * ldr + col];
+            C[(int64_t)row * ldc + col] = v;
+          }
+        }
+      }
+    }
+}
+
 // VEC: a thread owns four consecutive columns of a row (N, ldr and ldc multiples of 4, rows of R and C aligned for one
 // access of four elements): 16-byte loads from every plane.
 template <typename T, bool VEC = false>
@@ -1814,6 +1947,23 @@ static int launch_f32_small(hipStream_t st, const GemmGroup* grp, const void* A,
   return EMI_OK;
 }
 
+// gemm_f32_tiled_kernel on one product, with `part` in `planes` planes of kps.
+static int launch_f32_tiled(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K, int64_t lda,
+                            int64_t ldb, int64_t ldr, int64_t ldc, int trans_a, int trans_b, float* part, int kps, int planes) {
+  const dim3 grid((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128), (unsigned)planes);
+#define EMI_F32_TILED(AKM, BKM)                                                                                            \
+  hipLaunchKernelGGL((gemm_f32_tiled_kernel<AKM, BKM>), grid, dim3(256), 0, st, static_cast<const float*>(A),              \
+                     static_cast<const float*>(B), static_cast<const float*>(R), static_cast<float*>(C), M, N, K, lda,     \
+                     ldb, ldr, ldc, part, kps)
+  if (!trans_a && trans_b) EMI_F32_TILED(false, false);
+  else if (!trans_a && !trans_b) EMI_F32_TILED(false, true);
+  else if (trans_a && !trans_b) EMI_F32_TILED(true, true);
+  else EMI_F32_TILED(true, false);
+#undef EMI_F32_TILED
+  EMI_CHECK_LAUNCH("emi_gemm(fp32 windows)");
+  return EMI_OK;
+}
+
 // gemm_f32.hip and gemm_bf16_pipe.hip add their planes with the same kernel
 int launch_bf16_splitk_reduce(hipStream_t st, const float* part, const uint16_t* R, uint16_t* C, int M, int N, int splits, int64_t ldr,
                               int64_t ldc) {
@@ -1919,14 +2069,27 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
       (trans_a || ((reinterpret_cast<uintptr_t>(A) & 15) == 0 && lda % 4 == 0)) &&
       (!trans_b || ((reinterpret_cast<uintptr_t>(B) & 15) == 0 && ldb % 4 == 0))) {
     const int splits = generic_splits(M, N, K);
+    const bool window = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0 && lda % 4 == 0 && ldb % 4 == 0;
+    const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
     if (splits > 1 && workspace_holds(workspace, workspace_bytes, splits, M, N)) {
       // few tiles and a long contraction: planes of K, added in fixed order by the reduce kernel
-      const int kps = (int)((((K + splits - 1) / splits) + 31) / 32 * 32), planes = (int)((K + kps - 1) / kps);
+      int kps = (int)((((K + splits - 1) / splits) + 31) / 32 * 32), planes = (int)((K + kps - 1) / kps);
       float* part = static_cast<float*>(workspace);
-      if (const int rc = launch_f32_small(st, nullptr, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, part, kps, planes))
-        return rc;
+      int rc;
+      if (window && tiles128 * planes >= 192) {
+        // one block per CU and no second round: at most 256 / tiles planes (never more than the workspace holds)
+        const int64_t want = 256 / tiles128 < splits ? 256 / tiles128 : splits;
+        kps = (int)((((K + want - 1) / want) + 31) / 32 * 32);
+        planes = (int)((K + kps - 1) / kps);
+        rc = launch_f32_tiled(st, A, B, nullptr, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, part, kps, planes);
+      } else {
+        rc = launch_f32_small(st, nullptr, A, B, nullptr, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, part, kps, planes);
+      }
+      if (rc != EMI_OK) return rc;
       return launch_f32_splitk_reduce(st, part, static_cast<const float*>(R), static_cast<float*>(C), (int)M, (int)N, planes, ldr, ldc);
     }
+    if (window && tiles128 >= 192)
+      return launch_f32_tiled(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, nullptr, 0, 1);
     return launch_f32_small(st, nullptr, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, nullptr, 0, 1);
   }
   return launch_generic<float>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);

@@ -69,3 +69,37 @@ def test_f32_rows_that_are_no_whole_pieces(ta, tb, M, N, K, count):
         _check(o, p, b, "group")
     for o, p, r, b in zip(ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), list(Rs)), prods, Rrs, bounds):
         _check(o, p + r, b, "group + residual")
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [
+    (2050, 1538, 262),       # 128-tiles, every edge ragged
+    (258, 290, 20010),       # 128-tiles in planes of K
+    (130, 70, 258),          # 32-tiles
+])
+def test_f32_windows_of_odd_rows(ta, tb, M, N, K):
+    """Aligned rows that are two elements short of whole 16-byte pieces, with NaN between them, and no memory behind the
+    last row: nothing of either enters the product, nothing is written between the rows of the result."""
+    from enzyme_ad.jax import _native as nat
+    rng = np.random.default_rng(M + N + K + 2 * ta + tb)
+
+    def window(rows, cols):
+        a = rng.standard_normal((rows, cols))
+        ld = cols + 2
+        room = torch.full((rows * ld - 2,), float("nan"), device="cuda")
+        t = torch.as_strided(room, (rows, cols), (ld, 1))
+        t.copy_(torch.from_numpy(a))
+        return t, ld, host(t)
+
+    A, lda, Ar = window(*((K, M) if ta else (M, K)))
+    B, ldb, Br = window(*((N, K) if tb else (K, N)))
+    R, ldr, Rr = window(M, N)
+    C = torch.full((M, N + 2), 7.0, device="cuda")
+    a, b = Ar.T if ta else Ar, Br.T if tb else Br
+    lib = nat.lib()
+    nbytes = lib.emi_gemm_workspace_bytes(M, N, K, ta, tb, nat.EMI_F32)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
+    nat.check(lib.emi_gemm_ws(torch.cuda.current_stream().cuda_stream, A.data_ptr(), B.data_ptr(), R.data_ptr(), C.data_ptr(), ws.data_ptr(),
+                              nbytes, M, N, K, lda, ldb, ldr, N + 2, ta, tb, nat.EMI_F32))
+    _check(C[:, :N], a @ b + Rr, (K + 2) * 2.0 ** -23 * (np.abs(a) @ np.abs(b) + np.abs(Rr)), "windows")
+    assert bool((C[:, N:] == 7.0).all())
