@@ -361,6 +361,10 @@ template <typename T> int launch_adjoint(hipStream_t st, Adjoint<T> a, int* band
   return EMI_OK;
 }
 
+// In pairs: the bands' sums are longer than the chains within them (768 columns: 96 bands of 43 rows), and added one by
+// one they decided the error.
+__device__ __forceinline__ float sum8(const float (&t)[8]) { return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7])); }
+
 // The sum over the bands of 16 columns per block: 16 band lanes with up to eight loads in flight each, met through LDS in
 // order.  The result is valid in threads 0 .. 15.
 __device__ __forceinline__ float sum_bands16(const float* __restrict__ part, int bands, int N, int n, float (*red)[16]) {
@@ -371,8 +375,7 @@ __device__ __forceinline__ float sum_bands16(const float* __restrict__ part, int
       float t[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) t[u] = b0 + 16 * u < bands ? part[(int64_t)(b0 + 16 * u) * N + n] : 0.f;
-#pragma unroll
-      for (int u = 0; u < 8; u++) v += t[u];
+      v += sum8(t);
     }
   }
   red[bl][col] = v;
@@ -422,8 +425,7 @@ __global__ __launch_bounds__(1024) void step_norm_adjoint_kernel(const float* __
           float t[8];
 #pragma unroll
           for (int u = 0; u < 8; u++) t[u] = b0 + lanes * u < bands ? part[(int64_t)(b0 + lanes * u) * D + n] : 0.f;
-#pragma unroll
-          for (int u = 0; u < 8; u++) v += t[u];
+          v += sum8(t);
         }
       }
       if (lanes > 1) {
