@@ -5,8 +5,9 @@
 //
 // A block of four wavefronts owns 16 queries (forward, dQ) or 16 keys (dK/dV). The 16-row tiles of the other sequence axis
 // are dealt to the wavefronts in turn, each accumulates over its own tiles, and the four partial results are added
-// through the LDS at the end (the forward pass scales them to a common maximum first); that is the only barrier. Operands
-// come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
+// through the LDS at the end (the forward pass scales them to a common maximum first); that is the only barrier. A masked
+// score has the weight 0 and its row is multiplied by it, so a NaN or an infinity in a row of v also reaches earlier queries
+// of the same 16-row tile. Operands come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
 // 16 rows are one chain of them, so with one wavefront per 16 rows (the earlier form) the longest row set the time and too
 // few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 24,
 // 24 heads x 1000 x 64 89 / 280 -> 56 / 161 (55 / 48 TFLOP/s), 64 heads x 2048 x 128 1329 / 4010 -> 795 / 2907 (86 / 59);
