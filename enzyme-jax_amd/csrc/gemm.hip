@@ -249,26 +249,19 @@ __device__ __forceinline__ void epilogue_bf16(f32x16_t (&acc)[TM][TN], EMI_LDS u
   }
 }
 
-// Software pipeline, NSTAGE == 2: tile t+1 streams into the other LDS stage while
-// tile t is multiplied; one barrier per tile.
-// NSTAGE == 4: tiles t+2 and t+3 are in flight while tile t is multiplied and
-// tile t+1 has already landed, so the operand fragments of the first k-step of
-// tile t+1 are fetched before the barrier and the MFMA stream never waits on LDS.
-// Loads past the end of K are still issued (they read as zeros) so that the
-// number of outstanding loads is a compile-time constant.
-template <int BM, int BN, int BK, int NSTAGE, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const uint16_t* __restrict__ A,
+// 128 x 128 tiles with a k-major A (the weight gradients; gemm_bf16_pipe.hip has the k-contiguous ones): tile t+1 streams
+// into the other LDS stage while tile t is multiplied; one barrier per tile.
+template <bool B_KMAJOR>
+__global__ __launch_bounds__(256) void gemm_bf16_kernel(const uint16_t* __restrict__ A,
                                                                  const uint16_t* __restrict__ B, const uint16_t* R,
                                                                  uint16_t* C, int M, int N, int K, int lda, int ldb,
                                                                  int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes,
                                                                  int vec_ok, float* __restrict__ part, int k_per_split,
                                                                  GemmGroup grp) {
-  constexpr int NW = WM * WN;
+  constexpr int BM = 128, BN = 128, BK = 64, WM = 2, WN = 2, NW = WM * WN;
   constexpr int KS = BK / 16;
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE = A_BYTES + B_BYTES;
-  constexpr int LPT = (A_BYTES + B_BYTES) / 1024 / NW;      // direct-to-LDS loads per wave per tile
-  static_assert(NSTAGE == 2 || NSTAGE == 4, "NSTAGE");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
   EMI_LDS uint8_t* smem = (EMI_LDS uint8_t*)smem_raw;
 
@@ -304,10 +297,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const uint16_t* 
   auto issue_loads = [&](int stage, int k0) {
     EMI_LDS uint8_t* sA = smem + stage * STAGE;
     EMI_LDS uint8_t* sB = sA + A_BYTES;
-    if constexpr (A_KMAJOR)
-      load_tile_kmajor<BM, BK, NW>(rA, sA, wave, lane, m0, M, lda, k0, K);
-    else
-      load_tile_kcontig<BM, BK, NW>(rA, sA, wave, lane, (uint32_t)m0 * (uint32_t)lda * 2u, lda, k0, K);
+    load_tile_kmajor<BM, BK, NW>(rA, sA, wave, lane, m0, M, lda, k0, K);
     if constexpr (B_KMAJOR)
       load_tile_kmajor<BN, BK, NW>(rB, sB, wave, lane, n0, N, ldb, k0, K);
     else
@@ -326,11 +316,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const uint16_t* 
     const EMI_LDS uint8_t* sA = smem + stage * STAGE;
     const EMI_LDS uint8_t* sB = sA + A_BYTES;
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int base = wm * (BM / WM) + i * 32;
-      if constexpr (A_KMAJOR) a[i] = frag_kmajor<BM>(sA, base, kk, lane);
-      else a[i] = frag_kcontig<BK>(sA, base, kk, lane);
-    }
+    for (int i = 0; i < TM; i++) a[i] = frag_kmajor<BM>(sA, wm * (BM / WM) + i * 32, kk, lane);
 #pragma unroll
     for (int j = 0; j < TN; j++) {
       const int base = wn * (BN / WN) + j * 32;
@@ -354,56 +340,31 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_kernel(const uint16_t* 
   // Operand fragments are double buffered: the LDS reads of the next k-step are
   // issued before the MFMAs of the current one so their latency hides behind them.
   bf16x8_t fa[2][TM], fb[2][TN];
-  if constexpr (NSTAGE == 2) {
-    for (int pair = 0; pair < npairs; pair++) {        // one pass unless several products are summed into this tile
-      if (npairs > 1) {
-        rA = make_rsrc(grp.A[pair], a_bytes);
-        rB = make_rsrc(grp.B[pair], b_bytes);
-      }
-      issue_loads(0, k_lo);
-      wait_vmcnt<0>();
-      __syncthreads();
-      for (int t = 0; t < nk; t++) {
-        if (t + 1 < nk) issue_loads((t + 1) & 1, k_lo + (t + 1) * BK);
-        load_frags(t & 1, 0, fa[0], fb[0]);
-#pragma unroll
-        for (int kk = 0; kk < KS; kk++) {
-          if (kk + 1 < KS) load_frags(t & 1, kk + 1, fa[(kk + 1) & 1], fb[(kk + 1) & 1]);
-          __builtin_amdgcn_sched_barrier(0);
-          mfma_step(fa[kk & 1], fb[kk & 1]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        wait_vmcnt<0>();     // next stage has landed
-        __syncthreads();     // and everyone is done reading this one
-      }
+  for (int pair = 0; pair < npairs; pair++) {        // one pass unless several products are summed into this tile
+    if (npairs > 1) {
+      rA = make_rsrc(grp.A[pair], a_bytes);
+      rB = make_rsrc(grp.B[pair], b_bytes);
     }
-  } else {
-    static_assert(KS % 2 == 0, "fragment double buffering assumes an even number of k-steps per tile");
     issue_loads(0, k_lo);
-    issue_loads(1, k_lo + BK);
-    issue_loads(2, k_lo + 2 * BK);
-    wait_vmcnt<LPT>();     // tiles 0 and 1 have landed
+    wait_vmcnt<0>();
     __syncthreads();
-    load_frags(0, 0, fa[0], fb[0]);
     for (int t = 0; t < nk; t++) {
-      issue_loads((t + 3) & 3, k_lo + (t + 3) * BK);
+      if (t + 1 < nk) issue_loads((t + 1) & 1, k_lo + (t + 1) * BK);
+      load_frags(t & 1, 0, fa[0], fb[0]);
 #pragma unroll
       for (int kk = 0; kk < KS; kk++) {
-        if (kk + 1 < KS) load_frags(t & 3, kk + 1, fa[(kk + 1) & 1], fb[(kk + 1) & 1]);
-        else load_frags((t + 1) & 3, 0, fa[0], fb[0]);
+        if (kk + 1 < KS) load_frags(t & 1, kk + 1, fa[(kk + 1) & 1], fb[(kk + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);
         mfma_step(fa[kk & 1], fb[kk & 1]);
         __builtin_amdgcn_sched_barrier(0);
       }
-      wait_vmcnt<LPT>();   // everything but the newest tile (t+3) has landed: tiles <= t+2
-      __syncthreads();     // visible to all; tile t's stage may be refilled next iteration
+      wait_vmcnt<0>();     // next stage has landed
+      __syncthreads();     // and everyone is done reading this one
     }
-    wait_vmcnt<0>();       // drain the zero-filled loads past the end of K before LDS is reused
-    __syncthreads();
   }
 
   constexpr int WR = BM / WM, WC = BN / WN;
-  static_assert(NW * WR * WC * 2 <= NSTAGE * STAGE, "epilogue staging does not fit in the LDS allocation");
+  static_assert(NW * WR * WC * 2 <= 2 * STAGE, "epilogue staging does not fit in the LDS allocation");
   if (part != nullptr) {
     // accumulator layout (swapped operands): register 4q+e of lane l holds row l%32, column 8q + 4(l/32) + e
     float* pz = part + (int64_t)split * M * N;
@@ -1594,15 +1555,16 @@ static int generic_splits(int64_t M, int64_t N, int64_t K) {
   return (int)(s < 2 ? 1 : (s > 256 ? 256 : s));
 }
 
-template <int BM, int BN, int BK, int NSTAGE, int WM, int WN, bool AK, bool BKM>
+template <bool BKM>
 static int launch_bf16(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K, int lda,
                        int ldb, int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, float* part = nullptr, int splits = 1) {
   // 16-byte epilogue accesses need aligned rows of C (and R)
   const int vec_ok = ((reinterpret_cast<uintptr_t>(C) & 15) == 0 && ldc % 8 == 0 &&
                       (R == nullptr || ((reinterpret_cast<uintptr_t>(R) & 15) == 0 && ldr % 8 == 0)))
                          ? 1 : 0;
-  auto kern = gemm_bf16_kernel<BM, BN, BK, NSTAGE, WM, WN, AK, BKM>;
-  constexpr int smem = NSTAGE * (BM + BN) * BK * 2;
+  constexpr int BM = 128, BN = 128, BK = 64;
+  auto kern = gemm_bf16_kernel<BKM>;
+  constexpr int smem = 2 * (BM + BN) * BK * 2;
   static bool configured = false;   // idempotent; a race only repeats the call
   if (!configured) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
@@ -1613,7 +1575,7 @@ static int launch_bf16(hipStream_t st, const void* A, const void* B, const void*
   if (part != nullptr && splits > 1) {
     const int kps = (((K + splits - 1) / splits) + BK - 1) / BK * BK;
     const int nz = (K + kps - 1) / kps;
-    hipLaunchKernelGGL(kern, dim3(tiles * nz), dim3(WM * WN * 64), smem, st, static_cast<const uint16_t*>(A),
+    hipLaunchKernelGGL(kern, dim3(tiles * nz), dim3(256), smem, st, static_cast<const uint16_t*>(A),
                        static_cast<const uint16_t*>(B), static_cast<const uint16_t*>(R), static_cast<uint16_t*>(C), M, N, K,
                        lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok, part, kps, GemmGroup{});
     EMI_CHECK_LAUNCH("emi_gemm(split-K)");
@@ -1621,7 +1583,7 @@ static int launch_bf16(hipStream_t st, const void* A, const void* B, const void*
     EMI_CHECK_LAUNCH("emi_gemm(split-K reduce)");
     return EMI_OK;
   }
-  hipLaunchKernelGGL(kern, dim3(tiles), dim3(WM * WN * 64), smem, st, static_cast<const uint16_t*>(A),
+  hipLaunchKernelGGL(kern, dim3(tiles), dim3(256), smem, st, static_cast<const uint16_t*>(A),
                      static_cast<const uint16_t*>(B), static_cast<const uint16_t*>(R), static_cast<uint16_t*>(C), M, N, K,
                      lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok, static_cast<float*>(nullptr), 0, GemmGroup{});
   EMI_CHECK_LAUNCH("emi_gemm");
@@ -1657,7 +1619,7 @@ static int launch_bf16_pingpong_grouped(hipStream_t st, const GemmGroup& g, int 
 
 // Products with a k-major A: the 128x128 kernel on a group of them (GemmGroup): one launch, count times the tiles (or,
 // summed, count times the contraction).
-template <bool AK, bool BKM>
+template <bool BKM>
 static int launch_bf16_grouped(hipStream_t st, const GemmGroup& g, int M, int N, int K, int lda, int ldb, int ldr, int ldc,
                                uint32_t a_bytes, uint32_t b_bytes, void* workspace, size_t workspace_bytes) {
   constexpr int BM = 128, BN = 128, BK = 64;
@@ -1665,7 +1627,7 @@ static int launch_bf16_grouped(hipStream_t st, const GemmGroup& g, int M, int N,
   const int nout = g.sum ? 1 : g.count;
   for (int i = 0; i < nout; i++)
     if ((reinterpret_cast<uintptr_t>(g.C[i]) & 15) || (g.R[i] != nullptr && (reinterpret_cast<uintptr_t>(g.R[i]) & 15))) vec_ok = 0;
-  auto kern = gemm_bf16_kernel<BM, BN, BK, 2, 2, 2, AK, BKM>;
+  auto kern = gemm_bf16_kernel<BKM>;
   constexpr int smem = 2 * (BM + BN) * BK * 2;
   static bool configured = false;   // idempotent; a race only repeats the call
   if (!configured) {
@@ -1679,7 +1641,7 @@ static int launch_bf16_grouped(hipStream_t st, const GemmGroup& g, int M, int N,
   // contraction a last round that leaves most CUs idle costs more than the larger tile gains; with a long one it does not
   // (12 x [768, 2048] x 8192: 351 vs 462 us).
   if (!g.sum && group_tiles >= 192 && (4 * group_tiles >= 3 * rounds * 256 || K >= 4096))
-    return launch_bf16_pingpong_grouped<AK, BKM>(st, g, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok);
+    return launch_bf16_pingpong_grouped<true, BKM>(st, g, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, vec_ok);
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   const int splits = g.sum ? 1 : grouped_splits(M, N, K, g.count);
   if (splits > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
@@ -1852,11 +1814,11 @@ static int launch_bf16_kmajor(hipStream_t st, const void* A, const void* B, cons
                               int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, void* workspace, size_t workspace_bytes) {
   const int splits = bf16_splits(M, N, K);
   if (splits > 1 && workspace_holds(workspace, workspace_bytes, splits, M, N))
-    return launch_bf16<128, 128, 64, 2, 2, 2, true, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes,
+    return launch_bf16<BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes,
                                                          static_cast<float*>(workspace), splits);
   const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
   if (big_tiles >= 192) return launch_bf16_pingpong<true, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
-  return launch_bf16<128, 128, 64, 2, 2, 2, true, BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
+  return launch_bf16<BKM>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
 }
 
 // A k-contiguous: the ping-pong kernel or one of the shapes of gemm_bf16_pipe.hip, with or without splits of K.
@@ -2230,8 +2192,8 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
                                 n, k, (int)lda, (int)ldb, ldr, ldc, vec_ok, trans_b, sum ? 1 : 0);
       }
       if (trans_a && !trans_b)
-        return launch_bf16_grouped<true, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
-      return launch_bf16_grouped<true, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
+        return launch_bf16_grouped<true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
+      return launch_bf16_grouped<false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
     }
   }
   if (dtype == EMI_F32 && count >= 2 && K > 0 && M > 8 && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && ldc >= N) {
