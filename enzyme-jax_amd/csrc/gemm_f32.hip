@@ -8,9 +8,9 @@
 // k each, filled by direct-to-LDS loads (16 bytes a lane, no staging registers) NST - 1 stages ahead, one barrier per
 // stage, and three shapes of block between which the launcher chooses by how the tiles divide over the CUs (f32_plan()).
 // Measured, us, against 32 x 32 tiles read straight from global memory and 128 x 128 tiles staged through registers
-// (NT / NN / TN form): 256 x 288 x 288: 8.2 -> 4.8 / 7.5 -> 5.3 / 7.5 -> 4.8; 256 x 288 x 768 12.6 -> 7.5; 2000 x 768 x 768
-// 53 -> 30; 2000 x 768 x 2048 90 -> 59; 2048 x 768 x 2000 (TN) 122 -> 56 (113 TFLOP/s); 300 x 4096 x 11008 441 -> 237;
-// 4096^3 1258 -> 988 (139 TFLOP/s of 157).  What is left on the small ones is the latency of the first loads and the launch.
+// (NT / NN / TN form): 256 x 288 x 288: 8.2 -> 5.0 / 7.5 -> 5.4 / 7.5 -> 4.9; 256 x 288 x 768 12.6 -> 7.5; 2000 x 768 x 768
+// 53 -> 32; 2000 x 768 x 2048 90 -> 62; 2048 x 768 x 2000 (TN) 122 -> 61 (103 TFLOP/s); 300 x 4096 x 11008 441 -> 241;
+// 4096^3 1258 -> 1013 (136 TFLOP/s of 157).  What is left on the small ones is the latency of the first loads and the launch.
 #include <type_traits>
 
 #include "emi_device.h"
@@ -348,9 +348,10 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 }
 
 // Which block and how many splits.  The estimate is of the CU with the most blocks, in microseconds, with the rates that
-// each block shape was measured at: a stage of 32 k of a 128 x 128 tile takes 2.0 alone on a CU and 1.92 next to others
-// (139 TFLOP/s on 4096^3; the matrix cores' own limit is 157), a 64 x 64 tile 0.72 alone, 1.13 for two blocks and 0.54 a
-// block from four on, a stage of 64 k of a 32 x 32 tile whose wavefronts share k 0.42 alone, 0.36 a block from three on.
+// each block shape was measured at (before the sums were cut into chains, which costs each about 2 %): a stage of 32 k of a
+// 128 x 128 tile takes 2.0 alone on a CU and 1.92 next to others (139 TFLOP/s on 4096^3; the matrix cores' own limit is
+// 157), a 64 x 64 tile 0.72 alone, 1.13 for two blocks and 0.54 a block from four on, a stage of 64 k of a 32 x 32 tile
+// whose wavefronts share k 0.42 alone, 0.36 a block from three on.
 // The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s); results over 4 M elements, whose planes
 // leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split.
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int64_t most) {
