@@ -1944,7 +1944,7 @@ int launch_f32_splitk_reduce(hipStream_t st, const float* part, const float* R, 
 int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
                     void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
                     int64_t ldc, int trans_a, int trans_b, int sum);
-size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum);
+size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a);
 
 // gemm_skinny.hip
 int launch_skinny(hipStream_t st, const void* A, const void* B, const void* R, void* C, void* workspace, size_t workspace_bytes,
@@ -1970,7 +1970,7 @@ extern "C" size_t emi_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
     if (s > splits) splits = s;
   }
   const size_t need = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
-  const size_t f32 = dtype == EMI_F32 ? gemm_f32_workspace_bytes(M, N, K, 1, 0) : 0;
+  const size_t f32 = dtype == EMI_F32 ? gemm_f32_workspace_bytes(M, N, K, 1, 0, trans_a) : 0;
   return f32 > need ? f32 : need;
 }
 
@@ -2130,7 +2130,7 @@ extern "C" size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t
     if (grouped > need) need = grouped;
   }
   if (count >= 2 && count <= kMaxGroup && dtype == EMI_F32 && M > 0 && N > 0 && K > 0) {
-    const size_t grouped = gemm_f32_workspace_bytes(M, N, K, count, sum ? 1 : 0);
+    const size_t grouped = gemm_f32_workspace_bytes(M, N, K, count, sum ? 1 : 0, trans_a);
     if (grouped > need) need = grouped;
   }
   return need;

@@ -353,12 +353,13 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 // 157), a 64 x 64 tile 0.72 alone, 1.13 for two blocks and 0.54 a block from four on, a stage of 64 k of a 32 x 32 tile
 // whose wavefronts share k 0.42 alone, 0.36 a block from three on.
 // The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s); results over 4 M elements, whose planes
-// leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split.
-F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int64_t most) {
+// leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few
+// rows of a k-major A are no such product (4 x 64 x 20000, us: 126 in one pass, 12 split).
+F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
   struct Shape { int tile, bk; double fixed, rate[4]; };              // rate[b - 1]: per stage, b blocks on the CU; the last one per block
   static const Shape shapes[3] = {{128, 32, 4.0, {2.0, 3.84, 5.76, 1.92}}, {64, 32, 3.0, {0.72, 1.13, 1.60, 0.54}}, {32, 64, 2.5, {0.42, 0.72, 1.08, 0.36}}};
   F32Plan best{2, 1};
-  const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && M > 8 && K > 8;
+  const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && (M > 8 || trans_a) && K > 8;
   double least = 1e30;
   for (int c = 0; c < 3; c++) {
     const Shape& s = shapes[c];
@@ -377,8 +378,8 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int64_t mo
   return best;
 }
 
-size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum) {
-  const int z = f32_plan(M, N, K, count, sum, kAnySplits).splits;
+size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a) {
+  const int z = f32_plan(M, N, K, count, sum, trans_a, kAnySplits).splits;
   return z > 1 ? (size_t)z * M * N * sizeof(float) : 0;
 }
 
@@ -403,7 +404,7 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   }
   g.count = count;
   g.sum = sum;
-  const F32Plan p = f32_plan(M, N, K, count, sum, splits_held(workspace, workspace_bytes, M, N));
+  const F32Plan p = f32_plan(M, N, K, count, sum, trans_a, splits_held(workspace, workspace_bytes, M, N));
   const F32Call c{g.A[0], g.B[0], g.R[0], g.C[0], (int)M, (int)N, (int)K, (int)lda, (int)ldb, ldr, ldc, static_cast<float*>(workspace),
                   p.splits, count > 1 ? &g : nullptr};
   switch (p.config) {

@@ -123,3 +123,14 @@ def test_f32_windows_of_odd_rows(ta, tb, M, N, K):
                               nbytes, M, N, K, lda, ldb, ldr, N + 2, ta, tb, nat.EMI_F32))
     _check(C[:, :N], a @ b + Rr, (K + 2) * 2.0 ** -23 * (np.abs(a) @ np.abs(b) + np.abs(Rr)), "windows")
     assert bool((C[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 4100), (4, 688, 5692), (8, 68, 20000), (5, 688, 5689)])
+def test_f32_gradients_of_few_rows(M, N, K):
+    """A handful of rows of a k-major A against a long contraction: split where rows are whole 16-byte pieces."""
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + N + K)
+    (A, Ar), (B, Br), (R, Rr) = (dev(rng.standard_normal(s), "f32") for s in ((K, M), (K, N), (M, N)))
+    bound = (K + 2) * 2.0 ** -23 * (np.abs(Ar).T @ np.abs(Br) + np.abs(Rr))
+    _check(ops.gemm(A, B, True, False), Ar.T @ Br, bound, "one product")
+    _check(ops.gemm(A, B, True, False, R), Ar.T @ Br + Rr, bound, "one product + residual")

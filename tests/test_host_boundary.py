@@ -87,19 +87,29 @@ def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K
     """Without room for the planes the blocks are not those that the splits were to multiply: there are more of them, enough
     for half of the 256 CUs or the smallest ones there are.  With room for some planes there are at most as many splits."""
     lib = _lib()
-    plan, blocks, trans_b = ((lib._ZN3emi9bf16_planEllliiil, [(256, 256), (128, 128), (128, 128), (128, 64), (64, 64), (32, 32)], (1,))
-                             if dtype == "bf16" else (lib._ZN3emi8f32_planEllliil, [(128, 128), (64, 64), (32, 32)], ()))
-    plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * (2 + len(trans_b)) + [C.c_int64]
+    plan, blocks, trans = ((lib._ZN3emi9bf16_planEllliiil, [(256, 256), (128, 128), (128, 128), (128, 64), (64, 64), (32, 32)], 1)
+                           if dtype == "bf16" else (lib._ZN3emi8f32_planEllliiil, [(128, 128), (64, 64), (32, 32)], 0))      # of B, of A
+    plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
     tiles = lambda p: -(-M // blocks[p.shape][0]) * -(-N // blocks[p.shape][1])
-    free, one = (plan(M, N, K, count, total, *trans_b, most) for most in (1 << 20, 1))
+    free, one = (plan(M, N, K, count, total, trans, most) for most in (1 << 20, 1))
     assert free.splits > 1 and one.splits == 1
     assert tiles(one) > tiles(free) and (tiles(one) >= 128 or one.shape == len(blocks) - 1)
     for most in range(2, free.splits + 2):
-        assert 1 <= plan(M, N, K, count, total, *trans_b, most).splits <= most
+        assert 1 <= plan(M, N, K, count, total, trans, most).splits <= most
     code = 16 if dtype == "bf16" else 11
     need = (lib.emi_gemm_grouped_workspace_bytes(count, M, N, K, 0, 1, total, code) if count > 1 else
             lib.emi_gemm_workspace_bytes(M, N, K, 0, 1, code))
     assert need >= free.splits * M * N * 4
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 688, 5689), (4, 64, 20000), (8, 4096, 4096)])
+def test_a_few_rows_of_a_gradient_are_split(M, N, K):
+    """dW = dY^T . X of a few columns of dY is no product of a few tokens: nothing else splits its long contraction."""
+    lib = _lib()
+    assert lib.emi_gemm_workspace_bytes(M, N, K, 1, 0, 11) >= 4 * M * N * 4
+    plan = lib._ZN3emi8f32_planEllliiil
+    plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
+    assert plan(M, N, K, 1, 0, 1, 1 << 20).splits >= 4 and plan(M, N, K, 1, 0, 0, 1 << 20).splits == 1
 
 
 def _handler(name):
