@@ -2184,7 +2184,14 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
       if (!trans_a) {
         int vec_ok = ldc % 8 == 0 && ldr % 8 == 0;
         for (int i = 0; i < nout; i++) vec_ok = vec_ok && al16(C[i]) && al16(g.R[i]);
-        const Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b, splits_held(workspace, workspace_bytes, M, N));
+        const int64_t held = splits_held(workspace, workspace_bytes, M, N);
+        const Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b, held);
+        if (!sum && faster_one_by_one(plan, bf16_plan(M, N, K, 1, 0, trans_b, held), count)) {
+          for (int i = 0; i < count; i++)
+            if (const int rc = emi_gemm_ws(stream, A[i], B[i], g.R[i], C[i], workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, 0, trans_b, dtype))
+              return rc;
+          return EMI_OK;
+        }
         if (plan.shape == 0)
           return trans_b ? launch_bf16_pingpong_grouped<false, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok)
                          : launch_bf16_pingpong_grouped<false, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok);

@@ -398,7 +398,7 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
   static const Shape shapes[6] = {{256, 256, 64, 4.0, {1.0, 2.0, 3.0}, 1.0},  {128, 128, 64, 4.0, {0.61, 0.90, 1.45}, 0.50},
                                   {128, 128, 64, 3.5, {0.57, 1.14, 1.71}, 0.57}, {128, 64, 64, 3.0, {0.36, 0.62, 1.0}, 0.33},
                                   {64, 64, 64, 2.8, {0.31, 0.39, 0.59}, 0.22},   {32, 32, 256, 2.2, {0.55, 1.10, 1.65}, 0.55}};
-  Bf16Plan best{1, 1};
+  Bf16Plan best{1, 1, 0.0};
   double least = 1e30;
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && M > 8 && K > 8;
   for (int c = 0; c < 6; c++) {
@@ -415,7 +415,7 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
       const double t = s.fixed + per * stage + (z > 1 ? 3.0 + 0.7e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
         least = t;
-        best = Bf16Plan{c, (int)z};
+        best = Bf16Plan{c, (int)z, t};
       }
     }
   }

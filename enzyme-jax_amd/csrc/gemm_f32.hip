@@ -358,7 +358,7 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
   struct Shape { int tile, bk; double fixed, rate[4]; };              // rate[b - 1]: per stage, b blocks on the CU; the last one per block
   static const Shape shapes[3] = {{128, 32, 4.0, {2.0, 3.84, 5.76, 1.92}}, {64, 32, 3.0, {0.72, 1.13, 1.60, 0.54}}, {32, 64, 2.5, {0.42, 0.72, 1.08, 0.36}}};
-  F32Plan best{2, 1};
+  F32Plan best{2, 1, 0.0};
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && (M > 8 || trans_a) && K > 8;
   double least = 1e30;
   for (int c = 0; c < 3; c++) {
@@ -371,7 +371,7 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_
       const double t = s.fixed + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
         least = t;
-        best = F32Plan{c, (int)z};
+        best = F32Plan{c, (int)z, t};
       }
     }
   }
@@ -404,7 +404,16 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   }
   g.count = count;
   g.sum = sum;
-  const F32Plan p = f32_plan(M, N, K, count, sum, trans_a, splits_held(workspace, workspace_bytes, M, N));
+  const int64_t held = splits_held(workspace, workspace_bytes, M, N);
+  const F32Plan p = f32_plan(M, N, K, count, sum, trans_a, held);
+  if (count > 1 && !sum && faster_one_by_one(p, f32_plan(M, N, K, 1, 0, trans_a, held), count)) {
+    for (int i = 0; i < count; i++) {
+      const void* r = R != nullptr ? R[i] : nullptr;
+      if (const int rc = launch_f32_gemm(st, 1, A + i, B + i, &r, C + i, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0))
+        return rc;
+    }
+    return EMI_OK;
+  }
   const F32Call c{g.A[0], g.B[0], g.R[0], g.C[0], (int)M, (int)N, (int)K, (int)lda, (int)ldb, ldr, ldc, static_cast<float*>(workspace),
                   p.splits, count > 1 ? &g : nullptr};
   switch (p.config) {

@@ -8,10 +8,12 @@ namespace emi {
 struct Bf16Plan {
   int shape;        // 0: the 256 x 256 ping-pong kernel of gemm.hip; otherwise a block shape of gemm_bf16_pipe.hip
   int splits;       // splits of K
+  double us;        // the estimate
 };
 struct F32Plan {
   int config;       // 0: blocks of 128 x 128, 1: 64 x 64, 2: 32 x 32 (gemm_f32.hip)
   int splits;
+  double us;
 };
 
 // The best of the plans with at most `most` splits.  A shape that was chosen for its splits is a poor one without them, so
@@ -26,6 +28,14 @@ inline int64_t splits_held(const void* workspace, size_t bytes, int64_t M, int64
   if (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0) return 1;
   const int64_t n = (int64_t)(bytes / ((size_t)M * N * sizeof(float)));
   return n < 1 ? 1 : n < kAnySplits ? n : kAnySplits;
+}
+
+// Whether products that can run as one launch, each in a single pass over K, run one by one: where each split over K is so
+// much faster that together they are (us, one launch | one by one: 2 x 16 x 4096 x 11008, B k-major, bf16 54 | 35;
+// 4 x 64 x 64 x 16384, fp32, both k-major 119 | 41).  Each costs a launch and the gap before it, and the estimates are good
+// to a fifth (3 x 16 x 4096 x 11008, both k-contiguous, estimated as equal: 50 | 58).
+template <typename Plan> inline bool faster_one_by_one(const Plan& group, const Plan& one, int count) {
+  return one.splits > 1 && 1.2 * count * (one.us + 1.0) < group.us;
 }
 
 int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void* const* A, const void* const* B, const void* const* R,

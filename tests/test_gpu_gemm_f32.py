@@ -134,3 +134,21 @@ def test_f32_gradients_of_few_rows(M, N, K):
     bound = (K + 2) * 2.0 ** -23 * (np.abs(Ar).T @ np.abs(Br) + np.abs(Rr))
     _check(ops.gemm(A, B, True, False), Ar.T @ Br, bound, "one product")
     _check(ops.gemm(A, B, True, False, R), Ar.T @ Br + Rr, bound, "one product + residual")
+
+
+@pytest.mark.parametrize("dt,ta,tb,M,N,K,count", [("f32", 1, 0, 64, 64, 8192, 4), ("f32", 0, 0, 300, 64, 4096, 2), ("bf16", 0, 0, 16, 1032, 8200, 3),
+                                                  ("bf16", 0, 1, 24, 72, 16400, 2)])
+def test_groups_that_run_faster_one_by_one(dt, ta, tb, M, N, K, count):
+    """Few tiles and a long contraction: each product of the group is split over K.  Their planes share the workspace, one
+    after the other on the stream."""
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + N + K + ta)
+    As, Ars = zip(*[dev(rng.standard_normal((K, M) if ta else (M, K)), dt) for _ in range(count)])
+    Bs, Brs = zip(*[dev(rng.standard_normal((N, K) if tb else (K, N)), dt) for _ in range(count)])
+    Rs, Rrs = zip(*[dev(rng.standard_normal((M, N)), dt) for _ in range(count)])
+    unit = 2.0 ** -8 if dt == "bf16" else 0.0
+    for rs, adds in ((None, [0.0] * count), (list(Rs), Rrs)):
+        for o, a, b, r in zip(ops.gemm_grouped(list(As), list(Bs), bool(ta), bool(tb), rs), Ars, Brs, adds):
+            x, y = a.T if ta else a, b.T if tb else b
+            ref = x @ y + r
+            _check(o, ref, unit * np.abs(ref) + (K + 2) * 2.0 ** -23 * (np.abs(x) @ np.abs(y) + np.abs(r)), "group")

@@ -77,7 +77,7 @@ def test_plain_launchers_reject_bad_arguments_before_touching_the_gpu():
 
 
 class _Plan(C.Structure):
-    _fields_ = [("shape", C.c_int), ("splits", C.c_int)]
+    _fields_ = [("shape", C.c_int), ("splits", C.c_int), ("us", C.c_double)]
 
 
 @pytest.mark.parametrize("dtype,M,N,K,count,total", [
