@@ -2186,7 +2186,7 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
         for (int i = 0; i < nout; i++) vec_ok = vec_ok && al16(C[i]) && al16(g.R[i]);
         const int64_t held = splits_held(workspace, workspace_bytes, M, N);
         const Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b, held);
-        if (!sum && faster_one_by_one(plan, bf16_plan(M, N, K, 1, 0, trans_b, held), count)) {
+        if (!sum && faster_one_by_one(plan, bf16_plan(M, N, K, 1, 0, trans_b, held), count, 1.3)) {
           for (int i = 0; i < count; i++)
             if (const int rc = emi_gemm_ws(stream, A[i], B[i], g.R[i], C[i], workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, 0, trans_b, dtype))
               return rc;

@@ -347,17 +347,20 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 #undef EMI_F32_PIPE
 }
 
-// Which block and how many splits.  The estimate is of the CU with the most blocks, in microseconds, with the rates that
-// each block shape was measured at (before the sums were cut into chains, which costs each about 2 %): a stage of 32 k of a
-// 128 x 128 tile takes 2.0 alone on a CU and 1.92 next to others (139 TFLOP/s on 4096^3; the matrix cores' own limit is
-// 157), a 64 x 64 tile 0.72 alone, 1.13 for two blocks and 0.54 a block from four on, a stage of 64 k of a 32 x 32 tile
-// whose wavefronts share k 0.42 alone, 0.36 a block from three on.
+// Which block and how many splits.  The estimate is of the CU with the most blocks, in microseconds: a start, which grows
+// with the blocks that come after one another, and the stages at the rate that each block shape was measured at.  A stage of
+// 32 k of a 128 x 128 tile takes 2.04 alone on a CU and 1.91 next to others (136 TFLOP/s on 4096^3; the matrix cores' own
+// limit is 157), a 64 x 64 tile 0.64 alone, 1.1 for two blocks and 0.485 a block from four on, a stage of 64 k of a 32 x 32
+// tile whose wavefronts share k 0.40 alone, 0.32 a block from four on.  The start of a further block is 2.5, 0.65 and 1.2:
+// with two to four stages to a block it decides (2048 x 768 x 128, both k-major: 32-tiles 13.6, 64-tiles 9.0).
 // The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s); results over 4 M elements, whose planes
 // leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few
 // rows of a k-major A are no such product (4 x 64 x 20000, us: 126 in one pass, 12 split).
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
-  struct Shape { int tile, bk; double fixed, rate[4]; };              // rate[b - 1]: per stage, b blocks on the CU; the last one per block
-  static const Shape shapes[3] = {{128, 32, 4.0, {2.0, 3.84, 5.76, 1.92}}, {64, 32, 3.0, {0.72, 1.13, 1.60, 0.54}}, {32, 64, 2.5, {0.42, 0.72, 1.08, 0.36}}};
+  struct Shape { int tile, bk; double one, base, block, rate[4]; };     // start of one block, of b: base + b block; rate[b - 1]: per
+                                                                        // stage, b blocks on the CU; the last one per block
+  static const Shape shapes[3] = {{128, 32, 4.8, 4.0, 2.5, {2.04, 3.86, 5.82, 1.91}}, {64, 32, 3.4, 4.0, 0.65, {0.64, 1.10, 1.50, 0.485}},
+                                  {32, 64, 3.4, 2.5, 1.2, {0.40, 0.69, 1.00, 0.32}}};
   F32Plan best{2, 1, 0.0};
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && (M > 8 || trans_a) && K > 8;
   double least = 1e30;
@@ -368,7 +371,8 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_
     if (blocks > 0x3fffffff) continue;
     for (int64_t z = 1; z <= 64 && z <= most && (z == 1 || (may_split && steps >= 4 * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
-      const double t = s.fixed + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
+      const double t = (b == 1 ? s.one : s.base + s.block * b) + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) +
+                       (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
         least = t;
         best = F32Plan{c, (int)z, t};
@@ -406,7 +410,7 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   g.sum = sum;
   const int64_t held = splits_held(workspace, workspace_bytes, M, N);
   const F32Plan p = f32_plan(M, N, K, count, sum, trans_a, held);
-  if (count > 1 && !sum && faster_one_by_one(p, f32_plan(M, N, K, 1, 0, trans_a, held), count)) {
+  if (count > 1 && !sum && faster_one_by_one(p, f32_plan(M, N, K, 1, 0, trans_a, held), count, 1.08)) {
     for (int i = 0; i < count; i++) {
       const void* r = R != nullptr ? R[i] : nullptr;
       if (const int rc = launch_f32_gemm(st, 1, A + i, B + i, &r, C + i, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0))

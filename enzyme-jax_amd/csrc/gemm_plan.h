@@ -31,11 +31,12 @@ inline int64_t splits_held(const void* workspace, size_t bytes, int64_t M, int64
 }
 
 // Whether products that can run as one launch, each in a single pass over K, run one by one: where each split over K is so
-// much faster that together they are (us, one launch | one by one: 2 x 16 x 4096 x 11008, B k-major, bf16 54 | 35;
-// 4 x 64 x 64 x 16384, fp32, both k-major 119 | 41).  Each costs a launch and the gap before it, and the estimates are good
-// to a fifth (3 x 16 x 4096 x 11008, both k-contiguous, estimated as equal: 50 | 58).
-template <typename Plan> inline bool faster_one_by_one(const Plan& group, const Plan& one, int count) {
-  return one.splits > 1 && 1.2 * count * (one.us + 1.0) < group.us;
+// much faster that together they are, by more than the estimates are off (`margin`: bf16 products of a few rows are
+// estimated up to a third too fast, fp32 ones hardly).  A launch more each, and the gap before it.  us, one launch | one by one:
+// bf16, B k-major, 2 x 16 x 4096 x 11008 55 | 38 (3 of them 59 | 62: as one); fp32, both k-major, 4 x 64 x 64 x 16384
+// 119 | 41, 4 x 768 x 768 x 16384 791 | 635, 4 x 768 x 768 x 4096 198 | 210 (as one).
+template <typename Plan> inline bool faster_one_by_one(const Plan& group, const Plan& one, int count, double margin) {
+  return one.splits > 1 && margin * count * (one.us + 1.0) < group.us;
 }
 
 int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void* const* A, const void* const* B, const void* const* R,

@@ -84,8 +84,8 @@ class _Plan(C.Structure):
     ("bf16", 256, 11008, 4096, 1, 0), ("bf16", 300, 11008, 4096, 1, 0), ("bf16", 300, 1000, 16392, 1, 0), ("bf16", 512, 768, 32000, 1, 0),
     ("bf16", 300, 4096, 11008, 2, 1), ("f32", 256, 4096, 11008, 1, 0), ("f32", 512, 768, 32000, 1, 0), ("f32", 300, 4096, 4096, 3, 1)])
 def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K, count, total):
-    """Without room for the planes the blocks are not those that the splits were to multiply: there are more of them, enough
-    for half of the 256 CUs or the smallest ones there are.  With room for some planes there are at most as many splits."""
+    """Without room for the planes the blocks are not the few that the splits were to multiply: there are enough for half of
+    the 256 CUs, or the smallest ones there are.  With room for some planes there are at most as many splits."""
     lib = _lib()
     plan, blocks, trans = ((lib._ZN3emi9bf16_planEllliiil, [(256, 256), (128, 128), (128, 128), (128, 64), (64, 64), (32, 32)], 1)
                            if dtype == "bf16" else (lib._ZN3emi8f32_planEllliiil, [(128, 128), (64, 64), (32, 32)], 0))      # of B, of A
@@ -93,7 +93,7 @@ def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K
     tiles = lambda p: -(-M // blocks[p.shape][0]) * -(-N // blocks[p.shape][1])
     free, one = (plan(M, N, K, count, total, trans, most) for most in (1 << 20, 1))
     assert free.splits > 1 and one.splits == 1
-    assert tiles(one) > tiles(free) and (tiles(one) >= 128 or one.shape == len(blocks) - 1)
+    assert tiles(one) >= 128 or (tiles(one) > tiles(free) and one.shape == len(blocks) - 1)
     for most in range(2, free.splits + 2):
         assert 1 <= plan(M, N, K, count, total, trans, most).splits <= most
     code = 16 if dtype == "bf16" else 11
