@@ -8,9 +8,9 @@
 // k each, filled by direct-to-LDS loads (16 bytes a lane, no staging registers) NST - 1 stages ahead, one barrier per
 // stage, and three shapes of block between which the launcher chooses by how the tiles divide over the CUs (f32_plan()).
 // Measured, us, against 32 x 32 tiles read straight from global memory and 128 x 128 tiles staged through registers
-// (NT / NN / TN form): 256 x 288 x 288: 8.2 -> 5.0 / 7.5 -> 5.4 / 7.5 -> 4.9; 256 x 288 x 768 12.6 -> 7.5; 2000 x 768 x 768
-// 53 -> 32; 2000 x 768 x 2048 90 -> 62; 2048 x 768 x 2000 (TN) 122 -> 61 (103 TFLOP/s); 300 x 4096 x 11008 441 -> 241;
-// 4096^3 1258 -> 1013 (136 TFLOP/s of 157).  What is left on the small ones is the latency of the first loads and the launch.
+// (NT / NN / TN form): 256 x 288 x 288: 8.2 -> 4.9 / 7.5 -> 5.4 / 7.5 -> 4.9; 256 x 288 x 768 12.6 -> 7.3; 2000 x 768 x 768
+// 53 -> 33; 2000 x 768 x 2048 90 -> 63; 2048 x 768 x 2000 (TN) 122 -> 60 (105 TFLOP/s); 300 x 4096 x 11008 441 -> 241;
+// 4096^3 1258 -> 1007 (136 TFLOP/s of 157).  What is left on the small ones is the latency of the first loads and the launch.
 #include <type_traits>
 
 #include "emi_device.h"
