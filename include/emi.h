@@ -118,14 +118,12 @@ int emi_gemm(emi_stream_t stream, const void* A, const void* B, const void* R, v
 /* The same with an optional scratch buffer of emi_gemm_workspace_bytes() bytes (0
  * for shapes that need none).  With it, the single-token adjoint dX = dY.W
  * (trans_a = trans_b = 0, M <= 8) sums row bands of W in many blocks (about 3x
- * faster), and products with few output tiles and a long contraction split K
- * over more blocks, each leaving an fp32 partial [M,N] plane: the weight
- * gradients of a small model on the 128x128 kernel, and in the bf16
- * Y = X.W^T form the shapes with more than 128 tiles of 128x128 but fewer than
- * 192 of 256x256 and K >= 8192 (the classifier adjoint [8192,32000].[32000,768]
- * of a 110M model) on the 256x256 kernel.  The planes are added in a fixed
- * order, with R, before the single rounding.  Without the buffer, or for any
- * other shape, the call is emi_gemm. */
+ * faster), and products whose tiles do not fill the chip split a long contraction
+ * over more blocks, each leaving an fp32 partial [M,N] plane (few tokens, narrow
+ * results, weight gradients of a small model, the classifier adjoint
+ * [8192,32000].[32000,768] of a 110M model).  The planes are added in a fixed
+ * order, with R, before the single rounding.  A smaller buffer, or none, is
+ * planned for: block shape and splits are the best of those that it holds. */
 size_t emi_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, int dtype);
 int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, const void* R, void* C,
                 void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
@@ -138,9 +136,10 @@ int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, const void* R
  * A, B, R, C: tables of `count` pointers (R null, or one entry per result, all set or all null).
  *   sum == 0:  C[i] = op(A[i]) . op(B[i]) [+ R[i]]            (entries may repeat: one X against three weights)
  *   sum == 1:  C[0] = sum_i op(A[i]) . op(B[i]) [+ R[0]]      (products added in index order)
- * Shapes, leading dimensions and flags as for emi_gemm, the same for every product.  Small aligned bf16 products run
- * as one launch; anything else runs as `count` emi_gemm_ws calls with the same results up to the
- * rounding of the intermediate sums (sum == 1 then rounds C[0] to its type between products).  The workspace (size
+ * Shapes, leading dimensions and flags as for emi_gemm, the same for every product.  Aligned products run as
+ * one launch unless each fills the chip, or is so much faster split over K, on its own; those and anything else run as `count`
+ * emi_gemm_ws calls with the same results up to the rounding of the intermediate sums (sum == 1 then rounds C[0] to its
+ * type between products; with sum == 1 aligned products are one launch).  The workspace (size
  * from emi_gemm_grouped_workspace_bytes, may be null) holds split-K partials. */
 #define EMI_GEMM_GROUP_MAX 48
 size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, int sum,
