@@ -137,9 +137,9 @@ int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, const void* R
  *   sum == 0:  C[i] = op(A[i]) . op(B[i]) [+ R[i]]            (entries may repeat: one X against three weights)
  *   sum == 1:  C[0] = sum_i op(A[i]) . op(B[i]) [+ R[0]]      (products added in index order)
  * Shapes, leading dimensions and flags as for emi_gemm, the same for every product.  Aligned products run as
- * one launch unless each fills the chip, or is so much faster split over K, on its own; those and anything else run as `count`
- * emi_gemm_ws calls with the same results up to the rounding of the intermediate sums (sum == 1 then rounds C[0] to its
- * type between products; with sum == 1 aligned products are one launch).  The workspace (size
+ * one launch, unless each fills the chip on its own or, independent, is so much faster split over K; those and anything else
+ * run as `count` emi_gemm_ws calls with the same results up to the rounding of the intermediate sums (sum == 1 then rounds
+ * C[0] to its type between products).  The workspace (size
  * from emi_gemm_grouped_workspace_bytes, may be null) holds split-K partials. */
 #define EMI_GEMM_GROUP_MAX 48
 size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, int sum,
