@@ -1,19 +1,18 @@
-// fp32 products on v_mfma_f32_32x32x2_f32, operands streamed global -> LDS.
+// fp32 products on v_mfma_f32_32x32x2_f32, operands streamed global -> LDS: those of few stages or few tiles.  What has more
+// of both runs on the bf16 instructions (gemm_f32_split.hip); f32_plan() draws the line.
 //
 //   C[M,N] = op(A) . op(B) [+ R]      fp32 throughout
 //
 // An fp32 matrix instruction keeps its SIMD's matrix core busy for 64 cycles and needs 512 bytes of operands, a quarter
-// of what the LDS delivers in that time to four SIMDs: nothing but the matrix cores has to be the limit, provided that
-// loads are in flight all the time and that every CU has the same share of the work.  So: a ring of NST LDS stages of BK
-// k each, filled by direct-to-LDS loads (16 bytes a lane, no staging registers) NST - 1 stages ahead, one barrier per
-// stage, and three shapes of block between which the launcher chooses by how the tiles divide over the CUs (f32_plan()).
-// Measured, us, against 32 x 32 tiles read straight from global memory and 128 x 128 tiles staged through registers
-// (NT / NN / TN form): 256 x 288 x 288: 8.2 -> 4.9 / 7.5 -> 5.4 / 7.5 -> 4.9; 256 x 288 x 768 12.6 -> 7.3; 2000 x 768 x 768
-// 53 -> 33; 2000 x 768 x 2048 90 -> 63; 2048 x 768 x 2000 (TN) 122 -> 60 (105 TFLOP/s); 300 x 4096 x 11008 441 -> 241;
-// 4096^3 1258 -> 1007 (136 TFLOP/s of 157).  What is left on the small ones is the latency of the first loads and the launch.
+// of what the LDS delivers in that time to four SIMDs.  On few tiles what counts is that loads are in flight all the time and
+// that every CU has the same share of the work.  So: a ring of NST LDS stages of BK k each, filled by direct-to-LDS loads
+// (16 bytes a lane, no staging registers) NST - 1 stages ahead, one barrier per stage, and blocks of 64 x 64, or of 32 x 32
+// whose eight wavefronts share k.  Measured, us (NT / NN / TN form): 256 x 288 x 288 4.9 / 5.4 / 4.9; 256 x 288 x 768 7.3;
+// 256 x 768 x 768 7.8.  What is left is the latency of the first loads and the launch.
 #include <type_traits>
 
 #include "emi_device.h"
+#include "gemm_f32.h"
 #include "gemm_plan.h"
 
 namespace emi {
@@ -21,21 +20,6 @@ namespace emi {
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
 #define EMI_LDS __attribute__((address_space(3)))
 constexpr uint32_t kOob = 0x80000000u;   // beyond any buffer's num_records: loads return 0
-
-// Several products of one shape in one launch.  sum == 0: C[i] = op(A[i]) . op(B[i]) [+ R[i]];  sum == 1: every product
-// is accumulated into the tile of C[0] (+ R[0]), pair after pair.
-constexpr int kMaxF32Group = 48;
-struct F32Group {
-  const float* A[kMaxF32Group];
-  const float* B[kMaxF32Group];
-  const float* R[kMaxF32Group];
-  float* C[kMaxF32Group];
-  int count, sum;
-};
-struct F32Single {};
-
-// gemm.hip: adds `splits` planes [M, N] (+ R) into C in plane order
-int launch_f32_splitk_reduce(hipStream_t st, const float* part, const float* R, float* C, int M, int N, int splits, int64_t ldr, int64_t ldc);
 
 template <int N> __device__ __forceinline__ void f32_wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt");
@@ -191,7 +175,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
 
   // A sum over K in one chain is off by the square root of its length, so a chain ends after FLUSH stages (32 k of a
   // wavefront, 64 where wavefronts share k) and goes into `total`; after every stage that happens while the next one's
-  // fragments are on their way.  2 % of the time; relative error of 4096^3 11e-7 -> 2.3e-7, of 2048 x 768 x 2000 5.7e-7 -> 1.5e-7.
+  // fragments are on their way.  2 % of the time; relative error of 2048 x 768 x 2000 5.7e-7 -> 1.5e-7.
   constexpr int FLUSH = WK > 1 ? 8 : 1;
   constexpr f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16_t acc[TM][TN], total[TM][TN];
@@ -298,16 +282,6 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
 // host side
 // ---------------------------------------------------------------------------
 
-struct F32Call {
-  const float *A, *B, *R;
-  float* C;
-  int M, N, K, lda, ldb;
-  int64_t ldr, ldc;
-  float* part;
-  int splits;
-  const F32Group* grp;       // nullptr: the single product of A and B
-};
-
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool AKM, bool BKM, bool GROUPED>
 static int launch_f32_one(hipStream_t st, const F32Call& c) {
   auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, GROUPED>;
@@ -348,31 +322,45 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 }
 
 // Which block and how many splits.  The estimate is of the CU with the most blocks, in microseconds: a start, which grows
-// with the blocks that come after one another, and the stages at the rate that each block shape was measured at.  A stage of
-// 32 k of a 128 x 128 tile takes 2.04 alone on a CU and 1.91 next to others (136 TFLOP/s on 4096^3; the matrix cores' own
-// limit is 157), a 64 x 64 tile 0.64 alone, 1.1 for two blocks and 0.485 a block from four on, a stage of 64 k of a 32 x 32
-// tile whose wavefronts share k 0.40 alone, 0.32 a block from four on.  The start of a further block is 2.5, 0.65 and 1.2:
-// with two to four stages to a block it decides (2048 x 768 x 128, both k-major: 32-tiles 13.6, 64-tiles 9.0).
-// The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s); results over 4 M elements, whose planes
+// with the blocks that come after one another, and the stages at the rate that each block shape was measured at.
+// The fp32 instructions: a stage of 32 k of a 64 x 64 tile takes 0.64 alone, 1.1 for two blocks and 0.485 a block from four on,
+// a stage of 64 k of a 32 x 32 tile whose wavefronts share k 0.40 alone, 0.32 a block from four on; the start of a further
+// block is 0.65 and 1.2.  The bf16 instructions (gemm_f32_split.hip), a stage of 32 k: 1.0, 0.82 and 0.56 for one block of
+// 128 x 128, 128 x 64 and 64 x 64 on a CU, 1.0, 0.58 and 0.34 a block for more, and 0.37, 0.25 and 0.17 more for each block
+// that the chip has per CU (its clock falls as it fills; 0.37, 0.12 and 0.03 up to one); their start is dearer (6.0, 3.8, 3.3; 1.0 more from a k-major A).
+// So the fp32 instructions keep what has few stages or few rows, us, 32- or 64-tiles | the best of the others: 256 x 768 x 768
+// 7.8 | 16, 512 x 768 x 768 12.5 | 14.7, 777 x 512 x 1408 18.7 | 19.3, 768 x 768 x 32 (TN) 5.0 | 5.5; and beyond: 2000 x 768 x 768
+// 33 | 25.6, 2000 x 768 x 2048 62 | 48, 768 x 768 x 4096 (TN, four) 208 | 146, 4096^3 1025 | 732.
+// The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s; 1 more where it follows a split kernel's
+// long epilogue); results over 4 M elements, whose planes
 // leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few
 // rows of a k-major A are no such product (4 x 64 x 20000, us: 126 in one pass, 12 split).
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
   struct Shape { int tile, bk; double one, base, block, rate[4]; };     // start of one block, of b: base + b block; rate[b - 1]: per
                                                                         // stage, b blocks on the CU; the last one per block
-  static const Shape shapes[3] = {{128, 32, 4.8, 4.0, 2.5, {2.04, 3.86, 5.82, 1.91}}, {64, 32, 3.4, 4.0, 0.65, {0.64, 1.10, 1.50, 0.485}},
-                                  {32, 64, 3.4, 2.5, 1.2, {0.40, 0.69, 1.00, 0.32}}};
-  F32Plan best{2, 1, 0.0};
+  static const Shape shapes[2] = {{64, 32, 3.4, 4.0, 0.65, {0.64, 1.10, 1.50, 0.485}}, {32, 64, 3.4, 2.5, 1.2, {0.40, 0.69, 1.00, 0.32}}};
+  struct Split { int bm, bn; double base, block, one, one_fill, rate, fill; };
+  static const Split splits[3] = {{128, 128, 1.6, 4.4, 1.0, 0.37, 1.0, 0.37}, {128, 64, 2.0, 1.8, 0.82, 0.12, 0.58, 0.25},
+                                  {64, 64, 1.2, 2.1, 0.56, 0.03, 0.34, 0.17}};
+  F32Plan best{1, 1, 0.0};
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && (M > 8 || trans_a) && K > 8;
   double least = 1e30;
-  for (int c = 0; c < 3; c++) {
-    const Shape& s = shapes[c];
-    const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
-    const int64_t blocks = (M + s.tile - 1) / s.tile * ((N + s.tile - 1) / s.tile) * (sum ? 1 : count);
+  for (int c = 0; c < 5; c++) {
+    const int bm = c < 2 ? shapes[c].tile : splits[c - 2].bm, bn = c < 2 ? shapes[c].tile : splits[c - 2].bn, bk = c < 2 ? shapes[c].bk : 32;
+    const int64_t steps = (K + bk - 1) / bk * (sum ? count : 1);
+    const int64_t blocks = (M + bm - 1) / bm * ((N + bn - 1) / bn) * (sum ? 1 : count);
     if (blocks > 0x3fffffff) continue;
     for (int64_t z = 1; z <= 64 && z <= most && (z == 1 || (may_split && steps >= 4 * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
-      const double t = (b == 1 ? s.one : s.base + s.block * b) + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b) +
-                       (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
+      double t = z > 1 ? (c < 2 ? 3.0 : 4.0) + 1e-6 * M * N * (z + 1) : 0.0;
+      if (c < 2) {
+        const Shape& s = shapes[c];
+        t += (b == 1 ? s.one : s.base + s.block * b) + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b);
+      } else {
+        const Split& s = splits[c - 2];
+        t += s.base + s.block * b + (trans_a ? 1.0 : 0.0) + per * ((b == 1 ? s.one : s.rate * b) + (b == 1 ? s.one_fill : s.fill) * (blocks * z / 256.0));
+      }
+      if (c > 1) t *= 1.04;                                       // near the line the fp32 instructions stay
       if (t < least) {
         least = t;
         best = F32Plan{c, (int)z, t};
@@ -420,10 +408,12 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   }
   const F32Call c{g.A[0], g.B[0], g.R[0], g.C[0], (int)M, (int)N, (int)K, (int)lda, (int)ldb, ldr, ldc, static_cast<float*>(workspace),
                   p.splits, count > 1 ? &g : nullptr};
-  switch (p.config) {
-    case 0: return launch_f32_shape<128, 128, 4, 2, 1, 32, 2>(st, c, trans_a, trans_b);
-    case 1: return launch_f32_shape<64, 64, 2, 2, 1, 32, 2>(st, c, trans_a, trans_b);
-    default: return launch_f32_shape<32, 32, 1, 1, 8, 64, 5>(st, c, trans_a, trans_b);
+  // (the split kernels address a tile of the result with 31 bits too)
+  const bool wide = 128 * ldc >= 0x1fffffff || 128 * N >= 0x1fffffff || (R != nullptr && 128 * ldr >= 0x1fffffff);
+  switch (wide && p.config > 1 ? 0 : p.config) {
+    case 0: return launch_f32_shape<64, 64, 2, 2, 1, 32, 2>(st, c, trans_a, trans_b);
+    case 1: return launch_f32_shape<32, 32, 1, 1, 8, 64, 5>(st, c, trans_a, trans_b);
+    default: return launch_f32_bf16x3(st, c, p.config - 2, trans_a, trans_b);
   }
 }
 

@@ -1,0 +1,72 @@
+"""fp32 products on the bf16 matrix cores: the sizes at which each block shape is chosen and its tiles, stages in flight and
+splits end, and operands that three bf16 numbers do not hold (infinite, NaN, beyond the largest bf16, below what the
+third one reaches), which are multiplied as fp32 numbers.  Against float64 products."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import dev, host
+
+pytestmark = pytest.mark.gpu
+
+# blocks of 64 x 64; of 128 x 64 with fewer stages than are in flight; of 128 x 128, two splits
+SIZES = [(1000, 1028, 1036), (2052, 2044, 68), (1996, 772, 2052)]
+
+
+def _operands(rng, M, N, K, ta, tb):
+    return rng.standard_normal((K, M) if ta else (M, K)), rng.standard_normal((N, K) if tb else (K, N))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", SIZES + [(1060, 1092, 2052), (4100, 2052, 36), (777, 4096, 772)])
+def test_errors_of_an_fp32_product(ta, tb, M, N, K):
+    """Within (K + 2) 2^-23 sum |a b|, as any order of fp32 sums is (three dropped products of 2^-25 each are less than what
+    the roundings of a shorter chain leave of it), and in the mean square no further off than chains of 64 terms."""
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + N + K + 2 * ta + tb)
+    a, b = _operands(rng, M, N, K, ta, tb)
+    (A, Ar), (B, Br), (R, Rr) = dev(a, "f32"), dev(b, "f32"), dev(rng.standard_normal((M, N)), "f32")
+    x, y = Ar.T if ta else Ar, Br.T if tb else Br
+    ref = x @ y
+    got = host(ops.gemm(A, B, bool(ta), bool(tb), R))
+    bound = (K + 2) * 2.0 ** -23 * (np.abs(x) @ np.abs(y) + np.abs(Rr))
+    assert np.all(np.abs(got - ref - Rr) <= bound)
+    got = host(ops.gemm(A, B, bool(ta), bool(tb)))
+    assert np.linalg.norm(got - ref) <= 2.0 ** -24 * np.sqrt((64 + K / 32) / 2) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0)])
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("what", ["infinite", "nan", "huge", "tiny", "tiny rows", "zero"])
+def test_numbers_that_do_not_split(what, ta, tb, M, N, K):
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + N + K + 2 * ta + tb)
+    a, b = _operands(rng, M, N, K, ta, tb)
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    at = lambda m, k: (k, m) if ta else (m, k)                  # of row m of the result, term k
+    if what == "infinite":
+        a[at(3, 5)], a[at(M - 1, K - 1)] = np.inf, -np.inf
+        b[(N - 2, 7) if tb else (7, N - 2)] = np.inf
+    elif what == "nan":
+        a[at(M // 2, K - 2)] = np.nan
+    elif what == "huge":                                        # finite, but rounds to an infinite bf16
+        a[at(3, 5)] = 3.4e38
+        b *= np.float32(1e-3)
+    elif what == "tiny":
+        a *= np.float32(1e-36)
+    elif what == "tiny rows":                                   # beside ordinary ones: what they lose is below those' roundings
+        a[(slice(None), slice(5, 9)) if ta else slice(5, 9)] *= np.float32(1e-36)
+    else:
+        a[:] = 0
+    A, B = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    got = host(ops.gemm(A, B, bool(ta), bool(tb)))
+    x, y = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref = x @ y
+        mag = np.abs(x) @ np.abs(y)
+    finite = np.isfinite(ref)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    slack = 2.0 ** -130 * np.abs(y).sum(0)[None, :] if what == "tiny rows" else 2.0 ** -149 * K     # the last bit of l; denormal results
+    bound = (K + 2) * 2.0 ** -23 * mag + slack
+    assert np.all(np.abs(got[finite] - ref[finite]) <= bound[finite])
