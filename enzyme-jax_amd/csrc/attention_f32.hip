@@ -9,7 +9,7 @@
 // score has the weight 0 and its row is multiplied by it, so a NaN or an infinity in a row of v also reaches earlier queries
 // of the same 16-row tile. Operands come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
 // 16 rows are one chain of them, so with one wavefront per 16 rows (the earlier form) the longest row set the time and too
-// few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 24,
+// few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 11,
 // 24 heads x 1000 x 64 89 / 280 -> 56 / 161 (55 / 48 TFLOP/s), 64 heads x 2048 x 128 1329 / 4010 -> 795 / 2907 (86 / 59);
 // the loads of K, V and Q through the L1 come next.
 // As on the bf16 path everything is computed transposed: the score tile is S^T[other row, own row], so lane l owns row
@@ -122,11 +122,14 @@ __device__ __forceinline__ void merge_store(float* __restrict__ row, bool write,
 // Which 16 rows and which head a block has.  Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its
 // own; here every XCD gets a run of whole heads, so that a head's other operands are fetched into one L2 instead of eight.
 struct BlockRows { int tile, bh; };
-__device__ __forceinline__ BlockRows block_rows(int tiles) {
-  const int total = (int)(gridDim.x * gridDim.y), id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+__device__ __forceinline__ BlockRows block_rows(int tiles, int total, int id) {
   const int per = total >> 3, extra = total & 7, xcd = id & 7;
   const int w = xcd * per + (xcd < extra ? xcd : extra) + (id >> 3);
   return {w % tiles, w / tiles};
+}
+
+__device__ __forceinline__ BlockRows block_rows(int tiles) {
+  return block_rows(tiles, (int)(gridDim.x * gridDim.y), (int)(blockIdx.y * gridDim.x + blockIdx.x));
 }
 
 __device__ __forceinline__ float groups_max(float x) {      // over the four lanes that share l % 16
@@ -226,16 +229,12 @@ __global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* 
 // dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T, delta = rowsum(dO * O), which it also
 // leaves for the dK/dV kernel.
 template <int NT>
-__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                      const float* __restrict__ v, const float* __restrict__ o,
-                                                                      const float* __restrict__ d_o,
-                                                                      const float* __restrict__ lse, float* __restrict__ delta,
-                                                                      float* __restrict__ dq, AttnShapeF32 sh, float scale,
-                                                                      int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
+__device__ __forceinline__ void bwd_dq_rows(const BlockRows own, const float* __restrict__ q, const float* __restrict__ k,
+                                            const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ d_o,
+                                            const float* __restrict__ lse, float* __restrict__ delta, float* __restrict__ dq,
+                                            AttnShapeF32 sh, float scale, int causal, float (&buf)[kWaves][kWaves * NT][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
   const int tiles = (sh.seq + 15) >> 4;
-  const BlockRows own = block_rows(tiles);
   const int q0 = (tiles - 1 - own.tile) * 16;
   const int bh = own.bh;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
@@ -255,7 +254,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const floa
 #pragma unroll
       for (int t = 0; t < 4; t++) dl += of[c][t] * dof[c][t];
     dl = groups_sum(dl);
-    if (wave == 0 && G == 0 && myq < sh.seq) delta[(int64_t)bh * sh.seq + myq] = dl;
+    if (delta != nullptr && wave == 0 && G == 0 && myq < sh.seq) delta[(int64_t)bh * sh.seq + myq] = dl;
   }
   const int nkeys = causal ? (q0 + 16 < sh.seq ? q0 + 16 : sh.seq) : sh.seq;
   f32q_t acc[NT];
@@ -282,17 +281,14 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const floa
 }
 
 // dV = P^T dO, dK = scale dS^T Q: a block per 16 keys, walking the queries that see them.
-template <int NT>
-__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                       const float* __restrict__ v,
-                                                                       const float* __restrict__ d_o,
-                                                                       const float* __restrict__ lse,
-                                                                       const float* __restrict__ delta, float* __restrict__ dk,
-                                                                       float* __restrict__ dv, AttnShapeF32 sh, float scale,
-                                                                       int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
+// DELTA: from the rows of o, where nothing has left delta.
+template <int NT, bool DELTA>
+__device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* __restrict__ q, const float* __restrict__ k,
+                                             const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ d_o,
+                                             const float* __restrict__ lse, const float* __restrict__ delta, float* __restrict__ dk,
+                                             float* __restrict__ dv, AttnShapeF32 sh, float scale, int causal,
+                                             float (&buf)[kWaves][kWaves * NT][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
-  const BlockRows own = block_rows((sh.seq + 15) >> 4);
   const int key0 = own.tile * 16;                                  // the earliest keys see the most queries
   const int bh = own.bh;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
@@ -302,7 +298,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const flo
   load_rows<NT>(k + base, sh.ss, key0, last, lane, kf);
   load_rows<NT>(v + base, sh.ss, key0, last, lane, vf);
   const float* lrow = lse + (int64_t)bh * sh.seq;
-  const float* drow = delta + (int64_t)bh * sh.seq;
+  [[maybe_unused]] const float* drow = DELTA ? nullptr : delta + (int64_t)bh * sh.seq;
   f32q_t acck[NT], accv[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) acck[n] = accv[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
@@ -317,7 +313,18 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const flo
       const int qi = qb + 4 * G + r;
       const int qc = qi < last ? qi : last;
       lq[r] = lrow[qc];
-      dq_[r] = drow[qc];
+      if constexpr (!DELTA) dq_[r] = drow[qc];
+    }
+    if constexpr (DELTA) {
+      float of[NT][4], dl = 0.f;
+      load_rows<NT>(o + base, sh.ss, qb, last, lane, of);
+#pragma unroll
+      for (int c = 0; c < NT; c++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) dl += of[c][t] * dof[c][t];
+      dl = groups_sum(dl);                              // of query qb + l % 16
+#pragma unroll
+      for (int r = 0; r < 4; r++) dq_[r] = __shfl(dl, 4 * G + r);
     }
     f32q_t s = rows_dot<NT>(qf, kf);                   // register r: query qb + 4 G + r, key mykey
     f32q_t dp = rows_dot<NT>(dof, vf);
@@ -336,6 +343,42 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const flo
   merge_store<NT>(dk + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, acck, one, buf);
   __syncthreads();
   merge_store<NT>(dv + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, accv, one, buf);
+}
+
+template <int NT>
+__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                      const float* __restrict__ v, const float* __restrict__ o,
+                                                                      const float* __restrict__ d_o,
+                                                                      const float* __restrict__ lse, float* __restrict__ delta,
+                                                                      float* __restrict__ dq, AttnShapeF32 sh, float scale,
+                                                                      int causal) {
+  __shared__ float buf[kWaves][kWaves * NT][64];
+  bwd_dq_rows<NT>(block_rows((sh.seq + 15) >> 4), q, k, v, o, d_o, lse, delta, dq, sh, scale, causal, buf);
+}
+template <int NT>
+__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                       const float* __restrict__ v,
+                                                                       const float* __restrict__ d_o,
+                                                                       const float* __restrict__ lse,
+                                                                       const float* __restrict__ delta, float* __restrict__ dk,
+                                                                       float* __restrict__ dv, AttnShapeF32 sh, float scale,
+                                                                       int causal) {
+  __shared__ float buf[kWaves][kWaves * NT][64];
+  bwd_dkv_rows<NT, false>(block_rows((sh.seq + 15) >> 4), q, k, v, nullptr, d_o, lse, delta, dk, dv, sh, scale, causal, buf);
+}
+
+// Both as one launch (grid.z: 0 dK/dV, 1 dQ), for sequences and heads that leave the chip half empty: the two run side by side
+// instead of one after the other, and dK/dV forms delta itself.
+template <int NT>
+__global__ __launch_bounds__(64 * kWaves) void attn_bwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                   const float* __restrict__ v, const float* __restrict__ o,
+                                                                   const float* __restrict__ d_o, const float* __restrict__ lse,
+                                                                   float* __restrict__ dq, float* __restrict__ dk,
+                                                                   float* __restrict__ dv, AttnShapeF32 sh, float scale, int causal) {
+  __shared__ float buf[kWaves][kWaves * NT][64];
+  const BlockRows own = block_rows((sh.seq + 15) >> 4);
+  if (blockIdx.z == 0) bwd_dkv_rows<NT, true>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, buf);
+  else bwd_dq_rows<NT>(own, q, k, v, o, d_o, lse, nullptr, dq, sh, scale, causal, buf);
 }
 
 static bool f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
@@ -380,6 +423,17 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
+  // One launch while two would each leave much of the chip idle; with more blocks the registers that dQ then takes for dK/dV's
+  // sake cost more.  us, two | one: 6 heads x 256 x 48 (96 blocks) 17.3 | 11.3, 24 x 512 x 64 (768) 73 | 58, 64 x 300 x 64 (1216)
+  // 62 | 59, 24 x 1000 x 64 (1512) 160 | 163; 8 x 1000 x 128 (504) 142 | 132, 128 x 128 x 128 (1024) 71 | 81.
+  if ((int64_t)grid.x * grid.y <= (head_dim <= 64 ? 1024 : 512)) {
+    EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
+                          hipLaunchKernelGGL(attn_bwd_f32_kernel<NT>, dim3(grid.x, grid.y, 2), dim3(64 * kWaves), 0, st, (const float*)q,
+                                             (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, (float*)dq,
+                                             (float*)dk, (float*)dv, shp, scale, causal));
+    EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma)");
+    return EMI_OK;
+  }
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
                         hipLaunchKernelGGL(attn_bwd_dq_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q,
                                            (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, delta,
