@@ -335,36 +335,56 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 // long epilogue); results over 4 M elements, whose planes
 // leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few
 // rows of a k-major A are no such product (4 x 64 x 20000, us: 126 in one pass, 12 split).
+struct F32Shape { int bm, bn, bk, config; };
+constexpr int kF32Shapes = 5;
+static const F32Shape kF32Shape[kF32Shapes] = {{64, 64, 32, 1}, {32, 32, 64, 2}, {128, 128, 32, 0}, {128, 64, 32, 1}, {64, 64, 32, 1}};   // two fp32, three bf16
+
+// Microseconds of the products in blocks of shape c over z splits; not finite where it cannot be.
+static double f32_estimate(int c, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t z) {
+  struct Fp32 { double one, base, block, rate[4]; };      // start of one block, of b: base + b block; rate[b - 1]: per stage, b blocks on
+                                                          // the CU; the last one per block
+  static const Fp32 fp32[2] = {{3.4, 4.0, 0.65, {0.64, 1.10, 1.50, 0.485}}, {3.4, 2.5, 1.2, {0.40, 0.69, 1.00, 0.32}}};
+  struct Bf16 { double base, block, one, one_fill, rate, fill; };
+  static const Bf16 bf16[3] = {{1.6, 4.4, 1.0, 0.37, 1.0, 0.37}, {2.0, 1.8, 0.82, 0.12, 0.58, 0.25}, {1.2, 2.1, 0.56, 0.03, 0.34, 0.17}};
+  const F32Shape& s = kF32Shape[c];
+  const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
+  const int64_t blocks = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * (sum ? 1 : count);
+  if (blocks > 0x3fffffff || (z > 1 && steps < 4 * z)) return 1e30;
+  const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
+  if (c < 2) {
+    const Fp32& r = fp32[c];
+    return (b == 1 ? r.one : r.base + r.block * b) + per * (b < 4 ? r.rate[b - 1] : r.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
+  }
+  const Bf16& r = bf16[c - 2];
+  const double t = r.base + r.block * b + (trans_a ? 1.0 : 0.0) +
+                   per * ((b == 1 ? r.one : r.rate * b) + (b == 1 ? r.one_fill : r.fill) * (blocks * z / 256.0));
+  return 1.04 * (t + (z > 1 ? 4.0 + 1e-6 * M * N * (z + 1) : 0.0));       // near the line the fp32 instructions stay
+}
+
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
-  struct Shape { int tile, bk; double one, base, block, rate[4]; };     // start of one block, of b: base + b block; rate[b - 1]: per
-                                                                        // stage, b blocks on the CU; the last one per block
-  static const Shape shapes[2] = {{64, 32, 3.4, 4.0, 0.65, {0.64, 1.10, 1.50, 0.485}}, {32, 64, 3.4, 2.5, 1.2, {0.40, 0.69, 1.00, 0.32}}};
-  struct Split { int bm, bn; double base, block, one, one_fill, rate, fill; };
-  static const Split splits[3] = {{128, 128, 1.6, 4.4, 1.0, 0.37, 1.0, 0.37}, {128, 64, 2.0, 1.8, 0.82, 0.12, 0.58, 0.25},
-                                  {64, 64, 1.2, 2.1, 0.56, 0.03, 0.34, 0.17}};
-  F32Plan best{1, 1, 0.0};
+  F32Plan best{2, 1, 0.0};
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && (M > 8 || trans_a) && K > 8;
   double least = 1e30;
-  for (int c = 0; c < 5; c++) {
-    const int bm = c < 2 ? shapes[c].tile : splits[c - 2].bm, bn = c < 2 ? shapes[c].tile : splits[c - 2].bn, bk = c < 2 ? shapes[c].bk : 32;
-    const int64_t steps = (K + bk - 1) / bk * (sum ? count : 1);
-    const int64_t blocks = (M + bm - 1) / bm * ((N + bn - 1) / bn) * (sum ? 1 : count);
-    if (blocks > 0x3fffffff) continue;
-    for (int64_t z = 1; z <= 64 && z <= most && (z == 1 || (may_split && steps >= 4 * z)); z++) {
-      const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
-      double t = z > 1 ? (c < 2 ? 3.0 : 4.0) + 1e-6 * M * N * (z + 1) : 0.0;
-      if (c < 2) {
-        const Shape& s = shapes[c];
-        t += (b == 1 ? s.one : s.base + s.block * b) + per * (b < 4 ? s.rate[b - 1] : s.rate[3] * b);
-      } else {
-        const Split& s = splits[c - 2];
-        t += s.base + s.block * b + (trans_a ? 1.0 : 0.0) + per * ((b == 1 ? s.one : s.rate * b) + (b == 1 ? s.one_fill : s.fill) * (blocks * z / 256.0));
-      }
-      if (c > 1) t *= 1.04;                                       // near the line the fp32 instructions stay
+  for (int c = 0; c < kF32Shapes; c++)
+    for (int64_t z = 1; z <= (may_split ? 64 : 1) && z <= most; z++) {
+      const double t = f32_estimate(c, M, N, K, count, sum, trans_a, z);
       if (t < least) {
         least = t;
-        best = F32Plan{c, (int)z, t};
+        best = F32Plan{kF32Shape[c].config, (int)z, t};
       }
+    }
+  return best;
+}
+
+// Which of the shapes of the plan's blocks.
+static int f32_shape(const F32Plan& p, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a) {
+  int best = 1;
+  double least = 1e30;
+  for (int c = 0; c < kF32Shapes; c++) {
+    const double t = kF32Shape[c].config == p.config ? f32_estimate(c, M, N, K, count, sum, trans_a, p.splits) : 1e30;
+    if (t < least) {
+      least = t;
+      best = c;
     }
   }
   return best;
@@ -410,10 +430,11 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
                   p.splits, count > 1 ? &g : nullptr};
   // (the split kernels address a tile of the result with 31 bits too)
   const bool wide = 128 * ldc >= 0x1fffffff || 128 * N >= 0x1fffffff || (R != nullptr && 128 * ldr >= 0x1fffffff);
-  switch (wide && p.config > 1 ? 0 : p.config) {
+  const int shape = f32_shape(p, M, N, K, count, sum, trans_a);
+  switch (wide && shape > 1 ? 0 : shape) {
     case 0: return launch_f32_shape<64, 64, 2, 2, 1, 32, 2>(st, c, trans_a, trans_b);
     case 1: return launch_f32_shape<32, 32, 1, 1, 8, 64, 5>(st, c, trans_a, trans_b);
-    default: return launch_f32_bf16x3(st, c, p.config - 2, trans_a, trans_b);
+    default: return launch_f32_bf16x3(st, c, shape - 2, trans_a, trans_b);
   }
 }
 

@@ -11,7 +11,7 @@ struct Bf16Plan {
   double us;        // the estimate
 };
 struct F32Plan {
-  int config;       // 0: blocks of 64 x 64, 1: 32 x 32 (gemm_f32.hip), 2: 128 x 128, 3: 128 x 64, 4: 64 x 64 (gemm_f32_split.hip)
+  int config;       // 0: blocks of 128 x 128, 1: of 64 columns, 2: 32 x 32 (gemm_f32.hip)
   int splits;
   double us;
 };
