@@ -10,6 +10,11 @@
 
 namespace emi {
 
+__device__ __forceinline__ float4 pack_raw(const float (&v)[4]) { return make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ uint4 pack_raw(const float (&v)[8]) {
+  return make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+}
+
 // ---------------------------------------------------------------------------
 // RMSNorm (test/llama.py:6-10): y = gamma * x * rsqrt(mean(x^2) + eps)
 // TPR threads cooperate on one row (64 = one wavefront per row, four rows per
@@ -93,11 +98,14 @@ template <int TPR, int NV> __device__ __forceinline__ void row_reduce_n(float (&
 // Adjoint.  Blocks walk rows with a grid stride, NR rows per step, and keep this
 // thread's share of dgamma in registers; partial[blockIdx*RPB + rib][dim] is reduced
 // by colsum_kernel.  dx = [dx_add +] r*g - x * r^3 * mean(g*x), g = dy*gamma.
-template <typename T, int TPR, int NCH, int NR>
+// ROPE: dy is the cotangent of the rotated result; each piece is rotated back (and rounded to T, as a pass of its own over
+// dy would leave it) on its way in, by the angles of the row's position row % seq.  16 x 2048 rows of 4096 fp32,
+// us: rotation 180 and this 269 -> 271: the angles come from the L1, and what bounds both is x, dy in and dx out (5.9 TB/s).
+template <typename T, int TPR, int NCH, int NR, bool ROPE>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                           const T* __restrict__ dy, const T* dx_add, T* dx,
                                                           float* __restrict__ partial, int64_t rows, int dim,
-                                                          float eps) {
+                                                          float eps, const float2* __restrict__ table, int seq, int head_dim) {
   // NCH groups of 8 elements per thread, held as 16-byte pieces (8 bf16 or 4 floats) so that consecutive lanes cover
   // consecutive 16 bytes (the access shape of the streaming loads and stores)
   constexpr int RPB = 256 / TPR, N = Chunk<T>::N, NC = NCH * 8 / N;
@@ -118,17 +126,28 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
   // reduction (shuffles, LDS, barrier) of the current one, which keeps twice the
   // bytes in flight per block.
   typename Chunk<T>::Raw xn[NR][NC], gn[NR][NC];      // kept in storage format to save registers
+  [[maybe_unused]] float4 tn[NR][NC][N / 4];          // two (cos, sin) entries each
   auto load_step = [&](int64_t sg) {
 #pragma unroll
     for (int u = 0; u < NR; u++) {
       const int64_t row = (sg * NR + u) * RPB + rib;
+      [[maybe_unused]] const float2* angles = nullptr;
+      if constexpr (ROPE) angles = table + (int64_t)((uint32_t)row % (uint32_t)seq) * (head_dim >> 1);
 #pragma unroll
       for (int j = 0; j < NC; j++) {
         const int c = tir + j * TPR;
         if (sg < nstep && row < rows && c < nchunk) {
+          if constexpr (ROPE) {
+            const float4* t = reinterpret_cast<const float4*>(angles + (((uint32_t)(c * N) % (uint32_t)head_dim) >> 1));
+#pragma unroll
+            for (int q = 0; q < N / 4; q++) tn[u][j][q] = t[q];
+          }
           xn[u][j] = Chunk<T>::load_raw(x + row * dim + c * N);
           gn[u][j] = Chunk<T>::load_raw(dy + row * dim + c * N);
         } else {
+          if constexpr (ROPE)
+#pragma unroll
+            for (int q = 0; q < N / 4; q++) tn[u][j][q] = make_float4(1.f, 0.f, 1.f, 0.f);
           xn[u][j] = typename Chunk<T>::Raw{};
           gn[u][j] = typename Chunk<T>::Raw{};
         }
@@ -147,6 +166,18 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
       for (int j = 0; j < NC; j++) {
         xc[u][j] = xn[u][j];
         gc[u][j] = gn[u][j];
+        if constexpr (ROPE) {
+          float v[N], o[N];
+          Chunk<T>::unpack(gc[u][j], v);
+#pragma unroll
+          for (int p = 0; p < N / 2; p++) {
+            const float4 t = tn[u][j][p >> 1];
+            const float cs = (p & 1) ? t.z : t.x, sp = (p & 1) ? -t.w : -t.y;
+            o[2 * p] = cs * v[2 * p] - sp * v[2 * p + 1];
+            o[2 * p + 1] = sp * v[2 * p] + cs * v[2 * p + 1];
+          }
+          gc[u][j] = pack_raw(o);
+        }
         float xv[N], gv[N];
         Chunk<T>::unpack(xc[u][j], xv);
         Chunk<T>::unpack(gc[u][j], gv);
@@ -638,7 +669,9 @@ static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, 
 
 template <typename T>
 static int rmsnorm_bwd_launch(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add,
-                              void* dx, void* dgamma, void* ws, int64_t rows, int64_t dim, float eps) {
+                              void* dx, void* dgamma, void* ws, int64_t rows, int64_t dim, float eps, const float* table = nullptr,
+                              int seq = 1, int head_dim = 2) {
+  const float2* tp = reinterpret_cast<const float2*>(table);
   const T* xp = static_cast<const T*>(x);
   const T* gp = static_cast<const T*>(gamma);
   const T* dyp = static_cast<const T*>(dy);
@@ -652,15 +685,21 @@ static int rmsnorm_bwd_launch(hipStream_t st, const void* x, const void* gamma, 
     hipLaunchKernelGGL(rmsnorm_bwd_generic_kernel<T>, dim3((unsigned)grid), dim3(256), 0, st, xp, gp, dyp, ap, dxp, part,
                        rows, dim, eps);
   } else {
-#define EMI_RMS_BWD(TPR, NCH)                                                                                   \
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, TPR, NCH, (sizeof(T) == 2 ? 2 : 1)>), dim3((unsigned)grid), dim3(256), 0, st, xp, gp, dyp, ap, dxp, \
-                     part, rows, (int)dim, eps)
+#define EMI_RMS_BWD_R(TPR, NCH, ROPE)                                                                                                         \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, TPR, NCH, (sizeof(T) == 2 ? 2 : 1), ROPE>), dim3((unsigned)grid), dim3(256), 0, st, xp, gp, dyp, \
+                     ap, dxp, part, rows, (int)dim, eps, tp, seq, head_dim)
+#define EMI_RMS_BWD(TPR, NCH)                          \
+  do {                                                 \
+    if (tp != nullptr) EMI_RMS_BWD_R(TPR, NCH, true);  \
+    else EMI_RMS_BWD_R(TPR, NCH, false);               \
+  } while (0)
     if (tpr == 64 && nch == 1) EMI_RMS_BWD(64, 1);
     else if (tpr == 64) EMI_RMS_BWD(64, 2);
     else if (nch == 1) EMI_RMS_BWD(256, 1);
     else if (nch == 2) EMI_RMS_BWD(256, 2);
     else EMI_RMS_BWD(256, 4);
 #undef EMI_RMS_BWD
+#undef EMI_RMS_BWD_R
   }
   EMI_CHECK_LAUNCH("emi_rmsnorm_bwd");
   // [nparts, dim] -> [ceil(nparts/CS_ROWS), dim] -> ... -> dgamma
@@ -729,6 +768,29 @@ extern "C" int emi_rmsnorm_bwd(emi_stream_t stream, const void* x, const void* g
   EMI_DISPATCH_DTYPE("emi_rmsnorm_bwd", dtype,
                      rmsnorm_bwd_launch<float>(st, x, gamma, dy, dx_add, dx, dgamma, workspace, rows, dim, eps),
                      rmsnorm_bwd_launch<bf16>(st, x, gamma, dy, dx_add, dx, dgamma, workspace, rows, dim, eps));
+}
+
+extern "C" int emi_rmsnorm_bwd_rope(emi_stream_t stream, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx,
+                                    void* dgamma, const float* rope_table, void* workspace, size_t workspace_bytes, int64_t rows, int64_t dim,
+                                    int64_t seq, int64_t head_dim, float eps, int dtype) {
+  EMI_REQUIRE(rows > 0 && dim > 0 && seq > 0 && head_dim > 0, "emi_rmsnorm_bwd_rope: bad shape rows=%lld dim=%lld seq=%lld head_dim=%lld",
+              (long long)rows, (long long)dim, (long long)seq, (long long)head_dim);
+  EMI_REQUIRE(rows <= 0x7fffffff && seq <= 0x7fffffff, "emi_rmsnorm_bwd_rope: rows=%lld or seq=%lld too large", (long long)rows, (long long)seq);
+  EMI_REQUIRE(x && gamma && dy && dx && dgamma && rope_table, "emi_rmsnorm_bwd_rope: null buffer");
+  EMI_REQUIRE(aligned16(x) && aligned16(gamma) && aligned16(dy) && aligned16(dx) && aligned16(dx_add) && aligned16(rope_table) &&
+                  aligned16(workspace),
+              "emi_rmsnorm_bwd_rope: buffers must be 16-byte aligned");
+  EMI_REQUIRE(dtype == EMI_F32 || dtype == EMI_BF16, "emi_rmsnorm_bwd_rope: unsupported dtype code %d (want 11=f32 or 16=bf16)", dtype);
+  EMI_REQUIRE(dim % 8 == 0 && dim <= 8192 && dim % head_dim == 0 && head_dim % (dtype == EMI_BF16 ? 8 : 4) == 0,
+              "emi_rmsnorm_bwd_rope: rows of %lld elements in heads of %lld are not whole 16-byte pieces (at most 8192 elements)", (long long)dim,
+              (long long)head_dim);
+  const size_t need = emi_rmsnorm_bwd_workspace_bytes(rows, dim);
+  EMI_REQUIRE(workspace != nullptr && workspace_bytes >= need, "emi_rmsnorm_bwd_rope: workspace of %zu bytes needed, got %zu", need,
+              workspace_bytes);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == EMI_F32)
+    return rmsnorm_bwd_launch<float>(st, x, gamma, dy, dx_add, dx, dgamma, workspace, rows, dim, eps, rope_table, (int)seq, (int)head_dim);
+  return rmsnorm_bwd_launch<bf16>(st, x, gamma, dy, dx_add, dx, dgamma, workspace, rows, dim, eps, rope_table, (int)seq, (int)head_dim);
 }
 
 // ---------------------------------------------------------------------------

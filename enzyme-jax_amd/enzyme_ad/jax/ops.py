@@ -19,6 +19,7 @@ instead of costing an extra pass over HBM.
 import math
 
 import ctypes
+import functools
 import threading
 
 import torch
@@ -184,7 +185,21 @@ class Tape(metaclass=_PerThread):
             if c.shape != o.shape or c.dtype != o.dtype:
                 raise ValueError("cotangent %s/%s does not match output %s/%s" % (tuple(c.shape), c.dtype, tuple(o.shape), o.dtype))
             ct[id(o)] = c if id(o) not in ct else add(ct[id(o)], c)
+        # a rotation whose operand is an RMSNorm result that nothing else reads or asks for: its cotangent goes to the norm's
+        # rule as it is, which rotates it back in its own pass
+        uses = _pass().uses
+        norms = {id(o) for _, o, rule in self.nodes if getattr(rule, "_emi_rotated", False)} - {id(w) for w in wrt}
+        rotated = {}
         for inputs, output, rule in reversed(self.nodes):
+            rotation = getattr(rule, "_emi_rotation", None)
+            if rotation is not None:
+                y = id(inputs[0])
+                if y in norms and uses.get(y) == 1 and y not in ct and id(output) in ct and ct[id(output)].is_contiguous():
+                    ct[y] = ct.pop(id(output))
+                    rotated[y] = rotation
+                    continue
+            elif id(output) in rotated:
+                rule = functools.partial(rule, rotation=rotated.pop(id(output)))
             if isinstance(output, tuple):                # the rule takes the tuple of cotangents (None = zero)
                 c = tuple(ct.pop(id(o), None) for o in output)
                 if all(x is None for x in c):
@@ -298,17 +313,23 @@ def rmsnorm(x, gamma, eps=1e-5):
     y = torch.empty_like(x)
     N.check(N.lib().emi_rmsnorm_fwd(_stream(), _p(x), _p(gamma), _p(y), rows, D, eps, _code(x)))
 
-    def rule(c, acc):
+    def rule(c, acc, rotation=None):
         dx = torch.empty_like(x)
         dgamma = _grad_target(gamma, acc[1])
         if dgamma is None:
             dgamma = torch.empty_like(gamma)
         nbytes = N.lib().emi_rmsnorm_bwd_workspace_bytes(rows, D)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        if rotation is not None:                     # c is the cotangent of rope(y): rotated back on its way in
+            table, S, d = rotation
+            N.check(N.lib().emi_rmsnorm_bwd_rope(_stream(), _p(x), _p(gamma), _p(c), _p(acc[0]), _p(dx), _p(dgamma), _p(table),
+                                                 _p(ws), nbytes, rows, D, S, d, eps, _code(x)))
+            return dx, _accumulate(acc[1], dgamma)
         N.check(N.lib().emi_rmsnorm_bwd(_stream(), _p(x), _p(gamma), _p(c), _p(acc[0]), _p(dx), _p(dgamma), _p(ws),
                                         nbytes, rows, D, eps, _code(x)))
         return dx, _accumulate(acc[1], dgamma)
 
+    rule._emi_rotated = D % 8 == 0 and D <= 8192 and rows <= 0x7fffffff      # takes a rotation
     Tape.record((x, gamma), y, rule)
     tans = _tan(x, gamma)
     if tans is not None and (tans[0] is not None or tans[1] is not None):
@@ -360,6 +381,8 @@ def rope(x, n_heads, theta=10000.0, pos0=0, inverse=False):
         N.check(N.lib().emi_rope(_stream(), _p(c), _p(table), _p(g), B, S, n_heads, d, int(not inverse), _code(c)))
         return (_accumulate(acc[0], g),)
 
+    if not inverse and d % (16 // x.element_size()) == 0:
+        rule._emi_rotation = (table, S, d)
     Tape.record((x,), y, rule)
     tans = _tan(x)
     if tans is not None and tans[0] is not None:

@@ -60,6 +60,12 @@ int emi_rmsnorm_bwd(emi_stream_t stream, const void* x, const void* gamma, const
                     const void* dx_add, void* dx, void* dgamma, void* workspace,
                     size_t workspace_bytes, int64_t rows, int64_t dim, float eps, int dtype);
 
+/* The adjoint of rope(rmsnorm(x)): emi_rmsnorm_bwd on dy rotated back by the angles of emi_rope_table (position = row %
+ * seq, heads of head_dim), in one pass over dy.  dim a multiple of 8 up to 8192, whole heads of whole 16-byte pieces. */
+int emi_rmsnorm_bwd_rope(emi_stream_t stream, const void* x, const void* gamma, const void* dy, const void* dx_add,
+                         void* dx, void* dgamma, const float* rope_table, void* workspace, size_t workspace_bytes,
+                         int64_t rows, int64_t dim, int64_t seq, int64_t head_dim, float eps, int dtype);
+
 /* emi_rmsnorm_bwd without a workspace argument, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid it).  No counterpart in the reference.  The dgamma
  * partial rows go to an array of EMI_RMSNORM_BWD_NOALLOC_MAX_BYTES that the library holds on every device it
