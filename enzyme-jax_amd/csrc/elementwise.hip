@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "emi_device.h"
+#include "rmsnorm.h"
 
 namespace emi {
 
@@ -308,8 +309,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_generic_kernel(const T* __res
 // the last pass writes type T.
 constexpr int CS_ROWS = 512;
 template <typename TO>
-__global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ partial, int nparts, int64_t dim,
-                                                      TO* __restrict__ out) {
+__device__ __forceinline__ void colsum_block(const float* __restrict__ partial, int nparts, int64_t dim, TO* __restrict__ out) {
   __shared__ float red[64][64 + 4];
   const int cq = threadIdx.x & 15, rl = threadIdx.x >> 4;
   const int64_t col = (int64_t)blockIdx.x * 64 + cq * 4;
@@ -351,6 +351,18 @@ __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ 
       out[(int64_t)blockIdx.y * dim + c] = from_f32<TO>(t);
     }
   }
+}
+
+template <typename TO>
+__global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ partial, int nparts, int64_t dim,
+                                                      TO* __restrict__ out) {
+  colsum_block<TO>(partial, nparts, dim, out);
+}
+
+// Those of several adjoints (grid.z) as one launch: a small model has two a layer, and each took 3 us of launch.
+template <typename TO>
+__global__ __launch_bounds__(1024) void colsums_kernel(Colsums c, int nparts, int64_t dim) {
+  colsum_block<TO>(c.part[blockIdx.z], nparts, dim, static_cast<TO*>(c.out[blockIdx.z]));
 }
 
 // ---------------------------------------------------------------------------
@@ -667,10 +679,10 @@ static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, 
   return EMI_OK;
 }
 
+// dx, and the partial rows of dgamma in `ws`.
 template <typename T>
-static int rmsnorm_bwd_launch(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add,
-                              void* dx, void* dgamma, void* ws, int64_t rows, int64_t dim, float eps, const float* table = nullptr,
-                              int seq = 1, int head_dim = 2) {
+static int rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, void* ws,
+                            int64_t rows, int64_t dim, float eps, const float* table, int seq, int head_dim) {
   const float2* tp = reinterpret_cast<const float2*>(table);
   const T* xp = static_cast<const T*>(x);
   const T* gp = static_cast<const T*>(gamma);
@@ -702,6 +714,15 @@ static int rmsnorm_bwd_launch(hipStream_t st, const void* x, const void* gamma, 
 #undef EMI_RMS_BWD_R
   }
   EMI_CHECK_LAUNCH("emi_rmsnorm_bwd");
+  return EMI_OK;
+}
+
+template <typename T>
+static int rmsnorm_bwd_launch(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, void* dgamma,
+                              void* ws, int64_t rows, int64_t dim, float eps, const float* table = nullptr, int seq = 1, int head_dim = 2) {
+  if (const int rc = rmsnorm_bwd_rows<T>(st, x, gamma, dy, dx_add, dx, ws, rows, dim, eps, table, seq, head_dim)) return rc;
+  const int64_t nparts = rmsnorm_partial_rows(rows, dim);
+  float* part = static_cast<float*>(ws);
   // [nparts, dim] -> [ceil(nparts/CS_ROWS), dim] -> ... -> dgamma
   float* cur = part;
   float* nxt = part + nparts * dim;
@@ -718,6 +739,32 @@ static int rmsnorm_bwd_launch(hipStream_t st, const void* x, const void* gamma, 
   hipLaunchKernelGGL(colsum_kernel<T>, dim3(blocks_for(dim, 64), 1), dim3(1024), 0, st, cur, (int)n, dim,
                      static_cast<T*>(dgamma));
   EMI_CHECK_LAUNCH("emi_rmsnorm_bwd(colsum)");
+  return EMI_OK;
+}
+
+int64_t rmsnorm_partial_rows(int64_t rows, int64_t dim) {
+  int tpr, nch;
+  int64_t grid, nparts;
+  rms_bwd_shape(rows, dim, &tpr, &nch, &grid, &nparts);
+  return nparts;
+}
+bool rmsnorm_one_pass(int64_t dim) { return dim % 8 == 0 && dim <= 8192; }
+
+int launch_rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, float* part,
+                            int64_t rows, int64_t dim, float eps, int dtype) {
+  EMI_REQUIRE(aligned16(x) && aligned16(gamma) && aligned16(dy) && aligned16(dx) && aligned16(dx_add) && aligned16(part),
+              "emi_rmsnorm_bwd: buffers must be 16-byte aligned");
+  return dtype == EMI_F32 ? rmsnorm_bwd_rows<float>(st, x, gamma, dy, dx_add, dx, part, rows, dim, eps, nullptr, 1, 2)
+                          : rmsnorm_bwd_rows<bf16>(st, x, gamma, dy, dx_add, dx, part, rows, dim, eps, nullptr, 1, 2);
+}
+
+int launch_colsums(hipStream_t st, const Colsums& c, int count, int64_t part_rows, int64_t dim, int dtype) {
+  if (count <= 0) return EMI_OK;
+  if (count > kMaxColsums || part_rows > CS_ROWS) return emi_fail(EMI_INTERNAL, "column sums: %d of %lld rows", count, (long long)part_rows);
+  const dim3 grid(blocks_for(dim, 64), 1, (unsigned)count);
+  if (dtype == EMI_F32) hipLaunchKernelGGL(colsums_kernel<float>, grid, dim3(1024), 0, st, c, (int)part_rows, dim);
+  else hipLaunchKernelGGL(colsums_kernel<bf16>, grid, dim3(1024), 0, st, c, (int)part_rows, dim);
+  EMI_CHECK_LAUNCH("emi_rmsnorm_bwd(colsums)");
   return EMI_OK;
 }
 

@@ -6,10 +6,12 @@
 // than a Python operator costs: the dim-288 model on 256 tokens spent 2.6 ms on the host for 1.25 ms of kernels.
 // In reverse the weight gradients dW = dY^T X feed nothing else, so they wait until `group` layers are done and run grouped
 // by shape (q, k, v, o; w1, w3; w2), which fills the chip where one layer's would not; a group of one runs them in place.
+// So do the column sums of the RMSNorm adjoints (dim-288 model, six layers: 11 launches of 3 us less, 858 -> 830 us).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "../../include/emi.h"
+#include "rmsnorm.h"
 
 extern "C" int emi_fail(int code, const char* fmt, ...);
 
@@ -103,9 +105,14 @@ size_t forward_scratch(const Dims& d) {
                emi_gemm_workspace_bytes(T, d.D, d.H, 0, 1, d.dtype)});
 }
 
+// dgamma's partial rows wait until the group is done and are summed by one launch
+bool norms_wait(const Dims& d) { return emi::rmsnorm_one_pass(d.D); }
+size_t norm_part_bytes(const Dims& d) { return (size_t)emi::rmsnorm_partial_rows(d.T(), d.D) * d.D * sizeof(float); }
+
 struct ReverseScratch {
   void *dxb, *dg, *ws;
   size_t ws_bytes;
+  float* parts;                                           // partial rows of dgamma, two adjoints a layer of the group
 };
 ReverseScratch carve_reverse(void* base, const Dims& d, int group, int transposed, size_t* bytes) {
   Carve c{static_cast<uint8_t*>(base), 0};
@@ -127,6 +134,7 @@ ReverseScratch carve_reverse(void* base, const Dims& d, int group, int transpose
   for (int i = 1; i <= m1; i++) need = most({need, emi_gemm_grouped_workspace_bytes(i, d.D, d.H, T, 1, 0, 0, d.dtype)});
   s.ws_bytes = need;
   s.ws = c.take(need);
+  s.parts = static_cast<float*>(c.take(norms_wait(d) ? 2 * (size_t)group * norm_part_bytes(d) : 0));
   if (bytes != nullptr) *bytes = c.at;
   return s;
 }
@@ -185,6 +193,26 @@ int wait(emi_stream_t st, Pending& p, const void* dy, const void* x, void* dw, i
   p.b[p.n] = x;
   p.c[p.n++] = dw;
   return EMI_OK;
+}
+
+// RMSNorm adjoints whose column sums wait.
+struct Norms {
+  emi::Colsums c;
+  int n = 0;
+};
+int flush(emi_stream_t st, Norms& p, const Dims& d) {
+  const int n = p.n;
+  p.n = 0;
+  return emi::launch_colsums(static_cast<hipStream_t>(st), p.c, n, emi::rmsnorm_partial_rows(d.T(), d.D), d.D, d.dtype);
+}
+int norm_adjoint(emi_stream_t st, Norms& p, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, void* dgamma,
+                 const ReverseScratch& r, const Dims& d) {
+  if (!norms_wait(d)) return emi_rmsnorm_bwd(st, x, gamma, dy, dx_add, dx, dgamma, r.ws, r.ws_bytes, d.T(), d.D, d.eps, d.dtype);
+  if (p.n == emi::kMaxColsums) EMI_TRY(flush(st, p, d));
+  float* part_rows = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(r.parts) + p.n * norm_part_bytes(d));
+  p.c.part[p.n] = part_rows;
+  p.c.out[p.n++] = dgamma;
+  return emi::launch_rmsnorm_bwd_rows(static_cast<hipStream_t>(st), x, gamma, dy, dx_add, dx, part_rows, d.T(), d.D, d.eps, d.dtype);
 }
 
 int check_layers(const char* name, const Dims& d, const void* const* w, std::initializer_list<const void*> ptrs) {
@@ -285,6 +313,7 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
                           : emi_strided_copy(stream, weights[i], transposed[i], 3, out, ss, 0, ds, 0, (int)d.elt()));
     }
   Pending sq, up, down;                                   // [D, D], [H, D], [D, H]
+  Norms norms;
   const int64_t hd = d.hd();
   for (int64_t l = layers - 1; l >= 0; l--) {
     const void *w[kWeights], *b[kWeights];
@@ -314,7 +343,7 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
       void* out[1] = {r.dxb};
       EMI_TRY(emi_gemm_grouped(stream, 2, a2, b2, nullptr, out, r.ws, r.ws_bytes, T, D, H, H, tb ? H : D, D, D, 0, tb, 1, dtype));
     }
-    EMI_TRY(emi_rmsnorm_bwd(stream, s.x1, w[kFfn], r.dxb, dy, c.dx1, g[kFfn], r.ws, r.ws_bytes, T, D, d.eps, dtype));
+    EMI_TRY(norm_adjoint(stream, norms, s.x1, w[kFfn], r.dxb, dy, c.dx1, g[kFfn], r, d));
     EMI_TRY(emi_gemm_ws(stream, c.dx1, b[kO], nullptr, r.dxb, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, dtype));
     if (d.rope_attention()) {
       EMI_TRY(emi_attn_bwd_rope(stream, s.q, s.k, s.v, s.att, s.lse, r.dxb, c.dq, c.dk, c.dv, rope_table, r.ws, r.ws_bytes, d.B, d.heads, d.S, hd,
@@ -331,7 +360,7 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     }
     // the first layer's cotangent leaves; a caller's accumulated one is added by its own launch
     void* dx_l = l == 0 ? dx : c.dx;
-    EMI_TRY(emi_rmsnorm_bwd(stream, x_l, w[kAtt], r.dxb, c.dx1, dx_l, g[kAtt], r.ws, r.ws_bytes, T, D, d.eps, dtype));
+    EMI_TRY(norm_adjoint(stream, norms, x_l, w[kAtt], r.dxb, c.dx1, dx_l, g[kAtt], r, d));
     if (l == 0 && dx_add != nullptr) EMI_TRY(emi_add(stream, dx, dx_add, dx, T * D, dtype));
     EMI_TRY(wait(stream, sq, c.dq, s.xb1, g[kQ], D, D, T, r, dtype));
     EMI_TRY(wait(stream, sq, c.dk, s.xb1, g[kK], D, D, T, r, dtype));
@@ -342,6 +371,7 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     if (ends_group) {
       EMI_TRY(flush(stream, sq, D, D, T, r, dtype));
       EMI_TRY(flush(stream, up, H, D, T, r, dtype));
+      EMI_TRY(flush(stream, norms, d));
     }
     dy = dx_l;
   }
