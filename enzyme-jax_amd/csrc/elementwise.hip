@@ -39,9 +39,25 @@ template <int TPR> __device__ __forceinline__ void row_reduce2(float& a, float& 
   }
 }
 
-template <typename T, int TPR, int NCH>
+// N consecutive elements of the sum of `count` fp32 planes, `plane` elements apart, in plane order.
+template <int N> __device__ __forceinline__ void add_planes(const float* p, int64_t plane, int count, float (&v)[N]) {
+#pragma unroll
+  for (int e = 0; e < N; e++) v[e] = 0.f;
+#pragma unroll 4
+  for (int z = 0; z < count; z++)
+#pragma unroll
+    for (int q = 0; q < N / 4; q++) {
+      const float4 t = *reinterpret_cast<const float4*>(p + z * plane + 4 * q);
+      v[4 * q] += t.x; v[4 * q + 1] += t.y; v[4 * q + 2] += t.z; v[4 * q + 3] += t.w;
+    }
+}
+
+// PLANES: x is the result of a product that was split over K, still in planes, and its residual; it is added up here as the
+// reduction of its own would (3 to 4 us a launch), stored to x_out and normalised.
+template <typename T, int TPR, int NCH, bool PLANES>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
-                                                          T* __restrict__ y, int64_t rows, int dim, float eps) {
+                                                          T* __restrict__ y, int64_t rows, int dim, float eps,
+                                                          const float* __restrict__ planes, int count, T* x_out) {
   // NCH groups of 8 elements per thread, held as 16-byte pieces (8 bf16 or 4 floats): consecutive lanes cover
   // consecutive 16 bytes, the access shape the streaming loads and stores want.
   constexpr int RPB = 256 / TPR, N = Chunk<T>::N, NC = NCH * 8 / N;
@@ -58,7 +74,18 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ 
   for (int j = 0; j < NC; j++) {
     const int c = tir + j * TPR;
     if (active && c < nchunk) {
-      Chunk<T>::load(xr + c * N, v[j]);
+      if constexpr (PLANES) {
+        float r[N];
+        add_planes<N>(planes + row * dim + c * N, rows * (int64_t)dim, count, v[j]);
+        ChunkCached<T>::load(xr + c * N, r);
+#pragma unroll
+        for (int e = 0; e < N; e++) v[j][e] += r[e];
+        const typename Chunk<T>::Raw raw = pack_raw(v[j]);
+        Chunk<T>::unpack(raw, v[j]);
+        ChunkCached<T>::store(x_out + row * dim + c * N, v[j]);
+      } else {
+        Chunk<T>::load(xr + c * N, v[j]);
+      }
 #pragma unroll
       for (int e = 0; e < N; e++) ss += v[j][e] * v[j][e];
     }
@@ -99,14 +126,17 @@ template <int TPR, int NV> __device__ __forceinline__ void row_reduce_n(float (&
 // Adjoint.  Blocks walk rows with a grid stride, NR rows per step, and keep this
 // thread's share of dgamma in registers; partial[blockIdx*RPB + rib][dim] is reduced
 // by colsum_kernel.  dx = [dx_add +] r*g - x * r^3 * mean(g*x), g = dy*gamma.
-// ROPE: dy is the cotangent of the rotated result; each piece is rotated back (and rounded to T, as a pass of its own over
+// kNormPlanes: dy points to `count` fp32 planes of a product that was split over K, added up here as its reduction would.
+// kNormRope: dy is the cotangent of the rotated result; each piece is rotated back (and rounded to T, as a pass of its own over
 // dy would leave it) on its way in, by the angles of the row's position row % seq.  16 x 2048 rows of 4096 fp32,
 // us: rotation 180 and this 269 -> 271: the angles come from the L1, and what bounds both is x, dy in and dx out (5.9 TB/s).
-template <typename T, int TPR, int NCH, int NR, bool ROPE>
+enum { kNormPlain, kNormRope, kNormPlanes };
+template <typename T, int TPR, int NCH, int NR, int MODE>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                           const T* __restrict__ dy, const T* dx_add, T* dx,
                                                           float* __restrict__ partial, int64_t rows, int dim,
-                                                          float eps, const float2* __restrict__ table, int seq, int head_dim) {
+                                                          float eps, const float2* __restrict__ table, int seq, int head_dim, int count) {
+  constexpr bool ROPE = MODE == kNormRope;
   // NCH groups of 8 elements per thread, held as 16-byte pieces (8 bf16 or 4 floats) so that consecutive lanes cover
   // consecutive 16 bytes (the access shape of the streaming loads and stores)
   constexpr int RPB = 256 / TPR, N = Chunk<T>::N, NC = NCH * 8 / N;
@@ -144,7 +174,13 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
             for (int q = 0; q < N / 4; q++) tn[u][j][q] = t[q];
           }
           xn[u][j] = Chunk<T>::load_raw(x + row * dim + c * N);
-          gn[u][j] = Chunk<T>::load_raw(dy + row * dim + c * N);
+          if constexpr (MODE == kNormPlanes) {
+            float v[N];
+            add_planes<N>(reinterpret_cast<const float*>(dy) + row * dim + c * N, rows * (int64_t)dim, count, v);
+            gn[u][j] = pack_raw(v);
+          } else {
+            gn[u][j] = Chunk<T>::load_raw(dy + row * dim + c * N);
+          }
         } else {
           if constexpr (ROPE)
 #pragma unroll
@@ -655,7 +691,7 @@ static inline void rms_bwd_shape(int64_t rows, int64_t dim, int* tpr, int* nch, 
 
 template <typename T>
 static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, void* y, int64_t rows, int64_t dim,
-                              float eps) {
+                              float eps, const float* planes = nullptr, int count = 0, void* x_out = nullptr) {
   const T* xp = static_cast<const T*>(x);
   const T* gp = static_cast<const T*>(gamma);
   T* yp = static_cast<T*>(y);
@@ -666,14 +702,21 @@ static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, 
     hipLaunchKernelGGL(rmsnorm_fwd_generic_kernel<T>, dim3((unsigned)rows), dim3(256), 0, st, xp, gp, yp, rows, dim, eps);
   } else {
     const unsigned g = blocks_for(rows, 256 / tpr);
-#define EMI_RMS_FWD(TPR, NCH) \
-  hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, TPR, NCH>), dim3(g), dim3(256), 0, st, xp, gp, yp, rows, (int)dim, eps)
+#define EMI_RMS_FWD_P(TPR, NCH, PLANES)                                                                                                  \
+  hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, TPR, NCH, PLANES>), dim3(g), dim3(256), 0, st, xp, gp, yp, rows, (int)dim, eps, planes, count, \
+                     static_cast<T*>(x_out))
+#define EMI_RMS_FWD(TPR, NCH)                           \
+  do {                                                  \
+    if (count > 0) EMI_RMS_FWD_P(TPR, NCH, true);       \
+    else EMI_RMS_FWD_P(TPR, NCH, false);                \
+  } while (0)
     if (tpr == 64 && nch == 1) EMI_RMS_FWD(64, 1);
     else if (tpr == 64) EMI_RMS_FWD(64, 2);
     else if (nch == 1) EMI_RMS_FWD(256, 1);
     else if (nch == 2) EMI_RMS_FWD(256, 2);
     else EMI_RMS_FWD(256, 4);
 #undef EMI_RMS_FWD
+#undef EMI_RMS_FWD_P
   }
   EMI_CHECK_LAUNCH("emi_rmsnorm_fwd");
   return EMI_OK;
@@ -682,7 +725,7 @@ static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, 
 // dx, and the partial rows of dgamma in `ws`.
 template <typename T>
 static int rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, void* ws,
-                            int64_t rows, int64_t dim, float eps, const float* table, int seq, int head_dim) {
+                            int64_t rows, int64_t dim, float eps, const float* table, int seq, int head_dim, int planes = 0) {
   const float2* tp = reinterpret_cast<const float2*>(table);
   const T* xp = static_cast<const T*>(x);
   const T* gp = static_cast<const T*>(gamma);
@@ -697,13 +740,14 @@ static int rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, co
     hipLaunchKernelGGL(rmsnorm_bwd_generic_kernel<T>, dim3((unsigned)grid), dim3(256), 0, st, xp, gp, dyp, ap, dxp, part,
                        rows, dim, eps);
   } else {
-#define EMI_RMS_BWD_R(TPR, NCH, ROPE)                                                                                                         \
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, TPR, NCH, (sizeof(T) == 2 ? 2 : 1), ROPE>), dim3((unsigned)grid), dim3(256), 0, st, xp, gp, dyp, \
-                     ap, dxp, part, rows, (int)dim, eps, tp, seq, head_dim)
-#define EMI_RMS_BWD(TPR, NCH)                          \
-  do {                                                 \
-    if (tp != nullptr) EMI_RMS_BWD_R(TPR, NCH, true);  \
-    else EMI_RMS_BWD_R(TPR, NCH, false);               \
+#define EMI_RMS_BWD_M(TPR, NCH, MODE)                                                                                                         \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, TPR, NCH, (sizeof(T) == 2 ? 2 : 1), MODE>), dim3((unsigned)grid), dim3(256), 0, st, xp, gp, dyp, \
+                     ap, dxp, part, rows, (int)dim, eps, tp, seq, head_dim, planes)
+#define EMI_RMS_BWD(TPR, NCH)                                    \
+  do {                                                           \
+    if (tp != nullptr) EMI_RMS_BWD_M(TPR, NCH, kNormRope);       \
+    else if (planes > 0) EMI_RMS_BWD_M(TPR, NCH, kNormPlanes);   \
+    else EMI_RMS_BWD_M(TPR, NCH, kNormPlain);                    \
   } while (0)
     if (tpr == 64 && nch == 1) EMI_RMS_BWD(64, 1);
     else if (tpr == 64) EMI_RMS_BWD(64, 2);
@@ -711,7 +755,7 @@ static int rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, co
     else if (nch == 2) EMI_RMS_BWD(256, 2);
     else EMI_RMS_BWD(256, 4);
 #undef EMI_RMS_BWD
-#undef EMI_RMS_BWD_R
+#undef EMI_RMS_BWD_M
   }
   EMI_CHECK_LAUNCH("emi_rmsnorm_bwd");
   return EMI_OK;
@@ -750,12 +794,22 @@ int64_t rmsnorm_partial_rows(int64_t rows, int64_t dim) {
 }
 bool rmsnorm_one_pass(int64_t dim) { return dim % 8 == 0 && dim <= 8192; }
 
-int launch_rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, float* part,
-                            int64_t rows, int64_t dim, float eps, int dtype) {
+int launch_rmsnorm_bwd_rows(hipStream_t st, const void* x, const void* gamma, const void* dy, int dy_planes, const void* dx_add, void* dx,
+                            float* part, int64_t rows, int64_t dim, float eps, int dtype) {
   EMI_REQUIRE(aligned16(x) && aligned16(gamma) && aligned16(dy) && aligned16(dx) && aligned16(dx_add) && aligned16(part),
               "emi_rmsnorm_bwd: buffers must be 16-byte aligned");
-  return dtype == EMI_F32 ? rmsnorm_bwd_rows<float>(st, x, gamma, dy, dx_add, dx, part, rows, dim, eps, nullptr, 1, 2)
-                          : rmsnorm_bwd_rows<bf16>(st, x, gamma, dy, dx_add, dx, part, rows, dim, eps, nullptr, 1, 2);
+  if (dy_planes > 0 && !rmsnorm_one_pass(dim)) return emi_fail(EMI_INTERNAL, "emi_rmsnorm_bwd: planes of %lld columns", (long long)dim);
+  return dtype == EMI_F32 ? rmsnorm_bwd_rows<float>(st, x, gamma, dy, dx_add, dx, part, rows, dim, eps, nullptr, 1, 2, dy_planes)
+                          : rmsnorm_bwd_rows<bf16>(st, x, gamma, dy, dx_add, dx, part, rows, dim, eps, nullptr, 1, 2, dy_planes);
+}
+
+int launch_rmsnorm_fwd_planes(hipStream_t st, const float* planes, int count, const void* r, const void* gamma, void* x, void* y,
+                              int64_t rows, int64_t dim, float eps, int dtype) {
+  EMI_REQUIRE(aligned16(planes) && aligned16(r) && aligned16(gamma) && aligned16(x) && aligned16(y),
+              "emi_rmsnorm_fwd: buffers must be 16-byte aligned");
+  if (count < 1 || !rmsnorm_one_pass(dim)) return emi_fail(EMI_INTERNAL, "emi_rmsnorm_fwd: %d planes of %lld columns", count, (long long)dim);
+  return dtype == EMI_F32 ? rmsnorm_fwd_launch<float>(st, r, gamma, y, rows, dim, eps, planes, count, x)
+                          : rmsnorm_fwd_launch<bf16>(st, r, gamma, y, rows, dim, eps, planes, count, x);
 }
 
 int launch_colsums(hipStream_t st, const Colsums& c, int count, int64_t part_rows, int64_t dim, int dtype) {

@@ -1771,7 +1771,7 @@ static int pingpong_splits(int64_t M, int64_t N, int64_t K, bool k_contiguous) {
 
 static int launch_bf16_pingpong_splitk(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K,
                                        int lda, int ldb, int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, float* part,
-                                       int splits) {
+                                       int splits, int* planes) {
   auto kern = gemm_bf16_pingpong_kernel<false, false, false, 5>;
   constexpr int smem = 2 * 65536;
   static bool configured = false;   // idempotent; a race only repeats the call
@@ -1787,6 +1787,10 @@ static int launch_bf16_pingpong_splitk(hipStream_t st, const void* A, const void
                      static_cast<const uint16_t*>(nullptr), static_cast<uint16_t*>(nullptr), M, N, K, lda, ldb, ldr, ldc, a_bytes,
                      b_bytes, 0, NoGroup{}, SplitEpi{part, kps});
   EMI_CHECK_LAUNCH("emi_gemm(split-K, 256-tiles)");
+  if (planes != nullptr) {
+    *planes = nz;
+    return EMI_OK;
+  }
   launch_splitk_reduce<bf16>(st, part, R, C, M, N, nz, (int64_t)ldr, (int64_t)ldc);
   EMI_CHECK_LAUNCH("emi_gemm(split-K reduce)");
   return EMI_OK;
@@ -1824,21 +1828,21 @@ static int launch_bf16_kmajor(hipStream_t st, const void* A, const void* B, cons
 // A k-contiguous: the ping-pong kernel or one of the shapes of gemm_bf16_pipe.hip, with or without splits of K.
 static int launch_bf16_kcontig(hipStream_t st, const void* A, const void* B, const void* R, void* C, int M, int N, int K, int lda, int ldb,
                                int ldr, int ldc, uint32_t a_bytes, uint32_t b_bytes, int trans_b, void* workspace,
-                               size_t workspace_bytes) {
+                               size_t workspace_bytes, int* planes) {
   const int pps = pingpong_splits(M, N, K, trans_b);
   if (pps > 1 && workspace_holds(workspace, workspace_bytes, pps, M, N))
-    return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, static_cast<float*>(workspace), pps);
+    return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, static_cast<float*>(workspace), pps, planes);
   const Bf16Plan plan = bf16_plan(M, N, K, 1, 0, trans_b, splits_held(workspace, workspace_bytes, M, N));
   float* part = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
   if (plan.shape == 0) {
     if (part != nullptr)
-      return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, part, plan.splits);
+      return launch_bf16_pingpong_splitk(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes, part, plan.splits, planes);
     return trans_b ? launch_bf16_pingpong<false, false>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes)
                    : launch_bf16_pingpong<false, true>(st, A, B, R, C, M, N, K, lda, ldb, ldr, ldc, a_bytes, b_bytes);
   }
   const int vec_ok = (reinterpret_cast<uintptr_t>(C) & 15) == 0 && ldc % 8 == 0 &&
                      (R == nullptr || ((reinterpret_cast<uintptr_t>(R) & 15) == 0 && ldr % 8 == 0));
-  return launch_bf16_pipe(st, plan, 1, &A, &B, &R, &C, part, M, N, K, lda, ldb, ldr, ldc, vec_ok, trans_b, 0);
+  return launch_bf16_pipe(st, plan, 1, &A, &B, &R, &C, part, M, N, K, lda, ldb, ldr, ldc, vec_ok, trans_b, 0, planes);
 }
 
 template <typename T>
@@ -1943,7 +1947,7 @@ int launch_f32_splitk_reduce(hipStream_t st, const float* part, const float* R, 
 // gemm_f32.hip
 int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
                     void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
-                    int64_t ldc, int trans_a, int trans_b, int sum);
+                    int64_t ldc, int trans_a, int trans_b, int sum, int* planes);
 size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a);
 
 // gemm_skinny.hip
@@ -1983,6 +1987,14 @@ extern "C" int emi_gemm(emi_stream_t stream, const void* A, const void* B, const
 extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, const void* R, void* C, void* workspace,
                            size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
                            int64_t ldc, int trans_a, int trans_b, int dtype) {
+  return gemm_run(static_cast<hipStream_t>(stream), A, B, R, C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b,
+                  dtype, nullptr);
+}
+
+int emi::gemm_run(hipStream_t st, const void* A, const void* B, const void* R, void* C, void* workspace, size_t workspace_bytes, int64_t M,
+                  int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr, int64_t ldc, int trans_a, int trans_b, int dtype,
+                  int* planes) {
+  if (planes != nullptr) *planes = 0;
   EMI_REQUIRE(M >= 0 && N >= 0 && K >= 0, "emi_gemm: negative dimension M=%lld N=%lld K=%lld", (long long)M, (long long)N,
               (long long)K);
   EMI_REQUIRE(M <= 0x7fffffff && N <= 0x7fffffff && K <= 0x7fffffff, "emi_gemm: dimension exceeds 2^31-1");
@@ -1992,7 +2004,6 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
   EMI_REQUIRE(lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && ldc >= N && (R == nullptr || ldr >= N),
               "emi_gemm: leading dimension smaller than the row length (lda=%lld ldb=%lld ldr=%lld ldc=%lld)",
               (long long)lda, (long long)ldb, (long long)ldr, (long long)ldc);
-  hipStream_t st = static_cast<hipStream_t>(stream);
   if (K > 0 && (R == nullptr || ldr >= N)) {
     // single-token forms (mat-vec and its adjoints): weight-bandwidth-bound kernels
     const int rc = launch_skinny(st, A, B, R, C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, dtype);
@@ -2013,7 +2024,7 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
       const int m = (int)M, n = (int)N, k = (int)K;
       const uint32_t ab = (uint32_t)a_bytes, bb = (uint32_t)b_bytes;
       if (!trans_a)
-        return launch_bf16_kcontig(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, trans_b, workspace, workspace_bytes);
+        return launch_bf16_kcontig(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, trans_b, workspace, workspace_bytes, planes);
       if (!trans_b)
         return launch_bf16_kmajor<true>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
       return launch_bf16_kmajor<false>(st, A, B, R, C, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
@@ -2021,7 +2032,7 @@ extern "C" int emi_gemm_ws(emi_stream_t stream, const void* A, const void* B, co
     return launch_generic<bf16>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
   }
   {
-    const int rc = launch_f32_gemm(st, 1, &A, &B, &R, &C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0);
+    const int rc = launch_f32_gemm(st, 1, &A, &B, &R, &C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0, planes);
     if (rc >= 0) return rc;
   }
   // rows that do not divide into 16-byte pieces, k-contiguous ones at least aligned: 32x32 tiles, K split over the block's
@@ -2139,6 +2150,14 @@ extern "C" size_t emi_gemm_grouped_workspace_bytes(int count, int64_t M, int64_t
 extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* const* A, const void* const* B, const void* const* R,
                                 void* const* C, void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
                                 int64_t lda, int64_t ldb, int64_t ldr, int64_t ldc, int trans_a, int trans_b, int sum, int dtype) {
+  return gemm_grouped_run(static_cast<hipStream_t>(stream), count, A, B, R, C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a,
+                          trans_b, sum, dtype, nullptr);
+}
+
+int emi::gemm_grouped_run(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
+                          void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
+                          int64_t ldc, int trans_a, int trans_b, int sum, int dtype, int* planes) {
+  if (planes != nullptr) *planes = 0;
   EMI_REQUIRE(count >= 1 && count <= kMaxGroup, "emi_gemm_grouped: count %d not in 1..%d", count, kMaxGroup);
   EMI_REQUIRE(A && B && C, "emi_gemm_grouped: null pointer table");
   EMI_REQUIRE(M >= 0 && N >= 0 && K >= 0 && M <= 0x7fffffff && N <= 0x7fffffff && K <= 0x7fffffff,
@@ -2148,7 +2167,6 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
   for (int i = 0; i < count; i++) EMI_REQUIRE(A[i] && B[i], "emi_gemm_grouped: null operand %d", i);
   for (int i = 0; i < nout; i++) EMI_REQUIRE(C[i], "emi_gemm_grouped: null result %d", i);
   if (M == 0 || N == 0) return EMI_OK;
-  hipStream_t st = static_cast<hipStream_t>(stream);
   bool fast = dtype == EMI_BF16 && count >= 2 && K > 0 && M > 8;
   if (fast) {
     const int64_t a_rows = trans_a ? K : M, b_rows = trans_b ? N : K;
@@ -2188,7 +2206,7 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
         const Bf16Plan plan = bf16_plan(M, N, K, count, sum ? 1 : 0, trans_b, held);
         if (!sum && faster_one_by_one(plan, bf16_plan(M, N, K, 1, 0, trans_b, held), count, 1.3)) {
           for (int i = 0; i < count; i++)
-            if (const int rc = emi_gemm_ws(stream, A[i], B[i], g.R[i], C[i], workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, 0, trans_b, dtype))
+            if (const int rc = emi_gemm_ws(st, A[i], B[i], g.R[i], C[i], workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, 0, trans_b, dtype))
               return rc;
           return EMI_OK;
         }
@@ -2196,7 +2214,7 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
           return trans_b ? launch_bf16_pingpong_grouped<false, false>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok)
                          : launch_bf16_pingpong_grouped<false, true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, vec_ok);
         return launch_bf16_pipe(st, plan, count, A, B, any_r ? R : nullptr, C, plan.splits > 1 ? static_cast<float*>(workspace) : nullptr, m,
-                                n, k, (int)lda, (int)ldb, ldr, ldc, vec_ok, trans_b, sum ? 1 : 0);
+                                n, k, (int)lda, (int)ldb, ldr, ldc, vec_ok, trans_b, sum ? 1 : 0, planes);
       }
       if (trans_a && !trans_b)
         return launch_bf16_grouped<true>(st, g, m, n, k, (int)lda, (int)ldb, (int)ldr, (int)ldc, ab, bb, workspace, workspace_bytes);
@@ -2212,7 +2230,7 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
     }
     if (!any_r || (all_r && ldr >= N)) {
       const int rc = launch_f32_gemm(st, count, A, B, any_r ? R : nullptr, C, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc,
-                                     trans_a, trans_b, sum ? 1 : 0);
+                                     trans_a, trans_b, sum ? 1 : 0, planes);
       if (rc >= 0) return rc;
       // independent products with odd rows: one grid plane each, unless one by one they would be split over K and together
       // they still leave the chip idle
@@ -2237,7 +2255,7 @@ extern "C" int emi_gemm_grouped(emi_stream_t stream, int count, const void* cons
   for (int i = 0; i < count; i++) {
     const void* r = sum ? (i == 0 ? (R ? R[0] : nullptr) : C[0]) : (R ? R[i] : nullptr);
     void* c = sum ? C[0] : C[i];
-    const int rc = emi_gemm_ws(stream, A[i], B[i], r, c, workspace, workspace_bytes, M, N, K, lda, ldb, (sum && i > 0) ? ldc : ldr, ldc,
+    const int rc = emi_gemm_ws(st, A[i], B[i], r, c, workspace, workspace_bytes, M, N, K, lda, ldb, (sum && i > 0) ? ldc : ldr, ldc,
                                trans_a, trans_b, dtype);
     if (rc != EMI_OK) return rc;
   }

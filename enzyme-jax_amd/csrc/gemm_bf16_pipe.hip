@@ -345,6 +345,7 @@ struct PipeCall {
   float* part;
   int splits;
   const PipeGroup* grp;       // nullptr: the single product of A and B
+  int* planes;                // not null: splits stay planes in `part`, *planes of them (gemm_run)
 };
 
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, bool GROUPED>
@@ -371,6 +372,10 @@ static int launch_pipe_one(hipStream_t st, const PipeCall& c) {
     hipLaunchKernelGGL(kern, dim3(tiles * outer), dim3(WM * WN * WK * 64), smem, st, c.A, c.B, c.R, c.C, c.M, c.N, c.K, c.lda, c.ldb,
                        c.ldr, c.ldc, c.vec_ok, part, sps, PipeSingle{});
   EMI_CHECK_LAUNCH("emi_gemm");
+  if (part != nullptr && c.planes != nullptr) {
+    *c.planes = nz;
+    return EMI_OK;
+  }
   if (part != nullptr) return launch_bf16_splitk_reduce(st, part, c.R, c.C, c.M, c.N, nz, c.ldr, c.ldc);
   return EMI_OK;
 }
@@ -426,7 +431,7 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
 // (plan.shape >= 1; the caller has checked 16-byte rows).  vec_ok: 16-byte rows of C and R.
 int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void* const* A, const void* const* B, const void* const* R,
                      void* const* C, float* part, int M, int N, int K, int lda, int ldb, int64_t ldr, int64_t ldc, int vec_ok, int trans_b,
-                     int sum) {
+                     int sum, int* planes) {
   PipeGroup g{};
   for (int i = 0; i < count; i++) {
     g.A[i] = static_cast<const uint16_t*>(A[i]);
@@ -439,7 +444,7 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
   g.count = count;
   g.sum = sum;
   const PipeCall c{g.A[0], g.B[0], g.R[0], g.C[0], M, N, K, lda, ldb, ldr, ldc, vec_ok, part, part != nullptr ? plan.splits : 1,
-                   count > 1 ? &g : nullptr};
+                   count > 1 ? &g : nullptr, planes};
   switch (plan.shape) {
     case 1: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 2>(st, c, trans_b);
     case 2: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 3>(st, c, trans_b);

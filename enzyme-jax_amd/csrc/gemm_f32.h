@@ -25,6 +25,7 @@ struct F32Call {
   float* part;
   int splits;
   const F32Group* grp;       // nullptr: the single product of A and B
+  int* planes;               // not null: splits stay planes in `part`, *planes of them (gemm_run)
 };
 
 // gemm.hip: adds `splits` planes [M, N] (+ R) into C in plane order

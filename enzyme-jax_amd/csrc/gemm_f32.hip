@@ -305,6 +305,10 @@ static int launch_f32_one(hipStream_t st, const F32Call& c) {
     hipLaunchKernelGGL(kern, dim3(tiles * outer), dim3(WM * WN * WK * 64), smem, st, c.A, c.B, c.R, c.C, c.M, c.N, c.K, c.lda, c.ldb,
                        c.ldr, c.ldc, part, sps, F32Single{});
   EMI_CHECK_LAUNCH("emi_gemm(fp32)");
+  if (part != nullptr && c.planes != nullptr) {
+    *c.planes = nz;
+    return EMI_OK;
+  }
   if (part != nullptr) return launch_f32_splitk_reduce(st, part, c.R, c.C, c.M, c.N, nz, c.ldr, c.ldc);
   return EMI_OK;
 }
@@ -399,7 +403,7 @@ size_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K, int count, int 
 // operands that the kernels' 16-byte pieces do not fit (the caller has other kernels for those).
 int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
                     void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
-                    int64_t ldc, int trans_a, int trans_b, int sum) {
+                    int64_t ldc, int trans_a, int trans_b, int sum, int* planes) {
   // pieces are four elements along the stored rows; a stage's panel of an operand is addressed with 31 bits
   if (K <= 0 || count > kMaxF32Group || lda % 4 || ldb % 4 || (trans_a ? M : K) % 4 || (trans_b ? K : N) % 4 ||
       128 * lda + K >= 0x1fffffff || 128 * ldb + K >= 0x1fffffff)
@@ -421,13 +425,13 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   if (count > 1 && !sum && faster_one_by_one(p, f32_plan(M, N, K, 1, 0, trans_a, held), count, 1.08)) {
     for (int i = 0; i < count; i++) {
       const void* r = R != nullptr ? R[i] : nullptr;
-      if (const int rc = launch_f32_gemm(st, 1, A + i, B + i, &r, C + i, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0))
+      if (const int rc = launch_f32_gemm(st, 1, A + i, B + i, &r, C + i, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0, nullptr))
         return rc;
     }
     return EMI_OK;
   }
   const F32Call c{g.A[0], g.B[0], g.R[0], g.C[0], (int)M, (int)N, (int)K, (int)lda, (int)ldb, ldr, ldc, static_cast<float*>(workspace),
-                  p.splits, count > 1 ? &g : nullptr};
+                  p.splits, count > 1 ? &g : nullptr, planes};
   // (the split kernels address a tile of the result with 31 bits too)
   const bool wide = 128 * ldc >= 0x1fffffff || 128 * N >= 0x1fffffff || (R != nullptr && 128 * ldr >= 0x1fffffff);
   const int shape = f32_shape(p, M, N, K, count, sum, trans_a);

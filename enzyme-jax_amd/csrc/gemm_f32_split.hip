@@ -426,6 +426,10 @@ static int launch_split_one(hipStream_t st, const F32Call& c) {
     hipLaunchKernelGGL(kern, dim3(tiles * outer), dim3(WM * WN * WK * 64), smem, st, c.A, c.B, c.R, c.C, c.M, c.N, c.K, c.lda, c.ldb, c.ldr,
                        c.ldc, part, sps, F32Single{});
   EMI_CHECK_LAUNCH("emi_gemm(fp32)");
+  if (part != nullptr && c.planes != nullptr) {
+    *c.planes = nz;
+    return EMI_OK;
+  }
   if (part != nullptr) return launch_f32_splitk_reduce(st, part, c.R, c.C, c.M, c.N, nz, c.ldr, c.ldc);
   return EMI_OK;
 }

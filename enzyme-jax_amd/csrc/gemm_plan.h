@@ -41,6 +41,15 @@ template <typename Plan> inline bool faster_one_by_one(const Plan& group, const 
 
 int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void* const* A, const void* const* B, const void* const* R,
                      void* const* C, float* part, int M, int N, int K, int lda, int ldb, int64_t ldr, int64_t ldc, int vec_ok, int trans_b,
-                     int sum);
+                     int sum, int* planes);
+
+// emi_gemm_ws and emi_gemm_grouped for a caller that adds the planes of a product split over K itself: with `planes` not null
+// such a product leaves *planes fp32 planes [M, N] in the workspace, to be added in order and then to R, and C unwritten;
+// *planes is 0 where C is complete.
+int gemm_run(hipStream_t st, const void* A, const void* B, const void* R, void* C, void* workspace, size_t workspace_bytes, int64_t M,
+             int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr, int64_t ldc, int trans_a, int trans_b, int dtype, int* planes);
+int gemm_grouped_run(hipStream_t st, int count, const void* const* A, const void* const* B, const void* const* R, void* const* C,
+                     void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
+                     int64_t ldc, int trans_a, int trans_b, int sum, int dtype, int* planes);
 
 }  // namespace emi

@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include "../../include/emi.h"
+#include "gemm_plan.h"
 #include "rmsnorm.h"
 
 extern "C" int emi_fail(int code, const char* fmt, ...);
@@ -144,10 +145,22 @@ ReverseScratch carve_reverse(void* base, const Dims& d, int group, int transpose
     if (int rc__ = (call)) return rc__; \
   } while (0)
 
-int forward_layer(emi_stream_t st, const void* const* w, const void* x, const float* table, const Saved& s, void* out, void* ws, size_t wsb,
-                  const Dims& d) {
+// y = rmsnorm(x) gamma, with x = a b^T + r by the product that comes before it.
+int product_and_norm(emi_stream_t st, const void* a, const void* b, const void* r, void* x, const void* gamma, void* y, void* ws, size_t wsb,
+                     int64_t K, const Dims& d) {
+  int planes = 0;
+  EMI_TRY(emi::gemm_run(static_cast<hipStream_t>(st), a, b, r, x, ws, wsb, d.T(), d.D, K, K, K, d.D, d.D, 0, 1, d.dtype,
+                        emi::rmsnorm_one_pass(d.D) ? &planes : nullptr));
+  if (planes > 0)
+    return emi::launch_rmsnorm_fwd_planes(static_cast<hipStream_t>(st), static_cast<const float*>(ws), planes, r, gamma, x, y, d.T(), d.D, d.eps,
+                                          d.dtype);
+  return emi_rmsnorm_fwd(st, x, gamma, y, d.T(), d.D, d.eps, d.dtype);
+}
+
+// From s.xb1, the normalised x, on; with the next layer's gamma and xb1, or the result alone.
+int forward_layer(emi_stream_t st, const void* const* w, const void* x, const float* table, const Saved& s, void* out, const void* next_gamma,
+                  void* next_xb, void* ws, size_t wsb, const Dims& d) {
   const int64_t T = d.T(), D = d.D, H = d.H;
-  EMI_TRY(emi_rmsnorm_fwd(st, x, w[kAtt], s.xb1, T, D, d.eps, d.dtype));
   if (d.rope_projection()) {
     EMI_TRY(emi_gemm_rope(st, s.xb1, w[kQ], s.q, table, T, D, D, d.S, d.hd(), d.dtype));
     EMI_TRY(emi_gemm_rope(st, s.xb1, w[kK], s.k, table, T, D, D, d.S, d.hd(), d.dtype));
@@ -159,8 +172,7 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
     EMI_TRY(emi_rope(st, s.q, table, s.q, 2 * d.B, d.S, d.heads, d.hd(), 0, d.dtype));
   }
   EMI_TRY(emi_attn_fwd(st, s.q, s.k, s.v, s.att, s.lse, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
-  EMI_TRY(emi_gemm_ws(st, s.att, w[kO], x, s.x1, ws, wsb, T, D, D, D, D, D, D, 0, 1, d.dtype));
-  EMI_TRY(emi_rmsnorm_fwd(st, s.x1, w[kFfn], s.xb2, T, D, d.eps, d.dtype));
+  EMI_TRY(product_and_norm(st, s.att, w[kO], x, s.x1, w[kFfn], s.xb2, ws, wsb, D, d));
   if (d.swiglu_epilogue()) {
     EMI_TRY(emi_gemm_ws(st, s.xb2, w[kW1], nullptr, s.h1, ws, wsb, T, H, D, D, D, H, H, 0, 1, d.dtype));
     EMI_TRY(emi_gemm_swiglu_fwd(st, s.xb2, w[kW3], s.h1, s.h3, s.g, T, H, D, d.dtype));
@@ -170,6 +182,7 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
     EMI_TRY(emi_gemm_grouped(st, 2, a, b, nullptr, c, ws, wsb, T, H, D, D, D, H, H, 0, 1, 0, d.dtype));
     EMI_TRY(emi_swiglu_fwd(st, s.h1, s.h3, s.g, T * H, d.dtype));
   }
+  if (next_xb != nullptr) return product_and_norm(st, s.g, w[kW2], s.x1, out, next_gamma, next_xb, ws, wsb, H, d);
   return emi_gemm_ws(st, s.g, w[kW2], s.x1, out, ws, wsb, T, D, H, H, H, D, D, 0, 1, d.dtype);
 }
 
@@ -205,14 +218,15 @@ int flush(emi_stream_t st, Norms& p, const Dims& d) {
   p.n = 0;
   return emi::launch_colsums(static_cast<hipStream_t>(st), p.c, n, emi::rmsnorm_partial_rows(d.T(), d.D), d.D, d.dtype);
 }
-int norm_adjoint(emi_stream_t st, Norms& p, const void* x, const void* gamma, const void* dy, const void* dx_add, void* dx, void* dgamma,
-                 const ReverseScratch& r, const Dims& d) {
+// dy in `dy`, or in `planes` planes of the workspace.
+int norm_adjoint(emi_stream_t st, Norms& p, const void* x, const void* gamma, const void* dy, int planes, const void* dx_add, void* dx,
+                 void* dgamma, const ReverseScratch& r, const Dims& d) {
   if (!norms_wait(d)) return emi_rmsnorm_bwd(st, x, gamma, dy, dx_add, dx, dgamma, r.ws, r.ws_bytes, d.T(), d.D, d.eps, d.dtype);
   if (p.n == emi::kMaxColsums) EMI_TRY(flush(st, p, d));
   float* part_rows = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(r.parts) + p.n * norm_part_bytes(d));
   p.c.part[p.n] = part_rows;
   p.c.out[p.n++] = dgamma;
-  return emi::launch_rmsnorm_bwd_rows(static_cast<hipStream_t>(st), x, gamma, dy, dx_add, dx, part_rows, d.T(), d.D, d.eps, d.dtype);
+  return emi::launch_rmsnorm_bwd_rows(static_cast<hipStream_t>(st), x, gamma, planes > 0 ? r.ws : dy, planes, dx_add, dx, part_rows, d.T(), d.D, d.eps, d.dtype);
 }
 
 int check_layers(const char* name, const Dims& d, const void* const* w, std::initializer_list<const void*> ptrs) {
@@ -282,7 +296,12 @@ extern "C" int emi_llama_layers_fwd(emi_stream_t stream, const void* const* weig
     if (buffer == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_fwd: null buffer for layer %lld", (long long)l);
     const Saved s = carve_saved(buffer, d);
     void* out = l + 1 < layers ? s.out : y;
-    EMI_TRY(forward_layer(stream, w, x, rope_table, s, out, workspace, workspace_bytes, d));
+    void* next = l + 1 < layers ? saved[keep ? l + 1 : 0] : nullptr;
+    if (l + 1 < layers && next == nullptr)
+      return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_fwd: null buffer for layer %lld", (long long)(l + 1));
+    if (l == 0) EMI_TRY(emi_rmsnorm_fwd(stream, x, w[kAtt], s.xb1, d.T(), dim, eps, dtype));
+    EMI_TRY(forward_layer(stream, w, x, rope_table, s, out, part(weights[kAtt], (size_t)dim * (size_t)(l + 1) * d.elt()),
+                          next != nullptr ? carve_saved(next, d).xb1 : nullptr, workspace, workspace_bytes, d));
     x = out;
   }
   return EMI_OK;
@@ -314,6 +333,8 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     }
   Pending sq, up, down;                                   // [D, D], [H, D], [D, H]
   Norms norms;
+  int planes = 0;                                         // of the product that the next RMSNorm adjoint reads
+  int* const leave = norms_wait(d) ? &planes : nullptr;
   const int64_t hd = d.hd();
   for (int64_t l = layers - 1; l >= 0; l--) {
     const void *w[kWeights], *b[kWeights];
@@ -341,9 +362,10 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     {
       const void *a2[2] = {c.dh1, c.dh3}, *b2[2] = {b[kW1], b[kW3]};
       void* out[1] = {r.dxb};
-      EMI_TRY(emi_gemm_grouped(stream, 2, a2, b2, nullptr, out, r.ws, r.ws_bytes, T, D, H, H, tb ? H : D, D, D, 0, tb, 1, dtype));
+      EMI_TRY(emi::gemm_grouped_run(static_cast<hipStream_t>(stream), 2, a2, b2, nullptr, out, r.ws, r.ws_bytes, T, D, H, H, tb ? H : D, D, D, 0,
+                                    tb, 1, dtype, leave));
     }
-    EMI_TRY(norm_adjoint(stream, norms, s.x1, w[kFfn], r.dxb, dy, c.dx1, g[kFfn], r, d));
+    EMI_TRY(norm_adjoint(stream, norms, s.x1, w[kFfn], r.dxb, planes, dy, c.dx1, g[kFfn], r, d));
     EMI_TRY(emi_gemm_ws(stream, c.dx1, b[kO], nullptr, r.dxb, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, dtype));
     if (d.rope_attention()) {
       EMI_TRY(emi_attn_bwd_rope(stream, s.q, s.k, s.v, s.att, s.lse, r.dxb, c.dq, c.dk, c.dv, rope_table, r.ws, r.ws_bytes, d.B, d.heads, d.S, hd,
@@ -356,11 +378,12 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     {
       const void *a3[3] = {c.dq, c.dk, c.dv}, *b3[3] = {b[kQ], b[kK], b[kV]};
       void* out[1] = {r.dxb};
-      EMI_TRY(emi_gemm_grouped(stream, 3, a3, b3, nullptr, out, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, 1, dtype));
+      EMI_TRY(emi::gemm_grouped_run(static_cast<hipStream_t>(stream), 3, a3, b3, nullptr, out, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, 1, dtype,
+                                    leave));
     }
     // the first layer's cotangent leaves; a caller's accumulated one is added by its own launch
     void* dx_l = l == 0 ? dx : c.dx;
-    EMI_TRY(norm_adjoint(stream, norms, x_l, w[kAtt], r.dxb, c.dx1, dx_l, g[kAtt], r, d));
+    EMI_TRY(norm_adjoint(stream, norms, x_l, w[kAtt], r.dxb, planes, c.dx1, dx_l, g[kAtt], r, d));
     if (l == 0 && dx_add != nullptr) EMI_TRY(emi_add(stream, dx, dx_add, dx, T * D, dtype));
     EMI_TRY(wait(stream, sq, c.dq, s.xb1, g[kQ], D, D, T, r, dtype));
     EMI_TRY(wait(stream, sq, c.dk, s.xb1, g[kK], D, D, T, r, dtype));
