@@ -8,10 +8,10 @@
 // from 128 x 128 down to 32 x 32 (whose eight wavefronts share k), and a launcher that chooses by how the tiles divide over
 // the CUs (bf16_plan).  Eight wavefronts of 32 x 64 on a 128 x 128 tile read 1.5 times the LDS bytes of four of 64 x 64 and
 // are still faster: two of them on a SIMD hide each other's LDS and barrier latency.
-// Measured, us, against the two-stage 128 x 128 kernel of gemm.hip (k-contiguous B): 777 x 768 x 768 12.2 -> 6.8;
-// 777 x 768 x 2048 18.7 -> 12.5; 64 x 768 x 768 9.9 -> 4.2; 300 x 5632 x 2048 23.2 -> 15.0; 1000 x 4096 x 4096 47.5 -> 37.0;
+// Measured, us, against the two-stage 128 x 128 kernel of gemm.hip (k-contiguous B): 777 x 768 x 768 12.2 -> 5.5;
+// 777 x 768 x 2048 18.7 -> 9.0; 64 x 768 x 768 9.9 -> 4.2; 300 x 5632 x 2048 23.2 -> 13.2; 1000 x 4096 x 4096 47.5 -> 37.0;
 // 8192 x 768 x 768 15.4 -> 15.2, x 2048 30.5 -> 29.1; 8192 x 2304 x 768 42.4 -> 37.1 (782 TFLOP/s); k-major B:
-// 777 x 768 x 768 15.5 -> 6.6; 1000 x 4096 x 4096 64.4 -> 38.2; 8192 x 768 x 2048 36.6 -> 30.4.
+// 777 x 768 x 768 15.5 -> 5.8; 1000 x 4096 x 4096 64.4 -> 36.6; 8192 x 768 x 2048 36.6 -> 30.4.
 #include <type_traits>
 #include <utility>
 
@@ -91,8 +91,12 @@ template <int ROWS, int BK, int NW, bool KM> struct PipeOperand {
   }
 };
 
-// WM x WN wavefronts tile the block's BM x BN; WK wavefronts share the k of every stage (k-step ks of 32 to wavefront
-// ks % WK) and are added in wavefront order at the end.  part != nullptr: split-K, split z owns the stages
+// WM x WN wavefronts tile the block's BM x BN; WK times as many share the k of every stage (k-step ks of 32 to the wavefronts
+// ks % WK) and are added in wavefront order at the end.  A wavefront alone on its SIMD issues an instruction every 7 to 8 cycles,
+// and a stage is forty for its loads and as many around its fragments and products: on few tiles that chain, and not the
+// loads (64 bytes a cycle and CU, 258 cycles for 64 x 64 x 64), set the time.  Twice the wavefronts and stages twice as long, us:
+// 777 x 768 x 768 6.8 -> 5.5, x 2048 13.5 -> 9.0; 512 x 1024 x 1024 7.6 -> 6.0; 300 x 5632 x 2048 15.2 -> 13.2; 1000 x 2048 x 2048
+// 14.5 -> 13.2; k-major B, three products summed: 777 x 768 x 768 14.8 -> 11.2.  part != nullptr: split-K, split z owns the stages
 // [z * steps_per_split, ...) of the contraction (of the whole sum, where products are summed) and leaves its tile in
 // part[z][M][N] for the reduction over splits.
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, bool GROUPED>
@@ -103,7 +107,6 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
   constexpr int NW = WM * WN * WK;
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
   constexpr int KS = BK / 32 / WK;                                // k-steps of 32 per wavefront and stage
-  static_assert(WK == 1 || (WM == 1 && WN == 1), "wavefronts share either the tile or k");
   static_assert(NST >= 2 && KS >= 1 && BK == 32 * WK * KS, "stages");
   using OA = PipeOperand<BM, BK, NW, false>;
   using OB = PipeOperand<BN, BK, NW, BKM>;
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l15 = lane & 15, g = lane >> 4;
-  const int wk = WK == 1 ? 0 : wave, wm = WK == 1 ? wave / WN : 0, wn = WK == 1 ? wave % WN : 0;
+  const int wk = wave / (WM * WN), wm = wave % (WM * WN) / WN, wn = wave % WN;
 
   // workgroup ids go round the XCDs: give each XCD (own L2) a run of neighbouring tiles, eight tile rows deep, so that it
   // reads a few panels of both operands many times; splits and products outermost
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
     const int kq = l15 >> 2;
 #pragma unroll
     for (int b = 0; b < TN; b++) {
-      const int col = wn * (BN / WN) + b * 16 + (l15 & 3) * 4, k = 8 * g + kq;
+      const int col = wn * (BN / WN) + b * 16 + (l15 & 3) * 4, k = 32 * wk + 8 * g + kq;
       tr_at[b] = (uint32_t)(uintptr_t)smem + (uint32_t)(OA::BYTES + k * (BN * 2) + (((col >> 3) ^ OB::kswz(k)) << 4) + (col & 7) * 2);
     }
   }
@@ -220,12 +223,11 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
       constexpr int c = decltype(cc)::value;
       const int ks = c * WK + wk;
       if constexpr (BKM) {
-        static_assert(WK == 1, "k-major operands do not share k");
         u32x2_t t[TN][2];
 #pragma unroll
         for (int b = 0; b < TN; b++) {
-          t[b][0] = pipe_tr_read<c * 32 * BN * 2>(tr_at[b] + stage_off);
-          t[b][1] = pipe_tr_read<(c * 32 + 4) * BN * 2>(tr_at[b] + stage_off);
+          t[b][0] = pipe_tr_read<c * WK * 32 * BN * 2>(tr_at[b] + stage_off);
+          t[b][1] = pipe_tr_read<(c * WK * 32 + 4) * BN * 2>(tr_at[b] + stage_off);
         }
 #pragma unroll
         for (int a = 0; a < TM; a++) pa[a] = read_kc(sa, wm * (BM / WM) + a * 16 + l15, ks);
@@ -274,8 +276,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
 #pragma unroll
     for (int b = 0; b < TN; b++) *reinterpret_cast<EMI_LDS f32x4_t*>(mine + (a * 16 + l15) * RS + b * 16 + g * 4) = acc[a][b];
   if constexpr (WK > 1) __syncthreads();
-  constexpr int PPR = WC / 8, PIECES = WR * PPR, THREADS = WK > 1 ? NW * 64 : 64;
-  const int me = WK > 1 ? (int)threadIdx.x : lane;
+  constexpr int PPR = WC / 8, PIECES = WR * PPR, THREADS = WK * 64;
+  const int tile_wave = wave % (WM * WN), me = wk * 64 + lane;
 #pragma unroll
   for (int e = 0; e < (PIECES + THREADS - 1) / THREADS; e++) {
     const int at = e * THREADS + me;
@@ -286,7 +288,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
     for (int q = 0; q < 8; q++) v[q] = 0.f;
 #pragma unroll
     for (int w = 0; w < WK; w++) {
-      const EMI_LDS float* src = (WK > 1 ? (EMI_LDS float*)smem + w * (WR * RS) : mine) + row * RS + c8;
+      const EMI_LDS float* src = (EMI_LDS float*)smem + (w * WM * WN + tile_wave) * (WR * RS) + row * RS + c8;
       const f32x4_t lo = *reinterpret_cast<const EMI_LDS f32x4_t*>(src), hi = *reinterpret_cast<const EMI_LDS f32x4_t*>(src + 4);
 #pragma unroll
       for (int q = 0; q < 4; q++) {
@@ -385,7 +387,7 @@ static int launch_pipe_shape(hipStream_t st, const PipeCall& c, int trans_b) {
   if (trans_b)
     return c.grp != nullptr ? launch_pipe_one<BM, BN, WM, WN, WK, BK, NST, false, true>(st, c)
                             : launch_pipe_one<BM, BN, WM, WN, WK, BK, NST, false, false>(st, c);
-  if constexpr (WK == 1)
+  if constexpr (BN >= 64)
     return c.grp != nullptr ? launch_pipe_one<BM, BN, WM, WN, WK, BK, NST, true, true>(st, c)
                             : launch_pipe_one<BM, BN, WM, WN, WK, BK, NST, true, false>(st, c);
   return -1;
@@ -394,15 +396,17 @@ static int launch_pipe_shape(hipStream_t st, const PipeCall& c, int trans_b) {
 // Which block and how many splits of K.  The estimate is of the CU with the most blocks, in microseconds, with the rates
 // each block shape was measured at; shape 0 is the 256 x 256 ping-pong kernel of gemm.hip, whose clock falls as it fills
 // the chip (1.0 a stage of 64 k on one CU, 1.45 on all), 1 the 128 x 128 tile of which two fit a CU (0.61 alone, 0.90 two),
-// 2 the same tile in a ring of three stages (0.57, one to a CU), 3 128 x 64 (0.36 / 0.66), 4 64 x 64 (0.31 / 0.39 / 0.59),
-// 5 a 32 x 32 tile whose eight wavefronts share stages of 256 k (0.55).  The reduction over splits is a launch of its own;
+// 2 the same tile in a ring of three stages whose k two wavefronts share (0.52, one to a CU), 3 128 x 64 (a stage of 128 k 0.62
+// alone, 1.24 two), 4 64 x 64 (a stage of 128 k 0.35 alone, 0.43 with B k-major, 0.68 two, 0.38 to 0.40 a block from three on, which also start one after
+// the other),
+// 5 a 32 x 32 tile whose eight wavefronts share stages of 256 k (0.30, one after the other).  The reduction over splits is a launch of its own;
 // results over 4 M elements, whose planes leave the caches, are not split (but see pingpong_splits of gemm.hip), nor are
 // the products of a few tokens, which have kernels of their own (gemm_skinny.hip).
 Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b, int64_t most) {
   struct Shape { int bm, bn, bk; double fixed, rate[3], more; };        // rate[b - 1]: per stage, b blocks on the CU; more: per block from four on
-  static const Shape shapes[6] = {{256, 256, 64, 4.0, {1.0, 2.0, 3.0}, 1.0},  {128, 128, 64, 4.0, {0.61, 0.90, 1.45}, 0.50},
-                                  {128, 128, 64, 3.5, {0.57, 1.14, 1.71}, 0.57}, {128, 64, 64, 3.0, {0.36, 0.62, 1.0}, 0.33},
-                                  {64, 64, 64, 2.8, {0.31, 0.39, 0.59}, 0.22},   {32, 32, 256, 2.2, {0.55, 1.10, 1.65}, 0.55}};
+  static const Shape shapes[6] = {{256, 256, 64, 4.0, {1.0, 2.0, 3.0}, 1.0},   {128, 128, 64, 4.0, {0.61, 0.90, 1.45}, 0.50},
+                                  {128, 128, 64, 4.0, {0.52, 1.04, 1.56}, 0.52}, {128, 64, 128, 3.2, {0.62, 1.24, 2.0}, 0.66},
+                                  {64, 64, 128, 3.4, {0.35, 0.68, 1.14}, 0.40},  {32, 32, 256, 3.4, {0.30, 0.62, 0.95}, 0.33}};
   Bf16Plan best{1, 1, 0.0};
   double least = 1e30;
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && M > 8 && K > 8;
@@ -416,8 +420,10 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
     for (int64_t z = 1; z <= 16 && z <= most && (z == 1 || (split && steps >= 4 * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
       double stage = b < 4 ? s.rate[b - 1] : s.more * b;
+      if (c == 4 && b == 1 && !trans_b) stage = 0.43;
+      const double later = c == 4 && b > 2 ? 1.0 * (b - 2) : c == 5 ? 1.8 * (b - 1) : 0.0;      // the start of blocks that come after others
       if (c == 0) stage *= 1.0 + 0.45 * (blocks * z < 256 ? blocks * z / 256.0 : 1.0);
-      const double t = s.fixed + per * stage + (z > 1 ? 3.0 + 0.7e-6 * M * N * (z + 1) : 0.0);
+      const double t = s.fixed + later + per * stage + (z > 1 ? 3.0 + 0.7e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
         least = t;
         best = Bf16Plan{c, (int)z, t};
@@ -445,11 +451,16 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
   g.sum = sum;
   const PipeCall c{g.A[0], g.B[0], g.R[0], g.C[0], M, N, K, lda, ldb, ldr, ldc, vec_ok, part, part != nullptr ? plan.splits : 1,
                    count > 1 ? &g : nullptr, planes};
+  // With no more than one block to a CU and more than a few stages, deeper rings, which then fit (us, the ring of two | three:
+  // 777 x 768 x 768 5.5 | 5.5, x 2048 9.2 | 9.0, k-major B, three summed 14.1 | 11.2; 4096 x 512 x 512 6.5 | 7.0).
+  const int rows = plan.shape == 3 ? 128 : 64;
+  const int64_t blocks = (int64_t)((M + rows - 1) / rows) * ((N + 63) / 64) * (sum || count == 1 ? c.splits : count);
+  const bool single = blocks <= 256 && (int64_t)K * (sum ? count : 1) > 1024;
   switch (plan.shape) {
     case 1: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 2>(st, c, trans_b);
-    case 2: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 3>(st, c, trans_b);
-    case 3: return launch_pipe_shape<128, 64, 4, 2, 1, 64, 3>(st, c, trans_b);
-    case 4: return launch_pipe_shape<64, 64, 2, 2, 1, 64, 3>(st, c, trans_b);
+    case 2: return launch_pipe_shape<128, 128, 4, 2, 2, 64, 3>(st, c, trans_b);
+    case 3: return single ? launch_pipe_shape<128, 64, 4, 2, 2, 128, 3>(st, c, trans_b) : launch_pipe_shape<128, 64, 4, 2, 1, 64, 3>(st, c, trans_b);
+    case 4: return single ? launch_pipe_shape<64, 64, 2, 2, 2, 128, 3>(st, c, trans_b) : launch_pipe_shape<64, 64, 2, 2, 2, 128, 2>(st, c, trans_b);
     default: return launch_pipe_shape<32, 32, 1, 1, 8, 256, 3>(st, c, trans_b);
   }
 }
