@@ -6,12 +6,12 @@
 // matrix-vector products - RMSNorm, the rotation, SwiGLU, residuals, the new cache row - is done where its operand is
 // loaded or its result leaves, and the cache is not copied to append a row to it.
 //   forward, per layer:  norm + wq,wk,wv + rotation | attention over cache and own row (| combine) | wo + residual |
-//                        norm + w1,w3 + SwiGLU | w2 + residual
+//                        norm + w1,w3 + SwiGLU | w2 + residual;  with a short cache attention + wo + residual are one
 //   reverse, per layer:  w2^T dy and dw2 | SwiGLU' | w1^T dh1 + w3^T dh3 and dw1, dw3 | norm' (+ residual) |
 //                        wo^T dy and dwo | sum | attention' | dq, inverse rotation | wq^T dq + ... and dwq, dwk, dwv | norm'
 // The forward call leaves what the reverse one needs in `saved`.
-// Measured against the same step operator by operator (us): dim 288, 6 layers, fp32: forward 1071 -> 128 (99 launches ->
-// 31), with the reverse from StableHLO text at position 255 4042 -> 447 (289 launches -> 92); dim 4096, 2 layers, bf16,
+// Measured against the same step operator by operator (us): dim 288, 6 layers, fp32: forward 1071 -> 100 (99 launches ->
+// 25), with the reverse from StableHLO text at position 255 4042 -> 447 (289 launches -> 92); dim 4096, 2 layers, bf16,
 // 4096 keys: forward 370 -> 211 (4.5 TB/s over weights and cache; 31 launches and two copies of each cache before).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -52,19 +52,99 @@ template <typename T> __device__ __forceinline__ float normed(float x, float gam
 // forward: products of a normalised vector
 // ---------------------------------------------------------------------------
 // A wavefront owns two rows at a time: MODE 0, rows 2p and 2p + 1 of [w0; w1; w2] (q, k, v: a rotation pair of q or k);
-// MODE 1, row p of w0 and of w1 (h1, h3 of the SwiGLU).  The rows stream through in batches of UN 16-byte pieces per lane,
+// MODE 1, row p of w0 and of w1 (h1, h3 of the SwiGLU); MODE 2, rows 2p and 2p + 1 of w0 (wo) times the attention's result,
+// which each block works out for itself (step_attention).  The rows stream through in batches of UN 16-byte pieces per lane,
 // the next pair's first batch requested while the current one is summed, and the first pair's before the block normalises
 // the vector: each block keeps gamma x / rms(x) in LDS (the two halves of an eight-element piece apart, so that a
 // lane's reads of 16 bytes do not collide).
 template <typename T> struct NormGemv {
-  const T *x, *gamma;
+  const T *x, *gamma;    // MODE 2: x is the residual
   const T* w[3];
-  T* y[3];               // MODE 0: q, k, v;  MODE 1: h1, h3, g
+  T* y[3];               // MODE 0: q, k, v;  MODE 1: h1, h3, g;  MODE 2: x + w0 att
   float* rms;            // 1 / rms(x), for the adjoint
   const float2* table;   // MODE 0: (cos, sin) of pair i at i % table_pairs
   int N, K, table_pairs;
   float eps;
+  // MODE 2: the attention whose result the vector is
+  const T *q, *k_cache, *v_cache, *k_own, *v_own;
+  T* att;
+  float* lse;
+  int heads, head_dim, keys;
+  float scale;
 };
+
+// att of one query over a short cache and its own row, into the vector's LDS image: a row of 16 lanes holds a head (one
+// 16-byte piece a lane), 16 heads at a time, kStepKeys keys requested together.  Each such round costs every block one
+// latency of the L2, about 1.2 us a layer; the launch it saves costs 4 us where the host is the bound and 3 where the GPU is.
+// So it is taken up to two rounds (StepDims::short_cache).  Forward, separate -> together, us (6 layers at dim 288 and 768,
+// else 2):                  1 round            2 rounds           4 rounds
+//   f32  288,  6 heads      126 -> 100         123 -> 103         124 -> 106
+//   f32  768, 12 heads      134 -> 117         134 -> 124         134 -> 138
+//   bf16 2048, 16 heads    82.5 -> 76.8       82.4 -> 79.9       82.7 -> 86.3
+//   bf16 4096, 32 heads                      168.5 -> 165.5     168.5 -> 174.1
+constexpr int kStepKeys = 8, kStepRounds = 2;
+template <typename T> __device__ __forceinline__ void step_attention(const NormGemv<T>& a, float* xs, int pieces, bool store) {
+  using Raw = typename ChunkCached<T>::Raw;
+  constexpr int V = ChunkCached<T>::N;
+  const int l16 = threadIdx.x & 15;
+  const bool mine = l16 * V < a.head_dim;
+  for (int h = threadIdx.x >> 4; h < a.heads; h += 16) {
+    const int at = h * a.head_dim + l16 * V;
+    float qf[V], acc[V];
+#pragma unroll
+    for (int e = 0; e < V; e++) qf[e] = acc[e] = 0.f;
+    if (mine) ChunkCached<T>::load(a.q + at, qf);
+    float mx = -INFINITY, sum = 0.f;
+    for (int s0 = 0; s0 < a.keys; s0 += kStepKeys) {
+      Raw kr[kStepKeys], vr[kStepKeys];
+#pragma unroll
+      for (int u = 0; u < kStepKeys; u++) {
+        const int s = s0 + u;
+        kr[u] = vr[u] = Raw{};
+        if (mine && s < a.keys) {
+          const bool own = s == a.keys - 1;
+          kr[u] = ChunkCached<T>::load_raw((own ? a.k_own : a.k_cache + (int64_t)s * a.K) + at);
+          vr[u] = ChunkCached<T>::load_raw((own ? a.v_own : a.v_cache + (int64_t)s * a.K) + at);
+        }
+      }
+      float sc[kStepKeys], nm = mx;
+#pragma unroll
+      for (int u = 0; u < kStepKeys; u++) {
+        float kf[V], dot = 0.f;
+        ChunkCached<T>::unpack(kr[u], kf);
+#pragma unroll
+        for (int e = 0; e < V; e++) dot = fmaf(qf[e], kf[e], dot);
+        dot = row16_sum(dot);
+        sc[u] = s0 + u < a.keys ? dot * a.scale : -INFINITY;
+        nm = fmaxf(nm, sc[u]);
+      }
+      const float alpha = mx == -INFINITY ? 0.f : __expf(mx - nm);
+      sum *= alpha;
+#pragma unroll
+      for (int e = 0; e < V; e++) acc[e] *= alpha;
+      mx = nm;
+#pragma unroll
+      for (int u = 0; u < kStepKeys; u++) {
+        const float p = sc[u] == -INFINITY ? 0.f : __expf(sc[u] - mx);
+        sum += p;
+        float vf[V];
+        ChunkCached<T>::unpack(vr[u], vf);
+#pragma unroll
+        for (int e = 0; e < V; e++) acc[e] = fmaf(p, vf[e], acc[e]);
+      }
+    }
+    const float inv = 1.0f / sum;
+    if (mine) {
+#pragma unroll
+      for (int e = 0; e < V; e++) acc[e] = round_to<T>(acc[e] * inv);
+      if (store) ChunkCached<T>::store(a.att + at, acc);
+#pragma unroll
+      for (int g = 0; g < V / 4; g++)
+        *reinterpret_cast<f4*>(xs + (g * pieces + at / V) * 4) = f4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+    }
+    if (store && l16 == 0) a.lse[h] = mx + __logf(sum);
+  }
+}
 
 template <typename T, int MODE, int UN, bool WHOLE>       // WHOLE: rows are whole batches
 __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
@@ -74,9 +154,12 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
   __shared__ float scratch[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nb = (a.K + BATCH - 1) / BATCH, pieces = nb * 64 * UN;     // pieces of the padded vector
-  const int P = MODE == 0 ? 3 * a.N / 2 : a.N;
+  const int P = MODE == 0 ? 3 * a.N / 2 : MODE == 1 ? a.N : a.N / 2;
   auto rows = [&](int p, const T*& r0, const T*& r1) {
-    if constexpr (MODE == 0) {
+    if constexpr (MODE == 2) {
+      r0 = a.w[0] + (int64_t)(2 * p) * a.K;
+      r1 = r0 + a.K;
+    } else if constexpr (MODE == 0) {
       const int m = 2 * p / a.N;
       r0 = (m == 0 ? a.w[0] : m == 1 ? a.w[1] : a.w[2]) + (int64_t)(2 * p - m * a.N) * a.K;
       r1 = r0 + a.K;
@@ -102,29 +185,36 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
     rows(p0, r0, r1);
     issue(r0, r1, 0, c0, c1);
   }
-  // the vector: the norm's result, rounded to T as the operator-by-operator form stores it
-  float ss = 0.f;
-  for (int c = threadIdx.x; c * V < a.K; c += 256) {
-    float xv[V];
-    ChunkCached<T>::load(a.x + c * V, xv);
+  // the vector: the attention's or the norm's result, rounded to T as the operator-by-operator form stores it
+  if constexpr (MODE == 2) {
+    step_attention<T>(a, xs, pieces, blockIdx.x == 0);
+    for (int c = a.K / V + threadIdx.x; c < pieces; c += 256)
 #pragma unroll
-    for (int e = 0; e < V; e++) ss = fmaf(xv[e], xv[e], ss);
-  }
-  const float rs = 1.0f / sqrtf(block_sum_f32(ss, scratch) / a.K + a.eps);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.rms = rs;
-  for (int c = threadIdx.x; c < pieces; c += 256) {
-    float o[V];
-#pragma unroll
-    for (int e = 0; e < V; e++) o[e] = 0.f;
-    if (c * V < a.K) {
-      float xv[V], gv[V];
+      for (int h = 0; h < V / 4; h++) *reinterpret_cast<f4*>(xs + (h * pieces + c) * 4) = f4{0.f, 0.f, 0.f, 0.f};
+  } else {
+    float ss = 0.f;
+    for (int c = threadIdx.x; c * V < a.K; c += 256) {
+      float xv[V];
       ChunkCached<T>::load(a.x + c * V, xv);
-      ChunkCached<T>::load(a.gamma + c * V, gv);
 #pragma unroll
-      for (int e = 0; e < V; e++) o[e] = normed<T>(xv[e], gv[e], rs);
+      for (int e = 0; e < V; e++) ss = fmaf(xv[e], xv[e], ss);
     }
+    const float rs = 1.0f / sqrtf(block_sum_f32(ss, scratch) / a.K + a.eps);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.rms = rs;
+    for (int c = threadIdx.x; c < pieces; c += 256) {
+      float o[V];
 #pragma unroll
-    for (int h = 0; h < V / 4; h++) *reinterpret_cast<f4*>(xs + (h * pieces + c) * 4) = f4{o[4 * h], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]};
+      for (int e = 0; e < V; e++) o[e] = 0.f;
+      if (c * V < a.K) {
+        float xv[V], gv[V];
+        ChunkCached<T>::load(a.x + c * V, xv);
+        ChunkCached<T>::load(a.gamma + c * V, gv);
+#pragma unroll
+        for (int e = 0; e < V; e++) o[e] = normed<T>(xv[e], gv[e], rs);
+      }
+#pragma unroll
+      for (int h = 0; h < V / 4; h++) *reinterpret_cast<f4*>(xs + (h * pieces + c) * 4) = f4{o[4 * h], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]};
+    }
   }
   __syncthreads();
 
@@ -150,6 +240,15 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
     }
   };
   auto finish = [&](int p) {
+    if constexpr (MODE == 2) {                             // rows and residual in fp32, rounded once
+      const float v0 = wave_sum(s0), v1 = wave_sum(s1);
+      s0 = s1 = 0.f;
+      if (lane == 0) {
+        a.y[0][2 * p] = from_f32<T>(v0 + to_f32(a.x[2 * p]));
+        a.y[0][2 * p + 1] = from_f32<T>(v1 + to_f32(a.x[2 * p + 1]));
+      }
+      return;
+    }
     const float v0 = round_to<T>(wave_sum(s0)), v1 = round_to<T>(wave_sum(s1));
     s0 = s1 = 0.f;
     if (lane != 0) return;
@@ -202,7 +301,7 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
 
 template <typename T, int MODE> int launch_norm_gemv(hipStream_t st, const NormGemv<T>& a) {
   constexpr int V = ChunkCached<T>::N;
-  const int P = MODE == 0 ? 3 * a.N / 2 : a.N;
+  const int P = MODE == 0 ? 3 * a.N / 2 : MODE == 1 ? a.N : a.N / 2;
   // two blocks a CU: each normalises the vector once for all its pairs
   const unsigned grid = (unsigned)((P + 3) / 4 < 512 ? (P + 3) / 4 : 512);
 #define EMI_NORM_GEMV(UN)                                                                                                      \
@@ -499,6 +598,10 @@ struct StepDims {
     const int64_t want = (keys * heads / 512 + 63) / 64 * 64;
     return (int)(want < 128 ? 128 : want > 512 ? 512 : want);
   }
+  bool short_cache() const {                              // attention inside the product with wo: step_attention
+    const int lanes = hd() / (dtype == EMI_BF16 ? 8 : 4);
+    return lanes <= 16 && (heads + 15) / 16 * ((pos + kStepKeys) / kStepKeys) <= kStepRounds;
+  }
   int nsplit() const { return (int)((pos + 1 + kpb() - 1) / kpb()); }
 };
 
@@ -587,10 +690,24 @@ int step_fwd(hipStream_t st, const void* const* w, const void* x_, const void* k
     a.table_pairs = (int)d.table_pairs;
     a.N = (int)D, a.K = (int)D, a.eps = d.eps;
     if (int rc = launch_norm_gemv<T, 0>(st, a)) return rc;
-    if (int rc = launch_llama_step_attn_fwd(st, s.q, kc + l * d.pos * D, vc + l * d.pos * D, s.k, s.v, s.att, s.lse, tail.part,
-                                            (int)d.heads, (int)d.pos, d.hd(), d.kpb(), d.scale, d.dtype))
-      return rc;
-    if (int rc = launch_skinny(st, s.att, wo + l * D * D, x, s.x1, nullptr, 0, 1, D, D, D, D, D, D, 0, 1, d.dtype)) return rc;
+    if (d.short_cache()) {
+      NormGemv<T> o{};
+      o.x = x;
+      o.w[0] = wo + l * D * D;
+      o.y[0] = s.x1;
+      o.N = (int)D, o.K = (int)D;
+      o.q = s.q, o.k_own = s.k, o.v_own = s.v;
+      o.k_cache = kc + l * d.pos * D, o.v_cache = vc + l * d.pos * D;
+      o.att = s.att, o.lse = s.lse;
+      o.heads = (int)d.heads, o.head_dim = d.hd(), o.keys = (int)d.pos + 1;
+      o.scale = d.scale;
+      if (int rc = launch_norm_gemv<T, 2>(st, o)) return rc;
+    } else {
+      if (int rc = launch_llama_step_attn_fwd(st, s.q, kc + l * d.pos * D, vc + l * d.pos * D, s.k, s.v, s.att, s.lse, tail.part,
+                                              (int)d.heads, (int)d.pos, d.hd(), d.kpb(), d.scale, d.dtype))
+        return rc;
+      if (int rc = launch_skinny(st, s.att, wo + l * D * D, x, s.x1, nullptr, 0, 1, D, D, D, D, D, D, 0, 1, d.dtype)) return rc;
+    }
     NormGemv<T> f{};
     f.x = s.x1;
     f.gamma = g2 + l * D;
