@@ -8,10 +8,10 @@
 //   forward, per layer:  norm + wq,wk,wv + rotation | attention over cache and own row (| combine) | wo + residual |
 //                        norm + w1,w3 + SwiGLU | w2 + residual;  with a short cache attention + wo + residual are one
 //   reverse, per layer:  w2^T dy and dw2 | SwiGLU' | w1^T dh1 + w3^T dh3 and dw1, dw3 | norm' (+ residual) |
-//                        wo^T dy and dwo | sum | attention' | dq, inverse rotation | wq^T dq + ... and dwq, dwk, dwv | norm'
+//                        wo^T dy and dwo | sum | attention' (|) dq, inverse rotation | wq^T dq + ... and dwq, dwk, dwv | norm'
 // The forward call leaves what the reverse one needs in `saved`.
 // Measured against the same step operator by operator (us): dim 288, 6 layers, fp32: forward 1071 -> 100 (99 launches ->
-// 25), with the reverse from StableHLO text at position 255 4042 -> 447 (289 launches -> 92); dim 4096, 2 layers, bf16,
+// 25), with the reverse from StableHLO text at position 255 4042 -> 412 (289 launches -> 86); dim 4096, 2 layers, bf16,
 // 4096 keys: forward 370 -> 211 (4.5 TB/s over weights and cache; 31 launches and two copies of each cache before).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -28,8 +28,8 @@ int launch_llama_step_attn_fwd(hipStream_t st, const void* q, const void* k_cach
                                float scale, int dtype);                                                      // attention_step.hip
 int launch_llama_step_attn_bwd(hipStream_t st, const void* q, const void* k_cache, const void* v_cache, const void* k_tail,
                                const void* v_tail, const void* o, const float* lse, const void* d_o, void* dk_cache, void* dv_cache,
-                               void* dk_tail, void* dv_tail, float* part, int heads, int pos, int head_dim, int keys_per_block, float scale,
-                               int dtype);
+                               void* dk_tail, void* dv_tail, float* part, const float* table, int table_pairs, float* fq, float* fk, float* fv,
+                               int heads, int pos, int head_dim, int keys_per_block, float scale, int dtype);
 
 namespace {
 
@@ -556,32 +556,6 @@ __global__ __launch_bounds__(1024) void step_norm_adjoint_kernel(const float* __
   }
 }
 
-// dq of a head from its blocks' shares, turned back by the position's angle; dk of the token's own row turned back; dv.
-template <typename T>
-__global__ __launch_bounds__(128) void step_qkv_cotangents_kernel(const float* __restrict__ part, int nsplit, const T* __restrict__ dk,
-                                                                  const T* __restrict__ dv, const float2* __restrict__ table,
-                                                                  int table_pairs, float* __restrict__ fq, float* __restrict__ fk,
-                                                                  float* __restrict__ fv, int head_dim) {
-  const int h = blockIdx.x;
-  const float* p0 = part + (int64_t)h * nsplit * (head_dim + 2);
-  for (int i = threadIdx.x; i < head_dim / 2; i += 128) {
-    float q0 = 0.f, q1 = 0.f;
-    for (int s = 0; s < nsplit; s++) {
-      q0 += p0[s * (head_dim + 2) + 2 * i];
-      q1 += p0[s * (head_dim + 2) + 2 * i + 1];
-    }
-    const int at = h * head_dim + 2 * i;
-    const float2 t = table[(at >> 1) % table_pairs];
-    const float k0 = to_f32(dk[at]), k1 = to_f32(dk[at + 1]);
-    fq[at] = t.x * q0 + t.y * q1;
-    fq[at + 1] = t.x * q1 - t.y * q0;
-    fk[at] = t.x * k0 + t.y * k1;
-    fk[at + 1] = t.x * k1 - t.y * k0;
-    fv[at] = to_f32(dv[at]);
-    fv[at + 1] = to_f32(dv[at + 1]);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -812,11 +786,9 @@ int step_bwd(hipStream_t st, const void* const* w, const void* x_, const void* k
     EMI_CHECK_LAUNCH("emi_llama_step_bwd(sum)");
     const int64_t cache = l * d.pos * D;
     if (int rc = launch_llama_step_attn_bwd(st, s.q, kc + cache, vc + cache, s.k, s.v, s.att, s.lse, k.datt, gr[11] + cache, gr[12] + cache,
-                                            k.dk, k.dv, k.attn, (int)d.heads, (int)d.pos, d.hd(), d.kpb(), d.scale, d.dtype))
+                                            k.dk, k.dv, k.attn, table, (int)d.table_pairs, k.f0, k.f1, k.f2, (int)d.heads, (int)d.pos, d.hd(),
+                                            d.kpb(), d.scale, d.dtype))
       return rc;
-    hipLaunchKernelGGL(step_qkv_cotangents_kernel<T>, dim3((unsigned)d.heads), dim3(128), 0, st, k.attn, d.nsplit(), k.dk, k.dv,
-                       (const float2*)table, (int)d.table_pairs, k.f0, k.f1, k.f2, d.hd());
-    EMI_CHECK_LAUNCH("emi_llama_step_bwd(q, k, v)");
     a = Adjoint<T>{};
     a.w[0] = wq + l * D * D, a.dw[0] = gr[2] + l * D * D, a.dy[0] = k.f0;
     a.w[1] = wk + l * D * D, a.dw[1] = gr[3] + l * D * D, a.dy[1] = k.f1;

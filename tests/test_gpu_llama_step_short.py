@@ -1,6 +1,6 @@
 """The single-token step over a short cache, whose attention is worked out inside the product with wo: one and two rounds of
 keys and of heads, the first cache and head count beyond them, heads that fill a row of 16 lanes, rows that are no whole
-batch of loads, and an own key without a finite score."""
+batch of loads, and keys without a finite score.  The reverse turns dq and dk back where a head's only block leaves them."""
 import numpy as np
 import pytest
 import torch
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
     ("f32", 288, 6, 7), ("f32", 288, 6, 8), ("f32", 288, 6, 15), ("f32", 288, 6, 16),     # 8, 9, 16 | 17 keys
     ("f32", 64, 16, 15), ("f32", 68, 17, 7), ("f32", 68, 17, 8),                          # 16, 17 heads | 17 and 9 keys
     ("f32", 1024, 16, 3),                                                                 # head_dim 64: all 16 lanes
-    ("f32", 516, 3, 2),                                                                   # head_dim 172: the general kernels
+    ("f32", 516, 3, 2), ("bf16", 352, 2, 40),                                             # two pieces a lane: the general kernels
     ("bf16", 1024, 8, 11), ("bf16", 264, 33, 1), ("bf16", 256, 32, 7), ("bf16", 1056, 12, 9),
 ])
 def test_short_cache_matches_oracle(dt, dim, heads, pos):
