@@ -440,7 +440,7 @@ template <typename T, bool VEC, int NCH>
 __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                             const T* __restrict__ v, const T* __restrict__ o,
                                                             const float* __restrict__ lse, const T* __restrict__ d_o,
-                                                            float* __restrict__ part, T* __restrict__ dk, T* __restrict__ dv,
+                                                            float* part, T* dk, T* dv,          // no restrict: step_qkv_rows reads them back
                                                             StepShape sh, float scale) {
   using E = Elems<T, VEC>;
   using Raw = typename E::Raw;
