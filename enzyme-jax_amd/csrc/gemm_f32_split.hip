@@ -23,6 +23,7 @@ namespace emi {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 #define EMI_LDS __attribute__((address_space(3)))
@@ -109,6 +110,16 @@ template <int ROWS, int THREADS, int PF, bool KM> struct SplitOperand {
       *reinterpret_cast<EMI_LDS u32x4_t*>(to) = u32x4_t{v[0], v[1], v[2], v[3]};
     else
       *reinterpret_cast<EMI_LDS u32x2_t*>(to) = u32x2_t{v[0], v[1]};
+  }
+  // The numbers as they are, for the tiles that are multiplied in fp32: [quad][slot] in pieces of four k.
+  __device__ __forceinline__ void store_f32(int f, EMI_LDS uint8_t* lds) {
+    EMI_LDS uint8_t* to = lds + (k0 >> 2) * KP + slot(KM ? threadIdx.x % ROWS : threadIdx.x / (32 / E)) * 16;
+#pragma unroll
+    for (int e = 0; e < E; e += 4)
+      *reinterpret_cast<EMI_LDS f32x4_t*>(to + e * KP) = f32x4_t{x[f][e], x[f][e + 1], x[f][e + 2], x[f][e + 3]};      // quads q, q + 4
+  }
+  static __device__ __forceinline__ f32x4_t quad(const EMI_LDS uint8_t* lds, int q, int r) {
+    return *reinterpret_cast<const EMI_LDS f32x4_t*>(lds + q * KP + slot(r) * 16);
   }
   static __device__ __forceinline__ bf16x8_t frag(const EMI_LDS uint8_t* lds, int plane, int piece, int r) {
     return *reinterpret_cast<const EMI_LDS bf16x8_t*>(lds + plane * PLANE + piece * KP + slot(r) * 16);
@@ -278,7 +289,9 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 4) void gemm_f32_split_kernel(cons
     if (t + u < nsteps) stage(t + u, u);
   end_chain();
 
-  // Where the split does not hold, the tile is multiplied again in fp32 as it is: numbers that are infinite, NaN or round
+  // Where the split does not hold, the tile is multiplied again in fp32 as it is, in stages through the LDS (us for the whole
+  // product, ordinary numbers | all tiles again | the same on the fp32 kernels alone: 2000 x 768 x 768 28 | 56 | 33,
+  // 777 x 4096 x 4096 163 | 428 | 230, 4096^3 741 | 1730 | 1012): numbers that are infinite, NaN or round
   // to an infinite h (some sum is not finite then), and panels without a number of 2^-95 or more, whose l may be
   // below what bf16 holds.
   bool odd = false;
@@ -302,57 +315,54 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 4) void gemm_f32_split_kernel(cons
   seen = 0;
 #pragma unroll
   for (int w = 0; w < NW; w++) seen |= flags[w];
-  if ((seen & kSums) != 0 || (seen & (kBitsA | kNormalA)) == kBitsA || (seen & (kBitsB | kNormalB)) == kBitsB) {
-    int pair = 0, k0 = step0 * BK;
+  const bool again = (seen & kSums) != 0 || (seen & (kBitsA | kNormalA)) == kBitsA || (seen & (kBitsB | kNormalB)) == kBitsB;
+  if (__builtin_amdgcn_readfirstlane(again) != 0) {
+    __syncthreads();
+    at_pair = 0, at_k = step0 * BK, to_load = nsteps;
     if constexpr (GROUPED) {
       if (grp.sum) {
-        pair = step0 / ksteps;
-        k0 = (step0 - pair * ksteps) * BK;
-        A = grp.A[pair];
-        B = grp.B[pair];
+        at_pair = step0 / ksteps;
+        at_k = (step0 - at_pair * ksteps) * BK;
+        A = grp.A[at_pair];
+        B = grp.B[at_pair];
       }
     }
 #pragma unroll
     for (int a = 0; a < TM; a++)
 #pragma unroll
       for (int b = 0; b < TN; b++) total[a][b] = zero;
+    load(0);
     for (int t = 0; t < nsteps; t++) {
+      EMI_LDS uint8_t* s = smem + (t & 1) * STAGE;
+      oa.store_f32(0, s);
+      ob.store_f32(0, s + OA::BYTES);
+      load(0);
+      sync();                                                      // (the other stage is written once all are here again)
 #pragma unroll
       for (int a = 0; a < TM; a++)
 #pragma unroll
         for (int b = 0; b < TN; b++) big[a][b] = zero;
-      for (int k = k0; k < k0 + BK && k < K && (WK == 1 || (t & 1) == wk); k += 2) {
-        const bool in = k + g < K;
-        float fa[TM], fb[TN];
 #pragma unroll
-        for (int a = 0; a < TM; a++) {
-          const int r = wm * (BM / WM) + a * 32 + i;
-          fa[a] = in && r < rows_a ? A[a_row + (k + g) * a_k + (AKM ? r : (int64_t)r * lda)] : 0.f;
-        }
+      for (int c = 0; c < 4 / WK; c++) {                           // eight k: the two halves of the wavefront have four each
+        const int q = 2 * (wk * (4 / WK) + c) + g;
+        f32x4_t fa[TM], fb[TN];
 #pragma unroll
-        for (int b = 0; b < TN; b++) {
-          const int r = wn * (BN / WN) + b * 32 + i;
-          fb[b] = in && r < rows_b ? B[b_row + (k + g) * b_k + (BKM ? r : (int64_t)r * ldb)] : 0.f;
-        }
+        for (int a = 0; a < TM; a++) fa[a] = OA::quad(s, q, wm * (BM / WM) + a * 32 + i);
 #pragma unroll
-        for (int a = 0; a < TM; a++)
+        for (int b = 0; b < TN; b++) fb[b] = OB::quad(s + OA::BYTES, q, wn * (BN / WN) + b * 32 + i);
 #pragma unroll
-          for (int b = 0; b < TN; b++) big[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a], fb[b], big[a][b], 0, 0, 0);
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int a = 0; a < TM; a++)
+#pragma unroll
+            for (int b = 0; b < TN; b++) big[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][e], fb[b][e], big[a][b], 0, 0, 0);
       }
 #pragma unroll
       for (int a = 0; a < TM; a++)
 #pragma unroll
         for (int b = 0; b < TN; b++) total[a][b] += big[a][b];
-      k0 += BK;
-      if constexpr (GROUPED) {
-        if (k0 >= K && t + 1 < nsteps) {
-          k0 = 0;
-          pair++;
-          A = grp.A[pair];
-          B = grp.B[pair];
-        }
-      }
     }
+    __syncthreads();
   }
 
   // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32 x 32 tile.  Of two wavefronts that
