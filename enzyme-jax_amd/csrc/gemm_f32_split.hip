@@ -3,7 +3,9 @@
 //   C[M,N] = op(A) . op(B) [+ R]      fp32 in, fp32 out, errors no larger than those of the fp32 instructions
 //
 // A bf16 matrix instruction multiplies sixteen times as fast as an fp32 one.  An fp32 number is the sum of three bf16
-// numbers, exactly: h = bf16(x), m = bf16(x - h), l = x - h - m (8 + 8 + 8 bits, the differences exact).  Of the nine
+// numbers, exactly: h = bf16(x), m = bf16(x - h), l = x - h - m (8 + 8 + 8 bits, the differences exact).  That holds from 2^-102
+// on; a tile whose operands hold a smaller number (but 0) is multiplied in fp32 as it is, so that neither a row of small numbers
+// nor a single one loses bits to its neighbours (rows of 1e-36 beside rows of N(0, 1): 1.4e-7; 2.7e-5 without that).  Of the nine
 // products of two such sums hh, hm, mh, mm, hl, lh are taken; the other three are below 2^-25 of the whole.  Products of
 // bf16 are exact and summed in fp32: hh in sums of their own, so that what the small ones round off is 2^-8 smaller, and
 // both end in `total` every PF stages (64 or 96 k), which keeps the chains short.  Relative error against float64, this | the
@@ -28,11 +30,13 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 #define EMI_LDS __attribute__((address_space(3)))
 constexpr uint32_t kOob = 0x80000000u;   // beyond any buffer's num_records: loads return 0
+constexpr int kDenormal = 1 << 4 | 1 << 7;   // of v_cmp_class: negative, positive
 
 // N numbers; h, m, l: two numbers in a word.  Step by step over all of them: an instruction that needs the result of the
-// one before it waits for it.
-template <int N> __device__ __forceinline__ void split(const float (&x)[N], uint32_t (&h)[N / 2], uint32_t (&m)[N / 2], uint32_t (&l)[N / 2]) {
-  float r[N], t[N];
+// one before it waits for it.  rest: what is left for l.
+template <int N>
+__device__ __forceinline__ void split(const float (&x)[N], uint32_t (&h)[N / 2], uint32_t (&m)[N / 2], uint32_t (&l)[N / 2], float (&r)[N]) {
+  float t[N];
   auto round = [&](uint32_t (&to)[N / 2], const float (&v)[N]) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < N / 2; q++) to[q] = pack_bf16x2(v[2 * q], v[2 * q + 1]);
@@ -68,12 +72,22 @@ template <int ROWS, int THREADS, int PF, bool KM> struct SplitOperand {
   uint32_t voff, at;                                              // of the first number in memory, of the piece in the LDS
   int k0;                                                         // the first k
   float x[PF + 2][E];                                             // the stages in flight; two more to begin with
-  uint32_t seen;                                                  // the bits of everything split
+  // What has been split may have held a number that is not the sum of its parts: bf16 holds what is left for l, eight bits, unless
+  // that is a denormal fp32 number, and from 2^-102 on it is 0 or at least 2^-126.  The class of what is left takes an
+  // instruction of the vector and one of the scalar unit a number, the least number but 0 one and a half of the vector
+  // unit; the second are fewer for a wavefront that is alone on its SIMD, the first hide among four.  us, neither | class |
+  // least: 2000 x 768 x 768 (128 x 64) 26.3 | 28.9 | 26.6, 1000 x 768 x 768 (64 x 64) 18.1 | 19.1 | 18.7, 777 x 4096 x 4096
+  // (128 x 128) 169 | 170 | 172, 2048^3 97.8 | 98.2 | 99.8.
+  static constexpr bool BY_CLASS = THREADS == 1024;
+  uint64_t lost;                                                  // lanes
+  uint32_t least;                                                 // bits << 1, less one
+  __device__ __forceinline__ bool inexact() const { return BY_CLASS ? lost != 0 : least < (25u << 24) - 1; }
   __device__ __forceinline__ void init(int rows_left, int ld) {
     const int tid = threadIdx.x;
     const int row = KM ? tid % ROWS : tid / (32 / E), q = KM ? tid / ROWS : tid % (32 / E);
     k0 = 4 * q;                                                   // E == 4: quad q of the 32 k; E == 8: quads q and q + 4
-    seen = 0;
+    lost = 0;
+    least = 0xffffffffu;
     voff = row < rows_left ? (uint32_t)(KM ? k0 * ld + row : row * ld + k0) * 4u : kOob;
     at = (uint32_t)((q & 3) * KP + slot(row) * 16 + (q >> 2) * 8);
   }
@@ -98,9 +112,18 @@ template <int ROWS, int THREADS, int PF, bool KM> struct SplitOperand {
   }
   __device__ __forceinline__ void store(int f, EMI_LDS uint8_t* lds) {
     uint32_t h[E / 2], m[E / 2], l[E / 2];
+    float rest[E];
+    split<E>(x[f], h, m, l, rest);
+    if constexpr (BY_CLASS) {
+      bool any = false;
 #pragma unroll
-    for (int q = 0; q < E; q += 2) seen |= __float_as_uint(x[f][q]) | __float_as_uint(x[f][q + 1]);
-    split<E>(x[f], h, m, l);
+      for (int q = 0; q < E; q++) any = any | __builtin_amdgcn_classf(rest[q], kDenormal);
+      lost |= __builtin_amdgcn_ballot_w64(any);
+    } else {
+#pragma unroll
+      for (int q = 0; q < E; q += 2)
+        least = min(min(least, (__float_as_uint(x[f][q]) << 1) - 1), (__float_as_uint(x[f][q + 1]) << 1) - 1);      // 0 wraps round
+    }
     put(lds + at, h);
     put(lds + at + PLANE, m);
     put(lds + at + 2 * PLANE, l);
@@ -291,10 +314,9 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 4) void gemm_f32_split_kernel(cons
 
   // Where the split does not hold, the tile is multiplied again in fp32 as it is, in stages through the LDS (us for the whole
   // product, ordinary numbers | all tiles again | the same on the fp32 kernels alone: 2000 x 768 x 768 28 | 56 | 33,
-  // 777 x 4096 x 4096 163 | 428 | 230, 4096^3 741 | 1730 | 1012): numbers that are infinite, NaN or round
-  // to an infinite h (some sum is not finite then), and panels without a number of 2^-95 or more, whose l may be
-  // below what bf16 holds.
-  bool odd = false;
+  // 777 x 4096 x 4096 163 | 428 | 230, 4096^3 741 | 1730 | 1012): a number that may not be the sum of its parts, and numbers that
+  // are infinite, NaN or round to an infinite h (some sum is not finite then).
+  bool odd = oa.inexact() || ob.inexact();
 #pragma unroll
   for (int a = 0; a < TM; a++)
 #pragma unroll
@@ -304,18 +326,14 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 4) void gemm_f32_split_kernel(cons
       for (int r = 0; r < 16; r++) z = __builtin_fmaf(total[a][b][r], 0.f, z);
       odd = odd || z != 0.f;
     }
-  enum { kSums = 1, kBitsA = 2, kNormalA = 4, kBitsB = 8, kNormalB = 16 };
-  uint32_t seen = __any(odd) ? kSums : 0;
-  seen |= (__any((oa.seen & 0x7fffffffu) != 0) ? kBitsA : 0) | (__any((oa.seen & 0x70000000u) != 0) ? kNormalA : 0);
-  seen |= (__any((ob.seen & 0x7fffffffu) != 0) ? kBitsB : 0) | (__any((ob.seen & 0x70000000u) != 0) ? kNormalB : 0);
   EMI_LDS uint32_t* flags = (EMI_LDS uint32_t*)smem;
+  const uint32_t seen = __any(odd);
   __syncthreads();
   if (lane == 0) flags[wave] = seen;
   __syncthreads();
-  seen = 0;
+  uint32_t again = 0;
 #pragma unroll
-  for (int w = 0; w < NW; w++) seen |= flags[w];
-  const bool again = (seen & kSums) != 0 || (seen & (kBitsA | kNormalA)) == kBitsA || (seen & (kBitsB | kNormalB)) == kBitsB;
+  for (int w = 0; w < NW; w++) again |= flags[w];
   if (__builtin_amdgcn_readfirstlane(again) != 0) {
     __syncthreads();
     at_pair = 0, at_k = step0 * BK, to_load = nsteps;

@@ -54,7 +54,7 @@ def test_numbers_that_do_not_split(what, ta, tb, M, N, K):
         b *= np.float32(1e-3)
     elif what == "tiny":
         a *= np.float32(1e-36)
-    elif what == "tiny rows":                                   # beside ordinary ones: what they lose is below those' roundings
+    elif what == "tiny rows":                                   # beside ordinary ones
         a[(slice(None), slice(5, 9)) if ta else slice(5, 9)] *= np.float32(1e-36)
     else:
         a[:] = 0
@@ -67,9 +67,37 @@ def test_numbers_that_do_not_split(what, ta, tb, M, N, K):
     finite = np.isfinite(ref)
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
-    slack = 2.0 ** -130 * np.abs(y).sum(0)[None, :] if what == "tiny rows" else 2.0 ** -149 * K     # the last bit of l; denormal results
-    bound = (K + 2) * 2.0 ** -23 * mag + slack
+    bound = (K + 2) * 2.0 ** -23 * mag + 2.0 ** -149 * K         # denormal results
     assert np.all(np.abs(got[finite] - ref[finite]) <= bound[finite])
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(964, 772, 100), (900, 1092, 132), (1060, 1092, 2052)])
+@pytest.mark.parametrize("scale", [1e-31, 1e-34, 1e-37, 1e-41])
+def test_small_numbers_keep_their_bits(scale, ta, tb, M, N, K):
+    """A row of A, a column of B and single terms far below their neighbours are as exact as any other: what a number loses
+    is not measured by the largest one of its tile.  An fp32 sum of K terms, plus the step of denormal products."""
+    from enzyme_ad.jax import ops
+    rng = np.random.default_rng(M + N + K + 2 * ta + tb)
+    a0, b0 = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+
+    def check(a, b, what):
+        put = lambda t, turn: torch.from_numpy(np.ascontiguousarray(t.T if turn else t)).cuda()
+        got = host(ops.gemm(put(a, ta), put(b, tb), bool(ta), bool(tb)))
+        x, y = a.astype(np.float64), b.astype(np.float64)
+        err, bound = np.abs(got - x @ y), (K + 2) * 2.0 ** -23 * (np.abs(x) @ np.abs(y)) + 2.0 ** -149 * K
+        assert np.all(err <= bound), "%s: worst error / bound %.2f" % (what, float(np.max(err / bound)))
+
+    a, b = a0.copy(), b0.copy()
+    a[5:9] *= np.float32(scale)
+    b[:, N - 3:] *= np.float32(scale)
+    check(a, b0, "rows of A")
+    check(a0, b, "columns of B")
+    check(a, b0 * np.float32(1e20), "rows of A against large numbers")
+    a, b = a0.copy(), b0.copy()
+    a[:, K // 2:] *= np.float32(scale)
+    b[:K // 2] = 0
+    check(a, b, "terms whose neighbours meet zeros")
 
 
 @pytest.mark.parametrize("M,N,K", [(2000, 768, 768), (776, 4096, 4096)])
