@@ -9,7 +9,7 @@
 // score has the weight 0 and its row is multiplied by it, so a NaN or an infinity in a row of v also reaches earlier queries
 // of the same 16-row tile. Operands come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
 // 16 rows are one chain of them, so with one wavefront per 16 rows (the earlier form) the longest row set the time and too
-// few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 11,
+// few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 9,
 // 24 heads x 1000 x 64 89 / 280 -> 56 / 161 (55 / 48 TFLOP/s), 64 heads x 2048 x 128 1329 / 4010 -> 795 / 2907 (86 / 59);
 // the loads of K, V and Q through the L1 come next.
 // As on the bf16 path everything is computed transposed: the score tile is S^T[other row, own row], so lane l owns row
@@ -226,60 +226,6 @@ __global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* 
   if (wave == 0 && G == 0 && myq < sh.seq) lse[(int64_t)bh * sh.seq + myq] = top + logf(sum);
 }
 
-// dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T, delta = rowsum(dO * O), which it also
-// leaves for the dK/dV kernel.
-template <int NT>
-__device__ __forceinline__ void bwd_dq_rows(const BlockRows own, const float* __restrict__ q, const float* __restrict__ k,
-                                            const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ d_o,
-                                            const float* __restrict__ lse, float* __restrict__ delta, float* __restrict__ dq,
-                                            AttnShapeF32 sh, float scale, int causal, float (&buf)[kWaves][kWaves * NT][64]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
-  const int tiles = (sh.seq + 15) >> 4;
-  const int q0 = (tiles - 1 - own.tile) * 16;
-  const int bh = own.bh;
-  const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
-  const int last = sh.seq - 1;
-  const int myq = q0 + (lane & 15);
-  const int qc = myq < last ? myq : last;
-  float qf[NT][4], dof[NT][4];
-  load_rows<NT>(q + base, sh.ss, q0, last, lane, qf);
-  load_rows<NT>(d_o + base, sh.ss, q0, last, lane, dof);
-  const float L = lse[(int64_t)bh * sh.seq + qc];
-  float dl = 0.f;
-  {
-    float of[NT][4];
-    load_rows<NT>(o + base, sh.ss, q0, last, lane, of);
-#pragma unroll
-    for (int c = 0; c < NT; c++)
-#pragma unroll
-      for (int t = 0; t < 4; t++) dl += of[c][t] * dof[c][t];
-    dl = groups_sum(dl);
-    if (delta != nullptr && wave == 0 && G == 0 && myq < sh.seq) delta[(int64_t)bh * sh.seq + myq] = dl;
-  }
-  const int nkeys = causal ? (q0 + 16 < sh.seq ? q0 + 16 : sh.seq) : sh.seq;
-  f32q_t acc[NT];
-#pragma unroll
-  for (int n = 0; n < NT; n++) acc[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
-  for (int kb = 16 * wave; kb < nkeys; kb += 16 * kWaves) {
-    float kf[NT][4], vf[NT][4], kx[4][NT];
-    load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
-    load_rows<NT>(v + base, sh.ss, kb, last, lane, vf);
-    load_cols<NT>(k + base, sh.ss, kb, last, lane, kx);        // for dQ += dS . K
-    f32q_t s = rows_dot<NT>(kf, qf);
-    const f32q_t dp = rows_dot<NT>(vf, dof);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int key = kb + 4 * G + r;
-      const bool valid = key < nkeys && (!causal || key <= myq);
-      const float p = valid ? expf(s[r] * scale - L) : 0.f;
-      s[r] = p * (dp[r] - dl) * scale;
-    }
-    mma_cols<NT>(kx, s, acc);
-  }
-  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
-  merge_store<NT>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf);
-}
-
 // dV = P^T dO, dK = scale dS^T Q: a block per 16 keys, walking the queries that see them.
 // DELTA: from the rows of o, where nothing has left delta.
 template <int NT, bool DELTA>
@@ -346,16 +292,6 @@ __device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* _
 }
 
 template <int NT>
-__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                      const float* __restrict__ v, const float* __restrict__ o,
-                                                                      const float* __restrict__ d_o,
-                                                                      const float* __restrict__ lse, float* __restrict__ delta,
-                                                                      float* __restrict__ dq, AttnShapeF32 sh, float scale,
-                                                                      int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
-  bwd_dq_rows<NT>(block_rows((sh.seq + 15) >> 4), q, k, v, o, d_o, lse, delta, dq, sh, scale, causal, buf);
-}
-template <int NT>
 __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                        const float* __restrict__ v,
                                                                        const float* __restrict__ d_o,
@@ -367,18 +303,74 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const flo
   bwd_dkv_rows<NT, false>(block_rows((sh.seq + 15) >> 4), q, k, v, nullptr, d_o, lse, delta, dk, dv, sh, scale, causal, buf);
 }
 
-// Both as one launch (grid.z: 0 dK/dV, 1 dQ), for sequences and heads that leave the chip half empty: the two run side by side
+// dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T, delta = rowsum(dO * O), which it also
+// leaves for the dK/dV kernel.
+// BOTH: one launch (grid.z: 0 dK/dV, 1 dQ) for sequences and heads that leave the chip half empty: the two run side by side
 // instead of one after the other, and dK/dV forms delta itself.
-template <int NT>
-__global__ __launch_bounds__(64 * kWaves) void attn_bwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                   const float* __restrict__ v, const float* __restrict__ o,
-                                                                   const float* __restrict__ d_o, const float* __restrict__ lse,
-                                                                   float* __restrict__ dq, float* __restrict__ dk,
-                                                                   float* __restrict__ dv, AttnShapeF32 sh, float scale, int causal) {
+// dQ stands in its kernel, dK/dV in a function of its own: the order of the loads that the compiler makes of either depends
+// on that.  us, dQ in a function | here: 24 heads x 1000 x 96 261 | 247, 8 x 3000 x 128 784 | 768; dK/dV in its kernel | in a
+// function: 24 x 1000 x 32 105 | 98, 64 x 1024 x 48 294 | 284.
+template <int NT, bool BOTH>
+__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                      const float* __restrict__ v, const float* __restrict__ o,
+                                                                      const float* __restrict__ d_o,
+                                                                      const float* __restrict__ lse, float* __restrict__ delta,
+                                                                      float* __restrict__ dq, float* __restrict__ dk,
+                                                                      float* __restrict__ dv, AttnShapeF32 sh, float scale,
+                                                                      int causal) {
   __shared__ float buf[kWaves][kWaves * NT][64];
-  const BlockRows own = block_rows((sh.seq + 15) >> 4);
-  if (blockIdx.z == 0) bwd_dkv_rows<NT, true>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, buf);
-  else bwd_dq_rows<NT>(own, q, k, v, o, d_o, lse, nullptr, dq, sh, scale, causal, buf);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
+  const int tiles = (sh.seq + 15) >> 4;
+  const BlockRows own = block_rows(tiles);
+  if constexpr (BOTH) {
+    if (blockIdx.z == 0) {
+      bwd_dkv_rows<NT, true>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, buf);
+      return;
+    }
+  }
+  const int q0 = (tiles - 1 - own.tile) * 16;
+  const int bh = own.bh;
+  const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
+  const int last = sh.seq - 1;
+  const int myq = q0 + (lane & 15);
+  const int qc = myq < last ? myq : last;
+  float qf[NT][4], dof[NT][4];
+  load_rows<NT>(q + base, sh.ss, q0, last, lane, qf);
+  load_rows<NT>(d_o + base, sh.ss, q0, last, lane, dof);
+  const float L = lse[(int64_t)bh * sh.seq + qc];
+  float dl = 0.f;
+  {
+    float of[NT][4];
+    load_rows<NT>(o + base, sh.ss, q0, last, lane, of);
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+      for (int t = 0; t < 4; t++) dl += of[c][t] * dof[c][t];
+    dl = groups_sum(dl);
+    if (!BOTH && wave == 0 && G == 0 && myq < sh.seq) delta[(int64_t)bh * sh.seq + myq] = dl;
+  }
+  const int nkeys = causal ? (q0 + 16 < sh.seq ? q0 + 16 : sh.seq) : sh.seq;
+  f32q_t acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; n++) acc[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
+  for (int kb = 16 * wave; kb < nkeys; kb += 16 * kWaves) {
+    float kf[NT][4], vf[NT][4], kx[4][NT];
+    load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
+    load_rows<NT>(v + base, sh.ss, kb, last, lane, vf);
+    load_cols<NT>(k + base, sh.ss, kb, last, lane, kx);        // for dQ += dS . K
+    f32q_t s = rows_dot<NT>(kf, qf);
+    const f32q_t dp = rows_dot<NT>(vf, dof);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int key = kb + 4 * G + r;
+      const bool valid = key < nkeys && (!causal || key <= myq);
+      const float p = valid ? expf(s[r] * scale - L) : 0.f;
+      s[r] = p * (dp[r] - dl) * scale;
+    }
+    mma_cols<NT>(kx, s, acc);
+  }
+  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
+  merge_store<NT>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf);
 }
 
 static bool f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
@@ -423,21 +415,33 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
-  // One launch while two would each leave much of the chip idle; with more blocks the registers that dQ then takes for dK/dV's
-  // sake cost more.  us, two | one: 6 heads x 256 x 48 (96 blocks) 17.3 | 11.3, 24 x 512 x 64 (768) 73 | 58, 64 x 300 x 64 (1216)
-  // 62 | 59, 24 x 1000 x 64 (1512) 160 | 163; 8 x 1000 x 128 (504) 142 | 132, 128 x 128 x 128 (1024) 71 | 81.
-  if ((int64_t)grid.x * grid.y <= (head_dim <= 64 ? 1024 : 512)) {
+  // One launch while two would each leave much of the chip idle, up to `most` blocks.  Of causal rows the late ones are the
+  // longest and end alone, so that the other kernel's blocks find room; with rows of more than 1024 there are too few of them,
+  // and without the mask all blocks end together and the one launch gains only while it is small.  Heads of 128 take 188
+  // registers in the one launch (dQ those of dK/dV), one block a CU, where the two have two and three.
+  // us, two | one, heads x length x head size (blocks): causal 6 x 256 x 48 (96) 14.7 | 9.2, 24 x 512 x 48 (768) 54 | 37,
+  // 24 x 512 x 64 (768) 72 | 59, 32 x 512 x 64 (1024) 1.16 times, 256 x 64 x 64 (1024) 0.96, 8 x 2048 x 64 (1024) 0.95,
+  // 6 x 2000 x 48 (750) 0.90, 8 x 1000 x 96 (504) 110 | 86, 12 x 512 x 128 (384) 1.25, 64 x 128 x 128 (512) 38 | 43,
+  // 4 x 2000 x 128 (500) 0.84; all keys 12 x 777 x 48 (588) 1.11, 128 x 128 x 48 (1024) 1.09, 12 x 1000 x 32 (756) 0.84,
+  // 64 x 128 x 96 (512) 1.04, 8 x 1000 x 96 (504) 139 | 149, 6 x 500 x 128 (192) 0.93, 8 x 1000 x 128 (504) 179 | 240.
+  const bool middling = seq >= 192 && seq <= 1024;
+  int64_t most;
+  if (!causal) most = head_dim <= 48 ? (seq < 512 ? 1024 : 640) : head_dim <= 112 ? (seq < 256 ? 512 : 448) : 128;
+  else if (head_dim <= 48) most = seq <= 1024 ? 1024 : 512;
+  else if (head_dim <= 64) most = middling ? 1024 : 512;
+  else most = head_dim <= 112 || middling ? 512 : 192;
+  if ((int64_t)grid.x * grid.y <= most) {
     EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                          hipLaunchKernelGGL(attn_bwd_f32_kernel<NT>, dim3(grid.x, grid.y, 2), dim3(64 * kWaves), 0, st, (const float*)q,
-                                             (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, (float*)dq,
-                                             (float*)dk, (float*)dv, shp, scale, causal));
+                          hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, true>), dim3(grid.x, grid.y, 2), dim3(64 * kWaves), 0, st,
+                                             (const float*)q, (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse,
+                                             nullptr, (float*)dq, (float*)dk, (float*)dv, shp, scale, causal));
     EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma)");
     return EMI_OK;
   }
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL(attn_bwd_dq_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q,
+                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, false>), grid, dim3(64 * kWaves), 0, st, (const float*)q,
                                            (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, delta,
-                                           (float*)dq, shp, scale, causal));
+                                           (float*)dq, nullptr, nullptr, shp, scale, causal));
   EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dq)");
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
                         hipLaunchKernelGGL(attn_bwd_dkv_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q,

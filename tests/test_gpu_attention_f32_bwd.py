@@ -11,7 +11,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("layout", ["bhsd", "bshd"])
-@pytest.mark.parametrize("B,h,S,d", [(4, 16, 256, 64), (4, 16, 257, 64), (1, 7, 31, 48), (2, 32, 128, 128), (2, 32, 129, 128), (1, 3, 47, 112)])
+@pytest.mark.parametrize("B,h,S,d", [(4, 16, 256, 64), (4, 16, 257, 64), (1, 7, 31, 48), (2, 32, 128, 128), (2, 32, 129, 128), (1, 3, 47, 112),
+                                     # heads of 128: rows of middling length, few short ones, few long ones; long rows of 48; without the mask
+                                     (2, 16, 255, 128), (2, 16, 257, 128), (1, 12, 128, 128), (1, 2, 1040, 128), (1, 8, 1030, 48), (1, 8, 1041, 48),
+                                     (1, 28, 256, 96), (1, 32, 255, 96), (1, 20, 512, 48), (3, 11, 512, 48)])
 def test_f32_attention_adjoint_as_one_launch_or_two(B, h, S, d, layout, causal):
     from enzyme_ad.jax import ops
     rng = np.random.default_rng(S * d + h)
