@@ -8,10 +8,12 @@
 // from 128 x 128 down to 32 x 32 (whose eight wavefronts share k), and a launcher that chooses by how the tiles divide over
 // the CUs (bf16_plan).  Eight wavefronts of 32 x 64 on a 128 x 128 tile read 1.5 times the LDS bytes of four of 64 x 64 and
 // are still faster: two of them on a SIMD hide each other's LDS and barrier latency.
-// Measured, us, against the two-stage 128 x 128 kernel of gemm.hip (k-contiguous B): 777 x 768 x 768 12.2 -> 5.5;
+// Measured with all operands in the caches, us, against the two-stage 128 x 128 kernel of gemm.hip (k-contiguous B): 777 x 768 x 768 12.2 -> 5.5;
 // 777 x 768 x 2048 18.7 -> 9.0; 64 x 768 x 768 9.9 -> 4.2; 300 x 5632 x 2048 23.2 -> 13.2; 1000 x 4096 x 4096 47.5 -> 37.0;
 // 8192 x 768 x 768 15.4 -> 15.2, x 2048 30.5 -> 29.1; 8192 x 2304 x 768 42.4 -> 37.1 (782 TFLOP/s); k-major B:
-// 777 x 768 x 768 15.5 -> 5.8; 1000 x 4096 x 4096 64.4 -> 36.6; 8192 x 768 x 2048 36.6 -> 30.4.
+// 777 x 768 x 768 15.5 -> 5.8; 1000 x 4096 x 4096 64.4 -> 36.6; 8192 x 768 x 2048 36.6 -> 30.4.  With weights from beyond the
+// L2s, as a model has them: 777 x 768 x 768 6.2, x 2048 9.9, 512 x 1024 x 1024 6.9, 300 x 5632 x 2048 14.7, 1000 x 2048 x 2048 15.3,
+// 1000 x 4096 x 4096 40, 8192 x 768 x 768 16.3, x 2048 33.
 #include <type_traits>
 #include <utility>
 
@@ -94,7 +96,7 @@ template <int ROWS, int BK, int NW, bool KM> struct PipeOperand {
 // WM x WN wavefronts tile the block's BM x BN; WK times as many share the k of every stage (k-step ks of 32 to the wavefronts
 // ks % WK) and are added in wavefront order at the end.  A wavefront alone on its SIMD issues an instruction every 7 to 8 cycles,
 // and a stage is forty for its loads and as many around its fragments and products: on few tiles that chain, and not the
-// loads (64 bytes a cycle and CU, 258 cycles for 64 x 64 x 64), set the time.  Twice the wavefronts and stages twice as long, us:
+// loads (64 bytes a cycle and CU, 258 cycles for 64 x 64 x 64), set the time.  Twice the wavefronts and stages twice as long, us, operands in the caches:
 // 777 x 768 x 768 6.8 -> 5.5, x 2048 13.5 -> 9.0; 512 x 1024 x 1024 7.6 -> 6.0; 300 x 5632 x 2048 15.2 -> 13.2; 1000 x 2048 x 2048
 // 14.5 -> 13.2; k-major B, three products summed: 777 x 768 x 768 14.8 -> 11.2.  part != nullptr: split-K, split z owns the stages
 // [z * steps_per_split, ...) of the contraction (of the whole sum, where products are summed) and leaves its tile in
@@ -393,20 +395,23 @@ static int launch_pipe_shape(hipStream_t st, const PipeCall& c, int trans_b) {
   return -1;
 }
 
-// Which block and how many splits of K.  The estimate is of the CU with the most blocks, in microseconds, with the rates
-// each block shape was measured at; shape 0 is the 256 x 256 ping-pong kernel of gemm.hip, whose clock falls as it fills
-// the chip (1.0 a stage of 64 k on one CU, 1.45 on all), 1 the 128 x 128 tile of which two fit a CU (0.61 alone, 0.90 two),
-// 2 the same tile in a ring of three stages whose k two wavefronts share (0.52, one to a CU), 3 128 x 64 (a stage of 128 k 0.62
-// alone, 1.24 two), 4 64 x 64 (a stage of 128 k 0.35 alone, 0.43 with B k-major, 0.68 two, 0.38 to 0.40 a block from three on, which also start one after
-// the other),
-// 5 a 32 x 32 tile whose eight wavefronts share stages of 256 k (0.30, one after the other).  The reduction over splits is a launch of its own;
-// results over 4 M elements, whose planes leave the caches, are not split (but see pingpong_splits of gemm.hip), nor are
-// the products of a few tokens, which have kernels of their own (gemm_skinny.hip).
+// Which block and how many splits of K.  The estimate is of the CU with the most blocks, in microseconds: a start, the stages
+// at the rate that each block shape was measured at with one, two, three and more blocks on the CU, the start of blocks that
+// come after others, and what several results in one launch cost more.  Shape 0 is the 256 x 256 ping-pong kernel of gemm.hip,
+// whose clock falls as it fills the chip, 1 the 128 x 128 tile of which two fit a CU, 2 the same tile in a ring of three stages
+// whose k two wavefronts share, one to a CU, 3 128 x 64, 4 64 x 64, both in stages of 128 k, 5 a 32 x 32 tile whose eight
+// wavefronts share stages of 256 k.  Fitted to 666 products of 16 to 8192 tokens whose weights, 64 MB of them in turn, come
+// from beyond the L2s, each with every block and number of splits: 0.6 % behind the fastest of them in the geometric mean.
+// The reduction over splits is a launch of its own; results over 4 M elements, whose planes leave the caches, are not split
+// (but see pingpong_splits of gemm.hip), nor are the products of a few tokens, which have kernels of their own
+// (gemm_skinny.hip).  A split of 64 x 64 tiles has at least 384 k, as the reduction costs as much as 8 of its stages (us, splits
+// of 512 | 384 k at least, B k-major, summed: 16 x 1024 x 1024 x 3 8.5 | 8.0, 16 x 288 x 768 x 2 7.4 | 7.0).
 Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b, int64_t most) {
-  struct Shape { int bm, bn, bk; double fixed, rate[3], more; };        // rate[b - 1]: per stage, b blocks on the CU; more: per block from four on
-  static const Shape shapes[6] = {{256, 256, 64, 4.0, {1.0, 2.0, 3.0}, 1.0},   {128, 128, 64, 4.0, {0.61, 0.90, 1.45}, 0.50},
-                                  {128, 128, 64, 4.0, {0.52, 1.04, 1.56}, 0.52}, {128, 64, 128, 3.2, {0.62, 1.24, 2.0}, 0.66},
-                                  {64, 64, 128, 3.4, {0.35, 0.68, 1.14}, 0.40},  {32, 32, 256, 3.4, {0.30, 0.62, 0.95}, 0.33}};
+  struct Shape { int bm, bn, bk; double fixed, group, rate[3], more; };      // rate[b - 1]: per stage, b blocks on the CU; more: per block
+                                                                            // from four on; group: more with several results
+  static const Shape shapes[6] = {
+      {256, 256, 64, 4.0, 0.8, {1.0, 2.0, 3.0}, 1.0},    {128, 128, 64, 3.9, 0.2, {0.59, 0.855, 1.6}, 0.515}, {128, 128, 64, 4.3, 0.8, {0.535, 1.07, 1.6}, 0.535},
+      {128, 64, 128, 3.45, 0.45, {0.6, 1.24, 2.0}, 0.6}, {64, 64, 128, 3.15, 0.2, {0.355, 0.785, 1.10}, 0.41}, {32, 32, 256, 3.4, 0.0, {0.30, 0.62, 1.4}, 0.363}};
   Bf16Plan best{1, 1, 0.0};
   double least = 1e30;
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && M > 8 && K > 8;
@@ -417,13 +422,13 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
     const int64_t blocks = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * (sum ? 1 : count);
     if (blocks > 0x3fffffff) continue;
     const bool split = may_split && (c != 0 || trans_b);
-    for (int64_t z = 1; z <= 16 && z <= most && (z == 1 || (split && steps >= 4 * z)); z++) {
+    for (int64_t z = 1; z <= 16 && z <= most && (z == 1 || (split && steps >= (c == 4 ? 3 : 4) * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
       double stage = b < 4 ? s.rate[b - 1] : s.more * b;
-      if (c == 4 && b == 1 && !trans_b) stage = 0.43;
-      const double later = c == 4 && b > 2 ? 1.0 * (b - 2) : c == 5 ? 1.8 * (b - 1) : 0.0;      // the start of blocks that come after others
+      if (c == 4 && !trans_b) stage = b == 1 ? 0.385 : b == 3 ? 1.14 : stage;
+      const double later = c == 4 && b > 2 ? 1.0 * (b - 2) : c == 5 ? 1.75 * (b - 1) : 0.0;     // the start of blocks that come after others
       if (c == 0) stage *= 1.0 + 0.45 * (blocks * z < 256 ? blocks * z / 256.0 : 1.0);
-      const double t = s.fixed + later + per * stage + (z > 1 ? 3.0 + 0.7e-6 * M * N * (z + 1) : 0.0);
+      const double t = s.fixed + (count > 1 && !sum ? s.group : 0.0) + later + per * stage + (z > 1 ? 2.8 + 0.78e-6 * M * N * (z + 1) : 0.0);
       if (t < least) {
         least = t;
         best = Bf16Plan{c, (int)z, t};
@@ -431,6 +436,23 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
     }
   }
   return best;
+}
+
+// The kernel of a plan's blocks: 0 the ping-pong kernel, 1, 2 blocks of 128 x 128, 3, 4 of 128 x 64, 5 to 7 of 64 x 64, 8 of
+// 32 x 32.
+// Deeper rings, of stages of 128 k, where a block has its CU to itself and enough stages to fill them; 64 x 64 blocks of four
+// wavefronts and 64 k a stage, three of which fit a CU, where three there are.  us, ring of two | three, 64 x 64: 300 x 768 x 768
+// 6.7 | 6.1 (B k-major), 300 x 2816 x 1024 8.2 | 7.1, 256 x 2048 x 768 6.9 | 6.2, 300 x 1408 x 512 5.5 | 5.0, with B k-major
+// 5.8 | 5.4, 512 x 512 x 512 with B k-major 5.0 | 5.3; 128 x 64, of 64 k and eight wavefronts | of 128 and sixteen: 512 x 768 x 768 (three) 9.1 | 8.4,
+// 2048 x 768 x 288 5.5 | 6.2, 1000 x 1408 x 512 6.6 | 6.9; 64 x 64, of 128 | of 64 k, three to a CU: 1500 x 512 x 512 (three) 9.7 | 9.2.
+int bf16_kernel(const Bf16Plan& plan, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b) {
+  if (plan.shape < 3) return plan.shape;
+  if (plan.shape == 5) return 8;
+  const int rows = plan.shape == 3 ? 128 : 64;
+  const int64_t blocks = (M + rows - 1) / rows * ((N + 63) / 64) * (sum || count == 1 ? plan.splits : count), all_k = K * (sum ? count : 1);
+  if (plan.shape == 3) return blocks <= 256 && all_k > 640 * plan.splits ? 4 : 3;
+  if (blocks <= 256 && all_k >= (trans_b || N > 768 ? 512 : 640)) return 6;
+  return blocks > 512 && blocks <= 768 ? 7 : 5;
 }
 
 // C[i] = A[i] . op(B[i]) [+ R[i]] for i < count, or with `sum` the one sum of the products (+ R[0]), as the plan says
@@ -451,16 +473,14 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
   g.sum = sum;
   const PipeCall c{g.A[0], g.B[0], g.R[0], g.C[0], M, N, K, lda, ldb, ldr, ldc, vec_ok, part, part != nullptr ? plan.splits : 1,
                    count > 1 ? &g : nullptr, planes};
-  // With no more than one block to a CU and more than a few stages, deeper rings, which then fit (us, the ring of two | three:
-  // 777 x 768 x 768 5.5 | 5.5, x 2048 9.2 | 9.0, k-major B, three summed 14.1 | 11.2; 4096 x 512 x 512 6.5 | 7.0).
-  const int rows = plan.shape == 3 ? 128 : 64;
-  const int64_t blocks = (int64_t)((M + rows - 1) / rows) * ((N + 63) / 64) * (sum || count == 1 ? c.splits : count);
-  const bool single = blocks <= 256 && (int64_t)K * (sum ? count : 1) > 1024;
-  switch (plan.shape) {
+  switch (bf16_kernel(plan, M, N, K, count, sum, trans_b)) {
     case 1: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 2>(st, c, trans_b);
     case 2: return launch_pipe_shape<128, 128, 4, 2, 2, 64, 3>(st, c, trans_b);
-    case 3: return single ? launch_pipe_shape<128, 64, 4, 2, 2, 128, 3>(st, c, trans_b) : launch_pipe_shape<128, 64, 4, 2, 1, 64, 3>(st, c, trans_b);
-    case 4: return single ? launch_pipe_shape<64, 64, 2, 2, 2, 128, 3>(st, c, trans_b) : launch_pipe_shape<64, 64, 2, 2, 2, 128, 2>(st, c, trans_b);
+    case 3: return launch_pipe_shape<128, 64, 4, 2, 1, 64, 3>(st, c, trans_b);
+    case 4: return launch_pipe_shape<128, 64, 4, 2, 2, 128, 3>(st, c, trans_b);
+    case 5: return launch_pipe_shape<64, 64, 2, 2, 2, 128, 2>(st, c, trans_b);
+    case 6: return launch_pipe_shape<64, 64, 2, 2, 2, 128, 3>(st, c, trans_b);
+    case 7: return launch_pipe_shape<64, 64, 2, 2, 1, 64, 3>(st, c, trans_b);
     default: return launch_pipe_shape<32, 32, 1, 1, 8, 256, 3>(st, c, trans_b);
   }
 }

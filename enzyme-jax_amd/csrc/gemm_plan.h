@@ -22,6 +22,7 @@ struct F32Plan {
 // 60 | 104, 512 x 768 x 32000 89 | 238; fp32: 256 x 4096 x 11008 247 | 677, 512 x 768 x 32000 330 | 1955).
 constexpr int64_t kAnySplits = 1 << 20;
 Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b, int64_t most);      // gemm_bf16_pipe.hip
+int bf16_kernel(const Bf16Plan& plan, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b);
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most);        // gemm_f32.hip
 
 inline int64_t splits_held(const void* workspace, size_t bytes, int64_t M, int64_t N) {

@@ -17,19 +17,28 @@ def _check(got, ref, mag, n, what):
     assert np.all(err <= bound), "%s: worst error / bound %.2f" % (what, float(np.max(err / bound)))
 
 
-@pytest.mark.parametrize("tb", [1, 0])
-@pytest.mark.parametrize("M,N,K,count", [
+# what each is there for; tests/test_host_boundary.py holds them to reaching every kernel
+SIZES = [
     (9, 8, 8, 2),             # less than one piece of every stage
     (33, 24, 264, 3),         # 32-tiles whose wavefronts share k (k-contiguous B), one piece past a stage
     (64, 768, 768, 3),        # exact 32-tiles
     (40, 104, 8200, 2),       # few tiles, long contraction: splits, a ragged last stage
-    (300, 1400, 520, 2),      # 64-tiles, ragged rows and columns
-    (777, 2040, 776, 2),      # 128 x 64 tiles, ragged
+    (300, 1400, 520, 2),      # 64-tiles in a ring of three stages, ragged rows and columns
+    (300, 2808, 1032, 2),     # a group: 64-tiles, two to a CU, in a ring of two
+    (1500, 504, 512, 3),      # a group: 64-tiles of 64 k a stage, three to a CU (k-contiguous B)
+    (30, 2800, 504, 12),      # the same, k-major B
+    (777, 2040, 776, 2),      # 128 x 64 tiles of 128 k a stage, ragged
     (1000, 4088, 520, 2),     # 128-tiles, three stages
-    (3000, 1032, 328, 2),     # 128-tiles, two to a CU; summed: one pass over both
-    (600, 2056, 4104, 2),     # splits; summed: splits that straddle the products
-    (300, 1000, 16392, 2),    # 256-tiles with splits (k-contiguous B)
-])
+    (3000, 1032, 328, 2),     # 128 x 64 tiles of 64 k a stage; a group: 128-tiles, two to a CU; summed: one pass over both
+    (600, 2056, 4104, 2),     # 128-tiles with splits; summed: splits that straddle the products
+    (300, 1000, 16392, 2),    # 64-tiles and 128 x 64 with splits
+    (1000, 2056, 8200, 1),    # 256-tiles with splits (k-contiguous B)
+    (2056, 2048, 8200, 1),    # more than 4 M results: 256-tiles with splits all the same (k-contiguous B)
+]
+
+
+@pytest.mark.parametrize("tb", [1, 0])
+@pytest.mark.parametrize("M,N,K,count", SIZES)
 def test_bf16_tiles_stages_and_splits(tb, M, N, K, count):
     from enzyme_ad.jax import ops
     rng = np.random.default_rng(M + 3 * N + 7 * K + tb)

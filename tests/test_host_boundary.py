@@ -102,6 +102,26 @@ def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K
     assert need >= free.splits * M * N * 4
 
 
+def test_the_sizes_of_the_bf16_gpu_test_reach_every_kernel():
+    """Whatever the estimates are fitted to: each kernel runs there, both ways of storing B, and with splits those that have
+    them (blocks of 32 x 32 take a k-contiguous B only)."""
+    from test_gpu_gemm_bf16_shapes import SIZES
+    lib = _lib()
+    plan, kernel = lib._ZN3emi9bf16_planEllliiil, lib._ZN3emi11bf16_kernelERKNS_8Bf16PlanEllliii
+    plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
+    kernel.restype, kernel.argtypes = C.c_int, [C.POINTER(_Plan)] + [C.c_int64] * 3 + [C.c_int] * 3
+    ran, split = set(), set()
+    for M, N, K, count in SIZES:
+        for tb in (1, 0):
+            for n, total in ((1, 0), (count, 0), (count, 1)):
+                p = plan(M, N, K, n, total, tb, 1 << 20)
+                ran.add((kernel(C.byref(p), M, N, K, n, total, tb), tb))
+                if p.splits > 1:
+                    split.add(p.shape)
+    assert {k for k, tb in ran if tb} == set(range(9)) and {k for k, tb in ran if not tb} >= set(range(1, 8))
+    assert split >= {0, 1, 2, 3, 4, 5}
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 688, 5689), (4, 64, 20000), (8, 4096, 4096)])
 def test_a_few_rows_of_a_gradient_are_split(M, N, K):
     """dW = dY^T . X of a few columns of dY is no product of a few tokens: nothing else splits its long contraction."""
