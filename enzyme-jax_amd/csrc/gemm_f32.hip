@@ -339,9 +339,9 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 // long epilogue); results over 4 M elements, whose planes
 // leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few
 // rows of a k-major A are no such product (4 x 64 x 20000, us: 126 in one pass, 12 split).
-struct F32Shape { int bm, bn, bk, config; };
+struct F32Shape { int bm, bn, bk; };
 constexpr int kF32Shapes = 5;
-static const F32Shape kF32Shape[kF32Shapes] = {{64, 64, 32, 1}, {32, 32, 64, 2}, {128, 128, 32, 0}, {128, 64, 32, 1}, {64, 64, 32, 1}};   // two fp32, three bf16
+static const F32Shape kF32Shape[kF32Shapes] = {{64, 64, 32}, {32, 32, 64}, {128, 128, 32}, {128, 64, 32}, {64, 64, 32}};   // two fp32, three bf16
 
 // Microseconds of the products in blocks of shape c over z splits; not finite where it cannot be.
 static double f32_estimate(int c, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t z) {
@@ -366,7 +366,7 @@ static double f32_estimate(int c, int64_t M, int64_t N, int64_t K, int count, in
 }
 
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
-  F32Plan best{2, 1, 0.0};
+  F32Plan best{1, 1, 0.0};
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && (M > 8 || trans_a) && K > 8;
   double least = 1e30;
   for (int c = 0; c < kF32Shapes; c++)
@@ -374,23 +374,9 @@ F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_
       const double t = f32_estimate(c, M, N, K, count, sum, trans_a, z);
       if (t < least) {
         least = t;
-        best = F32Plan{kF32Shape[c].config, (int)z, t};
+        best = F32Plan{c, (int)z, t};
       }
     }
-  return best;
-}
-
-// Which of the shapes of the plan's blocks.
-static int f32_shape(const F32Plan& p, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a) {
-  int best = 1;
-  double least = 1e30;
-  for (int c = 0; c < kF32Shapes; c++) {
-    const double t = kF32Shape[c].config == p.config ? f32_estimate(c, M, N, K, count, sum, trans_a, p.splits) : 1e30;
-    if (t < least) {
-      least = t;
-      best = c;
-    }
-  }
   return best;
 }
 
@@ -434,11 +420,10 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
                   p.splits, count > 1 ? &g : nullptr, planes};
   // (the split kernels address a tile of the result with 31 bits too)
   const bool wide = 128 * ldc >= 0x1fffffff || 128 * N >= 0x1fffffff || (R != nullptr && 128 * ldr >= 0x1fffffff);
-  const int shape = f32_shape(p, M, N, K, count, sum, trans_a);
-  switch (wide && shape > 1 ? 0 : shape) {
+  switch (wide && p.shape > 1 ? 0 : p.shape) {
     case 0: return launch_f32_shape<64, 64, 2, 2, 1, 32, 2>(st, c, trans_a, trans_b);
     case 1: return launch_f32_shape<32, 32, 1, 1, 8, 64, 5>(st, c, trans_a, trans_b);
-    default: return launch_f32_bf16x3(st, c, shape - 2, trans_a, trans_b);
+    default: return launch_f32_bf16x3(st, c, p.shape - 2, trans_a, trans_b);
   }
 }
 

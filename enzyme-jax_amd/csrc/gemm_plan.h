@@ -11,7 +11,8 @@ struct Bf16Plan {
   double us;        // the estimate
 };
 struct F32Plan {
-  int config;       // 0: blocks of 128 x 128, 1: of 64 columns, 2: 32 x 32 (gemm_f32.hip)
+  int shape;        // on the fp32 instructions 0: blocks of 64 x 64, 1: 32 x 32 (gemm_f32.hip); on the bf16 instructions 2: 128 x 128,
+                    // 3: 128 x 64, 4: 64 x 64 (gemm_f32_split.hip)
   int splits;
   double us;
 };

@@ -88,12 +88,12 @@ def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K
     the 256 CUs, or the smallest ones there are.  With room for some planes there are at most as many splits."""
     lib = _lib()
     plan, blocks, trans = ((lib._ZN3emi9bf16_planEllliiil, [(256, 256), (128, 128), (128, 128), (128, 64), (64, 64), (32, 32)], 1)
-                           if dtype == "bf16" else (lib._ZN3emi8f32_planEllliiil, [(128, 128), (64, 64), (32, 32)], 0))      # of B, of A
+                           if dtype == "bf16" else (lib._ZN3emi8f32_planEllliiil, [(64, 64), (32, 32), (128, 128), (128, 64), (64, 64)], 0))      # of B, of A
     plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
     tiles = lambda p: -(-M // blocks[p.shape][0]) * -(-N // blocks[p.shape][1])
     free, one = (plan(M, N, K, count, total, trans, most) for most in (1 << 20, 1))
     assert free.splits > 1 and one.splits == 1
-    assert tiles(one) >= 128 or (tiles(one) > tiles(free) and one.shape == len(blocks) - 1)
+    assert tiles(one) >= 128 or (tiles(one) > tiles(free) and blocks[one.shape] == (32, 32))
     for most in range(2, free.splits + 2):
         assert 1 <= plan(M, N, K, count, total, trans, most).splits <= most
     code = 16 if dtype == "bf16" else 11
