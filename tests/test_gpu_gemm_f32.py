@@ -16,17 +16,26 @@ def _check(got, ref, bound, what):
     assert np.all(err <= bound), "%s: worst error / bound %.2f" % (what, float(np.max(err / bound)))
 
 
-@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K,count", [
+# what each is there for; tests/test_host_boundary.py holds them to reaching every kernel
+SIZES = [
     (4, 4, 4, 2),            # less than one piece of every stage
     (32, 32, 64, 3),         # exactly one 32-tile and one stage
     (36, 28, 68, 3),         # a ragged row of tiles, one piece past a stage
     (100, 512, 516, 3),      # 32-tiles, ragged rows
     (12, 20, 20004, 2),      # a single tile: splits of a long contraction, ragged last stage
-    (704, 2812, 1028, 2),    # 64-tiles, ragged columns
-    (1996, 772, 2052, 2),    # 64-tiles, splits; summed: splits that straddle the products
-    (2052, 2044, 68, 2),     # 128-tiles, ragged both ways
-])
+    (260, 1028, 772, 2),     # 64-tiles of the fp32 instructions, splits
+    (704, 2812, 1028, 2),    # ragged columns: 64-tiles of the bf16 instructions; a group: of the fp32 ones
+    (708, 1540, 292, 2),     # 128 x 64, ragged both ways
+    (1996, 772, 2052, 2),    # 128-tiles, splits; summed: splits that straddle the products
+    (2052, 2044, 68, 2),     # 64-tiles of the fp32 instructions, ragged both ways
+    (1412, 260, 772, 3),     # a group: 128 x 64; summed: its splits straddle the products
+    (516, 772, 2052, 2),     # a group: 64-tiles of the bf16 instructions
+    (1004, 772, 516, 2),     # summed: 64-tiles of the bf16 instructions
+]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,count", SIZES)
 def test_f32_tiles_stages_and_splits(ta, tb, M, N, K, count):
     from enzyme_ad.jax import ops
     rng = np.random.default_rng(M + 3 * N + 7 * K + 2 * ta + tb)

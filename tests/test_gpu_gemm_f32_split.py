@@ -9,8 +9,15 @@ from gpu_util import dev, host
 
 pytestmark = pytest.mark.gpu
 
-# blocks of 64 x 64; of 128 x 64 with fewer stages than are in flight; of 128 x 128, two splits
-SIZES = [(1000, 1028, 1036), (2052, 2044, 68), (1996, 772, 2052)]
+# what each is there for; tests/test_host_boundary.py holds them to reaching every kernel
+SIZES = [
+    (900, 1028, 2052),       # blocks of 64 x 64, a last round of one stage
+    (1004, 772, 36),         # the same where A is k-contiguous, no more stages than are in flight
+    (516, 2052, 28),         # 128 x 64, fewer stages than are in flight
+    (900, 1284, 1036),       # the same, three splits
+    (2004, 1540, 36),        # 128 x 128, fewer stages than are in flight
+    (708, 1092, 2052),       # the same, four splits
+]
 
 
 def _operands(rng, M, N, K, ta, tb):
@@ -18,7 +25,7 @@ def _operands(rng, M, N, K, ta, tb):
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", SIZES + [(1060, 1092, 2052), (4100, 2052, 36), (777, 4096, 772)])
+@pytest.mark.parametrize("M,N,K", SIZES + [(1000, 1028, 1036), (1996, 772, 2052), (1060, 1092, 2052), (777, 4096, 772)])
 def test_errors_of_an_fp32_product(ta, tb, M, N, K):
     """Within (K + 2) 2^-23 sum |a b|, as any order of fp32 sums is (three dropped products of 2^-25 each are less than what
     the roundings of a shorter chain leave of it), and in the mean square no further off than chains of 64 terms."""
@@ -37,7 +44,7 @@ def test_errors_of_an_fp32_product(ta, tb, M, N, K):
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0)])
 @pytest.mark.parametrize("M,N,K", SIZES)
-@pytest.mark.parametrize("what", ["infinite", "nan", "huge", "tiny", "tiny rows", "zero"])
+@pytest.mark.parametrize("what", ["infinite", "nan", "huge", "tiny", "tiny rows", "tiny products", "denormal", "zero"])
 def test_numbers_that_do_not_split(what, ta, tb, M, N, K):
     from enzyme_ad.jax import ops
     rng = np.random.default_rng(M + N + K + 2 * ta + tb)
@@ -56,6 +63,12 @@ def test_numbers_that_do_not_split(what, ta, tb, M, N, K):
         a *= np.float32(1e-36)
     elif what == "tiny rows":                                   # beside ordinary ones
         a[(slice(None), slice(5, 9)) if ta else slice(5, 9)] *= np.float32(1e-36)
+    elif what == "tiny products":                               # of numbers that split
+        a *= np.float32(1e-20)
+        b *= np.float32(1e-21)
+    elif what == "denormal":                                    # and exactly a bf16 number
+        a = np.copysign(np.float32(2.0 ** -130), a)
+        b *= np.float32(1e10)
     else:
         a[:] = 0
     A, B = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()

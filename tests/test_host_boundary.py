@@ -122,6 +122,29 @@ def test_the_sizes_of_the_bf16_gpu_test_reach_every_kernel():
     assert split >= {0, 1, 2, 3, 4, 5}
 
 
+def test_the_sizes_of_the_f32_gpu_tests_reach_every_kernel():
+    """As above: both instructions' blocks, A k-contiguous and k-major, for one product, a group and a sum; in the test of numbers that
+    do not split every kernel on the bf16 instructions, whole and with splits, and one with less than the stages in flight."""
+    import test_gpu_gemm_f32
+    import test_gpu_gemm_f32_split
+    lib = _lib()
+    plan = lib._ZN3emi8f32_planEllliiil
+    plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
+
+    def ran(sizes, n, total, ta):
+        plans = [(plan(M, N, K, n or count, total, ta, 1 << 20), K) for M, N, K, count in sizes]
+        return {p.shape for p, _ in plans}, {p.shape for p, _ in plans if p.splits > 1}, {p.shape for p, K in plans if K <= (64 if p.shape == 2 else 32)}
+
+    for ta in (0, 1):
+        sizes = test_gpu_gemm_f32.SIZES
+        one, one_split, _ = ran(sizes, 1, 0, ta)
+        both, both_split, _ = ran(sizes, 0, 1, ta)
+        assert one == set(range(5)) and ran(sizes, 0, 0, ta)[0] == set(range(5)) and both == set(range(5))
+        assert one_split >= {0, 1, 2} and both_split >= {0, 1, 2, 3}
+        kernels, split, few = ran([s + (1,) for s in test_gpu_gemm_f32_split.SIZES], 1, 0, ta)
+        assert kernels >= {2, 3, 4} and split >= {2, 3} and few >= {2, 3}
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 688, 5689), (4, 64, 20000), (8, 4096, 4096)])
 def test_a_few_rows_of_a_gradient_are_split(M, N, K):
     """dW = dY^T . X of a few columns of dY is no product of a few tokens: nothing else splits its long contraction."""
