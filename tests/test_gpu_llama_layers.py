@@ -37,7 +37,18 @@ def _reference(xr, wr, dyr, layers, heads):
     return h, d, grads
 
 
-@pytest.mark.parametrize("dt,dim,hidden,layers,heads,batch,seq,pending", [
+# products split over K whose planes the next RMSNorm (or, in reverse, its adjoint) adds up; tests/test_host_boundary.py holds them to that
+SPLIT_SIZES = [
+    ("bf16", 1024, 2816, 2, 8, 1, 257, None),     # w2: a wavefront to a row
+    ("bf16", 2048, 5632, 2, 16, 2, 65, None),     # w2: 256 threads to a row
+    ("bf16", 4096, 264, 1, 32, 1, 77, None),      # wo, two pieces a thread
+    ("bf16", 2048, 8200, 2, 16, 2, 515, None),    # w2 in 256-tiles
+    ("f32", 1032, 2824, 2, 43, 1, 33, None),      # wo and w2, 256 threads to a row of 129 pairs of pieces
+]
+
+
+@pytest.mark.parametrize("dt,dim,hidden,layers,heads,batch,seq,pending", SPLIT_SIZES + [
+    ("f32", 32, 24, 51, 2, 1, 9, None),       # more norms in a group than one launch sums
     ("f32", 64, 72, 5, 2, 1, 33, 2),          # groups of two: the second one's first dy lies in the last slot of the first
     ("f32", 288, 768, 3, 6, 1, 9, None),
     ("f32", 128, 264, 2, 2, 3, 77, 1),        # one layer's cotangents at a time

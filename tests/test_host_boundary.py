@@ -145,6 +145,20 @@ def test_the_sizes_of_the_f32_gpu_tests_reach_every_kernel():
         assert kernels >= {2, 3, 4} and split >= {2, 3} and few >= {2, 3}
 
 
+def test_the_layers_whose_norms_add_planes_have_split_products():
+    from test_gpu_llama_layers import SPLIT_SIZES
+    lib = _lib()
+    split = []
+    for dt, D, H, layers, _, batch, seq, _ in SPLIT_SIZES:
+        plan = lib._ZN3emi9bf16_planEllliiil if dt == "bf16" else lib._ZN3emi8f32_planEllliiil
+        plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
+        T, trans = batch * seq, int(dt == "bf16")                                                     # of the weight, of fp32 activations
+        split.append([plan(T, D, K, 1, 0, trans, 1 << 20) for K in [D] + [H] * (layers > 1)])          # wo; w2 before another layer
+        sums = [plan(T, D, K, n, 1, 0, 1 << 20) for K, n in ((H, 2), (D, 3))]                          # the weights read in place
+        assert any(p.splits > 1 for p in split[-1]) and any(p.splits > 1 for p in sums)
+    assert split[2][0].splits > 1 and split[4][0].splits > 1 and (split[3][1].shape, split[3][1].splits > 1) == (0, True)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 688, 5689), (4, 64, 20000), (8, 4096, 4096)])
 def test_a_few_rows_of_a_gradient_are_split(M, N, K):
     """dW = dY^T . X of a few columns of dY is no product of a few tokens: nothing else splits its long contraction."""
