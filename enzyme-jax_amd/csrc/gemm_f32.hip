@@ -7,7 +7,7 @@
 // of what the LDS delivers in that time to four SIMDs.  On few tiles what counts is that loads are in flight all the time and
 // that every CU has the same share of the work.  So: a ring of NST LDS stages of BK k each, filled by direct-to-LDS loads
 // (16 bytes a lane, no staging registers) NST - 1 stages ahead, one barrier per stage, and blocks of 64 x 64, or of 32 x 32
-// whose eight wavefronts share k.  Measured, us (NT / NN / TN form): 256 x 288 x 288 4.9 / 5.4 / 4.9; 256 x 288 x 768 7.3;
+// whose eight wavefronts share k (128 x 128 where a contraction is one stage).  Measured, us (NT / NN / TN form): 256 x 288 x 288 4.9 / 5.4 / 4.9; 256 x 288 x 768 7.3;
 // 256 x 768 x 768 7.8.  What is left is the latency of the first loads and the launch.
 #include <type_traits>
 
@@ -326,43 +326,44 @@ static int launch_f32_shape(hipStream_t st, const F32Call& c, int trans_a, int t
 }
 
 // Which block and how many splits.  The estimate is of the CU with the most blocks, in microseconds: a start, which grows
-// with the blocks that come after one another, and the stages at the rate that each block shape was measured at.
-// The fp32 instructions: a stage of 32 k of a 64 x 64 tile takes 0.64 alone, 1.1 for two blocks and 0.485 a block from four on,
-// a stage of 64 k of a 32 x 32 tile whose wavefronts share k 0.40 alone, 0.32 a block from four on; the start of a further
-// block is 0.65 and 1.2.  The bf16 instructions (gemm_f32_split.hip), a stage of 32 k: 1.0, 0.82 and 0.56 for one block of
-// 128 x 128, 128 x 64 and 64 x 64 on a CU, 1.0, 0.58 and 0.34 a block for more, and 0.37, 0.25 and 0.17 more for each block
-// that the chip has per CU (its clock falls as it fills; 0.37, 0.12 and 0.03 up to one); their start is dearer (6.0, 3.8, 3.3; 1.0 more from a k-major A).
-// So the fp32 instructions keep what has few stages or few rows, us, 32- or 64-tiles | the best of the others: 256 x 768 x 768
-// 7.8 | 16, 512 x 768 x 768 12.5 | 14.7, 777 x 512 x 1408 18.7 | 19.3, 768 x 768 x 32 (TN) 5.0 | 5.5; and beyond: 2000 x 768 x 768
-// 33 | 25.6, 2000 x 768 x 2048 62 | 48, 768 x 768 x 4096 (TN, four) 208 | 146, 4096^3 1025 | 732.
-// The reduction over splits is a launch of its own (3, plus its planes at 4 TB/s; 1 more where it follows a split kernel's
-// long epilogue); results over 4 M elements, whose planes
-// leave the caches, and the products of a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few
-// rows of a k-major A are no such product (4 x 64 x 20000, us: 126 in one pass, 12 split).
+// with the blocks that come after one another, and the stages at the rate of each block shape; a stage on the bf16 instructions
+// takes longer the more blocks the chip has per CU, as its clock falls while it fills, and of a k-major A.  Fitted to 4000
+// products of 16 to 4096 tokens by weights of 288 x 288 to 4096 x 11008, 64 MB of them in turn from beyond the L2s, each with the
+// blocks and splits that could be the fastest: 0.2 % behind the fastest of them in the geometric mean and 14 % at the worst
+// (0.9 and 26 % with rates taken at a few sizes with operands in the caches).  The fp32 blocks of 128 x 128 are for weight
+// gradients of one stage: 12 of 1024 x 1024 x 19 17.8 us, 18.9 in blocks of 64 x 64, four of 2048 x 2048 x 24 21.6 | 23.4.
+// The fp32 instructions keep what has few stages or few rows, us, the better of their blocks | of the others: 256 x 768 x 768
+// 7.8 | 16, 840 x 768 x 768 17.2 | 18.4, 362 x 2048 x 768 17.5 | 19.5, 768 x 2048 x 36 (TN) 6.7 | 7.3; and beyond: 693 x 768 x 768 17.1 | 17.1,
+// 1136 x 768 x 768 19.9 | 19.6, 2056 x 768 x 768 30.9 | 26.1, 180 x 11008 x 4096 167 | 137, 3122 x 768 x 288 (two) 33.8 | 29.
+// The reduction over splits is a launch of its own; results over 4 M elements, whose planes leave the caches, and the products of
+// a few tokens, which have kernels of their own (gemm_skinny.hip), are not split; a few rows of a k-major A are no such product
+// (4 x 64 x 20000, us: 126 in one pass, 12 split).
 struct F32Shape { int bm, bn, bk; };
-constexpr int kF32Shapes = 5;
-static const F32Shape kF32Shape[kF32Shapes] = {{64, 64, 32}, {32, 32, 64}, {128, 128, 32}, {128, 64, 32}, {64, 64, 32}};   // two fp32, three bf16
+constexpr int kF32Shapes = 6;                             // three of the fp32 instructions, three of the bf16
+static const F32Shape kF32Shape[kF32Shapes] = {{64, 64, 32}, {32, 32, 64}, {128, 128, 32}, {128, 128, 32}, {128, 64, 32}, {64, 64, 32}};
 
 // Microseconds of the products in blocks of shape c over z splits; not finite where it cannot be.
 static double f32_estimate(int c, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t z) {
   struct Fp32 { double one, base, block, rate[4]; };      // start of one block, of b: base + b block; rate[b - 1]: per stage, b blocks on
                                                           // the CU; the last one per block
-  static const Fp32 fp32[2] = {{3.4, 4.0, 0.65, {0.64, 1.10, 1.50, 0.485}}, {3.4, 2.5, 1.2, {0.40, 0.69, 1.00, 0.32}}};
-  struct Bf16 { double base, block, one, one_fill, rate, fill; };
-  static const Bf16 bf16[3] = {{1.6, 4.4, 1.0, 0.37, 1.0, 0.37}, {2.0, 1.8, 0.82, 0.12, 0.58, 0.25}, {1.2, 2.1, 0.56, 0.03, 0.34, 0.17}};
+  static const Fp32 fp32[3] = {{3.4, 3.25, 0.75, {0.68, 1.10, 1.615, 0.496}}, {3.2, 2.1, 1.16, {0.405, 0.69, 0.995, 0.35}},
+                               {6.3, 4.0, 2.3, {2.01, 3.76, 5.94, 1.95}}};
+  struct Bf16 { double base, block, one, one_fill, rate, fill; };        // per stage, one block on the CU | each of several; _fill: times blocks per CU of the chip
+  static const Bf16 bf16[3] = {{3.2, 4.35, 0.76, 0.59, 0.975, 0.377}, {3.6, 1.6, 0.687, 0.228, 0.532, 0.25}, {2.3, 2.15, 0.511, 0.159, 0.359, 0.128}};
   const F32Shape& s = kF32Shape[c];
   const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
   const int64_t blocks = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * (sum ? 1 : count);
   if (blocks > 0x3fffffff || (z > 1 && steps < 4 * z)) return 1e30;
   const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
-  if (c < 2) {
+  const double several = count > 1 && !sum ? 0.6 : 0.0;   // results in one launch
+  if (c < 3) {
     const Fp32& r = fp32[c];
-    return (b == 1 ? r.one : r.base + r.block * b) + per * (b < 4 ? r.rate[b - 1] : r.rate[3] * b) + (z > 1 ? 3.0 + 1e-6 * M * N * (z + 1) : 0.0);
+    return (b == 1 ? r.one : r.base + r.block * b) + several + per * (b < 4 ? r.rate[b - 1] : r.rate[3] * b) +
+           (z > 1 ? 2.8 + 1e-6 * M * N * (z + 1) : 0.0);
   }
-  const Bf16& r = bf16[c - 2];
-  const double t = r.base + r.block * b + (trans_a ? 1.0 : 0.0) +
-                   per * ((b == 1 ? r.one : r.rate * b) + (b == 1 ? r.one_fill : r.fill) * (blocks * z / 256.0));
-  return 1.04 * (t + (z > 1 ? 4.0 + 1e-6 * M * N * (z + 1) : 0.0));       // near the line the fp32 instructions stay
+  const Bf16& r = bf16[c - 3];
+  const double stage = (b == 1 ? r.one : r.rate * b) + (b == 1 ? r.one_fill : r.fill) * (blocks * z / 256.0);
+  return r.base + r.block * b + several + (trans_a ? 1.06 : 1.0) * per * stage + (z > 1 ? 3.7 + 0.5e-6 * M * N * (z + 1) : 0.0);
 }
 
 F32Plan f32_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_a, int64_t most) {
@@ -408,7 +409,7 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
   g.sum = sum;
   const int64_t held = splits_held(workspace, workspace_bytes, M, N);
   const F32Plan p = f32_plan(M, N, K, count, sum, trans_a, held);
-  if (count > 1 && !sum && faster_one_by_one(p, f32_plan(M, N, K, 1, 0, trans_a, held), count, 1.08)) {
+  if (count > 1 && !sum && faster_one_by_one(p, f32_plan(M, N, K, 1, 0, trans_a, held), count, 1.0)) {
     for (int i = 0; i < count; i++) {
       const void* r = R != nullptr ? R[i] : nullptr;
       if (const int rc = launch_f32_gemm(st, 1, A + i, B + i, &r, C + i, workspace, workspace_bytes, M, N, K, lda, ldb, ldr, ldc, trans_a, trans_b, 0, nullptr))
@@ -420,10 +421,11 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
                   p.splits, count > 1 ? &g : nullptr, planes};
   // (the split kernels address a tile of the result with 31 bits too)
   const bool wide = 128 * ldc >= 0x1fffffff || 128 * N >= 0x1fffffff || (R != nullptr && 128 * ldr >= 0x1fffffff);
-  switch (wide && p.shape > 1 ? 0 : p.shape) {
+  switch (wide && p.shape > 2 ? 0 : p.shape) {
     case 0: return launch_f32_shape<64, 64, 2, 2, 1, 32, 2>(st, c, trans_a, trans_b);
     case 1: return launch_f32_shape<32, 32, 1, 1, 8, 64, 5>(st, c, trans_a, trans_b);
-    default: return launch_f32_bf16x3(st, c, p.shape - 2, trans_a, trans_b);
+    case 2: return launch_f32_shape<128, 128, 4, 2, 1, 32, 2>(st, c, trans_a, trans_b);
+    default: return launch_f32_bf16x3(st, c, p.shape - 3, trans_a, trans_b);
   }
 }
 

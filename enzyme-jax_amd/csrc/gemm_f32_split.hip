@@ -11,9 +11,10 @@
 // both end in `total` every PF stages (64 or 96 k), which keeps the chains short.  Relative error against float64, this | the
 // fp32 instructions with chains of 32: 2000 x 768 x 768 0.8e-7 | 1.3e-7, 4096^3 1.3e-7 | 2.3e-7, 256 x 288 x 32000 1.3e-7 | 1.9e-7.
 // What bounds it: 6 products at the rate that random bf16 numbers leave the clock at (1.7 GHz: 300 TFLOP/s), and on a CU the
-// issue of the split beside the matrix instructions, 5.5 instructions a number, of which a wavefront issues one in 7.7 cycles.
-// Measured, us, 64- and 128-tiles of the fp32 instructions | this: 2000 x 768 x 768 33 | 25.6; 2000 x 2048 x 768 55 | 44;
-// 2048 x 768 x 2000 (TN, four) 223 | 164; 777 x 4096 x 4096 237 | 163; 4096^3 1025 | 732 (188 TFLOP/s).
+// issue of the split beside the matrix instructions, 5.5 instructions a number and 1.5 to 2 that test it, of which a wavefront issues
+// one in 7.7 cycles.
+// Measured, us, 64- and 128-tiles of the fp32 instructions | this: 2000 x 768 x 768 33 | 26.4; 2000 x 2048 x 768 55 | 44;
+// 2048 x 768 x 2000 (TN, four) 223 | 164; 777 x 4096 x 4096 237 | 171; 4096^3 1025 | 741 (185 TFLOP/s).
 // Wavefronts that only split beside others that only multiply, eight wavefronts a block instead of sixteen, fragments read a
 // k-step ahead: all the same 1.03 us a stage of a 128 x 128 block, or slower.
 #include <type_traits>
@@ -57,10 +58,10 @@ __device__ __forceinline__ void split(const float (&x)[N], uint32_t (&h)[N / 2],
   round(l, r);
 }
 
-// One operand of a block: ROWS rows (of A: rows of C; of B: columns of C) by 32 of the contraction per stage, loaded by 512
-// threads into registers, split, and laid into the LDS as three planes of 16-byte pieces: [kp][slot], piece kp of a row
-// holding the eight k  4 kp .. + 3 and 16 + 4 kp .. + 3, in that order.  A thread takes a whole piece (128 rows) or half of
-// one (64 rows), so that four or eight lanes read 64 or 128 consecutive bytes of a k-contiguous row.  slot(row) and the 32 bytes
+// One operand of a block: ROWS rows (of A: rows of C; of B: columns of C) by 32 of the contraction per stage, loaded
+// into registers, split, and laid into the LDS as three planes of 16-byte pieces: [kp][slot], piece kp of a row holding the
+// eight k  4 kp .. + 3 and 16 + 4 kp .. + 3, in that order.  A thread takes half a piece (1024 threads for 128 rows, 512 for 64)
+// or a whole one (512 for 128), so that eight or four lanes read 128 or 64 consecutive bytes of a k-contiguous row.  slot(row) and the 32 bytes
 // between the kp's spread the lanes of one pass of an LDS write over all banks.
 template <int ROWS, int THREADS, int PF, bool KM> struct SplitOperand {
   static constexpr int KP = ROWS * 16 + 32, PLANE = 4 * KP, BYTES = 3 * PLANE;
@@ -313,8 +314,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 4) void gemm_f32_split_kernel(cons
   end_chain();
 
   // Where the split does not hold, the tile is multiplied again in fp32 as it is, in stages through the LDS (us for the whole
-  // product, ordinary numbers | all tiles again | the same on the fp32 kernels alone: 2000 x 768 x 768 28 | 56 | 33,
-  // 777 x 4096 x 4096 163 | 428 | 230, 4096^3 741 | 1730 | 1012): a number that may not be the sum of its parts, and numbers that
+  // product, ordinary numbers | all tiles again | the same on the fp32 kernels alone: 2000 x 768 x 768 26.4 | 56 | 33,
+  // 777 x 4096 x 4096 171 | 428 | 230, 4096^3 741 | 1730 | 1012): a number that may not be the sum of its parts, and numbers that
   // are infinite, NaN or round to an infinite h (some sum is not finite then).
   bool odd = oa.inexact() || ob.inexact();
 #pragma unroll

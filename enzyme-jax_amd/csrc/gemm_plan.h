@@ -11,8 +11,8 @@ struct Bf16Plan {
   double us;        // the estimate
 };
 struct F32Plan {
-  int shape;        // on the fp32 instructions 0: blocks of 64 x 64, 1: 32 x 32 (gemm_f32.hip); on the bf16 instructions 2: 128 x 128,
-                    // 3: 128 x 64, 4: 64 x 64 (gemm_f32_split.hip)
+  int shape;        // on the fp32 instructions 0: blocks of 64 x 64, 1: 32 x 32, 2: 128 x 128 (gemm_f32.hip); on the bf16
+                    // instructions 3: 128 x 128, 4: 128 x 64, 5: 64 x 64 (gemm_f32_split.hip)
   int splits;
   double us;
 };

@@ -24,13 +24,14 @@ SIZES = [
     (100, 512, 516, 3),      # 32-tiles, ragged rows
     (12, 20, 20004, 2),      # a single tile: splits of a long contraction, ragged last stage
     (260, 1028, 772, 2),     # 64-tiles of the fp32 instructions, splits
-    (704, 2812, 1028, 2),    # ragged columns: 64-tiles of the bf16 instructions; a group: of the fp32 ones
+    (704, 2812, 1028, 2),    # ragged columns: 64-tiles of the bf16 instructions, summed too; a group: of the fp32 ones
     (708, 1540, 292, 2),     # 128 x 64, ragged both ways
     (1996, 772, 2052, 2),    # 128-tiles, splits; summed: splits that straddle the products
-    (2052, 2044, 68, 2),     # 64-tiles of the fp32 instructions, ragged both ways
+    (2052, 2044, 68, 2),     # 64-tiles of the fp32 instructions, ragged both ways; a group, summed: 128 x 64
+    (772, 1412, 28, 6),      # a group: 128-tiles of the fp32 instructions, one stage
     (1412, 260, 772, 3),     # a group: 128 x 64; summed: its splits straddle the products
-    (516, 772, 2052, 2),     # a group: 64-tiles of the bf16 instructions
-    (1004, 772, 516, 2),     # summed: 64-tiles of the bf16 instructions
+    (516, 1092, 516, 3),     # a group: 64-tiles of the bf16 instructions; summed: 128-tiles with splits
+    (1004, 772, 516, 2),     # 64-tiles of the fp32 instructions; a group: 128 x 64; summed: 128-tiles with splits
 ]
 
 

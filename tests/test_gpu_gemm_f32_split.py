@@ -11,11 +11,11 @@ pytestmark = pytest.mark.gpu
 
 # what each is there for; tests/test_host_boundary.py holds them to reaching every kernel
 SIZES = [
-    (900, 1028, 2052),       # blocks of 64 x 64, a last round of one stage
-    (1004, 772, 36),         # the same where A is k-contiguous, no more stages than are in flight
-    (516, 2052, 28),         # 128 x 64, fewer stages than are in flight
+    (780, 2308, 772),        # blocks of 64 x 64, a last round of one stage
+    (180, 2820, 1284),       # the same, three splits
+    (4004, 2372, 28),        # 128 x 64, fewer stages than are in flight
     (900, 1284, 1036),       # the same, three splits
-    (2004, 1540, 36),        # 128 x 128, fewer stages than are in flight
+    (716, 2756, 100),        # 128 x 128, a last round of one stage
     (708, 1092, 2052),       # the same, four splits
 ]
 
@@ -85,7 +85,7 @@ def test_numbers_that_do_not_split(what, ta, tb, M, N, K):
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(964, 772, 100), (900, 1092, 132), (1060, 1092, 2052)])
+@pytest.mark.parametrize("M,N,K", [s for s in SIZES if s[2] > 32])
 @pytest.mark.parametrize("scale", [1e-31, 1e-34, 1e-37, 1e-41])
 def test_small_numbers_keep_their_bits(scale, ta, tb, M, N, K):
     """A row of A, a column of B and single terms far below their neighbours are as exact as any other: what a number loses

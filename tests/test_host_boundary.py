@@ -88,7 +88,7 @@ def test_a_product_is_planned_with_the_splits_its_workspace_holds(dtype, M, N, K
     the 256 CUs, or the smallest ones there are.  With room for some planes there are at most as many splits."""
     lib = _lib()
     plan, blocks, trans = ((lib._ZN3emi9bf16_planEllliiil, [(256, 256), (128, 128), (128, 128), (128, 64), (64, 64), (32, 32)], 1)
-                           if dtype == "bf16" else (lib._ZN3emi8f32_planEllliiil, [(64, 64), (32, 32), (128, 128), (128, 64), (64, 64)], 0))      # of B, of A
+                           if dtype == "bf16" else (lib._ZN3emi8f32_planEllliiil, [(64, 64), (32, 32), (128, 128), (128, 128), (128, 64), (64, 64)], 0))      # of B, of A
     plan.restype, plan.argtypes = _Plan, [C.c_int64] * 3 + [C.c_int] * 3 + [C.c_int64]
     tiles = lambda p: -(-M // blocks[p.shape][0]) * -(-N // blocks[p.shape][1])
     free, one = (plan(M, N, K, count, total, trans, most) for most in (1 << 20, 1))
@@ -133,16 +133,17 @@ def test_the_sizes_of_the_f32_gpu_tests_reach_every_kernel():
 
     def ran(sizes, n, total, ta):
         plans = [(plan(M, N, K, n or count, total, ta, 1 << 20), K) for M, N, K, count in sizes]
-        return {p.shape for p, _ in plans}, {p.shape for p, _ in plans if p.splits > 1}, {p.shape for p, K in plans if K <= (64 if p.shape == 2 else 32)}
+        return {p.shape for p, _ in plans}, {p.shape for p, _ in plans if p.splits > 1}, {p.shape for p, K in plans if K <= 32}
 
+    sizes = test_gpu_gemm_f32.SIZES
+    assert ran(sizes, 0, 0, 0)[0] | ran(sizes, 0, 0, 1)[0] == set(range(6))
     for ta in (0, 1):
-        sizes = test_gpu_gemm_f32.SIZES
         one, one_split, _ = ran(sizes, 1, 0, ta)
         both, both_split, _ = ran(sizes, 0, 1, ta)
-        assert one == set(range(5)) and ran(sizes, 0, 0, ta)[0] == set(range(5)) and both == set(range(5))
-        assert one_split >= {0, 1, 2} and both_split >= {0, 1, 2, 3}
+        assert one >= {0, 1, 3, 4, 5} and ran(sizes, 0, 0, ta)[0] >= set(range(5)) and both >= {0, 1, 3, 4, 5}
+        assert one_split >= {0, 1, 3} and both_split >= {0, 1, 3, 4}
         kernels, split, few = ran([s + (1,) for s in test_gpu_gemm_f32_split.SIZES], 1, 0, ta)
-        assert kernels >= {2, 3, 4} and split >= {2, 3} and few >= {2, 3}
+        assert kernels >= {3, 4, 5} and split >= {3, 4, 5} and 4 in few
 
 
 def test_the_layers_whose_norms_add_planes_have_split_products():
