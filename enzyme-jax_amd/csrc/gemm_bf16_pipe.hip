@@ -400,35 +400,44 @@ static int launch_pipe_shape(hipStream_t st, const PipeCall& c, int trans_b) {
 // come after others, and what several results in one launch cost more.  Shape 0 is the 256 x 256 ping-pong kernel of gemm.hip,
 // whose clock falls as it fills the chip, 1 the 128 x 128 tile of which two fit a CU, 2 the same tile in a ring of three stages
 // whose k two wavefronts share, one to a CU, 3 128 x 64, 4 64 x 64, both in stages of 128 k, 5 a 32 x 32 tile whose eight
-// wavefronts share stages of 256 k.  Fitted to 666 products of 16 to 8192 tokens whose weights, 64 MB of them in turn, come
-// from beyond the L2s, each with every block and number of splits: 0.6 % behind the fastest of them in the geometric mean.
+// wavefronts share stages of 256 k, 6 64 x 64 in stages of 64 k.  Fitted to products of 16 to 8192 tokens whose weights, 64 MB of
+// them in turn, come from beyond the L2s, each with the blocks and splits that could be the fastest.  A k-major B has rates of
+// its own, and with it 6 competes with 4: its stages hold a contraction of two or three of 128 k, or of splits so short, with
+// less waste.  On 3991 other products the plan is 0.2 % (k-contiguous B) and 0.7 % (k-major; 2.1 % by the rates of the former)
+// behind the fastest in the geometric mean.  us, B k-major, by those | these: 646 x 768 x 288 4.8 | 4.3, 18 x 288 x 288 x 3 summed
+// 7.3 | 6.2, 32 x 768 x 2048 7.2 | 6.6, 344 x 768 x 2048 x 2 summed 14.6 | 12.3, 2499 x 1024 x 2816 30.5 | 24.5.
 // The reduction over splits is a launch of its own; results over 4 M elements, whose planes leave the caches, are not split
 // (but see pingpong_splits of gemm.hip), nor are the products of a few tokens, which have kernels of their own
-// (gemm_skinny.hip).  A split of 64 x 64 tiles has at least 384 k, as the reduction costs as much as 8 of its stages (us, splits
-// of 512 | 384 k at least, B k-major, summed: 16 x 1024 x 1024 x 3 8.5 | 8.0, 16 x 288 x 768 x 2 7.4 | 7.0).
+// (gemm_skinny.hip).  A split of 64 x 64 tiles, and any with a k-major B, has at least three stages, others four.
 Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b, int64_t most) {
-  struct Shape { int bm, bn, bk; double fixed, group, rate[3], more; };      // rate[b - 1]: per stage, b blocks on the CU; more: per block
-                                                                            // from four on; group: more with several results
+  struct Shape { int bm, bn, bk; double fixed, group, rate[3], more, later; };      // rate[b - 1]: per stage, b blocks on the CU; more: per
+                                                                                   // block from four on; group: with several results; later:
+                                                                                   // the start of each block that comes after others
   static const Shape shapes[6] = {
-      {256, 256, 64, 4.0, 0.8, {1.0, 2.0, 3.0}, 1.0},    {128, 128, 64, 3.9, 0.2, {0.59, 0.855, 1.6}, 0.515}, {128, 128, 64, 4.3, 0.8, {0.535, 1.07, 1.6}, 0.535},
-      {128, 64, 128, 3.45, 0.45, {0.6, 1.24, 2.0}, 0.6}, {64, 64, 128, 3.15, 0.2, {0.355, 0.785, 1.10}, 0.41}, {32, 32, 256, 3.4, 0.0, {0.30, 0.62, 1.4}, 0.363}};
+      {256, 256, 64, 4.0, 0.8, {1.0, 2.0, 3.0}, 1.0, 0.0},      {128, 128, 64, 3.9, 0.2, {0.59, 0.855, 1.6}, 0.515, 0.0},
+      {128, 128, 64, 4.3, 0.3, {0.535, 1.07, 1.6}, 0.535, 0.0}, {128, 64, 128, 3.45, 0.45, {0.6, 1.24, 2.0}, 0.6, 0.0},
+      {64, 64, 128, 3.15, 0.2, {0.355, 0.785, 1.10}, 0.41, 0.0}, {32, 32, 256, 3.4, 0.0, {0.30, 0.62, 1.4}, 0.363, 1.75}};
+  static const Shape kmajor[7] = {
+      {256, 256, 64, 4.0, 0.45, {1.0, 2.0, 3.0}, 1.0, 0.0},          {128, 128, 64, 5.1, 0.45, {0.585, 0.82, 1.435}, 0.50, 0.25},
+      {128, 128, 64, 5.0, 0.45, {0.52, 1.05, 1.535}, 0.535, 3.35},    {128, 64, 128, 3.75, 0.45, {0.635, 1.20, 1.87}, 0.60, 0.5},
+      {64, 64, 128, 3.0, 0.45, {0.415, 0.735, 1.29}, 0.41, 1.5},      {}, {64, 64, 64, 2.65, 0.45, {0.345, 0.43, 0.57}, 0.22, 0.9}};
   Bf16Plan best{1, 1, 0.0};
   double least = 1e30;
   const bool may_split = (sum || count == 1) && M * N <= (4 << 20) && M > 8 && K > 8;
-  for (int c = 0; c < 6; c++) {
+  for (int c = 0; c < (trans_b ? 6 : 7); c++) {
     if ((c == 0 && sum && count > 1) || (c == 5 && !trans_b)) continue;        // what those kernels do not do
-    const Shape& s = shapes[c];
+    const Shape& s = trans_b ? shapes[c] : kmajor[c];
     const int64_t steps = (K + s.bk - 1) / s.bk * (sum ? count : 1);
     const int64_t blocks = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * (sum ? 1 : count);
     if (blocks > 0x3fffffff) continue;
     const bool split = may_split && (c != 0 || trans_b);
-    for (int64_t z = 1; z <= 16 && z <= most && (z == 1 || (split && steps >= (c == 4 ? 3 : 4) * z)); z++) {
+    for (int64_t z = 1; z <= 16 && z <= most && (z == 1 || (split && steps >= (c == 4 || !trans_b ? 3 : 4) * z)); z++) {
       const int64_t b = (blocks * z + 255) / 256, per = (steps + z - 1) / z;
       double stage = b < 4 ? s.rate[b - 1] : s.more * b;
-      if (c == 4 && !trans_b) stage = b == 1 ? 0.385 : b == 3 ? 1.14 : stage;
-      const double later = c == 4 && b > 2 ? 1.0 * (b - 2) : c == 5 ? 1.75 * (b - 1) : 0.0;     // the start of blocks that come after others
+      const double later = c == 4 && trans_b ? (b > 2 ? 1.0 * (b - 2) : 0.0) : s.later * (b - 1);
       if (c == 0) stage *= 1.0 + 0.45 * (blocks * z < 256 ? blocks * z / 256.0 : 1.0);
-      const double t = s.fixed + (count > 1 && !sum ? s.group : 0.0) + later + per * stage + (z > 1 ? 2.8 + 0.78e-6 * M * N * (z + 1) : 0.0);
+      const double t = s.fixed + (count > 1 && !sum ? s.group : 0.0) + later + per * stage +
+                       (z == 1 ? 0.0 : trans_b ? 2.8 + 0.78e-6 * M * N * (z + 1) : 2.65 + 1e-6 * M * N * (z + 1));
       if (t < least) {
         least = t;
         best = Bf16Plan{c, (int)z, t};
@@ -438,20 +447,27 @@ Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int count, int sum, int tran
   return best;
 }
 
-// The kernel of a plan's blocks: 0 the ping-pong kernel, 1, 2 blocks of 128 x 128, 3, 4 of 128 x 64, 5 to 7 of 64 x 64, 8 of
+// The kernel of a plan's blocks: 0 the ping-pong kernel, 1, 2, 9 blocks of 128 x 128, 3, 4 of 128 x 64, 5 to 7 of 64 x 64, 8 of
 // 32 x 32.
-// Deeper rings, of stages of 128 k, where a block has its CU to itself and enough stages to fill them; 64 x 64 blocks of four
-// wavefronts and 64 k a stage, three of which fit a CU, where three there are.  us, ring of two | three, 64 x 64: 300 x 768 x 768
-// 6.7 | 6.1 (B k-major), 300 x 2816 x 1024 8.2 | 7.1, 256 x 2048 x 768 6.9 | 6.2, 300 x 1408 x 512 5.5 | 5.0, with B k-major
-// 5.8 | 5.4, 512 x 512 x 512 with B k-major 5.0 | 5.3; 128 x 64, of 64 k and eight wavefronts | of 128 and sixteen: 512 x 768 x 768 (three) 9.1 | 8.4,
-// 2048 x 768 x 288 5.5 | 6.2, 1000 x 1408 x 512 6.6 | 6.9; 64 x 64, of 128 | of 64 k, three to a CU: 1500 x 512 x 512 (three) 9.7 | 9.2.
+// More wavefronts and deeper rings, of stages of 128 k, where a block has its CU to itself and enough stages to fill them; 64 x 64
+// blocks of four wavefronts and 64 k a stage, three of which fit a CU, where three there are, and of a k-major B where the
+// plan says so or a contraction is of two or three stages.  us:
+// 128 x 128, eight wavefronts | sixteen that share k: 1714 x 1408 x 512 8.4 | 8.7, 981 x 2816 x 1024 12.3 | 12.2, 520 x 4096 x 4096 36 | 33,
+// 779 x 1408 x 512 (two) 9.1 | 9.8, 662 x 1024 x 1024 (three) 13.3 | 13.6, 3705 x 1024 x 1024 (three summed, B k-major) 30.6 | 31.3;
+// 128 x 64, of 64 k and eight wavefronts | of 128 and sixteen: 512 x 768 x 768 (three) 9.1 | 8.4, 2048 x 768 x 288 5.5 | 6.2,
+// 1000 x 1408 x 512 6.6 | 6.9, 3714 x 288 x 288 (three summed, B k-major) 9.7 | 10.1;
+// 64 x 64, ring of two | three: 300 x 768 x 768 (B k-major) 6.7 | 6.1, 300 x 2816 x 1024 8.2 | 7.1, 256 x 2048 x 768 6.9 | 6.2,
+// 300 x 1408 x 512 5.5 | 5.0, with B k-major 5.8 | 5.4, 493 x 512 x 512 4.7 | 4.9, 531 x 512 x 512 5.3 | 5.0;
+// 64 x 64, of 128 | of 64 k: 1500 x 512 x 512 (three) 9.7 | 9.2, B k-major 270 x 768 x 288 4.6 | 4.4, 800 x 768 x 288 4.9 | 4.6.
 int bf16_kernel(const Bf16Plan& plan, int64_t M, int64_t N, int64_t K, int count, int sum, int trans_b) {
+  if (plan.shape == 2 && K < (count == 1 ? 1024 * plan.splits : sum ? 2560 : 2048)) return 9;
   if (plan.shape < 3) return plan.shape;
-  if (plan.shape == 5) return 8;
+  if (plan.shape >= 5) return plan.shape == 5 ? 8 : 7;
   const int rows = plan.shape == 3 ? 128 : 64;
   const int64_t blocks = (M + rows - 1) / rows * ((N + 63) / 64) * (sum || count == 1 ? plan.splits : count), all_k = K * (sum ? count : 1);
-  if (plan.shape == 3) return blocks <= 256 && all_k > 640 * plan.splits ? 4 : 3;
-  if (blocks <= 256 && all_k >= (trans_b || N > 768 ? 512 : 640)) return 6;
+  if (plan.shape == 3) return blocks <= 256 && all_k > 640 * plan.splits && K > 320 ? 4 : 3;
+  if (blocks <= 256 && all_k >= (trans_b || N > 768 || blocks > 64 ? 512 : 640)) return 6;
+  if (!trans_b) return all_k < 384 * plan.splits ? 7 : 5;
   return blocks > 512 && blocks <= 768 ? 7 : 5;
 }
 
@@ -481,6 +497,7 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
     case 5: return launch_pipe_shape<64, 64, 2, 2, 2, 128, 2>(st, c, trans_b);
     case 6: return launch_pipe_shape<64, 64, 2, 2, 2, 128, 3>(st, c, trans_b);
     case 7: return launch_pipe_shape<64, 64, 2, 2, 1, 64, 3>(st, c, trans_b);
+    case 9: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 3>(st, c, trans_b);
     default: return launch_pipe_shape<32, 32, 1, 1, 8, 256, 3>(st, c, trans_b);
   }
 }

@@ -28,10 +28,12 @@ SIZES = [
     (1500, 504, 512, 3),      # a group: 64-tiles of 64 k a stage, three to a CU (k-contiguous B)
     (30, 2800, 504, 12),      # the same, k-major B
     (777, 2040, 776, 2),      # 128 x 64 tiles of 128 k a stage, ragged
-    (1000, 4088, 520, 2),     # 128-tiles, three stages
+    (900, 520, 328, 2),       # a group: 128 x 64 tiles of 64 k a stage (k-major B)
+    (1000, 4088, 520, 2),     # 128-tiles in a ring of three stages, eight wavefronts
     (3000, 1032, 328, 2),     # 128 x 64 tiles of 64 k a stage; a group: 128-tiles, two to a CU; summed: one pass over both
-    (600, 2056, 4104, 2),     # 128-tiles with splits; summed: splits that straddle the products
-    (300, 1000, 16392, 2),    # 64-tiles and 128 x 64 with splits
+    (600, 2056, 4104, 2),     # 128-tiles, of sixteen wavefronts; with splits (k-contiguous B); summed: splits that straddle the products
+    (777, 264, 2056, 2),      # summed: 128 x 64 tiles with splits (k-major B)
+    (300, 1000, 16392, 2),    # 64-tiles with splits
     (1000, 2056, 8200, 1),    # 256-tiles with splits (k-contiguous B)
     (2056, 2048, 8200, 1),    # more than 4 M results: 256-tiles with splits all the same (k-contiguous B)
 ]

@@ -118,8 +118,8 @@ def test_the_sizes_of_the_bf16_gpu_test_reach_every_kernel():
                 ran.add((kernel(C.byref(p), M, N, K, n, total, tb), tb))
                 if p.splits > 1:
                     split.add(p.shape)
-    assert {k for k, tb in ran if tb} == set(range(9)) and {k for k, tb in ran if not tb} >= set(range(1, 8))
-    assert split >= {0, 1, 2, 3, 4, 5}
+    assert {k for k, tb in ran if tb} == set(range(10)) and {k for k, tb in ran if not tb} >= set(range(1, 8)) | {9}
+    assert split == set(range(7))
 
 
 def test_the_sizes_of_the_f32_gpu_tests_reach_every_kernel():
