@@ -12,8 +12,8 @@
 // 777 x 768 x 2048 18.7 -> 9.0; 64 x 768 x 768 9.9 -> 4.2; 300 x 5632 x 2048 23.2 -> 13.2; 1000 x 4096 x 4096 47.5 -> 37.0;
 // 8192 x 768 x 768 15.4 -> 15.2, x 2048 30.5 -> 29.1; 8192 x 2304 x 768 42.4 -> 37.1 (782 TFLOP/s); k-major B:
 // 777 x 768 x 768 15.5 -> 5.8; 1000 x 4096 x 4096 64.4 -> 36.6; 8192 x 768 x 2048 36.6 -> 30.4.  With weights from beyond the
-// L2s, as a model has them: 777 x 768 x 768 6.2, x 2048 9.9, 512 x 1024 x 1024 6.9, 300 x 5632 x 2048 14.7, 1000 x 2048 x 2048 15.3,
-// 1000 x 4096 x 4096 40, 8192 x 768 x 768 16.3, x 2048 33.
+// L2s, as a model has them: 777 x 768 x 768 5.9, x 2048 9.5, 512 x 1024 x 1024 6.5, 300 x 5632 x 2048 14.6, 1000 x 2048 x 2048 13.7,
+// 1000 x 4096 x 4096 36.6, 8192 x 768 x 768 15.4, x 2048 29.6.
 #include <type_traits>
 #include <utility>
 

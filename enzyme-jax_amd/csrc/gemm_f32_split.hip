@@ -13,8 +13,8 @@
 // What bounds it: 6 products at the rate that random bf16 numbers leave the clock at (1.7 GHz: 300 TFLOP/s), and on a CU the
 // issue of the split beside the matrix instructions, 5.5 instructions a number and 1.5 to 2 that test it, of which a wavefront issues
 // one in 7.7 cycles.
-// Measured, us, 64- and 128-tiles of the fp32 instructions | this: 2000 x 768 x 768 33 | 26.4; 2000 x 2048 x 768 55 | 44;
-// 2048 x 768 x 2000 (TN, four) 223 | 164; 777 x 4096 x 4096 237 | 171; 4096^3 1025 | 741 (185 TFLOP/s).
+// Measured, us, 64- and 128-tiles of the fp32 instructions | this: 2000 x 768 x 768 32.5 | 26.1; 2000 x 2048 x 768 59 | 41;
+// 2048 x 768 x 2000 (TN, four) 223 | 170; 777 x 4096 x 4096 232 | 162; 4096^3 1008 | 730 (188 TFLOP/s).
 // Wavefronts that only split beside others that only multiply, eight wavefronts a block instead of sixteen, fragments read a
 // k-step ahead: all the same 1.03 us a stage of a 128 x 128 block, or slower.
 #include <type_traits>
@@ -314,8 +314,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 4) void gemm_f32_split_kernel(cons
   end_chain();
 
   // Where the split does not hold, the tile is multiplied again in fp32 as it is, in stages through the LDS (us for the whole
-  // product, ordinary numbers | all tiles again | the same on the fp32 kernels alone: 2000 x 768 x 768 26.4 | 56 | 33,
-  // 777 x 4096 x 4096 171 | 428 | 230, 4096^3 741 | 1730 | 1012): a number that may not be the sum of its parts, and numbers that
+  // product, ordinary numbers | all tiles again | the same on the fp32 kernels alone: 2000 x 768 x 768 26 | 56 | 33,
+  // 777 x 4096 x 4096 162 | 428 | 232, 4096^3 730 | 1730 | 1008): a number that may not be the sum of its parts, and numbers that
   // are infinite, NaN or round to an infinite h (some sum is not finite then).
   bool odd = oa.inexact() || ob.inexact();
 #pragma unroll
