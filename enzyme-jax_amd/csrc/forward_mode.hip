@@ -171,7 +171,8 @@ struct JvpShape {
 // Exp :1182, Div :1133, Sub :1312, reduce max/add StableHLOAutoDiffOpInterfaceImpl.cpp:1833-1916):
 //   tS = scale (tq k^T + q tk^T);  tP = P (tS - rowsum(P tS));  to = tP v + P tv
 //      = sum_j p_j tS_j v_j - (sum_j p_j tS_j) o + sum_j p_j tv_j,   p_j = exp(S_j - lse)
-// One wavefront per query row, one key per lane and 64 keys per sweep; head_dim <= 256.
+// One wavefront per query row, one key per lane and 64 keys per sweep; head_dim <= 256.  For the shapes that the matrix-core
+// kernels (attention.hip, attention_f32.hip) do not take.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_jvp_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                                        const float* __restrict__ lse, const T* __restrict__ tq,
@@ -238,6 +239,10 @@ bool al16(const void* p) { return p == nullptr || (reinterpret_cast<uintptr_t>(p
 int launch_attn_jvp_mfma(hipStream_t st, const void* q, const void* k, const void* v, const float* lse, const void* tq,
                          const void* tk, const void* tv, void* to, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
                          int64_t sb, int64_t shh, int64_t ss, float scale, int causal, int dtype);
+// attention_f32.hip
+int launch_attn_jvp_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const float* lse, const void* tq,
+                             const void* tk, const void* tv, void* to, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
+                             int64_t sb, int64_t shh, int64_t ss, float scale, int causal);
 }  // namespace emi
 
 using namespace emi;
@@ -307,8 +312,10 @@ extern "C" int emi_attn_jvp(emi_stream_t stream, const void* q, const void* k, c
   EMI_REQUIRE(q && k && v && lse && to, "emi_attn_jvp: null buffer");
   hipStream_t st = static_cast<hipStream_t>(stream);
   {
-    const int rc = launch_attn_jvp_mfma(st, q, k, v, lse, tq, tk, tv, to, batch, heads, seq, head_dim, stride_b, stride_h,
-                                        stride_s, scale, causal, dtype);
+    const int rc = dtype == EMI_F32 ? launch_attn_jvp_f32_mfma(st, q, k, v, lse, tq, tk, tv, to, batch, heads, seq, head_dim, stride_b,
+                                                               stride_h, stride_s, scale, causal)
+                                    : launch_attn_jvp_mfma(st, q, k, v, lse, tq, tk, tv, to, batch, heads, seq, head_dim, stride_b, stride_h,
+                                                           stride_s, scale, causal, dtype);
     if (rc >= 0) return rc;
   }
   const JvpShape sh{(int)seq, (int)heads, stride_b, stride_h, stride_s};

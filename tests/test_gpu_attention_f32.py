@@ -50,3 +50,46 @@ def test_f32_attention_keeps_non_finite_values():
         o = ops.attention(q, k, bad, 2, layout="bhsd")
         assert torch.equal(o[0, 0], clean[0, 0]) and torch.equal(o[0, 1, :at - at % 16], clean[0, 1, :at - at % 16])
         assert not torch.isfinite(o[0, 1, at:]).any()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,h,S,d", [(1, 1, 1, 16), (1, 3, 17, 32), (2, 5, 63, 48), (1, 7, 64, 64), (1, 2, 130, 80), (1, 9, 250, 128), (1, 19, 513, 128),
+                                     (2, 12, 545, 96), (3, 9, 700, 80), (5, 40, 31, 112), (2, 3, 515, 64)])
+def test_f32_attention_tangent_tiles(B, h, S, d, causal):
+    """One and two sets of 16 queries a block (head sizes from 80 on, rows and blocks enough: 513, 545, 700 causal; 200 pairs of
+    tiles without the mask), the last set cut or empty.  A tangent entry is the sum of S products with weights of 2d products
+    each, minus the mean weight times a sum of S: two such sums, each within the bound of the module, of terms as large as
+    sqrt(2 d) scale = sqrt(2) times the entries' own size."""
+    from enzyme_ad.jax import ops, jvp
+    rng = np.random.default_rng(7 * S + d)
+    (q, qr), (k, kr), (v, vr), (tq, tqr), (tk, tkr), (tv, tvr) = (dev(rng.standard_normal((B, h, S, d)), "f32") for _ in range(6))
+
+    def fn(a, b, c):
+        return ops.attention(a, b, c, h, causal=causal, layout="bhsd")
+
+    bound = 4 * (d + S) * 2.0 ** -23
+    for given in ((1, 1, 1), (1, 0, 0), (0, 1, 0), (0, 0, 1)):
+        _, to = jvp(fn, (q, k, v), tuple(t if g else None for t, g in zip((tq, tk, tv), given)))
+        want = L.attention_jvp(qr, kr, vr, *(t * g for t, g in zip((tqr, tkr, tvr), given)), causal=causal)
+        size = max(float(np.max(np.abs(want))), 1.0)      # one key: the tangent is tv, what q and k give is rounding
+        assert float(np.max(np.abs(host(to) - want))) <= bound * size, given
+
+
+def test_f32_attention_tangent_of_other_layouts():
+    """Rows that do not start on 16-byte boundaries go to the kernel of one wavefront per query; both layouts agree with it."""
+    from enzyme_ad.jax import ops, jvp
+    rng = np.random.default_rng(11)
+    B, h, S, d = 2, 4, 70, 80
+    x = [dev(rng.standard_normal((B, S, h * d)), "f32") for _ in range(6)]
+    heads = lambda a: np.ascontiguousarray(a.reshape(B, S, h, d).transpose(0, 2, 1, 3))
+    want = L.attention_jvp(*(heads(r) for _, r in x), causal=True)
+    bound = 4 * (d + S) * 2.0 ** -23 * float(np.max(np.abs(want)))
+    for shift in (0, 1):
+        args = []
+        for t, _ in x:
+            room = torch.empty(t.numel() + 4, device=t.device)
+            moved = room[shift:shift + t.numel()].view(t.shape)
+            moved.copy_(t)
+            args.append(moved)
+        _, to = jvp(lambda a, b, c: ops.attention(a, b, c, h), tuple(args[:3]), tuple(args[3:]))
+        assert float(np.max(np.abs(heads(host(to)) - want))) <= bound, shift
