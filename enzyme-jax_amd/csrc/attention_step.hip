@@ -65,10 +65,9 @@ struct StepShape {
   // the whole-step path (llama_step.hip): the last key, the token's own, lies outside the cache, in rows of its own
   const void *k_tail = nullptr, *v_tail = nullptr;
   void *dk_tail = nullptr, *dv_tail = nullptr;
-  // its reverse with one block a head: the fp32 cotangents before the rotation
-  const float2* table = nullptr;
-  int table_pairs = 0;
-  float *fq = nullptr, *fk = nullptr, *fv = nullptr;
+  // its reverse: the cotangent of o as do_bands rows [heads * head_dim] to be added up
+  const float* do_part = nullptr;
+  int do_bands = 0;
 };
 
 // Row s of a head's cache (base: the head's first row), or the token's own row (tail: its row of all heads; off: the
@@ -404,43 +403,13 @@ __global__ __launch_bounds__(64) void attn_step_combine_kernel(const float* __re
   if (lane == 0) lse[bh] = mx + __logf(l);
 }
 
-// dq of a head from its blocks' shares, turned back by the position's angle; dk of the token's own row turned back; dv.
-template <typename T>
-__device__ __forceinline__ void step_qkv_rows(const float* p0, int nsplit, const T* dk, const T* dv, const float2* __restrict__ table,
-                                              int table_pairs, float* __restrict__ fq, float* __restrict__ fk, float* __restrict__ fv, int h,
-                                              int head_dim) {
-  for (int i = threadIdx.x; i < head_dim / 2; i += (int)blockDim.x) {
-    float q0 = 0.f, q1 = 0.f;
-    for (int s = 0; s < nsplit; s++) {
-      q0 += p0[s * (head_dim + 2) + 2 * i];
-      q1 += p0[s * (head_dim + 2) + 2 * i + 1];
-    }
-    const int at = h * head_dim + 2 * i;
-    const float2 t = table[(at >> 1) % table_pairs];
-    const float k0 = to_f32(dk[at]), k1 = to_f32(dk[at + 1]);
-    fq[at] = t.x * q0 + t.y * q1;
-    fq[at + 1] = t.x * q1 - t.y * q0;
-    fk[at] = t.x * k0 + t.y * k1;
-    fk[at + 1] = t.x * k1 - t.y * k0;
-    fv[at] = to_f32(dv[at]);
-    fv[at + 1] = to_f32(dv[at + 1]);
-  }
-}
-template <typename T>
-__global__ __launch_bounds__(128) void step_qkv_cotangents_kernel(const float* __restrict__ part, int nsplit, const T* __restrict__ dk,
-                                                                  const T* __restrict__ dv, const float2* __restrict__ table,
-                                                                  int table_pairs, float* __restrict__ fq, float* __restrict__ fk,
-                                                                  float* __restrict__ fv, int head_dim) {
-  step_qkv_rows(part + (int64_t)blockIdx.x * nsplit * (head_dim + 2), nsplit, dk, dv, table, table_pairs, fq, fk, fv, (int)blockIdx.x, head_dim);
-}
-
 // dV_s = p_s dO; dP_s = dO . V_s; dS_s = p_s (dP_s - dO . O); dQ = scale sum_s dS_s K_s;
 // dK_s = scale dS_s Q.  p is recomputed from lse; one pass over the keys of the block.
 template <typename T, bool VEC, int NCH>
 __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                             const T* __restrict__ v, const T* __restrict__ o,
                                                             const float* __restrict__ lse, const T* __restrict__ d_o,
-                                                            float* part, T* dk, T* dv,          // no restrict: step_qkv_rows reads them back
+                                                            float* __restrict__ part, T* __restrict__ dk, T* __restrict__ dv,
                                                             StepShape sh, float scale) {
   using E = Elems<T, VEC>;
   using Raw = typename E::Raw;
@@ -456,6 +425,24 @@ __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict_
   const T *ktail = static_cast<const T*>(sh.k_tail), *vtail = static_cast<const T*>(sh.v_tail);
   const float L = lse[bh];
 
+  __shared__ float dos[256];                        // the whole step: dO of the head, added up from its bands
+  if (sh.do_part != nullptr) {
+    for (int e = threadIdx.x >> 2; e < sh.head_dim; e += 64) {
+      const float* p = sh.do_part + qoff + e;
+      float v = 0.f;
+      for (int b0 = threadIdx.x & 3; b0 < sh.do_bands; b0 += 32) {
+        float t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) t[u] = p[(int64_t)(b0 + 4 * u < sh.do_bands ? b0 + 4 * u : b0) * sh.q_sb];
+#pragma unroll
+        for (int u = 0; u < 8; u++) t[u] = b0 + 4 * u < sh.do_bands ? t[u] : 0.f;
+        v += ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+      }
+      v = quad_sum(v);
+      if ((threadIdx.x & 3) == 0) dos[e] = to_f32(from_f32<T>(v));
+    }
+    __syncthreads();
+  }
   float qf[MAXC][NE], dof[MAXC][NE];
   int coff[MAXC];                                   // element offset of chunk c inside a row (a lane's idle chunks: 0)
   float delta = 0.f;
@@ -467,7 +454,12 @@ __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict_
     if (c < nch) {
       float of[NE];
       E::load(q + qoff + coff[c], qf[c]);
-      E::load(d_o + qoff + coff[c], dof[c]);
+      if (sh.do_part == nullptr) {
+        E::load(d_o + qoff + coff[c], dof[c]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < NE; e++) dof[c][e] = dos[coff[c] + e];
+      }
       E::load(o + qoff + coff[c], of);
 #pragma unroll
       for (int e = 0; e < NE; e++) delta = fmaf(dof[c][e], of[e], delta);
@@ -558,13 +550,6 @@ __global__ __launch_bounds__(256) void attn_step_bwd_kernel(const T* __restrict_
 #pragma unroll
         for (int e = 0; e < NE; e++) out[(l16 + 16 * c) * NE + e] = acc[c][e];
       }
-  }
-  // A head of the whole step in one block: dq is whole and the token's own row is among the block's keys, so what
-  // step_qkv_cotangents does with one share is done here.
-  if (sh.fq != nullptr) {
-    __syncthreads();                                      // the block's own stores to part and the rows
-    step_qkv_rows(part + (int64_t)bh * (sh.head_dim + 2), 1, static_cast<const T*>(sh.dk_tail), static_cast<const T*>(sh.dv_tail), sh.table,
-                  sh.table_pairs, sh.fq, sh.fk, sh.fv, h, sh.head_dim);
   }
 }
 
@@ -821,14 +806,12 @@ int launch_llama_step_attn_fwd(hipStream_t st, const void* q, const void* k_cach
   sh.v_tail = v_tail;
   return launch_step_fwd(st, q, k_cache, v_cache, o, lse, part, sh, heads, true, scale, dtype);
 }
-// fq, fk, fv: the cotangents of q and k before the rotation and of v, fp32.  dq goes through part [heads][blocks][head_dim + 2];
-// with one block a head that block turns them back itself, a launch of 1.3 to 1.9 us less a layer (3 to 4 where the host is the
-// bound).  Step and reverse, us: fp32, dim 288, 6 layers, 31 earlier keys 352 -> 343 replayed, 255 keys 387 -> 379 replayed and
-// 430 -> 412 from StableHLO text; bf16, dim 768, 255 keys 605 -> 596.  With several blocks a head the sum over them remains.
+// do_part: the cotangent of o as do_bands rows to be added up.  dq leaves as shares in part [heads][blocks][head_dim + 2], which
+// the caller adds up.
 int launch_llama_step_attn_bwd(hipStream_t st, const void* q, const void* k_cache, const void* v_cache, const void* k_tail,
-                               const void* v_tail, const void* o, const float* lse, const void* d_o, void* dk_cache, void* dv_cache,
-                               void* dk_tail, void* dv_tail, float* part, const float* table, int table_pairs, float* fq, float* fk, float* fv,
-                               int heads, int pos, int head_dim, int keys_per_block, float scale, int dtype) {
+                               const void* v_tail, const void* o, const float* lse, const float* do_part, int do_bands, void* dk_cache,
+                               void* dv_cache, void* dk_tail, void* dv_tail, float* part, int heads, int pos, int head_dim, int keys_per_block,
+                               float scale, int dtype) {
   const int64_t D = (int64_t)heads * head_dim;
   StepShape sh{heads, pos + 1, head_dim, D, head_dim, (int64_t)pos * D, head_dim, D};
   sh.kpb = keys_per_block;
@@ -836,23 +819,9 @@ int launch_llama_step_attn_bwd(hipStream_t st, const void* q, const void* k_cach
   sh.v_tail = v_tail;
   sh.dk_tail = dk_tail;
   sh.dv_tail = dv_tail;
-  const int nsplit = (pos + keys_per_block) / keys_per_block;
-  const float2* angles = reinterpret_cast<const float2*>(table);
-  if (nsplit == 1) {
-    sh.table = angles;
-    sh.table_pairs = table_pairs;
-    sh.fq = fq, sh.fk = fk, sh.fv = fv;
-  }
-  if (int rc = launch_step_bwd(st, q, k_cache, v_cache, o, lse, d_o, nullptr, dk_cache, dv_cache, part, sh, heads, true, scale, dtype)) return rc;
-  if (nsplit == 1) return EMI_OK;
-  if (dtype == EMI_BF16)
-    hipLaunchKernelGGL(step_qkv_cotangents_kernel<bf16>, dim3((unsigned)heads), dim3(128), 0, st, part, nsplit, (const bf16*)dk_tail,
-                       (const bf16*)dv_tail, angles, table_pairs, fq, fk, fv, head_dim);
-  else
-    hipLaunchKernelGGL(step_qkv_cotangents_kernel<float>, dim3((unsigned)heads), dim3(128), 0, st, part, nsplit, (const float*)dk_tail,
-                       (const float*)dv_tail, angles, table_pairs, fq, fk, fv, head_dim);
-  EMI_CHECK_LAUNCH("emi_llama_step_bwd(q, k, v)");
-  return EMI_OK;
+  sh.do_part = do_part;
+  sh.do_bands = do_bands;
+  return launch_step_bwd(st, q, k_cache, v_cache, o, lse, nullptr, nullptr, dk_cache, dv_cache, part, sh, heads, true, scale, dtype);
 }
 }  // namespace emi
 

@@ -216,6 +216,10 @@ __device__ __forceinline__ float row16_sum(float v) {          // over the 16 la
   v += ror16<2>(v);
   return v + ror16<1>(v);
 }
+__device__ __forceinline__ float quad_sum(float v) {           // over four neighbouring lanes
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0xb1, 0xf, 0xf, true));
+  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x4e, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float sum_xor32(float v) {          // over lanes l and l ^ 32
   const emi_u32x2_t p = pair32(v);
   return __uint_as_float(p[0]) + __uint_as_float(p[1]);

@@ -7,11 +7,11 @@
 // loaded or its result leaves, and the cache is not copied to append a row to it.
 //   forward, per layer:  norm + wq,wk,wv + rotation | attention over cache and own row (| combine) | wo + residual |
 //                        norm + w1,w3 + SwiGLU | w2 + residual;  with a short cache attention + wo + residual are one
-//   reverse, per layer:  w2^T dy and dw2 | SwiGLU' | w1^T dh1 + w3^T dh3 and dw1, dw3 | norm' (+ residual) |
-//                        wo^T dy and dwo | sum | attention' (|) dq, inverse rotation | wq^T dq + ... and dwq, dwk, dwv | norm'
+//   reverse, per layer:  norm' + w2^T dy and dw2 | SwiGLU' + w1^T dh1 + w3^T dh3 and dw1, dw3 | norm' + wo^T dy and dwo |
+//                        attention' | inverse rotation + wq^T dq + ... and dwq, dwk, dwv
 // The forward call leaves what the reverse one needs in `saved`.
 // Measured against the same step operator by operator (us): dim 288, 6 layers, fp32: forward 1071 -> 100 (99 launches ->
-// 25), with the reverse from StableHLO text at position 255 4042 -> 412 (289 launches -> 86); dim 4096, 2 layers, bf16,
+// 25), with the reverse from StableHLO text at position 255 4042 -> 330 (289 launches -> 62); dim 4096, 2 layers, bf16,
 // 4096 keys: forward 370 -> 211 (4.5 TB/s over weights and cache; 31 launches and two copies of each cache before).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -27,9 +27,9 @@ int launch_llama_step_attn_fwd(hipStream_t st, const void* q, const void* k_cach
                                const void* v_tail, void* o, float* lse, float* part, int heads, int pos, int head_dim, int keys_per_block,
                                float scale, int dtype);                                                      // attention_step.hip
 int launch_llama_step_attn_bwd(hipStream_t st, const void* q, const void* k_cache, const void* v_cache, const void* k_tail,
-                               const void* v_tail, const void* o, const float* lse, const void* d_o, void* dk_cache, void* dv_cache,
-                               void* dk_tail, void* dv_tail, float* part, const float* table, int table_pairs, float* fq, float* fk, float* fv,
-                               int heads, int pos, int head_dim, int keys_per_block, float scale, int dtype);
+                               const void* v_tail, const void* o, const float* lse, const float* do_part, int do_bands, void* dk_cache,
+                               void* dv_cache, void* dk_tail, void* dv_tail, float* part, int heads, int pos, int head_dim, int keys_per_block,
+                               float scale, int dtype);
 
 namespace {
 
@@ -336,224 +336,266 @@ __global__ __launch_bounds__(1024) void step_norm_kernel(const T* __restrict__ x
 // ---------------------------------------------------------------------------
 // reverse: W^T dy and dW = dy x^T of up to three matrices [K, N] that share x (and the cotangent of x)
 // ---------------------------------------------------------------------------
-// Every row of a matrix is read once (for the cotangent of x) while its gradient's row is written; HBM-bound on both.  A
-// thread owns one 16-byte piece of columns; a block's row lanes (as many as its columns leave) take the rows of a band in
-// turn, two register sets of UN rows in flight, and meet through LDS.  The bands' sums [bands][N] go to `part` in fp32.
+// Every row of a matrix is read once (for the cotangent of x) while its gradient's row is written; HBM-bound on both.  A block
+// owns `width` 16-byte pieces of columns and a band of rows; its row lanes (256 / width) take the band's rows in turn, two
+// register sets of UN rows in flight, and meet in the wavefront and through LDS.  The bands' sums [bands][N] go to `part` in fp32.
+//
+// What lies between two such products needs a value of every band: the norm's adjoint, the SwiGLU's, the inverse rotation.  The
+// kernel behind works it out itself, for its band's rows alone, while its first rows of W are on their way, so bands are few
+// (at most kMostBands, of narrow blocks) and the norm's one sum over all columns, which is linear in them, arrives as a share
+// of every block (`dots`).  Five launches a layer; nine when the bands were 96 and their sums launches of their own (a
+// norm's 5.7 us of one block, the others 2.6).
 template <typename T> struct Adjoint {
   const T* w[3];
   T* dw[3];
-  const float* dy[3];
   const T *x, *gamma;      // the products' operand: x, or with gamma the normalised gamma x rms
   const float* rms;
-  float* part;
-  int count, K, N, rows_per_band;
+  float *part, *dots;      // results; dots, with gamma: each block's share of the sum over the columns of part gamma x rms
+  int count, K, N, rows_per_band, width;
+  // the rows' cotangent: from the sums of the product behind, [in_bands][K]
+  const float *in, *in_dots;
+  int in_bands, in_ndots;
+  const T *nx, *ngamma;    // kNorm: the norm between, of nx; its adjoint plus `residual` leaves as dx (fp32) or dx_t
+  const float *nrms, *residual;
+  float* dx;
+  T *dx_t, *dgamma;
+  const T *h1, *h3;        // kSwiglu
+  const T *dk, *dv;        // kAttention: in is [heads][in_bands][head_dim + 2], dq's shares; dk, dv of the token's own row
+  const float2* table;
+  int table_pairs, head_dim;
 };
+enum { kNorm, kSwiglu, kAttention };
 
-template <typename T, bool STREAM>
+// In pairs: added one by one the bands' sums decided the error.
+template <int N> __device__ __forceinline__ float sum_pairs(float (&t)[N]) {
+#pragma unroll
+  for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; i++) t[i] += t[i + n];
+  return t[0];
+}
+// The sum of n values `stride` apart, by four neighbouring lanes; all four receive it.  Unconditional loads: the compiler
+// waits for each guarded one.
+__device__ __forceinline__ float bands_sum(const float* __restrict__ p, int64_t stride, int n) {
+  float v = 0.f;
+  for (int b0 = threadIdx.x & 3; b0 < n; b0 += 32) {
+    float t[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) t[u] = p[(b0 + 4 * u < n ? b0 + 4 * u : b0) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; u++) t[u] = b0 + 4 * u < n ? t[u] : 0.f;
+    v += sum_pairs(t);
+  }
+  return quad_sum(v);
+}
+
+// The cotangent of rows r_begin .. r_end, into LDS; four lanes a row.
+template <typename T, int FROM>
+__device__ __forceinline__ void rows_cotangent(const Adjoint<T>& a, int r_begin, int r_end, bool write, float* dy, float* scratch) {
+  float rs = 0.f, mean = 0.f;
+  if constexpr (FROM == kNorm) {
+    float dot = 0.f;
+    for (int i = threadIdx.x; i < a.in_ndots; i += 256) dot += a.in_dots[i];
+    mean = block_sum_f32(dot, scratch) / a.K;
+    rs = *a.nrms;
+  }
+  const bool first = (threadIdx.x & 3) == 0;
+  for (int r = r_begin + (threadIdx.x >> 2); r < r_end; r += 64) {
+    float o;
+    if constexpr (FROM == kNorm) {
+      const float d = bands_sum(a.in + r, a.K, a.in_bands);
+      const float xh = to_f32(a.nx[r]) * rs;
+      o = rs * (d * to_f32(a.ngamma[r]) - xh * mean);
+      if (a.residual != nullptr) o += a.residual[r];
+      if (write && first) {
+        a.dgamma[r] = from_f32<T>(d * xh);
+        if (a.dx_t != nullptr) a.dx_t[r] = from_f32<T>(o);
+        else a.dx[r] = o;
+      }
+    } else if constexpr (FROM == kSwiglu) {
+      const int k = r < a.K ? r : r - a.K;
+      float d1, d3;
+      emi_swiglu_adjoint(to_f32(a.h1[k]), to_f32(a.h3[k]), bands_sum(a.in + k, a.K, a.in_bands), &d1, &d3);
+      o = r < a.K ? d1 : d3;
+    } else {                                               // the rows of a pair turned back by the position's angle
+      const int m = r / a.K, k = r - m * a.K;
+      if (m == 2) {
+        o = to_f32(a.dv[k]);
+      } else {
+        const int h = k / a.head_dim, e = k - h * a.head_dim;
+        float own, other;
+        if (m == 0) {
+          const float* p = a.in + (int64_t)h * a.in_bands * (a.head_dim + 2);
+          own = bands_sum(p + e, a.head_dim + 2, a.in_bands);
+          other = bands_sum(p + (e ^ 1), a.head_dim + 2, a.in_bands);
+        } else {
+          own = to_f32(a.dk[k]);
+          other = to_f32(a.dk[k ^ 1]);
+        }
+        const float2 t = a.table[(k >> 1) % a.table_pairs];
+        o = (k & 1) == 0 ? t.x * own + t.y * other : t.x * own - t.y * other;
+      }
+    }
+    if (first) dy[r - r_begin] = o;
+  }
+}
+
+template <typename T, int FROM, bool STREAM>
 __global__ __launch_bounds__(256) void step_adjoint_kernel(Adjoint<T> a) {
   using Raw = typename ChunkCached<T>::Raw;
   constexpr int V = ChunkCached<T>::N, UN = 8;
-  __shared__ float red[256][V + 1];
-  const int pieces = a.N / V;
-  const int width = pieces < 256 ? pieces : 256, lanes = 256 / width;       // columns of a block, row lanes
-  const int rl = threadIdx.x / width, cl = threadIdx.x % width;
-  const int piece = blockIdx.x * width + cl, n = piece * V;
-  const bool live = rl < lanes && piece < pieces;
+  extern __shared__ float dy[];                            // [rows_per_band]
+  __shared__ float red[4][64][V + 1];
+  __shared__ float scratch[4];
+  const int pieces = a.N / V, lanes = 256 / a.width;
+  const int rl = threadIdx.x / a.width, cl = threadIdx.x % a.width;
+  const int piece = blockIdx.x * a.width + cl, n = piece * V;
+  const bool live = piece < pieces;
   const int total = a.count * a.K;
   const int r_begin = blockIdx.y * a.rows_per_band, r_end = r_begin + a.rows_per_band < total ? r_begin + a.rows_per_band : total;
-  float acc[V], xv[V];
+  float acc[V], xv[V], gx[V];                              // gx: gamma x rms before it is rounded
 #pragma unroll
-  for (int e = 0; e < V; e++) acc[e] = xv[e] = 0.f;
+  for (int e = 0; e < V; e++) acc[e] = xv[e] = gx[e] = 0.f;
+  auto matrix = [&](int r) { return a.count == 1 ? 0 : r / a.K; };
+  auto pick = [](auto&& p, int m) { return m == 0 ? p[0] : m == 1 ? p[1] : p[2]; };
+  auto issue = [&](int r0, Raw(&w)[UN]) {
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      const int r = r0 + u * lanes < r_end ? r0 + u * lanes : r_end - 1;            // past the band: its last row, unused
+      const int m = matrix(r), k = r - m * a.K;
+      w[u] = Chunk<T>::load_raw(pick(a.w, m) + (int64_t)k * a.N + n);
+    }
+  };
+  auto consume = [&](int r0, const Raw(&w)[UN]) {
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      const int r = r0 + u * lanes;
+      if (r < r_end) {
+        const int m = matrix(r), k = r - m * a.K;
+        const float d = dy[r - r_begin];
+        float wv[V], o[V];
+        ChunkCached<T>::unpack(w[u], wv);
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+          acc[e] = fmaf(d, wv[e], acc[e]);
+          o[e] = d * xv[e];
+        }
+        T* dst = pick(a.dw, m) + (int64_t)k * a.N + n;
+        if constexpr (STREAM) Chunk<T>::store(dst, o);
+        else ChunkCached<T>::store(dst, o);
+      }
+    }
+  };
+  Raw w0[UN], w1[UN];
+  int r = r_begin + rl;
   if (live) {
+    if (r < r_end) issue(r, w0);
     ChunkCached<T>::load(a.x + n, xv);
     if (a.gamma != nullptr) {
       float gv[V];
       ChunkCached<T>::load(a.gamma + n, gv);
       const float rs = *a.rms;
 #pragma unroll
-      for (int e = 0; e < V; e++) xv[e] = normed<T>(xv[e], gv[e], rs);
+      for (int e = 0; e < V; e++) {
+        gx[e] = gv[e] * (xv[e] * rs);
+        xv[e] = round_to<T>(gx[e]);
+      }
     }
-    auto matrix = [&](int r) { return a.count == 1 ? 0 : r / a.K; };
-    auto pick = [](auto&& p, int m) { return m == 0 ? p[0] : m == 1 ? p[1] : p[2]; };
-    auto issue = [&](int r0, Raw(&w)[UN], float(&d)[UN]) {
-#pragma unroll
-      for (int u = 0; u < UN; u++) {
-        const int r = r0 + u * lanes < r_end ? r0 + u * lanes : r_end - 1;            // past the band: its last row, unused
-        const int m = matrix(r), k = r - m * a.K;
-        w[u] = Chunk<T>::load_raw(pick(a.w, m) + (int64_t)k * a.N + n);
-        d[u] = pick(a.dy, m)[k];
-      }
-    };
-    auto consume = [&](int r0, const Raw(&w)[UN], const float(&d)[UN]) {
-#pragma unroll
-      for (int u = 0; u < UN; u++) {
-        const int r = r0 + u * lanes;
-        if (r < r_end) {
-          const int m = matrix(r), k = r - m * a.K;
-          float wv[V], o[V];
-          ChunkCached<T>::unpack(w[u], wv);
-#pragma unroll
-          for (int e = 0; e < V; e++) {
-            acc[e] = fmaf(d[u], wv[e], acc[e]);
-            o[e] = d[u] * xv[e];
-          }
-          T* dst = pick(a.dw, m) + (int64_t)k * a.N + n;
-          if constexpr (STREAM) Chunk<T>::store(dst, o);
-          else ChunkCached<T>::store(dst, o);
-        }
-      }
-    };
-    Raw w0[UN], w1[UN];
-    float d0[UN], d1[UN];
-    int r = r_begin + rl;
-    if (r < r_end) issue(r, w0, d0);
+  }
+  rows_cotangent<T, FROM>(a, r_begin, r_end, blockIdx.x == 0, dy, scratch);
+  __syncthreads();
+  if (live) {
     while (r < r_end) {
       const int r1 = r + UN * lanes;
-      if (r1 < r_end) issue(r1, w1, d1);
-      consume(r, w0, d0);
+      if (r1 < r_end) issue(r1, w1);
+      consume(r, w0);
       if (r1 >= r_end) break;
       r = r1 + UN * lanes;
-      if (r < r_end) issue(r, w0, d0);
-      consume(r1, w1, d1);
+      if (r < r_end) issue(r, w0);
+      consume(r1, w1);
     }
   }
-  if (lanes > 1) {
+  // the row lanes of a wavefront, then the wavefronts
 #pragma unroll
-    for (int e = 0; e < V; e++) red[threadIdx.x][e] = acc[e];
-    __syncthreads();
-    if (rl == 0 && live) {
-      for (int l = 1; l < lanes; l++)
-#pragma unroll
-        for (int e = 0; e < V; e++) acc[e] += red[l * width + cl][e];
-    }
+  for (int e = 0; e < V; e++) {
+    if (a.width <= 32) acc[e] = sum_xor32(acc[e]);
+    if (a.width <= 16) acc[e] = sum_xor16(acc[e]);
+    if (a.width <= 8) acc[e] += ror16<8>(acc[e]);
+    red[threadIdx.x >> 6][threadIdx.x & 63][e] = acc[e];
   }
-  if (rl == 0 && live) {
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  float dot = 0.f;
+  if ((int)threadIdx.x < a.width && live) {
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+      acc[e] = (red[0][threadIdx.x][e] + red[1][threadIdx.x][e]) + (red[2][threadIdx.x][e] + red[3][threadIdx.x][e]);
+      dot = fmaf(acc[e], gx[e], dot);
+    }
     float* dst = a.part + (int64_t)blockIdx.y * a.N + n;
 #pragma unroll
     for (int e = 0; e < V; e += 4) *reinterpret_cast<f4*>(dst + e) = f4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
   }
+  if (a.gamma == nullptr) return;
+  dot = wave_sum(dot);
+  if (threadIdx.x == 0) a.dots[blockIdx.y * gridDim.x + blockIdx.x] = dot;
 }
 
-// Bands of rows: about two blocks per CU where there are rows enough, at least two rows per row lane.
-template <typename T> int adjoint_bands(int count, int K, int N) {
+// Blocks: as narrow as leaves eight of them side by side (a row's share is at least 128 bytes), so that bands are few, and about
+// two per CU where there are rows enough, at least two a row lane.
+constexpr int kMostBands = 64, kMostRows = 4096;           // rows: of a band, their cotangent stands in LDS
+struct AdjointGrid { int width, cols, bands, rows_per_band; };
+template <typename T> AdjointGrid adjoint_grid(int count, int K, int N) {
   constexpr int V = ChunkCached<T>::N;
-  const int pieces = N / V, width = pieces < 256 ? pieces : 256, lanes = 256 / width, cols = (pieces + width - 1) / width;
-  int bands = (512 + cols - 1) / cols;
-  const int most = (count * K + 2 * lanes - 1) / (2 * lanes);
+  const int pieces = N / V, total = count * K;
+  AdjointGrid g;
+  g.width = 64;
+  while (g.width > 8 && pieces < 8 * g.width) g.width /= 2;
+  g.cols = (pieces + g.width - 1) / g.width;
+  const int lanes = 256 / g.width, most = (total + 2 * lanes - 1) / (2 * lanes);
+  int bands = (512 + g.cols - 1) / g.cols;
   if (bands > most) bands = most;
-  if (bands > 96 && N <= 1024) bands = 96;           // short vectors: the bands are summed by one block (step_norm_adjoint_kernel)
-  return bands < 1 ? 1 : bands;
+  if (bands > kMostBands) bands = kMostBands;
+  if (bands < (total + kMostRows - 1) / kMostRows) bands = (total + kMostRows - 1) / kMostRows;
+  g.rows_per_band = (total + bands - 1) / bands;
+  g.bands = (total + g.rows_per_band - 1) / g.rows_per_band;
+  return g;
 }
 
-template <typename T> int launch_adjoint(hipStream_t st, Adjoint<T> a, int* bands) {
-  constexpr int V = ChunkCached<T>::N;
-  const int pieces = a.N / V, width = pieces < 256 ? pieces : 256;
-  const int want = adjoint_bands<T>(a.count, a.K, a.N), total = a.count * a.K;
-  a.rows_per_band = (total + want - 1) / want;
-  *bands = (total + a.rows_per_band - 1) / a.rows_per_band;
-  const dim3 grid((unsigned)((pieces + width - 1) / width), (unsigned)*bands);
-  if ((size_t)total * a.N * sizeof(T) > ((size_t)32 << 20))
-    hipLaunchKernelGGL((step_adjoint_kernel<T, true>), grid, dim3(256), 0, st, a);
+template <typename T, int FROM> int launch_adjoint(hipStream_t st, Adjoint<T> a, const AdjointGrid& g) {
+  a.width = g.width;
+  a.rows_per_band = g.rows_per_band;
+  const dim3 grid((unsigned)g.cols, (unsigned)g.bands);
+  const size_t lds = (size_t)g.rows_per_band * sizeof(float);
+  if ((size_t)a.count * a.K * a.N * sizeof(T) > ((size_t)32 << 20))
+    hipLaunchKernelGGL((step_adjoint_kernel<T, FROM, true>), grid, dim3(256), lds, st, a);
   else
-    hipLaunchKernelGGL((step_adjoint_kernel<T, false>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((step_adjoint_kernel<T, FROM, false>), grid, dim3(256), lds, st, a);
   EMI_CHECK_LAUNCH("emi_llama_step(adjoint products)");
   return EMI_OK;
 }
 
-// In pairs: the bands' sums are longer than the chains within them (768 columns: 96 bands of 43 rows), and added one by
-// one they decided the error.
-__device__ __forceinline__ float sum8(const float (&t)[8]) { return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7])); }
-
-// The sum over the bands of 16 columns per block: 16 band lanes with up to eight loads in flight each, met through LDS in
-// order.  The result is valid in threads 0 .. 15.
-__device__ __forceinline__ float sum_bands16(const float* __restrict__ part, int bands, int N, int n, float (*red)[16]) {
-  const int col = threadIdx.x & 15, bl = threadIdx.x >> 4;
-  float v = 0.f;
-  if (n < N) {
-    for (int b0 = bl; b0 < bands; b0 += 128) {
-      float t[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) t[u] = b0 + 16 * u < bands ? part[(int64_t)(b0 + 16 * u) * N + n] : 0.f;
-      v += sum8(t);
-    }
-  }
-  red[bl][col] = v;
-  __syncthreads();
-  if (bl == 0) {
-    v = 0.f;
-#pragma unroll
-    for (int b = 0; b < 16; b++) v += red[b][col];
-  }
-  return v;
-}
-
-// OUT 0: the sum as T;  1: as fp32;  2: the sum is dg, (dh1, dh3) of the SwiGLU as fp32.
-template <typename T, int OUT>
-__global__ __launch_bounds__(256) void step_bands_kernel(const float* __restrict__ part, int bands, int N, T* __restrict__ y,
-                                                         float* __restrict__ f0, float* __restrict__ f1, const T* __restrict__ h1,
-                                                         const T* __restrict__ h3) {
-  __shared__ float red[16][16];
-  const int n = blockIdx.x * 16 + (threadIdx.x & 15);
-  const float v = sum_bands16(part, bands, N, n, red);
-  if (threadIdx.x >= 16 || n >= N) return;
-  if constexpr (OUT == 0) y[n] = from_f32<T>(v);
-  else if constexpr (OUT == 1) f0[n] = v;
-  else emi_swiglu_adjoint(to_f32(h1[n]), to_f32(h3[n]), v, f0 + n, f1 + n);
-}
-
-// Adjoint of y = gamma x rms: from the cotangent of y (the sum of `bands` rows, or T with bands == 0) the one of gamma, and
-// the one of x plus the residual's, as fp32 (for the next products) or T.  One block: the vector is short.
+// The first norm's adjoint of the reverse pass, whose cotangent is the caller's: one band and its dot.  One block: the vector is short.
 template <typename T>
-__global__ __launch_bounds__(1024) void step_norm_adjoint_kernel(const float* __restrict__ part, int bands, const T* __restrict__ ct,
-                                                                 const T* __restrict__ x, const T* __restrict__ gamma,
-                                                                 const float* __restrict__ rms, const float* __restrict__ residual,
-                                                                 T* __restrict__ dgamma, float* __restrict__ dx, T* __restrict__ dx_t, int D) {
-  extern __shared__ float dy[];                         // [D], then [1024] for band lanes
+__global__ __launch_bounds__(1024) void step_cotangent_kernel(const T* __restrict__ ct, const T* __restrict__ x, const T* __restrict__ gamma,
+                                                              const float* __restrict__ rms, float* __restrict__ part, float* __restrict__ dots,
+                                                              int D) {
   __shared__ float scratch[16];
   const float rs = *rms;
-  if (bands > 1) {
-    // band lanes: as many columns side by side as there are, the threads left share the bands
-    const int width = D < 1024 ? D : 1024, lanes = 1024 / width;
-    const int bl = threadIdx.x / width, cl = threadIdx.x % width;
-    float* red = dy + D;
-    for (int n0 = 0; n0 < D; n0 += width) {
-      const int n = n0 + cl;
-      float v = 0.f;
-      if (bl < lanes && n < D) {
-        for (int b0 = bl; b0 < bands; b0 += lanes * 8) {
-          float t[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) t[u] = b0 + lanes * u < bands ? part[(int64_t)(b0 + lanes * u) * D + n] : 0.f;
-          v += sum8(t);
-        }
-      }
-      if (lanes > 1) {
-        red[threadIdx.x] = v;
-        __syncthreads();
-        if (bl == 0) {
-          v = 0.f;
-          for (int l = 0; l < lanes; l++) v += red[l * width + cl];
-        }
-        __syncthreads();
-      }
-      if (bl == 0 && n < D) dy[n] = v;
-    }
-    __syncthreads();
-  } else {
-    for (int n = threadIdx.x; n < D; n += 1024) dy[n] = bands == 1 ? part[n] : to_f32(ct[n]);
-    __syncthreads();
-  }
-  float dot = 0.f;                                      // sum of dy gamma xhat
-  for (int n = threadIdx.x; n < D; n += 1024) dot = fmaf(dy[n] * to_f32(gamma[n]), to_f32(x[n]) * rs, dot);
-  const float mean = block_sum_f32(dot, scratch) / D;
+  float dot = 0.f;
   for (int n = threadIdx.x; n < D; n += 1024) {
-    const float xh = to_f32(x[n]) * rs, d = dy[n];
-    dgamma[n] = from_f32<T>(d * xh);
-    float v = rs * (d * to_f32(gamma[n]) - xh * mean);
-    if (residual != nullptr) v += residual[n];
-    if (dx_t != nullptr) dx_t[n] = from_f32<T>(v);
-    else dx[n] = v;
+    const float d = to_f32(ct[n]);
+    part[n] = d;
+    dot = fmaf(d, to_f32(gamma[n]) * (to_f32(x[n]) * rs), dot);
   }
+  dot = block_sum_f32(dot, scratch);
+  if (threadIdx.x == 0) *dots = dot;
+}
+// The last one's, which no product follows: 64 columns a block.
+template <typename T> __global__ __launch_bounds__(256) void step_norm_rows_kernel(Adjoint<T> a) {
+  __shared__ float dy[64], scratch[4];
+  const int r0 = blockIdx.x * 64;
+  rows_cotangent<T, kNorm>(a, r0, r0 + 64 < a.K ? r0 + 64 : a.K, true, dy, scratch);
 }
 
 // ---------------------------------------------------------------------------
@@ -577,6 +619,12 @@ struct StepDims {
     return lanes <= 16 && (heads + 15) / 16 * ((pos + kStepKeys) / kStepKeys) <= kStepRounds;
   }
   int nsplit() const { return (int)((pos + 1 + kpb() - 1) / kpb()); }
+  // the adjoint's: the product behind adds up its blocks' shares, so 64 keys, one pass of its loads, until they fill the chip
+  int kpb_bwd() const {
+    const int64_t want = ((pos + 1) * heads / 512 + 63) / 64 * 64;
+    return (int)(want < 64 ? 64 : want > 512 ? 512 : want);
+  }
+  int nsplit_bwd() const { return (int)((pos + kpb_bwd()) / kpb_bwd()); }
 };
 
 struct Carve {                                            // consecutive 256-byte aligned pieces of a buffer
@@ -698,46 +746,32 @@ int step_fwd(hipStream_t st, const void* const* w, const void* x_, const void* k
   return EMI_OK;
 }
 
-// Scratch of the reverse pass; L, pos do not enter except through the attention's blocks.
+// Scratch of the reverse pass; L does not enter, pos only through the attention's blocks.  A product reads the sums of the one
+// before while it leaves its own: two sets.
 template <typename T> struct BwdWork {
-  float *part, *attn, *dx_a, *dx_b, *f0, *f1, *f2, *dsum;
-  T *datt, *dk, *dv;
+  float *part[2], *dots, *attn, *dx_a, *dx_b;
+  T *dk, *dv;
 };
 template <typename T> BwdWork<T> carve_bwd(Carve& c, const StepDims& d) {
   BwdWork<T> s;
-  auto rows = [&](int count, int64_t K, int64_t N) { return (size_t)adjoint_bands<T>(count, (int)K, (int)N) * N; };
-  size_t part = rows(1, d.D, d.H);
-  for (size_t n : {rows(2, d.H, d.D), rows(1, d.D, d.D), rows(3, d.D, d.D)})
-    if (n > part) part = n;
-  s.part = c.take<float>(part);
-  s.attn = c.take<float>((size_t)d.heads * d.nsplit() * (d.hd() + 2));
+  size_t part = (size_t)d.D, dots = 1;
+  auto take = [&](int count, int64_t K, int64_t N) {
+    const AdjointGrid g = adjoint_grid<T>(count, (int)K, (int)N);
+    if ((size_t)g.bands * N > part) part = (size_t)g.bands * N;
+    if ((size_t)g.bands * g.cols > dots) dots = (size_t)g.bands * g.cols;
+  };
+  take(1, d.D, d.H);
+  take(2, d.H, d.D);
+  take(1, d.D, d.D);
+  take(3, d.D, d.D);
+  for (float*& p : s.part) p = c.take<float>(part);
+  s.dots = c.take<float>(dots);
+  s.attn = c.take<float>((size_t)d.heads * d.nsplit_bwd() * (d.hd() + 2));
   s.dx_a = c.take<float>(d.D);
   s.dx_b = c.take<float>(d.D);
-  s.f0 = c.take<float>(d.D > d.H ? d.D : d.H);
-  s.f1 = c.take<float>(d.D > d.H ? d.D : d.H);
-  s.f2 = c.take<float>(d.D);
-  s.dsum = c.take<float>(d.D);
-  s.datt = c.take<T>(d.D);
   s.dk = c.take<T>(d.D);
   s.dv = c.take<T>(d.D);
   return s;
-}
-
-template <typename T>
-int norm_adjoint(hipStream_t st, const BwdWork<T>& k, int bands, const T* ct, const T* x, const T* gamma, const float* rms,
-                 const float* residual, T* dgamma, float* dx, T* dx_t, int D) {
-  const float* part = k.part;
-  if (bands > 1 && (int64_t)bands * D > 96 * 1024) {       // more than one block should sum: its own launch
-    hipLaunchKernelGGL((step_bands_kernel<T, 1>), dim3((unsigned)((D + 15) / 16)), dim3(256), 0, st, k.part, bands, D, (T*)nullptr, k.dsum,
-                       (float*)nullptr, (const T*)nullptr, (const T*)nullptr);
-    EMI_CHECK_LAUNCH("emi_llama_step_bwd(bands)");
-    part = k.dsum;
-    bands = 1;
-  }
-  hipLaunchKernelGGL(step_norm_adjoint_kernel<T>, dim3(1), dim3(1024), (size_t)(D + 1024) * sizeof(float), st, part, bands, ct, x, gamma, rms,
-                     residual, dgamma, dx, dx_t, D);
-  EMI_CHECK_LAUNCH("emi_llama_step_bwd(norm)");
-  return EMI_OK;
 }
 
 template <typename T>
@@ -757,47 +791,59 @@ int step_bwd(hipStream_t st, const void* const* w, const void* x_, const void* k
   const size_t layer_bytes = probe.at;
   Carve all{(uint8_t*)const_cast<void*>(saved), layer_bytes * (size_t)d.L};
   SavedAll<T> tail = carve_tail<T>(all, d);
-  float *dx = k.dx_a, *dx1 = k.dx_b;
-  if (int rc = norm_adjoint<T>(st, k, 0, (const T*)dy, tail.x_out, (const T*)w[9], tail.rms, nullptr, gr[10], dx, nullptr, (int)D)) return rc;
+  const AdjointGrid gw2 = adjoint_grid<T>(1, (int)D, (int)H), gw13 = adjoint_grid<T>(2, (int)H, (int)D), gwo = adjoint_grid<T>(1, (int)D, (int)D),
+                    gqkv = adjoint_grid<T>(3, (int)D, (int)D);
+  hipLaunchKernelGGL(step_cotangent_kernel<T>, dim3(1), dim3(1024), 0, st, (const T*)dy, tail.x_out, (const T*)w[9], tail.rms, k.part[1], k.dots,
+                     (int)D);
+  EMI_CHECK_LAUNCH("emi_llama_step_bwd(cotangent)");
+  // what the norm between two products needs: of the layer's input, or of the result
+  Adjoint<T> norm{};
+  norm.in = k.part[1], norm.in_dots = k.dots, norm.in_bands = norm.in_ndots = 1;
+  norm.nx = tail.x_out, norm.ngamma = (const T*)w[9], norm.nrms = tail.rms;
+  norm.dgamma = gr[10], norm.dx = k.dx_a;
   for (int64_t l = d.L - 1; l >= 0; l--) {
     Carve c{(uint8_t*)const_cast<void*>(saved), layer_bytes * (size_t)l};
     const Saved<T> s = carve_layer<T>(c, d);
     const T* x = l == 0 ? (const T*)x_ : s.x;
-    int bands = 1;
-    Adjoint<T> a{};
-    a.w[0] = w2 + l * D * H, a.dw[0] = gr[8] + l * D * H, a.dy[0] = dx;                       // w2 [D, H]
-    a.x = s.g, a.part = k.part, a.count = 1, a.K = (int)D, a.N = (int)H;
-    if (int rc = launch_adjoint<T>(st, a, &bands)) return rc;
-    hipLaunchKernelGGL((step_bands_kernel<T, 2>), dim3((unsigned)((H + 15) / 16)), dim3(256), 0, st, k.part, bands, (int)H, (T*)nullptr, k.f0,
-                       k.f1, s.h1, s.h3);
-    EMI_CHECK_LAUNCH("emi_llama_step_bwd(swiglu)");
+    Adjoint<T> a = norm;
+    a.w[0] = w2 + l * D * H, a.dw[0] = gr[8] + l * D * H;                                     // w2 [D, H]
+    a.x = s.g, a.part = k.part[0], a.count = 1, a.K = (int)D, a.N = (int)H;
+    if (int rc = launch_adjoint<T, kNorm>(st, a, gw2)) return rc;
     a = Adjoint<T>{};
-    a.w[0] = w1 + l * H * D, a.dw[0] = gr[7] + l * H * D, a.dy[0] = k.f0;                     // w1, w3 [H, D]
-    a.w[1] = w3 + l * H * D, a.dw[1] = gr[9] + l * H * D, a.dy[1] = k.f1;
-    a.x = s.x1, a.gamma = g2 + l * D, a.rms = s.rms2, a.part = k.part, a.count = 2, a.K = (int)H, a.N = (int)D;
-    if (int rc = launch_adjoint<T>(st, a, &bands)) return rc;
-    if (int rc = norm_adjoint<T>(st, k, bands, nullptr, s.x1, g2 + l * D, s.rms2, dx, gr[6] + l * D, dx1, nullptr, (int)D)) return rc;
+    a.w[0] = w1 + l * H * D, a.dw[0] = gr[7] + l * H * D;                                     // w1, w3 [H, D]
+    a.w[1] = w3 + l * H * D, a.dw[1] = gr[9] + l * H * D;
+    a.x = s.x1, a.gamma = g2 + l * D, a.rms = s.rms2;
+    a.part = k.part[1], a.dots = k.dots, a.count = 2, a.K = (int)H, a.N = (int)D;
+    a.in = k.part[0], a.in_bands = gw2.bands, a.h1 = s.h1, a.h3 = s.h3;
+    if (int rc = launch_adjoint<T, kSwiglu>(st, a, gw13)) return rc;
     a = Adjoint<T>{};
-    a.w[0] = wo + l * D * D, a.dw[0] = gr[5] + l * D * D, a.dy[0] = dx1;                      // wo [D, D]
-    a.x = s.att, a.part = k.part, a.count = 1, a.K = (int)D, a.N = (int)D;
-    if (int rc = launch_adjoint<T>(st, a, &bands)) return rc;
-    hipLaunchKernelGGL((step_bands_kernel<T, 0>), dim3((unsigned)((D + 15) / 16)), dim3(256), 0, st, k.part, bands, (int)D, k.datt,
-                       (float*)nullptr, (float*)nullptr, (const T*)nullptr, (const T*)nullptr);
-    EMI_CHECK_LAUNCH("emi_llama_step_bwd(sum)");
+    a.w[0] = wo + l * D * D, a.dw[0] = gr[5] + l * D * D;                                     // wo [D, D]
+    a.x = s.att, a.part = k.part[0], a.count = 1, a.K = (int)D, a.N = (int)D;
+    a.in = k.part[1], a.in_dots = k.dots, a.in_bands = gw13.bands, a.in_ndots = gw13.bands * gw13.cols;
+    a.nx = s.x1, a.ngamma = g2 + l * D, a.nrms = s.rms2, a.residual = k.dx_a;
+    a.dgamma = gr[6] + l * D, a.dx = k.dx_b;
+    if (int rc = launch_adjoint<T, kNorm>(st, a, gwo)) return rc;
     const int64_t cache = l * d.pos * D;
-    if (int rc = launch_llama_step_attn_bwd(st, s.q, kc + cache, vc + cache, s.k, s.v, s.att, s.lse, k.datt, gr[11] + cache, gr[12] + cache,
-                                            k.dk, k.dv, k.attn, table, (int)d.table_pairs, k.f0, k.f1, k.f2, (int)d.heads, (int)d.pos, d.hd(),
-                                            d.kpb(), d.scale, d.dtype))
+    if (int rc = launch_llama_step_attn_bwd(st, s.q, kc + cache, vc + cache, s.k, s.v, s.att, s.lse, k.part[0], gwo.bands, gr[11] + cache,
+                                            gr[12] + cache, k.dk, k.dv, k.attn, (int)d.heads, (int)d.pos, d.hd(), d.kpb_bwd(), d.scale, d.dtype))
       return rc;
     a = Adjoint<T>{};
-    a.w[0] = wq + l * D * D, a.dw[0] = gr[2] + l * D * D, a.dy[0] = k.f0;
-    a.w[1] = wk + l * D * D, a.dw[1] = gr[3] + l * D * D, a.dy[1] = k.f1;
-    a.w[2] = wv + l * D * D, a.dw[2] = gr[4] + l * D * D, a.dy[2] = k.f2;
-    a.x = x, a.gamma = g1 + l * D, a.rms = s.rms1, a.part = k.part, a.count = 3, a.K = (int)D, a.N = (int)D;
-    if (int rc = launch_adjoint<T>(st, a, &bands)) return rc;
-    if (int rc = norm_adjoint<T>(st, k, bands, nullptr, x, g1 + l * D, s.rms1, dx1, gr[1] + l * D, dx, l == 0 ? gr[0] : nullptr, (int)D))
-      return rc;
+    a.w[0] = wq + l * D * D, a.dw[0] = gr[2] + l * D * D;
+    a.w[1] = wk + l * D * D, a.dw[1] = gr[3] + l * D * D;
+    a.w[2] = wv + l * D * D, a.dw[2] = gr[4] + l * D * D;
+    a.x = x, a.gamma = g1 + l * D, a.rms = s.rms1;
+    a.part = k.part[1], a.dots = k.dots, a.count = 3, a.K = (int)D, a.N = (int)D;
+    a.in = k.attn, a.in_bands = d.nsplit_bwd(), a.dk = k.dk, a.dv = k.dv;
+    a.table = (const float2*)table, a.table_pairs = (int)d.table_pairs, a.head_dim = d.hd();
+    if (int rc = launch_adjoint<T, kAttention>(st, a, gqkv)) return rc;
+    norm = Adjoint<T>{};
+    norm.in = k.part[1], norm.in_dots = k.dots, norm.in_bands = gqkv.bands, norm.in_ndots = gqkv.bands * gqkv.cols;
+    norm.nx = x, norm.ngamma = g1 + l * D, norm.nrms = s.rms1, norm.residual = k.dx_b;
+    norm.dgamma = gr[1] + l * D, norm.dx = k.dx_a;
   }
+  norm.dx_t = gr[0], norm.K = (int)D;
+  hipLaunchKernelGGL(step_norm_rows_kernel<T>, dim3((unsigned)((D + 63) / 64)), dim3(256), 0, st, norm);
+  EMI_CHECK_LAUNCH("emi_llama_step_bwd(norm)");
   return EMI_OK;
 }
 

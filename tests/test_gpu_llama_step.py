@@ -57,6 +57,27 @@ def test_llama_step_matches_oracle(dt, dim, hidden, layers, heads, pos):
         check(gw[k], rgw[k], dt, "d" + k, factor=2.0 if k == "wk" and dt == "bf16" else 1.0)
 
 
+@pytest.mark.parametrize("dt,dim,hidden,heads,pos", [
+    ("f32", 272, 520, 4, 70),             # blocks of 8 pieces, the last one cut; two blocks of keys
+    ("f32", 16, 131080, 1, 3),            # half a block of pieces; more rows than the bands of at most 4096 take
+    ("f32", 528, 1412, 6, 130),           # 16 pieces; bands that do not divide the rows
+    ("f32", 1040, 300, 5, 4),             # 32
+    ("f32", 2064, 36, 12, 64),            # 64; nine bands' worth of rows in a hidden layer shorter than a band
+    ("bf16", 4160, 72, 20, 5),            # 64, and one row lane a wavefront
+])
+def test_llama_step_adjoint_blocks(dt, dim, hidden, heads, pos):
+    """Block widths and bands of the reverse products, whose sums the next product adds up for its own rows."""
+    from enzyme_ad.jax import llama, vjp
+    cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), (dy, dyr)) = _inputs(dt, dim, hidden, 2 if dim < 1000 else 1, heads, pos, dim + pos)
+    y, pull = vjp(lambda x, w, k, v: llama.forward_step(x, cfg, w, k, v), x, wd, kc, vc)
+    gx, gw, gk, gv = pull(dy)
+    ry, rdx, rgw, rdk, rdv = L.forward_step_vjp(xr, cfg, wr, kcr, vcr, dyr)
+    for got, want, name in ((y, ry, "y"), (gx, rdx, "dx"), (gk, rdk, "dkey_cache"), (gv, rdv, "dvalue_cache")):
+        check(got, want, dt, name)
+    for k in wd:
+        check(gw[k], rgw[k], dt, "d" + k, factor=2.0 if k == "wk" and dt == "bf16" else 1.0)      # see above
+
+
 def test_llama_step_accumulates_and_repeats():
     """The step's cotangents add to what other uses of its operands contribute, and are the same bits run to run."""
     from enzyme_ad.jax import llama, ops, vjp
