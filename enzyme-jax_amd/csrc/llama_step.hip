@@ -389,30 +389,43 @@ __device__ __forceinline__ float bands_sum(const float* __restrict__ p, int64_t 
   return quad_sum(v);
 }
 
-// The cotangent of rows r_begin .. r_end, into LDS; four lanes a row.
+// The cotangent of rows r_begin .. r_end, into LDS; four lanes a row.  The norm's mean needs the whole block: the first rows' sums
+// are requested before it.
 template <typename T, int FROM>
 __device__ __forceinline__ void rows_cotangent(const Adjoint<T>& a, int r_begin, int r_end, bool write, float* dy, float* scratch) {
-  float rs = 0.f, mean = 0.f;
+  const bool first = (threadIdx.x & 3) == 0;
+  int r = r_begin + (threadIdx.x >> 2);
   if constexpr (FROM == kNorm) {
     float dot = 0.f;
     for (int i = threadIdx.x; i < a.in_ndots; i += 256) dot += a.in_dots[i];
-    mean = block_sum_f32(dot, scratch) / a.K;
-    rs = *a.nrms;
-  }
-  const bool first = (threadIdx.x & 3) == 0;
-  for (int r = r_begin + (threadIdx.x >> 2); r < r_end; r += 64) {
-    float o;
-    if constexpr (FROM == kNorm) {
-      const float d = bands_sum(a.in + r, a.K, a.in_bands);
-      const float xh = to_f32(a.nx[r]) * rs;
-      o = rs * (d * to_f32(a.ngamma[r]) - xh * mean);
-      if (a.residual != nullptr) o += a.residual[r];
+    const float rs = *a.nrms;
+    float d = 0.f, g = 0.f, xh = 0.f, res = 0.f;
+    auto load = [&]() {
+      if (r < r_end) {
+        g = to_f32(a.ngamma[r]);
+        xh = to_f32(a.nx[r]) * rs;
+        if (a.residual != nullptr) res = a.residual[r];
+        d = bands_sum(a.in + r, a.K, a.in_bands);
+      }
+    };
+    load();
+    const float mean = block_sum_f32(dot, scratch) / a.K;
+    while (r < r_end) {
+      const float o = rs * (d * g - xh * mean) + res;
       if (write && first) {
         a.dgamma[r] = from_f32<T>(d * xh);
         if (a.dx_t != nullptr) a.dx_t[r] = from_f32<T>(o);
         else a.dx[r] = o;
       }
-    } else if constexpr (FROM == kSwiglu) {
+      if (first) dy[r - r_begin] = o;
+      r += 64;
+      load();
+    }
+    return;
+  }
+  for (; r < r_end; r += 64) {
+    float o;
+    if constexpr (FROM == kSwiglu) {
       const int k = r < a.K ? r : r - a.K;
       float d1, d3;
       emi_swiglu_adjoint(to_f32(a.h1[k]), to_f32(a.h3[k]), bands_sum(a.in + k, a.K, a.in_bands), &d1, &d3);
