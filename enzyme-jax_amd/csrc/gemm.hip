@@ -2068,6 +2068,19 @@ int emi::gemm_run(hipStream_t st, const void* A, const void* B, const void* R, v
   return launch_generic<float>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
 }
 
+int emi::gemm_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b,
+                   int dtype) {
+  // rows of whole 16-byte pieces, operands and results of less than 2 GiB
+  const int64_t v = dtype == EMI_BF16 ? 8 : 4, most = 0x7fffff00LL / (dtype == EMI_BF16 ? 2 : 4), b_rows = trans_b ? N : K;
+  if (M <= 8 || N <= 0 || K <= 0 || N % v || K % v || ldb % v || M * K >= most || b_rows * ldb >= most || M * N >= most) return -1;
+  uintptr_t all = reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(t.h1) |
+                  reinterpret_cast<uintptr_t>(t.h3) | reinterpret_cast<uintptr_t>(t.table);
+  for (int i = 0; i < 3; i++) all |= reinterpret_cast<uintptr_t>(t.B[i]) | reinterpret_cast<uintptr_t>(t.C[i]);
+  if (all & 15) return -1;
+  return dtype == EMI_BF16 ? launch_bf16_pipe_tail(st, A, B, t, (int)M, (int)N, (int)K, (int)ldb, trans_b)
+                           : launch_f32_tail(st, A, B, t, M, N, K, ldb, trans_b);
+}
+
 extern "C" int emi_swiglu_fwd(emi_stream_t stream, const void* a, const void* b, void* g, int64_t n, int dtype);
 extern "C" int emi_swiglu_bwd(emi_stream_t stream, const void* a, const void* b, const void* dg, void* da, void* db, int64_t n,
                               int dtype);

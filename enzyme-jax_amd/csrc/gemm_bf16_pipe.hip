@@ -101,11 +101,50 @@ template <int ROWS, int BK, int NW, bool KM> struct PipeOperand {
 // 14.5 -> 13.2; k-major B, three products summed: 777 x 768 x 768 14.8 -> 11.2.  part != nullptr: split-K, split z owns the stages
 // [z * steps_per_split, ...) of the contraction (of the whole sum, where products are summed) and leaves its tile in
 // part[z][M][N] for the reduction over splits.
-template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, bool GROUPED>
+// MODE: as in gemm_f32.hip; a lane has eight columns, four rotation pairs.  The product is rounded before the elementwise operator
+// as it is when it goes through memory.  us, separate launches | together: gated 777 x 2048 x 768 21.8 | 14.0, 61 x 2048 x 768 7.2 | 6.5, 2181 x 1408 x
+// 512 24.9 | 16.7; rotated 990 x 2048 x 2048 (three) 36.5 | 31.2, 777 x 768 x 768 12.2 | 9.3; adjoint 985 x 5632 x 2048 40.8 | 32.4,
+// 777 x 2048 x 768 12.9 | 9.1.  Its other operand is read after the contraction: requested before, its registers cost the 128 x 128
+// blocks more (990 x 2048 x 2048 49.6).
+template <int MODE> struct PipeArg { using type = PipeSingle; };
+template <> struct PipeArg<kTailGroup> { using type = PipeGroup; };
+template <> struct PipeArg<kTailGated> {
+  struct type {
+    const uint16_t* B1;
+    uint16_t *C1, *G;
+  };
+};
+template <> struct PipeArg<kTailRotated> {
+  struct type {
+    const uint16_t* B[3];
+    uint16_t* C[3];
+    const float2* table;
+    int seq, head_dim, rotated;
+  };
+};
+template <> struct PipeArg<kTailAdjoint> {
+  struct type {
+    const uint16_t *h1, *h3;
+    uint16_t* d3;
+  };
+};
+__device__ __forceinline__ void unpack8(const u32x4_t r, float (&v)[8]) {
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    v[2 * q] = __uint_as_float(r[q] << 16);
+    v[2 * q + 1] = __uint_as_float(r[q] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ u32x4_t pack8(const float (&v)[8]) {
+  return u32x4_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, int MODE>
 __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const uint16_t* A, const uint16_t* B, const uint16_t* R,
                                                                          uint16_t* C, int M, int N, int K, int lda, int ldb, int64_t ldr,
                                                                          int64_t ldc, int vec_ok, float* part, int steps_per_split,
-                                                                         std::conditional_t<GROUPED, PipeGroup, PipeSingle> grp) {
+                                                                         typename PipeArg<MODE>::type grp) {
+  constexpr bool GROUPED = MODE == kTailGroup;
   constexpr int NW = WM * WN * WK;
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
   constexpr int KS = BK / 32 / WK;                                // k-steps of 32 per wavefront and stage
@@ -142,6 +181,11 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
       R = grp.R[outer];
       C = grp.C[outer];
     }
+  }
+  if constexpr (MODE == kTailGated) nsteps *= 2;
+  if constexpr (MODE == kTailRotated) {
+    B = grp.B[outer];
+    C = grp.C[outer];
   }
   if (part != nullptr) {
     step0 = outer * steps_per_split;
@@ -181,6 +225,12 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
         B = grp.B[at_pair];
       }
     }
+    if constexpr (MODE == kTailGated) {
+      if (at_k >= K) {
+        at_k = 0;
+        B = grp.B1;
+      }
+    }
   };
 
   f32x4_t acc[TM][TN];
@@ -207,7 +257,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
 #pragma unroll
   for (int s = 0; s < NST - 1; s++) issue();
   int slot = 0;
-  for (int t = 0; t < nsteps; t++) {
+  auto contract = [&](int steps) __attribute__((always_inline)) {
+  for (int t = 0; t < steps; t++) {
     pipe_wait_vmcnt<(NST - 2) * LPT>();                    // this stage has landed
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();                          // everyone's part of it, and the stage before is free again
@@ -266,6 +317,21 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  };
+  [[maybe_unused]] f32x4_t gate[TM][TN];                   // gated: the tile of h1
+  if constexpr (MODE == kTailGated) {
+    contract(ksteps);
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++) {
+        gate[a][b] = acc[a][b];
+        acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    contract(ksteps);
+  } else {
+    contract(nsteps);
+  }
   pipe_wait_vmcnt<0>();                                    // the zero-filled loads past the end
   __syncthreads();
 
@@ -273,19 +339,17 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
   // in the idle ring as fp32 rows; they are read back eight columns a lane, met by the residual and rounded once.
   constexpr int WR = BM / WM, WC = BN / WN, RS = WC + 4;
   EMI_LDS float* mine = (EMI_LDS float*)smem + wave * (WR * RS);
+  auto lay = [&](const f32x4_t (&t)[TM][TN]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int a = 0; a < TM; a++)
+    for (int a = 0; a < TM; a++)
 #pragma unroll
-    for (int b = 0; b < TN; b++) *reinterpret_cast<EMI_LDS f32x4_t*>(mine + (a * 16 + l15) * RS + b * 16 + g * 4) = acc[a][b];
-  if constexpr (WK > 1) __syncthreads();
-  constexpr int PPR = WC / 8, PIECES = WR * PPR, THREADS = WK * 64;
+      for (int b = 0; b < TN; b++) *reinterpret_cast<EMI_LDS f32x4_t*>(mine + (a * 16 + l15) * RS + b * 16 + g * 4) = t[a][b];
+    if constexpr (WK > 1) __syncthreads();
+  };
+  constexpr int PPR = WC / 8, PIECES = WR * PPR, THREADS = WK * 64, EACH = (PIECES + THREADS - 1) / THREADS;
   const int tile_wave = wave % (WM * WN), me = wk * 64 + lane;
-#pragma unroll
-  for (int e = 0; e < (PIECES + THREADS - 1) / THREADS; e++) {
-    const int at = e * THREADS + me;
-    if (PIECES % THREADS != 0 && at >= PIECES) break;
+  auto take = [&](int at, float (&v)[8]) __attribute__((always_inline)) {
     const int row = at / PPR, c8 = (at % PPR) * 8;
-    float v[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) v[q] = 0.f;
 #pragma unroll
@@ -298,8 +362,69 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
         v[4 + q] += hi[q];
       }
     }
+  };
+  [[maybe_unused]] u32x4_t h1[EACH];
+  if constexpr (MODE == kTailGated) {
+    lay(gate);
+#pragma unroll
+    for (int e = 0; e < EACH; e++) {
+      const int at = e * THREADS + me;
+      if (PIECES % THREADS != 0 && at >= PIECES) break;
+      float v[8];
+      take(at, v);
+      h1[e] = pack8(v);
+    }
+    if constexpr (WK > 1) __syncthreads();
+  }
+  lay(acc);
+#pragma unroll
+  for (int e = 0; e < EACH; e++) {
+    const int at = e * THREADS + me;
+    if (PIECES % THREADS != 0 && at >= PIECES) break;
+    const int row = at / PPR, c8 = (at % PPR) * 8;
+    float v[8];
+    take(at, v);
     const int grow = m0 + wm * WR + row, gcol = n0 + wn * WC + c8;
     if (grow >= M || gcol >= N) continue;
+    if constexpr (MODE >= kTailGated) {                    // rows of whole pieces, results without a gap between them
+      const int64_t to = (int64_t)grow * N + gcol;
+      const u32x4_t y = pack8(v);
+      if constexpr (MODE == kTailGated) {
+        float a[8], o[8];
+        unpack8(h1[e], a);
+        unpack8(y, v);
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = emi_swiglu(a[q], v[q]);
+        *reinterpret_cast<u32x4_t*>(C + to) = h1[e];
+        *reinterpret_cast<u32x4_t*>(grp.C1 + to) = y;
+        *reinterpret_cast<u32x4_t*>(grp.G + to) = pack8(o);
+      } else if constexpr (MODE == kTailAdjoint) {
+        float a[8], b[8], d1[8], d3[8];
+        unpack8(*reinterpret_cast<const u32x4_t*>(grp.h1 + to), a);
+        unpack8(*reinterpret_cast<const u32x4_t*>(grp.h3 + to), b);
+        unpack8(y, v);
+#pragma unroll
+        for (int q = 0; q < 8; q++) emi_swiglu_adjoint(a[q], b[q], v[q], &d1[q], &d3[q]);
+        *reinterpret_cast<u32x4_t*>(C + to) = pack8(d1);
+        *reinterpret_cast<u32x4_t*>(grp.d3 + to) = pack8(d3);
+      } else {
+        u32x4_t z = y;
+        if (outer < grp.rotated) {
+          float o[8];
+          unpack8(y, v);
+          const float2* angles = grp.table + (int64_t)(grow % grp.seq) * (grp.head_dim >> 1);
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const float2 t = angles[((gcol + 2 * q) % grp.head_dim) >> 1];
+            o[2 * q] = t.x * v[2 * q] - t.y * v[2 * q + 1];
+            o[2 * q + 1] = t.y * v[2 * q] + t.x * v[2 * q + 1];
+          }
+          z = pack8(o);
+        }
+        *reinterpret_cast<u32x4_t*>(C + to) = z;
+      }
+      continue;
+    }
     if (part != nullptr) {
       float* dst = part + (int64_t)grow * N + gcol;
       if ((N & 3) == 0 && gcol + 8 <= N) {
@@ -316,15 +441,12 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
     const uint16_t* res = R != nullptr ? R + (int64_t)grow * ldr + gcol : nullptr;
     if (vec_ok && gcol + 8 <= N) {
       if (res != nullptr) {
-        const u32x4_t r = *reinterpret_cast<const u32x4_t*>(res);
+        float r[8];
+        unpack8(*reinterpret_cast<const u32x4_t*>(res), r);
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          v[2 * q] += __uint_as_float(r[q] << 16);
-          v[2 * q + 1] += __uint_as_float(r[q] & 0xffff0000u);
-        }
+        for (int q = 0; q < 8; q++) v[q] += r[q];
       }
-      const u32x4_t o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
-      *reinterpret_cast<u32x4_t*>(dst) = o;
+      *reinterpret_cast<u32x4_t*>(dst) = pack8(v);
     } else {
 #pragma unroll
       for (int q = 0; q < 8; q++)
@@ -354,7 +476,7 @@ struct PipeCall {
 
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, bool GROUPED>
 static int launch_pipe_one(hipStream_t st, const PipeCall& c) {
-  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, BKM, GROUPED>;
+  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, BKM, GROUPED ? kTailGroup : kTailNone>;
   constexpr int ring = NST * (BM + BN) * BK * 2, tile = WM * WN * WK * (BM / WM) * (BN / WN + 4) * 4;
   constexpr int smem = ring > tile ? ring : tile;
   static_assert(smem <= 160 * 1024, "LDS of a CU");
@@ -499,6 +621,72 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
     case 7: return launch_pipe_shape<64, 64, 2, 2, 1, 64, 3>(st, c, trans_b);
     case 9: return launch_pipe_shape<128, 128, 4, 2, 1, 64, 3>(st, c, trans_b);
     default: return launch_pipe_shape<32, 32, 1, 1, 8, 256, 3>(st, c, trans_b);
+  }
+}
+
+// The products of gemm_plan.h whose result goes through an elementwise operator.
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, int MODE>
+static int launch_pipe_tail_one(hipStream_t st, const uint16_t* A, const uint16_t* B, const ProductTail& t, int M, int N, int K, int ldb) {
+  auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, BKM, MODE>;
+  constexpr int ring = NST * (BM + BN) * BK * 2, tile = WM * WN * WK * (BM / WM) * (BN / WN + 4) * 4;
+  constexpr int smem = ring > tile ? ring : tile;
+  static bool configured = false;   // idempotent; a race only repeats the call
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+    configured = true;
+  }
+  typename PipeArg<MODE>::type arg{};
+  if constexpr (MODE == kTailGated) {
+    arg = {static_cast<const uint16_t*>(t.B[1]), static_cast<uint16_t*>(t.C[1]), static_cast<uint16_t*>(t.C[2])};
+  } else if constexpr (MODE == kTailRotated) {
+    for (int i = 0; i < t.count; i++) {
+      arg.B[i] = static_cast<const uint16_t*>(t.B[i]);
+      arg.C[i] = static_cast<uint16_t*>(t.C[i]);
+    }
+    arg.table = reinterpret_cast<const float2*>(t.table);
+    arg.seq = t.seq, arg.head_dim = t.head_dim, arg.rotated = t.rotated;
+  } else {
+    arg = {static_cast<const uint16_t*>(t.h1), static_cast<const uint16_t*>(t.h3), static_cast<uint16_t*>(t.C[1])};
+  }
+  const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * (MODE == kTailRotated ? t.count : 1);
+  hipLaunchKernelGGL(kern, dim3(tiles), dim3(WM * WN * WK * 64), smem, st, A, B, (const uint16_t*)nullptr, static_cast<uint16_t*>(t.C[0]), M, N, K,
+                     K, ldb, (int64_t)0, (int64_t)N, 1, (float*)nullptr, 0, arg);
+  EMI_CHECK_LAUNCH("emi_gemm(elementwise tail)");
+  return EMI_OK;
+}
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST>
+static int launch_pipe_tail_shape(hipStream_t st, const uint16_t* A, const uint16_t* B, const ProductTail& t, int M, int N, int K, int ldb, int trans_b) {
+  if (t.mode == kTailGated) return launch_pipe_tail_one<BM, BN, WM, WN, WK, BK, NST, false, kTailGated>(st, A, B, t, M, N, K, ldb);
+  if (t.mode == kTailRotated) return launch_pipe_tail_one<BM, BN, WM, WN, WK, BK, NST, false, kTailRotated>(st, A, B, t, M, N, K, ldb);
+  if (trans_b) return launch_pipe_tail_one<BM, BN, WM, WN, WK, BK, NST, false, kTailAdjoint>(st, A, B, t, M, N, K, ldb);
+  if constexpr (BN >= 64) return launch_pipe_tail_one<BM, BN, WM, WN, WK, BK, NST, true, kTailAdjoint>(st, A, B, t, M, N, K, ldb);
+  return -1;
+}
+
+// Against the separate launches by the plan's own estimates, and a pass of 2.4 us and the bytes it moves; a gated tile leaves
+// three results, 1.2 to 2.2 us.  Over 135 products of 32 to 5000 rows by 768 x 288 to 5632 x 2048: 1.22 to 1.33 times as fast
+// as the separate launches, none slower by more than 2 %.  What is for the 256-tiles goes there.
+int launch_bf16_pipe_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int M, int N, int K, int ldb, int trans_b) {
+  if (t.mode != kTailAdjoint && !trans_b) return -1;
+  const int count = t.mode == kTailGated ? 2 : t.mode == kTailRotated ? t.count : 1, sum = t.mode == kTailGated;
+  const Bf16Plan p = bf16_plan(M, N, K, count, sum, trans_b, 1), group = bf16_plan(M, N, K, count, 0, trans_b, 1),
+                 one = bf16_plan(M, N, K, 1, 0, trans_b, kAnySplits);
+  const double singly = count * (one.us + 1.0) - 1.0, apart = singly < group.us ? singly : group.us;
+  const double moved = 2e-6 / 5.0 * M * N * (t.mode == kTailRotated ? 2 * t.rotated : t.mode == kTailGated ? 3 : 5);
+  const double results = t.mode != kTailGated ? 0.0 : p.shape == 5 ? 1.2 : 2.2;
+  if (p.shape == 0 || one.shape == 0 || p.us + results >= apart + 2.4 + moved) return -1;
+  const uint16_t *a = static_cast<const uint16_t*>(A), *b = static_cast<const uint16_t*>(B);
+  switch (bf16_kernel(p, M, N, K, count, sum, trans_b)) {
+    case 1: return launch_pipe_tail_shape<128, 128, 4, 2, 1, 64, 2>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 2: return launch_pipe_tail_shape<128, 128, 4, 2, 2, 64, 3>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 3: return launch_pipe_tail_shape<128, 64, 4, 2, 1, 64, 3>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 4: return launch_pipe_tail_shape<128, 64, 4, 2, 2, 128, 3>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 5: return launch_pipe_tail_shape<64, 64, 2, 2, 2, 128, 2>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 6: return launch_pipe_tail_shape<64, 64, 2, 2, 2, 128, 3>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 7: return launch_pipe_tail_shape<64, 64, 2, 2, 1, 64, 3>(st, a, b, t, M, N, K, ldb, trans_b);
+    case 9: return launch_pipe_tail_shape<128, 128, 4, 2, 1, 64, 3>(st, a, b, t, M, N, K, ldb, trans_b);
+    default: return launch_pipe_tail_shape<32, 32, 1, 1, 8, 256, 3>(st, a, b, t, M, N, K, ldb, trans_b);
   }
 }
 

@@ -90,11 +90,43 @@ template <int ROWS, int BK, int NW, bool KM> struct F32Operand {
 // instruction t of chunk j contracts k = 8j + 4g + t, so that a k-contiguous operand is read in 16-byte pieces.
 // part != nullptr: split-K, split z owns the stages [z * steps_per_split, ...) of the contraction (of the whole sum, where
 // products are summed) and leaves its tile in part[z][M][N] for the reduction over splits.
-template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool AKM, bool BKM, bool GROUPED>
+// MODE (gemm_plan.h), beside a single product and a group: gated, the products with w1 and w3 one after the other in one block,
+// whose tiles meet in the SwiGLU; rotated, up to three results, each lane exchanging its column with its neighbour's; adjoint,
+// the SwiGLU's adjoint of the tile.  us,
+// separate launches | this: gated 183 x 768 x 288 10.8 | 8.3, 308 x 1408 x 512 18.9 | 18.1; rotated, three results, 236 x 288 x 288 7.9 | 6.0,
+// 62 x 768 x 768 11.1 | 8.7; adjoint 223 x 768 x 288 7.9 | 5.9, 198 x 1408 x 512 12.5 | 10.2.
+template <int MODE> struct F32Arg { using type = F32Single; };
+template <> struct F32Arg<kTailGroup> { using type = F32Group; };
+template <> struct F32Arg<kTailGated> {
+  struct type {
+    const float* B1;
+    float *C1, *G;
+  };
+};
+template <> struct F32Arg<kTailRotated> {
+  struct type {
+    const float* B[3];
+    float* C[3];
+    const float2* table;
+    int seq, head_dim, rotated;
+  };
+};
+template <> struct F32Arg<kTailAdjoint> {
+  struct type {
+    const float *h1, *h3;
+    float* d3;
+  };
+};
+__device__ __forceinline__ float lane_xor1(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0xb1, 0xf, 0xf, true));
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool AKM, bool BKM, int MODE>
 __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const float* A, const float* B, const float* R, float* C, int M,
                                                                         int N, int K, int lda, int ldb, int64_t ldr, int64_t ldc,
                                                                         float* part, int steps_per_split,
-                                                                        std::conditional_t<GROUPED, F32Group, F32Single> grp) {
+                                                                        typename F32Arg<MODE>::type grp) {
+  constexpr bool GROUPED = MODE == kTailGroup;
   constexpr int NW = WM * WN * WK;
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
   constexpr int CH = BK / 8 / WK;                                 // 8-wide chunks per wavefront and stage
@@ -132,6 +164,11 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
       R = grp.R[outer];
       C = grp.C[outer];
     }
+  }
+  if constexpr (MODE == kTailGated) nsteps *= 2;
+  if constexpr (MODE == kTailRotated) {
+    B = grp.B[outer];
+    C = grp.C[outer];
   }
   if (part != nullptr) {
     step0 = outer * steps_per_split;
@@ -171,6 +208,12 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
         B = grp.B[at_pair];
       }
     }
+    if constexpr (MODE == kTailGated) {
+      if (at_k >= K) {
+        at_k = 0;
+        B = grp.B1;
+      }
+    }
   };
 
   // A sum over K in one chain is off by the square root of its length, so a chain ends after FLUSH stages (32 k of a
@@ -192,6 +235,36 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
         acc[a][b] = zero;
       }
   };
+
+  // Which element of the result this lane's e-th is.  Wavefronts that share k meet in the LDS; otherwise register r of lane l
+  // holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32 x 32 tile.
+  constexpr int EACH = WK > 1 ? 1024 / (NW * 64) : 16 * TM * TN;
+  auto row_of = [&](int e) __attribute__((always_inline)) {
+    if constexpr (WK > 1) return m0 + ((e * NW * 64 + (int)threadIdx.x) >> 5);
+    else return m0 + wm * (BM / WM) + e / (16 * TN) * 32 + (e % 16 >> 2) * 8 + g * 4 + (e & 3);
+  };
+  auto col_of = [&](int e) __attribute__((always_inline)) {
+    if constexpr (WK > 1) return n0 + ((e * NW * 64 + (int)threadIdx.x) & 31);
+    else return n0 + wn * (BN / WN) + e / 16 % TN * 32 + i;
+  };
+  // What an elementwise operator needs beside the product is requested ahead of the ring's loads: after the contraction, each
+  // load behind the stores before it, it cost 4 to 8 us (64 x 64 blocks).
+  [[maybe_unused]] float beside[2][EACH];
+  if constexpr (MODE == kTailRotated || MODE == kTailAdjoint) {
+#pragma unroll
+    for (int e = 0; e < EACH; e++) {
+      const int row = row_of(e) < M ? row_of(e) : M - 1, col = col_of(e) < N ? col_of(e) : N - 1;
+      if constexpr (MODE == kTailAdjoint) {
+        const int64_t at = (int64_t)row * ldc + col;
+        beside[0][e] = grp.h1[at];
+        beside[1][e] = grp.h3[at];
+      } else {
+        const float2 t = outer < grp.rotated ? grp.table[(int64_t)(row % grp.seq) * (grp.head_dim >> 1) + ((col % grp.head_dim) >> 1)] : make_float2(1.f, 0.f);
+        beside[0][e] = t.x;
+        beside[1][e] = t.y;
+      }
+    }
+  }
 
 #pragma unroll
   for (int s = 0; s < NST - 1; s++) issue();
@@ -229,23 +302,54 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  for (int t = 0; t < nsteps;) {
-    if constexpr (FLUSH > 1) {
+  auto contract = [&](int steps) __attribute__((always_inline)) {
+    for (int t = 0; t < steps;) {
+      if constexpr (FLUSH > 1) {
 #pragma unroll 1
-      for (const int end = t + FLUSH < nsteps ? t + FLUSH : nsteps; t < end; t++) stage();
-      end_chain();
-    } else {
-      stage();
-      t++;
+        for (const int end = t + FLUSH < steps ? t + FLUSH : steps; t < end; t++) stage();
+        end_chain();
+      } else {
+        stage();
+        t++;
+      }
     }
+    if constexpr (FLUSH == 1) end_chain();
+  };
+  f32x16_t gate[TM][TN];                                   // gated: the tile of h1
+  if constexpr (MODE == kTailGated) {
+    contract(ksteps);
+#pragma unroll
+    for (int a = 0; a < TM; a++)
+#pragma unroll
+      for (int b = 0; b < TN; b++) {
+        gate[a][b] = total[a][b];
+        total[a][b] = zero;
+      }
+    contract(ksteps);
+  } else {
+    contract(nsteps);
   }
-  if constexpr (FLUSH == 1) end_chain();
 
-  // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32 x 32 tile
-  auto put = [&](int row, int col, float v) __attribute__((always_inline)) {
+  // element e of this lane's: what the elementwise operator reads beside it has been there since before the contraction
+  auto put = [&](int row, int col, float v, float h1, float p, float q) __attribute__((always_inline)) {
+    if constexpr (MODE == kTailRotated) {                  // the pair's other column is the neighbouring lane's, of the same row
+      const float other = lane_xor1(v);
+      v = (col & 1) == 0 ? p * v - q * other : q * other + p * v;
+    }
     if (row < M && col < N) {
       if (part != nullptr) {
         part[(int64_t)row * N + col] = v;
+      } else if constexpr (MODE == kTailGated) {
+        const int64_t at = (int64_t)row * ldc + col;
+        C[at] = h1;
+        grp.C1[at] = v;
+        grp.G[at] = emi_swiglu(h1, v);
+      } else if constexpr (MODE == kTailAdjoint) {
+        const int64_t at = (int64_t)row * ldc + col;
+        float d1, d3;
+        emi_swiglu_adjoint(p, q, v, &d1, &d3);
+        C[at] = d1;
+        grp.d3[at] = d3;
       } else {
         if (R != nullptr) v += R[(int64_t)row * ldr + col];
         C[(int64_t)row * ldc + col] = v;
@@ -254,27 +358,35 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
   };
   f32_wait_vmcnt<0>();                                     // the zero-filled loads past the end
   if constexpr (WK > 1) {
-    __syncthreads();
     EMI_LDS float* red = (EMI_LDS float*)smem;             // [WK][32][32 + 1]
+    float sum[EACH], h1[EACH];
+    auto meet = [&](const f32x16_t& t) __attribute__((always_inline)) {
+      __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 16; r++) red[(wk * 32 + (r >> 2) * 8 + g * 4 + (r & 3)) * 33 + i] = total[0][0][r];
-    __syncthreads();
+      for (int r = 0; r < 16; r++) red[(wk * 32 + (r >> 2) * 8 + g * 4 + (r & 3)) * 33 + i] = t[r];
+      __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 1024 / (NW * 64); e++) {
-      const int at = e * NW * 64 + threadIdx.x, row = at >> 5, col = at & 31;
-      float v = 0.f;
+      for (int e = 0; e < EACH; e++) {
+        const int at = e * NW * 64 + threadIdx.x, row = at >> 5, col = at & 31;
+        sum[e] = 0.f;
 #pragma unroll
-      for (int w = 0; w < WK; w++) v += red[(w * 32 + row) * 33 + col];
-      put(m0 + row, n0 + col, v);
+        for (int w = 0; w < WK; w++) sum[e] += red[(w * 32 + row) * 33 + col];
+      }
+    };
+    if constexpr (MODE == kTailGated) {
+      meet(gate[0][0]);
+#pragma unroll
+      for (int e = 0; e < EACH; e++) h1[e] = sum[e];
     }
+    meet(total[0][0]);
+#pragma unroll
+    for (int e = 0; e < EACH; e++) put(row_of(e), col_of(e), sum[e], h1[e], beside[0][e], beside[1][e]);
   } else {
 #pragma unroll
-    for (int a = 0; a < TM; a++)
-#pragma unroll
-      for (int b = 0; b < TN; b++)
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          put(m0 + wm * (BM / WM) + a * 32 + (r >> 2) * 8 + g * 4 + (r & 3), n0 + wn * (BN / WN) + b * 32 + i, total[a][b][r]);
+    for (int e = 0; e < EACH; e++) {
+      const int a = e / (16 * TN), b = e / 16 % TN, r = e % 16;
+      put(row_of(e), col_of(e), total[a][b][r], gate[a][b][r], beside[0][e], beside[1][e]);
+    }
   }
 }
 
@@ -284,7 +396,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
 
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool AKM, bool BKM, bool GROUPED>
 static int launch_f32_one(hipStream_t st, const F32Call& c) {
-  auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, GROUPED>;
+  auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, GROUPED ? kTailGroup : kTailNone>;
   constexpr int smem = NST * (BM + BN) * BK * 4;
   static_assert(WK == 1 || smem >= WK * 32 * 33 * 4, "the wavefronts' tiles meet in the ring");
   static bool configured = false;   // idempotent; a race only repeats the call
@@ -427,6 +539,63 @@ int launch_f32_gemm(hipStream_t st, int count, const void* const* A, const void*
     case 2: return launch_f32_shape<128, 128, 4, 2, 1, 32, 2>(st, c, trans_a, trans_b);
     default: return launch_f32_bf16x3(st, c, p.shape - 3, trans_a, trans_b);
   }
+}
+
+// The products of gemm_plan.h whose result goes through an elementwise operator, on the fp32 instructions.
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, int MODE>
+static int launch_f32_tail_one(hipStream_t st, const float* A, const float* B, const ProductTail& t, int M, int N, int K, int ldb) {
+  auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, false, BKM, MODE>;
+  constexpr int smem = NST * (BM + BN) * BK * 4;
+  static bool configured = false;   // idempotent; a race only repeats the call
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+    configured = true;
+  }
+  typename F32Arg<MODE>::type arg{};
+  if constexpr (MODE == kTailGated) {
+    arg = {static_cast<const float*>(t.B[1]), static_cast<float*>(t.C[1]), static_cast<float*>(t.C[2])};
+  } else if constexpr (MODE == kTailRotated) {
+    for (int i = 0; i < t.count; i++) {
+      arg.B[i] = static_cast<const float*>(t.B[i]);
+      arg.C[i] = static_cast<float*>(t.C[i]);
+    }
+    arg.table = reinterpret_cast<const float2*>(t.table);
+    arg.seq = t.seq, arg.head_dim = t.head_dim, arg.rotated = t.rotated;
+  } else {
+    arg = {static_cast<const float*>(t.h1), static_cast<const float*>(t.h3), static_cast<float*>(t.C[1])};
+  }
+  const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * (MODE == kTailRotated ? t.count : 1);
+  hipLaunchKernelGGL(kern, dim3(tiles), dim3(WM * WN * WK * 64), smem, st, A, B, (const float*)nullptr, static_cast<float*>(t.C[0]), M, N, K, K,
+                     ldb, (int64_t)0, (int64_t)N, (float*)nullptr, 0, arg);
+  EMI_CHECK_LAUNCH("emi_gemm(fp32, elementwise tail)");
+  return EMI_OK;
+}
+template <int BM, int BN, int WM, int WN, int WK, int BK, int NST>
+static int launch_f32_tail_shape(hipStream_t st, const float* A, const float* B, const ProductTail& t, int M, int N, int K, int ldb, int trans_b) {
+  if (t.mode == kTailGated) return launch_f32_tail_one<BM, BN, WM, WN, WK, BK, NST, false, kTailGated>(st, A, B, t, M, N, K, ldb);
+  if (t.mode == kTailRotated) return launch_f32_tail_one<BM, BN, WM, WN, WK, BK, NST, false, kTailRotated>(st, A, B, t, M, N, K, ldb);
+  return trans_b ? launch_f32_tail_one<BM, BN, WM, WN, WK, BK, NST, false, kTailAdjoint>(st, A, B, t, M, N, K, ldb)
+                 : launch_f32_tail_one<BM, BN, WM, WN, WK, BK, NST, true, kTailAdjoint>(st, A, B, t, M, N, K, ldb);
+}
+
+// Against the separate launches by the plan's own estimates, and a pass of 2.4 us and the bytes it moves.  Gated, a block's two
+// products cost what a sum of two does; a block's elementwise part, 0.8 us of a 32 x 32 tile and 3 of 64 x 64.  What has tiles and
+// stages enough stays with the bf16 instructions and a pass (1970 x 2048 x 768 adjoint 56 | 63 here).
+int launch_f32_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b) {
+  if (128 * K + K >= 0x1fffffff || 128 * ldb + K >= 0x1fffffff || (t.mode != kTailAdjoint && !trans_b)) return -1;
+  const int count = t.mode == kTailGated ? 2 : t.mode == kTailRotated ? t.count : 1;
+  double together[2];
+  for (int c = 0; c < 2; c++) {
+    const int64_t blocks = (M + kF32Shape[c].bm - 1) / kF32Shape[c].bm * ((N + kF32Shape[c].bn - 1) / kF32Shape[c].bn) * (t.mode == kTailRotated ? count : 1);
+    together[c] = f32_estimate(c, M, N, K, count, t.mode == kTailGated, 0, 1) + (c == 0 ? 3.0 : 0.8) * ((blocks + 255) / 256);
+  }
+  const int shape = together[1] < together[0];
+  const double moved = 4e-6 / 5.0 * M * N * (t.mode == kTailRotated ? 2 * t.rotated : t.mode == kTailGated ? 3 : 5);
+  if (together[shape] >= f32_plan(M, N, K, count, 0, 0, count > 1 ? 1 : kAnySplits).us + 2.4 + moved) return -1;
+  const float *a = static_cast<const float*>(A), *b = static_cast<const float*>(B);
+  return shape == 0 ? launch_f32_tail_shape<64, 64, 2, 2, 1, 32, 2>(st, a, b, t, (int)M, (int)N, (int)K, (int)ldb, trans_b)
+                    : launch_f32_tail_shape<32, 32, 1, 1, 8, 64, 5>(st, a, b, t, (int)M, (int)N, (int)K, (int)ldb, trans_b);
 }
 
 }  // namespace emi

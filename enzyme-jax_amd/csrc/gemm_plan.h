@@ -54,4 +54,20 @@ int gemm_grouped_run(hipStream_t st, int count, const void* const* A, const void
                      void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldr,
                      int64_t ldc, int trans_a, int trans_b, int sum, int dtype, int* planes);
 
+// Products whose result goes through an elementwise operator, where that operator is worked out before the result leaves: what
+// is left of a small model between two products are passes of 2 to 4 us over it.  Each returns -1 where the separate launches
+// are the faster ones, or alone possible, and has then launched nothing.  A kTail... is the MODE of the product kernels.
+enum { kTailNone, kTailGroup, kTailGated, kTailRotated, kTailAdjoint };
+struct ProductTail {
+  int mode;
+  const void* B[3];            // gated: W3 in B[1];  rotated: the weights of up to three results
+  void* C[3];                  // gated: h1, h3, g;  rotated: the results;  adjoint: dh1, dh3
+  const float* table;          // rotated: results 0 .. rotated - 1 by the angle of row % seq
+  int seq, head_dim, rotated, count;
+  const void *h1, *h3;         // adjoint: the SwiGLU's operands; the product is the cotangent of its result
+};
+int launch_bf16_pipe_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int M, int N, int K, int ldb, int trans_b);      // gemm_bf16_pipe.hip
+int launch_f32_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b);      // gemm_f32.hip
+int gemm_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b, int dtype);   // gemm.hip
+
 }  // namespace emi

@@ -2,8 +2,10 @@
 // layers whose weights are stacked, and the reverse pass with every gradient.
 //
 // No kernel of its own: it issues the launchers of emi.h in the order in which ops.attention_block, ops.ffn and their rules
-// do.  A layer is nine to twelve launches forward and about twenty in reverse, and a small model's are 3 to 10 us each, less
+// do.  A layer is seven to twelve launches forward and about twenty in reverse, and a small model's are 3 to 10 us each, less
 // than a Python operator costs: the dim-288 model on 256 tokens spent 2.6 ms on the host for 1.25 ms of kernels.
+// The rotation of q and k, the SwiGLU and its adjoint are part of the products before them where that is faster (gemm_tail):
+// bf16 layer forward 68 -> 56 us at dim 768 on 777 tokens, 131 -> 116 at dim 1024 on 2000; fp32 50 -> 46 at dim 288 on 200.
 // In reverse the weight gradients dW = dY^T X feed nothing else, so they wait until `group` layers are done and run grouped
 // by shape (q, k, v, o; w1, w3; w2), which fills the chip where one layer's would not; a group of one runs them in place.
 // So do the column sums of the RMSNorm adjoints (dim-288 model, six layers: 11 launches of 3 us less, 858 -> 830 us).
@@ -166,14 +168,22 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
     EMI_TRY(emi_gemm_rope(st, s.xb1, w[kK], s.k, table, T, D, D, d.S, d.hd(), d.dtype));
     EMI_TRY(emi_gemm_ws(st, s.xb1, w[kV], nullptr, s.v, ws, wsb, T, D, D, D, D, D, D, 0, 1, d.dtype));
   } else {
-    const void *a[3] = {s.xb1, s.xb1, s.xb1}, *b[3] = {w[kQ], w[kK], w[kV]};
-    void* c[3] = {s.q, s.k, s.v};
-    EMI_TRY(emi_gemm_grouped(st, 3, a, b, nullptr, c, ws, wsb, T, D, D, D, D, D, D, 0, 1, 0, d.dtype));
-    EMI_TRY(emi_rope(st, s.q, table, s.q, 2 * d.B, d.S, d.heads, d.hd(), 0, d.dtype));
+    emi::ProductTail t{emi::kTailRotated, {w[kQ], w[kK], w[kV]}, {s.q, s.k, s.v}, table, (int)d.S, (int)d.hd(), 2, 3, nullptr, nullptr};
+    if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(st), s.xb1, w[kQ], t, T, D, D, D, 1, d.dtype); rc > 0) return rc;
+    else if (rc < 0) {
+      const void *a[3] = {s.xb1, s.xb1, s.xb1}, *b[3] = {w[kQ], w[kK], w[kV]};
+      void* c[3] = {s.q, s.k, s.v};
+      EMI_TRY(emi_gemm_grouped(st, 3, a, b, nullptr, c, ws, wsb, T, D, D, D, D, D, D, 0, 1, 0, d.dtype));
+      EMI_TRY(emi_rope(st, s.q, table, s.q, 2 * d.B, d.S, d.heads, d.hd(), 0, d.dtype));
+    }
   }
   EMI_TRY(emi_attn_fwd(st, s.q, s.k, s.v, s.att, s.lse, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
   EMI_TRY(product_and_norm(st, s.att, w[kO], x, s.x1, w[kFfn], s.xb2, ws, wsb, D, d));
-  if (d.swiglu_epilogue()) {
+  emi::ProductTail t{emi::kTailGated, {w[kW1], w[kW3], nullptr}, {s.h1, s.h3, s.g}, nullptr, 0, 0, 0, 0, nullptr, nullptr};
+  if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(st), s.xb2, w[kW1], t, T, H, D, D, 1, d.dtype); rc > 0) {
+    return rc;
+  } else if (rc == 0) {
+  } else if (d.swiglu_epilogue()) {
     EMI_TRY(emi_gemm_ws(st, s.xb2, w[kW1], nullptr, s.h1, ws, wsb, T, H, D, D, D, H, H, 0, 1, d.dtype));
     EMI_TRY(emi_gemm_swiglu_fwd(st, s.xb2, w[kW3], s.h1, s.h3, s.g, T, H, D, d.dtype));
   } else {
@@ -353,7 +363,11 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     // the group's last layer writes its dx where the dy of the group's first one lies (the last slot's dx, of the group before)
     const bool ends_group = (done + 1) % group == 0 || l == 0;
     if (ends_group) EMI_TRY(flush(stream, down, D, H, T, r, dtype));
-    if (tb && d.swiglu_epilogue()) {
+    emi::ProductTail t{emi::kTailAdjoint, {}, {c.dh1, c.dh3, nullptr}, nullptr, 0, 0, 0, 0, s.h1, s.h3};
+    if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(stream), dy, b[kW2], t, T, H, D, tb ? D : H, tb, dtype); rc > 0) {
+      return rc;
+    } else if (rc == 0) {
+    } else if (tb && d.swiglu_epilogue()) {
       EMI_TRY(emi_gemm_swiglu_bwd(stream, dy, b[kW2], s.h1, s.h3, c.dh1, c.dh3, r.dg, (size_t)T * H * d.elt(), T, H, D, dtype));
     } else {
       EMI_TRY(emi_gemm_ws(stream, dy, b[kW2], nullptr, r.dg, r.ws, r.ws_bytes, T, H, D, D, tb ? D : H, H, H, 0, tb, dtype));

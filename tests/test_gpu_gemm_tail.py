@@ -1,0 +1,116 @@
+"""Products whose result goes through an elementwise operator before it leaves (gemm_tail of csrc/gemm_plan.h): the SwiGLU of
+two products (gated), the rotation of q and k, and the SwiGLU's adjoint, at the sizes where the tiles, stages and pieces of
+every kernel end.  Against float64 of the stored values: a product is off by half a unit of its type and the roundings of its
+sum, n * 2^-24 * sum |a b| to first order, twice that allowed; the operator passes that on times its derivative, and rounds
+its result once more (fp32: the hardware's exponential and reciprocal, a unit or two each, 2^-19 allowed)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import dev, host
+
+pytestmark = pytest.mark.gpu
+GATED, ROTATED, ADJOINT = 2, 3, 4
+
+
+class _Tail(ctypes.Structure):
+    _fields_ = [("mode", ctypes.c_int), ("B", ctypes.c_void_p * 3), ("C", ctypes.c_void_p * 3), ("table", ctypes.c_void_p), ("seq", ctypes.c_int),
+                ("head_dim", ctypes.c_int), ("rotated", ctypes.c_int), ("count", ctypes.c_int), ("h1", ctypes.c_void_p), ("h3", ctypes.c_void_p)]
+
+
+def _run(x, w, tail, M, N, K, tb, dt):
+    from enzyme_ad.jax import _native
+    f = _native.lib()._ZN3emi9gemm_tailEP12ihipStream_tPKvS3_RKNS_11ProductTailEllllii
+    f.restype = ctypes.c_int
+    f.argtypes = [ctypes.c_void_p] * 3 + [ctypes.POINTER(_Tail)] + [ctypes.c_int64] * 4 + [ctypes.c_int] * 2
+    return f(torch.cuda.current_stream().cuda_stream, x.data_ptr(), w.data_ptr(), ctypes.byref(tail), M, N, K, K if tb else N, tb,
+             16 if dt == "bf16" else 11)
+
+
+def _product(xr, wr, tb, dt):
+    w = wr.T if tb else wr
+    p, mag, k = xr @ w, np.abs(xr) @ np.abs(w), xr.shape[1]
+    return p, (2.0 ** -8 * np.abs(p) if dt == "bf16" else 0.0) + (k + 2) * 2.0 ** -23 * mag
+
+
+def _close(got, want, bound, dt, what):
+    err, room = np.abs(host(got) - want), bound + (2.0 ** -8 if dt == "bf16" else 2.0 ** -19) * np.abs(want)
+    assert np.all(err <= room), "%s: worst error / bound %.2f" % (what, float(np.max(err / room)))
+
+
+def _sigmoid(a):
+    return 1.0 / (1.0 + np.exp(-a))
+
+
+SIZES = {
+    ("f32", GATED): [(9, 8, 8), (33, 44, 68), (200, 772, 292), (308, 1404, 516)],
+    ("f32", ROTATED): [(9, 8, 8), (35, 72, 68), (235, 288, 292), (721, 288, 284)],
+    ("f32", ADJOINT): [(9, 8, 8), (35, 76, 68), (198, 1412, 516), (817, 764, 284)],
+    ("bf16", GATED): [(9, 8, 8), (33, 24, 264), (300, 2040, 776), (450, 2808, 1032), (1500, 768, 288), (1500, 1400, 520), (2181, 2040, 776)],
+    ("bf16", ROTATED): [(9, 8, 8), (300, 1400, 520), (450, 520, 520), (600, 776, 776), (340, 2056, 2056), (1000, 776, 776), (4001, 1400, 520),
+                        (5000, 24, 264)],
+    ("bf16", ADJOINT): [(9, 8, 8), (33, 24, 264), (340, 520, 520), (1000, 776, 776), (777, 1400, 520), (1500, 776, 776), (2181, 1032, 1032),
+                        (1500, 2040, 776), (5000, 776, 776)],
+}
+CASES = [(dt, mode) + size for (dt, mode), sizes in SIZES.items() for size in sizes]
+
+
+@pytest.mark.parametrize("dt,mode,M,N,K", CASES)
+def test_products_with_an_elementwise_tail(dt, mode, M, N, K):
+    rng = np.random.default_rng(M + N + K + mode)
+    x, xr = dev(rng.standard_normal((M, K)), dt)
+    out = [torch.full((M, N), 7.0, device=x.device, dtype=x.dtype) for _ in range(3)]
+    for tb in (1, 0) if mode == ADJOINT else (1,):
+        ws = [dev(rng.standard_normal((N, K) if tb else (K, N)) / np.sqrt(K), dt) for _ in range(3)]
+        tail = _Tail(mode=mode)
+        for i in range(3):
+            tail.C[i] = out[i].data_ptr()
+        if mode == ADJOINT:
+            (h1, a), (h3, b) = (dev(rng.standard_normal((M, N)), dt) for _ in range(2))
+            tail.h1, tail.h3, tail.C[2] = h1.data_ptr(), h3.data_ptr(), None
+        else:
+            for i in range(3 if mode == ROTATED else 2):
+                tail.B[i] = ws[i][0].data_ptr()
+        if mode == ROTATED:
+            d, seq = max(e for e in (8, 4, 2, 36, 48) if N % e == 0 and e < N or e == 2), (M + 1) // 2
+            table, tr = dev(rng.standard_normal((seq, d // 2, 2)), "f32")
+            tail.table, tail.seq, tail.head_dim, tail.rotated, tail.count = table.data_ptr(), seq, d, 2, 3
+        assert _run(x, ws[0][0], tail, M, N, K, tb, dt) == 0
+        prods = [_product(xr, w[1], tb, dt) for w in ws]
+        if mode == GATED:
+            for i in range(2):
+                _close(out[i], prods[i][0], prods[i][1], dt, "h%d" % (1 + 2 * i))
+            a, b = host(out[0]), host(out[1])
+            _close(out[2], a * _sigmoid(a) * b, 0.0, dt, "g")
+        elif mode == ADJOINT:
+            (dg, e), s = prods[0], _sigmoid(a)
+            slope = 1.0 + a * (1.0 - s)
+            _close(out[0], dg * b * s * slope, np.abs(b * s) * (np.abs(slope) * e + 2.0 ** -19 * np.abs(dg) * (1.0 + np.abs(a))), dt, "dh1")
+            _close(out[1], dg * a * s, np.abs(a * s) * e, dt, "dh3")
+        else:
+            at, pair = np.arange(M)[:, None] % seq, np.arange(N)[None, :] % d // 2
+            c, s = tr[at, pair, 0], tr[at, pair, 1]
+            for i in range(2):
+                (p, e), other = prods[i], np.arange(N) ^ 1
+                sign = np.where(np.arange(N) % 2 == 0, -1.0, 1.0)
+                _close(out[i], c * p + sign * s * p[:, other], np.abs(c) * e + np.abs(s) * e[:, other] + 2.0 ** -22 * (np.abs(c * p) + np.abs(s * p[:, other])), dt, "result %d" % i)
+            _close(out[2], prods[2][0], prods[2][1], dt, "result 2")
+
+
+def test_what_the_kernels_do_not_take_is_left_to_the_separate_launches():
+    """Rows of no whole pieces, operands off 16 bytes, few rows, a k-major weight where there is no kernel: -1 and nothing written."""
+    x, w, h = (torch.ones(64 * 64 + 8, device="cuda") for _ in range(3))
+    out = [torch.full((64, 64), 7.0, device="cuda") for _ in range(3)]
+
+    def tail(mode, shift=0):
+        t = _Tail(mode=mode, h1=h.data_ptr() + shift, h3=h.data_ptr())
+        for i in range(3):
+            t.B[i], t.C[i] = w.data_ptr(), out[i].data_ptr()
+        return t
+
+    for M, N, K, tb, t in ((64, 62, 64, 1, tail(GATED)), (64, 64, 62, 1, tail(ADJOINT)), (8, 64, 64, 1, tail(GATED)), (64, 64, 64, 0, tail(GATED)),
+                           (64, 64, 64, 1, tail(ADJOINT, 4))):
+        assert _run(x, w, t, M, N, K, tb, "f32") == -1
+    assert all(bool((o == 7.0).all()) for o in out)
