@@ -437,8 +437,8 @@ __global__ __launch_bounds__(256) void rope_kernel(const T* x, const float2* __r
     const float cs = (p & 1) ? t[p >> 1].z : t[p >> 1].x;
     const float sn = (p & 1) ? t[p >> 1].w : t[p >> 1].y;
     const float sp = inverse ? -sn : sn;
-    o[2 * p] = cs * v[2 * p] - sp * v[2 * p + 1];
-    o[2 * p + 1] = sp * v[2 * p] + cs * v[2 * p + 1];
+    o[2 * p] = rotated_even(cs, sp, v[2 * p], v[2 * p + 1]);
+    o[2 * p + 1] = rotated_odd(cs, sp, v[2 * p], v[2 * p + 1]);
   }
   ChunkCached<T>::store(y + (int64_t)row * row_elems + col, o);
 }
@@ -455,8 +455,8 @@ __global__ __launch_bounds__(256) void rope_pair_kernel(const T* x, const float2
   const float2 t = table[(int64_t)s * (head_dim >> 1) + (in_head >> 1)];
   const float sp = inverse ? -t.y : t.y;
   const float v0 = to_f32(x[e]), v1 = to_f32(x[e + 1]);
-  y[e] = from_f32<T>(t.x * v0 - sp * v1);
-  y[e + 1] = from_f32<T>(sp * v0 + t.x * v1);
+  y[e] = from_f32<T>(rotated_even(t.x, sp, v0, v1));
+  y[e + 1] = from_f32<T>(rotated_odd(t.x, sp, v0, v1));
 }
 
 // ---------------------------------------------------------------------------

@@ -2075,7 +2075,8 @@ int emi::gemm_tail(hipStream_t st, const void* A, const void* B, const ProductTa
   if (M <= 8 || N <= 0 || K <= 0 || N % v || K % v || ldb % v || M * K >= most || b_rows * ldb >= most || M * N >= most) return -1;
   uintptr_t all = reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(t.h1) |
                   reinterpret_cast<uintptr_t>(t.h3) | reinterpret_cast<uintptr_t>(t.table);
-  for (int i = 0; i < 3; i++) all |= reinterpret_cast<uintptr_t>(t.B[i]) | reinterpret_cast<uintptr_t>(t.C[i]);
+  all |= reinterpret_cast<uintptr_t>(t.A1);
+  for (int i = 0; i < 3; i++) all |= reinterpret_cast<uintptr_t>(t.B[i]) | reinterpret_cast<uintptr_t>(t.B1[i]) | reinterpret_cast<uintptr_t>(t.C[i]);
   if (all & 15) return -1;
   return dtype == EMI_BF16 ? launch_bf16_pipe_tail(st, A, B, t, (int)M, (int)N, (int)K, (int)ldb, trans_b)
                            : launch_f32_tail(st, A, B, t, M, N, K, ldb, trans_b);

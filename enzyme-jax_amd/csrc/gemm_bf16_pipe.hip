@@ -119,7 +119,8 @@ template <> struct PipeArg<kTailRotated> {
     const uint16_t* B[3];
     uint16_t* C[3];
     const float2* table;
-    int seq, head_dim, rotated;
+    int seq, head_dim, rotated, pairs;
+    const uint16_t *A1, *B1[3];
   };
 };
 template <> struct PipeArg<kTailAdjoint> {
@@ -186,6 +187,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
   if constexpr (MODE == kTailRotated) {
     B = grp.B[outer];
     C = grp.C[outer];
+    nsteps *= grp.pairs;
   }
   if (part != nullptr) {
     step0 = outer * steps_per_split;
@@ -229,6 +231,13 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
       if (at_k >= K) {
         at_k = 0;
         B = grp.B1;
+      }
+    }
+    if constexpr (MODE == kTailRotated) {
+      if (at_k >= K && to_issue > 0) {
+        at_k = 0;
+        A = grp.A1;
+        B = grp.B1[outer];
       }
     }
   };
@@ -416,8 +425,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
 #pragma unroll
           for (int q = 0; q < 4; q++) {
             const float2 t = angles[((gcol + 2 * q) % grp.head_dim) >> 1];
-            o[2 * q] = t.x * v[2 * q] - t.y * v[2 * q + 1];
-            o[2 * q + 1] = t.y * v[2 * q] + t.x * v[2 * q + 1];
+            o[2 * q] = rotated_even(t.x, t.y, v[2 * q], v[2 * q + 1]);
+            o[2 * q + 1] = rotated_odd(t.x, t.y, v[2 * q], v[2 * q + 1]);
           }
           z = pack8(o);
         }
@@ -643,7 +652,10 @@ static int launch_pipe_tail_one(hipStream_t st, const uint16_t* A, const uint16_
     for (int i = 0; i < t.count; i++) {
       arg.B[i] = static_cast<const uint16_t*>(t.B[i]);
       arg.C[i] = static_cast<uint16_t*>(t.C[i]);
+      arg.B1[i] = static_cast<const uint16_t*>(t.B1[i]);
     }
+    arg.A1 = static_cast<const uint16_t*>(t.A1);
+    arg.pairs = t.A1 != nullptr ? 2 : 1;
     arg.table = reinterpret_cast<const float2*>(t.table);
     arg.seq = t.seq, arg.head_dim = t.head_dim, arg.rotated = t.rotated;
   } else {
@@ -669,15 +681,22 @@ static int launch_pipe_tail_shape(hipStream_t st, const uint16_t* A, const uint1
 // as the separate launches, none slower by more than 2 %.  What is for the 256-tiles goes there.
 int launch_bf16_pipe_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int M, int N, int K, int ldb, int trans_b) {
   if (t.mode != kTailAdjoint && !trans_b) return -1;
-  const int count = t.mode == kTailGated ? 2 : t.mode == kTailRotated ? t.count : 1, sum = t.mode == kTailGated;
-  const Bf16Plan p = bf16_plan(M, N, K, count, sum, trans_b, 1), group = bf16_plan(M, N, K, count, 0, trans_b, 1),
+  const int count = t.mode == kTailGated ? 2 : t.mode == kTailRotated ? t.count : 1, sum = t.mode == kTailGated, pairs = t.A1 != nullptr ? 2 : 1;
+  const Bf16Plan p = bf16_plan(M, N, (int64_t)K * pairs, count, sum, trans_b, 1), group = bf16_plan(M, N, K, count, 0, trans_b, 1),
                  one = bf16_plan(M, N, K, 1, 0, trans_b, kAnySplits);
-  const double singly = count * (one.us + 1.0) - 1.0, apart = singly < group.us ? singly : group.us;
+  double apart = count * (one.us + 1.0) - 1.0;
+  if (pairs == 2) {                                        // each result a launch that sums its two products, or two
+    const double summed = bf16_plan(M, N, K, 2, 1, trans_b, sum_splits(M, N, kAnySplits)).us;
+    apart = count * ((summed < 2 * one.us + 1.0 ? summed : 2 * one.us + 1.0) + 1.0) - 1.0;
+  } else if (group.us < apart) {
+    apart = group.us;
+  }
   const double moved = 2e-6 / 5.0 * M * N * (t.mode == kTailRotated ? 2 * t.rotated : t.mode == kTailGated ? 3 : 5);
+  const double pass = t.mode == kTailRotated && t.rotated == 0 ? 0.0 : 2.4 + moved;
   const double results = t.mode != kTailGated ? 0.0 : p.shape == 5 ? 1.2 : 2.2;
-  if (p.shape == 0 || one.shape == 0 || p.us + results >= apart + 2.4 + moved) return -1;
+  if (p.shape == 0 || (one.shape == 0 && pairs == 1) || p.us + results >= apart + pass) return -1;
   const uint16_t *a = static_cast<const uint16_t*>(A), *b = static_cast<const uint16_t*>(B);
-  switch (bf16_kernel(p, M, N, K, count, sum, trans_b)) {
+  switch (bf16_kernel(p, M, N, (int64_t)K * pairs, count, sum, trans_b)) {
     case 1: return launch_pipe_tail_shape<128, 128, 4, 2, 1, 64, 2>(st, a, b, t, M, N, K, ldb, trans_b);
     case 2: return launch_pipe_tail_shape<128, 128, 4, 2, 2, 64, 3>(st, a, b, t, M, N, K, ldb, trans_b);
     case 3: return launch_pipe_tail_shape<128, 64, 4, 2, 1, 64, 3>(st, a, b, t, M, N, K, ldb, trans_b);

@@ -108,7 +108,8 @@ template <> struct F32Arg<kTailRotated> {
     const float* B[3];
     float* C[3];
     const float2* table;
-    int seq, head_dim, rotated;
+    int seq, head_dim, rotated, pairs;
+    const float *A1, *B1[3];
   };
 };
 template <> struct F32Arg<kTailAdjoint> {
@@ -169,6 +170,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
   if constexpr (MODE == kTailRotated) {
     B = grp.B[outer];
     C = grp.C[outer];
+    nsteps *= grp.pairs;
   }
   if (part != nullptr) {
     step0 = outer * steps_per_split;
@@ -212,6 +214,13 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
       if (at_k >= K) {
         at_k = 0;
         B = grp.B1;
+      }
+    }
+    if constexpr (MODE == kTailRotated) {
+      if (at_k >= K && to_issue > 0) {
+        at_k = 0;
+        A = grp.A1;
+        B = grp.B1[outer];
       }
     }
   };
@@ -334,7 +343,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
   auto put = [&](int row, int col, float v, float h1, float p, float q) __attribute__((always_inline)) {
     if constexpr (MODE == kTailRotated) {                  // the pair's other column is the neighbouring lane's, of the same row
       const float other = lane_xor1(v);
-      v = (col & 1) == 0 ? p * v - q * other : q * other + p * v;
+      v = (col & 1) == 0 ? rotated_even(p, q, v, other) : rotated_odd(p, q, other, v);
     }
     if (row < M && col < N) {
       if (part != nullptr) {
@@ -559,7 +568,10 @@ static int launch_f32_tail_one(hipStream_t st, const float* A, const float* B, c
     for (int i = 0; i < t.count; i++) {
       arg.B[i] = static_cast<const float*>(t.B[i]);
       arg.C[i] = static_cast<float*>(t.C[i]);
+      arg.B1[i] = static_cast<const float*>(t.B1[i]);
     }
+    arg.A1 = static_cast<const float*>(t.A1);
+    arg.pairs = t.A1 != nullptr ? 2 : 1;
     arg.table = reinterpret_cast<const float2*>(t.table);
     arg.seq = t.seq, arg.head_dim = t.head_dim, arg.rotated = t.rotated;
   } else {
@@ -585,14 +597,17 @@ static int launch_f32_tail_shape(hipStream_t st, const float* A, const float* B,
 int launch_f32_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b) {
   if (128 * K + K >= 0x1fffffff || 128 * ldb + K >= 0x1fffffff || (t.mode != kTailAdjoint && !trans_b)) return -1;
   const int count = t.mode == kTailGated ? 2 : t.mode == kTailRotated ? t.count : 1;
+  const int pairs = t.A1 != nullptr ? 2 : 1;
   double together[2];
   for (int c = 0; c < 2; c++) {
     const int64_t blocks = (M + kF32Shape[c].bm - 1) / kF32Shape[c].bm * ((N + kF32Shape[c].bn - 1) / kF32Shape[c].bn) * (t.mode == kTailRotated ? count : 1);
-    together[c] = f32_estimate(c, M, N, K, count, t.mode == kTailGated, 0, 1) + (c == 0 ? 3.0 : 0.8) * ((blocks + 255) / 256);
+    together[c] = f32_estimate(c, M, N, K * pairs, count, t.mode == kTailGated, 0, 1) + (c == 0 ? 3.0 : 0.8) * ((blocks + 255) / 256);
   }
   const int shape = together[1] < together[0];
   const double moved = 4e-6 / 5.0 * M * N * (t.mode == kTailRotated ? 2 * t.rotated : t.mode == kTailGated ? 3 : 5);
-  if (together[shape] >= f32_plan(M, N, K, count, 0, 0, count > 1 ? 1 : kAnySplits).us + 2.4 + moved) return -1;
+  // (two products to a result: each result would be a launch that sums them)
+  const double apart = pairs == 2 ? count * (f32_plan(M, N, K, 2, 1, 0, kAnySplits).us + 1.0) : f32_plan(M, N, K, count, 0, 0, count > 1 ? 1 : kAnySplits).us;
+  if (together[shape] >= apart + (t.mode == kTailRotated && t.rotated == 0 ? 0.0 : 2.4 + moved)) return -1;
   const float *a = static_cast<const float*>(A), *b = static_cast<const float*>(B);
   return shape == 0 ? launch_f32_tail_shape<64, 64, 2, 2, 1, 32, 2>(st, a, b, t, (int)M, (int)N, (int)K, (int)ldb, trans_b)
                     : launch_f32_tail_shape<32, 32, 1, 1, 8, 64, 5>(st, a, b, t, (int)M, (int)N, (int)K, (int)ldb, trans_b);

@@ -32,6 +32,11 @@ inline int64_t splits_held(const void* workspace, size_t bytes, int64_t M, int64
   return n < 1 ? 1 : n < kAnySplits ? n : kAnySplits;
 }
 
+// Splits of a sum of two long products: none where its tiles of 128 leave hardly a CU idle.  Two blocks on every CU are estimated
+// at the rate of operands that the L2s still hold, which those of a long contraction are not: two of 1000 x 4096 x 4096, us,
+// in two splits 85 (estimate 71), in one pass 84 (73), one by one 80; two of 1000 x 4096 x 11008 212 (163), one by one 178.
+inline int64_t sum_splits(int64_t M, int64_t N, int64_t held) { return (M + 127) / 128 * ((N + 127) / 128) >= 192 ? 1 : held; }
+
 // Whether products that can run as one launch, each in a single pass over K, run one by one: where each split over K is so
 // much faster that together they are, by more than the estimates are off (`margin`: bf16 products of a few rows are
 // estimated up to a third too fast, fp32 ones hardly).  A launch more each, and the gap before it.  us, one launch | one by one:
@@ -65,6 +70,7 @@ struct ProductTail {
   const float* table;          // rotated: results 0 .. rotated - 1 by the angle of row % seq
   int seq, head_dim, rotated, count;
   const void *h1, *h3;         // adjoint: the SwiGLU's operands; the product is the cotangent of its result
+  const void *A1, *B1[3];      // rotated, unless A1 is null: each result is A B[i]^T + A1 B1[i]^T (a tangent's two products)
 };
 int launch_bf16_pipe_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int M, int N, int K, int ldb, int trans_b);      // gemm_bf16_pipe.hip
 int launch_f32_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b);      // gemm_f32.hip

@@ -168,7 +168,7 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
     EMI_TRY(emi_gemm_rope(st, s.xb1, w[kK], s.k, table, T, D, D, d.S, d.hd(), d.dtype));
     EMI_TRY(emi_gemm_ws(st, s.xb1, w[kV], nullptr, s.v, ws, wsb, T, D, D, D, D, D, D, 0, 1, d.dtype));
   } else {
-    emi::ProductTail t{emi::kTailRotated, {w[kQ], w[kK], w[kV]}, {s.q, s.k, s.v}, table, (int)d.S, (int)d.hd(), 2, 3, nullptr, nullptr};
+    emi::ProductTail t{emi::kTailRotated, {w[kQ], w[kK], w[kV]}, {s.q, s.k, s.v}, table, (int)d.S, (int)d.hd(), 2, 3, nullptr, nullptr, nullptr, {}};
     if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(st), s.xb1, w[kQ], t, T, D, D, D, 1, d.dtype); rc > 0) return rc;
     else if (rc < 0) {
       const void *a[3] = {s.xb1, s.xb1, s.xb1}, *b[3] = {w[kQ], w[kK], w[kV]};
@@ -179,7 +179,7 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
   }
   EMI_TRY(emi_attn_fwd(st, s.q, s.k, s.v, s.att, s.lse, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
   EMI_TRY(product_and_norm(st, s.att, w[kO], x, s.x1, w[kFfn], s.xb2, ws, wsb, D, d));
-  emi::ProductTail t{emi::kTailGated, {w[kW1], w[kW3], nullptr}, {s.h1, s.h3, s.g}, nullptr, 0, 0, 0, 0, nullptr, nullptr};
+  emi::ProductTail t{emi::kTailGated, {w[kW1], w[kW3], nullptr}, {s.h1, s.h3, s.g}, nullptr, 0, 0, 0, 0, nullptr, nullptr, nullptr, {}};
   if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(st), s.xb2, w[kW1], t, T, H, D, D, 1, d.dtype); rc > 0) {
     return rc;
   } else if (rc == 0) {
@@ -194,6 +194,110 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
   }
   if (next_xb != nullptr) return product_and_norm(st, s.g, w[kW2], s.x1, out, next_gamma, next_xb, ws, wsb, H, d);
   return emi_gemm_ws(st, s.g, w[kW2], s.x1, out, ws, wsb, T, D, H, H, H, D, D, 0, 1, d.dtype);
+}
+
+// ---- forward mode: the tangents of one layer behind its values --------------------------------------------------------------
+
+struct Tangents {                                         // of one layer
+  void *xb, *q, *k, *v, *att, *x1, *h1, *h3, *g, *out[2];  // (the second norm's goes where the first one's was); out: of even and odd layers
+};
+struct JvpScratch {
+  void* saved[2];                                         // of even and odd layers: a layer's product with w2 leaves the next one's xb1
+  Tangents t;
+  void* ws;
+  size_t ws_bytes;
+};
+JvpScratch carve_jvp(void* base, const Dims& d, size_t* bytes = nullptr) {
+  Carve c{static_cast<uint8_t*>(base), 0};
+  const int64_t T = d.T();
+  const size_t td = (size_t)T * d.D * d.elt(), th = (size_t)T * d.H * d.elt();
+  size_t n = 0;
+  carve_saved(nullptr, d, &n);
+  JvpScratch s;
+  for (void*& p : s.saved) p = c.take(n);
+  s.t.xb = c.take(td);
+  s.t.q = c.take(3 * td);
+  s.t.k = part(s.t.q, td);
+  s.t.v = part(s.t.q, 2 * td);
+  s.t.att = c.take(td);
+  s.t.x1 = c.take(td);
+  s.t.h1 = c.take(th);
+  s.t.h3 = c.take(th);
+  s.t.g = c.take(th);
+  for (void*& p : s.t.out) p = c.take(td);
+  s.ws_bytes = most({forward_scratch(d), emi_gemm_grouped_workspace_bytes(2, T, d.D, d.D, 0, 1, 1, d.dtype),
+                     emi_gemm_grouped_workspace_bytes(2, T, d.H, d.D, 0, 1, 1, d.dtype), emi_gemm_grouped_workspace_bytes(2, T, d.D, d.H, 0, 1, 1, d.dtype)});
+  s.ws = c.take(s.ws_bytes);
+  if (bytes != nullptr) *bytes = c.at;
+  return s;
+}
+
+// Estimates for one result of tangent_product: its two products one by one, and as one launch that sums them.
+struct TangentPlan {
+  double two, sum;
+  int64_t splits;
+};
+TangentPlan tangent_plan(int64_t N, int64_t K, const JvpScratch& k, const Dims& d) {
+  const int64_t T = d.T(), held = emi::splits_held(k.ws, k.ws_bytes, T, N), most = emi::sum_splits(T, N, held);
+  if (d.dtype == EMI_F32) return {2 * emi::f32_plan(T, N, K, 1, 0, 0, held).us + 1.0, emi::f32_plan(T, N, K, 2, 1, 0, most).us, most};
+  // (long sums that fill the chip run a tenth longer than estimated: two of 1000 x 4096 x 4096 84 us, one by one 80)
+  return {2 * emi::bf16_plan(T, N, K, 1, 0, 1, held).us + 1.0, emi::bf16_plan(T, N, K, 2, 1, 1, most).us * (most > 1 ? 1.0 : 1.1), most};
+}
+
+// ty = tx w^T + x tw^T [+ r]
+int tangent_product(emi_stream_t st, const void* tx, const void* x, const void* w, const void* tw, const void* r, void* ty, int64_t N, int64_t K,
+                    const JvpScratch& k, const Dims& d) {
+  const int64_t T = d.T();
+  const TangentPlan p = tangent_plan(N, K, k, d);
+  if (p.two < p.sum) {
+    EMI_TRY(emi_gemm_ws(st, x, tw, r, ty, k.ws, k.ws_bytes, T, N, K, K, K, N, N, 0, 1, d.dtype));
+    return emi_gemm_ws(st, tx, w, ty, ty, k.ws, k.ws_bytes, T, N, K, K, K, N, N, 0, 1, d.dtype);
+  }
+  const void *a[2] = {tx, x}, *b[2] = {w, tw}, *res[1] = {r};
+  void* out[1] = {ty};
+  return emi_gemm_grouped(st, 2, a, b, r != nullptr ? res : nullptr, out, p.splits > 1 ? k.ws : nullptr, p.splits > 1 ? k.ws_bytes : 0, T, N, K, K, K, N, N,
+                          0, 1, 1, d.dtype);
+}
+
+// Several results of tangent_product that share x and tx; the first `rotated` turned.  One launch where that is faster, or the
+// products with every tw as one group and those with every w, which add to them, as another (bf16: the 256-tiles of three
+// results fill the chip where one's do not, 1000 x 4096 x 4096 180 us, result by result 241).
+int tangent_products(emi_stream_t st, const void* tx, const void* x, std::initializer_list<int> which, const void* const* w, const void* const* tw,
+                     std::initializer_list<void*> out, int rotated, const float* table, int64_t N, const JvpScratch& k, const Dims& d) {
+  emi::ProductTail t{emi::kTailRotated, {}, {}, rotated ? table : nullptr, (int)d.S, (int)d.hd(), rotated, 0, nullptr, nullptr, x, {}};
+  for (int i : which) {
+    t.B[t.count] = w[i];
+    t.B1[t.count] = tw[i];
+    t.C[t.count] = out.begin()[t.count];
+    t.count++;
+  }
+  const int rc = emi::gemm_tail(static_cast<hipStream_t>(st), tx, t.B[0], t, d.T(), N, d.D, d.D, 1, d.dtype);
+  if (rc >= 0) return rc;
+  const TangentPlan p = tangent_plan(N, d.D, k, d);
+  const double group = d.dtype == EMI_F32 ? emi::f32_plan(d.T(), N, d.D, t.count, 0, 0, 1).us : emi::bf16_plan(d.T(), N, d.D, t.count, 0, 1, 1).us;
+  if (2 * group + 1.0 < t.count * ((p.two < p.sum ? p.two : p.sum) + 1.0)) {
+    const void *xs[3] = {x, x, x}, *txs[3] = {tx, tx, tx};
+    EMI_TRY(emi_gemm_grouped(st, t.count, xs, t.B1, nullptr, t.C, k.ws, k.ws_bytes, d.T(), N, d.D, d.D, d.D, N, N, 0, 1, 0, d.dtype));
+    EMI_TRY(emi_gemm_grouped(st, t.count, txs, t.B, t.C, t.C, k.ws, k.ws_bytes, d.T(), N, d.D, d.D, d.D, N, N, 0, 1, 0, d.dtype));
+  } else {
+    for (int i = 0; i < t.count; i++) EMI_TRY(tangent_product(st, tx, x, t.B[i], t.B1[i], nullptr, t.C[i], N, d.D, k, d));
+  }
+  return rotated ? emi_rope(st, t.C[0], table, t.C[0], rotated * d.B, d.S, d.heads, d.hd(), 0, d.dtype) : EMI_OK;      // (side by side)
+}
+
+// s: the layer's values;  tx: the tangent of its input x.
+int tangent_layer(emi_stream_t st, const void* const* w, const void* const* tw, const void* x, const void* tx, const float* table, const Saved& s,
+                  const JvpScratch& k, void* tout, const Dims& d) {
+  const Tangents& t = k.t;
+  const int64_t T = d.T(), D = d.D, H = d.H;
+  EMI_TRY(emi_rmsnorm_jvp(st, x, w[kAtt], tx, tw[kAtt], t.xb, T, D, d.eps, d.dtype));
+  EMI_TRY(tangent_products(st, t.xb, s.xb1, {kQ, kK, kV}, w, tw, {t.q, t.k, t.v}, 2, table, D, k, d));
+  EMI_TRY(emi_attn_jvp(st, s.q, s.k, s.v, s.lse, t.q, t.k, t.v, t.att, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
+  EMI_TRY(tangent_product(st, t.att, s.att, w[kO], tw[kO], tx, t.x1, D, D, k, d));
+  EMI_TRY(emi_rmsnorm_jvp(st, s.x1, w[kFfn], t.x1, tw[kFfn], t.xb, T, D, d.eps, d.dtype));
+  EMI_TRY(tangent_products(st, t.xb, s.xb2, {kW1, kW3}, w, tw, {t.h1, t.h3}, 0, nullptr, H, k, d));
+  EMI_TRY(emi_swiglu_jvp(st, s.h1, s.h3, t.h1, t.h3, t.g, T * H, d.dtype));
+  return tangent_product(st, t.g, s.g, w[kW2], tw[kW2], t.x1, tout, D, H, k, d);
 }
 
 // dW = dY^T X of one shape, waiting to run as one launch.
@@ -363,7 +467,7 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     // the group's last layer writes its dx where the dy of the group's first one lies (the last slot's dx, of the group before)
     const bool ends_group = (done + 1) % group == 0 || l == 0;
     if (ends_group) EMI_TRY(flush(stream, down, D, H, T, r, dtype));
-    emi::ProductTail t{emi::kTailAdjoint, {}, {c.dh1, c.dh3, nullptr}, nullptr, 0, 0, 0, 0, s.h1, s.h3};
+    emi::ProductTail t{emi::kTailAdjoint, {}, {c.dh1, c.dh3, nullptr}, nullptr, 0, 0, 0, 0, s.h1, s.h3, nullptr, {}};
     if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(stream), dy, b[kW2], t, T, H, D, tb ? D : H, tb, dtype); rc > 0) {
       return rc;
     } else if (rc == 0) {
@@ -411,6 +515,44 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
       EMI_TRY(flush(stream, norms, d));
     }
     dy = dx_l;
+  }
+  return EMI_OK;
+}
+
+extern "C" size_t emi_llama_layers_jvp_workspace_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype) {
+  const Dims d{1, batch, seq, dim, hidden, heads, 0.f, 0.f, dtype};
+  if (!d.ok()) return 0;
+  size_t n = 0;
+  carve_jvp(nullptr, d, &n);
+  return n;
+}
+
+extern "C" int emi_llama_layers_jvp(emi_stream_t stream, const void* const* weights, const void* const* tangents, const void* x, const void* tx,
+                                    const float* rope_table, void* y, void* ty, void* workspace, size_t workspace_bytes, int64_t layers,
+                                    int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, float eps, float scale, int dtype) {
+  const Dims d{layers, batch, seq, dim, hidden, heads, eps, scale, dtype};
+  if (int rc = check_layers("emi_llama_layers_jvp", d, weights, {x, tx, rope_table, y, ty, workspace, tangents})) return rc;
+  for (int i = 0; i < kWeights; i++)
+    if (tangents[i] == nullptr) return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_jvp: tangent %d is null", i);
+  size_t need = 0;
+  const JvpScratch k = carve_jvp(workspace, d, &need);
+  if (workspace_bytes < need)
+    return emi_fail(EMI_INVALID_ARGUMENT, "emi_llama_layers_jvp: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
+  for (int64_t l = 0; l < layers; l++) {
+    const void *w[kWeights], *tw[kWeights];
+    for (int i = 0; i < kWeights; i++) {
+      const size_t off = weight_elements(i, d) * (size_t)l * d.elt();
+      w[i] = part(weights[i], off);
+      tw[i] = part(tangents[i], off);
+    }
+    const bool last = l + 1 == layers;
+    const Saved s = carve_saved(k.saved[l & 1], d), next = carve_saved(k.saved[(l + 1) & 1], d);
+    if (l == 0) EMI_TRY(emi_rmsnorm_fwd(stream, x, w[kAtt], s.xb1, d.T(), dim, eps, dtype));
+    void *out = last ? y : s.out, *tout = last ? ty : k.t.out[l & 1];
+    EMI_TRY(forward_layer(stream, w, x, rope_table, s, out, part(w[kAtt], last ? 0 : (size_t)dim * d.elt()), last ? nullptr : next.xb1, k.ws, k.ws_bytes, d));
+    EMI_TRY(tangent_layer(stream, w, tw, x, tx, rope_table, s, k, tout, d));
+    x = out;
+    tx = tout;
   }
   return EMI_OK;
 }

@@ -87,6 +87,9 @@ SIGNATURES = {
     "emi_llama_layers_bwd": (c_int, [c_void_p, ctypes.POINTER(c_void_p), ctypes.POINTER(c_void_p), c_void_p, c_void_p,
                                      ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_void_p, ctypes.POINTER(c_void_p),
                                      ctypes.POINTER(c_void_p), c_int, c_void_p, c_size_t] + [c_i64] * 6 + [c_float, c_float, c_int]),
+    "emi_llama_layers_jvp_workspace_bytes": (c_size_t, [c_i64] * 5 + [c_int]),
+    "emi_llama_layers_jvp": (c_int, [c_void_p, ctypes.POINTER(c_void_p), ctypes.POINTER(c_void_p)] + [c_void_p] * 6 + [c_size_t] + [c_i64] * 6 +
+                             [c_float, c_float, c_int]),
     "emi_rmsnorm_jvp": (c_int, [c_void_p] * 6 + [c_i64, c_i64, c_float, c_int]),
     "emi_swiglu_jvp": (c_int, [c_void_p] * 6 + [c_i64, c_int]),
     "emi_attn_jvp": (c_int, [c_void_p] * 9 + [c_i64] * 7 + [c_float, c_int, c_int]),

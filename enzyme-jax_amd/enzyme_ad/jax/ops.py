@@ -1156,7 +1156,7 @@ def llama_step(x, weights, key_cache, value_cache, n_heads, table, eps=1e-5, sca
     _dev(x, *weights, key_cache, value_cache, table)
     _same_dtype(x, *weights, key_cache, value_cache)
     if len(weights) != len(STEP_WEIGHTS) or not llama_step_applies(x, weights, key_cache, value_cache, n_heads):
-        raise ValueError("llama_step: x %s, caches %s / %s, %d heads and these weights, or forward mode, are not served (see llama_step_applies)" %
+        raise ValueError("llama_step: x %s, caches %s / %s, %d heads and these weights or tangents are not served (see llama_step_applies)" %
                          (tuple(x.shape), tuple(key_cache.shape), tuple(value_cache.shape), n_heads))
     return _llama_step(x, weights, key_cache, value_cache, n_heads, table, eps, scale)
 
@@ -1193,10 +1193,17 @@ def _llama_step(x, weights, key_cache, value_cache, n_heads, table, eps=1e-5, sc
 
 
 def llama_layers_apply(x, weights, n_heads):
-    """Whether `llama_layers` serves these operands (else a layer runs operator by operator): reverse or no
-    differentiation, one dtype, contiguous aligned stacks, rows of whole 16-byte pieces, more than a few tokens."""
-    if Forward._active is not None or x.dim() != 3 or x.dtype not in _DTYPES:
+    """Whether `llama_layers` serves these operands (else a layer runs operator by operator): one dtype, contiguous aligned
+    stacks, rows of whole 16-byte pieces, more than a few tokens; under forward mode a tangent on every one of them, laid out
+    as they are, and no tape beside it."""
+    if x.dim() != 3 or x.dtype not in _DTYPES:
         return False
+    if Forward._active is not None:
+        if Tape._active is not None:
+            return False
+        for t in _tan(x, *weights):
+            if t is None or not t.is_contiguous() or t.data_ptr() & 15 or not t.is_cuda:
+                return False
     w1 = weights[6]
     stack = w1.shape[:-2]
     if w1.dim() not in (2, 3):
@@ -1220,7 +1227,7 @@ def llama_layers(x, weights, n_heads, table, eps=1e-5, scale=None):
     _dev(x, *weights, table)
     _same_dtype(x, *weights)
     if len(weights) != 9 or not llama_layers_apply(x, weights, n_heads):
-        raise ValueError("llama_layers: x %s with %d heads and these weights, or forward mode, are not served (see llama_layers_apply)" %
+        raise ValueError("llama_layers: x %s with %d heads and these weights or tangents are not served (see llama_layers_apply)" %
                          (tuple(x.shape), n_heads))
     return _llama_layers(x, weights, n_heads, table, eps, scale)
 
@@ -1236,6 +1243,14 @@ def _llama_layers(x, weights, n_heads, table, eps=1e-5, scale=None):
         scale = 1.0 / math.sqrt(D // n_heads)
     shape = (B, S, D, H, n_heads)
     dims = (L_,) + shape + (eps, float(scale), code)
+    if Forward._active is not None:
+        tx, *tw = _tan(x, *weights)
+        nws = lib.emi_llama_layers_jvp_workspace_bytes(*shape, code)
+        ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
+        y, ty = torch.empty_like(x), torch.empty_like(x)
+        N.check(lib.emi_llama_layers_jvp(_stream(), _ptr_table(weights), _ptr_table(tw), _p(x), _p(tx), _p(table), _p(y), _p(ty), _p(ws), nws, *dims))
+        _set_tan(y, ty)
+        return y
     nsaved = lib.emi_llama_layers_saved_bytes(*shape, code)
     keep = Tape._active is not None
     saved = [torch.empty(nsaved, dtype=torch.uint8, device=x.device) for _ in range(L_ if keep else 1)]

@@ -309,6 +309,15 @@ int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weights, void* 
                          int64_t layers, int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, float eps,
                          float scale, int dtype);
 
+/* Forward mode of the same layers: their values and the tangents of x and of every weight (in the
+ * order and shapes of weights; none null) carried through, y and ty[B, S, D].  workspace:
+ * emi_llama_layers_jvp_workspace_bytes. */
+size_t emi_llama_layers_jvp_workspace_bytes(int64_t batch, int64_t seq, int64_t dim, int64_t hidden, int64_t heads, int dtype);
+int emi_llama_layers_jvp(emi_stream_t stream, const void* const* weights, const void* const* tangents, const void* x,
+                         const void* tx, const float* rope_table, void* y, void* ty, void* workspace,
+                         size_t workspace_bytes, int64_t layers, int64_t batch, int64_t seq, int64_t dim, int64_t hidden,
+                         int64_t heads, float eps, float scale, int dtype);
+
 /* Forward mode of the single-token attention (emi_attn_step_fwd's layout, o and lse from
  * it): to = sum_s p_s (tS_s v_s + tv_s) - (sum_s p_s tS_s) o with tS_s = scale (tq.k_s + q.tk_s).
  * Null tq / tk / tv = zero tangent.  workspace: emi_attn_step_workspace_bytes(). */

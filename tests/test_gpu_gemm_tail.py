@@ -17,7 +17,8 @@ GATED, ROTATED, ADJOINT = 2, 3, 4
 
 class _Tail(ctypes.Structure):
     _fields_ = [("mode", ctypes.c_int), ("B", ctypes.c_void_p * 3), ("C", ctypes.c_void_p * 3), ("table", ctypes.c_void_p), ("seq", ctypes.c_int),
-                ("head_dim", ctypes.c_int), ("rotated", ctypes.c_int), ("count", ctypes.c_int), ("h1", ctypes.c_void_p), ("h3", ctypes.c_void_p)]
+                ("head_dim", ctypes.c_int), ("rotated", ctypes.c_int), ("count", ctypes.c_int), ("h1", ctypes.c_void_p), ("h3", ctypes.c_void_p),
+                ("A1", ctypes.c_void_p), ("B1", ctypes.c_void_p * 3)]
 
 
 def _run(x, w, tail, M, N, K, tb, dt):
@@ -97,6 +98,35 @@ def test_products_with_an_elementwise_tail(dt, mode, M, N, K):
                 sign = np.where(np.arange(N) % 2 == 0, -1.0, 1.0)
                 _close(out[i], c * p + sign * s * p[:, other], np.abs(c) * e + np.abs(s) * e[:, other] + 2.0 ** -22 * (np.abs(c * p) + np.abs(s * p[:, other])), dt, "result %d" % i)
             _close(out[2], prods[2][0], prods[2][1], dt, "result 2")
+
+
+PAIRS = [("f32", 9, 8, 8, 2), ("f32", 35, 72, 68, 2), ("f32", 130, 1408, 516, 0), ("f32", 235, 288, 292, 2), ("bf16", 9, 8, 8, 2), ("bf16", 33, 24, 264, 2),
+         ("bf16", 300, 1400, 520, 0), ("bf16", 450, 520, 520, 2), ("bf16", 777, 776, 776, 2), ("bf16", 1000, 2056, 2056, 0)]
+
+
+@pytest.mark.parametrize("dt,M,N,K,rotated", PAIRS)
+def test_results_of_two_products_each(dt, M, N, K, rotated):
+    """A tangent's two products, of three results (two turned) or of two, in one launch."""
+    rng = np.random.default_rng(M + N + K)
+    (x, xr), (x1, x1r) = (dev(rng.standard_normal((M, K)), dt) for _ in range(2))
+    count, d, seq = 3 if rotated else 2, 8, (M + 1) // 2
+    ws, w1s = ([dev(rng.standard_normal((N, K)) / np.sqrt(K), dt) for _ in range(count)] for _ in range(2))
+    out = [torch.full((M, N), 7.0, device=x.device, dtype=x.dtype) for _ in range(count)]
+    table, tr = dev(rng.standard_normal((seq, d // 2, 2)), "f32")
+    tail = _Tail(mode=ROTATED, table=table.data_ptr() if rotated else None, seq=seq, head_dim=d, rotated=rotated, count=count, A1=x1.data_ptr())
+    for i in range(count):
+        tail.B[i], tail.B1[i], tail.C[i] = ws[i][0].data_ptr(), w1s[i][0].data_ptr(), out[i].data_ptr()
+    assert _run(x, ws[0][0], tail, M, N, K, 1, dt) == 0
+    at, pair, other = np.arange(M)[:, None] % seq, np.arange(N)[None, :] % d // 2, np.arange(N) ^ 1
+    c, s, sign = tr[at, pair, 0], tr[at, pair, 1], np.where(np.arange(N) % 2 == 0, -1.0, 1.0)
+    for i in range(count):
+        p = xr @ ws[i][1].T + x1r @ w1s[i][1].T
+        mag = np.abs(xr) @ np.abs(ws[i][1]).T + np.abs(x1r) @ np.abs(w1s[i][1]).T
+        e = (2.0 ** -8 * np.abs(p) if dt == "bf16" else 0.0) + (2 * K + 2) * 2.0 ** -23 * mag
+        if i < rotated:
+            e = np.abs(c) * e + np.abs(s) * e[:, other] + 2.0 ** -22 * (np.abs(c * p) + np.abs(s * p[:, other]))
+            p = c * p + sign * s * p[:, other]
+        _close(out[i], p, e, dt, "result %d" % i)
 
 
 def test_what_the_kernels_do_not_take_is_left_to_the_separate_launches():

@@ -144,3 +144,41 @@ def test_llama_layers_refuse_what_they_do_not_serve():
         ops.llama_layers(x.bfloat16(), w, 2, table)
     with ops.Forward(), pytest.raises(ValueError):
         ops.llama_layers(x, w, 2, table)
+
+
+@pytest.mark.parametrize("dt,dim,hidden,layers,heads,batch,seq", [
+    ("f32", 64, 72, 5, 2, 1, 33),             # tiles of 32: two products to a result in one launch; layers take turns in two buffers
+    ("f32", 288, 768, 2, 6, 3, 100),
+    ("f32", 512, 1408, 1, 8, 2, 701),         # on the bf16 instructions: a launch to a result, and a pass to turn q and k
+    ("bf16", 128, 136, 3, 2, 2, 131),
+    ("bf16", 768, 2048, 1, 12, 1, 777),
+    ("bf16", 2048, 1024, 1, 16, 2, 512),      # wide enough for two products one after the other
+])
+def test_llama_layers_forward_mode(dt, dim, hidden, layers, heads, batch, seq):
+    """Values and tangents of the layers as one operator against the oracle; the values are those without tangents, and a
+    missing tangent takes the operators one by one to the same result as a zero one."""
+    from enzyme_ad.jax import jvp, llama, ops
+    cfg, wd, wr, x, xr, _, _ = _inputs(dt, dim, hidden, layers, heads, batch, seq)
+    rng = np.random.Generator(np.random.PCG64(3))
+    twd, twr = {}, {}
+    for k in wd:
+        twd[k], twr[k] = dev(rng.standard_normal(wr[k].shape) / np.sqrt(dim), dt)
+    tx, txr = dev(rng.standard_normal(xr.shape), dt)
+    names, table = list(llama.LAYER_KEYS), ops.rope_table(seq, dim // heads, device=x.device)
+
+    def fn(x, w):
+        return ops.llama_layers(x, [w[k] for k in names], heads, table)
+
+    y, ty = jvp(fn, (x, wd), (tx, twd))
+    h, t = xr, txr
+    for i in range(layers):
+        h, t = L.layer_jvp(h, L._layer_weights(wr, i), t, L._layer_weights(twr, i), heads)
+    check(y, h, dt, "y")
+    check(ty, t, dt, "ty")
+    assert torch.equal(y, fn(x, wd))
+    if layers == 1:
+        one, zero = {k: w[0] for k, w in wd.items()}, dict({k: w[0] for k, w in twd.items()}, wq=torch.zeros_like(wd["wq"][0]))
+        a = jvp(lambda x, w: llama.layer(x, w, heads), (x, one), (tx, zero))
+        b = jvp(lambda x, w: llama.layer(x, w, heads), (x, one), (tx, dict(zero, wq=None)))
+        tol = 1e-5 if dt == "f32" else 2e-2
+        assert rel_err(host(a[0]), host(b[0])) < tol and rel_err(host(a[1]), host(b[1])) < tol
