@@ -1555,7 +1555,9 @@ int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
                              int causal);
 int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o,
                              const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
-                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal);
+                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal,
+                             const float* unrope);
+bool attn_f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs);
 
 }  // namespace emi
 
@@ -1692,6 +1694,9 @@ static int attn_bwd_impl(emi_stream_t stream, const void* q, const void* k, cons
     if (!mfma_ok(a, dtype, {q, k, v, o, d_o, dq, dk, dv})) {
       EMI_REQUIRE(stride_h == head_dim && stride_s == heads * head_dim && stride_b == seq * stride_s,
                   "emi_attn_bwd_rope: this shape needs contiguous [batch, seq, heads, head_dim] operands");
+    }
+    if (!mfma_ok(a, dtype, {q, k, v, o, d_o, dq, dk, dv}) &&
+        !(dtype == EMI_F32 && attn_f32_mfma_ok(seq, head_dim, stride_b, stride_h, stride_s, {q, k, v, o, d_o, dq, dk, dv}))) {
       int rc = attn_bwd_impl(stream, q, k, v, o, lse, d_o, dq, dk, dv, workspace, workspace_bytes, batch, heads, seq, head_dim,
                              stride_b, stride_h, stride_s, scale, causal, dtype, nullptr);
       if (rc == EMI_OK) rc = emi_rope(stream, dq, unrope, dq, batch, seq, heads, head_dim, 1, dtype);
@@ -1749,7 +1754,7 @@ static int attn_bwd_impl(emi_stream_t stream, const void* q, const void* k, cons
   }
   if (dtype == EMI_F32) {
     const int rc = launch_attn_bwd_f32_mfma(st, q, k, v, o, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, stride_b,
-                                            stride_h, stride_s, scale, causal);
+                                            stride_h, stride_s, scale, causal, unrope);
     if (rc >= 0) return rc;
   }
   if (dtype == EMI_BF16)

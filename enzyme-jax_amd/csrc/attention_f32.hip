@@ -3,8 +3,8 @@
 // for head_dim a multiple of 16 up to 128 and rows that start on 16-byte boundaries.  Replaces the per-head
 // loop of test/llama.py:178-206 with the softmax of :13-18 for the fp32 configurations (stories15M: 6 heads x 48).
 //
-// A block of four wavefronts owns 16 queries (forward, dQ; the tangent 16 or 32) or 16 keys (dK/dV). The 16-row tiles of the other sequence axis
-// are dealt to the wavefronts in turn, each accumulates over its own tiles, and the four partial results are added
+// A block of four (or eight) wavefronts owns 16 queries (forward, dQ; the tangent 16 or 32) or 16 keys (dK/dV). The 16-row tiles of the other sequence axis
+// are dealt to the wavefronts in turn, each accumulates over its own tiles, and the partial results are added
 // through the LDS at the end (the forward pass scales them to a common maximum first); that is the only barrier. A masked
 // score has the weight 0 and its row is multiplied by it, so a NaN or an infinity in a row of v also reaches earlier queries
 // of the same 16-row tile. Operands come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
@@ -40,7 +40,8 @@ struct AttnShapeF32 {
 };
 
 constexpr float kMasked = -1.0e30f;
-constexpr int kWaves = 4;      // per block; merge_store deals the accumulator's four registers to them
+// Wavefronts a block (W): 4, or 8 where few blocks have long rows: eight_forward(), eight_adjoint().
+// merge_store deals the accumulator's four registers to the first four.
 
 __device__ __forceinline__ f32q_t mfma_f32(float a, float b, f32q_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -95,25 +96,48 @@ __device__ __forceinline__ void mma_cols(const float (&x)[4][NT], const f32q_t w
     for (int n = 0; n < NT; n++) acc[n] = mfma_f32(x[t][n], w[t], acc[n]);
 }
 
-// Adds the four wavefronts' accumulators and stores the sum: wavefront w takes register w of every lane, that is NT
-// consecutive elements of each of the 16 rows.  `mul[i]` scales wavefront i's share.  The LDS is free afterwards.
-template <int NT>
+// Adds the W wavefronts' accumulators and stores the sum: wavefront w < 4 takes register w of every lane, that is NT
+// consecutive elements of each of the 16 rows.  `mul[i]` scales wavefront i's share.  angles: null, or the row's (cos, sin) pairs,
+// by which it is turned back (the cotangent of a vector that was rotated).  The LDS is free after the next barrier.
+template <int NT, int W>
 __device__ __forceinline__ void merge_store(float* __restrict__ row, bool write, int lane, int wave, const f32q_t (&acc)[NT],
-                                            const float (&mul)[kWaves], float (&buf)[kWaves][kWaves * NT][64]) {
+                                            const float (&mul)[W], float (&buf)[W][4 * NT][64], const float2* __restrict__ angles = nullptr) {
 #pragma unroll
   for (int r = 0; r < 4; r++)
 #pragma unroll
     for (int n = 0; n < NT; n++) buf[wave][r * NT + n][lane] = acc[n][r];
+  const int first = NT * (4 * (lane >> 4) + wave);                 // this lane's first column
+  float2 turn[NT];
+#pragma unroll
+  for (int n = 0; n < NT; n++) turn[n] = angles != nullptr && wave < 4 ? angles[(first + n) >> 1] : make_float2(1.f, 0.f);
   __syncthreads();
+  if (W > 4 && wave >= 4) return;
   float x[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) {
     x[n] = 0.f;
 #pragma unroll
-    for (int i = 0; i < kWaves; i++) x[n] += buf[i][wave * NT + n][lane] * mul[i];
+    for (int i = 0; i < W; i++) x[n] += buf[i][wave * NT + n][lane] * mul[i];
+  }
+  if (angles != nullptr) {
+    float y[NT];                                                   // the pairs' other elements: with an odd NT some are other lanes'
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+      const int e = (first + n) ^ 1, j = e / NT;
+      if (NT % 2 == 0) {
+        y[n] = x[n ^ 1];
+      } else {
+        y[n] = 0.f;
+#pragma unroll
+        for (int i = 0; i < W; i++) y[n] += buf[i][(j & 3) * NT + e - j * NT][(lane & 15) | ((j >> 2) << 4)] * mul[i];
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+      x[n] = ((first + n) & 1) == 0 ? rotated_even(turn[n].x, -turn[n].y, x[n], y[n]) : rotated_odd(turn[n].x, -turn[n].y, y[n], x[n]);
   }
   if (write) {
-    float* p = row + NT * (4 * (lane >> 4) + wave);
+    float* p = row + first;
 #pragma unroll
     for (int n = 0; n < NT; n++) p[n] = x[n];
   }
@@ -140,13 +164,13 @@ __device__ __forceinline__ float groups_sum(float x) {
 }
 
 // Forward: o = softmax(scale q k^T) v, lse = log-sum-exp of the scaled scores.
-template <int NT>
-__global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+template <int NT, int W>
+__global__ __launch_bounds__(64 * W) void attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                    const float* __restrict__ v, float* __restrict__ o,
                                                                    float* __restrict__ lse, AttnShapeF32 sh, float scale,
                                                                    int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
-  __shared__ float stat[2][kWaves][16];
+  __shared__ float buf[W][4 * NT][64];
+  __shared__ float stat[2][W][16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
   const int tiles = (sh.seq + 15) >> 4;
   const BlockRows own = block_rows(tiles);
@@ -164,19 +188,19 @@ __global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* 
   for (int n = 0; n < NT; n++) acc[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
   // U key tiles per step, all their operands requested before the first product (one wait for memory per step)
   constexpr int U = NT <= 4 ? 2 : 1;
-  for (int k0 = 16 * wave; k0 < nkeys; k0 += 16 * kWaves * U) {
+  for (int k0 = 16 * wave; k0 < nkeys; k0 += 16 * W * U) {
     f32q_t s[U];
     float kf[U][NT][4], vx[U][4][NT];
     float mx = kMasked;
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (k0 + 16 * kWaves * u < nkeys) load_rows<NT>(k + base, sh.ss, k0 + 16 * kWaves * u, last, lane, kf[u]);
+      if (k0 + 16 * W * u < nkeys) load_rows<NT>(k + base, sh.ss, k0 + 16 * W * u, last, lane, kf[u]);
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (k0 + 16 * kWaves * u < nkeys) load_cols<NT>(v + base, sh.ss, k0 + 16 * kWaves * u, last, lane, vx[u]);
+      if (k0 + 16 * W * u < nkeys) load_cols<NT>(v + base, sh.ss, k0 + 16 * W * u, last, lane, vx[u]);
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int kb = k0 + 16 * kWaves * u;
+      const int kb = k0 + 16 * W * u;
       if (kb < nkeys) s[u] = rows_dot<NT>(kf[u], qf);
       else s[u] = f32q_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -203,7 +227,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* 
     for (int n = 0; n < NT; n++) acc[n] *= alpha;
 #pragma unroll
     for (int u = 0; u < U; u++)
-      if (k0 + 16 * kWaves * u < nkeys) mma_cols<NT>(vx[u], s[u], acc);
+      if (k0 + 16 * W * u < nkeys) mma_cols<NT>(vx[u], s[u], acc);
     m = m_new;
   }
   lsum = groups_sum(lsum);
@@ -212,28 +236,28 @@ __global__ __launch_bounds__(64 * kWaves) void attn_fwd_f32_kernel(const float* 
     stat[1][wave][lane] = lsum;
   }
   __syncthreads();
-  float mul[kWaves], top = kMasked, sum = 0.f;
+  float mul[W], top = kMasked, sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < kWaves; i++) top = fmaxf(top, stat[0][i][lane & 15]);     // wavefront 0 has key 0: finite
+  for (int i = 0; i < W; i++) top = fmaxf(top, stat[0][i][lane & 15]);     // wavefront 0 has key 0: finite
 #pragma unroll
-  for (int i = 0; i < kWaves; i++) {
+  for (int i = 0; i < W; i++) {
     mul[i] = expf(stat[0][i][lane & 15] - top);                                 // 0 for a wavefront without a tile
     sum += stat[1][i][lane & 15] * mul[i];
   }
 #pragma unroll
-  for (int i = 0; i < kWaves; i++) mul[i] *= 1.f / sum;
-  merge_store<NT>(o + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, mul, buf);
+  for (int i = 0; i < W; i++) mul[i] *= 1.f / sum;
+  merge_store<NT, W>(o + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, mul, buf);
   if (wave == 0 && G == 0 && myq < sh.seq) lse[(int64_t)bh * sh.seq + myq] = top + logf(sum);
 }
 
 // dV = P^T dO, dK = scale dS^T Q: a block per 16 keys, walking the queries that see them.
 // DELTA: from the rows of o, where nothing has left delta.
-template <int NT, bool DELTA>
+template <int NT, int W, bool DELTA>
 __device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* __restrict__ q, const float* __restrict__ k,
                                              const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ d_o,
                                              const float* __restrict__ lse, const float* __restrict__ delta, float* __restrict__ dk,
                                              float* __restrict__ dv, AttnShapeF32 sh, float scale, int causal,
-                                             float (&buf)[kWaves][kWaves * NT][64]) {
+                                             const float2* __restrict__ unrope, float (&buf)[W][4 * NT][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
   const int key0 = own.tile * 16;                                  // the earliest keys see the most queries
   const int bh = own.bh;
@@ -248,7 +272,7 @@ __device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* _
   f32q_t acck[NT], accv[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) acck[n] = accv[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
-  for (int qb = (causal ? key0 : 0) + 16 * wave; qb < sh.seq; qb += 16 * kWaves) {
+  for (int qb = (causal ? key0 : 0) + 16 * wave; qb < sh.seq; qb += 16 * W) {
     float qf[NT][4], dof[NT][4], qx[4][NT], dox[4][NT], lq[4], dq_[4];
     load_rows<NT>(q + base, sh.ss, qb, last, lane, qf);
     load_rows<NT>(d_o + base, sh.ss, qb, last, lane, dof);
@@ -285,22 +309,25 @@ __device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* _
     mma_cols<NT>(dox, s, accv);
     mma_cols<NT>(qx, dp, acck);
   }
-  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
-  merge_store<NT>(dk + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, acck, one, buf);
+  float one[W];
+#pragma unroll
+  for (int i = 0; i < W; i++) one[i] = 1.f;
+  merge_store<NT, W>(dk + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, acck, one, buf,
+                     unrope != nullptr ? unrope + (int64_t)(mykey < last ? mykey : last) * (8 * NT) : nullptr);
   __syncthreads();
-  merge_store<NT>(dv + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, accv, one, buf);
+  merge_store<NT, W>(dv + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, accv, one, buf);
 }
 
-template <int NT>
-__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+template <int NT, int W>
+__global__ __launch_bounds__(64 * W) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                        const float* __restrict__ v,
                                                                        const float* __restrict__ d_o,
                                                                        const float* __restrict__ lse,
                                                                        const float* __restrict__ delta, float* __restrict__ dk,
                                                                        float* __restrict__ dv, AttnShapeF32 sh, float scale,
-                                                                       int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
-  bwd_dkv_rows<NT, false>(block_rows((sh.seq + 15) >> 4), q, k, v, nullptr, d_o, lse, delta, dk, dv, sh, scale, causal, buf);
+                                                                       int causal, const float2* __restrict__ unrope) {
+  __shared__ float buf[W][4 * NT][64];
+  bwd_dkv_rows<NT, W, false>(block_rows((sh.seq + 15) >> 4), q, k, v, nullptr, d_o, lse, delta, dk, dv, sh, scale, causal, unrope, buf);
 }
 
 // dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T, delta = rowsum(dO * O), which it also
@@ -310,21 +337,21 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dkv_f32_kernel(const flo
 // dQ stands in its kernel, dK/dV in a function of its own: the order of the loads that the compiler makes of either depends
 // on that.  us, dQ in a function | here: 24 heads x 1000 x 96 261 | 247, 8 x 3000 x 128 784 | 768; dK/dV in its kernel | in a
 // function: 24 x 1000 x 32 105 | 98, 64 x 1024 x 48 294 | 284.
-template <int NT, bool BOTH>
-__global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+template <int NT, int W, bool BOTH>
+__global__ __launch_bounds__(64 * W) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                       const float* __restrict__ v, const float* __restrict__ o,
                                                                       const float* __restrict__ d_o,
                                                                       const float* __restrict__ lse, float* __restrict__ delta,
                                                                       float* __restrict__ dq, float* __restrict__ dk,
                                                                       float* __restrict__ dv, AttnShapeF32 sh, float scale,
-                                                                      int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
+                                                                      int causal, const float2* __restrict__ unrope) {
+  __shared__ float buf[W][4 * NT][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
   const int tiles = (sh.seq + 15) >> 4;
   const BlockRows own = block_rows(tiles);
   if constexpr (BOTH) {
     if (blockIdx.z == 0) {
-      bwd_dkv_rows<NT, true>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, buf);
+      bwd_dkv_rows<NT, W, true>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, unrope, buf);
       return;
     }
   }
@@ -353,7 +380,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const floa
   f32q_t acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; n++) acc[n] = f32q_t{0.f, 0.f, 0.f, 0.f};
-  for (int kb = 16 * wave; kb < nkeys; kb += 16 * kWaves) {
+  for (int kb = 16 * wave; kb < nkeys; kb += 16 * W) {
     float kf[NT][4], vf[NT][4], kx[4][NT];
     load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
     load_rows<NT>(v + base, sh.ss, kb, last, lane, vf);
@@ -369,8 +396,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const floa
     }
     mma_cols<NT>(kx, s, acc);
   }
-  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
-  merge_store<NT>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf);
+  float one[W];
+#pragma unroll
+  for (int i = 0; i < W; i++) one[i] = 1.f;
+  merge_store<NT, W>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf,
+                     unrope != nullptr ? unrope + (int64_t)qc * (8 * NT) : nullptr);
 }
 
 // Tangent: with p = exp(scale q k^T - lse) and tS = scale (tq k^T + q tk^T)
@@ -381,13 +411,13 @@ __global__ __launch_bounds__(64 * kWaves) void attn_bwd_dq_f32_kernel(const floa
 // 1122 x 64 3918 | 103, 32 x 1716 x 64 16918 | 405 (89 TFLOP/s), 96 x 1817 x 128 117047 | 2662 (91), 6 x 256 x 48 143 | 10;
 // error against float64 4.7e-7 | 4.2e-7 at 32 x 512 x 128.
 template <int NT, int QS>
-__global__ __launch_bounds__(64 * kWaves) void attn_jvp_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
+__global__ __launch_bounds__(64 * 4) void attn_jvp_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                    const float* __restrict__ v, const float* __restrict__ lse,
                                                                    const float* __restrict__ tq, const float* __restrict__ tk,
                                                                    const float* __restrict__ tv, float* __restrict__ to,
                                                                    AttnShapeF32 sh, float scale, int causal) {
-  __shared__ float buf[kWaves][kWaves * NT][64];
-  __shared__ float stat[QS][kWaves][16];
+  __shared__ float buf[4][4 * NT][64];
+  __shared__ float stat[QS][4][16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
   const int tiles = (sh.seq + 16 * QS - 1) / (16 * QS);
   const BlockRows own = block_rows(tiles);
@@ -408,7 +438,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_jvp_f32_kernel(const float* 
     for (int n = 0; n < NT; n++) acct[s][n] = acco[s][n] = f32q_t{0.f, 0.f, 0.f, 0.f};
   }
   const int nkeys = causal ? (q0 + 16 * QS < sh.seq ? q0 + 16 * QS : sh.seq) : sh.seq;
-  for (int kb = 16 * wave; kb < nkeys; kb += 16 * kWaves) {
+  for (int kb = 16 * wave; kb < nkeys; kb += 16 * 4) {
     float kf[NT][4], tkf[NT][4], vx[4][NT], tvx[4][NT];
     load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
     if (tk != nullptr) load_rows<NT>(tk + base, sh.ss, kb, last, lane, tkf);
@@ -440,17 +470,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_jvp_f32_kernel(const float* 
     if (G == 0) stat[s][wave][lane] = mu[s];
   }
   __syncthreads();
-  const float one[kWaves] = {1.f, 1.f, 1.f, 1.f};
+  const float one[4] = {1.f, 1.f, 1.f, 1.f};
 #pragma unroll
   for (int s = 0; s < QS; s++) {
     float m = 0.f;
 #pragma unroll
-    for (int i = 0; i < kWaves; i++) m += stat[s][i][lane & 15];
+    for (int i = 0; i < 4; i++) m += stat[s][i][lane & 15];
 #pragma unroll
     for (int n = 0; n < NT; n++) acct[s][n] -= m * acco[s][n];
     const int myq = q0 + 16 * s + (lane & 15);
     if (s > 0) __syncthreads();                                    // buf has been read
-    merge_store<NT>(to + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acct[s], one, buf);
+    merge_store<NT, 4>(to + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acct[s], one, buf);
   }
 }
 
@@ -460,6 +490,23 @@ static bool f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t
   for (const void* p : ptrs)
     if (reinterpret_cast<uintptr_t>(p) & 15) return false;
   return true;
+}
+
+bool attn_f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
+  return f32_mfma_ok(seq, d, sb, shh, ss, ptrs);
+}
+
+// Eight wavefronts a block where the blocks have a CU each and the longest row, which sets the time, is of tiles enough; heads of
+// 64 and rows without a mask fill the matrix cores sooner.  us, four | eight, heads x length x head size (blocks): forward, causal
+// 6 x 256 x 48 (96) 6.5 | 6.3, 6 x 512 x 48 (192) 10.0 | 8.9, 8 x 400 x 64 (200) 10.1 | 9.9, 6 x 128 x 48 (48) 4.7 | 5.2, 24 x 200 x 48 (312)
+// 7.0 | 8.1; adjoint (one launch), causal 6 x 256 x 48 9.8 | 8.8, 12 x 200 x 48 (156) 11.2 | 9.3, 6 x 512 x 48 19.6 | 14.8, 8 x 512 x 64 (256)
+// 29.5 | 25.1, 24 x 128 x 48 (192) 7.9 | 8.4, 12 x 256 x 64 (192) 16.4 | 18.2; all keys 8 x 256 x 48 (128) 10.2 | 9.2, 8 x 512 x 48 22.1 | 23.3.
+static bool eight_forward(int64_t blocks, int64_t seq, int64_t head_dim, int causal) {
+  return head_dim <= 64 && blocks <= 256 && seq >= (head_dim <= 48 && causal ? 192 : 384);
+}
+static bool eight_adjoint(int64_t blocks, int64_t seq, int64_t head_dim, int causal) {
+  if (head_dim > 48) return head_dim <= 64 && causal && seq >= 384 && blocks <= 256;
+  return seq >= 96 && (causal ? blocks <= 160 || (seq >= 256 && blocks <= 256) : blocks <= 128);
 }
 
 #define EMI_ATTN_F32_DISPATCH(NTV, CALL)      \
@@ -482,9 +529,13 @@ int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o})) return -1;
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
-  EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL(attn_fwd_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q, (const float*)k,
-                                           (const float*)v, (float*)o, lse, shp, scale, causal));
+#define EMI_FWD(W)                                                                                                                   \
+  EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),                                                                                        \
+                        hipLaunchKernelGGL((attn_fwd_f32_kernel<(W == 8 && NT > 4 ? 4 : NT), W>), grid, dim3(64 * W), 0, st, (const float*)q, \
+                                           (const float*)k, (const float*)v, (float*)o, lse, shp, scale, causal))
+  if (eight_forward((int64_t)grid.x * grid.y, seq, head_dim, causal)) EMI_FWD(8)
+  else EMI_FWD(4)
+#undef EMI_FWD
   EMI_CHECK_LAUNCH("emi_attn_fwd(fp32 mfma)");
   return EMI_OK;
 }
@@ -492,8 +543,10 @@ int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
 // dQ, dK, dV on the fp32 matrix-core path (delta: scratch for rowsum(dO * O)); -1 when the operands do not qualify.
 int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o,
                              const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
-                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal) {
+                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal,
+                             const float* unrope) {
   if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
+  const float2* angles = reinterpret_cast<const float2*>(unrope);
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
   // One launch while two would each leave much of the chip idle, up to `most` blocks.  Of causal rows the late ones are the
@@ -512,22 +565,26 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   else if (head_dim <= 64) most = middling ? 1024 : 512;
   else most = head_dim <= 112 || middling ? 512 : 192;
   if ((int64_t)grid.x * grid.y <= most) {
-    EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                          hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, true>), dim3(grid.x, grid.y, 2), dim3(64 * kWaves), 0, st,
-                                             (const float*)q, (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse,
-                                             nullptr, (float*)dq, (float*)dk, (float*)dv, shp, scale, causal));
+#define EMI_BOTH(W)                                                                                                                      \
+  EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),                                                                                            \
+                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<(W == 8 && NT > 4 ? 4 : NT), W, true>), dim3(grid.x, grid.y, 2), dim3(64 * W), 0, \
+                                           st, (const float*)q, (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, \
+                                           nullptr, (float*)dq, (float*)dk, (float*)dv, shp, scale, causal, angles))
+    if (eight_adjoint((int64_t)grid.x * grid.y, seq, head_dim, causal)) EMI_BOTH(8)
+    else EMI_BOTH(4)
+#undef EMI_BOTH
     EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma)");
     return EMI_OK;
   }
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, false>), grid, dim3(64 * kWaves), 0, st, (const float*)q,
+                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, 4, false>), grid, dim3(256), 0, st, (const float*)q,
                                            (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, delta,
-                                           (float*)dq, nullptr, nullptr, shp, scale, causal));
+                                           (float*)dq, nullptr, nullptr, shp, scale, causal, angles));
   EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dq)");
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL(attn_bwd_dkv_f32_kernel<NT>, grid, dim3(64 * kWaves), 0, st, (const float*)q,
+                        hipLaunchKernelGGL((attn_bwd_dkv_f32_kernel<NT, 4>), grid, dim3(256), 0, st, (const float*)q,
                                            (const float*)k, (const float*)v, (const float*)d_o, lse, delta, (float*)dk,
-                                           (float*)dv, shp, scale, causal));
+                                           (float*)dv, shp, scale, causal, angles));
   EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dkv)");
   return EMI_OK;
 }
@@ -542,7 +599,7 @@ int launch_attn_jvp_f32_mfma(hipStream_t st, const void* q, const void* k, const
   do {                                                                                                                          \
     const dim3 grid((unsigned)((seq + 16 * QS - 1) / (16 * QS)), (unsigned)(batch * heads));                                    \
     EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),                                                                                 \
-                          hipLaunchKernelGGL((attn_jvp_f32_kernel<NT, QS>), grid, dim3(64 * kWaves), 0, st, (const float*)q,    \
+                          hipLaunchKernelGGL((attn_jvp_f32_kernel<NT, QS>), grid, dim3(64 * 4), 0, st, (const float*)q,    \
                                              (const float*)k, (const float*)v, lse, (const float*)tq, (const float*)tk,         \
                                              (const float*)tv, (float*)to, shp, scale, causal));                                \
   } while (0)

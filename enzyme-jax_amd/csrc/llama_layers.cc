@@ -36,6 +36,8 @@ struct Dims {
   bool tiles(int64_t n) const { return T() % 256 == 0 && n % 256 == 0 && (T() / 256) * (n / 256) >= 192; }
   // the kernels with RoPE in their epilogues (ops.attention_block)
   bool rope_attention() const { return dtype == EMI_BF16 && (hd() == 64 || hd() == 128) && S >= 128; }
+  // the adjoints that turn dq and dk back as they store them
+  bool unrope_attention() const { return rope_attention() || (dtype == EMI_F32 && hd() % 16 == 0 && hd() <= 128); }
   bool rope_projection() const { return rope_attention() && tiles(D); }
   bool swiglu_epilogue() const { return dtype == EMI_BF16 && T() >= 256; }
 };
@@ -485,7 +487,7 @@ extern "C" int emi_llama_layers_bwd(emi_stream_t stream, const void* const* weig
     }
     EMI_TRY(norm_adjoint(stream, norms, s.x1, w[kFfn], r.dxb, planes, dy, c.dx1, g[kFfn], r, d));
     EMI_TRY(emi_gemm_ws(stream, c.dx1, b[kO], nullptr, r.dxb, r.ws, r.ws_bytes, T, D, D, D, D, D, D, 0, tb, dtype));
-    if (d.rope_attention()) {
+    if (d.unrope_attention()) {
       EMI_TRY(emi_attn_bwd_rope(stream, s.q, s.k, s.v, s.att, s.lse, r.dxb, c.dq, c.dk, c.dv, rope_table, r.ws, r.ws_bytes, d.B, d.heads, d.S, hd,
                                 d.S * D, hd, D, d.scale, 1, dtype));
     } else {

@@ -93,3 +93,33 @@ def test_f32_attention_tangent_of_other_layouts():
             args.append(moved)
         _, to = jvp(lambda a, b, c: ops.attention(a, b, c, h), tuple(args[:3]), tuple(args[3:]))
         assert float(np.max(np.abs(heads(host(to)) - want))) <= bound, shift
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,h,S,d", [(1, 3, 96, 48), (1, 5, 257, 32), (1, 2, 385, 64), (2, 3, 390, 16), (1, 7, 520, 48), (1, 40, 96, 48)])
+def test_f32_attention_eight_wavefronts(B, h, S, d, causal):
+    """Few blocks of long rows have eight wavefronts, some of them without a tile of a short row; one launch and two of the
+    adjoint beside each other.  Bounds as above."""
+    test_f32_attention_tiles(B, h, S, d, causal)
+
+
+@pytest.mark.parametrize("h,S,d", [(3, 40, 48), (6, 256, 48), (5, 33, 80), (2, 70, 32), (40, 300, 64), (3, 50, 40)])
+def test_f32_attention_adjoint_turns_its_operands_back(h, S, d):
+    """The inverse rotation where dq and dk leave, with an odd and an even number of 16-column tiles a head (a pair's elements in
+    two lanes or in one), against the adjoint and a pass over each: the same bits; head_dim 40 takes the passes."""
+    from enzyme_ad.jax import ops, _native
+    rng = np.random.default_rng(S + d)
+    q, k, v, do = (dev(rng.standard_normal((2, S, h * d)), "f32")[0] for _ in range(4))
+    table = ops.rope_table(S, d, device=q.device)
+    o, lse, shape = ops.attention_raw(q, k, v, h, d ** -0.5, True, "bshd")
+    B, S_, d_, sb, sh, ss = shape
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(lib.emi_attn_bwd_workspace_bytes(B, h, S, d), dtype=torch.uint8, device=q.device)
+    one, two = ([torch.empty_like(q) for _ in range(3)] for _ in range(2))
+    head = [t.data_ptr() for t in (q, k, v, o, lse, do)]
+    tail = [ws.data_ptr(), ws.numel(), B, h, S, d, sb, sh, ss, d ** -0.5, 1, 11]
+    _native.check(lib.emi_attn_bwd_rope(st, *head, *(t.data_ptr() for t in one), table.data_ptr(), *tail))
+    _native.check(lib.emi_attn_bwd(st, *head, *(t.data_ptr() for t in two), *tail))
+    for t in two[:2]:
+        _native.check(lib.emi_rope(st, t.data_ptr(), table.data_ptr(), t.data_ptr(), B, S, h, d, 1, 11))
+    assert all(torch.equal(a, b) for a, b in zip(one, two))
