@@ -52,12 +52,19 @@ template <int N> __device__ __forceinline__ void add_planes(const float* p, int6
     }
 }
 
+// What the 256 MB memory-side cache keeps of an array for the kernel behind, which reads it from its end (rope_kernel).  us, every
+// row a stream, read from the start | this: norm and rotation of 16 x 2048 x 4096 fp32 (537 MB) 370 | 345, of 268 MB 191 | 161, of
+// 134 MB bf16 87 | 83; keeping 208 MB 354, 272 MB 366.
+constexpr int64_t kMemoryCache = (int64_t)240 << 20;
+
+// Rows from keep_from on are stored through the caches, so that the memory-side cache holds them for the kernel that reads y next;
+// the ones before, which would only push each other out, as a stream.
 // PLANES: x is the result of a product that was split over K, still in planes, and its residual; it is added up here as the
 // reduction of its own would (3 to 4 us a launch), stored to x_out and normalised.
 template <typename T, int TPR, int NCH, bool PLANES>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                           T* __restrict__ y, int64_t rows, int dim, float eps,
-                                                          const float* __restrict__ planes, int count, T* x_out) {
+                                                          const float* __restrict__ planes, int count, T* x_out, int64_t keep_from) {
   // NCH groups of 8 elements per thread, held as 16-byte pieces (8 bf16 or 4 floats): consecutive lanes cover
   // consecutive 16 bytes, the access shape the streaming loads and stores want.
   constexpr int RPB = 256 / TPR, N = Chunk<T>::N, NC = NCH * 8 / N;
@@ -68,12 +75,13 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ 
   const bool active = row < rows;
   const int nchunk = dim / N;
   const T* xr = x + row * dim;
-  float v[NC][N];
+  float v[NC][N], g[NC][N];                                   // gamma beside the row: behind the row's sum it would be waited for
   float ss = 0.f, dummy = 0.f;
 #pragma unroll
   for (int j = 0; j < NC; j++) {
     const int c = tir + j * TPR;
     if (active && c < nchunk) {
+      ChunkCached<T>::load(gamma + c * N, g[j]);
       if constexpr (PLANES) {
         float r[N];
         add_planes<N>(planes + row * dim + c * N, rows * (int64_t)dim, count, v[j]);
@@ -97,11 +105,11 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ 
   for (int j = 0; j < NC; j++) {
     const int c = tir + j * TPR;
     if (active && c < nchunk) {
-      float g[N], o[N];
-      ChunkCached<T>::load(gamma + c * N, g);
+      float o[N];
 #pragma unroll
-      for (int e = 0; e < N; e++) o[e] = g[e] * v[j][e] * r;
-      Chunk<T>::store(yr + c * N, o);
+      for (int e = 0; e < N; e++) o[e] = g[j][e] * v[j][e] * r;
+      if (row >= keep_from) ChunkCached<T>::store(yr + c * N, o);
+      else Chunk<T>::store(yr + c * N, o);
     }
   }
 }
@@ -417,15 +425,16 @@ __global__ void rope_table_kernel(float2* __restrict__ table, int64_t seq, int h
 }
 
 // One block row of the grid per row of x (a sequence position of one sequence), a thread per 16-byte chunk (8 bf16 /
-// 4 fp32 elements): the indices are 32-bit and the position is the block's.  (Two or more rows per thread, with
+// 4 fp32 elements): the indices are 32-bit and the position is the block's.  Last rows first: they are what the kernel that made x
+// has left in the memory-side cache; and where x and y are more than that holds, y is a stream that leaves x there.  (Two or more rows per thread, with
 // their loads in flight together, measured slower: 75 -> 73 -> 64 % of peak for 2, 4, 8 rows in bf16.)
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kernel(const T* x, const float2* __restrict__ table, T* y, int seq,
-                                                   int row_elems, int head_dim, int inverse) {
+                                                   int row_elems, int head_dim, int inverse, int stream) {
   constexpr int V = ChunkCached<T>::N, NP = V / 2;
   const int col = (blockIdx.y * blockDim.x + threadIdx.x) * V;
   if (col >= row_elems) return;
-  const int row = blockIdx.x, s = row % seq;
+  const int row = gridDim.x - 1 - blockIdx.x, s = row % seq;
   const float4* tp = reinterpret_cast<const float4*>(table + (int64_t)s * (head_dim >> 1) + ((col % head_dim) >> 1));
   float4 t[NP / 2];                                          // two (cos, sin) entries each
 #pragma unroll
@@ -440,7 +449,8 @@ __global__ __launch_bounds__(256) void rope_kernel(const T* x, const float2* __r
     o[2 * p] = rotated_even(cs, sp, v[2 * p], v[2 * p + 1]);
     o[2 * p + 1] = rotated_odd(cs, sp, v[2 * p], v[2 * p + 1]);
   }
-  ChunkCached<T>::store(y + (int64_t)row * row_elems + col, o);
+  if (stream) Chunk<T>::store(y + (int64_t)row * row_elems + col, o);
+  else ChunkCached<T>::store(y + (int64_t)row * row_elems + col, o);
 }
 
 template <typename T>
@@ -702,9 +712,10 @@ static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, 
     hipLaunchKernelGGL(rmsnorm_fwd_generic_kernel<T>, dim3((unsigned)rows), dim3(256), 0, st, xp, gp, yp, rows, dim, eps);
   } else {
     const unsigned g = blocks_for(rows, 256 / tpr);
+    const int64_t keep_from = rows - kMemoryCache / (dim * (int64_t)sizeof(T));
 #define EMI_RMS_FWD_P(TPR, NCH, PLANES)                                                                                                  \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, TPR, NCH, PLANES>), dim3(g), dim3(256), 0, st, xp, gp, yp, rows, (int)dim, eps, planes, count, \
-                     static_cast<T*>(x_out))
+                     static_cast<T*>(x_out), keep_from)
 #define EMI_RMS_FWD(TPR, NCH)                           \
   do {                                                  \
     if (count > 0) EMI_RMS_FWD_P(TPR, NCH, true);       \
@@ -963,7 +974,7 @@ static int rope_launch(hipStream_t st, const void* x, const float* table, void* 
     const int bs = chunks >= 256 ? 256 : (chunks + 63) / 64 * 64;            // short rows: no idle wavefronts
     const dim3 grid((unsigned)rows, (unsigned)((chunks + bs - 1) / bs));
     hipLaunchKernelGGL(rope_kernel<T>, grid, dim3(bs), 0, st, static_cast<const T*>(x), tp, static_cast<T*>(y), (int)seq,
-                       (int)row_elems, (int)head_dim, inverse);
+                       (int)row_elems, (int)head_dim, inverse, (int)(2 * n * (int64_t)sizeof(T) > kMemoryCache));
   } else {
     hipLaunchKernelGGL(rope_pair_kernel<T>, dim3(blocks_for(n / 2, 256)), dim3(256), 0, st, static_cast<const T*>(x), tp,
                        static_cast<T*>(y), n / 2, (int)seq, (int)(heads * head_dim), (int)head_dim, inverse);

@@ -583,3 +583,28 @@ def test_rope_in_epilogues(ops, B, S, nh, d, D_in, dt):
             "dwv": rdv.reshape(T, D).T @ x2r}
     for name, w in zip(("dx", "dwq", "dwk", "dwv"), f1(do)):
         check(w, want[name], dt, "attention_block " + name)
+
+
+@pytest.mark.parametrize("dt,S,D", [("f32", 61438, 1024), ("f32", 61444, 1024), ("bf16", 70000, 2048), ("f32", 30723, 1024)])
+def test_norm_and_rotation_of_arrays_around_the_size_of_the_memory_side_cache(dt, S, D):
+    """All rows of an array of 240 MB are stored through the caches, the first ones of a larger one as a stream, and the rotation
+    streams where it reads and writes more than that; rows of either kind against float64 (sums of D squares: D * 2^-24 of
+    the row's norm; a rotation: two roundings)."""
+    from enzyme_ad.jax import ops
+    td = torch.float32 if dt == "f32" else torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(S)
+    x = torch.randn((1, S, D), generator=g, device="cuda").to(td)
+    gamma = (torch.randn(D, generator=g, device="cuda") * 0.25 + 1).to(td)
+    n = ops.rmsnorm(x, gamma)
+    y = ops.rope(n, D // 128)
+    keep = (240 << 20) // (D * x.element_size())
+    rows = sorted({r for r in (0, 1, S - keep - 1, S - keep, S - keep + 1, S // 2, S - 2, S - 1) if 0 <= r < S})
+    xr = x[0, rows].double()
+    want = gamma.double() * xr / torch.sqrt((xr * xr).mean(-1, keepdim=True) + 1e-5)
+    unit = 2.0 ** -22 if dt == "f32" else 2.0 ** -8
+    assert bool(((n[0, rows].double() - want).abs() <= (unit + D * 2.0 ** -24 / 8) * want.abs()).all())
+    pairs, (c, s) = n[0, rows].double().reshape(len(rows), -1, 64, 2), ops.rope_table(S, 128, device=x.device)[rows].double().unbind(-1)
+    c, s = c[:, None], s[:, None]
+    turned = torch.stack([c * pairs[..., 0] - s * pairs[..., 1], s * pairs[..., 0] + c * pairs[..., 1]], -1).reshape(len(rows), D)
+    size = pairs.abs().sum(-1, keepdim=True).expand(pairs.shape).reshape(len(rows), D)
+    assert bool(((y[0, rows].double() - turned).abs() <= unit * size).all())
