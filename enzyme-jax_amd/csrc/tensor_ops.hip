@@ -541,6 +541,44 @@ int launch_copy(hipStream_t st, const void* in, void* out, const CopyPlan& p) {
   return EMI_OK;
 }
 
+// Several arrays, each of whole bytes, in one launch: a block has kCopyBlock bytes of one of them, all its loads in flight at
+// once.  A replayed graph's arguments are a dozen arrays of a few KB and two or three of tens of MB: a launch each is 2 to 3 us on
+// the GPU and 5 on the host (dim-288 training step, 15 arguments, 98 MB, replayed: 855 -> 808 us; dim-768 model of 64 tokens, bf16, 353 ->
+// 282).
+constexpr int kCopyArrays = 48, kCopyUnroll = 16, kCopyBlock = kBlock * 16 * kCopyUnroll;
+struct CopyMany {
+  const uint8_t* src[kCopyArrays];
+  uint8_t* dst[kCopyArrays];
+  int64_t bytes[kCopyArrays];
+  int first[kCopyArrays + 1];                              // the first block of each
+  int count;
+};
+__global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyMany m) {
+  int a = 0;
+  while (a + 1 < m.count && (int)blockIdx.x >= m.first[a + 1]) a++;
+  const int64_t at = (int64_t)((int)blockIdx.x - m.first[a]) * kCopyBlock, left = m.bytes[a] - at;
+  const uint8_t* src = m.src[a] + at;
+  uint8_t* dst = m.dst[a] + at;
+  if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) != 0) {
+    const int n = left < kCopyBlock ? (int)left : kCopyBlock;
+    for (int i = threadIdx.x; i < n; i += kBlock) dst[i] = src[i];
+    return;
+  }
+  const int pieces = left < kCopyBlock ? (int)(left >> 4) : kCopyBlock / 16;
+  uint4 v[kCopyUnroll];
+#pragma unroll
+  for (int u = 0; u < kCopyUnroll; u++) {
+    const int c = u * kBlock + threadIdx.x;
+    v[u] = c < pieces ? stream_load(reinterpret_cast<const uint4*>(src) + c) : make_uint4(0, 0, 0, 0);
+  }
+#pragma unroll
+  for (int u = 0; u < kCopyUnroll; u++) {
+    const int c = u * kBlock + threadIdx.x;
+    if (c < pieces) *(reinterpret_cast<uint4*>(dst) + c) = v[u];
+  }
+  if (left < kCopyBlock && (int)threadIdx.x < (int)(left & 15)) dst[pieces * 16 + threadIdx.x] = src[pieces * 16 + threadIdx.x];
+}
+
 // ---------------------------------------------------------------------------
 // reductions over the middle index of x[outer, red, inner] (sum or max, fp32 accumulate)
 // ---------------------------------------------------------------------------
@@ -1019,4 +1057,35 @@ extern "C" int emi_select(emi_stream_t stream, const void* mask, const void* a, 
 #undef EMI_SEL_LAUNCH
   EMI_CHECK_LAUNCH("emi_select");
   return EMI_OK;
+}
+
+extern "C" int emi_copy_many(emi_stream_t stream, int count, const void* const* src, void* const* dst, const int64_t* bytes) {
+  EMI_REQUIRE(count >= 0 && (count == 0 || (src && dst && bytes)), "emi_copy_many: null table");
+  for (int i = 0; i < count; i++)
+    EMI_REQUIRE(bytes[i] >= 0 && bytes[i] < (int64_t)1 << 44 && (bytes[i] == 0 || (src[i] && dst[i])), "emi_copy_many: array %d: null or of %lld bytes", i,
+                (long long)bytes[i]);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  CopyMany m{};
+  int64_t blocks = 0;
+  auto flush = [&]() -> int {
+    if (m.count == 0) return EMI_OK;
+    m.first[m.count] = (int)blocks;
+    hipLaunchKernelGGL(copy_many_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, m);
+    EMI_CHECK_LAUNCH("emi_copy_many");
+    m.count = 0;
+    blocks = 0;
+    return EMI_OK;
+  };
+  for (int i = 0; i < count; i++) {
+    if (bytes[i] == 0 || src[i] == dst[i]) continue;
+    const int64_t mine = (bytes[i] + kCopyBlock - 1) / kCopyBlock;
+    if (m.count == kCopyArrays || blocks + mine > 0x7fffffff)
+      if (const int rc = flush()) return rc;
+    m.src[m.count] = static_cast<const uint8_t*>(src[i]);
+    m.dst[m.count] = static_cast<uint8_t*>(dst[i]);
+    m.bytes[m.count] = bytes[i];
+    m.first[m.count++] = (int)blocks;
+    blocks += mine;
+  }
+  return flush();
 }

@@ -38,6 +38,7 @@ SIGNATURES = {
     "emi_compare": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_int]),
     "emi_select": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int]),
     "emi_convert": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int]),
+    "emi_copy_many": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), ctypes.POINTER(c_void_p), ctypes.POINTER(c_i64)]),
     "emi_strided_copy": (c_int, [c_void_p, c_void_p, c_void_p, c_int, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64),
                                  c_i64, ctypes.POINTER(c_i64), c_i64, c_int]),
     "emi_reduce_workspace_bytes": (c_size_t, [c_i64, c_i64, c_i64, c_int]),

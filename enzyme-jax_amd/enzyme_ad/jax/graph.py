@@ -13,8 +13,12 @@ The result tensors belong to the graph and are overwritten by the next replay; c
 outlive it.  Argument shapes and dtypes are fixed at capture.  Nothing here records a memset
 node: buffers are cleared by fill kernels.
 """
+import bisect
+import ctypes
+
 import torch
 
+from . import _native as N
 from .primitives import tree_flatten, tree_unflatten
 
 
@@ -25,6 +29,8 @@ class Captured:
             if isinstance(l, torch.Tensor) and not l.is_cuda:
                 raise RuntimeError("argument is not in device memory: the HIP path has no CPU fallback")
         self._inputs = [l.clone() if isinstance(l, torch.Tensor) else l for l in leaves]
+        spans = sorted((t.data_ptr(), t.data_ptr() + max(t.untyped_storage().nbytes(), 1)) for t in self._inputs if isinstance(t, torch.Tensor))
+        self._starts, self._ends = [a for a, _ in spans], [b for _, b in spans]
         args = tree_unflatten(self._treedef, self._inputs)
         side = torch.cuda.Stream()                       # default priority
         side.wait_stream(torch.cuda.current_stream())
@@ -41,16 +47,39 @@ class Captured:
         leaves, treedef = tree_flatten(tuple(args))
         if len(leaves) != len(self._inputs):
             raise ValueError("captured with %d argument leaves, called with %d" % (len(self._inputs), len(leaves)))
+        pairs = []
         for s, a in zip(self._inputs, leaves):
             if isinstance(s, torch.Tensor):
                 if not isinstance(a, torch.Tensor) or a.shape != s.shape or a.dtype != s.dtype:
                     raise ValueError("argument does not match the captured %s/%s" % (tuple(s.shape), s.dtype))
-                s.copy_(a)                               # device-to-device copy kernel on the current stream
+                pairs.append((s, a))
             elif a != s:
                 raise ValueError("non-tensor argument %r differs from the captured %r" % (a, s))
+        self._copy_in(pairs)
         self.graph.replay()
         self.replays += 1
         return self._outputs
+
+    def _copy_in(self, pairs):
+        """New argument values into the graph's buffers, on the current stream: whole arrays on its device by one launch.  One by
+        one, in order, where an argument is itself one of those buffers (an output that is an argument passed through)."""
+        here = torch.cuda.current_device()
+        plain = [type(a) is torch.Tensor and a.device.type == "cuda" and a.device.index == here == s.device.index and a.is_contiguous()
+                 and s.is_contiguous() and not (a.is_conj() or a.is_neg()) for s, a in pairs]
+        for _, a in pairs:
+            p = a.data_ptr() if a.device.type == "cuda" and a.layout == torch.strided else 0
+            at = bisect.bisect_right(self._starts, p) - 1
+            if at >= 0 and p < self._ends[at]:
+                plain = [False] * len(pairs)
+                break
+        for (s, a), whole in zip(pairs, plain):
+            if not whole:
+                s.copy_(a)
+        pairs = [pair for pair, whole in zip(pairs, plain) if whole]
+        if pairs:
+            table, sizes = ctypes.c_void_p * len(pairs), ctypes.c_int64 * len(pairs)
+            N.check(N.lib().emi_copy_many(torch._C._cuda_getCurrentRawStream(here), len(pairs), table(*[a.data_ptr() for _, a in pairs]),
+                                          table(*[s.data_ptr() for s, _ in pairs]), sizes(*[s.numel() * s.element_size() for s, _ in pairs])))
 
 
 def capture(fn, *example_args):

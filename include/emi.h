@@ -389,6 +389,9 @@ int emi_select(emi_stream_t stream, const void* mask, const void* a, const void*
 int emi_strided_copy(emi_stream_t stream, const void* in, void* out, int rank, const int64_t* dims,
                      const int64_t* in_strides, int64_t in_offset, const int64_t* out_strides,
                      int64_t out_offset, int elem_bytes);
+/* dst[i] = src[i], bytes[i] bytes, for i < count: arrays on the device, the tables HOST arrays.  No
+ * destination overlaps another array of the call, but may be its own source. */
+int emi_copy_many(emi_stream_t stream, int count, const void* const* src, void* const* dst, const int64_t* bytes);
 /* y[o, i] = sum or max over r of x[o, r, i] (op = EMI_OP_ADD or EMI_OP_MAX), fp32
  * accumulation (stablehlo.reduce with an add / maximum body; Reduce rule
  * StableHLOAutoDiffOpInterfaceImpl.cpp:1833-1916).  x: [outer, red, inner] contiguous.

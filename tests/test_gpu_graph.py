@@ -78,3 +78,45 @@ def test_captured_text_step_replays_match_eager():
         torch.cuda.synchronize()
         for a, b in zip(got, eager):
             assert torch.equal(a, b)
+
+
+def test_copy_many():
+    """Arrays of no bytes, of fewer than a piece, off 16-byte boundaries on either side, of several blocks and of one block exactly,
+    more arrays than one launch takes; nothing beyond an array is written."""
+    from enzyme_ad.jax import _native
+    import ctypes
+    sizes = [0, 1, 15, 16, 17, 4095, 65535, 65536, 65537, 200003] + [33] * 60
+    shifts = [(0, 0), (0, 1), (3, 0), (5, 5)]
+    src, dst, want = [], [], []
+    for i, n in enumerate(sizes):
+        a, b = shifts[i % 4]
+        room = torch.randint(0, 255, (n + 32,), dtype=torch.uint8, device="cuda")
+        out = torch.full((n + 32,), 7, dtype=torch.uint8, device="cuda")
+        ref = out.clone()
+        ref[b:b + n] = room[a:a + n]
+        src.append(room[a:])
+        dst.append((out, b))
+        want.append(ref)
+    table = ctypes.c_void_p * len(sizes)
+    _native.check(_native.lib().emi_copy_many(torch.cuda.current_stream().cuda_stream, len(sizes), table(*[s.data_ptr() for s in src]),
+                                              table(*[o.data_ptr() + b for o, b in dst]), (ctypes.c_int64 * len(sizes))(*sizes)))
+    assert all(torch.equal(o, w) for (o, _), w in zip(dst, want))
+    assert _native.lib().emi_copy_many(None, 1, table(), table(), (ctypes.c_int64 * 1)(4)) == 3          # null array
+    assert _native.lib().emi_copy_many(None, 1, table(*[16] * len(sizes)), table(*[16] * len(sizes)), (ctypes.c_int64 * 1)(-1)) == 3
+
+
+def test_captured_takes_arguments_of_any_layout_and_its_own_buffers():
+    """Strided, host and misaligned arguments; an output that is one of the graph's argument buffers, passed back as another one,
+    is read before it is written, in the order of the arguments."""
+    from enzyme_ad.jax import ops
+    from enzyme_ad.jax.graph import capture
+    a, b = (torch.randn(300, 8, device="cuda") for _ in range(2))
+    g = capture(lambda a, b: (ops.add(a, b), a, b), a, b)
+    strided = torch.randn(8, 300, device="cuda").t()
+    off = torch.randn(300 * 8 + 1, device="cuda")[1:].view(300, 8)
+    for x, y in ((strided, off), (torch.randn(300, 8), b), (a, a), (off, strided)):
+        assert torch.equal(g(x, y)[0], x.cuda() + y.cuda())
+    _, ga, gb = g(a, b)
+    assert torch.equal(g(b, ga)[0], b + b)                # b into the first buffer, which is then the second argument
+    _, ga, gb = g(a, b)
+    assert torch.equal(g(gb, b)[0], b + b) and torch.equal(g(ga, gb)[0], b + b)
