@@ -39,17 +39,25 @@ template <int TPR> __device__ __forceinline__ void row_reduce2(float& a, float& 
   }
 }
 
-// N consecutive elements of the sum of `count` fp32 planes, `plane` elements apart, in plane order.
+// N consecutive elements of the sum of `count` fp32 planes, `plane` elements apart, in plane order; four planes requested together
+// (past the last one, it again, unused).
 template <int N> __device__ __forceinline__ void add_planes(const float* p, int64_t plane, int count, float (&v)[N]) {
 #pragma unroll
   for (int e = 0; e < N; e++) v[e] = 0.f;
-#pragma unroll 4
-  for (int z = 0; z < count; z++)
+  for (int z0 = 0; z0 < count; z0 += 4) {
+    float4 t[4][N / 4];
 #pragma unroll
-    for (int q = 0; q < N / 4; q++) {
-      const float4 t = *reinterpret_cast<const float4*>(p + z * plane + 4 * q);
-      v[4 * q] += t.x; v[4 * q + 1] += t.y; v[4 * q + 2] += t.z; v[4 * q + 3] += t.w;
-    }
+    for (int z = 0; z < 4; z++)
+#pragma unroll
+      for (int q = 0; q < N / 4; q++) t[z][q] = *reinterpret_cast<const float4*>(p + (z0 + z < count ? z0 + z : count - 1) * plane + 4 * q);
+#pragma unroll
+    for (int z = 0; z < 4; z++)
+      if (z0 + z < count)
+#pragma unroll
+        for (int q = 0; q < N / 4; q++) {
+          v[4 * q] += t[z][q].x; v[4 * q + 1] += t[z][q].y; v[4 * q + 2] += t[z][q].z; v[4 * q + 3] += t[z][q].w;
+        }
+  }
 }
 
 // What the 256 MB memory-side cache keeps of an array for the kernel behind, which reads it from its end (rope_kernel).  us, every
@@ -165,6 +173,9 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
   // reduction (shuffles, LDS, barrier) of the current one, which keeps twice the
   // bytes in flight per block.
   typename Chunk<T>::Raw xn[NR][NC], gn[NR][NC];      // kept in storage format to save registers
+  // few rows, whose time is latency: dx_add with the rest of the row; many: later, its registers cost more (rotated bf16 305 -> 322 us)
+  constexpr bool EARLY = MODE == kNormPlanes;
+  [[maybe_unused]] typename Chunk<T>::Raw an[NR][NC];
   [[maybe_unused]] float4 tn[NR][NC][N / 4];          // two (cos, sin) entries each
   auto load_step = [&](int64_t sg) {
 #pragma unroll
@@ -182,6 +193,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
             for (int q = 0; q < N / 4; q++) tn[u][j][q] = t[q];
           }
           xn[u][j] = Chunk<T>::load_raw(x + row * dim + c * N);
+          if (EARLY && dx_add != nullptr) an[u][j] = Chunk<T>::load_raw(dx_add + row * dim + c * N);
           if constexpr (MODE == kNormPlanes) {
             float v[N];
             add_planes<N>(reinterpret_cast<const float*>(dy) + row * dim + c * N, rows * (int64_t)dim, count, v);
@@ -195,6 +207,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
             for (int q = 0; q < N / 4; q++) tn[u][j][q] = make_float4(1.f, 0.f, 1.f, 0.f);
           xn[u][j] = typename Chunk<T>::Raw{};
           gn[u][j] = typename Chunk<T>::Raw{};
+          if constexpr (EARLY) an[u][j] = typename Chunk<T>::Raw{};
         }
       }
     }
@@ -203,6 +216,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
   int it = 0;
   for (int64_t sg = blockIdx.x; sg < nstep; sg += gridDim.x, ++it) {
     typename Chunk<T>::Raw xc[NR][NC], gc[NR][NC];
+    [[maybe_unused]] typename Chunk<T>::Raw ac[NR][NC];
     float red_v[2 * NR];
 #pragma unroll
     for (int u = 0; u < NR; u++) {
@@ -211,6 +225,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
       for (int j = 0; j < NC; j++) {
         xc[u][j] = xn[u][j];
         gc[u][j] = gn[u][j];
+        if constexpr (EARLY) ac[u][j] = an[u][j];
         if constexpr (ROPE) {
           float v[N], o[N];
           Chunk<T>::unpack(gc[u][j], v);
@@ -257,7 +272,8 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
           }
           if (dx_add != nullptr) {
             float a[N];
-            Chunk<T>::load(dx_add + row * dim + c * N, a);
+            if constexpr (EARLY) Chunk<T>::unpack(ac[u][j], a);
+            else Chunk<T>::load(dx_add + row * dim + c * N, a);
 #pragma unroll
             for (int e = 0; e < N; e++) o[e] += a[e];
           }
