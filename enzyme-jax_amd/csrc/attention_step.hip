@@ -722,19 +722,19 @@ int check_step(const char* name, int64_t batch, int64_t heads, int64_t seq_kv, i
 
 // Launches the forward kernel (sh.kpb keys per block) and the combine.  A head whose keys are in one block has nothing to
 // combine: its block stores the result itself (o is then given to the kernel), in pieces of 16 bytes where it reads so;
-// an o that those do not fit goes through the combine, which stores single elements.
+// an o that those do not fit goes through the combine, which stores single elements.  A null o: the shares stay in `part`.
 int launch_step_fwd(hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, float* part, const StepShape& sh,
                     int bh, bool vec, float scale, int dtype) {
   const int ne = dtype == EMI_BF16 ? 8 : 4;
   const int nsplit = (sh.seq_kv + sh.kpb - 1) / sh.kpb;
-  const bool direct = nsplit == 1 && (!vec || al16(o));
+  const bool direct = nsplit == 1 && o != nullptr && (!vec || al16(o));
   const dim3 grid((unsigned)nsplit, (unsigned)bh);
 #define EMI_STEP_FWD(T, VEC, NCH)                                                                                       \
   do {                                                                                                                   \
     hipLaunchKernelGGL((attn_step_fwd_kernel<T, VEC, NCH>), grid, dim3(256), 0, st, (const T*)q, (const T*)k,            \
                        (const T*)v, part, direct ? (T*)o : nullptr, lse, sh, scale);                                     \
     EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
-    if (!direct)                                                                                                         \
+    if (!direct && o != nullptr)                                                                                         \
       hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)o, lse, sh, nsplit); \
   } while (0)
 #define EMI_STEP_FWD1(T)                                                                                                \
@@ -742,7 +742,7 @@ int launch_step_fwd(hipStream_t st, const void* q, const void* k, const void* v,
     hipLaunchKernelGGL(attn_step_fwd1_kernel<T>, grid, dim3(256), 0, st, (const T*)q, (const T*)k, (const T*)v, part,    \
                        direct ? (T*)o : nullptr, lse, sh, scale);                                                        \
     EMI_CHECK_LAUNCH("emi_attn_step_fwd");                                                                               \
-    if (!direct)                                                                                                         \
+    if (!direct && o != nullptr)                                                                                         \
       hipLaunchKernelGGL(attn_step_combine_kernel<T>, dim3((unsigned)bh), dim3(64), 0, st, part, (T*)o, lse, sh, nsplit); \
   } while (0)
 #define EMI_STEP_FWD_T(T)                                              \

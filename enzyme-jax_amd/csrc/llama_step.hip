@@ -6,7 +6,8 @@
 // matrix-vector products - RMSNorm, the rotation, SwiGLU, residuals, the new cache row - is done where its operand is
 // loaded or its result leaves, and the cache is not copied to append a row to it.
 //   forward, per layer:  norm + wq,wk,wv + rotation | attention over cache and own row (| combine) | wo + residual |
-//                        norm + w1,w3 + SwiGLU | w2 + residual;  with a short cache attention + wo + residual are one
+//                        norm + w1,w3 + SwiGLU | w2 + residual;  with a short cache attention + wo + residual are one, with a longer
+//                        one combine + wo + residual
 //   reverse, per layer:  norm' + w2^T dy and dw2 | SwiGLU' + w1^T dh1 + w3^T dh3 and dw1, dw3 | norm' + wo^T dy and dwo |
 //                        attention' | inverse rotation + wq^T dq + ... and dwq, dwk, dwv
 // The forward call leaves what the reverse one needs in `saved`.
@@ -65,7 +66,9 @@ template <typename T> struct NormGemv {
   const float2* table;   // MODE 0: (cos, sin) of pair i at i % table_pairs
   int N, K, table_pairs;
   float eps;
-  // MODE 2: the attention whose result the vector is
+  // MODE 2: the attention whose result the vector is;  MODE 3: its shares [heads][shares][head_dim + 2] (sum, maximum, weight)
+  const float* part;
+  int shares;
   const T *q, *k_cache, *v_cache, *k_own, *v_own;
   T* att;
   float* lse;
@@ -146,6 +149,64 @@ template <typename T> __device__ __forceinline__ void step_attention(const NormG
   }
 }
 
+// att of one query from its key blocks' shares, into the vector's LDS image: a 16-byte piece a thread, eight shares requested
+// together.  One such round is a latency of the L2 where a launch that adds the shares up is 3 to 5 us; and with the launch gone
+// a short cache is dealt to more blocks.  Where
+// StepDims::combines() says so.  Forward replayed, us, a launch | this (shares, rounds): 4 layers at dim 512 fp32, 255 keys 87.3 | 80.6 (4, 1), 700
+// 92.4 | 87.3 (11, 2), 2000 97.5 | 91.8 (16, 2); dim 1024 bf16, 2000 keys 115 | 108; 2 layers at dim 2048 fp32, 255 keys 149 | 116 (4, 2), at 4096 338 | 314
+// (4, 4).  More: dim 768 fp32, 2000 keys 116 | 122 (32, 4), dim 2048 bf16 99 | 105 (32, 4), dim 4096 bf16, 4095 keys 205 | 210 (16, 4).
+constexpr int kCombineShares = 8;
+template <typename T> __device__ __forceinline__ void step_combine(const NormGemv<T>& a, float* xs, int pieces, bool store) {
+  constexpr int V = ChunkCached<T>::N;
+  const int stride = a.head_dim + 2;
+  for (int c = threadIdx.x; c * V < a.K; c += 256) {
+    const int h = c * V / a.head_dim, e0 = c * V - h * a.head_dim;
+    const float* p0 = a.part + (int64_t)h * a.shares * stride;
+    float acc[V], mx = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < V; e++) acc[e] = 0.f;
+    for (int s0 = 0; s0 < a.shares; s0 += kCombineShares) {
+      float2 v[kCombineShares][V / 2], st[kCombineShares];
+#pragma unroll
+      for (int u = 0; u < kCombineShares; u++) {           // past the last: it again, of weight zero
+        const float* p = p0 + (s0 + u < a.shares ? s0 + u : a.shares - 1) * stride;
+        st[u] = *reinterpret_cast<const float2*>(p + a.head_dim);
+#pragma unroll
+        for (int e = 0; e < V / 2; e++) v[u][e] = *reinterpret_cast<const float2*>(p + e0 + 2 * e);
+      }
+      float nm = mx;
+#pragma unroll
+      for (int u = 0; u < kCombineShares; u++) nm = fmaxf(nm, st[u].x);
+      const float alpha = mx == -INFINITY ? 0.f : __expf(mx - nm);
+      sum *= alpha;
+#pragma unroll
+      for (int e = 0; e < V; e++) acc[e] *= alpha;
+      mx = nm;
+#pragma unroll
+      for (int u = 0; u < kCombineShares; u++) {
+        if (s0 + u >= a.shares) continue;
+        const float w = st[u].x == -INFINITY ? 0.f : __expf(st[u].x - mx);      // (times a NaN it stays one)
+        sum = fmaf(w, st[u].y, sum);
+#pragma unroll
+        for (int e = 0; e < V / 2; e++) {
+          acc[2 * e] = fmaf(w, v[u][e].x, acc[2 * e]);
+          acc[2 * e + 1] = fmaf(w, v[u][e].y, acc[2 * e + 1]);
+        }
+      }
+    }
+    const float inv = 1.0f / sum;
+#pragma unroll
+    for (int e = 0; e < V; e++) acc[e] = round_to<T>(acc[e] * inv);
+    if (store) {
+      ChunkCached<T>::store(a.att + c * V, acc);
+      if (e0 == 0) a.lse[h] = mx + __logf(sum);
+    }
+#pragma unroll
+    for (int g = 0; g < V / 4; g++)
+      *reinterpret_cast<f4*>(xs + (g * pieces + c) * 4) = f4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  }
+}
+
 template <typename T, int MODE, int UN, bool WHOLE>       // WHOLE: rows are whole batches
 __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
   using Raw = typename ChunkCached<T>::Raw;
@@ -156,7 +217,7 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
   const int nb = (a.K + BATCH - 1) / BATCH, pieces = nb * 64 * UN;     // pieces of the padded vector
   const int P = MODE == 0 ? 3 * a.N / 2 : MODE == 1 ? a.N : a.N / 2;
   auto rows = [&](int p, const T*& r0, const T*& r1) {
-    if constexpr (MODE == 2) {
+    if constexpr (MODE >= 2) {
       r0 = a.w[0] + (int64_t)(2 * p) * a.K;
       r1 = r0 + a.K;
     } else if constexpr (MODE == 0) {
@@ -186,8 +247,9 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
     issue(r0, r1, 0, c0, c1);
   }
   // the vector: the attention's or the norm's result, rounded to T as the operator-by-operator form stores it
-  if constexpr (MODE == 2) {
-    step_attention<T>(a, xs, pieces, blockIdx.x == 0);
+  if constexpr (MODE >= 2) {
+    if constexpr (MODE == 2) step_attention<T>(a, xs, pieces, blockIdx.x == 0);
+    else step_combine<T>(a, xs, pieces, blockIdx.x == 0);
     for (int c = a.K / V + threadIdx.x; c < pieces; c += 256)
 #pragma unroll
       for (int h = 0; h < V / 4; h++) *reinterpret_cast<f4*>(xs + (h * pieces + c) * 4) = f4{0.f, 0.f, 0.f, 0.f};
@@ -240,7 +302,7 @@ __global__ __launch_bounds__(256) void step_norm_gemv_kernel(NormGemv<T> a) {
     }
   };
   auto finish = [&](int p) {
-    if constexpr (MODE == 2) {                             // rows and residual in fp32, rounded once
+    if constexpr (MODE >= 2) {                             // rows and residual in fp32, rounded once
       const float v0 = wave_sum(s0), v1 = wave_sum(s1);
       s0 = s1 = 0.f;
       if (lane == 0) {
@@ -620,13 +682,22 @@ struct StepDims {
   float eps, scale;
   int dtype;
   int hd() const { return (int)(D / heads); }
-  // keys per block: a head in one block while that is a pass of its loads, otherwise enough blocks for the chip
+  // keys per block: enough blocks for the chip; as few as 64 where the product behind adds up their shares, otherwise a head in
+  // one block while that is a pass of its loads
   int kpb() const {
-    const int64_t keys = pos + 1;
+    const int64_t keys = pos + 1, want = (keys * heads / 512 + 63) / 64 * 64;
+    const int64_t fine = want < 64 ? 64 : want > 512 ? 512 : want;
+    if (combines((keys + fine - 1) / fine)) return (int)fine;
     if (keys <= 256) return 256;
-    const int64_t want = (keys * heads / 512 + 63) / 64 * 64;
     return (int)(want < 128 ? 128 : want > 512 ? 512 : want);
   }
+  // whether the product with wo adds up this many shares a head (step_combine): two rounds, or more of at most eight shares
+  bool combines(int64_t shares) const {
+    const int64_t pieces = D / (dtype == EMI_BF16 ? 8 : 4);
+    const int64_t rounds = (pieces + 255) / 256 * ((shares + kCombineShares - 1) / kCombineShares);
+    return rounds <= 2 || (shares <= kCombineShares && rounds <= 4);
+  }
+  bool combine_inside() const { return nsplit() > 1 && combines(nsplit()); }
   bool short_cache() const {                              // attention inside the product with wo: step_attention
     const int lanes = hd() / (dtype == EMI_BF16 ? 8 : 4);
     return lanes <= 16 && (heads + 15) / 16 * ((pos + kStepKeys) / kStepKeys) <= kStepRounds;
@@ -738,10 +809,21 @@ int step_fwd(hipStream_t st, const void* const* w, const void* x_, const void* k
       o.scale = d.scale;
       if (int rc = launch_norm_gemv<T, 2>(st, o)) return rc;
     } else {
-      if (int rc = launch_llama_step_attn_fwd(st, s.q, kc + l * d.pos * D, vc + l * d.pos * D, s.k, s.v, s.att, s.lse, tail.part,
+      const bool inside = d.combine_inside();
+      if (int rc = launch_llama_step_attn_fwd(st, s.q, kc + l * d.pos * D, vc + l * d.pos * D, s.k, s.v, inside ? nullptr : s.att, s.lse, tail.part,
                                               (int)d.heads, (int)d.pos, d.hd(), d.kpb(), d.scale, d.dtype))
         return rc;
-      if (int rc = launch_skinny(st, s.att, wo + l * D * D, x, s.x1, nullptr, 0, 1, D, D, D, D, D, D, 0, 1, d.dtype)) return rc;
+      if (inside) {
+        NormGemv<T> o{};
+        o.x = x;
+        o.w[0] = wo + l * D * D;
+        o.y[0] = s.x1;
+        o.N = (int)D, o.K = (int)D;
+        o.part = tail.part, o.shares = d.nsplit();
+        o.att = s.att, o.lse = s.lse;
+        o.heads = (int)d.heads, o.head_dim = d.hd();
+        if (int rc = launch_norm_gemv<T, 3>(st, o)) return rc;
+      } else if (int rc = launch_skinny(st, s.att, wo + l * D * D, x, s.x1, nullptr, 0, 1, D, D, D, D, D, D, 0, 1, d.dtype)) return rc;
     }
     NormGemv<T> f{};
     f.x = s.x1;
