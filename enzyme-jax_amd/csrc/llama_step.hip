@@ -682,12 +682,16 @@ struct StepDims {
   float eps, scale;
   int dtype;
   int hd() const { return (int)(D / heads); }
-  // keys per block: enough blocks for the chip; as few as 64 where the product behind adds up their shares, otherwise a head in
-  // one block while that is a pass of its loads
+  // keys per block: enough blocks for the chip; as few as 64 where the product behind adds up their shares and that costs less than
+  // one block's longer chain of keys, otherwise a head in one block while that is a pass of its loads.  From 224 keys, and with two
+  // pieces of a head a lane, whose chain is six times as long a key, from 96.  us, one block | 64 keys: dim 1024 fp32, 4 layers, 72
+  // keys 111 | 116, 151 keys 115 | 117, 256 keys 120 | 117; dim 2048 bf16, 72 keys 88 | 91; in two pieces, dim 4096 fp32, 2 layers,
+  // 72 keys 300 | 305, 121 keys 311 | 305
   int kpb() const {
     const int64_t keys = pos + 1, want = (keys * heads / 512 + 63) / 64 * 64;
     const int64_t fine = want < 64 ? 64 : want > 512 ? 512 : want;
-    if (combines((keys + fine - 1) / fine)) return (int)fine;
+    const int64_t from = hd() / (dtype == EMI_BF16 ? 8 : 4) > 16 ? 96 : 224;
+    if (keys >= from && combines((keys + fine - 1) / fine)) return (int)fine;
     if (keys <= 256) return 256;
     return (int)(want < 128 ? 128 : want > 512 ? 512 : want);
   }

@@ -78,6 +78,21 @@ def test_llama_step_adjoint_blocks(dt, dim, hidden, heads, pos):
         check(gw[k], rgw[k], dt, "d" + k, factor=2.0 if k == "wk" and dt == "bf16" else 1.0)      # see above
 
 
+@pytest.mark.parametrize("dt,dim,heads,pos", [
+    ("f32", 96, 2, 222), ("f32", 96, 2, 223),         # 224 keys: the first count in blocks of 64, here four of them
+    ("f32", 288, 6, 511), ("bf16", 288, 6, 512),      # eight blocks are one round of loads; the ninth holds the token's own key alone
+    ("f32", 256, 4, 1023), ("f32", 256, 4, 1024),     # sixteen are two rounds, with one more a launch adds them up
+    ("f32", 384, 3, 94), ("f32", 384, 3, 95),         # two pieces of a head a lane: from 96 keys
+    ("f32", 1040, 5, 127), ("bf16", 2064, 12, 300),   # more pieces of the vector than threads
+    ("f32", 3120, 39, 230),                           # four rounds, the last with 12 of 256 threads
+])
+def test_llama_step_adds_up_blocks_of_keys(dt, dim, heads, pos):
+    """The product with wo adds up the attention's key blocks: one and several rounds of shares, and the edges of the rule."""
+    from enzyme_ad.jax import llama
+    cfg, wd, wr, ((x, xr), (kc, kcr), (vc, vcr), _) = _inputs(dt, dim, 40, 1, heads, pos, dim + pos)
+    check(llama.forward_step(x, cfg, wd, kc, vc), L.forward_step(xr, cfg, wr, kcr, vcr), dt, "y")
+
+
 def test_llama_step_accumulates_and_repeats():
     """The step's cotangents add to what other uses of its operands contribute, and are the same bits run to run."""
     from enzyme_ad.jax import llama, ops, vjp
