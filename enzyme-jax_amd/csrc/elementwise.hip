@@ -62,8 +62,14 @@ template <int N> __device__ __forceinline__ void add_planes(const float* p, int6
 
 // What the 256 MB memory-side cache keeps of an array for the kernel behind, which reads it from its end (rope_kernel).  us, every
 // row a stream, read from the start | this: norm and rotation of 16 x 2048 x 4096 fp32 (537 MB) 370 | 345, of 268 MB 191 | 161, of
-// 134 MB bf16 87 | 83; keeping 208 MB 354, 272 MB 366.
+// 134 MB bf16 87 | 83; keeping 208 MB 354, 272 MB 366.  An array that fits with its rotation is read from its start: a row's blocks
+// lie on one XCD then and small arrays are found in its L2; dim 3072, 17 MB fp32 from the end | from the start 17.1 | 14.8, 25 MB
+// bf16 21.0 | 19.2, 67 MB 45.2 | 44.7.
 constexpr int64_t kMemoryCache = (int64_t)240 << 20;
+
+// The L2s of the eight XCDs together.  Where a block has several rows, theirs and the rotation's are not on one XCD, and dirty lines
+// that the L2s could hold are only written back at the kernel's end: a stream.  us, cached | stream: dim 1024 fp32, 17 MB 17.2 | 16.3.
+constexpr int64_t kL2s = (int64_t)32 << 20;
 
 // Rows from keep_from on are stored through the caches, so that the memory-side cache holds them for the kernel that reads y next;
 // the ones before, which would only push each other out, as a stream.
@@ -441,16 +447,17 @@ __global__ void rope_table_kernel(float2* __restrict__ table, int64_t seq, int h
 }
 
 // One block row of the grid per row of x (a sequence position of one sequence), a thread per 16-byte chunk (8 bf16 /
-// 4 fp32 elements): the indices are 32-bit and the position is the block's.  Last rows first: they are what the kernel that made x
-// has left in the memory-side cache; and where x and y are more than that holds, y is a stream that leaves x there.  (Two or more rows per thread, with
+// 4 fp32 elements): the indices are 32-bit and the position is the block's.  Where x and y are more
+// than the memory-side cache holds: last rows first, which are what the kernel that made x has left there, and y is a stream that
+// leaves x there.  (Two or more rows per thread, with
 // their loads in flight together, measured slower: 75 -> 73 -> 64 % of peak for 2, 4, 8 rows in bf16.)
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kernel(const T* x, const float2* __restrict__ table, T* y, int seq,
-                                                   int row_elems, int head_dim, int inverse, int stream) {
+                                                   int row_elems, int head_dim, int inverse, int beyond) {
   constexpr int V = ChunkCached<T>::N, NP = V / 2;
   const int col = (blockIdx.y * blockDim.x + threadIdx.x) * V;
   if (col >= row_elems) return;
-  const int row = gridDim.x - 1 - blockIdx.x, s = row % seq;
+  const int row = beyond ? gridDim.x - 1 - blockIdx.x : blockIdx.x, s = row % seq;
   const float4* tp = reinterpret_cast<const float4*>(table + (int64_t)s * (head_dim >> 1) + ((col % head_dim) >> 1));
   float4 t[NP / 2];                                          // two (cos, sin) entries each
 #pragma unroll
@@ -465,7 +472,7 @@ __global__ __launch_bounds__(256) void rope_kernel(const T* x, const float2* __r
     o[2 * p] = rotated_even(cs, sp, v[2 * p], v[2 * p + 1]);
     o[2 * p + 1] = rotated_odd(cs, sp, v[2 * p], v[2 * p + 1]);
   }
-  if (stream) Chunk<T>::store(y + (int64_t)row * row_elems + col, o);
+  if (beyond) Chunk<T>::store(y + (int64_t)row * row_elems + col, o);
   else ChunkCached<T>::store(y + (int64_t)row * row_elems + col, o);
 }
 
@@ -728,7 +735,8 @@ static int rmsnorm_fwd_launch(hipStream_t st, const void* x, const void* gamma, 
     hipLaunchKernelGGL(rmsnorm_fwd_generic_kernel<T>, dim3((unsigned)rows), dim3(256), 0, st, xp, gp, yp, rows, dim, eps);
   } else {
     const unsigned g = blocks_for(rows, 256 / tpr);
-    const int64_t keep_from = rows - kMemoryCache / (dim * (int64_t)sizeof(T));
+    const int64_t row_bytes = dim * (int64_t)sizeof(T);
+    const int64_t keep_from = tpr < 256 && rows * row_bytes <= kL2s ? rows : rows - kMemoryCache / row_bytes;
 #define EMI_RMS_FWD_P(TPR, NCH, PLANES)                                                                                                  \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, TPR, NCH, PLANES>), dim3(g), dim3(256), 0, st, xp, gp, yp, rows, (int)dim, eps, planes, count, \
                      static_cast<T*>(x_out), keep_from)

@@ -585,7 +585,8 @@ def test_rope_in_epilogues(ops, B, S, nh, d, D_in, dt):
         check(w, want[name], dt, "attention_block " + name)
 
 
-@pytest.mark.parametrize("dt,S,D", [("f32", 61438, 1024), ("f32", 61444, 1024), ("bf16", 70000, 2048), ("f32", 30723, 1024)])
+@pytest.mark.parametrize("dt,S,D", [("f32", 61438, 1024), ("f32", 61444, 1024), ("bf16", 70000, 2048), ("f32", 30723, 1024),
+                                    ("f32", 8192, 1024), ("f32", 8193, 1024)])
 def test_norm_and_rotation_of_arrays_around_the_size_of_the_memory_side_cache(dt, S, D):
     """All rows of an array of 240 MB are stored through the caches, the first ones of a larger one as a stream, and the rotation
     streams where it reads and writes more than that; rows of either kind against float64 (sums of D squares: D * 2^-24 of
