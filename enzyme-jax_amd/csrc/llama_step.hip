@@ -12,7 +12,7 @@
 //                        attention' | inverse rotation + wq^T dq + ... and dwq, dwk, dwv
 // The forward call leaves what the reverse one needs in `saved`.
 // Measured against the same step operator by operator (us): dim 288, 6 layers, fp32: forward 1071 -> 100 (99 launches ->
-// 25), with the reverse from StableHLO text at position 255 4042 -> 330 (289 launches -> 62); dim 4096, 2 layers, bf16,
+// 25), with the reverse from StableHLO text at position 255 4042 -> 315 (289 launches -> 63); dim 4096, 2 layers, bf16,
 // 4096 keys: forward 370 -> 211 (4.5 TB/s over weights and cache; 31 launches and two copies of each cache before).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
