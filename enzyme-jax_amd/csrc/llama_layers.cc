@@ -161,10 +161,9 @@ int product_and_norm(emi_stream_t st, const void* a, const void* b, const void* 
   return emi_rmsnorm_fwd(st, x, gamma, y, d.T(), d.D, d.eps, d.dtype);
 }
 
-// From s.xb1, the normalised x, on; with the next layer's gamma and xb1, or the result alone.
-int forward_layer(emi_stream_t st, const void* const* w, const void* x, const float* table, const Saved& s, void* out, const void* next_gamma,
-                  void* next_xb, void* ws, size_t wsb, const Dims& d) {
-  const int64_t T = d.T(), D = d.D, H = d.H;
+// q, k, v from s.xb1, the normalised x.
+int forward_heads(emi_stream_t st, const void* const* w, const float* table, const Saved& s, void* ws, size_t wsb, const Dims& d) {
+  const int64_t T = d.T(), D = d.D;
   if (d.rope_projection()) {
     EMI_TRY(emi_gemm_rope(st, s.xb1, w[kQ], s.q, table, T, D, D, d.S, d.hd(), d.dtype));
     EMI_TRY(emi_gemm_rope(st, s.xb1, w[kK], s.k, table, T, D, D, d.S, d.hd(), d.dtype));
@@ -179,8 +178,15 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
       EMI_TRY(emi_rope(st, s.q, table, s.q, 2 * d.B, d.S, d.heads, d.hd(), 0, d.dtype));
     }
   }
-  EMI_TRY(emi_attn_fwd(st, s.q, s.k, s.v, s.att, s.lse, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
-  EMI_TRY(product_and_norm(st, s.att, w[kO], x, s.x1, w[kFfn], s.xb2, ws, wsb, D, d));
+  return EMI_OK;
+}
+int forward_attention(emi_stream_t st, const Saved& s, const Dims& d) {
+  return emi_attn_fwd(st, s.q, s.k, s.v, s.att, s.lse, d.B, d.heads, d.S, d.hd(), d.S * d.D, d.hd(), d.D, d.scale, 1, d.dtype);
+}
+
+// h1, h3 and the SwiGLU from s.xb2, the normalised x1.
+int forward_gated(emi_stream_t st, const void* const* w, const Saved& s, void* ws, size_t wsb, const Dims& d) {
+  const int64_t T = d.T(), D = d.D, H = d.H;
   emi::ProductTail t{emi::kTailGated, {w[kW1], w[kW3], nullptr}, {s.h1, s.h3, s.g}, nullptr, 0, 0, 0, 0, nullptr, nullptr, nullptr, {}};
   if (const int rc = emi::gemm_tail(static_cast<hipStream_t>(st), s.xb2, w[kW1], t, T, H, D, D, 1, d.dtype); rc > 0) {
     return rc;
@@ -194,17 +200,36 @@ int forward_layer(emi_stream_t st, const void* const* w, const void* x, const fl
     EMI_TRY(emi_gemm_grouped(st, 2, a, b, nullptr, c, ws, wsb, T, H, D, D, D, H, H, 0, 1, 0, d.dtype));
     EMI_TRY(emi_swiglu_fwd(st, s.h1, s.h3, s.g, T * H, d.dtype));
   }
-  if (next_xb != nullptr) return product_and_norm(st, s.g, w[kW2], s.x1, out, next_gamma, next_xb, ws, wsb, H, d);
-  return emi_gemm_ws(st, s.g, w[kW2], s.x1, out, ws, wsb, T, D, H, H, H, D, D, 0, 1, d.dtype);
+  return EMI_OK;
 }
 
-// ---- forward mode: the tangents of one layer behind its values --------------------------------------------------------------
+// The layer's result; with the next layer's gamma its xb1 too.
+int forward_result(emi_stream_t st, const void* const* w, const Saved& s, void* out, const void* next_gamma, void* next_xb, void* ws, size_t wsb,
+                   const Dims& d) {
+  if (next_xb != nullptr) return product_and_norm(st, s.g, w[kW2], s.x1, out, next_gamma, next_xb, ws, wsb, d.H, d);
+  return emi_gemm_ws(st, s.g, w[kW2], s.x1, out, ws, wsb, d.T(), d.D, d.H, d.H, d.H, d.D, d.D, 0, 1, d.dtype);
+}
+
+// From s.xb1 on.
+int forward_layer(emi_stream_t st, const void* const* w, const void* x, const float* table, const Saved& s, void* out, const void* next_gamma,
+                  void* next_xb, void* ws, size_t wsb, const Dims& d) {
+  EMI_TRY(forward_heads(st, w, table, s, ws, wsb, d));
+  EMI_TRY(forward_attention(st, s, d));
+  EMI_TRY(product_and_norm(st, s.att, w[kO], x, s.x1, w[kFfn], s.xb2, ws, wsb, d.D, d));
+  EMI_TRY(forward_gated(st, w, s, ws, wsb, d));
+  return forward_result(st, w, s, out, next_gamma, next_xb, ws, wsb, d);
+}
+
+// ---- forward mode: a layer's values and tangents ---------------------------------------------------------------
 
 struct Tangents {                                         // of one layer
-  void *xb, *q, *k, *v, *att, *x1, *h1, *h3, *g, *out[2];  // (the second norm's goes where the first one's was); out: of even and odd layers
+  void *xb, *q, *k, *v, *att, *x1, *h1, *h3, *g, *out;
 };
+// One set for all layers: a layer's result and the next one's xb1 go where its own x and xb1 have been read for the last time, the
+// second norm's tangent where the first one's was, h1 and its tangent where q, k, v and att were.  The fewer bytes, the more of
+// them the memory-side cache holds.
 struct JvpScratch {
-  void* saved[2];                                         // of even and odd layers: a layer's product with w2 leaves the next one's xb1
+  Saved s;
   Tangents t;
   void* ws;
   size_t ws_bytes;
@@ -213,20 +238,28 @@ JvpScratch carve_jvp(void* base, const Dims& d, size_t* bytes = nullptr) {
   Carve c{static_cast<uint8_t*>(base), 0};
   const int64_t T = d.T();
   const size_t td = (size_t)T * d.D * d.elt(), th = (size_t)T * d.H * d.elt();
-  size_t n = 0;
-  carve_saved(nullptr, d, &n);
+  const size_t heads = 4 * td > th ? 4 * td : th;
   JvpScratch s;
-  for (void*& p : s.saved) p = c.take(n);
+  s.s.xb1 = c.take(td);
+  s.s.h1 = s.s.q = c.take(heads);
+  s.s.k = part(s.s.q, td);
+  s.s.v = part(s.s.q, 2 * td);
+  s.s.att = part(s.s.q, 3 * td);
+  s.s.x1 = c.take(td);
+  s.s.xb2 = c.take(td);
+  s.s.h3 = c.take(th);
+  s.s.g = c.take(th);
+  s.s.out = c.take(td);
+  s.s.lse = static_cast<float*>(c.take((size_t)d.B * d.heads * d.S * sizeof(float)));
   s.t.xb = c.take(td);
-  s.t.q = c.take(3 * td);
+  s.t.h1 = s.t.q = c.take(heads);
   s.t.k = part(s.t.q, td);
   s.t.v = part(s.t.q, 2 * td);
-  s.t.att = c.take(td);
+  s.t.att = part(s.t.q, 3 * td);
   s.t.x1 = c.take(td);
-  s.t.h1 = c.take(th);
   s.t.h3 = c.take(th);
   s.t.g = c.take(th);
-  for (void*& p : s.t.out) p = c.take(td);
+  s.t.out = c.take(td);
   s.ws_bytes = most({forward_scratch(d), emi_gemm_grouped_workspace_bytes(2, T, d.D, d.D, 0, 1, 1, d.dtype),
                      emi_gemm_grouped_workspace_bytes(2, T, d.H, d.D, 0, 1, 1, d.dtype), emi_gemm_grouped_workspace_bytes(2, T, d.D, d.H, 0, 1, 1, d.dtype)});
   s.ws = c.take(s.ws_bytes);
@@ -287,18 +320,27 @@ int tangent_products(emi_stream_t st, const void* tx, const void* x, std::initia
   return rotated ? emi_rope(st, t.C[0], table, t.C[0], rotated * d.B, d.S, d.heads, d.hd(), 0, d.dtype) : EMI_OK;      // (side by side)
 }
 
-// s: the layer's values;  tx: the tangent of its input x.
-int tangent_layer(emi_stream_t st, const void* const* w, const void* const* tw, const void* x, const void* tx, const float* table, const Saved& s,
-                  const JvpScratch& k, void* tout, const Dims& d) {
+// A layer from s.xb1 on and its tangents; tx: the tangent of its input x.  Each tangent behind the values it is of: they share
+// weights and activations, which the memory-side cache keeps from one to the other.  us, all values first and a set of buffers for
+// odd and one for even layers | this, bf16: 4096 tokens at dim 2048 1755 | 1705, 16384 6214 | 6100, 16384 at dim 1024 2873 | 2835,
+// 5784 at dim 768 843 | 841.
+int tangent_layer(emi_stream_t st, const void* const* w, const void* const* tw, const void* x, const void* tx, const float* table,
+                  const JvpScratch& k, void* out, void* tout, const void* next_gamma, void* next_xb, const Dims& d) {
+  const Saved& s = k.s;
   const Tangents& t = k.t;
   const int64_t T = d.T(), D = d.D, H = d.H;
   EMI_TRY(emi_rmsnorm_jvp(st, x, w[kAtt], tx, tw[kAtt], t.xb, T, D, d.eps, d.dtype));
+  EMI_TRY(forward_heads(st, w, table, s, k.ws, k.ws_bytes, d));
   EMI_TRY(tangent_products(st, t.xb, s.xb1, {kQ, kK, kV}, w, tw, {t.q, t.k, t.v}, 2, table, D, k, d));
+  EMI_TRY(forward_attention(st, s, d));
   EMI_TRY(emi_attn_jvp(st, s.q, s.k, s.v, s.lse, t.q, t.k, t.v, t.att, d.B, d.heads, d.S, d.hd(), d.S * D, d.hd(), D, d.scale, 1, d.dtype));
+  EMI_TRY(product_and_norm(st, s.att, w[kO], x, s.x1, w[kFfn], s.xb2, k.ws, k.ws_bytes, D, d));
   EMI_TRY(tangent_product(st, t.att, s.att, w[kO], tw[kO], tx, t.x1, D, D, k, d));
   EMI_TRY(emi_rmsnorm_jvp(st, s.x1, w[kFfn], t.x1, tw[kFfn], t.xb, T, D, d.eps, d.dtype));
+  EMI_TRY(forward_gated(st, w, s, k.ws, k.ws_bytes, d));
   EMI_TRY(tangent_products(st, t.xb, s.xb2, {kW1, kW3}, w, tw, {t.h1, t.h3}, 0, nullptr, H, k, d));
   EMI_TRY(emi_swiglu_jvp(st, s.h1, s.h3, t.h1, t.h3, t.g, T * H, d.dtype));
+  EMI_TRY(forward_result(st, w, s, out, next_gamma, next_xb, k.ws, k.ws_bytes, d));
   return tangent_product(st, t.g, s.g, w[kW2], tw[kW2], t.x1, tout, D, H, k, d);
 }
 
@@ -548,11 +590,9 @@ extern "C" int emi_llama_layers_jvp(emi_stream_t stream, const void* const* weig
       tw[i] = part(tangents[i], off);
     }
     const bool last = l + 1 == layers;
-    const Saved s = carve_saved(k.saved[l & 1], d), next = carve_saved(k.saved[(l + 1) & 1], d);
-    if (l == 0) EMI_TRY(emi_rmsnorm_fwd(stream, x, w[kAtt], s.xb1, d.T(), dim, eps, dtype));
-    void *out = last ? y : s.out, *tout = last ? ty : k.t.out[l & 1];
-    EMI_TRY(forward_layer(stream, w, x, rope_table, s, out, part(w[kAtt], last ? 0 : (size_t)dim * d.elt()), last ? nullptr : next.xb1, k.ws, k.ws_bytes, d));
-    EMI_TRY(tangent_layer(stream, w, tw, x, tx, rope_table, s, k, tout, d));
+    if (l == 0) EMI_TRY(emi_rmsnorm_fwd(stream, x, w[kAtt], k.s.xb1, d.T(), dim, eps, dtype));
+    void *out = last ? y : k.s.out, *tout = last ? ty : k.t.out;
+    EMI_TRY(tangent_layer(stream, w, tw, x, tx, rope_table, k, out, tout, part(w[kAtt], last ? 0 : (size_t)dim * d.elt()), last ? nullptr : k.s.xb1, d));
     x = out;
     tx = tout;
   }

@@ -147,10 +147,12 @@ def test_llama_layers_refuse_what_they_do_not_serve():
 
 
 @pytest.mark.parametrize("dt,dim,hidden,layers,heads,batch,seq", [
-    ("f32", 64, 72, 5, 2, 1, 33),             # tiles of 32: two products to a result in one launch; layers take turns in two buffers
+    ("f32", 64, 72, 5, 2, 1, 33),             # tiles of 32: two products to a result in one launch; all layers in one set of buffers
     ("f32", 288, 768, 2, 6, 3, 100),
     ("f32", 512, 1408, 1, 8, 2, 701),         # on the bf16 instructions: a launch to a result, and a pass to turn q and k
+    ("f32", 64, 304, 3, 2, 2, 45),            # a hidden layer longer than q, k, v and the attention together
     ("bf16", 128, 136, 3, 2, 2, 131),
+    ("bf16", 64, 520, 2, 1, 1, 70),
     ("bf16", 768, 2048, 1, 12, 1, 777),
     ("bf16", 2048, 1024, 1, 16, 2, 512),      # wide enough for two products one after the other
 ])
