@@ -6,8 +6,8 @@
 // A block of four (or eight) wavefronts owns 16 queries (forward, dQ; the tangent 16 or 32) or 16 keys (dK/dV). The 16-row tiles of the other sequence axis
 // are dealt to the wavefronts in turn, each accumulates over its own tiles, and the partial results are added
 // through the LDS at the end (the forward pass scales them to a common maximum first); that is the only barrier. A masked
-// score has the weight 0 and its row is multiplied by it, so a NaN or an infinity in a row of v also reaches earlier queries
-// of the same 16-row tile. Operands come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
+// score has the weight 0 and its row is multiplied by it, so in the forward pass a NaN or an infinity in a row of v also reaches
+// earlier queries of the same 16-row tile; the tangent keeps it from them (non_finite_rows). Operands come straight from global memory. What bounds it: a wavefront issues one matrix instruction per 32 cycles and its own
 // 16 rows are one chain of them, so with one wavefront per 16 rows (the earlier form) the longest row set the time and too
 // few wavefronts hid the loads. Causal, forward / adjoint in us: 6 heads x 256 x 48 13.6 / 40 -> 9 / 9,
 // 24 heads x 1000 x 64 89 / 280 -> 56 / 161 (55 / 48 TFLOP/s), 64 heads x 2048 x 128 1329 / 4010 -> 795 / 2907 (86 / 59);
@@ -28,6 +28,7 @@
 #include <initializer_list>
 #include <stdint.h>
 
+#include "attention_row.h"
 #include "emi_device.h"
 
 namespace emi {
@@ -403,11 +404,40 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_dq_f32_kernel(const float* __
                      unrope != nullptr ? unrope + (int64_t)qc * (8 * NT) : nullptr);
 }
 
+// Where a row of v or tv that not all queries of a block see is not finite, the masked weight 0 would carry it to the others, as it
+// would those that stand in for rows past the end: the tangent's block works such queries out row by row.  It looks at these rows beside
+// the loads of q where the CU has another block meanwhile, and otherwise once they are in registers, in the last tile of
+// one or two wavefronts.  us, neither | before | after, causal heads x length x head size: 32 x 512 x 48 69 | 68 | 71, 32 x 1716 x 64 547 |
+// 540 | 546, 32 x 512 x 80 106 | 107 | 111; 32 x 512 x 96 123 | 128 | 122, 32 x 1716 x 96 826 | 867 | 804, 32 x 1716 x 128 1107 | 1121 | 1108.
+//
+// A NaN in one of the block's threads if the rows row0 .. end - 1 of a head (at most 16) hold a NaN or an infinity.
+template <int NT>
+__device__ __forceinline__ float non_finite_rows(const float* __restrict__ head, int64_t ss, int row0, int end) {
+  float z = 0.f;
+#pragma unroll
+  for (int u = 0; u < (NT + 3) / 4; u++) {
+    const int i = u * 256 + (int)threadIdx.x, r = row0 + i / (4 * NT);
+    const float4 x = *reinterpret_cast<const float4*>(head + (int64_t)(r < end ? r : end - 1) * ss + 4 * (i % (4 * NT)));
+    z = fmaf(x.x, 0.f, fmaf(x.y, 0.f, fmaf(x.z, 0.f, fmaf(x.w, 0.f, z))));
+  }
+  return z;
+}
+
+// A NaN if one of the values is a NaN or an infinity.
+template <int NT> __device__ __forceinline__ float non_finite(const float (&x)[4][NT]) {
+  float z = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int n = 0; n < NT; n++) z = fmaf(x[t][n], 0.f, z);
+  return z;
+}
+
 // Tangent: with p = exp(scale q k^T - lse) and tS = scale (tq k^T + q tk^T)
 //   to = sum_j p_j tv_j + sum_j p_j tS_j v_j - mu o,   o = sum_j p_j v_j,   mu = sum_j p_j tS_j
 // in one walk over the keys: six products, and two accumulators (the first two sums are one).  QS sets of 16 queries share every
-// row of K, V, tK and tV that is loaded.  A null tangent skips its loads and products.  What bounds it: as above, and with heads
-// of 128 one wavefront a SIMD (322 registers).  Causal, us, a wavefront per query without matrix instructions | this: 16 heads x
+// row of K, V, tK and tV that is loaded.  A null tangent skips its loads and products.  What bounds it: as above, and from heads
+// of 96 on one wavefront a SIMD (of 128: 322 registers with one set of queries, 500 with two).  Causal, us, a wavefront per query without matrix instructions | this: 16 heads x
 // 1122 x 64 3918 | 103, 32 x 1716 x 64 16918 | 405 (89 TFLOP/s), 96 x 1817 x 128 117047 | 2662 (91), 6 x 256 x 48 143 | 10;
 // error against float64 4.7e-7 | 4.2e-7 at 32 x 512 x 128.
 template <int NT, int QS>
@@ -418,6 +448,7 @@ __global__ __launch_bounds__(64 * 4) void attn_jvp_f32_kernel(const float* __res
                                                                    AttnShapeF32 sh, float scale, int causal) {
   __shared__ float buf[4][4 * NT][64];
   __shared__ float stat[QS][4][16];
+  __shared__ int by_row[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, G = lane >> 4;
   const int tiles = (sh.seq + 16 * QS - 1) / (16 * QS);
   const BlockRows own = block_rows(tiles);
@@ -438,8 +469,8 @@ __global__ __launch_bounds__(64 * 4) void attn_jvp_f32_kernel(const float* __res
     for (int n = 0; n < NT; n++) acct[s][n] = acco[s][n] = f32q_t{0.f, 0.f, 0.f, 0.f};
   }
   const int nkeys = causal ? (q0 + 16 * QS < sh.seq ? q0 + 16 * QS : sh.seq) : sh.seq;
-  for (int kb = 16 * wave; kb < nkeys; kb += 16 * 4) {
-    float kf[NT][4], tkf[NT][4], vx[4][NT], tvx[4][NT];
+  auto tile = [&](int kb, float (&vx)[4][NT], float (&tvx)[4][NT]) __attribute__((always_inline)) {
+    float kf[NT][4], tkf[NT][4];
     load_rows<NT>(k + base, sh.ss, kb, last, lane, kf);
     if (tk != nullptr) load_rows<NT>(tk + base, sh.ss, kb, last, lane, tkf);
     load_cols<NT>(v + base, sh.ss, kb, last, lane, vx);
@@ -463,6 +494,24 @@ __global__ __launch_bounds__(64 * 4) void attn_jvp_f32_kernel(const float* __res
       mma_cols<NT>(vx, w, acct[s]);
       if (tv != nullptr) mma_cols<NT>(tvx, p, acct[s]);
     }
+  };
+  int odd = 0;
+  if constexpr (QS == 1 && NT <= 5) {                              // two or more wavefronts a SIMD
+    float z = non_finite_rows<NT>(v + base, sh.ss, causal ? q0 : last, nkeys);
+    if (tv != nullptr) z += non_finite_rows<NT>(tv + base, sh.ss, causal ? q0 : last, nkeys);
+    odd = __any(z != 0.f);                                         // (NaN)
+    if (lane == 0) by_row[wave] = odd;
+    for (int kb = 16 * wave; kb < nkeys; kb += 16 * 4) {
+      float vx[4][NT], tvx[4][NT];
+      tile(kb, vx, tvx);
+    }
+  } else {
+    float vx[4][NT], tvx[4][NT];
+    int kb = 16 * wave;
+    for (; kb < nkeys; kb += 16 * 4) tile(kb, vx, tvx);
+    kb -= 16 * 4;
+    if (kb >= 0 && kb + 15 > (causal ? q0 : last)) odd = __any(non_finite<NT>(vx) + (tv != nullptr ? non_finite<NT>(tvx) : 0.f) != 0.f);
+    if (lane == 0) by_row[wave] = odd;
   }
 #pragma unroll
   for (int s = 0; s < QS; s++) {
@@ -481,6 +530,11 @@ __global__ __launch_bounds__(64 * 4) void attn_jvp_f32_kernel(const float* __res
     const int myq = q0 + 16 * s + (lane & 15);
     if (s > 0) __syncthreads();                                    // buf has been read
     merge_store<NT, 4>(to + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acct[s], one, buf);
+  }
+  if (by_row[0] | by_row[1] | by_row[2] | by_row[3]) {
+    __syncthreads();                                               // the rows have been stored
+    for (int qi = q0 + wave; qi < q0 + 16 * QS && qi < sh.seq; qi += 4)
+      attn_jvp_row<float>(q, k, v, lse[(int64_t)bh * sh.seq + qi], tq, tk, tv, to, qi, causal ? qi + 1 : sh.seq, {base, sh.ss, 16 * NT, lane, scale});
   }
 }
 

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "attention_row.h"
 #include "emi_device.h"
 
 namespace emi {
@@ -170,9 +171,8 @@ struct JvpShape {
 // o = P v, P = softmax(scale q k^T + causal mask)  (test/llama.py:13-18,178-206; DotGeneral :1166,
 // Exp :1182, Div :1133, Sub :1312, reduce max/add StableHLOAutoDiffOpInterfaceImpl.cpp:1833-1916):
 //   tS = scale (tq k^T + q tk^T);  tP = P (tS - rowsum(P tS));  to = tP v + P tv
-//      = sum_j p_j tS_j v_j - (sum_j p_j tS_j) o + sum_j p_j tv_j,   p_j = exp(S_j - lse)
-// One wavefront per query row, one key per lane and 64 keys per sweep; head_dim <= 256.  For the shapes that the matrix-core
-// kernels (attention.hip, attention_f32.hip) do not take.
+// One wavefront per query row (attn_jvp_row), for the shapes that the matrix-core kernels (attention.hip, attention_f32.hip) do
+// not take.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_jvp_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                                        const float* __restrict__ lse, const T* __restrict__ tq,
@@ -183,52 +183,7 @@ __global__ __launch_bounds__(256) void attn_jvp_kernel(const T* __restrict__ q, 
   const int bh = blockIdx.y;
   if (qi >= sh.seq) return;
   const int64_t base = (int64_t)(bh / sh.heads) * sh.sb + (int64_t)(bh % sh.heads) * sh.sh;
-  const T* qr = q + base + (int64_t)qi * sh.ss;
-  const T* tqr = tq ? tq + base + (int64_t)qi * sh.ss : nullptr;
-  const int nkeys = causal ? qi + 1 : sh.seq;
-  const float L = lse[(int64_t)bh * sh.seq + qi];
-  float mu = 0.f;
-  float acc_w[4] = {0.f, 0.f, 0.f, 0.f}, acc_o[4] = {0.f, 0.f, 0.f, 0.f}, acc_t[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < nkeys; k0 += 64) {
-    const int key = k0 + lane;
-    float p = 0.f, w = 0.f;
-    if (key < nkeys) {
-      const T* kr = k + base + (int64_t)key * sh.ss;
-      const T* tkr = tk ? tk + base + (int64_t)key * sh.ss : nullptr;
-      float s = 0.f, ts = 0.f;
-      for (int i = 0; i < d; i++) {
-        const float qv = to_f32(qr[i]), kv = to_f32(kr[i]);
-        s = fmaf(qv, kv, s);
-        if (tqr) ts = fmaf(to_f32(tqr[i]), kv, ts);
-        if (tkr) ts = fmaf(qv, to_f32(tkr[i]), ts);
-      }
-      p = expf(s * scale - L);
-      w = p * ts * scale;
-    }
-    mu += wave_sum(w);
-    const int cnt = nkeys - k0 < 64 ? nkeys - k0 : 64;
-    for (int j = 0; j < cnt; j++) {
-      const float pj = __shfl(p, j, 64), wj = __shfl(w, j, 64);
-      const T* vr = v + base + (int64_t)(k0 + j) * sh.ss;
-      const T* tvr = tv ? tv + base + (int64_t)(k0 + j) * sh.ss : nullptr;
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const int i = lane + c * 64;
-        if (i < d) {
-          const float vv = to_f32(vr[i]);
-          acc_w[c] = fmaf(wj, vv, acc_w[c]);
-          acc_o[c] = fmaf(pj, vv, acc_o[c]);
-          if (tvr) acc_t[c] = fmaf(pj, to_f32(tvr[i]), acc_t[c]);
-        }
-      }
-    }
-  }
-  T* out = to + base + (int64_t)qi * sh.ss;
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    const int i = lane + c * 64;
-    if (i < d) out[i] = from_f32<T>(acc_w[c] - mu * acc_o[c] + acc_t[c]);
-  }
+  attn_jvp_row<T>(q, k, v, lse[(int64_t)bh * sh.seq + qi], tq, tk, tv, to, qi, causal ? qi + 1 : sh.seq, {base, sh.ss, d, lane, scale});
 }
 
 bool al16(const void* p) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

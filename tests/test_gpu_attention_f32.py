@@ -123,3 +123,37 @@ def test_f32_attention_adjoint_turns_its_operands_back(h, S, d):
     for t in two[:2]:
         _native.check(lib.emi_rope(st, t.data_ptr(), table.data_ptr(), t.data_ptr(), B, S, h, d, 1, 11))
     assert all(torch.equal(a, b) for a, b in zip(one, two))
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("h,S,d", [(2, 100, 48), (3, 50, 40), (19, 530, 128)])
+def test_f32_attention_tangent_keeps_non_finite_values(h, S, d, causal):
+    """A NaN or an infinity in a row of v or of its tangent reaches the queries that see it and no other: one and two sets of 16
+    queries a block (530 of 19 heads), head_dim 40 in the kernel of one wavefront per query.  The row of the last key also stands
+    in for rows past the end; an infinity that every query sees stays one.  Bound of the finite entries as above."""
+    from enzyme_ad.jax import ops, jvp
+    rng = np.random.default_rng(S + d)
+    raw = [rng.standard_normal((1, h, S, d)) for _ in range(6)]
+    bound = 4 * (d + S) * 2.0 ** -23
+
+    def run(arrays):
+        a = [dev(x, "f32")[0] for x in arrays]
+        return host(jvp(lambda q, k, v: ops.attention(q, k, v, h, causal=causal, layout="bhsd"), tuple(a[:3]), tuple(a[3:]))[1])
+
+    clean = run(raw)
+    for which in (2, 5):
+        for at, value in ((S - 1, np.inf), (37, np.nan), (21, np.inf), (16, np.nan)):
+            bad, without = list(raw), list(raw)
+            bad[which], without[which] = raw[which].copy(), raw[which].copy()
+            bad[which][0, 1, at] = value
+            without[which][0, 1, at] = 0.0
+            got = run(bad)
+            seen = slice(at, S) if causal else slice(0, S)
+            assert np.array_equal(got[0, 0], clean[0, 0]) and np.array_equal(got[0, 2:], clean[0, 2:])
+            assert not np.isfinite(got[0, 1, seen]).any()
+            if which == 5 and value == np.inf:
+                assert np.isposinf(got[0, 1, seen]).all()
+            if causal:
+                want = L.attention_jvp(*(dev(x, "f32")[1][:, 1:2] for x in without), causal=True)
+                size = max(float(np.max(np.abs(want))), 1.0)
+                assert float(np.max(np.abs(got[0, 1, :at] - want[0, 0, :at]))) <= bound * size, (which, at, value)
