@@ -2189,7 +2189,7 @@ int emi::gemm_grouped_run(hipStream_t st, int count, const void* const* A, const
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     fast = lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && ldc >= N && (lda % 8 == 0) && (ldb % 8 == 0) &&
            (K % 8 == 0 || (trans_a && !trans_b)) && (!trans_a || M % 8 == 0) && (trans_b || N % 8 == 0) && a_bytes < 0x7fffff00LL && b_bytes < 0x7fffff00LL &&
-           ldr <= 0x7fffffff && ldc <= 0x7fffffff && ((M + 255) / 256) * ((N + 255) / 256) < 192;
+           ldr <= 0x7fffffff && ldc <= 0x7fffffff && bf16_one_launch(M, N);
     for (int i = 0; i < count && fast; i++) fast = al16(A[i]) && al16(B[i]);
     // a residual on some results only would need a null check per product: all or none
     bool any_r = false, all_r = true;

@@ -37,6 +37,9 @@ inline int64_t splits_held(const void* workspace, size_t bytes, int64_t M, int64
 // in two splits 85 (estimate 71), in one pass 84 (73), one by one 80; two of 1000 x 4096 x 11008 212 (163), one by one 178.
 inline int64_t sum_splits(int64_t M, int64_t N, int64_t held) { return (M + 127) / 128 * ((N + 127) / 128) >= 192 ? 1 : held; }
 
+// Whether several bf16 products of a shape are one launch at all: not where one alone has 256-tiles for most of the chip.
+inline bool bf16_one_launch(int64_t M, int64_t N) { return (M + 255) / 256 * ((N + 255) / 256) < 192; }
+
 // Whether products that can run as one launch, each in a single pass over K, run one by one: where each split over K is so
 // much faster that together they are, by more than the estimates are off (`margin`: bf16 products of a few rows are
 // estimated up to a third too fast, fp32 ones hardly).  A launch more each, and the gap before it.  us, one launch | one by one:

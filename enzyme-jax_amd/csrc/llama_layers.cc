@@ -279,14 +279,16 @@ TangentPlan tangent_plan(int64_t N, int64_t K, const JvpScratch& k, const Dims& 
   return {2 * emi::bf16_plan(T, N, K, 1, 0, 1, held).us + 1.0, emi::bf16_plan(T, N, K, 2, 1, 1, most).us * (most > 1 ? 1.0 : 1.1), most};
 }
 
-// ty = tx w^T + x tw^T [+ r]
+// ty = tx w^T + x tw^T [+ r].  As two products in the operators' order: w, which the value's own product has just read, is still in
+// the memory-side cache, and the sum is added to while it is.  bf16, dim 4096, us a layer, the other way round and the results
+// that share x in turn | this (operator by operator): 1500 tokens 2389 | 2374 (2411), 2000 2760 | 2752 (2756).
 int tangent_product(emi_stream_t st, const void* tx, const void* x, const void* w, const void* tw, const void* r, void* ty, int64_t N, int64_t K,
                     const JvpScratch& k, const Dims& d) {
   const int64_t T = d.T();
   const TangentPlan p = tangent_plan(N, K, k, d);
   if (p.two < p.sum) {
-    EMI_TRY(emi_gemm_ws(st, x, tw, r, ty, k.ws, k.ws_bytes, T, N, K, K, K, N, N, 0, 1, d.dtype));
-    return emi_gemm_ws(st, tx, w, ty, ty, k.ws, k.ws_bytes, T, N, K, K, K, N, N, 0, 1, d.dtype);
+    EMI_TRY(emi_gemm_ws(st, tx, w, r, ty, k.ws, k.ws_bytes, T, N, K, K, K, N, N, 0, 1, d.dtype));
+    return emi_gemm_ws(st, x, tw, ty, ty, k.ws, k.ws_bytes, T, N, K, K, K, N, N, 0, 1, d.dtype);
   }
   const void *a[2] = {tx, x}, *b[2] = {w, tw}, *res[1] = {r};
   void* out[1] = {ty};
@@ -295,8 +297,9 @@ int tangent_product(emi_stream_t st, const void* tx, const void* x, const void* 
 }
 
 // Several results of tangent_product that share x and tx; the first `rotated` turned.  One launch where that is faster, or the
-// products with every tw as one group and those with every w, which add to them, as another (bf16: the 256-tiles of three
-// results fill the chip where one's do not, 1000 x 4096 x 4096 180 us, result by result 241).
+// products with every w as one group and those with every tw, which add to them, as another (bf16: the 256-tiles of three
+// results fill the chip where one's do not, 1000 x 4096 x 4096 180 us, result by result 241; where one's do, a group would
+// run one by one, every sum out of the cache before it is added to: 2000 x 11008 x 4096 194 us a second product, 188 behind the first).
 int tangent_products(emi_stream_t st, const void* tx, const void* x, std::initializer_list<int> which, const void* const* w, const void* const* tw,
                      std::initializer_list<void*> out, int rotated, const float* table, int64_t N, const JvpScratch& k, const Dims& d) {
   emi::ProductTail t{emi::kTailRotated, {}, {}, rotated ? table : nullptr, (int)d.S, (int)d.hd(), rotated, 0, nullptr, nullptr, x, {}};
@@ -310,10 +313,11 @@ int tangent_products(emi_stream_t st, const void* tx, const void* x, std::initia
   if (rc >= 0) return rc;
   const TangentPlan p = tangent_plan(N, d.D, k, d);
   const double group = d.dtype == EMI_F32 ? emi::f32_plan(d.T(), N, d.D, t.count, 0, 0, 1).us : emi::bf16_plan(d.T(), N, d.D, t.count, 0, 1, 1).us;
-  if (2 * group + 1.0 < t.count * ((p.two < p.sum ? p.two : p.sum) + 1.0)) {
+  const bool one_launch = d.dtype == EMI_F32 || emi::bf16_one_launch(d.T(), N);
+  if (one_launch && 2 * group + 1.0 < t.count * ((p.two < p.sum ? p.two : p.sum) + 1.0)) {
     const void *xs[3] = {x, x, x}, *txs[3] = {tx, tx, tx};
-    EMI_TRY(emi_gemm_grouped(st, t.count, xs, t.B1, nullptr, t.C, k.ws, k.ws_bytes, d.T(), N, d.D, d.D, d.D, N, N, 0, 1, 0, d.dtype));
-    EMI_TRY(emi_gemm_grouped(st, t.count, txs, t.B, t.C, t.C, k.ws, k.ws_bytes, d.T(), N, d.D, d.D, d.D, N, N, 0, 1, 0, d.dtype));
+    EMI_TRY(emi_gemm_grouped(st, t.count, txs, t.B, nullptr, t.C, k.ws, k.ws_bytes, d.T(), N, d.D, d.D, d.D, N, N, 0, 1, 0, d.dtype));
+    EMI_TRY(emi_gemm_grouped(st, t.count, xs, t.B1, t.C, t.C, k.ws, k.ws_bytes, d.T(), N, d.D, d.D, d.D, N, N, 0, 1, 0, d.dtype));
   } else {
     for (int i = 0; i < t.count; i++) EMI_TRY(tangent_product(st, tx, x, t.B[i], t.B1[i], nullptr, t.C[i], N, d.D, k, d));
   }

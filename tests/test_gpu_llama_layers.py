@@ -184,3 +184,23 @@ def test_llama_layers_forward_mode(dt, dim, hidden, layers, heads, batch, seq):
         b = jvp(lambda x, w: llama.layer(x, w, heads), (x, one), (tx, dict(zero, wq=None)))
         tol = 1e-5 if dt == "f32" else 2e-2
         assert rel_err(host(a[0]), host(b[0])) < tol and rel_err(host(a[1]), host(b[1])) < tol
+
+
+def test_llama_layer_tangent_in_the_operators_order():
+    """Of so many tokens that each product is a launch, a tangent's two products run in the operators' order, each result's second
+    behind its first: the operators' bits, where the values are (no rotation and no gate, which the layer's products apply)."""
+    from enzyme_ad.jax import jvp, llama, ops
+    dim, heads = 2048, 16
+    _, wd, _, x, _, _, _ = _inputs("bf16", dim, 2304, 1, heads, 6, 1024)
+    rng = np.random.Generator(np.random.PCG64(4))
+    w = {k: torch.zeros_like(t[0]) if k in ("wq", "wk", "w1") else t[0].contiguous() for k, t in wd.items()}
+    tw = {k: dev(rng.standard_normal(tuple(t.shape)) / np.sqrt(dim), "bf16")[0] for k, t in w.items()}
+    tx = dev(rng.standard_normal(tuple(x.shape)), "bf16")[0]
+
+    def run():
+        return jvp(lambda x, w: llama.layer(x, w, heads), (x, w), (tx, tw))
+
+    y, ty = run()
+    with ops.Tape():                                     # under a tape the operators run one by one
+        want, twant = run()
+    assert torch.equal(y, want) and torch.equal(ty, twant)
