@@ -544,8 +544,10 @@ int launch_copy(hipStream_t st, const void* in, void* out, const CopyPlan& p) {
 // Several arrays, each of whole bytes, in one launch: a block has kCopyBlock bytes of one of them, all its loads in flight at
 // once.  A replayed graph's arguments are a dozen arrays of a few KB and two or three of tens of MB: a launch each is 2 to 3 us on
 // the GPU and 5 on the host (dim-288 training step, 15 arguments, 98 MB, replayed: 855 -> 808 us; dim-768 model of 64 tokens, bf16, 353 ->
-// 282).
-constexpr int kCopyArrays = 48, kCopyUnroll = 16, kCopyBlock = kBlock * 16 * kCopyUnroll;
+// 282).  Small blocks and loads through the caches, from which graphs read next.  Replay of a graph of two arrays of 256 MiB, us: a copy each
+// 205, blocks of 64 KiB streaming 216, of 16 KiB 192; one of 128 MiB 44, 52, 44.  Off 16-byte boundaries (copy_words), three arrays
+// of 32 MiB of which one | all are off by an element: a copy each 46 | 48, byte by byte 86 | 149, in words 44 | 43.
+constexpr int kCopyArrays = 48, kCopyUnroll = 4, kCopyBlock = kBlock * 16 * kCopyUnroll;
 struct CopyMany {
   const uint8_t* src[kCopyArrays];
   uint8_t* dst[kCopyArrays];
@@ -553,30 +555,49 @@ struct CopyMany {
   int first[kCopyArrays + 1];                              // the first block of each
   int count;
 };
+// A block's share in words that both addresses are whole numbers of, a batch of loads at a time; the rest byte by byte.
+template <typename W> __device__ __forceinline__ void copy_words(const uint8_t* src, uint8_t* dst, int n) {
+  constexpr int U = 16;
+  const int words = n / (int)sizeof(W);
+  const W* s = reinterpret_cast<const W*>(src);
+  W* d = reinterpret_cast<W*>(dst);
+  for (int w0 = threadIdx.x; w0 < words; w0 += U * kBlock) {
+    W v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = s[w0 + u * kBlock < words ? w0 + u * kBlock : w0];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (w0 + u * kBlock < words) d[w0 + u * kBlock] = v[u];
+  }
+  const int rest = n - words * (int)sizeof(W), at = words * (int)sizeof(W) + (int)threadIdx.x;
+  if ((int)threadIdx.x < rest) dst[at] = src[at];
+}
 __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyMany m) {
   int a = 0;
   while (a + 1 < m.count && (int)blockIdx.x >= m.first[a + 1]) a++;
   const int64_t at = (int64_t)((int)blockIdx.x - m.first[a]) * kCopyBlock, left = m.bytes[a] - at;
   const uint8_t* src = m.src[a] + at;
   uint8_t* dst = m.dst[a] + at;
-  if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) != 0) {
-    const int n = left < kCopyBlock ? (int)left : kCopyBlock;
-    for (int i = threadIdx.x; i < n; i += kBlock) dst[i] = src[i];
+  const int off = (int)((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15), n = left < kCopyBlock ? (int)left : kCopyBlock;
+  if (off != 0) {
+    if ((off & 3) == 0) copy_words<uint32_t>(src, dst, n);
+    else if ((off & 1) == 0) copy_words<uint16_t>(src, dst, n);
+    else copy_words<uint8_t>(src, dst, n);
     return;
   }
-  const int pieces = left < kCopyBlock ? (int)(left >> 4) : kCopyBlock / 16;
+  const int pieces = n >> 4;
   uint4 v[kCopyUnroll];
 #pragma unroll
   for (int u = 0; u < kCopyUnroll; u++) {
     const int c = u * kBlock + threadIdx.x;
-    v[u] = c < pieces ? stream_load(reinterpret_cast<const uint4*>(src) + c) : make_uint4(0, 0, 0, 0);
+    v[u] = c < pieces ? reinterpret_cast<const uint4*>(src)[c] : make_uint4(0, 0, 0, 0);
   }
 #pragma unroll
   for (int u = 0; u < kCopyUnroll; u++) {
     const int c = u * kBlock + threadIdx.x;
     if (c < pieces) *(reinterpret_cast<uint4*>(dst) + c) = v[u];
   }
-  if (left < kCopyBlock && (int)threadIdx.x < (int)(left & 15)) dst[pieces * 16 + threadIdx.x] = src[pieces * 16 + threadIdx.x];
+  if ((int)threadIdx.x < (n & 15)) dst[pieces * 16 + threadIdx.x] = src[pieces * 16 + threadIdx.x];
 }
 
 // ---------------------------------------------------------------------------

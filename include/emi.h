@@ -390,7 +390,8 @@ int emi_strided_copy(emi_stream_t stream, const void* in, void* out, int rank, c
                      const int64_t* in_strides, int64_t in_offset, const int64_t* out_strides,
                      int64_t out_offset, int elem_bytes);
 /* dst[i] = src[i], bytes[i] bytes, for i < count: arrays on the device, the tables HOST arrays.  No
- * destination overlaps another array of the call, but may be its own source. */
+ * destination overlaps another array of the call, but may be its own source.  Any alignment: what is
+ * off 16-byte boundaries goes in words of 4, 2 or 1 bytes. */
 int emi_copy_many(emi_stream_t stream, int count, const void* const* src, void* const* dst, const int64_t* bytes);
 /* y[o, i] = sum or max over r of x[o, r, i] (op = EMI_OP_ADD or EMI_OP_MAX), fp32
  * accumulation (stablehlo.reduce with an add / maximum body; Reduce rule

@@ -120,3 +120,35 @@ def test_captured_takes_arguments_of_any_layout_and_its_own_buffers():
     assert torch.equal(g(b, ga)[0], b + b)                # b into the first buffer, which is then the second argument
     _, ga, gb = g(a, b)
     assert torch.equal(g(gb, b)[0], b + b) and torch.equal(g(ga, gb)[0], b + b)
+
+
+def test_copy_many_of_words():
+    """Arrays whose two addresses are whole numbers of 4, of 2 and of no more than one byte: less than a word, less than a batch of a
+    block's loads, one batch and a little more, one block and a little more."""
+    from enzyme_ad.jax import _native
+    import ctypes
+    cases = [(n, a, b) for a, b in ((4, 0), (0, 12), (4, 8), (2, 0), (6, 12), (1, 3)) for n in (1, 5, 1023, 4095, 16384, 16391, 65536, 65543, 150001)]
+    room = torch.randint(0, 255, (200000,), dtype=torch.uint8, device="cuda")
+    out = [torch.full((n + 32,), 7, dtype=torch.uint8, device="cuda") for n, _, _ in cases]
+    table = ctypes.c_void_p * len(cases)
+    _native.check(_native.lib().emi_copy_many(torch.cuda.current_stream().cuda_stream, len(cases), table(*[room.data_ptr() + a for _, a, _ in cases]),
+                                              table(*[o.data_ptr() + b for o, (_, _, b) in zip(out, cases)]), (ctypes.c_int64 * len(cases))(*[c[0] for c in cases])))
+    for o, (n, a, b) in zip(out, cases):
+        assert torch.equal(o[b:b + n], room[a:a + n]) and bool((o[:b] == 7).all()) and bool((o[b + n:] == 7).all()), (n, a, b)
+
+
+def test_captured_takes_three_arguments_of_any_layout_and_its_own_buffers():
+    """As above with arguments enough for the one launch: whole arrays beside strided, host and misaligned ones, and outputs that are
+    the graph's argument buffers."""
+    from enzyme_ad.jax import ops
+    from enzyme_ad.jax.graph import capture
+    a, b, c = (torch.randn(300, 8, device="cuda") for _ in range(3))
+    g = capture(lambda a, b, c: (ops.add(ops.add(a, b), c), a, b, c), a, b, c)
+    strided = torch.randn(8, 300, device="cuda").t()
+    off = torch.randn(300 * 8 + 1, device="cuda")[1:].view(300, 8)
+    for x, y, z in ((a, b, c), (strided, off, b), (torch.randn(300, 8), b, off), (a, a, a), (off, strided, a)):
+        assert torch.equal(g(x, y, z)[0], (x.cuda() + y.cuda()) + z.cuda())
+    _, ga, gb, gc = g(a, b, c)
+    assert torch.equal(g(b, ga, c)[0], (b + b) + c)       # b into the first buffer, which is then the second argument
+    _, ga, gb, gc = g(a, b, c)
+    assert torch.equal(g(gc, a, gb)[0], (c + a) + a)      # (gb is read after a has gone into it)
