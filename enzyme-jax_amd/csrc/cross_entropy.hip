@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void xent_fwd_kernel(const T* __restrict__ log
                                                        int64_t vocab) {
   constexpr int N = Chunk<T>::N;
   __shared__ float red[8];
-  const int64_t row = gridDim.x - 1 - blockIdx.x;      // last rows first: the memory-side cache still holds them, and holds the first ones after
+  const int64_t row = blockIdx.x;
   const T* z = logits + row * vocab;
   const int64_t nchunk = (vocab + N - 1) / N;
   float m = -INFINITY, s = 0.f;
