@@ -695,13 +695,13 @@ struct StepDims {
     if (keys <= 256) return 256;
     return (int)(want < 128 ? 128 : want > 512 ? 512 : want);
   }
-  // whether the product with wo adds up this many shares a head (step_combine): two rounds, or more of at most eight shares
-  bool combines(int64_t shares) const {
-    const int64_t pieces = D / (dtype == EMI_BF16 ? 8 : 4);
-    const int64_t rounds = (pieces + 255) / 256 * ((shares + kCombineShares - 1) / kCombineShares);
-    return rounds <= 2 || (shares <= kCombineShares && rounds <= 4);
-  }
-  bool combine_inside() const { return nsplit() > 1 && combines(nsplit()); }
+  // step_combine's rounds of loads, and whether the product with wo adds up this many shares a head: two rounds, or more of at most
+  // eight shares
+  int64_t rounds(int64_t shares) const { return (D / (dtype == EMI_BF16 ? 8 : 4) + 255) / 256 * ((shares + kCombineShares - 1) / kCombineShares); }
+  bool combines(int64_t shares) const { return rounds(shares) <= 2 || (shares <= kCombineShares && rounds(shares) <= 4); }
+  // (four rounds only with the blocks of 64 keys that they allow: dim 4096 fp32, 2 layers, us, a launch | inside, 300 keys in blocks of 64
+  // 315 | 308, 512 to 1023 keys in blocks of 128 317 to 319 | 320 to 322)
+  bool combine_inside() const { return nsplit() > 1 && combines(nsplit()) && (rounds(nsplit()) <= 2 || kpb() == 64); }
   bool short_cache() const {                              // attention inside the product with wo: step_attention
     const int lanes = hd() / (dtype == EMI_BF16 ? 8 : 4);
     return lanes <= 16 && (heads + 15) / 16 * ((pos + kStepKeys) / kStepKeys) <= kStepRounds;
