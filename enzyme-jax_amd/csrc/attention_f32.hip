@@ -98,9 +98,10 @@ __device__ __forceinline__ void mma_cols(const float (&x)[4][NT], const f32q_t w
 }
 
 // Adds the W wavefronts' accumulators and stores the sum: wavefront w < 4 takes register w of every lane, that is NT
-// consecutive elements of each of the 16 rows.  `mul[i]` scales wavefront i's share.  angles: null, or the row's (cos, sin) pairs,
-// by which it is turned back (the cotangent of a vector that was rotated).  The LDS is free after the next barrier.
-template <int NT, int W>
+// consecutive elements of each of the 16 rows.  `mul[i]` scales wavefront i's share.  TURN: angles are the row's (cos, sin) pairs,
+// by which it is turned back (the cotangent of a vector that was rotated); a null pointer looked at instead cost the adjoint without a
+// rotation 2 to 3 % (heads of 128).  The LDS is free after the next barrier.
+template <int NT, int W, bool TURN = false>
 __device__ __forceinline__ void merge_store(float* __restrict__ row, bool write, int lane, int wave, const f32q_t (&acc)[NT],
                                             const float (&mul)[W], float (&buf)[W][4 * NT][64], const float2* __restrict__ angles = nullptr) {
 #pragma unroll
@@ -108,9 +109,11 @@ __device__ __forceinline__ void merge_store(float* __restrict__ row, bool write,
 #pragma unroll
     for (int n = 0; n < NT; n++) buf[wave][r * NT + n][lane] = acc[n][r];
   const int first = NT * (4 * (lane >> 4) + wave);                 // this lane's first column
-  float2 turn[NT];
+  [[maybe_unused]] float2 turn[NT];
+  if constexpr (TURN) {
 #pragma unroll
-  for (int n = 0; n < NT; n++) turn[n] = angles != nullptr && wave < 4 ? angles[(first + n) >> 1] : make_float2(1.f, 0.f);
+    for (int n = 0; n < NT; n++) turn[n] = wave < 4 ? angles[(first + n) >> 1] : make_float2(1.f, 0.f);
+  }
   __syncthreads();
   if (W > 4 && wave >= 4) return;
   float x[NT];
@@ -120,7 +123,7 @@ __device__ __forceinline__ void merge_store(float* __restrict__ row, bool write,
 #pragma unroll
     for (int i = 0; i < W; i++) x[n] += buf[i][wave * NT + n][lane] * mul[i];
   }
-  if (angles != nullptr) {
+  if constexpr (TURN) {
     float y[NT];                                                   // the pairs' other elements: with an odd NT some are other lanes'
 #pragma unroll
     for (int n = 0; n < NT; n++) {
@@ -253,7 +256,7 @@ __global__ __launch_bounds__(64 * W) void attn_fwd_f32_kernel(const float* __res
 
 // dV = P^T dO, dK = scale dS^T Q: a block per 16 keys, walking the queries that see them.
 // DELTA: from the rows of o, where nothing has left delta.
-template <int NT, int W, bool DELTA>
+template <int NT, int W, bool DELTA, bool TURN>
 __device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* __restrict__ q, const float* __restrict__ k,
                                              const float* __restrict__ v, const float* __restrict__ o, const float* __restrict__ d_o,
                                              const float* __restrict__ lse, const float* __restrict__ delta, float* __restrict__ dk,
@@ -313,13 +316,13 @@ __device__ __forceinline__ void bwd_dkv_rows(const BlockRows own, const float* _
   float one[W];
 #pragma unroll
   for (int i = 0; i < W; i++) one[i] = 1.f;
-  merge_store<NT, W>(dk + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, acck, one, buf,
-                     unrope != nullptr ? unrope + (int64_t)(mykey < last ? mykey : last) * (8 * NT) : nullptr);
+  merge_store<NT, W, TURN>(dk + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, acck, one, buf,
+                           TURN ? unrope + (int64_t)(mykey < last ? mykey : last) * (8 * NT) : nullptr);
   __syncthreads();
   merge_store<NT, W>(dv + base + (int64_t)mykey * sh.ss, mykey < sh.seq, lane, wave, accv, one, buf);
 }
 
-template <int NT, int W>
+template <int NT, int W, bool TURN>
 __global__ __launch_bounds__(64 * W) void attn_bwd_dkv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                        const float* __restrict__ v,
                                                                        const float* __restrict__ d_o,
@@ -328,7 +331,7 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_dkv_f32_kernel(const float* _
                                                                        float* __restrict__ dv, AttnShapeF32 sh, float scale,
                                                                        int causal, const float2* __restrict__ unrope) {
   __shared__ float buf[W][4 * NT][64];
-  bwd_dkv_rows<NT, W, false>(block_rows((sh.seq + 15) >> 4), q, k, v, nullptr, d_o, lse, delta, dk, dv, sh, scale, causal, unrope, buf);
+  bwd_dkv_rows<NT, W, false, TURN>(block_rows((sh.seq + 15) >> 4), q, k, v, nullptr, d_o, lse, delta, dk, dv, sh, scale, causal, unrope, buf);
 }
 
 // dQ = scale dS K with dS = P (dP - delta), P = exp(scale q k^T - lse), dP = dO V^T, delta = rowsum(dO * O), which it also
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_dkv_f32_kernel(const float* _
 // dQ stands in its kernel, dK/dV in a function of its own: the order of the loads that the compiler makes of either depends
 // on that.  us, dQ in a function | here: 24 heads x 1000 x 96 261 | 247, 8 x 3000 x 128 784 | 768; dK/dV in its kernel | in a
 // function: 24 x 1000 x 32 105 | 98, 64 x 1024 x 48 294 | 284.
-template <int NT, int W, bool BOTH>
+template <int NT, int W, bool BOTH, bool TURN>
 __global__ __launch_bounds__(64 * W) void attn_bwd_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                                       const float* __restrict__ v, const float* __restrict__ o,
                                                                       const float* __restrict__ d_o,
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_dq_f32_kernel(const float* __
   const BlockRows own = block_rows(tiles);
   if constexpr (BOTH) {
     if (blockIdx.z == 0) {
-      bwd_dkv_rows<NT, W, true>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, unrope, buf);
+      bwd_dkv_rows<NT, W, true, TURN>(own, q, k, v, o, d_o, lse, nullptr, dk, dv, sh, scale, causal, unrope, buf);
       return;
     }
   }
@@ -400,8 +403,8 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_dq_f32_kernel(const float* __
   float one[W];
 #pragma unroll
   for (int i = 0; i < W; i++) one[i] = 1.f;
-  merge_store<NT, W>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf,
-                     unrope != nullptr ? unrope + (int64_t)qc * (8 * NT) : nullptr);
+  merge_store<NT, W, TURN>(dq + base + (int64_t)myq * sh.ss, myq < sh.seq, lane, wave, acc, one, buf,
+                           TURN ? unrope + (int64_t)qc * (8 * NT) : nullptr);
 }
 
 // Where a row of v or tv that not all queries of a block see is not finite, the masked weight 0 would carry it to the others, as it
@@ -594,13 +597,10 @@ int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   return EMI_OK;
 }
 
-// dQ, dK, dV on the fp32 matrix-core path (delta: scratch for rowsum(dO * O)); -1 when the operands do not qualify.
-int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o,
-                             const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
-                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal,
-                             const float* unrope) {
-  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
-  const float2* angles = reinterpret_cast<const float2*>(unrope);
+template <bool TURN>
+static int launch_bwd(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* delta,
+                      void* dq, void* dk, void* dv, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss,
+                      float scale, int causal, const float2* angles) {
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
   // One launch while two would each leave much of the chip idle, up to `most` blocks.  Of causal rows the late ones are the
@@ -621,7 +621,7 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
   if ((int64_t)grid.x * grid.y <= most) {
 #define EMI_BOTH(W)                                                                                                                      \
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),                                                                                            \
-                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<(W == 8 && NT > 4 ? 4 : NT), W, true>), dim3(grid.x, grid.y, 2), dim3(64 * W), 0, \
+                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<(W == 8 && NT > 4 ? 4 : NT), W, true, TURN>), dim3(grid.x, grid.y, 2), dim3(64 * W), 0, \
                                            st, (const float*)q, (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, \
                                            nullptr, (float*)dq, (float*)dk, (float*)dv, shp, scale, causal, angles))
     if (eight_adjoint((int64_t)grid.x * grid.y, seq, head_dim, causal)) EMI_BOTH(8)
@@ -631,16 +631,28 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
     return EMI_OK;
   }
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, 4, false>), grid, dim3(256), 0, st, (const float*)q,
+                        hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<NT, 4, false, TURN>), grid, dim3(256), 0, st, (const float*)q,
                                            (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, delta,
                                            (float*)dq, nullptr, nullptr, shp, scale, causal, angles));
   EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dq)");
   EMI_ATTN_F32_DISPATCH((int)(head_dim / 16),
-                        hipLaunchKernelGGL((attn_bwd_dkv_f32_kernel<NT, 4>), grid, dim3(256), 0, st, (const float*)q,
+                        hipLaunchKernelGGL((attn_bwd_dkv_f32_kernel<NT, 4, TURN>), grid, dim3(256), 0, st, (const float*)q,
                                            (const float*)k, (const float*)v, (const float*)d_o, lse, delta, (float*)dk,
                                            (float*)dv, shp, scale, causal, angles));
   EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma dkv)");
   return EMI_OK;
+}
+
+// dQ, dK, dV on the fp32 matrix-core path (delta: scratch for rowsum(dO * O); unrope: null, or the table by which dq and dk are
+// turned back); -1 when the operands do not qualify.
+int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                             const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
+                             int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal,
+                             const float* unrope) {
+  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
+  const float2* angles = reinterpret_cast<const float2*>(unrope);
+  return angles == nullptr ? launch_bwd<false>(st, q, k, v, o, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, sb, shh, ss, scale, causal, angles)
+                           : launch_bwd<true>(st, q, k, v, o, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, sb, shh, ss, scale, causal, angles);
 }
 
 // Tangent on the fp32 matrix-core path (null tangents: zero); -1 when the operands do not qualify.
