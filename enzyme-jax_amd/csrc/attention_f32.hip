@@ -561,9 +561,15 @@ bool attn_f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t s
 static bool eight_forward(int64_t blocks, int64_t seq, int64_t head_dim, int causal) {
   return head_dim <= 64 && blocks <= 256 && seq >= (head_dim <= 48 && causal ? 192 : 384);
 }
-static bool eight_adjoint(int64_t blocks, int64_t seq, int64_t head_dim, int causal) {
-  if (head_dim > 48) return head_dim <= 64 && causal && seq >= 384 && blocks <= 256;
-  return seq >= 96 && (causal ? blocks <= 160 || (seq >= 256 && blocks <= 256) : blocks <= 128);
+// In the adjoint with heads of 48 and 64 a CU has room for one such block, and an XCD's run of rows is of two rounds of them from 160
+// blocks on: dQ's long rows come too late there unless they are the first of the run, which is a head then or a part of one.  us, four |
+// eight, forward and adjoint, heads of 48: 8 x 384 (192 blocks) 26.9 | 24.1, 6 x 640 (240) 39.1 | 35.4, 8 x 448 (224) 29.9 | 26.0, 2 x 2000 (250) 92 |
+// 87, but 14 x 256 (224) 22.0 | 23.3, 10 x 384 (240) 28.4 | 30.2, 9 x 448 (252) 28.8 | 32.0, 3 x 1300 (246) 61 | 66; of 64: 8 x 512 (256) 43.9 |
+// 39.4, 10 x 384 37.0 | 40.8, 5 x 800 (250) 55.7 | 58.5.  Heads of 32, two such blocks a CU: 9 x 448 28.0 | 26.5, 3 x 1300 55 | 50.
+static bool eight_adjoint(int64_t blocks, int64_t heads, int64_t seq, int64_t head_dim, int causal) {
+  const bool long_first = head_dim <= 32 || blocks <= 160 || (heads >= 6 && heads <= 8) || 8 % heads == 0;
+  if (head_dim > 48) return head_dim <= 64 && causal && seq >= 384 && blocks <= 256 && long_first;
+  return seq >= 96 && (causal ? blocks <= 160 || (seq >= 256 && blocks <= 256 && long_first) : blocks <= 128);
 }
 
 #define EMI_ATTN_F32_DISPATCH(NTV, CALL)      \
@@ -624,7 +630,7 @@ static int launch_bwd(hipStream_t st, const void* q, const void* k, const void* 
                         hipLaunchKernelGGL((attn_bwd_dq_f32_kernel<(W == 8 && NT > 4 ? 4 : NT), W, true, TURN>), dim3(grid.x, grid.y, 2), dim3(64 * W), 0, \
                                            st, (const float*)q, (const float*)k, (const float*)v, (const float*)o, (const float*)d_o, lse, \
                                            nullptr, (float*)dq, (float*)dk, (float*)dv, shp, scale, causal, angles))
-    if (eight_adjoint((int64_t)grid.x * grid.y, seq, head_dim, causal)) EMI_BOTH(8)
+    if (eight_adjoint((int64_t)grid.x * grid.y, grid.y, seq, head_dim, causal)) EMI_BOTH(8)
     else EMI_BOTH(4)
 #undef EMI_BOTH
     EMI_CHECK_LAUNCH("emi_attn_bwd(fp32 mfma)");

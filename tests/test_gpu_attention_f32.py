@@ -103,6 +103,12 @@ def test_f32_attention_eight_wavefronts(B, h, S, d, causal):
     test_f32_attention_tiles(B, h, S, d, causal)
 
 
+@pytest.mark.parametrize("B,h,S,d", [(1, 8, 321, 48), (1, 9, 321, 48), (1, 6, 430, 64), (1, 5, 590, 64), (2, 2, 650, 48), (1, 3, 900, 32)])
+def test_f32_attention_long_rows_of_several_heads(B, h, S, d):
+    """More than 160 blocks: eight wavefronts where an XCD's rows begin with a head's or are part of one, else four.  Bounds as above."""
+    test_f32_attention_tiles(B, h, S, d, True)
+
+
 @pytest.mark.parametrize("h,S,d", [(3, 40, 48), (6, 256, 48), (5, 33, 80), (2, 70, 32), (40, 300, 64), (3, 50, 40)])
 def test_f32_attention_adjoint_turns_its_operands_back(h, S, d):
     """The inverse rotation where dq and dk leave, with an odd and an even number of 16-column tiles a head (a pair's elements in
