@@ -144,3 +144,51 @@ def test_what_the_kernels_do_not_take_is_left_to_the_separate_launches():
                            (64, 64, 64, 1, tail(ADJOINT, 4))):
         assert _run(x, w, t, M, N, K, tb, "f32") == -1
     assert all(bool((o == 7.0).all()) for o in out)
+
+
+@pytest.mark.parametrize("dt,mode,M,N,K", CASES + [(dt, 5, M, N, K) for dt, M, N, K, _ in PAIRS])
+def test_tails_write_nothing_outside_their_results(dt, mode, M, N, K):
+    """Every size above (5: two products to each of three results), the results with room before and behind them."""
+    pairs = mode == 5
+    mode = ROTATED if pairs else mode
+    x, x1, w = (torch.randn(n, K, device="cuda").to(torch.bfloat16 if dt == "bf16" else torch.float32) for n in (M, M, N))
+    h = torch.randn(M, N, device="cuda").to(x.dtype)
+    table = torch.randn(M, N // 2, 2, device="cuda")
+    edge = 4096
+    for tb in (1, 0) if mode == ADJOINT else (1,):
+        room = [torch.full((M * N + 2 * edge,), 7.0, device="cuda", dtype=x.dtype) for _ in range(3)]
+        tail = _Tail(mode=mode, table=table.data_ptr(), seq=M, head_dim=N, rotated=2, count=3, h1=h.data_ptr(), h3=h.data_ptr(),
+                     A1=x1.data_ptr() if pairs else None)
+        for i in range(3):
+            tail.B[i], tail.B1[i], tail.C[i] = w.data_ptr(), w.data_ptr() if pairs else None, room[i].data_ptr() + edge * x.element_size()
+        rc = _run(x, w, tail, M, N, K, tb, dt)
+        written = {GATED: 3, ROTATED: 3, ADJOINT: 2}[mode] if rc == 0 else 0
+        assert rc == 0 or (pairs and rc == -1)           # (three results where the test above has two)
+        for i, r in enumerate(room):
+            inside = r[edge:edge + M * N]
+            assert bool((r[:edge] == 7.0).all()) and bool((r[edge + M * N:] == 7.0).all()), i
+            assert bool((inside != 7.0).any()) == (i < written)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_what_either_type_leaves_to_the_separate_launches(dt):
+    """As above in both types: rows and contractions of no whole pieces, few rows, operands and results off 16 bytes, a k-major weight
+    of two or three results."""
+    dtype, v = (torch.bfloat16, 8) if dt == "bf16" else (torch.float32, 4)
+    x, w, h = (torch.ones(64 * 64 + 16, device="cuda", dtype=dtype) for _ in range(3))
+    table = torch.ones(64 * 64 + 4, device="cuda")
+    room = [torch.full((64 * 64 + 16,), 7.0, device="cuda", dtype=dtype) for _ in range(3)]
+
+    def tail(mode, h1=0, c=0, b=0, angles=0):
+        t = _Tail(mode=mode, h1=h.data_ptr() + h1, h3=h.data_ptr(), table=table.data_ptr() + angles, seq=64, head_dim=8, rotated=2, count=3)
+        for i in range(3):
+            t.B[i], t.C[i] = w.data_ptr() + b, room[i].data_ptr() + c
+        return t
+
+    for mode in (GATED, ROTATED, ADJOINT):
+        for M, N, K in ((64, 64 - v // 2, 64), (64, 64, 64 - v // 2), (8, 64, 64)):
+            assert _run(x, w, tail(mode), M, N, K, 1, dt) == -1
+        assert _run(x, w, tail(mode, c=8), 64, 64, 64, 1, dt) == -1 and _run(x, w, tail(mode, b=8), 64, 64, 64, 1, dt) == -1
+        assert mode == ADJOINT or _run(x, w, tail(mode), 64, 64, 64, 0, dt) == -1
+    assert _run(x, w, tail(ADJOINT, h1=8), 64, 64, 64, 1, dt) == -1 and _run(x, w, tail(ROTATED, angles=8), 64, 64, 64, 1, dt) == -1
+    assert all(bool((r == 7.0).all()) for r in room)

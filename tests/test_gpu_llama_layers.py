@@ -204,3 +204,30 @@ def test_llama_layer_tangent_in_the_operators_order():
     with ops.Tape():                                     # under a tape the operators run one by one
         want, twant = run()
     assert torch.equal(y, want) and torch.equal(ty, twant)
+
+
+def test_llama_layers_jvp_checks_its_arguments():
+    """A short workspace, a null tangent, weight or operand, and shapes and types that are not served are errors before any launch."""
+    import ctypes
+    from enzyme_ad.jax import llama, ops
+    from enzyme_ad.jax import _native as N
+    lib, B, S, D, H, heads = N.lib(), 1, 33, 64, 72, 2
+    _, wd, _, x, _, _, _ = _inputs("f32", D, H, 2, heads, B, S)
+    w, table = [wd[k] for k in llama.LAYER_KEYS], ops.rope_table(S, D // heads, device=x.device)
+    y, ty = torch.full_like(x, 7.0), torch.full_like(x, 7.0)
+    need = lib.emi_llama_layers_jvp_workspace_bytes(B, S, D, H, heads, 11)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
+
+    def call(weights=w, tangents=w, tx=x, nws=need, dims=(2, B, S, D, H, heads), dt=11):
+        return lib.emi_llama_layers_jvp(torch.cuda.current_stream().cuda_stream, ptrs(weights), ptrs(tangents), x.data_ptr(),
+                                        None if tx is None else tx.data_ptr(), table.data_ptr(), y.data_ptr(), ty.data_ptr(), ws.data_ptr(), nws,
+                                        *dims, 1e-5, 0.2, dt)
+
+    for i in range(9):
+        assert call(tangents=w[:i] + [None] + w[i + 1:]) == 3 and call(weights=w[:i] + [None] + w[i + 1:]) == 3
+    assert call(tx=None) == 3 and call(nws=need - 1) == 3 and call(nws=0) == 3 and call(dt=7) == 3
+    for dims in ((0, B, S, D, H, heads), (2, 0, S, D, H, heads), (2, B, S, D, H, 3), (2, B, S, 62, H, heads), (2, B, S, D, 70, heads)):
+        assert call(dims=dims) == 3 and (dims[0] == 0 or lib.emi_llama_layers_jvp_workspace_bytes(*dims[1:], 11) == 0), dims
+    assert bool((y == 7.0).all()) and bool((ty == 7.0).all())
+    assert call() == 0 and bool((y != 7.0).any()) and bool((ty != 7.0).any())
