@@ -138,7 +138,7 @@ __device__ __forceinline__ void merge_store(float* __restrict__ row, bool write,
     }
 #pragma unroll
     for (int n = 0; n < NT; n++)
-      x[n] = ((first + n) & 1) == 0 ? rotated_even(turn[n].x, -turn[n].y, x[n], y[n]) : rotated_odd(turn[n].x, -turn[n].y, y[n], x[n]);
+      x[n] = ((first + n) & 1) == 0 ? rotated_even(turn[n].x, -turn[n].y, x[n], y[n]) : rotated_odd<float>(turn[n].x, -turn[n].y, y[n], x[n]);
   }
   if (write) {
     float* p = row + first;

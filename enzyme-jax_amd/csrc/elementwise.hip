@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void rope_kernel(const T* x, const float2* __r
     const float sn = (p & 1) ? t[p >> 1].w : t[p >> 1].y;
     const float sp = inverse ? -sn : sn;
     o[2 * p] = rotated_even(cs, sp, v[2 * p], v[2 * p + 1]);
-    o[2 * p + 1] = rotated_odd(cs, sp, v[2 * p], v[2 * p + 1]);
+    o[2 * p + 1] = rotated_odd<T>(cs, sp, v[2 * p], v[2 * p + 1]);
   }
   if (beyond) Chunk<T>::store(y + (int64_t)row * row_elems + col, o);
   else ChunkCached<T>::store(y + (int64_t)row * row_elems + col, o);
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void rope_pair_kernel(const T* x, const float2
   const float sp = inverse ? -t.y : t.y;
   const float v0 = to_f32(x[e]), v1 = to_f32(x[e + 1]);
   y[e] = from_f32<T>(rotated_even(t.x, sp, v0, v1));
-  y[e + 1] = from_f32<T>(rotated_odd(t.x, sp, v0, v1));
+  y[e + 1] = from_f32<T>(rotated_odd<float>(t.x, sp, v0, v1));
 }
 
 // ---------------------------------------------------------------------------

@@ -75,9 +75,11 @@ __device__ __forceinline__ void emi_swiglu_adjoint(float a, float b, float dg, f
 }
 
 // A rotation pair (v0, v1) turned by the angle of (cos, sin), shared by the rotation's own kernels and the products that apply it
-// to a tile: which of the two products is rounded is written down, so that both give the same bits.
+// to a tile: which of the two products is rounded is written down, so that both give the same bits.  T: of the odd element it is
+// c v1, of a 16-byte piece of bf16 s v0.
 __device__ __forceinline__ float rotated_even(float c, float s, float v0, float v1) { return fmaf(c, v0, -(s * v1)); }
-__device__ __forceinline__ float rotated_odd(float c, float s, float v0, float v1) { return fmaf(s, v0, c * v1); }
+template <typename T> __device__ __forceinline__ float rotated_odd(float c, float s, float v0, float v1) { return fmaf(c, v1, s * v0); }
+template <> __device__ __forceinline__ float rotated_odd<float>(float c, float s, float v0, float v1) { return fmaf(s, v0, c * v1); }
 
 // Eight consecutive elements as fp32 (one 16-byte load for bf16, two for fp32).
 template <typename T> struct Vec8;

@@ -426,7 +426,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_bf16_pipe_kernel(const u
           for (int q = 0; q < 4; q++) {
             const float2 t = angles[((gcol + 2 * q) % grp.head_dim) >> 1];
             o[2 * q] = rotated_even(t.x, t.y, v[2 * q], v[2 * q + 1]);
-            o[2 * q + 1] = rotated_odd(t.x, t.y, v[2 * q], v[2 * q + 1]);
+            o[2 * q + 1] = rotated_odd<bf16>(t.x, t.y, v[2 * q], v[2 * q + 1]);
           }
           z = pack8(o);
         }

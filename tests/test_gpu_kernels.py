@@ -79,6 +79,24 @@ def test_rope_large_positions_fp32(ops):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_rope_bits(ops, dt, inverse):
+    """Each element is one product added, unrounded, to the other one rounded to fp32: c v0 - [s v1], and s v0 + [c v1] in fp32 but
+    c v1 + [s v0] in bf16.  Products that rotate their own result round alike, so a bit here is a bit of every bf16 model's results."""
+    B, S, h, d = 2, 1024, 12, 64
+    x, _ = dev(np.random.default_rng(8).standard_normal((B, S, h * d)), dt)
+    table = ops.rope_table(S, d)
+    c, s = (table[..., i].double().cpu()[None, :, None, :] for i in range(2))
+    s = -s if inverse else s
+    v0, v1 = x.double().cpu().reshape(B, S, h, d // 2, 2).unbind(-1)
+    rounded = lambda t: t.float().double()
+    even = (c * v0 - rounded(s * v1)).float()
+    odd = (s * v0 + rounded(c * v1) if dt == "f32" else c * v1 + rounded(s * v0)).float()
+    want = torch.stack((even, odd), -1).reshape(B, S, h * d).to(x.dtype)
+    assert torch.equal(ops.rope(x, h, inverse=inverse).cpu(), want)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("n", [8, 1003, 4096 * 3 + 5])
 def test_swiglu_and_add(ops, dt, n):
     _say("swiglu", dt, n)
