@@ -541,16 +541,12 @@ __global__ __launch_bounds__(64 * 4) void attn_jvp_f32_kernel(const float* __res
   }
 }
 
-static bool f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
+bool attn_f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
   if (d % 16 != 0 || d > 128 || seq < 1) return false;
   if ((sb | shh | ss) & 3) return false;
   for (const void* p : ptrs)
     if (reinterpret_cast<uintptr_t>(p) & 15) return false;
   return true;
-}
-
-bool attn_f32_mfma_ok(int64_t seq, int64_t d, int64_t sb, int64_t shh, int64_t ss, std::initializer_list<const void*> ptrs) {
-  return f32_mfma_ok(seq, d, sb, shh, ss, ptrs);
 }
 
 // Eight wavefronts a block where the blocks have a CU each and the longest row, which sets the time, is of tiles enough; heads of
@@ -589,7 +585,7 @@ static bool eight_adjoint(int64_t blocks, int64_t heads, int64_t seq, int64_t he
 int launch_attn_fwd_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int64_t batch,
                              int64_t heads, int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale,
                              int causal) {
-  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o})) return -1;
+  if (!attn_f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o})) return -1;
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
   const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)(batch * heads));
 #define EMI_FWD(W)                                                                                                                   \
@@ -655,7 +651,7 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
                              const float* lse, float* delta, void* dq, void* dk, void* dv, int64_t batch, int64_t heads,
                              int64_t seq, int64_t head_dim, int64_t sb, int64_t shh, int64_t ss, float scale, int causal,
                              const float* unrope) {
-  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
+  if (!attn_f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, o, d_o, dq, dk, dv})) return -1;
   const float2* angles = reinterpret_cast<const float2*>(unrope);
   return angles == nullptr ? launch_bwd<false>(st, q, k, v, o, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, sb, shh, ss, scale, causal, angles)
                            : launch_bwd<true>(st, q, k, v, o, d_o, lse, delta, dq, dk, dv, batch, heads, seq, head_dim, sb, shh, ss, scale, causal, angles);
@@ -665,7 +661,7 @@ int launch_attn_bwd_f32_mfma(hipStream_t st, const void* q, const void* k, const
 int launch_attn_jvp_f32_mfma(hipStream_t st, const void* q, const void* k, const void* v, const float* lse, const void* tq,
                              const void* tk, const void* tv, void* to, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
                              int64_t sb, int64_t shh, int64_t ss, float scale, int causal) {
-  if (!f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, tq, tk, tv, to})) return -1;
+  if (!attn_f32_mfma_ok(seq, head_dim, sb, shh, ss, {q, k, v, tq, tk, tv, to})) return -1;
   const AttnShapeF32 shp{(int)seq, (int)heads, sb, shh, ss};
 #define EMI_JVP_F32(QS)                                                                                                         \
   do {                                                                                                                          \

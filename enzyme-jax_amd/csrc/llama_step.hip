@@ -53,15 +53,16 @@ template <typename T> __device__ __forceinline__ float normed(float x, float gam
 // forward: products of a normalised vector
 // ---------------------------------------------------------------------------
 // A wavefront owns two rows at a time: MODE 0, rows 2p and 2p + 1 of [w0; w1; w2] (q, k, v: a rotation pair of q or k);
-// MODE 1, row p of w0 and of w1 (h1, h3 of the SwiGLU); MODE 2, rows 2p and 2p + 1 of w0 (wo) times the attention's result,
-// which each block works out for itself (step_attention).  The rows stream through in batches of UN 16-byte pieces per lane,
+// MODE 1, row p of w0 and of w1 (h1, h3 of the SwiGLU); MODE 2 and 3, rows 2p and 2p + 1 of w0 (wo) times the attention's result,
+// which each block works out for itself, from the keys and values (2: step_attention) or by adding up its key blocks' shares (3:
+// step_combine).  The rows stream through in batches of UN 16-byte pieces per lane,
 // the next pair's first batch requested while the current one is summed, and the first pair's before the block normalises
 // the vector: each block keeps gamma x / rms(x) in LDS (the two halves of an eight-element piece apart, so that a
 // lane's reads of 16 bytes do not collide).
 template <typename T> struct NormGemv {
-  const T *x, *gamma;    // MODE 2: x is the residual
+  const T *x, *gamma;    // MODE 2, 3: x is the residual
   const T* w[3];
-  T* y[3];               // MODE 0: q, k, v;  MODE 1: h1, h3, g;  MODE 2: x + w0 att
+  T* y[3];               // MODE 0: q, k, v;  MODE 1: h1, h3, g;  MODE 2, 3: x + w0 att
   float* rms;            // 1 / rms(x), for the adjoint
   const float2* table;   // MODE 0: (cos, sin) of pair i at i % table_pairs
   int N, K, table_pairs;
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(1024) void step_norm_kernel(const T* __restrict__ x
 //
 // What lies between two such products needs a value of every band: the norm's adjoint, the SwiGLU's, the inverse rotation.  The
 // kernel behind works it out itself, for its band's rows alone, while its first rows of W are on their way, so bands are few
-// (at most kMostBands, of narrow blocks) and the norm's one sum over all columns, which is linear in them, arrives as a share
+// (kMostBands of narrow blocks; more only so that a band has at most kMostRows rows) and the norm's one sum over all columns, which is linear in them, arrives as a share
 // of every block (`dots`).  Five launches a layer; nine when the bands were 96 and their sums launches of their own (a
 // norm's 5.7 us of one block, the others 2.6).
 template <typename T> struct Adjoint {
@@ -948,7 +949,7 @@ int step_bwd(hipStream_t st, const void* const* w, const void* x_, const void* k
 
 bool dims_ok(const StepDims& d) {
   const int64_t V = d.dtype == EMI_BF16 ? 8 : 4;
-  // LDS: the padded vector of the product kernel, the vector of the norm's adjoint
+  // D: the padded vector of the product kernel stands in LDS
   return (d.dtype == EMI_BF16 || d.dtype == EMI_F32) && d.L > 0 && d.D > 0 && d.H > 0 && d.heads > 0 && d.D % d.heads == 0 &&
          d.D % V == 0 && d.H % V == 0 && d.hd() % V == 0 && d.hd() <= 256 && d.D <= 8192 && d.H <= (1 << 20) && d.heads <= 65535 && d.pos > 0 &&
          d.pos < (1 << 30) && d.table_pairs > 0 && (d.D / 2) % d.table_pairs == 0;

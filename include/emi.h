@@ -214,9 +214,9 @@ int emi_attn_bwd(emi_stream_t stream, const void* q, const void* k, const void* 
 
 /* emi_attn_bwd for q and k that are RoPE outputs (test/llama.py:161-168 in front of :178-206): dq and dk are the
  * cotangents of the vectors BEFORE the rotation, i.e. emi_attn_bwd followed by emi_rope(inverse) on dq and dk, with
- * the rotation applied as the MFMA kernels (bf16, head_dim 64 or 128) store their results, in fp32 before the one
- * rounding.  Other shapes run emi_attn_bwd and two emi_rope passes in place and need contiguous
- * [batch, seq, heads, head_dim] operands.  rope_table: [seq, head_dim/2] of (cos, sin), 16-byte aligned. */
+ * the rotation applied as the MFMA kernels (bf16, head_dim 64 or 128; fp32, head_dim a multiple of 16 up to 128) store
+ * their results, in fp32 before the one rounding.  Other shapes run emi_attn_bwd and two emi_rope passes in place.  All
+ * but the bf16 kernels' operands have to be contiguous [batch, seq, heads, head_dim].  rope_table: [seq, head_dim/2] of (cos, sin), 16-byte aligned. */
 int emi_attn_bwd_rope(emi_stream_t stream, const void* q, const void* k, const void* v, const void* o, const float* lse,
                       const void* d_o, void* dq, void* dk, void* dv, const float* rope_table, void* workspace,
                       size_t workspace_bytes, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim, int64_t stride_b,
