@@ -2068,6 +2068,14 @@ int emi::gemm_run(hipStream_t st, const void* A, const void* B, const void* R, v
   return launch_generic<float>(st, A, B, R, C, (int)M, (int)N, (int)K, lda, ldb, ldr, ldc, trans_a, trans_b, workspace, workspace_bytes);
 }
 
+int emi::reserve_lds(const void* kernel, int bytes, bool& configured) {
+  if (configured) return EMI_OK;
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+  configured = true;
+  return EMI_OK;
+}
+
 int emi::gemm_tail(hipStream_t st, const void* A, const void* B, const ProductTail& t, int64_t M, int64_t N, int64_t K, int64_t ldb, int trans_b,
                    int dtype) {
   // rows of whole 16-byte pieces, operands and results of less than 2 GiB

@@ -483,18 +483,19 @@ struct PipeCall {
   int* planes;                // not null: splits stay planes in `part`, *planes of them (gemm_run)
 };
 
+// The ring of stages, and in the same place the wavefronts' tiles on their way out.
+constexpr int pipe_lds(int bm, int bn, int wm, int wn, int wk, int bk, int nst) {
+  const int ring = nst * (bm + bn) * bk * 2, tile = wm * wn * wk * (bm / wm) * (bn / wn + 4) * 4;
+  return ring > tile ? ring : tile;
+}
+
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, bool GROUPED>
 static int launch_pipe_one(hipStream_t st, const PipeCall& c) {
   auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, BKM, GROUPED ? kTailGroup : kTailNone>;
-  constexpr int ring = NST * (BM + BN) * BK * 2, tile = WM * WN * WK * (BM / WM) * (BN / WN + 4) * 4;
-  constexpr int smem = ring > tile ? ring : tile;
+  constexpr int smem = pipe_lds(BM, BN, WM, WN, WK, BK, NST);
   static_assert(smem <= 160 * 1024, "LDS of a CU");
-  static bool configured = false;   // idempotent; a race only repeats the call
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
-    configured = true;
-  }
+  static bool configured = false;
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), smem, configured)) return rc;
   const int steps = ((c.K + BK - 1) / BK) * (GROUPED && c.grp->sum ? c.grp->count : 1);
   const int sps = (steps + c.splits - 1) / c.splits, nz = (steps + sps - 1) / sps;
   const int outer = GROUPED && !c.grp->sum ? c.grp->count : nz;
@@ -637,14 +638,9 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
 template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, int MODE>
 static int launch_pipe_tail_one(hipStream_t st, const uint16_t* A, const uint16_t* B, const ProductTail& t, int M, int N, int K, int ldb) {
   auto kern = gemm_bf16_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, BKM, MODE>;
-  constexpr int ring = NST * (BM + BN) * BK * 2, tile = WM * WN * WK * (BM / WM) * (BN / WN + 4) * 4;
-  constexpr int smem = ring > tile ? ring : tile;
-  static bool configured = false;   // idempotent; a race only repeats the call
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
-    configured = true;
-  }
+  constexpr int smem = pipe_lds(BM, BN, WM, WN, WK, BK, NST);
+  static bool configured = false;
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), smem, configured)) return rc;
   typename PipeArg<MODE>::type arg{};
   if constexpr (MODE == kTailGated) {
     arg = {static_cast<const uint16_t*>(t.B[1]), static_cast<uint16_t*>(t.C[1]), static_cast<uint16_t*>(t.C[2])};

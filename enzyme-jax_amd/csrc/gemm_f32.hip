@@ -408,12 +408,8 @@ static int launch_f32_one(hipStream_t st, const F32Call& c) {
   auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, AKM, BKM, GROUPED ? kTailGroup : kTailNone>;
   constexpr int smem = NST * (BM + BN) * BK * 4;
   static_assert(WK == 1 || smem >= WK * 32 * 33 * 4, "the wavefronts' tiles meet in the ring");
-  static bool configured = false;   // idempotent; a race only repeats the call
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
-    configured = true;
-  }
+  static bool configured = false;
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), smem, configured)) return rc;
   const int steps = ((c.K + BK - 1) / BK) * (GROUPED && c.grp->sum ? c.grp->count : 1);
   const int sps = (steps + c.splits - 1) / c.splits, nz = (steps + sps - 1) / sps;
   const int outer = GROUPED && !c.grp->sum ? c.grp->count : nz;
@@ -555,12 +551,8 @@ template <int BM, int BN, int WM, int WN, int WK, int BK, int NST, bool BKM, int
 static int launch_f32_tail_one(hipStream_t st, const float* A, const float* B, const ProductTail& t, int M, int N, int K, int ldb) {
   auto kern = gemm_f32_pipe_kernel<BM, BN, WM, WN, WK, BK, NST, false, BKM, MODE>;
   constexpr int smem = NST * (BM + BN) * BK * 4;
-  static bool configured = false;   // idempotent; a race only repeats the call
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return emi_fail(EMI_INTERNAL, "emi_gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
-    configured = true;
-  }
+  static bool configured = false;
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), smem, configured)) return rc;
   typename F32Arg<MODE>::type arg{};
   if constexpr (MODE == kTailGated) {
     arg = {static_cast<const float*>(t.B[1]), static_cast<float*>(t.C[1]), static_cast<float*>(t.C[2])};

@@ -53,6 +53,9 @@ int launch_bf16_pipe(hipStream_t st, const Bf16Plan& plan, int count, const void
                      void* const* C, float* part, int M, int N, int K, int lda, int ldb, int64_t ldr, int64_t ldc, int vec_ok, int trans_b,
                      int sum, int* planes);
 
+// Lets a kernel have `bytes` of LDS, once (`configured`: one to a kernel; a race only repeats the call).
+int reserve_lds(const void* kernel, int bytes, bool& configured);                                        // gemm.hip
+
 // emi_gemm_ws and emi_gemm_grouped for a caller that adds the planes of a product split over K itself: with `planes` not null
 // such a product leaves *planes fp32 planes [M, N] in the workspace, to be added in order and then to R, and C unwritten;
 // *planes is 0 where C is complete.
