@@ -544,8 +544,10 @@ int launch_copy(hipStream_t st, const void* in, void* out, const CopyPlan& p) {
 // Several arrays, each of whole bytes, in one launch: a block has kCopyBlock bytes of one of them, all its loads in flight at
 // once.  A replayed graph's arguments are a dozen arrays of a few KB and two or three of tens of MB: a launch each is 2 to 3 us on
 // the GPU and 5 on the host (dim-288 training step, 15 arguments, 98 MB, replayed: 855 -> 808 us; dim-768 model of 64 tokens, bf16, 353 ->
-// 282).  Small blocks and loads through the caches, from which graphs read next.  Replay of a graph of two arrays of 256 MiB, us: a copy each
-// 205, blocks of 64 KiB streaming 216, of 16 KiB 192; one of 128 MiB 44, 52, 44.  Off 16-byte boundaries (copy_words), three arrays
+// 282).  Small blocks, and a stream of loads, which leaves the caches to what the graph reads next. Replay of a
+// graph of three arrays of 256 MiB, us: a copy each 309, blocks of 64 KiB 323, of 16 KiB 289 (loads through the caches 295); of 64 MiB 86, 72, 69
+// (81); of four of 32 MiB 48, 53, 51 (48); the training step 791 with 64 KiB, 787 (811).
+// Off 16-byte boundaries (copy_words), three arrays
 // of 32 MiB of which one | all are off by an element: a copy each 46 | 48, byte by byte 86 | 149, in words 44 | 43.
 constexpr int kCopyArrays = 48, kCopyUnroll = 4, kCopyBlock = kBlock * 16 * kCopyUnroll;
 struct CopyMany {
@@ -590,7 +592,7 @@ __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyMany m) {
 #pragma unroll
   for (int u = 0; u < kCopyUnroll; u++) {
     const int c = u * kBlock + threadIdx.x;
-    v[u] = c < pieces ? reinterpret_cast<const uint4*>(src)[c] : make_uint4(0, 0, 0, 0);
+    v[u] = c < pieces ? stream_load(reinterpret_cast<const uint4*>(src) + c) : make_uint4(0, 0, 0, 0);
   }
 #pragma unroll
   for (int u = 0; u < kCopyUnroll; u++) {
