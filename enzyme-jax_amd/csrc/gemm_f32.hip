@@ -342,8 +342,10 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void gemm_f32_pipe_kernel(const
   // element e of this lane's: what the elementwise operator reads beside it has been there since before the contraction
   auto put = [&](int row, int col, float v, float h1, float p, float q) __attribute__((always_inline)) {
     if constexpr (MODE == kTailRotated) {                  // the pair's other column is the neighbouring lane's, of the same row
-      const float other = lane_xor1(v);
-      v = (col & 1) == 0 ? rotated_even(p, q, v, other) : rotated_odd<float>(p, q, other, v);
+      if (outer < grp.rotated) {                           // (turned by no angle, an infinity would make its neighbour a NaN)
+        const float other = lane_xor1(v);
+        v = (col & 1) == 0 ? rotated_even(p, q, v, other) : rotated_odd<float>(p, q, other, v);
+      }
     }
     if (row < M && col < N) {
       if (part != nullptr) {

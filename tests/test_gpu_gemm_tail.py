@@ -192,3 +192,25 @@ def test_what_either_type_leaves_to_the_separate_launches(dt):
         assert mode == ADJOINT or _run(x, w, tail(mode), 64, 64, 64, 0, dt) == -1
     assert _run(x, w, tail(ADJOINT, h1=8), 64, 64, 64, 1, dt) == -1 and _run(x, w, tail(ROTATED, angles=8), 64, 64, 64, 1, dt) == -1
     assert all(bool((r == 7.0).all()) for r in room)
+
+
+@pytest.mark.parametrize("dt,pairs", [(dt, pairs) for dt in ("f32", "bf16") for pairs in (0, 1)])
+@pytest.mark.parametrize("M,N,K", [(35, 72, 72), (233, 288, 288)])
+def test_a_result_that_is_not_turned_keeps_its_infinities(dt, pairs, M, N, K):
+    """One infinity or NaN in a weight's row j: column j of that result, and of a turned one its pair's other column, nothing else."""
+    for value in (float("inf"), float("nan")):
+        x, x1 = (torch.rand(M, K, device="cuda").to(torch.bfloat16 if dt == "bf16" else torch.float32) + 0.5 for _ in range(2))
+        ws, w1s = ([torch.randn(N, K, device="cuda").to(x.dtype) for _ in range(3)] for _ in range(2))
+        for i, j in enumerate((4, 11, N - 1)):
+            (w1s if pairs else ws)[i][j, 5] = value
+        out = [torch.full((M, N), 7.0, device="cuda", dtype=x.dtype) for _ in range(3)]
+        table = torch.rand(M, 4, 2, device="cuda") + 0.5
+        tail = _Tail(mode=ROTATED, table=table.data_ptr(), seq=M, head_dim=8, rotated=2, count=3, A1=x1.data_ptr() if pairs else None)
+        for i in range(3):
+            tail.B[i], tail.B1[i], tail.C[i] = ws[i].data_ptr(), w1s[i].data_ptr() if pairs else None, out[i].data_ptr()
+        assert _run(x, ws[0], tail, M, N, K, 1, dt) == 0
+        for o, columns in zip(out, ((4, 5), (10, 11), (N - 1,))):
+            wrong = torch.zeros(N, dtype=torch.bool, device="cuda")
+            wrong[list(columns)] = True
+            assert bool((o.isfinite() == ~wrong).all())
+        assert bool((out[2][:, N - 1].isnan() if value != value else out[2][:, N - 1] == value).all())
